@@ -328,6 +328,31 @@ __device__ __forceinline__ void warm_lines(const WeightJobs &pw, unsigned first,
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
+// ---- which tile a position of the XCD-aware order is ---------------------------------------
+// XCD x works on the positions [x * per, (x + 1) * per) and every XCD has an L2 of its own, so
+// what the launch fetches from the memory side is, per XCD, the distinct rows of A plus the
+// distinct columns of W in its range.  The order therefore walks the tile grid in panels of
+// `gn` tile columns (row tiles outermost inside a panel) such that a range of `per` positions
+// is close to a square of operand elements: gn BN = (per / gn) BM.  Plain row-major order
+// (gn = tiles_n) makes every XCD read the whole weight as soon as a range is a tile row
+// long: 28 MB instead of 7 MB for the QKV product of 256 rows at hidden 768.
+struct TilePanels {
+  int tiles_m, tiles_n, gn;
+  __device__ __forceinline__ void locate(int L, int &tile_m, int &tile_n) const {
+    const int panel = L / (tiles_m * gn);
+    const int r = L - panel * tiles_m * gn;
+    const int w = min(gn, tiles_n - panel * gn);   // the last panel may be narrower
+    tile_m = r / w;
+    tile_n = panel * gn + r - tile_m * w;
+  }
+};
+template <int BM, int BN>
+__device__ __forceinline__ TilePanels tile_panels(int tiles_m, int tiles_n, int per) {
+  int gn = (int)(__builtin_amdgcn_sqrtf((float)per * ((float)BM / (float)BN)) + 0.5f);
+  gn = max(gn, (per + tiles_m - 1) / tiles_m);   // a range taller than the grid is wider instead
+  return TilePanels{tiles_m, tiles_n, __builtin_amdgcn_readfirstlane(max(1, min(gn, tiles_n)))};
+}
+
 // ---- balanced work list of the streaming attention kernels -------------------------
 // Within an XCD the hardware deals consecutive workgroups to its 32 CUs round-robin
 // (slot s of the XCD lands on CU s % 32), and a launch of a few workgroups per CU is

@@ -1,6 +1,5 @@
 // The OperationType::FP32 flavour of the encoder layer on gfx950: every tensor
-// is float, every product runs on v_mfma_f32_32x32x2_f32 (true fp32 operands and
-// accumulators).  Three kernels:
+// is float and so is every accumulator.  Three kernels:
 //
 //   f32_gemm_kernel       C = A[M,K] . W[K,N] (+bias, +tanh-GELU), W row-major as the
 //                         caller stores it (no pre-pack: a row-major W tile already is the
@@ -17,9 +16,9 @@
 //                         scattered to the padded layout with zero fill
 //                         (layernorm.h:20-40, layernorm.cu:89-148 for float).
 //
-// fp32 MFMA runs at 1/16 of the fp16 rate, so both MFMA kernels are compute bound with
-// a trivial memory system: one LDS buffer pair, register-staged global loads, scalar
-// ds_read operands (4 LDS reads feed 256 clocks of MFMA).
+// fp32 MFMA runs at 1/16 of the bf16 rate: the products of the linear layers multiply each float as
+// a sum of three bfloat16 instead (see below), the attention stays on v_mfma_f32_32x32x2_f32, compute
+// bound with a trivial memory system (one LDS buffer pair, register-staged global loads).
 #include "common.h"
 
 namespace bt {
@@ -41,6 +40,58 @@ __device__ __forceinline__ float gelu_tanh(float x) {
 }
 
 // ---------------------------------------------------------------------------
+// float operands as bfloat16 triples
+// ---------------------------------------------------------------------------
+// A float has 24 significand bits, three bfloat16 have 3 x 8: x = h + m + l exactly, with
+// h = bf16(x), m = bf16(x - h), l = bf16(x - h - m) (round to nearest, so |m| <= 2^-9 |x| and
+// |l| <= 2^-18 |x|; both differences are exact).  A product of two floats is then nine bf16
+// products, each exact in the MFMA's float accumulator; the three smallest (m l, l m, l l: at most
+// 2^-26 of the product) are below the rounding of a float product and are left out.  Six
+// v_mfma_f32_32x32x16_bf16 do in 192 clocks what eight v_mfma_f32_32x32x2_f32 do in 512.
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+
+struct Bf16Triple {   // of two neighbouring elements: h, m and l as packed pairs
+  unsigned h, m, l;
+};
+__device__ __forceinline__ unsigned pack_bf16(float a, float b) {
+  return __builtin_bit_cast(unsigned, __builtin_convertvector(float2_t{a, b}, bf16x2_t));
+}
+__device__ __forceinline__ float bf16_low(unsigned p) { return __builtin_bit_cast(float, p << 16); }
+__device__ __forceinline__ float bf16_high(unsigned p) {
+  return __builtin_bit_cast(float, p & 0xffff0000u);
+}
+__device__ __forceinline__ Bf16Triple split_bf16(float a, float b) {
+  Bf16Triple t;
+  t.h = pack_bf16(a, b);
+  const float ra = a - bf16_low(t.h), rb = b - bf16_high(t.h);
+  t.m = pack_bf16(ra, rb);
+  t.l = pack_bf16(ra - bf16_low(t.m), rb - bf16_high(t.m));
+  return t;
+}
+__device__ __forceinline__ void split_bf16x8(bf16x8_t (&out)[3], const float (&x)[8]) {
+  uint4_t v[3];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const Bf16Triple t = split_bf16(x[2 * j], x[2 * j + 1]);
+    v[0][j] = t.h, v[1][j] = t.m, v[2][j] = t.l;
+  }
+#pragma unroll
+  for (int pl = 0; pl < 3; ++pl) out[pl] = __builtin_bit_cast(bf16x8_t, v[pl]);
+}
+// acc += a . b over the 16 k of one step, smallest terms first
+__device__ __forceinline__ float16_t mfma_triple(const bf16x8_t (&a)[3], const bf16x8_t (&b)[3],
+                                                 float16_t acc) {
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[2], b[0], acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[2], acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1], b[1], acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1], b[0], acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[1], acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[0], acc, 0, 0, 0);
+  return acc;
+}
+
+// ---------------------------------------------------------------------------
 // GEMM
 // ---------------------------------------------------------------------------
 struct F32GemmArgs {
@@ -54,73 +105,162 @@ struct F32GemmArgs {
   int gelu;
 };
 
-constexpr int kF32BK = 16;
 constexpr int kF32CUs = 256;
+// Extent of a buffer descriptor: at most 4 GiB - 1 (larger operands take the skinny kernel's
+// 64-bit addresses).
+__host__ __device__ inline unsigned f32_buffer_bytes(size_t floats) {
+  return floats * 4 > 0xffffffffull ? 0xffffffffu : (unsigned)(floats * 4);
+}
+constexpr unsigned kF32Outside = 0xfffffff0u;   // an offset outside every descriptor: reads as zero
+template <int N>
+__device__ __forceinline__ void f32_wait_vmcnt() {
+  static_assert(N >= 0 && N < 64, "vmcnt range");
+  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0F70);
+}
 
-// WGM x WGN waves, each a (BM/WGM) x (BN/WGN) block of 32x32 MFMA tiles.
-// LDS: A tile k-major [16][BM+4] (the gather / transposition happens in the store),
-// W tile [16][BN+32]; both strides make the operand reads of one wave conflict free.
-template <int BM, int BN, int WGM, int WGN>
-__global__ __launch_bounds__(64 * WGM *WGN) void f32_gemm_kernel(F32GemmArgs p) {
-  constexpr int THREADS = 64 * WGM * WGN;
-  constexpr int SA = BM + 4, SW = BN + 32;
-  constexpr int WM = BM / WGM, WN = BN / WGN, MT = WM / 32, NT = WN / 32;
-  constexpr int AV = BM * 4 / THREADS;     // float4 of A per thread and k-tile
-  constexpr int WV = BN * 4 / THREADS;     // float4 of W per thread and k-tile
-  static_assert(MT >= 1 && NT >= 1 && AV >= 1 && WV >= 1, "tile too small for the wave grid");
-  __shared__ float sA[2][kF32BK * SA];
-  __shared__ __attribute__((aligned(16))) float sW[2][kF32BK * SW];
+// Store of one 32x32 block: accumulator element i is row 8*(i/4) + 4*half + i%4, column l32.
+__device__ __forceinline__ void f32_store_block(const F32GemmArgs &p, const float16_t &acc, int m0,
+                                                int n0, int M, int l32, int half) {
+  const int col = n0 + l32;
+  if (col >= p.N) return;
+  const float bv = p.bias ? p.bias[col] : 0.f;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int row = m0 + 8 * (i >> 2) + 4 * half + (i & 3);
+    if (row >= M) continue;
+    float v = acc[i] + bv;
+    if (p.gelu) v = gelu_tanh(v);
+    p.c[(size_t)row * p.N + col] = v;
+  }
+}
+
+// One (32 MT) x (32 NT) tile per workgroup; its NW waves take the k range in turn, 16 k ("a slice")
+// at a time, and their sums are folded through LDS at the end.  A wave shares nothing with the others
+// until then: it copies its own slices global -> LDS (direct-to-LDS loads, no registers, no
+// barrier anywhere in the loop) into a private ring of DEPTH slices, reads them back in MFMA order
+// as floats and splits them into bf16 triples one slice ahead of the products.  Every element of
+// the tile is read from LDS once and split once, which waves side by side on a shared tile would
+// do two times each.  What bounds it is the issue port: a 64x64 tile's slice is 24 MFMAs (768 clocks of
+// the matrix pipe) and 176 vector instructions of the split, and a SIMD issues them one after the
+// other (an MFMA takes about 12 clocks of the port, a vector instruction 4).  2458 rows, hidden 768,
+// before (v_mfma_f32_32x32x2_f32, tiles of 128x128 to 64x64) and now: QKV 92 -> 60 us, projection
+// 39 -> 23, FFN1 114 -> 78, FFN2 137 -> 71 us (163 TFLOP/s); 32 rows: FFN2 121 -> 25 us.  Relative
+// error against float64 at k = 3072: 9.9e-7 -> 4.3e-7.
+//
+// LDS image of a slice: A as TM rows of 16 floats, the 16-byte chunk of a row XORed with
+// (row >> 2) & 3 (16 consecutive rows read one chunk from distinct banks); W as 16 k-rows of TN
+// floats such that k-rows e and e + 8, which the two halves of a wave read together, lie on
+// distinct banks (64 columns: the upper k-rows' columns XOR 32; 32 columns: the upper k-rows
+// exchanged in pairs).
+#if defined(__HIP_DEVICE_COMPILE__)
+template <int MT, int NT, int NW, int DEPTH, bool RAGGED>
+__device__ __forceinline__ void f32_gemm_tile(const F32GemmArgs &p) {
+  constexpr int TM = 32 * MT, TN = 32 * NT;
+  constexpr int NIA = TM / 16, NIW = TN / 16, NI = NIA + NIW;   // 1 KB load instructions per slice
+  constexpr int SLICE = (TM + TN) * 16;                         // floats
+  constexpr int ACC = TM * TN;                                  // floats of a wave's sums
+  constexpr int REGION = DEPTH * SLICE > ACC ? DEPTH * SLICE : ACC;
+  static_assert(NT == 1 || NT == 2, "the W image is laid out for 32 or 64 columns");
+  extern __shared__ __attribute__((aligned(1024))) float f32_smem[];
 
   const int M = p.valid_rows ? min(*p.valid_rows, p.rows_cap) : p.rows_cap;
-  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-  if (m0 >= M) return;
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int l32 = lane & 31, half = lane >> 5;
-  const int wm = wave / WGN, wn = wave % WGN;
-
-  // global -> register staging
-  const int a_kq = tid & 3;            // which float4 of the 16 k
-  constexpr int AROWS = THREADS / 4;   // tile rows covered by one pass of the workgroup
-  const float *a_src[AV];
-#pragma unroll
-  for (int i = 0; i < AV; ++i) {
-    const int r = m0 + (tid >> 2) + i * AROWS;
-    a_src[i] = nullptr;
-    if (r < M) {
-      const size_t row = p.a_row_index ? (size_t)p.a_row_index[r] : (size_t)r;
-      a_src[i] = p.a + row * p.K + 4 * a_kq;
-    }
+  int tile_m, tile_n;
+  {
+    const int tiles_m = (M + TM - 1) / TM, tiles_n = (p.N + TN - 1) / TN;
+    const int live = tiles_m * tiles_n, per = (live + 7) >> 3;
+    const int bid = (int)blockIdx.x, L = (bid & 7) * per + (bid >> 3);
+    if (bid >= per * 8 || L >= live) return;
+    tile_panels<TM, TN>(tiles_m, tiles_n, per).locate(L, tile_m, tile_n);
   }
-  constexpr int WPR = BN / 4;            // float4 per W tile row
-  constexpr int WROWS = THREADS / WPR;   // tile rows covered by one pass of the workgroup
-  const int w_k = tid / WPR, w_n = n0 + 4 * (tid % WPR);
-  const bool w_ok = w_n < p.N;
+  const int m0 = tile_m * TM, n0 = tile_n * TN;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l32 = lane & 31, half = lane >> 5;
+  float *ring = f32_smem + wave * REGION;
 
-  float4_t ra[AV], rw[WV];
-  auto fetch = [&](int k0) {
+  const int nk = (p.K + 15) >> 4;
+  const int mine = (nk - wave + NW - 1) / NW;   // slices wave, wave + NW, ...
+  const auto rs_a = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float *>(p.a_row_index ? p.a : p.a + (size_t)m0 * p.K), 0,
+      (int)f32_buffer_bytes(((size_t)p.rows_cap - (p.a_row_index ? 0 : m0)) * p.K), 0x00020000);
+  const auto rs_w = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float *>(p.w), 0, (int)f32_buffer_bytes((size_t)p.K * p.N), 0x00020000);
+  // byte offsets of this lane's pieces at k = 0.  Rows past M repeat the last live row, columns
+  // past N lie outside the descriptor (they read as zero); neither is stored.
+  unsigned aoff[NIA], woff[NIW];
 #pragma unroll
-    for (int i = 0; i < AV; ++i) {
-      ra[i] = float4_t{0.f, 0.f, 0.f, 0.f};
-      if (a_src[i] && k0 + 4 * a_kq < p.K) ra[i] = *(const float4_t *)(a_src[i] + k0);
+  for (int i = 0; i < NIA; ++i) {
+    const int row = i * 16 + (lane >> 2), chunk = (lane & 3) ^ ((row >> 2) & 3);
+    const int r = min(m0 + row, M - 1);
+    const unsigned src = p.a_row_index ? (unsigned)p.a_row_index[r] : (unsigned)(r - m0);
+    aoff[i] = (src * (unsigned)p.K + 4 * chunk) * 4u;
+  }
+#pragma unroll
+  for (int i = 0; i < NIW; ++i) {
+    constexpr int CPR = TN / 4;   // 16-byte chunks per k-row
+    const int at = i * 64 + lane, pos = at / CPR, c = at % CPR;
+    const int k = NT == 1 ? pos ^ ((pos >> 3) & 1) : pos;
+    const int n = 4 * (NT == 2 ? c ^ (8 * ((pos >> 3) & 1)) : c);
+    woff[i] = n0 + n < p.N ? ((unsigned)k * p.N + n0 + n) * 4u : kF32Outside;
+  }
+  // The loads of slice i of this wave.  Past the wave's last slice every offset lies outside: such
+  // loads fetch nothing, read as zero and keep the count of loads in flight the same in every step.
+  auto issue = [&](int i) {
+    const int k0 = (wave + i * NW) * 16;
+    const unsigned dead = i < mine ? 0u : kF32Outside;
+    float *dst = ring + (i % DEPTH) * SLICE;
+    const int a_k = k0 * 4, w_k = (int)((unsigned)k0 * p.N * 4u);
+#pragma unroll
+    for (int j = 0; j < NIA; ++j) {
+      const int row = j * 16 + (lane >> 2), k = k0 + 4 * ((lane & 3) ^ ((row >> 2) & 3));
+      // (of a last slice that reaches past k, only what lies before k is fetched)
+      const unsigned off = RAGGED && k >= p.K ? kF32Outside : aoff[j] | dead;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          rs_a, (__attribute__((address_space(3))) void *)(dst + j * 256), 16, (int)off, a_k, 0, 0);
     }
 #pragma unroll
-    for (int i = 0; i < WV; ++i) {
-      const int k = k0 + w_k + i * WROWS;
-      rw[i] = float4_t{0.f, 0.f, 0.f, 0.f};
-      if (w_ok && k < p.K) rw[i] = *(const float4_t *)(p.w + (size_t)k * p.N + w_n);
+    for (int j = 0; j < NIW; ++j) {
+      const int pos = (j * 64 + lane) / (TN / 4), k = k0 + (NT == 1 ? pos ^ ((pos >> 3) & 1) : pos);
+      const unsigned off = RAGGED && k >= p.K ? kF32Outside : woff[j] | dead;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          rs_w, (__attribute__((address_space(3))) void *)(dst + (NIA + j) * 256), 16, (int)off, w_k,
+          0, 0);
     }
   };
-  auto stash = [&](int buf) {
+  float4_t xa[MT][2];
+  float xw[NT][8];
+  auto read_slice = [&](int i) {
+    const float *src = ring + (i % DEPTH) * SLICE;
 #pragma unroll
-    for (int i = 0; i < AV; ++i) {
-      float *d = &sA[buf][(4 * a_kq) * SA + (tid >> 2) + i * AROWS];
+    for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) d[j * SA] = ra[i][j];
+      for (int j = 0; j < 2; ++j) {
+        const int row = mt * 32 + l32;
+        xa[mt][j] = *(const float4_t *)(src + row * 16 + 4 * ((2 * half + j) ^ ((row >> 2) & 3)));
+      }
+    const float *w = src + TM * 16;
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        if (NT == 2)
+          xw[nt][e] = w[(8 * half + e) * TN + ((nt * 32 + l32) ^ (32 * half))];
+        else
+          xw[nt][e] = w[((8 * half + e) ^ half) * TN + l32];
+      }
+  };
+  struct Operands {
+    bf16x8_t a[MT][3], w[NT][3];
+  };
+  auto split = [&](Operands &o) {
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      const float x[8] = {xa[mt][0][0], xa[mt][0][1], xa[mt][0][2], xa[mt][0][3],
+                          xa[mt][1][0], xa[mt][1][1], xa[mt][1][2], xa[mt][1][3]};
+      split_bf16x8(o.a[mt], x);
     }
 #pragma unroll
-    for (int i = 0; i < WV; ++i)
-      *(float4_t *)&sW[buf][(w_k + i * WROWS) * SW + 4 * (tid % WPR)] = rw[i];
+    for (int nt = 0; nt < NT; ++nt) split_bf16x8(o.w[nt], xw[nt]);
   };
 
   float16_t acc[MT][NT];
@@ -131,57 +271,163 @@ __global__ __launch_bounds__(64 * WGM *WGN) void f32_gemm_kernel(F32GemmArgs p) 
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[mt][nt][i] = 0.f;
 
-  const int nk = (p.K + kF32BK - 1) / kF32BK;
-  fetch(0);
-  stash(0);
-  __syncthreads();
-  int cur = 0;
-  for (int kt = 0; kt < nk; ++kt) {
-    if (kt + 1 < nk) fetch((kt + 1) * kF32BK);
-    const float *a_base = &sA[cur][half * SA + wm * WM + l32];
-    const float *w_base = &sW[cur][half * SW + wn * WN + l32];
-    // all operand fetches of the k-tile first, the MFMA chain after them: the fence keeps
-    // the compiler from sinking each ds_read next to its MFMA (which exposes the LDS
-    // latency once per MFMA pair instead of once per k-tile)
-    float af[kF32BK / 2][MT], bf[kF32BK / 2][NT];
-#pragma unroll
-    for (int kk = 0; kk < kF32BK / 2; ++kk) {
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) af[kk][mt] = a_base[2 * kk * SA + mt * 32];
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) bf[kk][nt] = w_base[2 * kk * SW + nt * 32];
-    }
+  // takes slice i from the ring (its loads are the oldest of DEPTH slices in flight) and sends
+  // the loads of slice i + DEPTH after it
+  auto take = [&](int i) {
+    f32_wait_vmcnt<(DEPTH - 1) * NI>();
     asm volatile("" ::: "memory");
+    read_slice(i);
+  };
+  auto refill = [&](int i) {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): the slot has been read
+    issue(i + DEPTH);
+  };
+  auto multiply = [&](const Operands &o) {
 #pragma unroll
-    for (int kk = 0; kk < kF32BK / 2; ++kk)
+    for (int t = 0; t < 6; ++t) {
+      constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pw[6] = {0, 2, 1, 0, 1, 0};   // smallest terms first
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt)
-          acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[kk][mt], bf[kk][nt], acc[mt][nt],
-                                                             0, 0, 0);
-    if (kt + 1 < nk) stash(cur ^ 1);
-    __syncthreads();
-    cur ^= 1;
+          acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(o.a[mt][pa[t]], o.w[nt][pw[t]],
+                                                                acc[mt][nt], 0, 0, 0);
+    }
+  };
+  if (mine > 0) {
+#pragma unroll
+    for (int i = 0; i < DEPTH; ++i) issue(i);
+    Operands o[2];
+    take(0);
+    split(o[0]);
+    refill(0);
+    // slice i is multiplied while slice i + 1 is read and split: one basic block, in which the
+    // vector instructions of the split are dealt out between the matrix instructions
+    auto step = [&](int i, const Operands &now, Operands &next) {
+      take(i + 1);
+      multiply(now);
+      split(next);
+      constexpr int kMfma = 6 * MT * NT, kSplit = (MT + NT) * 44;   // 44 vector instructions per 8 elements
+      __builtin_amdgcn_sched_group_barrier(0x100, 2 * MT + 8 * NT, 0);   // the LDS reads first
+#pragma unroll
+      for (int t = 0; t < kMfma; ++t) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, (kSplit + kMfma - 1) / kMfma, 0);
+      }
+      refill(i + 1);
+    };
+    for (int i = 0; i < mine; i += 2) {   // (an odd last slice is followed by an empty one)
+      step(i, o[0], o[1]);
+      step(i + 1, o[1], o[0]);
+    }
+    f32_wait_vmcnt<0>();   // the ring is about to be reused
   }
 
-  // accumulator element i of a 32x32 tile: row 8*(i/4) + 4*half + i%4, column l32
+  // fold: every wave leaves its sums in its own region (columns XOR 32 in rows with bit 2 set: the
+  // halves of a wave write distinct banks), then takes TM / NW rows of the tile over all regions
+  constexpr int XR = NT == 2 ? 32 : 0;
 #pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    const int col = n0 + wn * WN + nt * 32 + l32;
-    if (col >= p.N) continue;
-    const float bv = p.bias ? p.bias[col] : 0.f;
+  for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
+    for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
-        const int row = m0 + wm * WM + mt * 32 + 8 * (i >> 2) + 4 * half + (i & 3);
-        if (row >= M) continue;
-        float v = acc[mt][nt][i] + bv;
-        if (p.gelu) v = gelu_tanh(v);
-        p.c[(size_t)row * p.N + col] = v;
+        const int row = mt * 32 + 8 * (i >> 2) + 4 * half + (i & 3);
+        ring[row * TN + ((nt * 32 + l32) ^ (XR * half))] = acc[mt][nt][i];
       }
+  __syncthreads();
+  constexpr int LPR = TN / 4;            // lanes per row, four columns each
+  constexpr int RPP = 64 / LPR;          // rows per pass of a wave
+#pragma unroll
+  for (int r0 = 0; r0 < TM; r0 += RPP * NW) {
+    const int row = r0 + wave * RPP + lane / LPR, c = 4 * (lane % LPR);
+    if (TM % (RPP * NW) != 0 && row >= TM) continue;
+    const float *src = f32_smem + row * TN + (c ^ (XR * ((row >> 2) & 1)));
+    float4_t v = *(const float4_t *)src;
+#pragma unroll
+    for (int w = 1; w < NW; ++w) v += *(const float4_t *)(src + w * REGION);
+    const int m = m0 + row, n = n0 + c;
+    if (m >= M || n >= p.N) continue;
+    if (p.bias) v += float4_t{p.bias[n], p.bias[n + 1], p.bias[n + 2], p.bias[n + 3]};
+    if (p.gelu) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = gelu_tanh(v[e]);
+    }
+    *(float4_t *)(p.c + (size_t)m * p.N + n) = v;
   }
+}
+#endif
+
+template <int MT, int NT, int NW, int DEPTH, bool RAGGED>
+__global__ __launch_bounds__(64 * NW) void f32_gemm_kernel(F32GemmArgs p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  f32_gemm_tile<MT, NT, NW, DEPTH, RAGGED>(p);
+#endif
+}
+
+// Few rows: one 32x32 tile per workgroup, the k range dealt to its NW waves in steps of 16 and
+// folded through LDS at the end.  No LDS and no barrier in the loop: a wave takes its operands from
+// memory in MFMA order (A: 8 consecutive k of a row per lane, W: one column per lane), DEPTH steps
+// ahead.
+template <int NW>
+__global__ __launch_bounds__(64 * NW) void f32_gemm_skinny_kernel(F32GemmArgs p) {
+  constexpr int DEPTH = 4;
+  __shared__ float part[NW - 1][16][64];
+  const int M = p.valid_rows ? min(*p.valid_rows, p.rows_cap) : p.rows_cap;
+  const int m0 = blockIdx.y * 32, n0 = blockIdx.x * 32;
+  if (m0 >= M) return;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int l32 = lane & 31, half = lane >> 5;
+  const int r = min(m0 + l32, M - 1), n = min(n0 + l32, p.N - 1);
+  const float *a_src = p.a + (p.a_row_index ? (size_t)p.a_row_index[r] : (size_t)r) * p.K;
+  const float *w_src = p.w + n;
+  const int nk = (p.K + 15) / 16;
+
+  float4_t ra[DEPTH][2];
+  float rw[DEPTH][8];
+  auto fetch = [&](int kt, int s) {
+    const int k = 16 * kt + 8 * half;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      ra[s][j] = float4_t{0.f, 0.f, 0.f, 0.f};
+      if (k + 4 * j < p.K) ra[s][j] = *(const float4_t *)(a_src + k + 4 * j);
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) rw[s][e] = k + e < p.K ? w_src[(size_t)(k + e) * p.N] : 0.f;
+  };
+  float16_t acc;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+#pragma unroll
+  for (int s = 0; s < DEPTH - 1; ++s)
+    if (wave + s * NW < nk) fetch(wave + s * NW, s);
+  for (int kt = wave; kt < nk; kt += DEPTH * NW) {
+#pragma unroll
+    for (int s = 0; s < DEPTH; ++s) {
+      const int at = kt + s * NW;
+      if (at < nk) {
+        if (at + (DEPTH - 1) * NW < nk) fetch(at + (DEPTH - 1) * NW, (s + DEPTH - 1) % DEPTH);
+        bf16x8_t a[3], b[3];
+        const float xa[8] = {ra[s][0][0], ra[s][0][1], ra[s][0][2], ra[s][0][3],
+                             ra[s][1][0], ra[s][1][1], ra[s][1][2], ra[s][1][3]};
+        split_bf16x8(a, xa);
+        split_bf16x8(b, rw[s]);
+        acc = mfma_triple(a, b, acc);
+      }
+    }
+  }
+  if (wave > 0) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) part[wave - 1][i][lane] = acc[i];
+  }
+  __syncthreads();
+  if (wave > 0) return;
+#pragma unroll
+  for (int w = 0; w < NW - 1; ++w)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[i] += part[w][i][lane];
+  f32_store_block(p, acc, m0, n0, M, l32, half);
 }
 
 // ---------------------------------------------------------------------------
@@ -539,6 +785,25 @@ int launch_f32_ln(const void *src, const void *residual, const void *bias, const
   return BT_OK;
 }
 
+template <int MT, int NT, int NW, int DEPTH, bool RAGGED>
+static int launch_f32_gemm_as(const F32GemmArgs &p, hipStream_t s) {
+  constexpr int TM = 32 * MT, TN = 32 * NT, SLICE = (TM + TN) * 16;
+  constexpr size_t smem = (size_t)NW * (DEPTH * SLICE > TM * TN ? DEPTH * SLICE : TM * TN) * sizeof(float);
+  static_assert(smem <= 160 * 1024, "LDS budget");
+  static std::atomic<bool> configured[kMaxDevices];
+  const int rc = allow_dynamic_lds(f32_gemm_kernel<MT, NT, NW, DEPTH, RAGGED>, smem, configured,
+                                   "hipFuncSetAttribute(f32_gemm_kernel)");
+  if (rc != BT_OK) return rc;
+  const long long tiles = (long long)((p.rows_cap + TM - 1) / TM) * ((p.N + TN - 1) / TN);
+  f32_gemm_kernel<MT, NT, NW, DEPTH, RAGGED><<<(unsigned)((tiles + 7) / 8 * 8), 64 * NW, smem, s>>>(p);
+  return BT_OK;
+}
+template <int MT, int NT, int NW, int DEPTH>
+static int launch_f32_gemm(const F32GemmArgs &p, hipStream_t s) {
+  return p.K % 16 ? launch_f32_gemm_as<MT, NT, NW, DEPTH, true>(p, s)
+                  : launch_f32_gemm_as<MT, NT, NW, DEPTH, false>(p, s);
+}
+
 template <typename T>
 static int launch_generic_attention(const char *who, const void *qkv, void *out,
                                     const int *batch_idx, const int *seq_order,
@@ -604,37 +869,49 @@ extern "C" int bt_gemm_f32(const void *a, const int *a_row_index, const void *w,
   if (rows_cap == 0) return BT_OK;
   F32GemmArgs p{(const float *)a, (const float *)w, (const float *)bias, (float *)c, valid_rows,
                 a_row_index, rows_cap, n, k, gelu ? 1 : 0};
-  // Tile table: 0: 128x128, 8 waves | 1: 128x64, 4 waves | 2: 64x64, 4 waves.
-  // Choice by a two-term model per k-tile of 16: a workgroup alone on its CU needs
-  // `alone` us (latency bound), a CU shared by b workgroups needs b * `shared` us (MFMA
-  // bound); b = ceil(workgroups / CUs).  Constants measured on MI355X.
-  struct Cand { int id, bm, bn; float alone, shared; };
-  static const Cand cands[3] = {{0, 128, 128, 1.20f, 1.15f}, {1, 128, 64, 0.76f, 0.60f},
-                                {2, 64, 64, 0.49f, 0.32f}};
+  // Tile table: 0: 64x64 | 1: 64x32 | 2: 32x32 (four waves over k each) | 3: the skinny kernel.
+  // A tile takes `fixed` us plus, per turn of its four waves over k, `alone` us if it has the CU to
+  // itself and else its share of a busy CU, `shared` us.  Measured over the eight products of
+  // hidden 768 at 32..4800 rows on MI355X, the model picks the fastest tile in all of them:
+  // 32x32 while the launch leaves CUs idle, 64x64 once the split of the operands has to be
+  // amortised.
+  struct Cand { int id, bm, bn; float fixed, alone, shared; };
+  static const Cand cands[3] = {{0, 64, 64, 5.0f, 0.54f, 0.77f}, {1, 64, 32, 4.5f, 0.45f, 0.54f},
+                                {2, 32, 32, 4.0f, 0.40f, 0.325f}};
   int tile = option_f32_gemm_tile();
   if (tile < 0) {
     // the row count that matters is the live one; the hint is the caller's estimate of it
     const int rows = (valid_rows && rows_hint > 0 && rows_hint < rows_cap) ? rows_hint : rows_cap;
+    const float turns = (float)((k + 63) / 64);
     float best = 0.f;
     for (const Cand &cd : cands) {
       const long long wgs = (long long)((rows + cd.bm - 1) / cd.bm) * ((n + cd.bn - 1) / cd.bn);
-      const float b = (float)((wgs + kF32CUs - 1) / kF32CUs);
-      const float cost = fmaxf(cd.alone, b * cd.shared);
+      const float load = (float)wgs / (float)kF32CUs;
+      const float cost = cd.fixed + turns * fmaxf(cd.alone, load * cd.shared);
       if (tile < 0 || cost < best) {
         best = cost;
         tile = cd.id;
       }
     }
   }
-  const int bm = cands[tile].bm, bn = cands[tile].bn;
-  dim3 grid((n + bn - 1) / bn, (rows_cap + bm - 1) / bm);
-  BT_REQUIRE(grid.y <= 65535, BT_ERR_UNSUPPORTED, "bt_gemm_f32: too many rows");
+  // the tiled kernels address gathered rows and the weight with 32-bit byte offsets
+  if ((a_row_index && (long long)rows_cap * k * 4 > 0xffff0000ll) || (long long)n * k * 4 > 0xffff0000ll ||
+      (long long)k * 256 > 0xffff0000ll)
+    tile = 3;
   hipStream_t s = as_stream(stream);
-  switch (tile) {
-    case 0: f32_gemm_kernel<128, 128, 4, 2><<<grid, 512, 0, s>>>(p); break;
-    case 1: f32_gemm_kernel<128, 64, 2, 2><<<grid, 256, 0, s>>>(p); break;
-    default: f32_gemm_kernel<64, 64, 2, 2><<<grid, 256, 0, s>>>(p); break;
+  int rc = BT_OK;
+  if (tile == 0) {
+    rc = launch_f32_gemm<2, 2, 4, 2>(p, s);
+  } else if (tile == 1) {
+    rc = launch_f32_gemm<2, 1, 4, 3>(p, s);
+  } else if (tile == 2) {
+    rc = launch_f32_gemm<1, 1, 4, 4>(p, s);
+  } else {
+    const dim3 grid((n + 31) / 32, (rows_cap + 31) / 32);
+    BT_REQUIRE(grid.y <= 65535, BT_ERR_UNSUPPORTED, "bt_gemm_f32: too many rows");
+    f32_gemm_skinny_kernel<8><<<grid, 512, 0, s>>>(p);
   }
+  if (rc != BT_OK) return rc;
   BT_CHECK_LAUNCH("bt_gemm_f32");
   return BT_OK;
 }

@@ -409,8 +409,8 @@ extern "C" int bt_set_option(const char *name, int value) {
                "bt_set_option: attention_qb=%d must be -1, 1 or 2", value);
     g_attention_qb.store(value);
   } else if (!strcmp(name, "f32_gemm_tile")) {
-    BT_REQUIRE(value >= -1 && value <= 2, BT_ERR_INVALID_ARGUMENT,
-               "bt_set_option: f32_gemm_tile=%d outside [-1, 2]", value);
+    BT_REQUIRE(value >= -1 && value <= 3, BT_ERR_INVALID_ARGUMENT,
+               "bt_set_option: f32_gemm_tile=%d outside [-1, 3]", value);
     g_f32_gemm_tile.store(value);
   } else if (!strcmp(name, "attention_short_limit")) {
     BT_REQUIRE(value >= 0 && value <= 512, BT_ERR_INVALID_ARGUMENT,

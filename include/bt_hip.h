@@ -79,8 +79,8 @@ const char *bt_last_error_string(void);
  *   "prefetch"      1 (default) | 0: honour / ignore the prefetch hint of the attention entries
  *   "prefetch_min_grid"  512 (default): attention launches of fewer workgroups ignore the hint
  *                   (there the warm-up costs more than it returns); 1 = every launch honours it
- *   "f32_gemm_tile" -1 heuristic | 0: 128x128 tile, 8 waves | 1: 128x64, 4 waves | 2: 64x64, 4 waves
- *                   (bt_gemm_f32 only)
+ *   "f32_gemm_tile" -1 heuristic | 0: 64x64 tile | 1: 64x32 | 2: 32x32 (four waves over k each) | 3: 32x32,
+ *                   eight waves over k, 64-bit addresses (bt_gemm_f32 only)
  *   "attention_short_limit"  0 (default) .. 512: the host library sends sequences up to this
  *                   length to bt_attention_short when use_fused_attention is set; 0 = always
  *                   the streaming kernel, which measures faster at every length
@@ -439,9 +439,10 @@ int bt_splitk_layernorm(const void *partials, int splits, const void *residual,
 /*
  * ---- OperationType::FP32 ------------------------------------------------------
  * The float flavour of the layer: every tensor (activations, weights, biases, gamma,
- * beta, mask, attention bias) is float, products run on the fp32 MFMA with fp32
- * operands and accumulators.  Weights are read as the caller stores them ([K, N]
- * row-major): there is no pre-pack.
+ * beta, mask, attention bias) is float, and so are the accumulators of the products.  Weights are
+ * read as the caller stores them ([K, N] row-major): there is no pre-pack.  Inside the products a float is the exact sum of three bfloat16
+ * (24 significand bits) and the matrix cores multiply those, float accumulators: the results are
+ * at least as close to the exact product as v_mfma_f32_32x32x2_f32 brings them.
  *
  * bt_gemm_f32: c[M, n] = a[M, k] . w[k, n] (+ bias[n]) (then tanh-GELU when gelu != 0,
  * which needs a bias).  a_row_index (nullable, needs valid_rows): row r of A is

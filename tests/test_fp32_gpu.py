@@ -74,6 +74,31 @@ def test_gemm_f32_detects_transposed_or_shifted_operands(device):
     assert np.array_equal(g, np.roll(a, 5, axis=1))
 
 
+@pytest.mark.parametrize("tile", [0, 1, 2, 3])
+@pytest.mark.parametrize("rows,M,N,K", [(1, 1, 4, 4), (65, 33, 68, 20), (64, 64, 64, 64), (130, 97, 100, 1036),
+                                        (33, 32, 32, 16)])
+def test_gemm_f32_every_tile_at_its_edges(device, tile, rows, M, N, K):
+    """Each tile with remainders in rows, columns and k (fewer k than waves, a cut last slice),
+    gathered rows and the epilogue: as close to the exact product as a float accumulator gets."""
+    rs = np.random.RandomState(rows * 7 + K)
+    a = rs.standard_normal((rows, K)).astype(np.float32)
+    w = (rs.standard_normal((K, N)) * 0.2).astype(np.float32)
+    bias = rs.standard_normal(N).astype(np.float32)
+    index = np.concatenate([rs.permutation(rows)[:M], np.full(rows - M, 1 << 30)]).astype(np.int32)
+    exp = O.gemm(a[index[:M]].astype(np.float64), w.astype(np.float64), bias.astype(np.float64))
+    bound = 2.0 ** -24 * (2 + math.sqrt(K)) * (np.abs(a[index[:M]]).astype(np.float64) @ np.abs(w) + np.abs(bias))
+    ops.set_option("f32_gemm_tile", tile)
+    try:
+        out = torch.full((rows, N), 7.0, dtype=torch.float32, device=device)
+        g = ops.gemm_f32(_dev(a, device), _dev(w, device), _dev(bias, device),
+                         valid_rows=torch.tensor([M], dtype=torch.int32, device=device),
+                         a_row_index=_dev(index, device), rows_cap=rows, out=out).cpu().numpy()
+    finally:
+        ops.set_option("f32_gemm_tile", -1)
+    assert np.all(np.abs(g[:M] - exp) <= bound), (np.abs(g[:M] - exp) / bound).max()
+    assert np.all(g[M:] == 7.0)
+
+
 def test_gemm_f32_bias_gelu_and_gather(device):
     _say("gemm_f32 gelu + gather")
     rs = np.random.RandomState(11)
