@@ -389,12 +389,21 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &p) {
   // XCD-aware tile order over the live tiles
   int tile_m, tile_n;
   {
-    const int live = ((M + BM - 1) / BM) * p.tiles_n;
+    const int tiles_m = (M + BM - 1) / BM;
+    const int live = tiles_m * p.tiles_n;
     const int per = (live + 7) >> 3;
     const int L = (bid & 7) * per + (bid >> 3);
     if (bid >= per * 8 || L >= live) return;
-    tile_m = L / p.tiles_n;
-    tile_n = L - tile_m * p.tiles_n;
+    if (BM == 32 && tiles_m > 1) {
+      // A few hundred rows: the launch is as long as it takes to fetch the weight, and in row-major
+      // order every XCD fetches all of it (256 rows, QKV at hidden 768: 28 MB in all against
+      // 7 MB in panels; 12 layers at batch 1 x 256: -8 %).  With the larger tiles the panels gain
+      // nothing and their index arithmetic costs up to 1 %.
+      tile_panels<BM, BN>(tiles_m, p.tiles_n, per).locate(L, tile_m, tile_n);
+    } else {
+      tile_m = L / p.tiles_n;
+      tile_n = L - tile_m * p.tiles_n;
+    }
   }
   const int m0 = tile_m * BM, n0 = tile_n * BN;
   // a split-k launch gives grid row y the k range [y, y+1) * K / gridDim.y
