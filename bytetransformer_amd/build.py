@@ -22,7 +22,8 @@ INC = os.path.join(ROOT, "include")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 HIPCC = os.path.join(ROCM, "bin", "hipcc")
 
-KERNEL_SOURCES = ["padding.hip", "layernorm.hip", "gemm.hip", "attention.hip", "fp32_path.hip"]
+KERNEL_SOURCES = ["padding.hip", "layernorm.hip", "gemm.hip", "attention.hip",
+                  "attention_generic.hip", "fp32_path.hip"]
 HOST_SOURCES = ["attention.cc", "bert_transformer.cc", "bert_encoder.cc", "c_api.cc"]
 HOST_DEVICE_SOURCE = "layer_static_scratch.hip"
 TH_OP_SOURCES = ["ths_op_f.cc", "ths_op.cc"]
@@ -37,7 +38,8 @@ HIP_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
              "-Wno-unused-command-line-argument"]
 # The attention kernels' inputs are finite by contract (masking is by index, never
 # by NaN/inf), so max() needs no NaN quieting there: plain v_max_f32 / v_max3_f32.
-PER_FILE_FLAGS = {"attention.hip": ["-fno-honor-nans", "-mno-amdgpu-ieee"]}
+PER_FILE_FLAGS = {f: ["-fno-honor-nans", "-mno-amdgpu-ieee"]
+                  for f in ("attention.hip", "attention_generic.hip")}
 HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-Wall"]
 
 

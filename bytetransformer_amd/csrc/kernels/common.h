@@ -91,6 +91,26 @@ inline bool aligned16(std::initializer_list<const void *> ptrs) {
   return true;
 }
 
+// Arguments of the token-major attention entries (float, and fp16 of any head size).
+inline int check_generic_attention(const char *who, const void *qkv, const void *out, const int *batch_idx,
+                                   const void *atten_mask, const void *attention_bias, int batch_size,
+                                   int seq_len, int rows_cap, int head_num, int size_per_head,
+                                   int padded_rows) {
+  BT_REQUIRE(qkv && out && batch_idx, BT_ERR_INVALID_ARGUMENT, "%s: null pointer argument", who);
+  BT_REQUIRE(aligned16({qkv, out, atten_mask, attention_bias}), BT_ERR_INVALID_ARGUMENT,
+             "%s: tensor pointers must be 16-byte aligned", who);
+  BT_REQUIRE(batch_size > 0 && seq_len > 0 && head_num > 0 && rows_cap >= 0,
+             BT_ERR_INVALID_ARGUMENT, "%s: sizes must be positive", who);
+  BT_REQUIRE(size_per_head > 0 && size_per_head % 8 == 0 && size_per_head <= 128,
+             BT_ERR_UNSUPPORTED, "%s: size_per_head %d (supported: multiples of 8 up to 128)",
+             who, size_per_head);
+  BT_REQUIRE(batch_size <= 65535 && head_num <= 65535, BT_ERR_UNSUPPORTED,
+             "%s: batch_size / head_num exceed the grid limit", who);
+  BT_REQUIRE(!padded_rows || (long long)batch_size * seq_len <= rows_cap, BT_ERR_INVALID_ARGUMENT,
+             "%s: padded rows need rows_cap >= batch_size * seq_len", who);
+  return BT_OK;
+}
+
 // ---- wave64 reductions ----------------------------------------------------
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
