@@ -25,7 +25,7 @@
 // (attention_fused.cu:359, attention_fused_long.cu:254).  Tile rows past the
 // length are fetched from the last valid row (finite data, never out of
 // bounds) and their probabilities are forced to zero.
-#include "common.h"
+#include "attention_common.h"
 
 #include <type_traits>
 
@@ -33,11 +33,6 @@ namespace bt {
 
 constexpr int kAttThreads = 256;
 constexpr int kHeadDim = 64;
-constexpr float kNegBig = -1.0e30f;
-constexpr float kLog2e = 1.4426950408889634f;
-
-typedef float float2_t __attribute__((ext_vector_type(2)));
-
 constexpr int kPrefetchRanges = 4;
 
 struct AttArgs {
@@ -61,6 +56,7 @@ struct AttArgs {
   int xcd_map;         // 0: plain (tile, head, sequence) order, 1: XCD-aware, 2: XCD-aware and balanced over the CUs
   const int *mask_ok;  // optional int[256] from bt_mask_prefix_slots: all non-zero = the mask
                        // is the plain prefix mask of the lengths, and is then ignored
+  int every_key;       // 1: all S keys of a sequence take part, whatever its length
   const int4 *work_list;   // optional: entry w of bt_attention_worklist = what workgroup w of the
                            // balanced order works on {sequence or -1, head | tile << 16, first row, length}
 };
@@ -93,43 +89,6 @@ __device__ __forceinline__ AttItem att_item(const AttArgs &p) {
     it.exists = true;
   }
   return it;
-}
-
-__device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
-
-// Reductions over the four 16-lane rows of a wave (lanes l, l^16, l^32, l^48) with the
-// row-swap VALU instructions: after a swap of two copies of x, the pair holds x of
-// rows {0,0,2,2} / {1,1,3,3} (16-lane swap) or {0,1,0,1} / {2,3,2,3} (32-lane swap),
-// so one max / add per step folds the partner row in - no LDS round trip.  The empty
-// asm keeps the optimiser from treating the two results of a swap of equal inputs as
-// equal (it then drops the max / add).
-__device__ __forceinline__ void swap_rows16(float x, float &lo, float &hi) {
-  const unsigned u = __builtin_bit_cast(unsigned, x);
-  auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-  unsigned r0 = r[0], r1 = r[1];
-  asm volatile("" : "+v"(r0), "+v"(r1));
-  lo = __builtin_bit_cast(float, r0);
-  hi = __builtin_bit_cast(float, r1);
-}
-__device__ __forceinline__ void swap_rows32(float x, float &lo, float &hi) {
-  const unsigned u = __builtin_bit_cast(unsigned, x);
-  auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-  unsigned r0 = r[0], r1 = r[1];
-  asm volatile("" : "+v"(r0), "+v"(r1));
-  lo = __builtin_bit_cast(float, r0);
-  hi = __builtin_bit_cast(float, r1);
-}
-__device__ __forceinline__ float rows_max(float x) {
-  float a, b;
-  swap_rows16(x, a, b);
-  swap_rows32(fmaxf(a, b), a, b);
-  return fmaxf(a, b);
-}
-__device__ __forceinline__ float rows_sum(float x) {
-  float a, b;
-  swap_rows16(x, a, b);
-  swap_rows32(a + b, a, b);
-  return a + b;
 }
 
 // Cache warm-up on behalf of later kernels: the workgroups of the last quarter of the
@@ -170,16 +129,6 @@ __device__ __forceinline__ void prefetch_slice(const AttArgs &p) {
 __device__ __forceinline__ int swz_k(int row) { return (row >> 1) & 7; }
 __device__ __forceinline__ int swz_v(int row) { return ((row >> 1) & 3) << 1; }
 
-template <int N>
-__device__ __forceinline__ void att_wait_vmcnt() {
-  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0F70);
-}
-
-__device__ __forceinline__ void lds_dma16(const half_t *src, half_t *dst) {
-  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)src,
-                                   (__attribute__((address_space(3))) void *)dst, 16, 0, 0);
-}
-
 // V^T fragment for d-block db and key pair-block kk of a [keys][64] swizzled V
 // tile: 8 keys {32kk+4g+r, 32kk+16+4g+r} for d = 16db + (lane&15), g = lane>>4.
 __device__ __forceinline__ half8_t load_vt_frag(const half_t *sV, int kk, int db, int lq, int lg) {
@@ -196,78 +145,33 @@ __device__ __forceinline__ half8_t load_vt_frag(const half_t *sV, int kk, int db
   return half8_t{l4[0], l4[1], l4[2], l4[3], h4[0], h4[1], h4[2], h4[3]};
 }
 
-// The same fragment from the address of its first read (a tile's first key pair-block plus
-// the lane's own offset): the second read lies 16 rows further on.
-__device__ __forceinline__ half8_t load_vt_frag_at(const half_t *p0) {
-  const fp16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4f16(
-      (__attribute__((address_space(3))) fp16x4_t *)p0);
-  const fp16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4f16(
-      (__attribute__((address_space(3))) fp16x4_t *)(p0 + 16 * kHeadDim));
-  const half4_t l4 = __builtin_bit_cast(half4_t, lo), h4 = __builtin_bit_cast(half4_t, hi);
-  return half8_t{l4[0], l4[1], l4[2], l4[3], h4[0], h4[1], h4[2], h4[3]};
-}
-
 __device__ __forceinline__ half8_t load_k_frag(const half_t *sK, int kb, int dh, int lq, int lg) {
   const int row = 16 * kb + lq;
   return *(const half8_t *)(sK + row * kHeadDim + (((4 * dh + lg) ^ swz_k(row)) << 3));
-}
-
-// Additive mask term of four consecutive keys of one query row, in the exp2
-// domain: (mask - 1) * 10000 * log2(e)  (the reference's non-remove-padding
-// kernels, attention_fused.cu:234-237).  Keys at or past S get no term here; the
-// caller excludes them by index.
-__device__ __forceinline__ float4_t row4(const half_t *row, int key, int S, bool vec, float fill) {
-  float4_t m = {fill, fill, fill, fill};
-  if (vec && key + 3 < S) {
-    const half4_t h = *(const half4_t *)(row + key);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) m[r] = (float)h[r];
-  } else {
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      if (key + r < S) m[r] = (float)row[key + r];
-  }
-  return m;
-}
-__device__ __forceinline__ float4_t mask_bias4(const half_t *mask_row, int key, int S, bool vec) {
-  constexpr float kShift = 10000.0f * kLog2e;
-  return (row4(mask_row, key, S, vec, 1.f) - 1.0f) * kShift;
-}
-// Additive term of four consecutive keys in the exp2 domain: the mask shift (when a
-// mask row is given) plus the attention bias (softmax.h:41-46 adds it to the
-// scaled logits before the mask term).
-__device__ __forceinline__ float4_t add_terms4(const half_t *mask_row, const half_t *bias_row,
-                                               int key, int S, bool vec) {
-  float4_t t = {0.f, 0.f, 0.f, 0.f};
-  if (mask_row) t = mask_bias4(mask_row, key, S, vec);
-  if (bias_row) t += row4(bias_row, key, S, vec, 0.f) * kLog2e;
-  return t;
 }
 
 // ---------------------------------------------------------------------------
 // grouped / streaming kernel
 // ---------------------------------------------------------------------------
 constexpr int kKT = 64;                          // keys per streamed tile
-#ifndef BT_LAZY_MAX
-#define BT_LAZY_MAX 8.0f
-#endif
-constexpr float kLazyMax = BT_LAZY_MAX;          // see the running maximum in the tile loop
 constexpr int kTileHalfs = kKT * kHeadDim;       // one K or V tile
 
-// QB 16-query blocks per wave; workgroup covers 4*QB*16 queries.  ADD: a mask tensor and / or an
+// QB 16-query blocks per wave; workgroup covers 4*QB*16 queries.  KIND: a mask tensor and / or an
 // attention bias contribute additive terms to the logits.
 // KS = 2 (key split): eight waves; waves 4-7 work on the same queries as waves 0-3 but on
 // the other 64-key half of every 128-key ring slot, with their own running maximum, sum
 // and output, and the two halves are merged through LDS at the end.  The dependency chain
 // of a query tile - what bounds a launch of a few workgroups per CU, where the longest
 // sequence's workgroups finish last - is half as long, and twice the waves hide it.
-template <int QB, bool ADD, int STAGES, int KS = 1>
-__global__ __launch_bounds__(kAttThreads * KS, KS == 1 ? 2 : 4) void attention_grouped_kernel(AttArgs p) {
+template <int QB, int KIND, int STAGES, int KS = 1>
+__global__ __launch_bounds__(kAttThreads * KS, KS == 1 || KIND ? 2 : 4) void attention_grouped_kernel(AttArgs p) {
+  constexpr bool ADD = KIND != kAddNone;
   constexpr int BQ = 4 * QB * 16;
   constexpr int AHEAD = STAGES - 1;     // tiles in flight beyond the one being consumed
   constexpr int kSlotKeys = kKT * KS;   // keys per ring slot
   constexpr int kSlotHalfs = KS * 2 * kTileHalfs;
-  static_assert(STAGES == 2 || STAGES == 3, "ring depth");
+  static_assert(STAGES >= 2 && STAGES <= 4, "ring depth");
+  static_assert(!ADD || STAGES % 2 == 0, "the additive terms alternate between two register sets");
   static_assert(KS == 1 || KS == 2, "key split");
   __shared__ __attribute__((aligned(1024))) half_t ring[STAGES * kSlotHalfs];
 
@@ -305,14 +209,14 @@ __global__ __launch_bounds__(kAttThreads * KS, KS == 1 ? 2 : 4) void attention_g
   }
   // A mask tensor that the device-side check found to be the plain prefix mask adds 0 to
   // the logits of the sequence's keys and removes the others: the lengths say the same.
-  const half_t *mask = ADD ? p.mask : nullptr;
-  if (ADD && mask && p.mask_ok) {
+  const half_t *mask = KIND & kAddMask ? p.mask : nullptr;
+  if ((KIND & kAddMask) && p.mask_ok) {
     const int l = threadIdx.x & 63;
     const int ok = p.mask_ok[l] & p.mask_ok[l + 64] & p.mask_ok[l + 128] & p.mask_ok[l + 192];
     if (__builtin_amdgcn_ballot_w64(ok == 0) == 0) mask = nullptr;
   }
   // with a mask tensor every one of the S key rows takes part
-  const int klen = mask ? p.S : seq_len;
+  const int klen = mask || p.every_key ? p.S : seq_len;
   const int row_start = p.padded_rows ? b * p.S : seq_start;
   const int nq = p.padded_rows ? p.S : klen;
   const int q0 = qb_index * BQ;
@@ -351,14 +255,16 @@ __global__ __launch_bounds__(kAttThreads * KS, KS == 1 ? 2 : 4) void attention_g
   // address is one of these six lane constants plus a compile-time offset - ring stage,
   // key block - that fits the instruction's immediate field: no address arithmetic is
   // left in the loop over the key tiles (it was a quarter of its vector instructions).
-  int koff[2], voff[4];
+  int koff[2];
+  unsigned vaddr[4];   // (bytes, from the ring's start in LDS)
 #pragma unroll
   for (int dh = 0; dh < 2; ++dh) koff[dh] = lq * kHeadDim + (((4 * dh + lg) ^ swz_k(lq)) << 3);
 #pragma unroll
   for (int db = 0; db < 4; ++db) {
     const int row0 = 4 * lg + (lq >> 2);
     const int c = 2 * db + ((lq & 3) >> 1);
-    voff[db] = row0 * kHeadDim + ((c ^ swz_v(row0)) << 3) + 4 * (lq & 1);
+    vaddr[db] = lds_address(ring) +
+                2 * (row0 * kHeadDim + ((c ^ swz_v(row0)) << 3) + 4 * (lq & 1) + grp * 2 * kTileHalfs);
   }
 
   // Slot copy: 16 load instructions per 64-key tile (8 rows each; 0-7 = K, 8-15 = V),
@@ -398,34 +304,85 @@ __global__ __launch_bounds__(kAttThreads * KS, KS == 1 ? 2 : 4) void attention_g
 
   const bool wave_live = q0 + wave * QB * 16 < nq;
   const int ntiles = (klen + kSlotKeys - 1) / kSlotKeys;
-  if (ntiles > 0) issue_tile(0, 0);
-  if (AHEAD > 1 && ntiles > 1) issue_tile(1, 1);
 
   const float c = p.scale_log2e;
   // after the mask term is folded in, the logits already are in the exp2 domain
   const float cs = ADD ? 1.0f : c;
-  const bool mask_vec = (p.S & 3) == 0;
+  // The additive terms of a tile are requested one whole tile ahead, in front of that tile's K and V,
+  // into the register set that its parity names; fetched where they are used, every tile waited for
+  // memory a second time.  Batch 1 x 256 under its mask: 9.8 -> 7.6 us a launch, 6 x 250 (rows that
+  // start anywhere) 17.3 -> 10.5, 12 x 380 with a bias 31.9 -> 22.6.
+  const bool with_mask = (KIND & kAddMask) && mask;   // (the verdict may have dropped it)
+  uint2_t mask_raw[2][QB][4], bias_raw[2][QB][4];
+  auto term_row = [&](const half_t *tensor, int plane, int planes, int qb) {
+    return TermRow(tensor, (size_t)plane * p.S + min(q0 + (wave * QB + qb) * 16 + lq, p.S - 1), p.S,
+                   (size_t)planes * p.S);
+  };
+  const bool ragged_end = klen % kSlotKeys != 0;   // every tile but the last is full
+  auto fetch_terms = [&](int t, auto set_tag) {
+    constexpr int SET = decltype(set_tag)::value;
+    const int key = t * kSlotKeys + grp * kKT + lg * 4;
+    auto fetch = [&](auto inside_tag) {
+      constexpr bool INSIDE = decltype(inside_tag)::value;
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb) {
+        if (with_mask) {
+          const TermRow row = term_row(mask, b, p.B, qb);
+#pragma unroll
+          for (int kb = 0; kb < 4; ++kb) mask_raw[SET][qb][kb] = row.template fetch<INSIDE>(key + kb * 16);
+        }
+        if (KIND & kAddBias) {
+          const TermRow row = term_row(p.bias, head, p.heads, qb);
+#pragma unroll
+          for (int kb = 0; kb < 4; ++kb) bias_raw[SET][qb][kb] = row.template fetch<INSIDE>(key + kb * 16);
+        }
+      }
+    };
+    if (ragged_end && t == ntiles - 1)
+      fetch(std::false_type{});
+    else
+      fetch(std::true_type{});
+  };
+  // (two query blocks with both kinds of terms: one set of registers, requested at the top of the tile)
+  constexpr bool kTermsAhead = ADD && !(QB == 2 && KIND == kAddBoth);
+  if (kTermsAhead && ntiles > 0) fetch_terms(0, std::integral_constant<int, 0>{});
+#pragma unroll
+  for (int t = 0; t < AHEAD; ++t)
+    if (t < ntiles) issue_tile(t, t);
 
   // ST: the ring stage of tile t, a compile-time constant (the loop below is unrolled over
   // the stages)
   auto process_tile = [&](int t, auto masked_tag, auto stage_tag) {
     constexpr bool MASKED = decltype(masked_tag)::value;
     constexpr int ST = decltype(stage_tag)::value;
-    // this wave's share of tile t has landed once only tile t+1's four loads are outstanding
-    if (AHEAD > 1 && t + 1 < ntiles)
-      att_wait_vmcnt<4>();
+    // This wave's share of tile t has landed once only what was requested after it is outstanding: the
+    // four loads of each later tile and, from the second tile on, the terms of this one (four loads
+    // or more per query block).  A two-deep ring requests a tile last of all.
+    constexpr int TERMS = ADD && AHEAD > 1 ? 4 * QB : 0;
+    auto wait_tile = [&](auto terms_tag) {
+      constexpr int N = decltype(terms_tag)::value;
+      if (AHEAD > 2 && t + 2 < ntiles)
+        att_wait_vmcnt<8 + N>();
+      else if (AHEAD > 1 && t + 1 < ntiles)
+        att_wait_vmcnt<4 + N>();
+      else
+        att_wait_vmcnt<N>();
+    };
+    if (TERMS > 0 && t > 0)
+      wait_tile(std::integral_constant<int, TERMS>{});
     else
-      att_wait_vmcnt<0>();
+      wait_tile(std::integral_constant<int, 0>{});
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
+    if (kTermsAhead && t + 1 < ntiles) fetch_terms(t + 1, std::integral_constant<int, (ST + 1) & 1>{});
+    if (ADD && !kTermsAhead) fetch_terms(t, std::integral_constant<int, ST & 1>{});
     if (t + AHEAD < ntiles) issue_tile(t + AHEAD, (ST + AHEAD) % STAGES);
     // a wave whose queries all lie past the sequence, or whose half of the slot lies past
     // the last key, only copies and keeps the barriers
     const int k0 = t * kSlotKeys + grp * kKT;
     if (!wave_live || (KS > 1 && k0 >= klen)) return;
     const half_t *sK = ring + ST * kSlotHalfs + grp * 2 * kTileHalfs;
-    const half_t *sV = sK + kTileHalfs;
 
     // S^T = K . Q^T for this tile: 4 key blocks x QB query blocks
     float4_t s[4][QB];
@@ -440,19 +397,26 @@ __global__ __launch_bounds__(kAttThreads * KS, KS == 1 ? 2 : 4) void attention_g
         s[kb][qb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf1, qf[qb][1], s[kb][qb], 0, 0, 0);
       }
     }
-    if (ADD) {
+    if constexpr (ADD) {
+      auto apply = [&](auto kind_tag) {
+        constexpr int K = decltype(kind_tag)::value;
 #pragma unroll
-      for (int qb = 0; qb < QB; ++qb) {
-        const int q = min(q0 + (wave * QB + qb) * 16 + lq, p.S - 1);
-        const half_t *mrow = mask ? mask + ((size_t)b * p.S + q) * p.S : nullptr;
-        const half_t *brow = p.bias ? p.bias + ((size_t)head * p.S + q) * p.S : nullptr;
+        for (int qb = 0; qb < QB; ++qb)
 #pragma unroll
-        for (int kb = 0; kb < 4; ++kb) {
-          const float4_t bias = add_terms4(mrow, brow, k0 + kb * 16 + lg * 4, p.S, mask_vec);
-#pragma unroll
-          for (int r = 0; r < 4; ++r) s[kb][qb][r] = __builtin_fmaf(s[kb][qb][r], c, bias[r]);
-        }
-      }
+          for (int kb = 0; kb < 4; ++kb) {
+            uint2_t mv = mask_raw[ST & 1][qb][kb], bv = bias_raw[ST & 1][qb][kb];
+            if (MASKED) {
+              const int key = k0 + kb * 16 + lg * 4;
+              if (K & kAddMask) mv = term_row(mask, b, p.B, qb).in_order(mv, key);
+              if (K & kAddBias) bv = term_row(p.bias, head, p.heads, qb).in_order(bv, key);
+            }
+            s[kb][qb] = add_terms<K>(s[kb][qb], c, mv, bv);
+          }
+      };
+      if (with_mask || !(KIND & kAddMask))
+        apply(std::integral_constant<int, KIND>{});
+      else
+        apply(std::integral_constant<int, KIND & kAddBias>{});
     }
     if (MASKED) {
 #pragma unroll
@@ -463,6 +427,21 @@ __global__ __launch_bounds__(kAttThreads * KS, KS == 1 ? 2 : 4) void attention_g
 #pragma unroll
           for (int qb = 0; qb < QB; ++qb) s[kb][qb][r] = dead ? kNegBig : s[kb][qb][r];
         }
+    }
+
+    // the V^T fragments of the tile: keys 32 kk + 4 lg + .. (lo) and 16 rows further on (hi), on their
+    // way while the probabilities are computed
+    constexpr int kV = 2 * (ST * kSlotHalfs + kTileHalfs), kRow = 2 * kHeadDim;
+    uint2_t v_lo[2][4], v_hi[2][4];
+#pragma unroll
+    for (int db = 0; db < 4; ++db) {
+      v_lo[0][db] = lds_read_tr<kV>(vaddr[db]);
+      v_hi[0][db] = lds_read_tr<kV + 16 * kRow>(vaddr[db]);
+    }
+#pragma unroll
+    for (int db = 0; db < 4; ++db) {
+      v_lo[1][db] = lds_read_tr<kV + 32 * kRow>(vaddr[db]);
+      v_hi[1][db] = lds_read_tr<kV + 48 * kRow>(vaddr[db]);
     }
 
     half8_t pf[2][QB];
@@ -507,9 +486,14 @@ __global__ __launch_bounds__(kAttThreads * KS, KS == 1 ? 2 : 4) void attention_g
     // O^T += V^T . P^T ; k-slot (lg, s) <-> key 32*kk + 16*(s>>2) + 4*lg + (s&3)
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk) {
+      if (kk == 0)
+        lds_wait_tied<8>(v_lo[0], v_hi[0]);
+      else
+        lds_wait_tied<0>(v_lo[1], v_hi[1]);
 #pragma unroll
       for (int db = 0; db < 4; ++db) {
-        const half8_t vf = load_vt_frag_at(sV + kk * 32 * kHeadDim + voff[db]);
+        const half8_t vf = __builtin_bit_cast(
+            half8_t, uint4_t{v_lo[kk][db][0], v_lo[kk][db][1], v_hi[kk][db][0], v_hi[kk][db][1]});
 #pragma unroll
         for (int qb = 0; qb < QB; ++qb)
           o[db][qb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, pf[kk][qb], o[db][qb], 0, 0, 0);
@@ -519,8 +503,7 @@ __global__ __launch_bounds__(kAttThreads * KS, KS == 1 ? 2 : 4) void attention_g
         o[4][qb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, pf[kk][qb], o[4][qb], 0, 0, 0);
     }
   };
-  // every tile but the last is full: no masking code on the steady-state path
-  const bool ragged_end = klen % kSlotKeys != 0;
+  // no masking code on the steady-state path
   auto step = [&](int t, auto stage_tag) {
     if (ragged_end && t == ntiles - 1)
       process_tile(t, std::true_type{}, stage_tag);
@@ -531,8 +514,11 @@ __global__ __launch_bounds__(kAttThreads * KS, KS == 1 ? 2 : 4) void attention_g
   for (int t = 0; t < ntiles; t += STAGES) {
     step(t, std::integral_constant<int, 0>{});
     if (t + 1 < ntiles) step(t + 1, std::integral_constant<int, 1>{});
-    if constexpr (STAGES == 3) {
+    if constexpr (STAGES >= 3) {
       if (t + 2 < ntiles) step(t + 2, std::integral_constant<int, 2>{});
+    }
+    if constexpr (STAGES == 4) {
+      if (t + 3 < ntiles) step(t + 3, std::integral_constant<int, 3>{});
     }
   }
 
@@ -601,8 +587,9 @@ __global__ __launch_bounds__(kAttThreads) void attention_worklist_kernel(AttArgs
 // ---------------------------------------------------------------------------
 // short kernel: K, V resident in LDS, logits of the query tile in registers
 // ---------------------------------------------------------------------------
-template <int NKB, bool ADD>  // capacity in 16-key blocks (keys <= 16*NKB), NKB even; ADD as above
+template <int NKB, int KIND>  // capacity in 16-key blocks (keys <= 16*NKB), NKB even; KIND as above
 __global__ __launch_bounds__(kAttThreads) void attention_short_kernel(AttArgs p) {
+  constexpr bool ADD = KIND != kAddNone;
   constexpr int KEYS = NKB * 16;
   constexpr int BQ = 64;  // 4 waves x 16 queries
   extern __shared__ __attribute__((aligned(1024))) half_t att_smem[];
@@ -616,7 +603,7 @@ __global__ __launch_bounds__(kAttThreads) void attention_short_kernel(AttArgs p)
   }
   const int b = p.seq_order ? p.seq_order[item.rank] : item.rank, head = item.head;
   const int seq_start = p.batch_idx[b];
-  const int klen = ADD && p.mask ? p.S : p.batch_idx[b + 1] - seq_start;
+  const int klen = (KIND & kAddMask) || p.every_key ? p.S : p.batch_idx[b + 1] - seq_start;
   const int row_start = p.padded_rows ? b * p.S : seq_start;
   const int nq = p.padded_rows ? p.S : klen;
   const int q0 = item.qb * BQ;
@@ -681,14 +668,15 @@ __global__ __launch_bounds__(kAttThreads) void attention_short_kernel(AttArgs p)
   const float cs = ADD ? 1.0f : c;
   if (ADD) {
     const int qc = min(q, p.S - 1);
-    const half_t *mrow = p.mask ? p.mask + ((size_t)b * p.S + qc) * p.S : nullptr;
-    const half_t *brow = p.bias ? p.bias + ((size_t)head * p.S + qc) * p.S : nullptr;
-    const bool mask_vec = (p.S & 3) == 0;
+    const TermRow mrow(p.mask, (size_t)b * p.S + qc, p.S, (size_t)p.B * p.S);
+    const TermRow brow(p.bias, (size_t)head * p.S + qc, p.S, (size_t)p.heads * p.S);
 #pragma unroll
     for (int kb = 0; kb < NKB; ++kb) {
-      const float4_t bias = add_terms4(mrow, brow, kb * 16 + lg * 4, p.S, mask_vec);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) s[kb][r] = __builtin_fmaf(s[kb][r], c, bias[r]);
+      const int key = kb * 16 + lg * 4;
+      uint2_t mv = {0u, 0u}, bv = {0u, 0u};
+      if (KIND & kAddMask) mv = mrow.in_order(mrow.fetch<false>(key), key);
+      if (KIND & kAddBias) bv = brow.in_order(brow.fetch<false>(key), key);
+      s[kb] = add_terms<KIND>(s[kb], c, mv, bv);
     }
   }
   // exact softmax over the row: mask by index, max, exp, sum, normalise, round
@@ -811,22 +799,29 @@ static int check_att_args(const char *who, const void *qkv, const void *out, con
   return BT_OK;
 }
 
-template <int NKB, bool ADD>
+static int add_kind(const AttArgs &a) { return (a.mask ? kAddMask : 0) | (a.bias ? kAddBias : 0); }
+
+template <int NKB, int KIND>
 static int launch_short_impl(const AttArgs &a, hipStream_t s) {
   constexpr size_t smem = (size_t)2 * NKB * 16 * kHeadDim * sizeof(half_t);
   static_assert(smem <= 160 * 1024, "LDS budget");
   static std::atomic<bool> configured[kMaxDevices];
-  const int rc = allow_dynamic_lds(attention_short_kernel<NKB, ADD>, smem, configured,
+  const int rc = allow_dynamic_lds(attention_short_kernel<NKB, KIND>, smem, configured,
                                    "hipFuncSetAttribute(attention_short_kernel)");
   if (rc != BT_OK) return rc;
-  attention_short_kernel<NKB, ADD><<<a.nqb_grid, kAttThreads, smem, s>>>(a);
+  attention_short_kernel<NKB, KIND><<<a.nqb_grid, kAttThreads, smem, s>>>(a);
   BT_CHECK_LAUNCH("attention_short_kernel");
   return BT_OK;
 }
 
 template <int NKB>
 static int launch_short(const AttArgs &a, hipStream_t s) {
-  return a.mask || a.bias ? launch_short_impl<NKB, true>(a, s) : launch_short_impl<NKB, false>(a, s);
+  switch (add_kind(a)) {
+    case kAddNone: return launch_short_impl<NKB, kAddNone>(a, s);
+    case kAddMask: return launch_short_impl<NKB, kAddMask>(a, s);
+    case kAddBias: return launch_short_impl<NKB, kAddBias>(a, s);
+    default: return launch_short_impl<NKB, kAddBoth>(a, s);
+  }
 }
 
 }  // namespace bt
@@ -850,6 +845,7 @@ extern "C" int bt_attention_short(const void *qkv_heads, void *attention_output,
             (const half_t *)atten_mask, (const half_t *)attention_bias,
             {}, {}, batch_size, seq_len,
             rows_cap, head_num, scale * kLog2e, padded_rows};
+  a.every_key = drop_terms_of_one_key(seq_len, a.mask, a.bias);
   hipStream_t s = as_stream(stream);
   a.nqb_grid = att_grid(a, (seq_len + 63) / 64);
   rc = set_prefetch(a, a.nqb_grid, prefetch, prefetch_bytes, prefetch_count);
@@ -880,6 +876,21 @@ static GroupedPlan plan_grouped(AttArgs &a, int batch_size, int seq_len, int hea
   plan.wide = qb == 2 || (qb < 0 && blocks128 >= 1300);
   plan.grid = att_grid(a, plan.wide ? (seq_len + 127) / 128 : (seq_len + 63) / 64, true);
   return plan;
+}
+template <int KIND>
+static void launch_grouped(const AttArgs &a, bool wide, int seq_len, unsigned grid, hipStream_t s) {
+  // (the additive terms alternate between two register sets, so their kernels take an even ring)
+  constexpr int kWideStages = KIND == kAddNone ? 3 : 2;
+  // eight waves over two key halves: pays for a few long sequences that leave most CUs
+  // with one workgroup or none (batch 1 x 1024: 9.9 -> 8.7 us); with several workgroups
+  // per CU the four-wave form is faster (batch 16 x 512: 16.3 against 19.6 us)
+  const int ks = option_attention_key_split();
+  if (wide)
+    attention_grouped_kernel<2, KIND, kWideStages><<<grid, kAttThreads, 0, s>>>(a);
+  else if (ks == 1 || (ks < 0 && seq_len >= 512 && grid <= 256))
+    attention_grouped_kernel<1, KIND, 2, 2><<<grid, 2 * kAttThreads, 0, s>>>(a);
+  else
+    attention_grouped_kernel<1, KIND, 2><<<grid, kAttThreads, 0, s>>>(a);
 }
 AttListPlan att_worklist_plan(int B, int S, int heads) {
   AttListPlan out{0, 64, 0};
@@ -950,10 +961,10 @@ extern "C" int bt_attention_grouped(const void *qkv_heads, void *attention_outpu
             (const half_t *)atten_mask, (const half_t *)attention_bias,
             {}, {}, batch_size, seq_len,
             rows_cap, head_num, scale * kLog2e, padded_rows};
+  a.every_key = drop_terms_of_one_key(seq_len, a.mask, a.bias);
   a.mask_ok = a.mask ? mask_prefix_slots : nullptr;
   a.work_list = (const int4 *)work_list;   // read only when the launch uses the balanced order
   hipStream_t s = as_stream(stream);
-  const bool add = a.mask || a.bias;
   GroupedPlan plan = plan_grouped(a, batch_size, seq_len, head_num);
   if (no_offsets && a.xcd_map == 2) {   // the balanced order ranks the sequences by length
     a.xcd_map = 1;
@@ -962,26 +973,11 @@ extern "C" int bt_attention_grouped(const void *qkv_heads, void *attention_outpu
   const unsigned grid = plan.grid;
   rc = set_prefetch(a, grid, prefetch, prefetch_bytes, prefetch_count);
   if (rc) return rc;
-  if (plan.wide) {
-    if (add)
-      attention_grouped_kernel<2, true, 3><<<grid, kAttThreads, 0, s>>>(a);
-    else
-      attention_grouped_kernel<2, false, 3><<<grid, kAttThreads, 0, s>>>(a);
-  } else {
-    // eight waves over two key halves: pays for a few long sequences that leave most CUs
-    // with one workgroup or none (batch 1 x 1024: 9.9 -> 8.7 us); with several workgroups
-    // per CU the four-wave form is faster (batch 16 x 512: 16.3 against 19.6 us)
-    const int ks = option_attention_key_split();
-    if (ks == 1 || (ks < 0 && seq_len >= 512 && grid <= 256)) {
-      if (add)
-        attention_grouped_kernel<1, true, 2, 2><<<grid, 2 * kAttThreads, 0, s>>>(a);
-      else
-        attention_grouped_kernel<1, false, 2, 2><<<grid, 2 * kAttThreads, 0, s>>>(a);
-    } else if (add) {
-      attention_grouped_kernel<1, true, 2><<<grid, kAttThreads, 0, s>>>(a);
-    } else {
-      attention_grouped_kernel<1, false, 2><<<grid, kAttThreads, 0, s>>>(a);
-    }
+  switch (add_kind(a)) {
+    case kAddNone: launch_grouped<kAddNone>(a, plan.wide, seq_len, grid, s); break;
+    case kAddMask: launch_grouped<kAddMask>(a, plan.wide, seq_len, grid, s); break;
+    case kAddBias: launch_grouped<kAddBias>(a, plan.wide, seq_len, grid, s); break;
+    default: launch_grouped<kAddBoth>(a, plan.wide, seq_len, grid, s); break;
   }
   BT_CHECK_LAUNCH("attention_grouped_kernel");
   return BT_OK;

@@ -307,6 +307,45 @@ def test_attention_generic_f16(device, lens, S, heads, d, padded, att_order):
         assert np.all(err <= 2.0 ** -10 * np.abs(exp[r0:r0 + nq]) + 1e-4), (b, err.max())
 
 
+@pytest.mark.parametrize("kind", ["mask", "bias", "both"])
+@pytest.mark.parametrize("S,d", [(1, 64), (2, 64), (3, 128), (63, 64), (65, 64), (129, 64), (130, 32), (67, 128)])
+def test_additive_terms_at_odd_lengths(device, S, d, kind):
+    """Rows of the mask and of the bias start anywhere and end inside a tile: the 64-wide streaming
+    kernel (with one and with two query blocks, and its key-split form) and the generic one."""
+    rs = np.random.RandomState(S + d)
+    heads, lens = 3, [S, max(1, S // 2)]
+    B, H = len(lens), heads * d
+    bi = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    qkv = rs.standard_normal((B * S, 3 * H)).astype(np.float16)
+    mask = bias = None
+    if kind != "bias":
+        mask = (rs.rand(B, S, S) < 0.6).astype(np.float16)
+        mask[:, :, S // 2] = 1
+    if kind != "mask":
+        bias = rs.standard_normal((heads, S, S)).astype(np.float16)
+    padded = mask is not None
+    exp = _naive_attention(qkv.astype(np.float32), lens, S, heads, d, 0.125, padded,
+                           None if mask is None else mask.astype(np.float32),
+                           None if bias is None else bias.astype(np.float32))
+    args = dict(padded_rows=padded, mask=None if mask is None else _dev(mask, device),
+                bias=None if bias is None else _dev(bias, device))
+    got = [ops.attention_generic_f16(_dev(qkv, device), _dev(bi, device), B, S, heads, 0.125, **args)]
+    if d == 64:
+        by_head = _dev(np.ascontiguousarray(qkv.reshape(B * S, 3, heads, d).transpose(1, 2, 0, 3)), device)
+        for option, value in (("attention_qb", 1), ("attention_qb", 2), ("attention_key_split", 1)):
+            ops.set_option(option, value)
+            try:
+                got.append(ops.attention_grouped(by_head, _dev(bi, device), B, S, 0.125, **args))
+            finally:
+                ops.set_option(option, -1)
+    for i, g in enumerate(got):
+        for b, n in enumerate(lens):
+            r0, nq = (b * S, S) if padded else (bi[b], n)
+            err = np.abs(g.cpu().numpy()[r0:r0 + nq].astype(np.float64) - exp[r0:r0 + nq])
+            bound = 1e-4 if i == 0 else 2e-3   # (the 64-wide kernel rounds its probabilities to fp16)
+            assert np.all(err <= 2.0 ** -10 * np.abs(exp[r0:r0 + nq]) + bound), (i, b, err.max())
+
+
 def test_attention_f32_rows_sum_and_uniform_keys(device):
     """V = const per column: the output is that constant times sum(P) = 1 / (1 + 1e-6 / sum e),
     whatever Q and K are; identical keys give a uniform P."""
