@@ -48,10 +48,11 @@ void Attention<OpType>::infer(AttentionInferParam infer_param) {
   if (size_per_head_ != 64) {
     // the fp16 kernels are built for 64-wide heads; other head sizes (multiples of 8 up to 128) take the
     // generic kernel over token-major projections (the reference's unfused path for them)
-    check_bt_error(bt_attention_generic_f16(
+    check_bt_error(bt_attention_generic_f16_warm(
         infer_param.qkv, infer_param.attention_output, infer_param.et_param.batch_idx,
         infer_param.seq_order, mask, infer_param.attention_bias, infer_param.batch_size,
         infer_param.seq_len, rows_cap, head_num_, size_per_head_, scale, padded_rows,
+        infer_param.prefetch, infer_param.prefetch_bytes, infer_param.prefetch_count,
         infer_param.stream));
     return;
   }

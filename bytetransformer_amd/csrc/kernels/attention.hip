@@ -33,8 +33,6 @@ namespace bt {
 
 constexpr int kAttThreads = 256;
 constexpr int kHeadDim = 64;
-constexpr int kPrefetchRanges = 4;
-
 struct AttArgs {
   const half_t *qkv;   // [3][heads][rows_cap][64]
   half_t *out;         // [rows, heads*64]
@@ -43,11 +41,7 @@ struct AttArgs {
   const half_t *mask;     // optional [B,S,S] 0/1 mask, padded rows only: every key of the
                           // sequence's S rows takes part, shifted by (mask-1)*10000
   const half_t *bias;     // optional [heads,S,S] term added to the scaled logits
-  // optional: up to kPrefetchRanges ranges that the NEXT kernels will read (weights),
-  // touched line by line so they sit in the memory-side cache: range r holds the 128-byte
-  // lines [pf_end[r - 1], pf_end[r]) of their concatenation (pf_end[last] = 0: none)
-  const char *pf_base[kPrefetchRanges];
-  unsigned pf_end[kPrefetchRanges];
+  WarmDuty warm;          // ranges that the NEXT kernels will read (weights)
   int B, S, rows_cap, heads;
   float scale_log2e;   // scale * log2(e)
   int padded_rows;
@@ -89,36 +83,6 @@ __device__ __forceinline__ AttItem att_item(const AttArgs &p) {
     it.exists = true;
   }
   return it;
-}
-
-// Cache warm-up on behalf of later kernels: the workgroups of the last quarter of the
-// issue order (short sequences and dead tiles, which retire early) each touch one
-// dword per 128-byte line of their slice of the ranges.  The loads are the wave's last
-// instructions; nothing reads their results.
-__device__ __forceinline__ void prefetch_slice(const AttArgs &p) {
-  const unsigned lines = p.pf_end[kPrefetchRanges - 1];
-  if (!lines) return;
-  const unsigned z0 = (unsigned)((unsigned long long)gridDim.x * 3 / 4);
-  if (blockIdx.x < z0) return;
-  const unsigned duty = gridDim.x - z0;
-  const unsigned me = blockIdx.x - z0;
-  const unsigned per = (lines + duty - 1) / duty;
-  const unsigned first = me * per;
-  const unsigned last = first + per < lines ? first + per : lines;
-  for (unsigned l = first + threadIdx.x; l < last; l += blockDim.x) {
-    const char *base = p.pf_base[0];
-    unsigned begin = 0;
-#pragma unroll
-    for (int r = 1; r < kPrefetchRanges; ++r)
-      if (l >= p.pf_end[r - 1]) {
-        base = p.pf_base[r];
-        begin = p.pf_end[r - 1];
-      }
-    unsigned sink;
-    const char *addr = base + (unsigned long long)(l - begin) * 128;
-    asm volatile("global_load_dword %0, %1, off" : "=v"(sink) : "v"(addr) : "memory");
-  }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
 // 16-byte chunk swizzles of a [rows][64] fp16 tile (8 chunks per 128-byte row).
@@ -175,26 +139,30 @@ __global__ __launch_bounds__(kAttThreads * KS, KS == 1 || KIND ? 2 : 4) void att
   static_assert(KS == 1 || KS == 2, "key split");
   __shared__ __attribute__((aligned(1024))) half_t ring[STAGES * kSlotHalfs];
 
+  if (blockIdx.x >= p.warm.grid_work) {
+    warm_slice(p.warm);
+    return;
+  }
   int b, head, seq_start, seq_len, qb_index;
   if (p.xcd_map == 2 && p.work_list) {
     // the balanced order, looked up by an earlier launch: one scalar load
     const int4 w = p.work_list[blockIdx.x];
     if (w.x < 0) {
-      prefetch_slice(p);
+      warm_slice(p.warm);
       return;
     }
     b = w.x, head = w.y & 0xffff, qb_index = w.y >> 16, seq_start = w.z, seq_len = w.w;
   } else if (p.xcd_map == 2) {
     const AttWork w = att_work_balanced<BQ>(p, blockIdx.x);
     if (!w.exists) {
-      prefetch_slice(p);
+      warm_slice(p.warm);
       return;
     }
     b = w.b, head = w.head, seq_start = w.seq_start, seq_len = w.len, qb_index = w.qb;
   } else {
     const AttItem item = att_item(p);
     if (!item.exists) {
-      prefetch_slice(p);
+      warm_slice(p.warm);
       return;
     }
     b = p.seq_order ? p.seq_order[item.rank] : item.rank, head = item.head;
@@ -221,7 +189,7 @@ __global__ __launch_bounds__(kAttThreads * KS, KS == 1 || KIND ? 2 : 4) void att
   const int nq = p.padded_rows ? p.S : klen;
   const int q0 = qb_index * BQ;
   if (q0 >= nq) {
-    prefetch_slice(p);
+    warm_slice(p.warm);
     return;
   }
 
@@ -539,7 +507,7 @@ __global__ __launch_bounds__(kAttThreads * KS, KS == 1 || KIND ? 2 : 4) void att
     }
     __syncthreads();
     if (grp == 1) {
-      prefetch_slice(p);
+      warm_slice(p.warm);
       return;
     }
 #pragma unroll
@@ -570,7 +538,7 @@ __global__ __launch_bounds__(kAttThreads * KS, KS == 1 || KIND ? 2 : 4) void att
       *(half4_t *)(dst + 16 * db) = half4_t{(half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3]};
     }
   }
-  prefetch_slice(p);
+  warm_slice(p.warm);
 }
 
 // The balanced order of a launch of `entries` workgroups as a list: one wave per entry.
@@ -596,9 +564,13 @@ __global__ __launch_bounds__(kAttThreads) void attention_short_kernel(AttArgs p)
   half_t *sK = att_smem;                      // [KEYS][64] swizzled
   half_t *sV = att_smem + KEYS * kHeadDim;    // [KEYS][64] swizzled
 
+  if (blockIdx.x >= p.warm.grid_work) {
+    warm_slice(p.warm);
+    return;
+  }
   const AttItem item = att_item(p);
   if (!item.exists) {
-    prefetch_slice(p);
+    warm_slice(p.warm);
     return;
   }
   const int b = p.seq_order ? p.seq_order[item.rank] : item.rank, head = item.head;
@@ -608,7 +580,7 @@ __global__ __launch_bounds__(kAttThreads) void attention_short_kernel(AttArgs p)
   const int nq = p.padded_rows ? p.S : klen;
   const int q0 = item.qb * BQ;
   if (q0 >= nq) {
-    prefetch_slice(p);
+    warm_slice(p.warm);
     return;
   }
 
@@ -647,7 +619,7 @@ __global__ __launch_bounds__(kAttThreads) void attention_short_kernel(AttArgs p)
   __syncthreads();
   // no barrier follows: a wave whose 16 queries all lie past the sequence is done
   if (q0 + wave * 16 >= nq) {
-    prefetch_slice(p);
+    warm_slice(p.warm);
     return;
   }
 
@@ -727,42 +699,7 @@ __global__ __launch_bounds__(kAttThreads) void attention_short_kernel(AttArgs p)
       *(half4_t *)(dst_row + 16 * db) =
           half4_t{(half_t)o[db][0], (half_t)o[db][1], (half_t)o[db][2], (half_t)o[db][3]};
   }
-  prefetch_slice(p);
-}
-
-// The warm-up pays when the attention kernel runs long enough to hide it: measured
-// a gain of 4-6 % per forward with >= 2 workgroups per CU (batch 16 at 512 tokens
-// and up) and a loss of 2-3 % with smaller grids, which therefore skip it.  Each
-// duty workgroup (last quarter of the issue order; a half measured 0.7 % slower) touches at most four
-// lines per thread; the range is cut to that.
-static int set_prefetch(AttArgs &a, unsigned grid, const void *const *prefetch,
-                        const unsigned long long *bytes, int count) {
-  for (int r = 0; r < kPrefetchRanges; ++r) {
-    a.pf_base[r] = nullptr;
-    a.pf_end[r] = 0;
-  }
-  BT_REQUIRE(count >= 0 && count <= kPrefetchRanges, BT_ERR_INVALID_ARGUMENT,
-             "attention: prefetch_count=%d outside [0, %d]", count, kPrefetchRanges);
-  BT_REQUIRE(count == 0 || (prefetch && bytes), BT_ERR_INVALID_ARGUMENT,
-             "attention: prefetch ranges need their pointers and sizes");
-  if (!count || !option_prefetch()) return BT_OK;
-  if (grid < (unsigned)option_prefetch_min_grid()) return BT_OK;
-  const unsigned long long duty = grid - (unsigned long long)grid * 3 / 4;
-  unsigned long long left = duty * 4 * kAttThreads;   // lines the duty workgroups take on
-  unsigned end = 0;
-  for (int r = 0; r < kPrefetchRanges; ++r) {
-    if (r < count && prefetch[r] && left) {
-      // one dword at the start of each 128-byte line; a last line of fewer than four bytes
-      // is left alone, so no byte outside the range is read
-      unsigned long long lines = (bytes[r] + 124) / 128;
-      if (lines > left) lines = left;
-      left -= lines;
-      a.pf_base[r] = (const char *)prefetch[r];
-      end += (unsigned)lines;
-    }
-    a.pf_end[r] = end;
-  }
-  return BT_OK;
+  warm_slice(p.warm);
 }
 
 // Size of the 1-D grid for `nqb` query tiles per sequence; fills the mapping fields.
@@ -843,12 +780,12 @@ extern "C" int bt_attention_short(const void *qkv_heads, void *attention_output,
              "bt_attention_short: seq_len=%d exceeds 512, use bt_attention_grouped", seq_len);
   AttArgs a{(const half_t *)qkv_heads, (half_t *)attention_output, batch_idx, seq_order,
             (const half_t *)atten_mask, (const half_t *)attention_bias,
-            {}, {}, batch_size, seq_len,
+            {}, batch_size, seq_len,
             rows_cap, head_num, scale * kLog2e, padded_rows};
   a.every_key = drop_terms_of_one_key(seq_len, a.mask, a.bias);
   hipStream_t s = as_stream(stream);
   a.nqb_grid = att_grid(a, (seq_len + 63) / 64);
-  rc = set_prefetch(a, a.nqb_grid, prefetch, prefetch_bytes, prefetch_count);
+  rc = plan_warm_duty("bt_attention_short", a.warm, a.nqb_grid, prefetch, prefetch_bytes, prefetch_count);
   if (rc) return rc;
   if (seq_len <= 64) return launch_short<4>(a, s);
   if (seq_len <= 128) return launch_short<8>(a, s);
@@ -959,7 +896,7 @@ extern "C" int bt_attention_grouped(const void *qkv_heads, void *attention_outpu
   if (no_offsets) seq_order = nullptr;
   AttArgs a{(const half_t *)qkv_heads, (half_t *)attention_output, batch_idx, seq_order,
             (const half_t *)atten_mask, (const half_t *)attention_bias,
-            {}, {}, batch_size, seq_len,
+            {}, batch_size, seq_len,
             rows_cap, head_num, scale * kLog2e, padded_rows};
   a.every_key = drop_terms_of_one_key(seq_len, a.mask, a.bias);
   a.mask_ok = a.mask ? mask_prefix_slots : nullptr;
@@ -970,8 +907,8 @@ extern "C" int bt_attention_grouped(const void *qkv_heads, void *attention_outpu
     a.xcd_map = 1;
     plan.grid = ((unsigned)batch_size * head_num + 7) / 8 * 8 * a.nqb;
   }
-  const unsigned grid = plan.grid;
-  rc = set_prefetch(a, grid, prefetch, prefetch_bytes, prefetch_count);
+  unsigned grid = plan.grid;
+  rc = plan_warm_duty("bt_attention_grouped", a.warm, grid, prefetch, prefetch_bytes, prefetch_count);
   if (rc) return rc;
   switch (add_kind(a)) {
     case kAddNone: launch_grouped<kAddNone>(a, plan.wide, seq_len, grid, s); break;

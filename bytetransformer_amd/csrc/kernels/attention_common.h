@@ -134,4 +134,85 @@ __device__ __forceinline__ float4_t add_terms(float4_t s, float scale, uint2_t m
   return v;
 }
 
+// ---- cache warm-up on behalf of later kernels ------------------------------------------------
+// Ranges that the launches after this one will read (the layer's remaining weights): some workgroups
+// touch one dword per 128-byte line of their slice, so that the products find them in the memory-side
+// cache.  Range r holds the lines [end[r - 1], end[r]) of the concatenation (end[3] = 0: none).
+constexpr int kWarmRanges = 4;
+struct WarmDuty {
+  const char *base[kWarmRanges];
+  unsigned end[kWarmRanges];
+  unsigned first;       // the workgroups from here on take part
+  unsigned grid_work;   // workgroups of the attention itself: later ones do nothing else
+};
+// The loads are the wave's last instructions; nothing reads their results.
+__device__ __forceinline__ void warm_slice(const WarmDuty &w) {
+  const unsigned lines = w.end[kWarmRanges - 1];
+  if (!lines) return;
+  if (blockIdx.x < w.first) return;
+  const unsigned duty = gridDim.x - w.first;
+  const unsigned me = blockIdx.x - w.first;
+  const unsigned per = (lines + duty - 1) / duty;
+  const unsigned first = me * per;
+  const unsigned last = first + per < lines ? first + per : lines;
+  for (unsigned l = first + threadIdx.x; l < last; l += blockDim.x) {
+    const char *base = w.base[0];
+    unsigned begin = 0;
+#pragma unroll
+    for (int r = 1; r < kWarmRanges; ++r)
+      if (l >= w.end[r - 1]) {
+        base = w.base[r];
+        begin = w.end[r - 1];
+      }
+    unsigned sink;
+    const char *addr = base + (unsigned long long)(l - begin) * 128;
+    asm volatile("global_load_dword %0, %1, off" : "=v"(sink) : "v"(addr) : "memory");
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+// Who takes part, for a launch of `grid` workgroups (grown here by the ones that only warm).
+//   Two workgroups per CU and more (option prefetch_min_grid): the last quarter of the issue order -
+//   short sequences and dead tiles, which retire early - at four lines a thread (batch 16 at 512 tokens: -4
+//   to -6 % per forward; half of the grid measured 0.7 % slower).
+//   Fewer: the launch leaves CUs idle, and 96 to 208 workgroups of their own, about what fills the chip
+//   up, touch the weights meanwhile.  Left to the attention's own workgroups the touches lengthened
+//   it (+3 to +8 % per forward); with workgroups of their own 12 layers take 454 -> 412 us at batch
+//   1 x 32, 545 -> 490 at 1 x 256, 520 -> 477 at 4 x 96, 800 -> 762 at 7 x 217, 929 -> 875 at 6 x 250.
+inline int plan_warm_duty(const char *who, WarmDuty &w, unsigned &grid, const void *const *ranges,
+                          const unsigned long long *bytes, int count) {
+  for (int r = 0; r < kWarmRanges; ++r) {
+    w.base[r] = nullptr;
+    w.end[r] = 0;
+  }
+  w.first = w.grid_work = grid;
+  BT_REQUIRE(count >= 0 && count <= kWarmRanges, BT_ERR_INVALID_ARGUMENT,
+             "%s: prefetch_count=%d outside [0, %d]", who, count, kWarmRanges);
+  BT_REQUIRE(count == 0 || (ranges && bytes), BT_ERR_INVALID_ARGUMENT,
+             "%s: prefetch ranges need their pointers and sizes", who);
+  if (!count || !option_prefetch()) return BT_OK;
+  unsigned long long left;   // lines that the duty workgroups take on
+  if (grid < (unsigned)option_prefetch_min_grid()) {
+    const unsigned idle = grid < 256 ? 256 - grid : 0, extra = idle < 96 ? 96 : idle > 208 ? 208 : idle;
+    grid += extra;
+    left = (unsigned long long)extra * 8 * 256;
+  } else {
+    w.first = (unsigned)((unsigned long long)grid * 3 / 4);
+    left = (unsigned long long)(grid - w.first) * 4 * 256;
+  }
+  unsigned end = 0;
+  for (int r = 0; r < kWarmRanges; ++r) {
+    if (r < count && ranges[r] && left) {
+      // one dword at the start of each 128-byte line; a last line of fewer than four bytes
+      // is left alone, so no byte outside the range is read
+      unsigned long long lines = (bytes[r] + 124) / 128;
+      if (lines > left) lines = left;
+      left -= lines;
+      w.base[r] = (const char *)ranges[r];
+      end += (unsigned)lines;
+    }
+    w.end[r] = end;
+  }
+  return BT_OK;
+}
+
 }  // namespace bt

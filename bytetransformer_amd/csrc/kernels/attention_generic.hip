@@ -39,6 +39,7 @@ struct GenericAttArgs {
   int balanced;           // 1: the live query tiles are dealt evenly to the CUs (common.h)
   int d;                  // head size <= D
   int every_key;          // 1: all S keys of a sequence take part, whatever its length
+  WarmDuty warm;          // ranges that the launches after this one will read (weights)
 };
 
 // 16-byte chunk swizzles of a [64][D] tile, D / 8 chunks per row (compare swz_k / swz_v of the
@@ -63,15 +64,25 @@ __global__ __launch_bounds__(kGenThreads, 2) void attention_generic_kernel(Gener
   constexpr int NLD = CPR / 4;                // load instructions per wave for K, and as many for V
   __shared__ __attribute__((aligned(1024))) half_t ring[2 * 2 * kTile];
 
+  if (blockIdx.x >= p.warm.grid_work) {
+    warm_slice(p.warm);
+    return;
+  }
   int b, head, seq_start, seq_len, qb_index;
   if (p.balanced) {
     const AttWork w = att_work_balanced<BQ>(p, blockIdx.x);
-    if (!w.exists) return;
+    if (!w.exists) {
+      warm_slice(p.warm);
+      return;
+    }
     b = w.b, head = w.head, seq_start = w.seq_start, seq_len = w.len, qb_index = w.qb;
   } else {
     const unsigned lin = blockIdx.x, slot = lin >> 3;
     const unsigned pair = (slot / p.nqb) * 8 + (lin & 7);
-    if (pair >= (unsigned)(p.B * p.heads)) return;
+    if (pair >= (unsigned)(p.B * p.heads)) {
+      warm_slice(p.warm);
+      return;
+    }
     const int rank = pair / p.heads;
     head = pair % p.heads;
     b = p.seq_order ? p.seq_order[rank] : rank;
@@ -83,7 +94,10 @@ __global__ __launch_bounds__(kGenThreads, 2) void attention_generic_kernel(Gener
   const int row_start = p.padded_rows ? b * p.S : seq_start;
   const int nq = p.padded_rows ? p.S : seq_len;
   const int q0 = qb_index * BQ;
-  if (q0 >= nq) return;
+  if (q0 >= nq) {
+    warm_slice(p.warm);
+    return;
+  }
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -315,6 +329,7 @@ __global__ __launch_bounds__(kGenThreads, 2) void attention_generic_kernel(Gener
       *(half4_t *)(dst + 16 * db) = half4_t{(half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3]};
     }
   }
+  warm_slice(p.warm);
 }
 
 template <int ND, int KIND>
@@ -342,13 +357,15 @@ void launch_generic(const GenericAttArgs &p, int kind, bool wide, unsigned grid,
 
 using namespace bt;
 
-extern "C" int bt_attention_generic_f16(const void *qkv, void *out, const int *batch_idx,
-                                        const int *seq_order, const void *atten_mask,
-                                        const void *attention_bias, int batch_size, int seq_len,
-                                        int rows_cap, int head_num, int size_per_head,
-                                        float scale, int padded_rows, void *stream) {
+extern "C" int bt_attention_generic_f16_warm(const void *qkv, void *out, const int *batch_idx,
+                                             const int *seq_order, const void *atten_mask,
+                                             const void *attention_bias, int batch_size, int seq_len,
+                                             int rows_cap, int head_num, int size_per_head,
+                                             float scale, int padded_rows, const void *const *prefetch,
+                                             const unsigned long long *prefetch_bytes,
+                                             int prefetch_count, void *stream) {
   const char *who = "bt_attention_generic_f16";
-  const int rc = check_generic_attention(who, qkv, out, batch_idx, atten_mask, attention_bias, batch_size,
+  int rc = check_generic_attention(who, qkv, out, batch_idx, atten_mask, attention_bias, batch_size,
                                          seq_len, rows_cap, head_num, size_per_head, padded_rows);
   if (rc != BT_OK) return rc;
   GenericAttArgs p{(const half_t *)qkv, (half_t *)out, batch_idx, seq_order, (const half_t *)atten_mask,
@@ -368,7 +385,9 @@ extern "C" int bt_attention_generic_f16(const void *qkv, void *out, const int *b
   const unsigned per_xcd = ((unsigned)batch_size * head_num + 7) / 8 * p.nqb;
   const int order = option_attention_xcd_map();
   p.balanced = order == 3 || (order == 2 && per_xcd > 64 && batch_size <= 128);
-  const unsigned grid = p.balanced ? (per_xcd + 31) / 32 * 32 * 8 : per_xcd * 8;
+  unsigned grid = p.balanced ? (per_xcd + 31) / 32 * 32 * 8 : per_xcd * 8;
+  rc = plan_warm_duty(who, p.warm, grid, prefetch, prefetch_bytes, prefetch_count);
+  if (rc != BT_OK) return rc;
   hipStream_t s = as_stream(stream);
   const int kind = (p.mask ? kAddMask : 0) | (p.bias ? kAddBias : 0);
   switch ((size_per_head + 31) / 32) {
@@ -379,4 +398,14 @@ extern "C" int bt_attention_generic_f16(const void *qkv, void *out, const int *b
   }
   BT_CHECK_LAUNCH(who);
   return BT_OK;
+}
+
+extern "C" int bt_attention_generic_f16(const void *qkv, void *out, const int *batch_idx,
+                                        const int *seq_order, const void *atten_mask,
+                                        const void *attention_bias, int batch_size, int seq_len,
+                                        int rows_cap, int head_num, int size_per_head,
+                                        float scale, int padded_rows, void *stream) {
+  return bt_attention_generic_f16_warm(qkv, out, batch_idx, seq_order, atten_mask, attention_bias,
+                                       batch_size, seq_len, rows_cap, head_num, size_per_head, scale,
+                                       padded_rows, nullptr, nullptr, 0, stream);
 }

@@ -267,6 +267,17 @@ def gemm_qkv_bias_split_mask_rows(x, mask, wt_qkv, bias_qkv, head_num, size_per_
     return out, batch_idx, word_idx, seq_order
 
 
+def _warm_ranges(prefetch):
+    """prefetch: None, one tensor or up to four, the ranges later kernels will read."""
+    ranges = [] if prefetch is None else ([prefetch] if torch.is_tensor(prefetch) else list(prefetch))
+    n = len(ranges)
+    ptrs = (ctypes.c_void_p * max(n, 1))(*[t.data_ptr() for t in ranges])
+    sizes = (ctypes.c_ulonglong * max(n, 1))(*[t.numel() * t.element_size() for t in ranges])
+    for t in ranges:
+        _ptr(t)
+    return ptrs, sizes, n
+
+
 def _attention(fn, qkv_heads, batch_idx, batch_size, seq_len, scale, padded_rows, out,
                seq_order=None, mask=None, bias=None, prefetch=None, extra=()):
     _, head_num, rows_cap, d = qkv_heads.shape
@@ -274,13 +285,7 @@ def _attention(fn, qkv_heads, batch_idx, batch_size, seq_len, scale, padded_rows
         out = torch.zeros(rows_cap, head_num * d, dtype=qkv_heads.dtype, device=qkv_heads.device)
     if bias is not None and tuple(bias.shape) != (head_num, seq_len, seq_len):
         raise ValueError("attention bias must be [head_num, seq_len, seq_len]")
-    # prefetch: one tensor or up to four, the ranges later kernels will read
-    ranges = [] if prefetch is None else ([prefetch] if torch.is_tensor(prefetch) else list(prefetch))
-    n = len(ranges)
-    ptrs = (ctypes.c_void_p * max(n, 1))(*[t.data_ptr() for t in ranges])
-    sizes = (ctypes.c_ulonglong * max(n, 1))(*[t.numel() * t.element_size() for t in ranges])
-    for t in ranges:
-        _ptr(t)
+    ptrs, sizes, n = _warm_ranges(prefetch)
     _check(fn(_ptr(qkv_heads), _ptr(out), _ptr(batch_idx), _ptr(seq_order), _ptr(mask), _ptr(bias),
               batch_size, seq_len, rows_cap, head_num, d, float(scale), int(padded_rows),
               ptrs, sizes, n, *extra, _stream()))
@@ -430,16 +435,16 @@ def attention_f32(qkv, batch_idx, batch_size, seq_len, head_num, scale, padded_r
 
 
 def attention_generic_f16(qkv, batch_idx, batch_size, seq_len, head_num, scale, padded_rows=False,
-                          mask=None, bias=None, out=None, seq_order=None):
+                          mask=None, bias=None, out=None, seq_order=None, prefetch=None):
     """fp16 qkv [rows, 3 * hidden] (bias added) -> [rows, hidden]; head sizes 32, 64, 96, 128."""
     rows_cap, three_h = qkv.shape
     hidden = three_h // 3
     if out is None:
         out = torch.zeros(rows_cap, hidden, dtype=qkv.dtype, device=qkv.device)
-    _check(kernel_lib().bt_attention_generic_f16(
+    _check(kernel_lib().bt_attention_generic_f16_warm(
         _ptr(qkv), _ptr(out), _ptr(batch_idx), _ptr(seq_order), _ptr(mask), _ptr(bias), batch_size,
         seq_len, rows_cap, head_num, hidden // head_num, float(scale), int(padded_rows),
-        _stream()))
+        *_warm_ranges(prefetch), _stream()))
     return out
 
 

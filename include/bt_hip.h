@@ -77,8 +77,8 @@ const char *bt_last_error_string(void);
  *                   copies that pay for FFN1 and FFN2 (bt_add_bias_residual_layernorm_copy) | such
  *                   a layer makes no copies (or keeps the prologue for them).  Same results.
  *   "prefetch"      1 (default) | 0: honour / ignore the prefetch hint of the attention entries
- *   "prefetch_min_grid"  512 (default): attention launches of fewer workgroups ignore the hint
- *                   (there the warm-up costs more than it returns); 1 = every launch honours it
+ *   "prefetch_min_grid"  512 (default): attention launches of fewer workgroups leave the hint to
+ *                   workgroups of their own, larger ones to their last quarter; 1 = always the latter
  *   "f32_gemm_tile" -1 heuristic | 0: 64x64 tile | 1: 64x32 | 2: 32x32 (four waves over k each) | 3: 32x32,
  *                   eight waves over k, 64-bit addresses (bt_gemm_f32 only)
  *   "attention_short_limit"  0 (default) .. 512: the host library sends sequences up to this
@@ -300,7 +300,8 @@ int bt_gemm_qkv_bias_split_mask_rows(const void *from_tensor, const void *atten_
  *   prefetch, prefetch_bytes, prefetch_count (nullable / 0): up to 4 readable device
  *                     ranges (host arrays of pointers and sizes) that LATER kernels of the
  *                     stream will read, typically the layer's remaining weight matrices.
- *                     Workgroups that retire early touch them line by line so that they
+ *                     Workgroups that retire early, or that a launch too small to fill the
+ *                     chip gets on top, touch them line by line so that they
  *                     sit in the memory-side cache by then; purely a hint, the results do
  *                     not depend on it.  No counterpart in the reference.
  *   seq_order (nullable): a permutation of the sequence indices from
@@ -477,6 +478,14 @@ int bt_attention_generic_f16(const void *qkv, void *attention_output, const int 
                              const void *attention_bias, int batch_size, int seq_len,
                              int rows_cap, int head_num, int size_per_head, float scale,
                              int padded_rows, void *stream);
+/* ... with the cache hint of the 64-wide entries (prefetch, prefetch_bytes, prefetch_count). */
+int bt_attention_generic_f16_warm(const void *qkv, void *attention_output, const int *batch_idx,
+                                  const int *seq_order, const void *atten_mask,
+                                  const void *attention_bias, int batch_size, int seq_len,
+                                  int rows_cap, int head_num, int size_per_head, float scale,
+                                  int padded_rows, const void *const *prefetch,
+                                  const unsigned long long *prefetch_bytes, int prefetch_count,
+                                  void *stream);
 
 int bt_attention_f32(const void *qkv, void *attention_output, const int *batch_idx,
                      const int *seq_order, const void *atten_mask, const void *attention_bias, int batch_size,

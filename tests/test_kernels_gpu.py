@@ -1217,6 +1217,20 @@ def test_attention_prefetch_hint_changes_nothing(device, kind, lens, S):
         ops.set_option("prefetch_min_grid", 512)
 
 
+@pytest.mark.parametrize("B,S,heads,d", [(1, 33, 2, 32), (3, 200, 12, 128), (40, 64, 12, 96)])
+def test_generic_attention_prefetch_hint_changes_nothing(device, B, S, heads, d):
+    """Warm-up by workgroups of their own (small launches) and by the last quarter of the grid."""
+    rs = np.random.RandomState(S)
+    bi = np.arange(B + 1, dtype=np.int32) * S
+    qkv = _dev(rs.standard_normal((B * S, 3 * heads * d)).astype(np.float16), device)
+    base = ops.attention_generic_f16(qkv, _dev(bi, device), B, S, heads, 0.125)
+    for nbytes in (1, 131, (8 << 20) + 2):
+        whole = torch.full((nbytes + 8192,), 7, dtype=torch.uint8, device=device)
+        got = ops.attention_generic_f16(qkv, _dev(bi, device), B, S, heads, 0.125,
+                                        prefetch=[whole[4096:4096 + nbytes], whole[4096:4097]])
+        assert torch.equal(got, base) and bool((whole == 7).all()), nbytes
+
+
 def test_attention_large_logits_do_not_overflow(device):
     """Logits of a few hundred in magnitude (fp16 Q.K would overflow at 65504)."""
     rs = np.random.RandomState(9)
