@@ -178,6 +178,8 @@ __device__ __forceinline__ void warm_slice(const WarmDuty &w) {
 //   up, touch the weights meanwhile.  Left to the attention's own workgroups the touches lengthened
 //   it (+3 to +8 % per forward); with workgroups of their own 12 layers take 454 -> 412 us at batch
 //   1 x 32, 545 -> 490 at 1 x 256, 520 -> 477 at 4 x 96, 800 -> 762 at 7 x 217, 929 -> 875 at 6 x 250.
+//   More than 12 MB (BERT-large has 25 with the next layer's QKV weight) takes longer than the
+//   attention itself: 24 layers of hidden 1024 at 3 x 28, encoder entry 924 us with 12 MB, 935 with all.
 inline int plan_warm_duty(const char *who, WarmDuty &w, unsigned &grid, const void *const *ranges,
                           const unsigned long long *bytes, int count) {
   for (int r = 0; r < kWarmRanges; ++r) {
@@ -194,7 +196,7 @@ inline int plan_warm_duty(const char *who, WarmDuty &w, unsigned &grid, const vo
   if (grid < (unsigned)option_prefetch_min_grid()) {
     const unsigned idle = grid < 256 ? 256 - grid : 0, extra = idle < 96 ? 96 : idle > 208 ? 208 : idle;
     grid += extra;
-    left = (unsigned long long)extra * 8 * 256;
+    left = 98304;   // 12 MB: what fits beside an attention of 4 to 6 us
   } else {
     w.first = (unsigned)((unsigned long long)grid * 3 / 4);
     left = (unsigned long long)(grid - w.first) * 4 * 256;
