@@ -394,11 +394,13 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &p) {
     const int per = (live + 7) >> 3;
     const int L = (bid & 7) * per + (bid >> 3);
     if (bid >= per * 8 || L >= live) return;
-    if (BM == 32 && tiles_m > 1) {
+    if (BM == 32 && tiles_m > 3) {
       // A few hundred rows: the launch is as long as it takes to fetch the weight, and in row-major
       // order every XCD fetches all of it (256 rows, QKV at hidden 768: 28 MB in all against
-      // 7 MB in panels; 12 layers at batch 1 x 256: -8 %).  With the larger tiles the panels gain
-      // nothing and their index arithmetic costs up to 1 %.
+      // 7 MB in panels; 12 layers at batch 1 x 256: -8 %).  At two or three tile rows few workgroups
+      // share a fetch and those of one XCD wait on the same lines (24 layers of hidden 1024 at 46
+      // rows: 941 us in panels, 917 row-major).  With the larger tiles the panels gain nothing and
+      // their index arithmetic costs up to 1 %.
       tile_panels<BM, BN>(tiles_m, p.tiles_n, per).locate(L, tile_m, tile_n);
     } else {
       tile_m = L / p.tiles_n;
@@ -1078,15 +1080,15 @@ static long long estimated_rows(const GemmArgs &p) {
 
 // Measured times of every tile for this weight shape at the first table row of at least m
 // rows, or nullptr when the shape is not in the table or m lies outside it (the analytic
-// model then decides alone).  The rows are kTunedStep apart, the height of the tallest
-// tile, so the row used has the same number of row tiles as m or one more: run time moves
-// in steps with the number of rounds of workgroups, and interpolating between two row
-// counts on either side of such a step would describe neither.
+// model then decides alone).  The rows are at most kTunedStep apart where most launches are, the
+// height of the tallest tile (and closer below, where smaller tiles matter), so the row used has the same number
+// of row tiles as m or one more: run time moves in steps with the number of rounds of workgroups, and
+// interpolating between two row counts on either side of such a step would describe neither.
 static const float *tuned_times(long long m, int n, int k, int epi, int kn, int full) {
   if (cu_count() != 256) return nullptr;     // the table was measured on a 256-CU part
-  // below about a thousand rows a launch is latency bound and a loop of identical
-  // launches says little about the layer sequence
-  if (m < 1024 || m > kTunedRows[kTunedPoints - 1]) return nullptr;
+  if (m > kTunedRows[kTunedPoints - 1]) return nullptr;
+  // (the token-major QKV projection differs from the head-major one in where it stores)
+  if (epi == kEpiBias) epi = kEpiQkvSplit;
   for (const TunedShape &ts : kTunedShapes) {
     if (ts.n != n || ts.k != k || ts.epi != epi || ts.kn != kn || ts.full != full) continue;
     int at = 0;
@@ -1094,6 +1096,80 @@ static const float *tuned_times(long long m, int n, int k, int epi, int kn, int 
     return ts.us[at];
   }
   return nullptr;
+}
+
+// The row counts a tile is priced at.  A launch over padded sequences whose caller named no row
+// count holds 60 % of its capacity give or take: the mean of a handful of sequence lengths is off
+// by 10-20 %.  A tile priced at the middle alone may fit one round of the chip there and need two
+// a few rows later (7 sequences of up to 844 tokens, narrow products: 17.4 us a launch with the tile
+// this picks, 23.3 us with the one that was fastest at 60 %), so it is priced over the spread.
+struct LikelyRows {
+  long long rows[5];
+  float weight[5];
+  int count;
+  explicit LikelyRows(const GemmArgs &p) {
+    const long long m = estimated_rows(p);
+    const bool guess = (p.valid_rows || p.mask) && p.rows_hint <= 0;
+    count = guess ? 5 : 1;
+    for (int i = 0; i < count; ++i) {
+      rows[i] = guess ? (m * (8 + i) + 9) / 10 : m;
+      weight[i] = !guess ? 1.f : i == 2 ? 1.f / 3.f : 1.f / 6.f;
+    }
+  }
+};
+
+struct TileModel {
+  int id, bm, bn;
+  float step_us, fixed_us;   // one k-step of one tile; launch, fill and epilogue of one tile
+  float shared_us;           // > 0: one k-step's share of a CU that several tiles occupy
+};
+
+// Time of one launch of n columns and k reduction: fixed + k-steps x step time, where a step takes
+// `step_us` while every CU has one tile at most and then grows in whole rounds or, where several
+// workgroups share a CU, with its load.
+static float model_us(const TileModel &c, long long m, int n, int k) {
+  const int cus = cu_count();
+  const float nk = (float)(k / kBK);
+  const long long tiles = ((m + c.bm - 1) / c.bm) * ((n + c.bn - 1) / c.bn);
+  if (c.shared_us > 0.f) {
+    const float load = (float)tiles / (float)cus * c.shared_us;
+    return c.fixed_us + nk * (load > c.step_us ? load : c.step_us);
+  }
+  return (float)((tiles + cus - 1) / cus) * (nk * c.step_us + c.fixed_us - 1.8f) + 1.8f;
+}
+
+static int fastest_by_model(const LikelyRows &likely, int n, int k) {
+  // (fitted to the table's measurements: on average the choice is 1.2 % slower than the fastest
+  // tile, and 7 % or more in one case of twenty)
+  static const TileModel models[] = {{0, 256, 256, 1.45f, 5.7f, 0.f},   {13, 192, 192, 0.95f, 4.7f, 0.f},
+                                     {3, 256, 192, 1.10f, 4.35f, 0.f},  {12, 128, 192, 0.64f, 4.6f, 0.f},
+                                     {2, 256, 128, 0.79f, 4.4f, 0.f},   {1, 128, 128, 0.467f, 3.4f, 0.f},
+                                     {5, 128, 128, 0.66f, 3.6f, 0.70f}, {11, 96, 128, 0.41f, 3.0f, 0.f},
+                                     {10, 64, 128, 0.267f, 2.67f, 0.43f}, {9, 64, 64, 0.20f, 2.63f, 0.265f},
+                                     {4, 32, 64, 0.175f, 2.75f, 0.19f}};
+  int best_id = 0;
+  float best = 0.f;
+  for (const TileModel &c : models) {
+    float t = 0.f;
+    for (int i = 0; i < likely.count; ++i) t += likely.weight[i] * model_us(c, likely.rows[i], n, k);
+    if (best == 0.f || t < best) {
+      best = t;
+      best_id = c.id;
+    }
+  }
+  return best_id;
+}
+
+// The table's times of every tile over the likely rows (0 = not measured at all of them); false
+// when the table does not cover the launch.
+static bool tuned_mean(const LikelyRows &likely, int n, int k, int epi, int kn, int full, float *us) {
+  for (int i = 0; i < likely.count; ++i) {
+    const float *at = tuned_times(likely.rows[i], n, k, epi, kn, full);
+    if (!at) return false;
+    for (int t = 0; t < kTunedTiles; ++t)
+      us[t] = at[t] > 0.f && (i == 0 || us[t] > 0.f) ? (i == 0 ? 0.f : us[t]) + likely.weight[i] * at[t] : 0.f;
+  }
+  return true;
 }
 
 template <int EPI>
@@ -1113,54 +1189,31 @@ static int launch_gemm(GemmArgs p, hipStream_t s) {
   //   6, 7, 8                 tiles 2, 1 and 0 in the persistent form (gemm_tiles_flat); never
   //                           the model's choice, only the measured table's, and there
   //                           within a few per cent of the one-tile-per-workgroup form
-  // The choice minimises rounds x (k-steps x time of one k-step + fill and epilogue) with
-  // the per-tile constants below, for the estimated live rows; for the weight shapes of
-  // BERT-base and BERT-large a table of measured times (gemm_tuned.inc) then overrides it
-  // where another tile is clearly faster.
+  //   9:  64x64,  4, 2x2, 4   } one round of tiles on 256 CUs between the shapes above: a launch is
+  //  10:  64x128, 3, 2x2, 4   } as long as its largest tile while it fits one round, so the tile
+  //  11:  96x128, 3, 3x2, 4   } that just fills the chip wins.  Hidden 768, weights in the
+  //  12: 128x192, 3, 2x2, 4   } memory-side cache, best of tiles 0-8 and now: FFN2 at 920 rows 17.0 ->
+  //  13: 192x192, 2, 3x2, 4   } 13.0 us (9), at 2000 rows 20.6 -> 17.5 (10), at 5600 rows 35.6 -> 30.2
+  //                           (12); QKV at 3600 rows 19.6 -> 18.6 (13), at 1300 rows 9.6 -> 9.1 (11)
+  // The choice minimises the time of the launch: for the weight shapes of BERT-base and BERT-large
+  // by a table of measured times (gemm_tuned.inc) where it names a clearly faster tile, else by the
+  // model of model_us().
   const int forced = option_gemm_tile();
   int choice = forced;
   if (choice < 0) {
-    const int cus = cu_count();
-    const long long m_est = estimated_rows(p);
-    struct Cand {
-      int id, bm, bn;
-      float step_us, fixed_us;   // one k-step of one tile; fill + epilogue of one tile
-      bool shares_cu;            // several workgroups per CU: time grows with tiles / CUs, not in rounds
-    };
-    const Cand cands[5] = {{0, 256, 256, 1.29f, 3.4f, false},
-                           {3, 256, 192, 1.04f, 2.8f, false},
-                           {2, 256, 128, 0.62f, 2.3f, false},
-                           {1, 128, 128, 0.43f, 1.8f, false},
-                           {4, 32, 64, 0.16f, 2.6f, true}};
-    const float nk = (float)(p.K / kBK);
-    float best = 0.f;
-    for (const Cand &c : cands) {
-      const long long tiles = ((m_est + c.bm - 1) / c.bm) * ((p.N + c.bn - 1) / c.bn);
-      float t;
-      if (c.shares_cu) {
-        const float load = (float)tiles / (float)cus;
-        t = c.fixed_us + nk * c.step_us * (load > 1.f ? load : 1.f);
-      } else {
-        t = (float)((tiles + cus - 1) / cus) * (nk * c.step_us + c.fixed_us);
-      }
-      if (choice < 0 || t < best) {
-        best = t;
-        choice = c.id;
-      }
-    }
-  }
-  if (forced < 0) {
+    const LikelyRows likely(p);
+    float us[kTunedTiles];
+    choice = fastest_by_model(likely, p.N, p.K);
     // the table overrides the model only for a clear win: the timings come from a loop
     // of identical launches, and differences of a few per cent do not carry over to the
     // layer sequence
     // (a launch whose estimated live rows fill its capacity to within one tile row is looked
     // up among the all-live measurements)
-    const long long m_est = estimated_rows(p);
-    if (const float *us = tuned_times(m_est, p.N, p.K, EPI, p.w_kn, m_est + kTunedStep > p.rows_cap)) {
+    if (tuned_mean(likely, p.N, p.K, EPI, p.w_kn, estimated_rows(p) + kTunedStep > p.rows_cap, us)) {
       int tuned = -1;
       for (int t = 0; t < kTunedTiles; ++t)
         if (us[t] > 0.f && (tuned < 0 || us[t] < us[tuned])) tuned = t;
-      const float t_model = choice < kTunedTiles ? us[choice] : 0.f;
+      const float t_model = us[choice];
       const float margin = 1.f - 0.01f * (float)option_gemm_table_margin();
       if (tuned >= 0 && tuned != choice && (t_model <= 0.f || us[tuned] < margin * t_model))
         choice = tuned;
@@ -1183,6 +1236,16 @@ static int launch_gemm(GemmArgs p, hipStream_t s) {
       return launch_gemm_flat<128, 128, 3, 2, 2, 4, 0, EPI>(p, s);
     case 8:
       return launch_gemm_flat<256, 256, 2, 2, 4, 0, 1, EPI>(p, s);
+    case 9:
+      return launch_gemm_tile<64, 64, 4, 2, 2, 4, 0, EPI>(p, s);
+    case 10:
+      return launch_gemm_tile<64, 128, 3, 2, 2, 4, 0, EPI>(p, s);
+    case 11:
+      return launch_gemm_tile<96, 128, 3, 3, 2, 4, 0, EPI>(p, s);
+    case 12:
+      return launch_gemm_tile<128, 192, 3, 2, 2, 4, 0, EPI>(p, s);
+    case 13:
+      return launch_gemm_tile<192, 192, 2, 3, 2, 4, 0, EPI>(p, s);
     default:
       return launch_gemm_tile<128, 128, 3, 2, 2, 4, 0, EPI>(p, s);
   }
@@ -1287,8 +1350,13 @@ extern "C" int bt_gemm_splitk(const void *a, const void *wt, void *partials, int
   GemmArgs p{(const half_t *)a, (const half_t *)wt, nullptr, nullptr, valid_rows, nullptr,
              rows_cap,          n,                  k,       0,       0,          (float *)partials,
              weight_kn};
-  // the small tile only: splitting k is for launches whose k loop is the whole run time
-  return launch_gemm_tile<32, 64, 4, 1, 2, 2, 0, kEpiPartial>(p, as_stream(stream), splits);
+  // Small tiles only: splitting k is for launches whose k loop is the whole run time.  32 rows while
+  // one round of workgroups covers them all, then 64 (hidden 768, k 3072 in two splits with the
+  // LayerNorm behind it: 320 rows 11.6 against 12.1 us, 400 rows 14.0 against 13.0).
+  const long long rows = estimated_rows(p);
+  if ((rows + 31) / 32 * ((n + 63) / 64) * splits <= 256)
+    return launch_gemm_tile<32, 64, 4, 1, 2, 2, 0, kEpiPartial>(p, as_stream(stream), splits);
+  return launch_gemm_tile<64, 64, 4, 2, 2, 4, 0, kEpiPartial>(p, as_stream(stream), splits);
 }
 
 extern "C" int bt_gemm_bias_gelu(const void *a, const void *wt, const void *bias, void *c,

@@ -14,11 +14,13 @@ import os
 import sys
 
 M_STEP = 256                     # the tallest tile: run time steps with the count of row tiles
-M_GRID = tuple(range(M_STEP, 16384 + 1, M_STEP))
+M_GRID = (tuple(range(64, 1024, 64)) + tuple(range(1024, 2560, 128)) + tuple(range(2560, 8192, M_STEP))
+          + tuple(range(8192, 12288 + 1, 512)))
 HIDDEN = (768, 1024)
-TILES = (0, 1, 2, 3, 4, 5, 6, 7, 8)
+TILES = tuple(range(14))
 EPI_CODE = {"plain": 0, "gelu": 1, "qkv": 2}     # enum Epilogue of gemm.hip
-SMALL_TILE_MAX_ROWS = 3000      # the 32x64 tile is not worth timing beyond this
+SMALL_TILE_MAX_ROWS = 3000      # the 32x64 and 64x64 tiles are not worth timing beyond this
+LARGE_TILE_MIN_ROWS = 512       # nor the 192- and 256-row tiles below this
 INC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc", "kernels", "gemm_tuned.inc")
 
 
@@ -49,10 +51,12 @@ def measure(iters=32):
     padded batch: launches are sized for batch x seq_len rows, of which m are live) and with
     a row capacity of m (every row live: the padded path, or a caller that sizes its launches
     for the live rows), the
-    QKV product gathering its rows from the padded input through a word_idx of 16 runs, and
-    with the weights cold: the launches of one timing loop walk through enough copies of
-    the weight matrix to exceed the memory-side cache, as the layers of a model do.  Every
-    shape is timed with the weight in both layouts."""
+    QKV product gathering its rows from the padded input through a word_idx of 16 runs.  Its weight
+    is cold: the launches of one timing loop walk through enough copies of the weight matrix to
+    exceed the memory-side cache, as the layers of a model do.  The other weights have been touched
+    by the attention launch ahead of them and sit in that cache, so theirs walk through fewer
+    copies than fit it (and more than the L2s hold).  Every shape is timed with the weight in
+    both layouts."""
     import torch
     from . import ops
     dev = torch.device("cuda:0")
@@ -65,7 +69,8 @@ def measure(iters=32):
             for epi, n, k in (("qkv", 3 * h, h), ("plain", h, h), ("gelu", 4 * h, h),
                               ("plain", h, 4 * h)):
                 a = torch.randn(rows_cap, k, device=dev).half()
-                copies = min(iters, max(2, -(-300 * 2 ** 20 // (n * k * 2))))
+                span = (300 if epi == "qkv" else 90) * 2 ** 20
+                copies = min(max(iters, 40), max(2, -(-span // (n * k * 2))))
                 ws = [(torch.randn(k, n, device=dev) * 0.02).half() for _ in range(copies)]
                 wts = [ops.transpose_weight(w) for w in ws]
                 bias = torch.zeros(n, device=dev, dtype=torch.float16)
@@ -101,7 +106,9 @@ def measure(iters=32):
                         kn[0] = bool(layout)
                         us = {}
                         for tile in TILES:
-                            if tile == 4 and m > SMALL_TILE_MAX_ROWS:
+                            if tile in (4, 9) and m > SMALL_TILE_MAX_ROWS:
+                                continue
+                            if tile in (0, 2, 3, 6, 8, 13) and m < LARGE_TILE_MIN_ROWS:
                                 continue
                             ops.set_option("gemm_tile", tile)
                             us[str(tile)] = round(_time_kernel(call, iters), 2)

@@ -508,6 +508,50 @@ def test_splitk_gemm_and_layernorm(device, splits, restore, tight):
         assert np.abs(ref[:M].astype(np.float32) - g[:M].astype(np.float32)).max() <= 2e-2
 
 
+@pytest.mark.parametrize("tile,bm,bn", [(9, 64, 64), (10, 64, 128), (11, 96, 128), (12, 128, 192), (13, 192, 192)])
+@pytest.mark.parametrize("w_kn", [False, True])
+def test_gemm_mid_tiles_at_their_edges(device, tile, bm, bn, w_kn):
+    """One row or column less, exactly and one more than the tile, k shorter than the ring and longer,
+    rows gathered and not, all three epilogues: as tile 1 computes them, bit for bit."""
+    _say("gemm mid tiles", tile, w_kn)
+    rs = np.random.RandomState(tile)
+    for M, N, K in ((bm, bn, 64), (bm - 1, bn - 8, 128), (2 * bm + 1, 2 * bn + 8, 448), (1, 8, 192)):
+        rows = M + 3
+        a = _dev(rs.standard_normal((rows, K)).astype(np.float16), device)
+        w = _dev((rs.standard_normal((K, N)) * 0.05).astype(np.float16), device)
+        w = w if w_kn else w.t().contiguous()
+        bias = _dev(rs.standard_normal(N).astype(np.float16), device)
+        vr = torch.tensor([M], dtype=torch.int32, device=device)
+        got = []
+        for t in (tile, 1):
+            ops.set_option("gemm_tile", t)
+            try:
+                out = torch.full((2, rows, N), 3.0, dtype=torch.float16, device=device)
+                ops.gemm(a, w, valid_rows=vr, out=out[0], w_kn=w_kn)
+                ops.gemm_bias_gelu(a, w, bias, valid_rows=vr, out=out[1], w_kn=w_kn)
+            finally:
+                ops.set_option("gemm_tile", -1)
+            got.append(out)
+        assert torch.equal(got[0], got[1]), (M, N, K)
+        assert bool((got[0][:, M:] == 3.0).all())
+    heads, M = 3, bm + 5
+    H, rows = 64 * heads, M + 9
+    x = _dev(rs.standard_normal((rows, H)).astype(np.float16), device)
+    w = _dev((rs.standard_normal((H, 3 * H)) * 0.05).astype(np.float16), device)
+    w = w if w_kn else w.t().contiguous()
+    bias = _dev(rs.standard_normal(3 * H).astype(np.float16), device)
+    index = _dev(rs.permutation(rows).astype(np.int32), device)
+    vr = torch.tensor([M], dtype=torch.int32, device=device)
+    got = []
+    for t in (tile, 1):
+        ops.set_option("gemm_tile", t)
+        try:
+            got.append(ops.gemm_qkv_bias_split(x, w, bias, heads, valid_rows=vr, a_row_index=index, w_kn=w_kn))
+        finally:
+            ops.set_option("gemm_tile", -1)
+    assert torch.equal(got[0], got[1])
+
+
 @pytest.mark.parametrize("tile", [0, 1, 2, 3, 4, 5, 6, 7, 8])
 def test_gemm_bias_gelu(device, tile):
     _say("gemm_bias_gelu", tile)
