@@ -186,6 +186,8 @@ __device__ __forceinline__ float gelu_tanh_f32(float x) {
 // slots.  The 16 lanes that one ds_read_b128 pass serves then touch every bank once.
 __device__ __forceinline__ int swz(int row) { return (row >> 1) & 7; }
 
+// gemm_wave_k: columns of a tile, waves of a workgroup, k-steps in a wave's ring
+constexpr int kWaveKCols = 32, kWaveKWaves = 4, kWaveKDepth = 3;
 constexpr int kBK = 64;   // k extent of one LDS tile (halfs) = 8 chunks of 16 bytes
 
 // A [K, N] weight tile sits in LDS as 64 k-rows of BN halfs and is read with the LDS
@@ -196,7 +198,8 @@ constexpr int kBK = 64;   // k extent of one LDS tile (halfs) = 8 chunks of 16 b
 // row.  Returned in 16-byte chunks (the unit a loading lane moves).
 template <int BN>
 __device__ __forceinline__ int swz_kn(int k_row) {
-  static_assert(BN % 64 == 0, "whole 64-byte segment pairs");
+  static_assert(BN == 32 || BN % 64 == 0, "whole 64-byte segment pairs");
+  if (BN == 32) return 0;   // four k-rows are 256 contiguous bytes
   return (BN / 32) % 4 == 0 ? (k_row & 3) << 2 : ((k_row >> 1) & 1) << 2;
 }
 
@@ -351,6 +354,29 @@ __device__ __forceinline__ void regw_store(const RegW &w, half_t *sW) {
   }
 }
 
+// XCD-aware tile order over the live tiles of M rows; false: the workgroup has none.
+template <int BM, int BN>
+__device__ __forceinline__ bool tile_at(const GemmArgs &p, int M, int bid, int &tile_m, int &tile_n) {
+  const int tiles_m = (M + BM - 1) / BM;
+  const int live = tiles_m * p.tiles_n;
+  const int per = (live + 7) >> 3;
+  const int L = (bid & 7) * per + (bid >> 3);
+  if (bid >= per * 8 || L >= live) return false;
+  if (BM == 32 && tiles_m > 3) {
+    // A few hundred rows: the launch is as long as it takes to fetch the weight, and in row-major
+    // order every XCD fetches all of it (256 rows, QKV at hidden 768: 28 MB in all against
+    // 7 MB in panels; 12 layers at batch 1 x 256: -8 %).  At two or three tile rows few workgroups
+    // share a fetch and those of one XCD wait on the same lines (24 layers of hidden 1024 at 46
+    // rows: 941 us in panels, 917 row-major).  With the larger tiles the panels gain nothing and
+    // their index arithmetic costs up to 1 %.
+    tile_panels<BM, BN>(tiles_m, p.tiles_n, per).locate(L, tile_m, tile_n);
+  } else {
+    tile_m = L / p.tiles_n;
+    tile_n = L - tile_m * p.tiles_n;
+  }
+  return true;
+}
+
 template <int BM, int BN, int STAGES, int WM, int WN, int NP, int SCHED, int EPI, bool WKN>
 __device__ __forceinline__ void gemm_tile(const GemmArgs &p) {
   constexpr int BK = kBK;
@@ -386,27 +412,8 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &p) {
     M = p.valid_rows ? min(*p.valid_rows, p.rows_cap) : p.rows_cap;
   }
 
-  // XCD-aware tile order over the live tiles
   int tile_m, tile_n;
-  {
-    const int tiles_m = (M + BM - 1) / BM;
-    const int live = tiles_m * p.tiles_n;
-    const int per = (live + 7) >> 3;
-    const int L = (bid & 7) * per + (bid >> 3);
-    if (bid >= per * 8 || L >= live) return;
-    if (BM == 32 && tiles_m > 3) {
-      // A few hundred rows: the launch is as long as it takes to fetch the weight, and in row-major
-      // order every XCD fetches all of it (256 rows, QKV at hidden 768: 28 MB in all against
-      // 7 MB in panels; 12 layers at batch 1 x 256: -8 %).  At two or three tile rows few workgroups
-      // share a fetch and those of one XCD wait on the same lines (24 layers of hidden 1024 at 46
-      // rows: 941 us in panels, 917 row-major).  With the larger tiles the panels gain nothing and
-      // their index arithmetic costs up to 1 %.
-      tile_panels<BM, BN>(tiles_m, p.tiles_n, per).locate(L, tile_m, tile_n);
-    } else {
-      tile_m = L / p.tiles_n;
-      tile_n = L - tile_m * p.tiles_n;
-    }
-  }
+  if (!tile_at<BM, BN>(p, M, bid, tile_m, tile_n)) return;
   const int m0 = tile_m * BM, n0 = tile_n * BN;
   // a split-k launch gives grid row y the k range [y, y+1) * K / gridDim.y
   const int nk = EPI == kEpiPartial ? p.K / BK / (int)gridDim.y : p.K / BK;
@@ -975,6 +982,190 @@ __global__ __launch_bounds__((WM * WN + NP) * 64) void gemm_kernel(GemmArgs p) {
 #endif
 }
 
+// ---- a few rows: the waves share the k range, not the tile ----------------------------
+// One 32x32 tile per workgroup.  Its waves take the k-steps in turn (wave w: steps w, w + NW, ...),
+// each through a ring of its own that it fills and reads alone, so the loop has no barrier; their
+// sums are folded through LDS at the end, in wave order.  What bounds such a launch is the chain of
+// k-steps of one tile (barrier, LDS read, MFMAs: 0.18 us each in the 32x64 tile); here a wave has a
+// quarter of them, and with K = 768 all of its loads are in flight at once.  Projection of 230 rows at
+// hidden 768: 5.0 -> 4.4 us; 12 layers at batch 1 x 32 407 -> 397 us, 1 x 256 482 -> 476, captured
+// encoder at 4 x 96 469 -> 458.  Tried and slower: 32x64 tiles (half as many workgroups: 1 x 32 394 us
+// against 372 on one box), six or eight waves (a captured 4 x 96: 416 against 413), and a ring of 6 to 10
+// steps under the 32x64 tile (no gain to -8 %).
+#if defined(__HIP_DEVICE_COMPILE__)
+// The weight operand of 16 k out of a [K, N] image (load_kn_frag, as assembly: in front of the compiler's
+// own transpose read it waits for every direct-to-LDS load of this wave, that is, for the k-steps
+// requested ahead), and the wait for it while LEFT younger LDS operations may be outstanding.
+template <int KSTEP>
+__device__ __forceinline__ void kn_read_step(uint2_t (&w)[2], unsigned at) {
+  constexpr int kRow = kWaveKCols * (int)sizeof(half_t);
+  asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(w[0]) : "v"(at), "n"(KSTEP * 16 * kRow));
+  asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(w[1]) : "v"(at), "n"((KSTEP * 16 + 4) * kRow));
+}
+template <int LEFT>
+__device__ __forceinline__ half8_t lds_wait_operand(uint2_t (&w)[2]) {
+  asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(w[0]), "+v"(w[1]) : "n"(LEFT));
+  return __builtin_bit_cast(half8_t, uint4_t{w[0][0], w[0][1], w[1][0], w[1][1]});
+}
+
+template <int EPI, bool WKN>
+__device__ __forceinline__ void gemm_wave_k(const GemmArgs &p) {
+  constexpr int BM = 32, BN = kWaveKCols, BK = kBK, NW = kWaveKWaves, DEPTH = kWaveKDepth;
+  constexpr int KS = BK / 16;
+  constexpr int NIA = BM / 8, NI = (BM + BN) / 8;   // 1 KB load instructions per k-step
+  constexpr int STEP_HALFS = (BM + BN) * BK;
+  static_assert(BN == 32 && KS == 4, "one MFMA block; the loop body names its four k parts");
+  static_assert((DEPTH - 1) * NI < 64, "pipeline depth");
+  static_assert(BM * BN * sizeof(float) <= DEPTH * STEP_HALFS * sizeof(half_t), "sums fit the ring");
+  extern __shared__ __attribute__((aligned(1024))) half_t gemm_smem[];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int bid = (int)blockIdx.x;
+  half_t *ring = gemm_smem + wave * DEPTH * STEP_HALFS;
+  int M;
+  MaskRows mr{};
+  if (p.mask) {
+    mr = mask_rows_setup(p, wave, NW, lane, (int *)(gemm_smem + NW * DEPTH * STEP_HALFS));
+    M = min(mr.M, p.rows_cap);
+    if (bid == 0 && blockIdx.y == 0) mask_rows_write(p, mr, tid, NW * 64, lane);
+  } else {
+    M = p.valid_rows ? min(*p.valid_rows, p.rows_cap) : p.rows_cap;
+  }
+  int tile_m, tile_n;
+  if (!tile_at<BM, BN>(p, M, bid, tile_m, tile_n)) return;
+  const int m0 = tile_m * BM, n0 = tile_n * BN;
+  const int nk = EPI == kEpiPartial ? p.K / BK / (int)gridDim.y : p.K / BK;
+  const int k_first = EPI == kEpiPartial ? (int)blockIdx.y * nk * BK : 0;
+  const int mine = (nk - wave + NW - 1) / NW;   // (0 where there are fewer steps than waves)
+
+  const bool gather = p.a_row_index != nullptr || p.mask != nullptr;
+  const rsrc_t rs_a =
+      gather ? make_rsrc(p.a + k_first, ((size_t)p.rows_cap * p.K - k_first) * sizeof(half_t))
+             : make_rsrc(p.a + (size_t)m0 * p.K + k_first,
+                         ((size_t)(p.rows_cap - m0) * p.K - k_first) * sizeof(half_t));
+  const rsrc_t rs_w =
+      WKN ? make_rsrc(p.wt + (size_t)k_first * p.N + n0,
+                      ((size_t)(p.K - k_first) * p.N - n0) * sizeof(half_t))
+          : make_rsrc(p.wt + (size_t)n0 * p.K + k_first,
+                      ((size_t)(p.N - n0) * p.K - k_first) * sizeof(half_t));
+  int voff[NI];
+  {
+    MaskRowSpan span{};
+    if (p.mask) span = mask_rows_span(mr, p.mask_B, lane, m0, min(m0 + BM, M) - 1);
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int r = i * 8 + (lane >> 3);
+      const int kc = (lane & 7) ^ swz(r);
+      int row = i < NIA ? r : r - BM;
+      if (i < NIA && gather) {
+        const int live_row = min(m0 + r, M - 1);
+        row = p.mask ? mask_rows_map(mr, span, live_row) : p.a_row_index[live_row];
+      }
+      voff[i] = (row * p.K + kc * 8) * (int)sizeof(half_t);
+      if (WKN && i >= NIA) voff[i] = kn_load_offset<BN>(i - NIA, lane, p.N, p.N - n0);
+    }
+  }
+  const int w_step_bytes = (WKN ? BK * p.N : BK) * (int)sizeof(half_t);
+  auto issue = [&](int i, int slot) {
+    const int kt = wave + i * NW;
+    issue_stage_loads<NI, NIA>(rs_a, rs_w, voff, ring + slot * STEP_HALFS, 8 * BK,
+                               kt * BK * (int)sizeof(half_t), kt * w_step_bytes);
+  };
+#pragma unroll
+  for (int s = 0; s < DEPTH; ++s)
+    if (s < mine) issue(s, s);
+
+  float16_t acc;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) acc[v] = 0.f;
+  const int fr_row = lane & 31, fr_kc = lane >> 5;
+  unsigned kn_at;   // byte offset of this lane's first transpose read, from the weight image
+  {
+    const int lq = lane & 15, g2 = lane >> 4;
+    const int k_row = 8 * (g2 >> 1) + (lq >> 2), col = 16 * (g2 & 1) + 4 * (lq & 3);
+    kn_at = (k_row * BN + col) * (int)sizeof(half_t);
+  }
+  int slot = 0;
+  for (int s = 0; s < mine; ++s) {
+    wait_stages<NI, DEPTH - 1>(mine - 1 - s);
+    asm volatile("" ::: "memory");
+    const half_t *sA = ring + slot * STEP_HALFS, *sB = sA + BM * BK;
+    half8_t fa[KS];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+      fa[ks] = *(const half8_t *)(sA + fr_row * BK + (((2 * ks + fr_kc) ^ swz(fr_row)) * 8));
+    if constexpr (WKN) {
+      const unsigned at =
+          (unsigned)(unsigned long long)(__attribute__((address_space(3))) const half_t *)sB + kn_at;
+      uint2_t w[KS][2];
+      kn_read_step<0>(w[0], at);
+      kn_read_step<1>(w[1], at);
+      kn_read_step<2>(w[2], at);
+      kn_read_step<3>(w[3], at);
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(lds_wait_operand<6>(w[0]), fa[0], acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(lds_wait_operand<4>(w[1]), fa[1], acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(lds_wait_operand<2>(w[2]), fa[2], acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(lds_wait_operand<0>(w[3]), fa[3], acc, 0, 0, 0);
+    } else {
+      half8_t fw[KS];
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+        fw[ks] = *(const half8_t *)(sB + fr_row * BK + (((2 * ks + fr_kc) ^ swz(fr_row + BM)) * 8));
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(fw[ks], fa[ks], acc, 0, 0, 0);
+    }
+    if (s + DEPTH < mine) {
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): the slot has been read
+      issue(s + DEPTH, slot);
+    }
+    if (++slot == DEPTH) slot = 0;
+  }
+
+  // fold: quad q of a wave's sums (columns 8 q + 4 (lane >> 5) .. + 3 of row lane & 31) lies at 1 KB q
+  // of its ring, 16 bytes per lane; wave q < 4 adds quad q over the waves and stores it
+  {
+    float4_t *own = (float4_t *)ring;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      own[q * 64 + lane] = float4_t{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
+  }
+  __syncthreads();
+  if (NW > 4 && wave >= 4) return;
+  float4_t v = ((const float4_t *)gemm_smem)[wave * 64 + lane];
+#pragma unroll
+  for (int w = 1; w < NW; ++w)
+    v += ((const float4_t *)(gemm_smem + w * DEPTH * STEP_HALFS))[wave * 64 + lane];
+  const int m = m0 + fr_row, n = n0 + wave * 8 + fr_kc * 4;
+  if (m >= M || n >= p.N) return;
+  if (EPI == kEpiPartial) {
+    *(float4_t *)(p.c32 + ((size_t)blockIdx.y * p.rows_cap + m) * p.N + n) = v;
+    return;
+  }
+  if (EPI == kEpiBiasGelu || EPI == kEpiQkvSplit || EPI == kEpiBias) {
+    const half4_t b = *(const half4_t *)(p.bias + n);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] += (float)b[e];
+  }
+  if (EPI == kEpiBiasGelu) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = gelu_tanh_f32(v[e]);
+  }
+  half_t *dst = EPI == kEpiQkvSplit ? p.c + ((size_t)(n >> 6) * p.rows_cap + m) * 64 + (n & 63)
+                                    : p.c + (size_t)m * p.N + n;
+  *(half4_t *)dst = half4_t{(half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3]};
+}
+#endif  // __HIP_DEVICE_COMPILE__
+
+template <int EPI, bool WKN>
+__global__ __launch_bounds__(kWaveKWaves * 64) void gemm_wave_k_kernel(GemmArgs p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  gemm_wave_k<EPI, WKN>(p);
+#endif
+}
+
 // ---- weight pre-pack: wt[n][k] = w[k][n] for up to four matrices in one launch ---
 struct TransposeJob {
   const half_t *w;
@@ -1021,6 +1212,27 @@ template <int BM, int BN, int STAGES, int WM, int WN, int NP, int SCHED, int EPI
 static int launch_gemm_tile(GemmArgs p, hipStream_t s, int splits = 1) {
   return p.w_kn ? launch_gemm_tile_as<BM, BN, STAGES, WM, WN, NP, SCHED, EPI, true>(p, s, splits)
                 : launch_gemm_tile_as<BM, BN, STAGES, WM, WN, NP, SCHED, EPI, false>(p, s, splits);
+}
+
+template <int EPI, bool WKN>
+static int launch_gemm_wave_k_as(GemmArgs p, hipStream_t s, int splits) {
+  // (and 256 bytes for the lengths of a launch that counts the mask rows)
+  constexpr size_t smem = (size_t)kWaveKWaves * kWaveKDepth * (32 + kWaveKCols) * kBK * sizeof(half_t) + 256;
+  static_assert(smem <= 160 * 1024, "LDS budget");
+  static std::atomic<bool> configured[kMaxDevices];
+  const int rc = allow_dynamic_lds(gemm_wave_k_kernel<EPI, WKN>, smem, configured,
+                                   "hipFuncSetAttribute(gemm_wave_k_kernel)");
+  if (rc != BT_OK) return rc;
+  p.tiles_n = (p.N + kWaveKCols - 1) / kWaveKCols;
+  p.tile_grid = ((p.rows_cap + 31) / 32 * p.tiles_n + 7) / 8 * 8;
+  gemm_wave_k_kernel<EPI, WKN><<<dim3(p.tile_grid, splits), kWaveKWaves * 64, smem, s>>>(p);
+  BT_CHECK_LAUNCH("gemm_wave_k_kernel");
+  return BT_OK;
+}
+
+template <int EPI>
+static int launch_gemm_wave_k(GemmArgs p, hipStream_t s, int splits = 1) {
+  return p.w_kn ? launch_gemm_wave_k_as<EPI, true>(p, s, splits) : launch_gemm_wave_k_as<EPI, false>(p, s, splits);
 }
 
 static int cu_count();
@@ -1172,6 +1384,12 @@ static bool tuned_mean(const LikelyRows &likely, int n, int k, int epi, int kn, 
   return true;
 }
 
+// Whether the tiles of gemm_wave_k fit one round: a workgroup fills its CU's LDS, so a second round
+// doubles the launch.
+static bool wave_k_fits(const GemmArgs &p, int splits) {
+  return (estimated_rows(p) + 31) / 32 * ((p.N + kWaveKCols - 1) / kWaveKCols) * splits <= cu_count();
+}
+
 template <int EPI>
 static int launch_gemm(GemmArgs p, hipStream_t s) {
   // Tile table (rows x cols, ring depth, computing wave grid, loader waves):
@@ -1195,6 +1413,9 @@ static int launch_gemm(GemmArgs p, hipStream_t s) {
   //  12: 128x192, 3, 2x2, 4   } memory-side cache, best of tiles 0-8 and now: FFN2 at 920 rows 17.0 ->
   //  13: 192x192, 2, 3x2, 4   } 13.0 us (9), at 2000 rows 20.6 -> 17.5 (10), at 5600 rows 35.6 -> 30.2
   //                           (12); QKV at 3600 rows 19.6 -> 18.6 (13), at 1300 rows 9.6 -> 9.1 (11)
+  //  14:  32x32, four waves over k (gemm_wave_k): in place of tile 4 while its workgroups fit one
+  //                           round (the rule measured both ways: 1 x 256 with the FFN2 in 384
+  //                           workgroups 509 us, with tile 4 there 456)
   // The choice minimises the time of the launch: for the weight shapes of BERT-base and BERT-large
   // by a table of measured times (gemm_tuned.inc) where it names a clearly faster tile, else by the
   // model of model_us().
@@ -1219,7 +1440,10 @@ static int launch_gemm(GemmArgs p, hipStream_t s) {
         choice = tuned;
     }
   }
+  if (forced < 0 && choice == 4 && wave_k_fits(p, 1)) choice = 14;
   switch (choice) {
+    case 14:
+      return launch_gemm_wave_k<EPI>(p, s);
     case 0:
       return launch_gemm_tile<256, 256, 2, 2, 4, 0, 1, EPI>(p, s);
     case 2:
@@ -1350,10 +1574,12 @@ extern "C" int bt_gemm_splitk(const void *a, const void *wt, void *partials, int
   GemmArgs p{(const half_t *)a, (const half_t *)wt, nullptr, nullptr, valid_rows, nullptr,
              rows_cap,          n,                  k,       0,       0,          (float *)partials,
              weight_kn};
-  // Small tiles only: splitting k is for launches whose k loop is the whole run time.  32 rows while
+  // Small tiles only: splitting k is for launches whose k loop is the whole run time.  Waves over k while
+  // their tiles fit one round (12 layers at 1 x 32 in all: -2.4 %), 32 rows while
   // one round of workgroups covers them all, then 64 (hidden 768, k 3072 in two splits with the
   // LayerNorm behind it: 320 rows 11.6 against 12.1 us, 400 rows 14.0 against 13.0).
   const long long rows = estimated_rows(p);
+  if (wave_k_fits(p, splits)) return launch_gemm_wave_k<kEpiPartial>(p, as_stream(stream), splits);
   if ((rows + 31) / 32 * ((n + 63) / 64) * splits <= 256)
     return launch_gemm_tile<32, 64, 4, 1, 2, 2, 0, kEpiPartial>(p, as_stream(stream), splits);
   return launch_gemm_tile<64, 64, 4, 2, 2, 4, 0, kEpiPartial>(p, as_stream(stream), splits);

@@ -393,8 +393,8 @@ extern "C" const char *bt_last_error_string(void) { return g_last_error.c_str();
 extern "C" int bt_set_option(const char *name, int value) {
   BT_REQUIRE(name, BT_ERR_INVALID_ARGUMENT, "bt_set_option: null name");
   if (!strcmp(name, "gemm_tile")) {
-    BT_REQUIRE(value >= -1 && value <= 13, BT_ERR_INVALID_ARGUMENT,
-               "bt_set_option: gemm_tile=%d outside [-1, 13]", value);
+    BT_REQUIRE(value >= -1 && value <= 14, BT_ERR_INVALID_ARGUMENT,
+               "bt_set_option: gemm_tile=%d outside [-1, 14]", value);
     g_gemm_tile.store(value);
   } else if (!strcmp(name, "ln_weight_copy")) {
     BT_REQUIRE(value == 0 || value == 1, BT_ERR_INVALID_ARGUMENT,

@@ -53,6 +53,7 @@ const char *bt_last_error_string(void);
  *                   | 6, 7, 8: tiles 2, 1, 0 as persistent workgroups (about one per CU, each
  *                   running one load pipeline over several tiles of its XCD's range) | 9: 64x64 | 10: 64x128
  *                   | 11: 96x128 | 12: 128x192 | 13: 192x192 (4 or 6 computing + 4 loader waves)
+ *                   | 14: 32x32, four waves that take the k-steps in turn
  *   "gemm_table_margin"  4 (default), 0..100: per cent by which a tile's measured time must beat
  *                   that of the cost model's choice before the measured table overrides the
  *                   model (100 = the model alone decides)

@@ -552,6 +552,73 @@ def test_gemm_mid_tiles_at_their_edges(device, tile, bm, bn, w_kn):
     assert torch.equal(got[0], got[1])
 
 
+@pytest.mark.parametrize("w_kn", [False, True])
+@pytest.mark.parametrize("k_steps", [1, 3, 4, 5, 12, 13, 27])
+def test_gemm_waves_over_k(device, k_steps, w_kn):
+    """The tile whose four waves take the k-steps in turn: fewer steps than waves, rings that are reused and not,
+    rows and columns at and around the tile's edges, all epilogues, against float64.  One fp16 rounding of the result
+    and fp32 sums in four parts."""
+    _say("gemm waves over k", k_steps, w_kn)
+    rs = np.random.RandomState(k_steps)
+    K = 64 * k_steps
+    for M, N in ((1, 8), (31, 24), (32, 32), (33, 40), (64, 72), (97, 264)):
+        rows = M + 3
+        a = rs.standard_normal((rows, K)).astype(np.float16)
+        w = (rs.standard_normal((K, N)) * 0.05).astype(np.float16)
+        exp = a[:M].astype(np.float64) @ w.astype(np.float64)
+        tol = _gemm_tol(exp, K, np.abs(a).max(), np.abs(w).max())
+        wd = _dev(w, device) if w_kn else _dev(np.ascontiguousarray(w.T), device)
+        bias = rs.standard_normal(N).astype(np.float16)
+        vr = torch.tensor([M], dtype=torch.int32, device=device)
+        out = torch.full((2, rows, N), 3.0, dtype=torch.float16, device=device)
+        ops.set_option("gemm_tile", 14)
+        try:
+            ops.gemm(_dev(a, device), wd, valid_rows=vr, out=out[0], w_kn=w_kn)
+            ops.gemm_bias_gelu(_dev(a, device), wd, _dev(bias, device), valid_rows=vr, out=out[1], w_kn=w_kn)
+        finally:
+            ops.set_option("gemm_tile", -1)
+        got = out.cpu().numpy().astype(np.float64)
+        assert np.all(np.abs(got[0, :M] - exp) <= tol), (M, N)
+        x = exp + bias
+        gelu = x / (1 + np.exp(-2 * 0.7978845608028654 * (x + 0.044715 * x ** 3)))
+        # (the slope of GELU is below 1.13)
+        assert np.all(np.abs(got[1, :M] - gelu) <= 1.13 * tol + 2.0 ** -10 * np.abs(gelu) + 1e-5), (M, N)
+        assert np.all(got[:, M:] == 3.0)
+
+
+@pytest.mark.parametrize("w_kn", [False, True])
+@pytest.mark.parametrize("heads,size", [(1, 64), (3, 64), (2, 96)])
+def test_gemm_waves_over_k_qkv(device, heads, size, w_kn):
+    """The same tile under the QKV product, rows gathered and rows counted from the mask: as tile 1 computes them, up
+    to the order of the fp32 sums."""
+    _say("gemm waves over k, qkv", heads, size, w_kn)
+    rs = np.random.RandomState(heads * size)
+    H, B, S = heads * size, 3, 37
+    x = rs.standard_normal((B * S, H)).astype(np.float16)
+    w = (rs.standard_normal((H, 3 * H)) * 0.05).astype(np.float16)
+    wd = _dev(w, device) if w_kn else _dev(np.ascontiguousarray(w.T), device)
+    bias = _dev(rs.standard_normal(3 * H).astype(np.float16), device)
+    lens = [37, 1, 22]
+    mask = np.zeros((B, S, S), np.float16)
+    for b, n in enumerate(lens):
+        mask[b, :, :n] = 1
+    got = []
+    for t in (14, 1):
+        ops.set_option("gemm_tile", t)
+        try:
+            r = ops.gemm_qkv_bias_split_mask_rows(_dev(x, device), _dev(mask, device), wd, bias, heads, size, w_kn=w_kn)
+        finally:
+            ops.set_option("gemm_tile", -1)
+        got.append([v.cpu().numpy() for v in r])
+    live = sum(lens)
+    flat = [g[0].reshape(3, heads, B * S, 64)[:, :, :live] if size == 64 else g[0].reshape(B * S, 3 * H)[:live]
+            for g in got]
+    tol = 2 * _gemm_tol(flat[1].astype(np.float64), H, np.abs(x).max(), np.abs(w).max())
+    assert np.all(np.abs(flat[0].astype(np.float64) - flat[1].astype(np.float64)) <= tol)
+    for one, other in zip(got[0][1:], got[1][1:]):
+        assert np.array_equal(one, other)
+
+
 @pytest.mark.parametrize("tile", [0, 1, 2, 3, 4, 5, 6, 7, 8])
 def test_gemm_bias_gelu(device, tile):
     _say("gemm_bias_gelu", tile)
