@@ -97,10 +97,13 @@ inline int plan_weight_copies(long long live, long long padded_rows, int hidden,
   const int epilogue[4] = {split_heads ? BT_EPILOGUE_QKV_SPLIT : -1, BT_EPILOGUE_PLAIN,
                            BT_EPILOGUE_BIAS_GELU, BT_EPILOGUE_PLAIN};
   float gain[4] = {0.f, 0.f, 0.f, 0.f}, early = 0.f, total = 0.f;
-  bool want[4];
+  bool want[4], want_ln[4];
   for (int i = 0; i < 4; ++i) {
     if (epilogue[i] >= 0) gain[i] = bt_gemm_prepack_gain_us(live, n[i], k[i], epilogue[i]);
     want[i] = gain[i] > 1.0f;
+    // (the table's gain is less the 0.5 us per megabyte that a copy costs the prologue; the LayerNorm's
+    // launch makes one for half of that: 6.7 us without and 7.8 us with FFN1's 4.7 MB at batch 16 x 512)
+    want_ln[i] = gain[i] + 0.25e-6f * (float)n[i] * (float)k[i] * 2.f > 1.0f;
     if (want[i]) total += gain[i];
     if (want[i] && i < 2) early += gain[i];
   }
@@ -114,7 +117,7 @@ inline int plan_weight_copies(long long live, long long padded_rows, int hidden,
     // (measured where the table's gain is smallest, 1.5 us for FFN1 at batch 16 x 512: kernel time
     // -1 % per forward, wall time -0.5 % on one box and +0.6 % on another; with 4.5 us at
     // 16 x 1024, where the copy also replaces the prologue, -2 %)
-    ln_copy[i] = !prologue && ln_can_copy && i >= 2 && want[i];
+    ln_copy[i] = !prologue && ln_can_copy && i >= 2 && want_ln[i];
     count += copy[i];
   }
   return count;
