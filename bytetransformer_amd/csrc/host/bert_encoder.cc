@@ -79,7 +79,7 @@ void BertEncoder<OpType>::infer(BertEncoderInferParam<DataType_> ip) {
                                    is_remove_padding_ ? 0 : 1, 0, nullptr, nullptr, nullptr,
                                    nullptr, 0, nullptr, nullptr, stream));
   const int *valid_rows = is_remove_padding_ ? et_param.batch_idx + batch_size : nullptr;
-  const int rows_hint = ip.valid_rows_hint;
+  const int rows_hint = rows_to_plan_for(ip.valid_rows_hint, is_remove_padding_, batch_size, rows);
   const int L = (int)layers_.size();
 
   for (int l = 0; l < L; ++l) {

@@ -217,6 +217,7 @@ void BertTransformer<OpType>::bert_infer(BertTransformerInferParam infer_param) 
     transformer_out = inner_buf;  // FFN2 output reuses the dead qkv region
     valid_rows = et_param.batch_idx + batch_size;
     if (have_offsets && rows_hint > 0 && rows_hint < rows) packed_cap = rows_hint;
+    rows_hint = rows_to_plan_for(rows_hint, true, batch_size, rows);
   }
 
   if constexpr (OpType == OperationType::FP32) {

@@ -1336,6 +1336,29 @@ struct TileModel {
   float shared_us;           // > 0: one k-step's share of a CU that several tiles occupy
 };
 
+// Fitted to the table's measurements: on average the choice is 1.2 % slower than the fastest
+// tile, and 7 % or more in one case of twenty.
+static const TileModel kTileModels[] = {
+    {0, 256, 256, 1.45f, 5.7f, 0.f},     {13, 192, 192, 0.95f, 4.7f, 0.f},  {3, 256, 192, 1.10f, 4.35f, 0.f},
+    {12, 128, 192, 0.64f, 4.6f, 0.f},    {2, 256, 128, 0.79f, 4.4f, 0.f},   {1, 128, 128, 0.467f, 3.4f, 0.f},
+    {5, 128, 128, 0.66f, 3.6f, 0.70f},   {11, 96, 128, 0.41f, 3.0f, 0.f},   {10, 64, 128, 0.267f, 2.67f, 0.43f},
+    {9, 64, 64, 0.20f, 2.63f, 0.265f},   {4, 32, 64, 0.175f, 2.75f, 0.19f}};
+
+// Workgroups that count the mask rows first (bt_gemm_qkv_bias_split_mask_rows) do so once per tile in
+// every tile but the persistent ones: each round past the first pays for it.  Batch 16 x 1024, hidden
+// 768: 256x192 in two rounds 40.8 us by the table, which counts no mask, and 51.5 in the layer;
+// persistent 256x128 43.2 and 47.9.
+constexpr float kMaskRoundUs = 3.f;
+static float mask_rounds_us(int id, long long m, int n) {
+  for (const TileModel &c : kTileModels) {
+    if (c.id != id) continue;
+    const long long tiles = ((m + c.bm - 1) / c.bm) * ((n + c.bn - 1) / c.bn);
+    const long long at_once = (long long)cu_count() * (c.shared_us > 0.f ? 2 : 1);
+    return tiles > at_once ? kMaskRoundUs * (float)((tiles - 1) / at_once) : 0.f;
+  }
+  return 0.f;   // a persistent form
+}
+
 // Time of one launch of n columns and k reduction: fixed + k-steps x step time, where a step takes
 // `step_us` while every CU has one tile at most and then grows in whole rounds or, where several
 // workgroups share a CU, with its load.
@@ -1350,20 +1373,13 @@ static float model_us(const TileModel &c, long long m, int n, int k) {
   return (float)((tiles + cus - 1) / cus) * (nk * c.step_us + c.fixed_us - 1.8f) + 1.8f;
 }
 
-static int fastest_by_model(const LikelyRows &likely, int n, int k) {
-  // (fitted to the table's measurements: on average the choice is 1.2 % slower than the fastest
-  // tile, and 7 % or more in one case of twenty)
-  static const TileModel models[] = {{0, 256, 256, 1.45f, 5.7f, 0.f},   {13, 192, 192, 0.95f, 4.7f, 0.f},
-                                     {3, 256, 192, 1.10f, 4.35f, 0.f},  {12, 128, 192, 0.64f, 4.6f, 0.f},
-                                     {2, 256, 128, 0.79f, 4.4f, 0.f},   {1, 128, 128, 0.467f, 3.4f, 0.f},
-                                     {5, 128, 128, 0.66f, 3.6f, 0.70f}, {11, 96, 128, 0.41f, 3.0f, 0.f},
-                                     {10, 64, 128, 0.267f, 2.67f, 0.43f}, {9, 64, 64, 0.20f, 2.63f, 0.265f},
-                                     {4, 32, 64, 0.175f, 2.75f, 0.19f}};
+static int fastest_by_model(const LikelyRows &likely, int n, int k, bool mask) {
   int best_id = 0;
   float best = 0.f;
-  for (const TileModel &c : models) {
+  for (const TileModel &c : kTileModels) {
     float t = 0.f;
-    for (int i = 0; i < likely.count; ++i) t += likely.weight[i] * model_us(c, likely.rows[i], n, k);
+    for (int i = 0; i < likely.count; ++i)
+      t += likely.weight[i] * (model_us(c, likely.rows[i], n, k) + (mask ? mask_rounds_us(c.id, likely.rows[i], n) : 0.f));
     if (best == 0.f || t < best) {
       best = t;
       best_id = c.id;
@@ -1424,13 +1440,17 @@ static int launch_gemm(GemmArgs p, hipStream_t s) {
   if (choice < 0) {
     const LikelyRows likely(p);
     float us[kTunedTiles];
-    choice = fastest_by_model(likely, p.N, p.K);
+    choice = fastest_by_model(likely, p.N, p.K, p.mask != nullptr);
     // the table overrides the model only for a clear win: the timings come from a loop
     // of identical launches, and differences of a few per cent do not carry over to the
     // layer sequence
     // (a launch whose estimated live rows fill its capacity to within one tile row is looked
     // up among the all-live measurements)
     if (tuned_mean(likely, p.N, p.K, EPI, p.w_kn, estimated_rows(p) + kTunedStep > p.rows_cap, us)) {
+      if (p.mask)
+        for (int t = 0; t < kTunedTiles; ++t)
+          for (int i = 0; us[t] > 0.f && i < likely.count; ++i)
+            us[t] += likely.weight[i] * mask_rounds_us(t, likely.rows[i], p.N);
       int tuned = -1;
       for (int t = 0; t < kTunedTiles; ++t)
         if (us[t] > 0.f && (tuned < 0 || us[t] < us[tuned])) tuned = t;

@@ -15,11 +15,12 @@ import sys
 
 M_STEP = 256                     # the tallest tile: run time steps with the count of row tiles
 M_GRID = (tuple(range(64, 1024, 64)) + tuple(range(1024, 2560, 128)) + tuple(range(2560, 8192, M_STEP))
-          + tuple(range(8192, 12288 + 1, 512)))
+          + tuple(range(8192, 16384 + 1, 512)))
 HIDDEN = (768, 1024)
 TILES = tuple(range(14))
 EPI_CODE = {"plain": 0, "gelu": 1, "qkv": 2}     # enum Epilogue of gemm.hip
 SMALL_TILE_MAX_ROWS = 3000      # the 32x64 and 64x64 tiles are not worth timing beyond this
+MID_TILE_MAX_ROWS = 12288       # nor tiles 10 to 13 beyond this
 LARGE_TILE_MIN_ROWS = 512       # nor the 192- and 256-row tiles below this
 INC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc", "kernels", "gemm_tuned.inc")
 
@@ -107,6 +108,8 @@ def measure(iters=32):
                         us = {}
                         for tile in TILES:
                             if tile in (4, 9) and m > SMALL_TILE_MAX_ROWS:
+                                continue
+                            if tile in (10, 11, 12, 13) and m > MID_TILE_MAX_ROWS:
                                 continue
                             if tile in (0, 2, 3, 6, 8, 13) and m < LARGE_TILE_MIN_ROWS:
                                 continue
