@@ -15,7 +15,8 @@ import sys
 
 M_STEP = 256                     # the tallest tile: run time steps with the count of row tiles
 M_GRID = (tuple(range(64, 1024, 64)) + tuple(range(1024, 2560, 128)) + tuple(range(2560, 8192, M_STEP))
-          + tuple(range(8192, 16384 + 1, 512)))
+          + tuple(range(8192, 12288, 512))
+          + tuple(range(12288, 16384 + 1, 1024)))
 HIDDEN = (768, 1024)
 TILES = tuple(range(14))
 EPI_CODE = {"plain": 0, "gelu": 1, "qkv": 2}     # enum Epilogue of gemm.hip
@@ -164,7 +165,7 @@ def write_inc(rows, path=INC):
         lines.append("    {%d, %d, %d, %d, %d, {" % (n, k, epi, kn, full))
         for m in M_GRID:
             us = by_m.get(m, {})
-            lines.append("        {%s},   // %d rows" % (
+            lines.append("  {%s},   // %d rows" % (
                 ", ".join("%.2ff" % us.get(str(t), 0.0) for t in TILES), m))
         lines.append("    }},")
     lines.append("};")
