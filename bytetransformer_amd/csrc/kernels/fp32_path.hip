@@ -44,7 +44,9 @@ __device__ __forceinline__ float gelu_tanh(float x) {
 // ---------------------------------------------------------------------------
 // A float has 24 significand bits, three bfloat16 have 3 x 8: x = h + m + l exactly, with
 // h = bf16(x), m = bf16(x - h), l = bf16(x - h - m) (round to nearest, so |m| <= 2^-9 |x| and
-// |l| <= 2^-18 |x|; both differences are exact).  A product of two floats is then nine bf16
+// |l| <= 2^-18 |x|; both differences are exact).  That holds from 2^-110 on, where l is a multiple of
+// the smallest bfloat16, 2^-133, up to the largest bfloat16; F32SumRange says what happens beyond.
+// A product of two floats is then nine bf16
 // products, each exact in the MFMA's float accumulator; the three smallest (m l, l m, l l: at most
 // 2^-26 of the product) are below the rounding of a float product and are left out.  Six
 // v_mfma_f32_32x32x16_bf16 do in 192 clocks what eight v_mfma_f32_32x32x2_f32 do in 512.
@@ -118,6 +120,45 @@ __device__ __forceinline__ void f32_wait_vmcnt() {
   __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0F70);
 }
 
+// Where the split above does not hold, the sum shows it:
+//   * an infinity, or a float past the largest bfloat16 (3.39e38), is no sum of three bfloat16: x - h is
+//     inf - inf, and every sum that it enters comes out as NaN.  A product may also pass through an
+//     infinity on the way to a finite sum.  A sum that is not finite is formed again.
+//   * an operand below 2^-110 is taken to the nearest multiple of 2^-133.  Beside a sum of 2^-60 or more
+//     that is lost in float's own rounding unless the other operand is above 2^38; a smaller sum is
+//     formed again, except zero (rows of zeros are ordinary: padding).
+// "Again" means from the floats themselves by float multiply-adds, whatever float arithmetic makes of
+// them.  A launch that has such sums pays a chain of K for each.
+// (By the bits without the sign, gathered over all the sums of a lane: 12 layers at batch 16 x 256 take
+// 0.5 % longer than without the check, and 1.2 % longer with a branch for each sum.)
+struct F32SumRange {
+  unsigned largest = 0, smallest = ~0u;   // of 2 |bits|, and of 2 |bits| - 1: zero wraps to the top
+  __device__ __forceinline__ void add(float x) {
+    const unsigned twice = __builtin_bit_cast(unsigned, x) << 1;
+    largest = max(largest, twice);
+    smallest = min(smallest, twice - 1);
+  }
+  __device__ __forceinline__ bool split_held() const {
+    constexpr unsigned kInf = 0x7f800000u << 1, kTiny = (127u - 60) << 24;   // of infinity and of 2^-60
+    return largest < kInf && smallest >= kTiny - 1;
+  }
+};
+template <int V>   // one column, or four neighbouring ones
+__device__ __forceinline__ void f32_dot_again(const float *a_row, const float *w, int K, int N, float (&sum)[V]) {
+#pragma unroll
+  for (int v = 0; v < V; ++v) sum[v] = 0.f;
+  for (int k = 0; k < K; k += 4) {
+    const float4_t a = *(const float4_t *)(a_row + k);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int v = 0; v < V; ++v) sum[v] = __builtin_fmaf(a[e], w[(size_t)(k + e) * N + v], sum[v]);
+  }
+}
+__device__ __forceinline__ const float *f32_a_row(const F32GemmArgs &p, int m) {
+  return p.a + (size_t)(p.a_row_index ? p.a_row_index[m] : m) * p.K;
+}
+
 // Store of one 32x32 block: accumulator element i is row 8*(i/4) + 4*half + i%4, column l32.
 __device__ __forceinline__ void f32_store_block(const F32GemmArgs &p, const float16_t &acc, int m0,
                                                 int n0, int M, int l32, int half) {
@@ -128,7 +169,11 @@ __device__ __forceinline__ void f32_store_block(const F32GemmArgs &p, const floa
   for (int i = 0; i < 16; ++i) {
     const int row = m0 + 8 * (i >> 2) + 4 * half + (i & 3);
     if (row >= M) continue;
-    float v = acc[i] + bv;
+    float sum[1] = {acc[i]};
+    F32SumRange range;
+    range.add(sum[0]);
+    if (!range.split_held()) f32_dot_again(f32_a_row(p, row), p.w + col, p.K, p.N, sum);
+    float v = sum[0] + bv;
     if (p.gelu) v = gelu_tanh(v);
     p.c[(size_t)row * p.N + col] = v;
   }
@@ -339,22 +384,47 @@ __device__ __forceinline__ void f32_gemm_tile(const F32GemmArgs &p) {
   __syncthreads();
   constexpr int LPR = TN / 4;            // lanes per row, four columns each
   constexpr int RPP = 64 / LPR;          // rows per pass of a wave
+  constexpr int PASSES = TM / (RPP * NW);
+  static_assert(TM % (RPP * NW) == 0, "whole passes over the rows of a tile");
+  const int row0 = wave * RPP + lane / LPR, c = 4 * (lane % LPR);
+  float4_t v[PASSES];
+  F32SumRange range;
 #pragma unroll
-  for (int r0 = 0; r0 < TM; r0 += RPP * NW) {
-    const int row = r0 + wave * RPP + lane / LPR, c = 4 * (lane % LPR);
-    if (TM % (RPP * NW) != 0 && row >= TM) continue;
+  for (int i = 0; i < PASSES; ++i) {
+    const int row = row0 + i * RPP * NW;
     const float *src = f32_smem + row * TN + (c ^ (XR * ((row >> 2) & 1)));
-    float4_t v = *(const float4_t *)src;
+    v[i] = *(const float4_t *)src;
 #pragma unroll
-    for (int w = 1; w < NW; ++w) v += *(const float4_t *)(src + w * REGION);
-    const int m = m0 + row, n = n0 + c;
+    for (int w = 1; w < NW; ++w) v[i] += *(const float4_t *)(src + w * REGION);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) range.add(v[i][e]);
+  }
+  const int n = n0 + c;
+  if (!range.split_held()) {
+#pragma unroll
+    for (int i = 0; i < PASSES; ++i) {
+      const int m = m0 + row0 + i * RPP * NW;
+      if (m >= M || n >= p.N) continue;
+      float sum[4];
+      f32_dot_again(f32_a_row(p, m), p.w + n, p.K, p.N, sum);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        F32SumRange one;
+        one.add(v[i][e]);
+        if (!one.split_held()) v[i][e] = sum[e];
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < PASSES; ++i) {
+    const int m = m0 + row0 + i * RPP * NW;
     if (m >= M || n >= p.N) continue;
-    if (p.bias) v += float4_t{p.bias[n], p.bias[n + 1], p.bias[n + 2], p.bias[n + 3]};
+    if (p.bias) v[i] += float4_t{p.bias[n], p.bias[n + 1], p.bias[n + 2], p.bias[n + 3]};
     if (p.gelu) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = gelu_tanh(v[e]);
+      for (int e = 0; e < 4; ++e) v[i][e] = gelu_tanh(v[i][e]);
     }
-    *(float4_t *)(p.c + (size_t)m * p.N + n) = v;
+    *(float4_t *)(p.c + (size_t)m * p.N + n) = v[i];
   }
 }
 #endif

@@ -443,9 +443,15 @@ int bt_splitk_layernorm(const void *partials, int splits, const void *residual,
  * ---- OperationType::FP32 ------------------------------------------------------
  * The float flavour of the layer: every tensor (activations, weights, biases, gamma,
  * beta, mask, attention bias) is float, and so are the accumulators of the products.  Weights are
- * read as the caller stores them ([K, N] row-major): there is no pre-pack.  Inside the products a float is the exact sum of three bfloat16
- * (24 significand bits) and the matrix cores multiply those, float accumulators: the results are
- * at least as close to the exact product as v_mfma_f32_32x32x2_f32 brings them.
+ * read as the caller stores them ([K, N] row-major): there is no pre-pack.  Inside the products a
+ * float is the sum of three bfloat16 (24 significand bits, exact from 2^-110 to 3.39e38) and the
+ * matrix cores multiply those into float accumulators, without the three smallest of the nine partial
+ * products (2^-26 of the product): the results are at least as close to the exact product as
+ * v_mfma_f32_32x32x2_f32 brings them.  Beyond that range: a sum that comes out infinite, NaN or
+ * non-zero below 2^-60 is formed again by float multiply-adds, so infinities, NaN and operands near
+ * the ends of the float range give what float arithmetic gives.  What remains of the split there is
+ * an operand below 2^-110 that meets one above 2^38, or that vanishes (below 2^-134) in a sum of zero:
+ * an absolute error of up to 2^-134 times the other operand.
  *
  * bt_gemm_f32: c[M, n] = a[M, k] . w[k, n] (+ bias[n]) (then tanh-GELU when gelu != 0,
  * which needs a bias).  a_row_index (nullable, needs valid_rows): row r of A is

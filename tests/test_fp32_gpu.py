@@ -99,6 +99,51 @@ def test_gemm_f32_every_tile_at_its_edges(device, tile, rows, M, N, K):
     assert np.all(g[M:] == 7.0)
 
 
+@pytest.mark.parametrize("tile", [0, 1, 2, 3])
+def test_gemm_f32_at_the_ends_of_the_float_range(device, tile):
+    """The bfloat16 triples hold a float between 2^-110 and the largest bfloat16: infinities, NaN, floats past that
+    and sums of tiny operands must come out as float arithmetic has them, and rows without any as before."""
+    rs = np.random.RandomState(tile)
+    rows, N, K = 70, 68, 52
+    a = rs.standard_normal((rows, K)).astype(np.float32)
+    w = (rs.standard_normal((K, N)) * 0.1 + 0.01).astype(np.float32)
+    top = np.float32(3.4e38)               # a float, but rounds to an infinite bfloat16
+    a[3, 5], a[4, 0], a[5, 51] = np.inf, -np.inf, np.nan
+    a[6, :] = 0
+    a[6, 7] = top
+    a[7, 2], a[7, 9] = np.inf, -np.inf     # NaN wherever both weights have one sign
+    a[8, :], a[9, :] = a[8, :] * np.float32(1e-35), a[9, :] * np.float32(1e-38)
+    a[10, :] = a[10, :] * np.float32(2.0 ** -60)
+    a[65, :] = a[65, :] * np.float32(1e-30)
+    a[66, :] = 0
+    w[7, 64] = 0                           # 0 * inf
+    w[:, 65] = w[:, 65] * np.float32(2.0 ** -60)
+    w[11, 66] = np.inf
+    w[11, 67] = -top
+    with np.errstate(invalid="ignore", over="ignore"):
+        a64, w64 = a.astype(np.float64), w.astype(np.float64)
+        exp = a64 @ w64
+        exp[np.abs(exp) > np.finfo(np.float32).max] *= np.inf
+        # a float accumulator, and denormal products and sums: half of float's smallest step each
+        bound = 2.0 ** -24 * (2 + math.sqrt(K)) * (np.abs(a64) @ np.abs(w64)) + 2 * K * 2.0 ** -150
+    ops.set_option("f32_gemm_tile", tile)
+    try:
+        g = ops.gemm_f32(_dev(a, device), _dev(w, device)).cpu().numpy().astype(np.float64)
+    finally:
+        ops.set_option("f32_gemm_tile", -1)
+    # (a product of more than 3.4e38 on the way to a smaller sum may or may not overflow: leave such sums out)
+    with np.errstate(invalid="ignore", over="ignore"):
+        near = np.nan_to_num(np.abs(a64) @ np.abs(w64), nan=0.0, posinf=0.0) > 3e38
+    special = ~np.isfinite(exp)
+    assert special[3:6].all() and special[7].all() and special[:, 66].all() and np.isfinite(exp[6, :66]).all()
+    assert np.array_equal(g[special & ~near], exp[special & ~near], equal_nan=True)
+    usual = ~special & ~near
+    assert usual[8:11].sum() > 100 and usual[6, :66].all()
+    err = np.abs(g[usual] - exp[usual])
+    assert np.all(err <= bound[usual]), (err / bound[usual]).max()
+    assert np.all(g[66, :66] == 0)
+
+
 def test_gemm_f32_bias_gelu_and_gather(device):
     _say("gemm_f32 gelu + gather")
     rs = np.random.RandomState(11)
