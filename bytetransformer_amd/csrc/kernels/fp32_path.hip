@@ -108,12 +108,18 @@ struct F32GemmArgs {
 };
 
 constexpr int kF32CUs = 256;
-// Extent of a buffer descriptor: at most 4 GiB - 1 (larger operands take the skinny kernel's
-// 64-bit addresses).
-__host__ __device__ inline unsigned f32_buffer_bytes(size_t floats) {
-  return floats * 4 > 0xffffffffull ? 0xffffffffu : (unsigned)(floats * 4);
-}
+constexpr unsigned kF32MaxBytes = 0xffff0000u;   // the largest range that a tile addresses from one base
 constexpr unsigned kF32Outside = 0xfffffff0u;   // an offset outside every descriptor: reads as zero
+// Largest value over the 64 lanes (values >= 0), wave-uniform: the steps of wave_inclusive_sum.
+__device__ __forceinline__ int wave_largest(int v) {
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false));
+  return __builtin_amdgcn_readlane(v, 63);
+}
 template <int N>
 __device__ __forceinline__ void f32_wait_vmcnt() {
   static_assert(N >= 0 && N < 64, "vmcnt range");
@@ -224,21 +230,30 @@ __device__ __forceinline__ void f32_gemm_tile(const F32GemmArgs &p) {
   float *ring = f32_smem + wave * REGION;
 
   const int nk = (p.K + 15) >> 4;
-  const int mine = (nk - wave + NW - 1) / NW;   // slices wave, wave + NW, ...
-  const auto rs_a = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<float *>(p.a_row_index ? p.a : p.a + (size_t)m0 * p.K), 0,
-      (int)f32_buffer_bytes(((size_t)p.rows_cap - (p.a_row_index ? 0 : m0)) * p.K), 0x00020000);
+  // The rows of A that this tile reads: [first, first + span), at most a descriptor's worth of them.
+  // Gathered rows may lie anywhere in an operand whose extent nobody names, so the range comes from the
+  // tile's own indices; where they lie further apart (4 GiB), every sum is formed by f32_dot_again.
+  int first = m0, span = min(TM, M - m0), index = 0;
+  bool far = false;
+  if (p.a_row_index) {
+    index = p.a_row_index[min(m0 + (lane & (TM - 1)), M - 1)];
+    first = 0x7fffffff - wave_largest(0x7fffffff - index);
+    span = wave_largest(index) - first + 1;
+    far = (unsigned long long)span * p.K * 4 > kF32MaxBytes;
+  }
+  const int mine = far ? 0 : (nk - wave + NW - 1) / NW;   // slices wave, wave + NW, ...
+  const auto rs_a = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p.a + (size_t)first * p.K), 0,
+                                                      (int)((unsigned)span * (unsigned)p.K * 4u), 0x00020000);
   const auto rs_w = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<float *>(p.w), 0, (int)f32_buffer_bytes((size_t)p.K * p.N), 0x00020000);
+      const_cast<float *>(p.w), 0, (int)((unsigned)p.K * (unsigned)p.N * 4u), 0x00020000);
   // byte offsets of this lane's pieces at k = 0.  Rows past M repeat the last live row, columns
   // past N lie outside the descriptor (they read as zero); neither is stored.
   unsigned aoff[NIA], woff[NIW];
 #pragma unroll
   for (int i = 0; i < NIA; ++i) {
     const int row = i * 16 + (lane >> 2), chunk = (lane & 3) ^ ((row >> 2) & 3);
-    const int r = min(m0 + row, M - 1);
-    const unsigned src = p.a_row_index ? (unsigned)p.a_row_index[r] : (unsigned)(r - m0);
-    aoff[i] = (src * (unsigned)p.K + 4 * chunk) * 4u;
+    const int src = p.a_row_index ? __shfl(index, row, 64) : min(m0 + row, M - 1);
+    aoff[i] = ((unsigned)(src - first) * (unsigned)p.K + 4 * chunk) * 4u;
   }
 #pragma unroll
   for (int i = 0; i < NIW; ++i) {
@@ -400,7 +415,7 @@ __device__ __forceinline__ void f32_gemm_tile(const F32GemmArgs &p) {
     for (int e = 0; e < 4; ++e) range.add(v[i][e]);
   }
   const int n = n0 + c;
-  if (!range.split_held()) {
+  if (far || !range.split_held()) {
 #pragma unroll
     for (int i = 0; i < PASSES; ++i) {
       const int m = m0 + row0 + i * RPP * NW;
@@ -411,7 +426,7 @@ __device__ __forceinline__ void f32_gemm_tile(const F32GemmArgs &p) {
       for (int e = 0; e < 4; ++e) {
         F32SumRange one;
         one.add(v[i][e]);
-        if (!one.split_held()) v[i][e] = sum[e];
+        if (far || !one.split_held()) v[i][e] = sum[e];
       }
     }
   }
@@ -906,10 +921,8 @@ extern "C" int bt_gemm_f32(const void *a, const int *a_row_index, const void *w,
       }
     }
   }
-  // the tiled kernels address gathered rows and the weight with 32-bit byte offsets
-  if ((a_row_index && (long long)rows_cap * k * 4 > 0xffff0000ll) || (long long)n * k * 4 > 0xffff0000ll ||
-      (long long)k * 256 > 0xffff0000ll)
-    tile = 3;
+  // the tiled kernels address the weight, and the rows of a tile, with 32-bit byte offsets
+  if ((long long)n * k * 4 > kF32MaxBytes || (long long)k * 256 > kF32MaxBytes) tile = 3;
   hipStream_t s = as_stream(stream);
   int rc = BT_OK;
   if (tile == 0) {

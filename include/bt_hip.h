@@ -455,7 +455,8 @@ int bt_splitk_layernorm(const void *partials, int splits, const void *residual,
  *
  * bt_gemm_f32: c[M, n] = a[M, k] . w[k, n] (+ bias[n]) (then tanh-GELU when gelu != 0,
  * which needs a bias).  a_row_index (nullable, needs valid_rows): row r of A is
- * a[a_row_index[r], :].  rows_hint: expected live rows or 0, steers the tile shape only.
+ * a[a_row_index[r], :], any row of A (rows_cap bounds c and the live rows, not A).  rows_hint:
+ * expected live rows or 0, steers the tile shape only.
  * n % 4 == 0, k % 4 == 0.  Replaces the cuBLAS calls of
  * dense_layer_kernel_launcher<float> (bytetransformer/src/gemm.cu:32-39), the QKV bias
  * add of add_QKV_bias (attention_nofused_utils.cu:143-184) and

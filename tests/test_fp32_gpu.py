@@ -100,6 +100,34 @@ def test_gemm_f32_every_tile_at_its_edges(device, tile, rows, M, N, K):
 
 
 @pytest.mark.parametrize("tile", [0, 1, 2, 3])
+@pytest.mark.parametrize("rows,M,K", [(100, 20, 36), (5000, 70, 64), (1200000, 40, 1024)])
+def test_gemm_f32_gathers_any_row_of_a(device, tile, rows, M, K):
+    """rows_cap bounds the output and not the operand that the rows are gathered from: rows past it, and (the last
+    shape) rows of one tile more than 4 GiB apart."""
+    _say("gemm_f32 gather", tile, rows, M, K)
+    rs = np.random.RandomState(M + tile)
+    N = 72
+    index = np.concatenate([[rows - 1, 0, rows // 2], rs.permutation(rows)[:M - 3]]).astype(np.int32)
+    if K == 1024:                                       # (only the rows that are read are filled)
+        index[:] = np.where(np.arange(M) % 2, np.arange(M), rows - 1 - np.arange(M))
+    live = rs.standard_normal((M, K)).astype(np.float32)
+    a = torch.empty(rows, K, dtype=torch.float32, device=device)
+    a[torch.from_numpy(index.astype(np.int64)).to(device)] = _dev(live, device)
+    live = a[torch.from_numpy(index.astype(np.int64)).to(device)].cpu().numpy()   # (an index may come twice)
+    w = (rs.standard_normal((K, N)) * 0.1).astype(np.float32)
+    exp = O.gemm(live.astype(np.float64), w.astype(np.float64))
+    bound = 2.0 ** -24 * (2 + math.sqrt(K)) * (np.abs(live).astype(np.float64) @ np.abs(w))
+    ops.set_option("f32_gemm_tile", tile)
+    try:
+        g = ops.gemm_f32(a, _dev(w, device), valid_rows=torch.tensor([M], dtype=torch.int32, device=device),
+                         a_row_index=_dev(index, device), rows_cap=M).cpu().numpy()
+    finally:
+        ops.set_option("f32_gemm_tile", -1)
+    assert g.shape == (M, N)
+    assert np.all(np.abs(g - exp) <= bound), (np.abs(g - exp) / bound).max()
+
+
+@pytest.mark.parametrize("tile", [0, 1, 2, 3])
 def test_gemm_f32_at_the_ends_of_the_float_range(device, tile):
     """The bfloat16 triples hold a float between 2^-110 and the largest bfloat16: infinities, NaN, floats past that
     and sums of tiny operands must come out as float arithmetic has them, and rows without any as before."""
