@@ -820,11 +820,12 @@ static void launch_grouped(const AttArgs &a, bool wide, int seq_len, unsigned gr
   constexpr int kWideStages = KIND == kAddNone ? 3 : 2;
   // eight waves over two key halves: pays for a few long sequences that leave most CUs
   // with one workgroup or none (batch 1 x 1024: 9.9 -> 8.7 us); with several workgroups
-  // per CU the four-wave form is faster (batch 16 x 512: 16.3 against 19.6 us)
+  // per CU the four-wave form is faster (batch 16 x 512: 16.3 against 19.6 us).  Decided by the
+  // workgroups of the attention itself: those that a warm-up hint adds leave the sums as they are.
   const int ks = option_attention_key_split();
   if (wide)
     attention_grouped_kernel<2, KIND, kWideStages><<<grid, kAttThreads, 0, s>>>(a);
-  else if (ks == 1 || (ks < 0 && seq_len >= 512 && grid <= 256))
+  else if (ks == 1 || (ks < 0 && seq_len >= 512 && a.warm.grid_work <= 256))
     attention_grouped_kernel<1, KIND, 2, 2><<<grid, 2 * kAttThreads, 0, s>>>(a);
   else
     attention_grouped_kernel<1, KIND, 2><<<grid, kAttThreads, 0, s>>>(a);

@@ -1328,6 +1328,25 @@ def test_attention_prefetch_hint_changes_nothing(device, kind, lens, S):
         ops.set_option("prefetch_min_grid", 512)
 
 
+@pytest.mark.parametrize("lens,S,heads", [([656], 656, 12), ([1024], 1024, 12), ([1024], 1024, 16), ([1088], 1088, 16),
+                                          ([512, 300], 512, 12), ([640, 640], 640, 12)])
+def test_attention_prefetch_hint_leaves_the_choice_of_kernel(device, lens, S, heads):
+    """132 to 272 workgroups, on either side of the line up to which a long launch splits its keys, with the
+    choice left to the launch: the workgroups that a hint adds must not move it (the sums would run in another order)."""
+    _say("attention prefetch, automatic key split", lens, S, heads)
+    rs = np.random.RandomState(S + heads)
+    bi, M, qkv = _attention_case(rs, lens, S, heads, scale_q=1.0)
+    warm = torch.full((8 << 20,), 7, dtype=torch.uint8, device=device)
+    before = ops.get_option("attention_key_split")
+    ops.set_option("attention_key_split", -1)
+    try:
+        base, got = [ops.attention_grouped(_dev(qkv, device), _dev(bi, device), len(lens), S, 0.125, False, prefetch=w)
+                     for w in (None, warm)]
+    finally:
+        ops.set_option("attention_key_split", before)
+    assert torch.equal(got[:M], base[:M]) and bool((warm == 7).all())
+
+
 @pytest.mark.parametrize("B,S,heads,d", [(1, 33, 2, 32), (3, 200, 12, 128), (40, 64, 12, 96)])
 def test_generic_attention_prefetch_hint_changes_nothing(device, B, S, heads, d):
     """Warm-up by workgroups of their own (small launches) and by the last quarter of the grid."""
