@@ -50,6 +50,11 @@ __device__ __forceinline__ float rows_sum(float x) {
   return a + b;
 }
 
+// The tile loops take the maximum of the unscaled logits and mark keys that do not exist by -1e30 among
+// them.  That needs a positive scale, and one that keeps -1e30 far below every logit; under any other
+// the logits are multiplied first.
+inline bool scale_logits_first(float scale) { return !(scale >= 1e-20f); }
+
 template <int N>
 __device__ __forceinline__ void att_wait_vmcnt() {
   __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0F70);

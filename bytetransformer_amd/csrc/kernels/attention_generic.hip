@@ -34,6 +34,8 @@ struct GenericAttArgs {
   const half_t *bias;     // optional [heads,S,S]
   int B, S, heads;
   float scale_log2e;
+  float scale_in_exp2;    // without additive terms: what is left to multiply in the exponent ...
+  int scale_first;        // ... 1 where the logits are multiplied first (scale_logits_first)
   int padded_rows;
   int nqb;                // query tiles per sequence
   int balanced;           // 1: the live query tiles are dealt evenly to the CUs (common.h)
@@ -193,7 +195,7 @@ __global__ __launch_bounds__(kGenThreads, 2) void attention_generic_kernel(Gener
     for (int db = 0; db <= DB; ++db) o[db][qb] = float4_t{0.f, 0.f, 0.f, 0.f};
   }
   const half8_t ones = {1, 1, 1, 1, 1, 1, 1, 1};
-  const float c = p.scale_log2e, cs = ADD ? 1.0f : c;
+  const float c = p.scale_log2e, cs = ADD ? 1.0f : p.scale_in_exp2;
   const bool wave_live = q0 + wave * QB * 16 < nq;
   const int ntiles = (klen + kGenKeys - 1) / kGenKeys;
   if (ntiles > 0) {
@@ -239,14 +241,15 @@ __global__ __launch_bounds__(kGenThreads, 2) void attention_generic_kernel(Gener
         }
       if (t + 1 < ntiles) fetch_terms(t + 1);
     }
-    if (k0 + kGenKeys > klen) {
+    if ((!ADD && p.scale_first) || k0 + kGenKeys > klen) {
+      const float first = !ADD && p.scale_first ? c : 1.0f;
 #pragma unroll
       for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const bool dead = k0 + kb * 16 + lg * 4 + r >= klen;
 #pragma unroll
-          for (int qb = 0; qb < QB; ++qb) s[kb][qb][r] = dead ? kNegBig : s[kb][qb][r];
+          for (int qb = 0; qb < QB; ++qb) s[kb][qb][r] = dead ? kNegBig : s[kb][qb][r] * first;
         }
     }
 
@@ -370,7 +373,8 @@ extern "C" int bt_attention_generic_f16_warm(const void *qkv, void *out, const i
   if (rc != BT_OK) return rc;
   GenericAttArgs p{(const half_t *)qkv, (half_t *)out, batch_idx, seq_order, (const half_t *)atten_mask,
                    (const half_t *)attention_bias, batch_size, seq_len, head_num, scale * kLog2e,
-                   padded_rows ? 1 : 0};
+                   scale * kLog2e, 0, padded_rows ? 1 : 0};
+  if (scale_logits_first(p.scale_log2e)) p.scale_in_exp2 = 1.0f, p.scale_first = 1;
   p.d = size_per_head;
   // (mask given but nothing to add: its meaning on padded rows stays)
   p.every_key = drop_terms_of_one_key(seq_len, p.mask, p.bias) && padded_rows;

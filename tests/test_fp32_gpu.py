@@ -380,6 +380,28 @@ def test_attention_generic_f16(device, lens, S, heads, d, padded, att_order):
         assert np.all(err <= 2.0 ** -10 * np.abs(exp[r0:r0 + nq]) + 1e-4), (b, err.max())
 
 
+@pytest.mark.parametrize("scale", [-0.125, 0.0, -0.0, 1e-30, -3.0, 40.0])
+@pytest.mark.parametrize("d", [32, 48, 96, 128])
+def test_attention_generic_f16_takes_any_scale(device, scale, d):
+    """Sequences that end inside a tile, scales that are negative, zero or next to it, and large."""
+    rs = np.random.RandomState(d)
+    S, heads, lens = 150, 2, [150, 64, 7, 130]
+    B, H = len(lens), heads * d
+    bi = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    qkv = rs.standard_normal((B * S, 3 * H)).astype(np.float16)
+    bias = (0.5 * rs.standard_normal((heads, S, S))).astype(np.float16)
+    for b in (None, bias):
+        exp = _naive_attention(qkv.astype(np.float32), lens, S, heads, d, scale, False, None,
+                               None if b is None else b.astype(np.float32))
+        g = ops.attention_generic_f16(_dev(qkv, device), _dev(bi, device), B, S, heads, scale,
+                                      bias=None if b is None else _dev(b, device)).cpu().numpy()
+        # logits reach |scale| |q . k|, rounded to 2^-24 of themselves (and once more in the exponent)
+        top = abs(scale) * 8 * d
+        bound = 2.0 ** -10 * np.abs(exp[:bi[-1]]) + 1e-4 + 4 * 2.0 ** -24 * top
+        err = np.abs(g[:bi[-1]].astype(np.float64) - exp[:bi[-1]])
+        assert np.all(err <= bound), (scale, d, err.max())
+
+
 @pytest.mark.parametrize("kind", ["mask", "bias", "both"])
 @pytest.mark.parametrize("S,d", [(1, 64), (2, 64), (3, 128), (63, 64), (65, 64), (129, 64), (130, 32), (67, 128)])
 def test_additive_terms_at_odd_lengths(device, S, d, kind):
