@@ -736,8 +736,6 @@ static int check_att_args(const char *who, const void *qkv, const void *out, con
   return BT_OK;
 }
 
-static int add_kind(const AttArgs &a) { return (a.mask ? kAddMask : 0) | (a.bias ? kAddBias : 0); }
-
 template <int NKB, int KIND>
 static int launch_short_impl(const AttArgs &a, hipStream_t s) {
   constexpr size_t smem = (size_t)2 * NKB * 16 * kHeadDim * sizeof(half_t);
@@ -753,10 +751,11 @@ static int launch_short_impl(const AttArgs &a, hipStream_t s) {
 
 template <int NKB>
 static int launch_short(const AttArgs &a, hipStream_t s) {
-  switch (add_kind(a)) {
+  switch (add_kind(a.mask, a.bias, a.scale_log2e)) {
     case kAddNone: return launch_short_impl<NKB, kAddNone>(a, s);
     case kAddMask: return launch_short_impl<NKB, kAddMask>(a, s);
     case kAddBias: return launch_short_impl<NKB, kAddBias>(a, s);
+    case kAddZero: return launch_short_impl<NKB, kAddZero>(a, s);
     default: return launch_short_impl<NKB, kAddBoth>(a, s);
   }
 }
@@ -911,10 +910,11 @@ extern "C" int bt_attention_grouped(const void *qkv_heads, void *attention_outpu
   unsigned grid = plan.grid;
   rc = plan_warm_duty("bt_attention_grouped", a.warm, grid, prefetch, prefetch_bytes, prefetch_count);
   if (rc) return rc;
-  switch (add_kind(a)) {
+  switch (add_kind(a.mask, a.bias, a.scale_log2e)) {
     case kAddNone: launch_grouped<kAddNone>(a, plan.wide, seq_len, grid, s); break;
     case kAddMask: launch_grouped<kAddMask>(a, plan.wide, seq_len, grid, s); break;
     case kAddBias: launch_grouped<kAddBias>(a, plan.wide, seq_len, grid, s); break;
+    case kAddZero: launch_grouped<kAddZero>(a, plan.wide, seq_len, grid, s); break;
     default: launch_grouped<kAddBoth>(a, plan.wide, seq_len, grid, s); break;
   }
   BT_CHECK_LAUNCH("attention_grouped_kernel");

@@ -50,11 +50,6 @@ __device__ __forceinline__ float rows_sum(float x) {
   return a + b;
 }
 
-// The tile loops take the maximum of the unscaled logits and mark keys that do not exist by -1e30 among
-// them.  That needs a positive scale, and one that keeps -1e30 far below every logit; under any other
-// the logits are multiplied first.
-inline bool scale_logits_first(float scale) { return !(scale >= 1e-20f); }
-
 template <int N>
 __device__ __forceinline__ void att_wait_vmcnt() {
   __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0F70);
@@ -115,7 +110,15 @@ struct TermRow {
 };
 // Which additive terms a kernel applies (a template parameter: decided at run time, the choice is a branch
 // per four keys, and a tile of them takes twice as long).
-enum AddKind { kAddNone = 0, kAddMask = 1, kAddBias = 2, kAddBoth = 3 };
+enum AddKind { kAddNone = 0, kAddMask = 1, kAddBias = 2, kAddBoth = 3, kAddZero = 4 };
+// Without terms (kAddNone) the logits stay unscaled until they are in the exponent: the maximum is taken
+// over them as they are, and keys that do not exist are -1e30 among them.  That needs a positive scale, and
+// one that keeps -1e30 far below every logit; under any other the launch scales them first, as the ones
+// with terms do (kAddZero: a kernel of its own, because a flag in the loop cost every small launch 0.2 us).
+inline int add_kind(const half_t *mask, const half_t *bias, float scale) {
+  const int kind = (mask ? kAddMask : 0) | (bias ? kAddBias : 0);
+  return kind == kAddNone && !(scale >= 1e-20f) ? kAddZero : kind;
+}
 // A single key's probability does not depend on its term; what is left of a mask tensor is that
 // every one of the S keys takes part.  Returns that for launches of S = 1.
 inline bool drop_terms_of_one_key(int S, const half_t *&mask, const half_t *&bias) {

@@ -34,8 +34,6 @@ struct GenericAttArgs {
   const half_t *bias;     // optional [heads,S,S]
   int B, S, heads;
   float scale_log2e;
-  float scale_in_exp2;    // without additive terms: what is left to multiply in the exponent ...
-  int scale_first;        // ... 1 where the logits are multiplied first (scale_logits_first)
   int padded_rows;
   int nqb;                // query tiles per sequence
   int balanced;           // 1: the live query tiles are dealt evenly to the CUs (common.h)
@@ -195,7 +193,7 @@ __global__ __launch_bounds__(kGenThreads, 2) void attention_generic_kernel(Gener
     for (int db = 0; db <= DB; ++db) o[db][qb] = float4_t{0.f, 0.f, 0.f, 0.f};
   }
   const half8_t ones = {1, 1, 1, 1, 1, 1, 1, 1};
-  const float c = p.scale_log2e, cs = ADD ? 1.0f : p.scale_in_exp2;
+  const float c = p.scale_log2e, cs = ADD ? 1.0f : c;
   const bool wave_live = q0 + wave * QB * 16 < nq;
   const int ntiles = (klen + kGenKeys - 1) / kGenKeys;
   if (ntiles > 0) {
@@ -241,15 +239,14 @@ __global__ __launch_bounds__(kGenThreads, 2) void attention_generic_kernel(Gener
         }
       if (t + 1 < ntiles) fetch_terms(t + 1);
     }
-    if ((!ADD && p.scale_first) || k0 + kGenKeys > klen) {
-      const float first = !ADD && p.scale_first ? c : 1.0f;
+    if (k0 + kGenKeys > klen) {
 #pragma unroll
       for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const bool dead = k0 + kb * 16 + lg * 4 + r >= klen;
 #pragma unroll
-          for (int qb = 0; qb < QB; ++qb) s[kb][qb][r] = dead ? kNegBig : s[kb][qb][r] * first;
+          for (int qb = 0; qb < QB; ++qb) s[kb][qb][r] = dead ? kNegBig : s[kb][qb][r];
         }
     }
 
@@ -351,6 +348,7 @@ void launch_generic(const GenericAttArgs &p, int kind, bool wide, unsigned grid,
     case kAddNone: launch_generic_kind<ND, kAddNone>(p, wide, grid, s); break;
     case kAddMask: launch_generic_kind<ND, kAddMask>(p, wide, grid, s); break;
     case kAddBias: launch_generic_kind<ND, kAddBias>(p, wide, grid, s); break;
+    case kAddZero: launch_generic_kind<ND, kAddZero>(p, wide, grid, s); break;
     default: launch_generic_kind<ND, kAddBoth>(p, wide, grid, s); break;
   }
 }
@@ -373,8 +371,7 @@ extern "C" int bt_attention_generic_f16_warm(const void *qkv, void *out, const i
   if (rc != BT_OK) return rc;
   GenericAttArgs p{(const half_t *)qkv, (half_t *)out, batch_idx, seq_order, (const half_t *)atten_mask,
                    (const half_t *)attention_bias, batch_size, seq_len, head_num, scale * kLog2e,
-                   scale * kLog2e, 0, padded_rows ? 1 : 0};
-  if (scale_logits_first(p.scale_log2e)) p.scale_in_exp2 = 1.0f, p.scale_first = 1;
+                   padded_rows ? 1 : 0};
   p.d = size_per_head;
   // (mask given but nothing to add: its meaning on padded rows stays)
   p.every_key = drop_terms_of_one_key(seq_len, p.mask, p.bias) && padded_rows;
@@ -382,7 +379,8 @@ extern "C" int bt_attention_generic_f16_warm(const void *qkv, void *out, const i
   // long as its longest chain of tiles and more, shorter workgroups fill the chip better
   const long long blocks128 = (long long)((seq_len + 127) / 128) * head_num * batch_size;
   // (heads beyond 96 with additive terms would not fit the registers two query blocks at a time)
-  const bool wide = blocks128 >= 1300 && !(size_per_head > 96 && (p.mask || p.bias));
+  const int kind = add_kind(p.mask, p.bias, p.scale_log2e);
+  const bool wide = blocks128 >= 1300 && !(size_per_head > 96 && kind != kAddNone);
   p.nqb = wide ? (seq_len + 127) / 128 : (seq_len + 63) / 64;
   // the balanced order from the third round of 32 workgroups per XCD on and up to 128 sequences, or
   // always / never by the option (the conditions of the 64-wide kernel)
@@ -393,7 +391,6 @@ extern "C" int bt_attention_generic_f16_warm(const void *qkv, void *out, const i
   rc = plan_warm_duty(who, p.warm, grid, prefetch, prefetch_bytes, prefetch_count);
   if (rc != BT_OK) return rc;
   hipStream_t s = as_stream(stream);
-  const int kind = (p.mask ? kAddMask : 0) | (p.bias ? kAddBias : 0);
   switch ((size_per_head + 31) / 32) {
     case 1: launch_generic<1>(p, kind, wide, grid, s); break;
     case 2: launch_generic<2>(p, kind, wide, grid, s); break;

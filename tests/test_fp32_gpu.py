@@ -382,10 +382,11 @@ def test_attention_generic_f16(device, lens, S, heads, d, padded, att_order):
 
 @pytest.mark.parametrize("scale", [-0.125, 0.0, -0.0, 1e-30, -3.0, 40.0])
 @pytest.mark.parametrize("d", [32, 48, 96, 128])
-def test_attention_generic_f16_takes_any_scale(device, scale, d):
-    """Sequences that end inside a tile, scales that are negative, zero or next to it, and large."""
+@pytest.mark.parametrize("S,heads,lens", [(150, 2, [150, 64, 7, 130]), (70, 12, [70, 33, 64, 1, 66] * 22)])
+def test_attention_generic_f16_takes_any_scale(device, scale, d, S, heads, lens):
+    """Sequences that end inside a tile, scales that are negative, zero or next to it, and large; few
+    workgroups and enough of them for 128-query tiles."""
     rs = np.random.RandomState(d)
-    S, heads, lens = 150, 2, [150, 64, 7, 130]
     B, H = len(lens), heads * d
     bi = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
     qkv = rs.standard_normal((B * S, 3 * H)).astype(np.float16)

@@ -1361,6 +1361,24 @@ def test_generic_attention_prefetch_hint_changes_nothing(device, B, S, heads, d)
         assert torch.equal(got, base) and bool((whole == 7).all()), nbytes
 
 
+@pytest.mark.parametrize("scale", [-0.125, 0.0, 1e-30, -3.0])
+@pytest.mark.parametrize("qb", [1, 2])
+def test_attention_takes_any_scale(device, scale, qb):
+    """Scales that are negative, zero or next to it, sequences that end inside a tile and at its end."""
+    rs = np.random.RandomState(4)
+    lens, S, heads = [150, 128, 64, 7, 200], 200, 2
+    bi, M, qkv = _attention_case(rs, lens, S, heads)
+    exp = O.attention_packed(qkv[0, :, :M], qkv[1, :, :M], qkv[2, :, :M], bi, scale, 1e-6)
+    ops.set_option("attention_qb", qb)
+    try:
+        for fn in (ops.attention_short, ops.attention_grouped):
+            g = fn(_dev(qkv, device), _dev(bi, device), len(lens), S, scale, False).cpu().numpy()
+            # probabilities and outputs rounded to fp16
+            assert np.abs(g[:M].astype(np.float64) - exp).max() <= 4e-3, fn.__name__
+    finally:
+        ops.set_option("attention_qb", -1)
+
+
 def test_attention_large_logits_do_not_overflow(device):
     """Logits of a few hundred in magnitude (fp16 Q.K would overflow at 65504)."""
     rs = np.random.RandomState(9)
