@@ -287,6 +287,7 @@ __global__ __launch_bounds__(kAttThreads * KS, KS == 1 || KIND ? 2 : 4) void att
                    (size_t)planes * p.S);
   };
   const bool ragged_end = klen % kSlotKeys != 0;   // every tile but the last is full
+  [[maybe_unused]] const int masked_tile = ragged_end ? ntiles - 1 : -1;
   auto fetch_terms = [&](int t, auto set_tag) {
     constexpr int SET = decltype(set_tag)::value;
     const int key = t * kSlotKeys + grp * kKT + lg * 4;
@@ -471,9 +472,17 @@ __global__ __launch_bounds__(kAttThreads * KS, KS == 1 || KIND ? 2 : 4) void att
         o[4][qb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, pf[kk][qb], o[4][qb], 0, 0, 0);
     }
   };
-  // no masking code on the steady-state path
+  // No masking code on the steady-state path.  The kernels with terms compare with the number of the tile:
+  // asked the other way the compiler kept a loop of its own for sequences that end with a tile, and the
+  // wide kernel under mask and bias spilled 66 registers (32 x 500: 97 -> 74.7 us; 32 x 512: 134 -> 114).  The
+  // wide kernel without terms is faster the other way (32 x 512: 42.4 against 47 us).
   auto step = [&](int t, auto stage_tag) {
-    if (ragged_end && t == ntiles - 1)
+    bool masked;
+    if constexpr (ADD)
+      masked = t == masked_tile;
+    else
+      masked = ragged_end && t == ntiles - 1;
+    if (masked)
       process_tile(t, std::true_type{}, stage_tag);
     else
       process_tile(t, std::false_type{}, stage_tag);
