@@ -543,8 +543,14 @@ constexpr int kF32KT = 32;   // keys per tile
 // may be any bijection as long as both operands agree; it is chosen so that Q and K are
 // read as float4 (k = half*D/2 + step) and P needs no shuffle (key of step j in half h
 // = 8*(j/4) + 4*h + j%4, the accumulator's own row order).
+//
+// Two waves per SIMD are asked for because the accumulators then stay in the registers that vector
+// instructions read.  With one wave they lay in AGPRs: the compiler copied all of them on every turn of the
+// loop, and behind it read the last one 7 wait states after the last matrix instruction, which takes 18 -
+// wrong last columns at head sizes 96 and 128, another way in every run.  (tests/test_kernel_resources.py
+// looks for such reads in every kernel.)
 template <int ND, int NW>
-__global__ __launch_bounds__(64 * NW) void f32_attention_kernel(F32AttArgs p) {
+__global__ __launch_bounds__(64 * NW, 2) void f32_attention_kernel(F32AttArgs p) {
   constexpr int D = 32 * ND;
   constexpr int THREADS = 64 * NW, BQ = 32 * NW;   // 32 queries per wave
   constexpr int SK = D + 4, SV = D + 8;

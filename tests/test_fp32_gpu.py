@@ -442,6 +442,23 @@ def test_additive_terms_at_odd_lengths(device, S, d, kind):
             assert np.all(err <= 2.0 ** -10 * np.abs(exp[r0:r0 + nq]) + bound), (i, b, err.max())
 
 
+@pytest.mark.parametrize("d", [32, 64, 96, 128])
+@pytest.mark.parametrize("lens", [[32], [64], [128, 65], [127, 160], [256], [1024]])
+def test_attention_f32_last_columns(device, d, lens):
+    """Sequences whose last keys count in the last tile, so that the last product of a query's row changes every
+    column: all columns are there, and the same in every run."""
+    rs = np.random.RandomState(d)
+    heads, S = 3, max(lens)
+    bi = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    qkv = rs.standard_normal((bi[-1], 3 * heads * d)).astype(np.float32)
+    exp = _naive_attention(qkv, lens, S, heads, d, 1 / math.sqrt(d), False)
+    runs = [ops.attention_f32(_dev(qkv, device), _dev(bi, device), len(lens), S, heads, 1 / math.sqrt(d))
+            for _ in range(4)]
+    assert all(torch.equal(r, runs[0]) for r in runs)
+    err = np.abs(runs[0].cpu().numpy() - exp)
+    assert err.max() <= 2e-5, (err.max(), np.unique(np.nonzero(err > 2e-5)[1]))
+
+
 def test_attention_f32_rows_sum_and_uniform_keys(device):
     """V = const per column: the output is that constant times sum(P) = 1 / (1 + 1e-6 / sum e),
     whatever Q and K are; identical keys give a uniform P."""
