@@ -8,8 +8,10 @@
 // straight from memory into an LDS ring, V^T through the LDS transpose read, a lazy running maximum, row
 // sums on an MFMA with an all-ones operand.  Two things differ: the head size is the kernel's D = 32 ND
 // or less (columns past it stay zero in LDS and registers), and the probabilities enter the
-// second product as the sum of two fp16 numbers (22 significant bits), because this entry's
-// probabilities have always been floats.
+// second product as the sum of two fp16 numbers, because this entry's probabilities have always been
+// floats.  fp16 has few exponents, so they are computed 2^13 times as large as they are (the quotient O / l
+// does not see it; the lazy maximum lets them grow to four times that): 23 bits from 2^-15 of the largest
+// probability of a row on, and an absolute error of at most 2^-38 of it below.
 //
 // Before, this path ran on v_mfma_f32_32x32x2_f32 with every operand widened to float, at 1/16 of the
 // fp16 rate, 128 queries per workgroup and 328 registers at head size 128: batch 8 x 300, six
@@ -24,6 +26,9 @@ namespace {
 
 constexpr int kGenThreads = 256;
 constexpr int kGenKeys = 64;   // keys per tile
+constexpr float kGenShift = 13.0f;   // probabilities are exp2(x - m + kGenShift), ...
+constexpr float kGenLazy = 2.0f;     // ... where m lags behind the maximum by this much at most
+static_assert(kGenShift + kGenLazy < 16.0f, "the leading fp16 of a probability overflows at 2^16");
 
 struct GenericAttArgs {
   const half_t *qkv;      // [rows, 3H]
@@ -259,10 +264,10 @@ __global__ __launch_bounds__(kGenThreads, 2) void attention_generic_kernel(Gener
 #pragma unroll
         for (int r = 0; r < 4; ++r) mx = fmaxf(mx, s[kb][qb][r]);
       mx = rows_max(mx);
-      const float m_new = (mx - m_run[qb]) * cs > kLazyMax ? mx : m_run[qb];
-      const float mc = m_new * cs;
+      const float m_new = (mx - m_run[qb]) * cs > kGenLazy ? mx : m_run[qb];
+      const float mc = __builtin_fmaf(m_new, cs, -kGenShift);
       if (__builtin_amdgcn_ballot_w64(m_new != m_run[qb]) != 0) {
-        const float alpha = fast_exp2(m_run[qb] * cs - mc);
+        const float alpha = fast_exp2(__builtin_fmaf(m_run[qb], cs, -kGenShift) - mc);
 #pragma unroll
         for (int db = 0; db <= DB; ++db) o[db][qb] *= alpha;
       }
@@ -318,7 +323,7 @@ __global__ __launch_bounds__(kGenThreads, 2) void attention_generic_kernel(Gener
 
 #pragma unroll
   for (int qb = 0; qb < QB; ++qb) {
-    const float inv = __builtin_amdgcn_rcpf(o[DB][qb][0] + 1e-6f);
+    const float inv = 1.0f / (o[DB][qb][0] + 1e-6f * 8192.0f);   // (2^kGenShift)
     const int q = q0 + (wave * QB + qb) * 16 + lq;
     if (q >= nq) continue;
     half_t *dst = p.out + (size_t)(row_start + q) * H + head * d + 4 * lg;

@@ -380,6 +380,49 @@ def test_attention_generic_f16(device, lens, S, heads, d, padded, att_order):
         assert np.all(err <= 2.0 ** -10 * np.abs(exp[r0:r0 + nq]) + 1e-4), (b, err.max())
 
 
+@pytest.mark.parametrize("bits", [3, 10, 14, 20, 24])
+@pytest.mark.parametrize("d", [32, 96, 128])
+def test_attention_generic_f16_keeps_small_probabilities(device, d, bits):
+    """One key takes nearly all of the probability and has V = 0; the rest share 1.3 * 2^-bits of it each, and are
+    all that is in the result. Their probabilities are good to 2^-23 of themselves or 2^-38 of the largest one."""
+    S, heads = 70, 2
+    H = heads * d
+    qkv = np.zeros((S, 3 * H), np.float16)
+    qkv[:, 0:H:d] = 1                                        # Q: (1, 0, ...) in every head
+    top = np.float16(bits * math.log(2) - math.log(1.3))     # ln of (largest / another)
+    qkv[40, H:2 * H:d] = top                                 # K of the favoured key, in the first tile
+    rs = np.random.RandomState(bits)
+    qkv[:, 2 * H:] = (30000 + 20000 * rs.rand(S, H)).astype(np.float16)
+    qkv[40, 2 * H:] = 0
+    bi = np.array([0, S], np.int32)
+    exp = _naive_attention(qkv.astype(np.float32), [S], S, heads, d, 1.0, False)
+    g = ops.attention_generic_f16(_dev(qkv, device), _dev(bi, device), 1, S, heads, 1.0).cpu().numpy()
+    # one fp16 rounding (normal or denormal), the probabilities, and the exponential's 2^-22
+    bound = 2.0 ** -11 * np.abs(exp) + 2.0 ** -25 + np.abs(exp) * 2.0 ** -20 + S * 50000 * 2.0 ** -38
+    assert exp.min() > 1e-3 and np.all(np.abs(g.astype(np.float64) - exp) <= bound), np.abs(g / exp - 1).max()
+
+
+@pytest.mark.parametrize("d,S,lens", [(32, 300, [300, 77, 130]), (96, 128, [128, 65]), (128, 300, [300, 200]),
+                                      (128, 1024, [1024])])
+@pytest.mark.parametrize("sharp", [1.0, 4.0])
+def test_attention_generic_f16_is_as_exact_as_float_arithmetic(device, d, S, lens, sharp):
+    """Its distance from float64 is that of the float kernel on the same numbers with one rounding to fp16."""
+    rs = np.random.RandomState(S + d)
+    heads, B = 3, len(lens)
+    H = heads * d
+    bi = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    qkv = rs.standard_normal((bi[-1], 3 * H)).astype(np.float16)
+    qkv[:, :H] *= np.float16(sharp)
+    args = _dev(bi, device), B, S, heads, 1 / math.sqrt(d)
+    exp = _naive_attention(qkv.astype(np.float32), lens, S, heads, d, 1 / math.sqrt(d), False)
+    got = ops.attention_generic_f16(_dev(qkv, device), *args).cpu().numpy().astype(np.float64) - exp
+    wide = ops.attention_f32(_dev(qkv.astype(np.float32), device), *args).cpu().numpy()
+    wide = wide.astype(np.float16).astype(np.float64) - exp
+    rms = [float(np.sqrt((e ** 2).mean())) for e in (got, wide)]
+    _say("generic attention: rms error %.4e, float kernel rounded to fp16 %.4e" % tuple(rms))
+    assert rms[0] <= 1.002 * rms[1] and np.abs(got).max() <= 1.01 * np.abs(wide).max(), rms
+
+
 @pytest.mark.parametrize("scale", [-0.125, 0.0, -0.0, 1e-30, -3.0, 40.0])
 @pytest.mark.parametrize("d", [32, 48, 96, 128])
 @pytest.mark.parametrize("S,heads,lens", [(150, 2, [150, 64, 7, 130]), (70, 12, [70, 33, 64, 1, 66] * 22)])
