@@ -36,10 +36,10 @@ HIP_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
              "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
              "-mllvm", "-amdgpu-kernarg-preload-count=16",
              "-Wno-unused-command-line-argument"]
-# The attention kernels' inputs are finite by contract (masking is by index, never
-# by NaN/inf), so max() needs no NaN quieting there: plain v_max_f32 / v_max3_f32.
-PER_FILE_FLAGS = {f: ["-fno-honor-nans", "-mno-amdgpu-ieee"]
-                  for f in ("attention.hip", "attention_generic.hip")}
+# The 64-wide attention kernels' inputs are finite by contract (masking is by index, never
+# by NaN/inf), so max() needs no NaN quieting there: plain v_max_f32 / v_max3_f32.  (The other head
+# sizes have no such contract, and their kernels come out shorter without these flags.)
+PER_FILE_FLAGS = {"attention.hip": ["-fno-honor-nans", "-mno-amdgpu-ieee"]}
 HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-Wall"]
 
 

@@ -478,10 +478,12 @@ int bt_gemm_f32(const void *a, const int *a_row_index, const void *w, const void
  * there) and, without a mask, on padded rows.  seq_order (nullable) as in the fp16
  * entries: issue order only.  size_per_head a multiple of 8 up to 128.
  */
-/* The same kernel on fp16 tensors (operands widened to float on chip), for fp16 layers whose
- * head size the fp16 attention entries do not cover: size_per_head a multiple of 8 up to 128.
- * Role of the reference's unfused path for size_per_head != 64 (bert_transformer.h:132-133,
- * attention_nofused.cu:27-114). */
+/* The same arithmetic on fp16 tensors, for fp16 layers whose head size the fp16 attention entries do not
+ * cover: size_per_head a multiple of 8 up to 128.  Products on the fp16 matrix cores with float
+ * accumulators, softmax in float, probabilities as two fp16 numbers each (23 bits, an absolute error of
+ * at most 2^-38 of the row's largest).  A NaN reaches the outputs that depend on it; so does an infinity in
+ * V, as a NaN.  Role of the reference's unfused path for size_per_head != 64
+ * (bert_transformer.h:132-133, attention_nofused.cu:27-114). */
 int bt_attention_generic_f16(const void *qkv, void *attention_output, const int *batch_idx,
                              const int *seq_order, const void *atten_mask,
                              const void *attention_bias, int batch_size, int seq_len,

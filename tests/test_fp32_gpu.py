@@ -423,6 +423,25 @@ def test_attention_generic_f16_is_as_exact_as_float_arithmetic(device, d, S, len
     assert rms[0] <= 1.002 * rms[1] and np.abs(got).max() <= 1.01 * np.abs(wide).max(), rms
 
 
+@pytest.mark.parametrize("d", [48, 128])
+def test_attention_generic_f16_passes_nan_on(device, d):
+    """A NaN in Q, K or V reaches the outputs that depend on it and no others."""
+    rs = np.random.RandomState(d)
+    S, heads, lens = 150, 2, [150, 70, 130]
+    H = heads * d
+    bi = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    qkv = rs.standard_normal((bi[-1], 3 * H)).astype(np.float16)
+    want = np.zeros((bi[-1], H), bool)
+    qkv[5, 3] = np.nan                              # Q of one query, head 0
+    want[5, :d] = True
+    qkv[150 + 69, H + d + 1] = np.nan               # K of the second sequence's last key, head 1
+    want[150:220, d:] = True
+    qkv[220 + 64, 2 * H + 7] = np.nan               # V of one key of the third sequence, column 7 of head 0
+    want[220:, 7] = True
+    g = ops.attention_generic_f16(_dev(qkv, device), _dev(bi, device), 3, S, heads, 1 / math.sqrt(d)).cpu().numpy()
+    assert np.array_equal(np.isnan(g), want) and np.isfinite(g[~want]).all()
+
+
 @pytest.mark.parametrize("scale", [-0.125, 0.0, -0.0, 1e-30, -3.0, 40.0])
 @pytest.mark.parametrize("d", [32, 48, 96, 128])
 @pytest.mark.parametrize("S,heads,lens", [(150, 2, [150, 64, 7, 130]), (70, 12, [70, 33, 64, 1, 66] * 22)])
