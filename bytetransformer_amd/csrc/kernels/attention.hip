@@ -140,7 +140,7 @@ __global__ __launch_bounds__(kAttThreads * KS, KS == 1 || KIND ? 2 : 4) void att
   __shared__ __attribute__((aligned(1024))) half_t ring[STAGES * kSlotHalfs];
 
   if (blockIdx.x >= p.warm.grid_work) {
-    warm_slice(p.warm);
+    warm_slice<kAttThreads * KS>(p.warm);
     return;
   }
   int b, head, seq_start, seq_len, qb_index;
@@ -148,21 +148,21 @@ __global__ __launch_bounds__(kAttThreads * KS, KS == 1 || KIND ? 2 : 4) void att
     // the balanced order, looked up by an earlier launch: one scalar load
     const int4 w = p.work_list[blockIdx.x];
     if (w.x < 0) {
-      warm_slice(p.warm);
+      warm_slice<kAttThreads * KS>(p.warm);
       return;
     }
     b = w.x, head = w.y & 0xffff, qb_index = w.y >> 16, seq_start = w.z, seq_len = w.w;
   } else if (p.xcd_map == 2) {
     const AttWork w = att_work_balanced<BQ>(p, blockIdx.x);
     if (!w.exists) {
-      warm_slice(p.warm);
+      warm_slice<kAttThreads * KS>(p.warm);
       return;
     }
     b = w.b, head = w.head, seq_start = w.seq_start, seq_len = w.len, qb_index = w.qb;
   } else {
     const AttItem item = att_item(p);
     if (!item.exists) {
-      warm_slice(p.warm);
+      warm_slice<kAttThreads * KS>(p.warm);
       return;
     }
     b = p.seq_order ? p.seq_order[item.rank] : item.rank, head = item.head;
@@ -189,7 +189,7 @@ __global__ __launch_bounds__(kAttThreads * KS, KS == 1 || KIND ? 2 : 4) void att
   const int nq = p.padded_rows ? p.S : klen;
   const int q0 = qb_index * BQ;
   if (q0 >= nq) {
-    warm_slice(p.warm);
+    warm_slice<kAttThreads * KS>(p.warm);
     return;
   }
 
@@ -516,7 +516,7 @@ __global__ __launch_bounds__(kAttThreads * KS, KS == 1 || KIND ? 2 : 4) void att
     }
     __syncthreads();
     if (grp == 1) {
-      warm_slice(p.warm);
+      warm_slice<kAttThreads * KS>(p.warm);
       return;
     }
 #pragma unroll
@@ -547,7 +547,7 @@ __global__ __launch_bounds__(kAttThreads * KS, KS == 1 || KIND ? 2 : 4) void att
       *(half4_t *)(dst + 16 * db) = half4_t{(half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3]};
     }
   }
-  warm_slice(p.warm);
+  warm_slice<kAttThreads * KS>(p.warm);
 }
 
 // The balanced order of a launch of `entries` workgroups as a list: one wave per entry.
@@ -574,12 +574,12 @@ __global__ __launch_bounds__(kAttThreads) void attention_short_kernel(AttArgs p)
   half_t *sV = att_smem + KEYS * kHeadDim;    // [KEYS][64] swizzled
 
   if (blockIdx.x >= p.warm.grid_work) {
-    warm_slice(p.warm);
+    warm_slice<kAttThreads>(p.warm);
     return;
   }
   const AttItem item = att_item(p);
   if (!item.exists) {
-    warm_slice(p.warm);
+    warm_slice<kAttThreads>(p.warm);
     return;
   }
   const int b = p.seq_order ? p.seq_order[item.rank] : item.rank, head = item.head;
@@ -589,7 +589,7 @@ __global__ __launch_bounds__(kAttThreads) void attention_short_kernel(AttArgs p)
   const int nq = p.padded_rows ? p.S : klen;
   const int q0 = item.qb * BQ;
   if (q0 >= nq) {
-    warm_slice(p.warm);
+    warm_slice<kAttThreads>(p.warm);
     return;
   }
 
@@ -628,7 +628,7 @@ __global__ __launch_bounds__(kAttThreads) void attention_short_kernel(AttArgs p)
   __syncthreads();
   // no barrier follows: a wave whose 16 queries all lie past the sequence is done
   if (q0 + wave * 16 >= nq) {
-    warm_slice(p.warm);
+    warm_slice<kAttThreads>(p.warm);
     return;
   }
 
@@ -708,7 +708,7 @@ __global__ __launch_bounds__(kAttThreads) void attention_short_kernel(AttArgs p)
       *(half4_t *)(dst_row + 16 * db) =
           half4_t{(half_t)o[db][0], (half_t)o[db][1], (half_t)o[db][2], (half_t)o[db][3]};
   }
-  warm_slice(p.warm);
+  warm_slice<kAttThreads>(p.warm);
 }
 
 // Size of the 1-D grid for `nqb` query tiles per sequence; fills the mapping fields.

@@ -151,32 +151,15 @@ struct WarmDuty {
   const char *base[kWarmRanges];
   unsigned end[kWarmRanges];
   unsigned first;       // the workgroups from here on take part
+  unsigned per;         // lines of each
   unsigned grid_work;   // workgroups of the attention itself: later ones do nothing else
 };
-// The loads are the wave's last instructions; nothing reads their results.
+template <int THREADS>
 __device__ __forceinline__ void warm_slice(const WarmDuty &w) {
   const unsigned lines = w.end[kWarmRanges - 1];
-  if (!lines) return;
-  if (blockIdx.x < w.first) return;
-  const unsigned duty = gridDim.x - w.first;
-  const unsigned me = blockIdx.x - w.first;
-  const unsigned per = (lines + duty - 1) / duty;
-  const unsigned first = me * per;
-  const unsigned last = first + per < lines ? first + per : lines;
-  for (unsigned l = first + threadIdx.x; l < last; l += blockDim.x) {
-    const char *base = w.base[0];
-    unsigned begin = 0;
-#pragma unroll
-    for (int r = 1; r < kWarmRanges; ++r)
-      if (l >= w.end[r - 1]) {
-        base = w.base[r];
-        begin = w.end[r - 1];
-      }
-    unsigned sink;
-    const char *addr = base + (unsigned long long)(l - begin) * 128;
-    asm volatile("global_load_dword %0, %1, off" : "=v"(sink) : "v"(addr) : "memory");
-  }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  if (!lines || blockIdx.x < w.first) return;
+  const unsigned first = (blockIdx.x - w.first) * w.per;
+  touch_lines(w.base, w.end, first + threadIdx.x, min(first + w.per, lines), THREADS);
 }
 // Who takes part, for a launch of `grid` workgroups (grown here by the ones that only warm).
 //   Two workgroups per CU and more (option prefetch_min_grid): the last quarter of the issue order -
@@ -195,6 +178,7 @@ inline int plan_warm_duty(const char *who, WarmDuty &w, unsigned &grid, const vo
     w.end[r] = 0;
   }
   w.first = w.grid_work = grid;
+  w.per = 0;
   BT_REQUIRE(count >= 0 && count <= kWarmRanges, BT_ERR_INVALID_ARGUMENT,
              "%s: prefetch_count=%d outside [0, %d]", who, count, kWarmRanges);
   BT_REQUIRE(count == 0 || (ranges && bytes), BT_ERR_INVALID_ARGUMENT,
@@ -222,6 +206,7 @@ inline int plan_warm_duty(const char *who, WarmDuty &w, unsigned &grid, const vo
     }
     w.end[r] = end;
   }
+  if (end) w.per = (end + (grid - w.first) - 1) / (grid - w.first);
   return BT_OK;
 }
 

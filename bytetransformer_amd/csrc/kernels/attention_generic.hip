@@ -70,14 +70,14 @@ __global__ __launch_bounds__(kGenThreads, 2) void attention_generic_kernel(Gener
   __shared__ __attribute__((aligned(1024))) half_t ring[2 * 2 * kTile];
 
   if (blockIdx.x >= p.warm.grid_work) {
-    warm_slice(p.warm);
+    warm_slice<kGenThreads>(p.warm);
     return;
   }
   int b, head, seq_start, seq_len, qb_index;
   if (p.balanced) {
     const AttWork w = att_work_balanced<BQ>(p, blockIdx.x);
     if (!w.exists) {
-      warm_slice(p.warm);
+      warm_slice<kGenThreads>(p.warm);
       return;
     }
     b = w.b, head = w.head, seq_start = w.seq_start, seq_len = w.len, qb_index = w.qb;
@@ -85,7 +85,7 @@ __global__ __launch_bounds__(kGenThreads, 2) void attention_generic_kernel(Gener
     const unsigned lin = blockIdx.x, slot = lin >> 3;
     const unsigned pair = (slot / p.nqb) * 8 + (lin & 7);
     if (pair >= (unsigned)(p.B * p.heads)) {
-      warm_slice(p.warm);
+      warm_slice<kGenThreads>(p.warm);
       return;
     }
     const int rank = pair / p.heads;
@@ -100,7 +100,7 @@ __global__ __launch_bounds__(kGenThreads, 2) void attention_generic_kernel(Gener
   const int nq = p.padded_rows ? p.S : seq_len;
   const int q0 = qb_index * BQ;
   if (q0 >= nq) {
-    warm_slice(p.warm);
+    warm_slice<kGenThreads>(p.warm);
     return;
   }
 
@@ -334,7 +334,7 @@ __global__ __launch_bounds__(kGenThreads, 2) void attention_generic_kernel(Gener
       *(half4_t *)(dst + 16 * db) = half4_t{(half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3]};
     }
   }
-  warm_slice(p.warm);
+  warm_slice<kGenThreads>(p.warm);
 }
 
 template <int ND, int KIND>

@@ -329,23 +329,31 @@ __device__ __forceinline__ void transpose_tiles_64(const WeightJobs &pw, int t0,
   __syncthreads();
 }
 
-// One dword per 128-byte line of the ranges, lines [first, last) in steps of `stride`.
-__device__ __forceinline__ void warm_lines(const WeightJobs &pw, unsigned first, unsigned last,
-                                           unsigned stride) {
-  for (unsigned l = first; l < last; l += stride) {
-    const char *base = pw.warm[0];
-    unsigned begin = 0;
+// One dword of the lines l, l + stride, ... below `last` (range r holds the 128-byte lines
+// [end[r - 1], end[r]) of a concatenation of four).  Ordinary loads, four in flight, so that the compiler
+// knows which registers they return to: as assembly whose result nobody reads, their register was
+// reused for the next turn's address while the load was under way, an illegal access once in a long while.
+__device__ __forceinline__ void touch_lines(const char *const (&base)[4], const unsigned (&end)[4], unsigned l,
+                                            unsigned last, unsigned stride) {
+  constexpr int kFlight = 4;
+  unsigned long long at[4];   // where line 0 of the concatenation would lie, counted back from range r
 #pragma unroll
-    for (int r = 1; r < 4; ++r)
-      if (l >= pw.warm_end[r - 1]) {
-        base = pw.warm[r];
-        begin = pw.warm_end[r - 1];
-      }
-    unsigned sink;
-    const char *addr = base + (unsigned long long)(l - begin) * 128;
-    asm volatile("global_load_dword %0, %1, off" : "=v"(sink) : "v"(addr) : "memory");
+  for (int r = 0; r < 4; ++r) {
+    at[r] = (unsigned long long)base[r] - (r ? end[r - 1] : 0u) * 128ull;
+    asm volatile("" : "+s"(at[r]));   // (in registers: selected by line, the compiler loads it again for each)
   }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  for (; l < last; l += kFlight * stride) {
+    unsigned got[kFlight];
+#pragma unroll
+    for (int u = 0; u < kFlight; ++u) {
+      const unsigned line = min(l + u * stride, last - 1);
+      unsigned long long from = at[0];
+#pragma unroll
+      for (int r = 1; r < 4; ++r) from = line >= end[r - 1] ? at[r] : from;
+      __builtin_memcpy(&got[u], (const char *)(from + line * 128ull), sizeof(unsigned));
+    }
+    asm volatile("" ::"v"(got[0]), "v"(got[1]), "v"(got[2]), "v"(got[3]));   // (all have returned)
+  }
 }
 
 // ---- which tile a position of the XCD-aware order is ---------------------------------------

@@ -300,7 +300,7 @@ __global__ __launch_bounds__(kPrologueThreads) void layer_prologue_kernel(
     const unsigned per = (n_lines + kPackBlocks - 1) / kPackBlocks;
     const unsigned first = pb * per;
     const unsigned last = first + per < n_lines ? first + per : n_lines;
-    warm_lines(pw, first + tid, last, kPrologueThreads);
+    touch_lines(pw.warm, pw.warm_end, first + tid, last, kPrologueThreads);
   }
 }
 

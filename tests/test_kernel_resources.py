@@ -129,6 +129,68 @@ def test_no_kernel_reads_a_matrix_result_early(code_objects):
     assert not early, early
 
 
+LOAD = re.compile(r"(ds_read|ds_bpermute|ds_permute|ds_swizzle|global_load|buffer_load|flat_load|scratch_load)")
+COUNTED = {"lgkmcnt": re.compile(r"ds_"), "vmcnt": re.compile(r"(global|buffer|flat|scratch)_(load|store|atomic)")}
+
+
+def _touched_in_flight(name, code, after):
+    """Loads whose destination another instruction reads or writes before a wait has made sure of their return. (They
+    return in order, so `s_waitcnt counter(n)` has waited for a load with n or more counted operations behind it.)"""
+    found = []
+    used = [frozenset().union(*[_registers(t) for t in operands]) if operands else frozenset() for _, operands in code]
+    waits = []
+    for op, operands in code:
+        # (a function waits for everything before it does anything else)
+        text = "vmcnt(0) lgkmcnt(0)" if op == "s_swappc_b64" else " ".join(operands)
+        waits.append({c: int(n) for c, n in re.findall(r"(vmcnt|lgkmcnt)\((\d+)\)", text)} if op in ("s_waitcnt", "s_swappc_b64") else {})
+    for i, (op, operands) in enumerate(code):
+        if not LOAD.match(op) or "lds" in operands or "_lds_" in op:
+            continue                                     # (no register waits for a load into LDS)
+        counter = "lgkmcnt" if op.startswith("ds_") else "vmcnt"
+        result, least, todo = _registers(operands[0]), {}, [(j, 0) for j in after[i]]
+        while todo:
+            j, behind = todo.pop()
+            if least.get(j, 1 << 30) <= behind:
+                continue
+            least[j] = behind
+            if waits[j].get(counter, 1 << 30) <= behind:
+                continue
+            other, its = code[j]
+            if used[j] & result:
+                # (another load of the kind into the same registers returns after this one)
+                if not (LOAD.match(other) and COUNTED[counter].match(other) and _registers(its[0]) >= result and
+                        not any(_registers(t) & result for t in its[1:])):
+                    found.append("%s: %s %s in flight at %s %s" % (name, op, ", ".join(operands), other, ", ".join(its)))
+                continue
+            behind = min(behind + bool(COUNTED[counter].match(other)), 64)
+            todo += [(k, behind) for k in after[j]]
+    return found
+
+
+def test_no_kernel_touches_a_register_that_a_load_is_about_to_write(code_objects):
+    """Over every path through every kernel. (The cache warm-up left its loads in flight into a register that the
+    next turn of the loop computed an address in: an illegal access, once in a long while.)"""
+    touched, loads = [], 0
+    for code in code_objects:
+        for name, instructions, after in _functions(code):
+            loads += sum(bool(LOAD.match(op)) for op, _ in instructions)
+            touched += _touched_in_flight(name, instructions, after)
+    assert loads > 5000
+    assert not touched, (len(touched), touched[:20])
+
+
+def test_the_search_for_loads_in_flight_finds_them():
+    """On made-up code: the warm-up loop as it was, a wait that counts, and one that does not."""
+    load, other = ("global_load_dword", ["v0", "v[10:11]", "off"]), ("global_load_dword", ["v9", "v[10:11]", "off"])
+    use, wait = ("v_mov_b32_e32", ["v4", "v0"]), lambda n: ("s_waitcnt", ["vmcnt(%d)" % n])   # noqa: E731
+    end, line = ("s_endpgm", []), lambda n: [[i + 1] for i in range(n - 1)] + [[]]   # noqa: E731
+    address = ("v_lshl_add_u64", ["v[10:11]", "v[0:1]", "0", "v[2:3]"])
+    assert _touched_in_flight("k", [address, load, ("s_cbranch_execnz", ["0"]), wait(0), end], [[1], [2], [0, 3], [4], []])
+    assert not _touched_in_flight("k", [load, other, wait(1), use, end], line(5))
+    assert _touched_in_flight("k", [load, other, wait(2), use, end], line(5))
+    assert _touched_in_flight("k", [load, ("s_waitcnt", ["lgkmcnt(0)"]), use, end], line(4))
+
+
 def test_the_search_for_early_reads_finds_them():
     """On made-up code: straight on, with enough waiting, and around a loop."""
     mfma = ("v_mfma_f32_32x32x2_f32", ["a[0:15]", "v1", "v2", "a[0:15]"])

@@ -1347,6 +1347,28 @@ def test_attention_prefetch_hint_leaves_the_choice_of_kernel(device, lens, S, he
     assert torch.equal(got[:M], base[:M]) and bool((warm == 7).all())
 
 
+def test_warm_up_of_large_weights_only_reads(device):
+    """Ranges of several lines per thread (hidden 2048 and more), as the prologue and the attention's own
+    workgroups touch them: nothing changes, neither the results nor the ranges."""
+    rs = np.random.RandomState(5)
+    warm = [torch.full((n,), 7, dtype=torch.uint8, device=device) for n in (25 << 20, 8 << 20, 33 << 20, (33 << 20) + 3)]
+    mask = torch.zeros(3, 90, 90, dtype=torch.float16, device=device)
+    for b, n in enumerate((90, 17, 64)):
+        mask[b, :, :n] = 1
+    want = ops.layer_prologue(mask)
+    for _ in range(3):
+        got = ops.layer_prologue(mask, warm=warm)
+        assert all(torch.equal(g, w) for g, w in zip(got, want) if torch.is_tensor(g))
+    for lens, S, heads in (([90], 90, 2), ([300, 40], 320, 12), ([512] * 16, 512, 12)):
+        bi, M, qkv = _attention_case(rs, lens, S, heads)
+        qkv, bi = _dev(qkv, device), _dev(bi, device)
+        base = ops.attention_grouped(qkv, bi, len(lens), S, 0.125, False)
+        for _ in range(3):
+            got = ops.attention_grouped(qkv, bi, len(lens), S, 0.125, False, prefetch=warm)
+            assert torch.equal(got[:M], base[:M])
+    assert all(bool((w == 7).all()) for w in warm)
+
+
 @pytest.mark.parametrize("B,S,heads,d", [(1, 33, 2, 32), (3, 200, 12, 128), (40, 64, 12, 96)])
 def test_generic_attention_prefetch_hint_changes_nothing(device, B, S, heads, d):
     """Warm-up by workgroups of their own (small launches) and by the last quarter of the grid."""

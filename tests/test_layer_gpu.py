@@ -558,6 +558,14 @@ def test_head_sizes_other_than_64(device, dtype, head_size, heads, rm):
         assert mx <= tol[0] and mean <= tol[1] and pads_zero, (tag, mx, mean, pads_zero)
 
 
+def test_wide_layer_on_padded_rows(device):
+    """Hidden 2048 on padded rows past 320 tokens: the launch ahead of the layer warms 100 MB of weights."""
+    cfg = workload.EncoderConfig("wide", 2, 330, 32, layers=1, lens=(330, 201), seed=3)
+    wl = workload.make_workload(cfg, bias_std=0.05, random_affine=True)
+    got = _run_th_op(wl, device)
+    _check(O.masked_output(got, wl.lens), _oracle(wl), wl.lens, pads_must_be_zero=False, tag="hidden 2048")
+
+
 def test_hidden_size_rule_of_the_fp16_layer(device):
     """head_num * head_size must be a multiple of 64 on fp16 (the MFMA products step
     through k in tiles of 64); the float layer takes 12 x 40 = 480."""

@@ -1,0 +1,45 @@
+"""How many k slices the layer gives FFN2: the rule of include/bytetransformer/common.h, compiled as the host compiles it."""
+import os
+import subprocess
+
+import pytest
+
+from bytetransformer_amd import build
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+SOURCE = """
+#include <cstdio>
+#include <cstdlib>
+#include "bytetransformer/common.h"
+int main(int argc, char **argv) {
+  for (int i = 1; i + 3 < argc; i += 4)
+    std::printf("%d\\n", bytetransformer::splitk_splits(std::atoll(argv[i]), std::atoll(argv[i + 1]), std::atoi(argv[i + 2]),
+                                                       std::atoi(argv[i + 3])));
+}
+"""
+# capacity, expected rows, n, k -> slices
+CASES = [((32, 32, 768, 3072), 4), ((512, 192, 768, 3072), 4), ((512, 193, 768, 3072), 2), ((1024, 640, 768, 3072), 2),
+         ((1024, 641, 768, 3072), 1), ((1025, 300, 768, 3072), 1), ((512, 192, 1024, 4096), 4), ((512, 193, 1024, 4096), 2),
+         ((448, 448, 1024, 4096), 2), ((449, 449, 1024, 4096), 1), ((1000, 704, 1024, 4096), 1), ((128, 128, 1280, 5120), 4),
+         ((160, 160, 1280, 5120), 2), ((64, 64, 2048, 8192), 4), ((128, 128, 2048, 8192), 2), ((224, 224, 2048, 8192), 1),
+         ((1024, 704, 512, 2048), 2), ((1024, 705, 512, 2048), 1), ((32, 32, 256, 1024), 1), ((32, 32, 384, 2112), 1)]
+
+
+@pytest.fixture(scope="module")
+def answers(tmp_path_factory):
+    tmp = tmp_path_factory.mktemp("rule")
+    source, program = str(tmp / "rule.cc"), str(tmp / "rule")
+    with open(source, "w") as f:
+        f.write(SOURCE)
+    subprocess.run(["g++"] + build.HOST_FLAGS + ["-I", os.path.join(ROOT, "include"), "-I",
+                                                 os.path.join(build.ROCM, "include"), source, "-o", program], check=True)
+    env = {k: v for k, v in os.environ.items() if k != "BT_SPLITK"}
+    out = subprocess.run([program] + [str(v) for args, _ in CASES for v in args], check=True, stdout=subprocess.PIPE,
+                         text=True, env=env).stdout
+    return [int(v) for v in out.split()]
+
+
+@pytest.mark.parametrize("i", range(len(CASES)))
+def test_slices(answers, i):
+    args, want = CASES[i]
+    assert answers[i] == want, args
