@@ -330,12 +330,14 @@ __device__ __forceinline__ void transpose_tiles_64(const WeightJobs &pw, int t0,
 }
 
 // One dword of the lines l, l + stride, ... below `last` (range r holds the 128-byte lines
-// [end[r - 1], end[r]) of a concatenation of four).  Ordinary loads, four in flight, so that the compiler
+// [end[r - 1], end[r]) of a concatenation of four).  Ordinary loads, two in flight, so that the compiler
 // knows which registers they return to: as assembly whose result nobody reads, their register was
 // reused for the next turn's address while the load was under way, an illegal access once in a long while.
+// (One / two / four in flight, 12 layers in us: 1 x 32 360 / 366 / 379, 1 x 256 443 / 449 / 461, captured 4 x
+// 96 417 / 414 / 418, 6 x 250 under its mask 779 / 772 / 761.)
 __device__ __forceinline__ void touch_lines(const char *const (&base)[4], const unsigned (&end)[4], unsigned l,
                                             unsigned last, unsigned stride) {
-  constexpr int kFlight = 4;
+  constexpr int kFlight = 2;
   unsigned long long at[4];   // where line 0 of the concatenation would lie, counted back from range r
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
@@ -352,7 +354,7 @@ __device__ __forceinline__ void touch_lines(const char *const (&base)[4], const 
       for (int r = 1; r < 4; ++r) from = line >= end[r - 1] ? at[r] : from;
       __builtin_memcpy(&got[u], (const char *)(from + line * 128ull), sizeof(unsigned));
     }
-    asm volatile("" ::"v"(got[0]), "v"(got[1]), "v"(got[2]), "v"(got[3]));   // (all have returned)
+    asm volatile("" ::"v"(got[0]), "v"(got[1]));   // (both have returned)
   }
 }
 
