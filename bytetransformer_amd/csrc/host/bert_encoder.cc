@@ -185,7 +185,7 @@ void BertEncoder<OpType>::infer(BertEncoderInferParam<DataType_> ip) {
     // few rows, long k: FFN2 as split-k partial sums that the last LayerNorm folds in
     const long long rows_expected =
         !valid_rows ? rows : (rows_hint > 0 ? rows_hint : (rows * 3LL + 4) / 5);
-    const int splits = splitk_splits(rows, rows_expected, hidden, inter);
+    const int splits = splitk_splits(rows, rows_expected, inter);
     if (splits > 1) {
       const bool restore = last && is_remove_padding_;
       check_bt_error(bt_gemm_splitk(inter_matmul_buf, wt_out, splitk_buf, splits, valid_rows, rows,

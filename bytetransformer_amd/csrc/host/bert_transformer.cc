@@ -335,7 +335,7 @@ void BertTransformer<OpType>::bert_infer(BertTransformerInferParam infer_param) 
   // few rows, long k: FFN2 as split-k partial sums that the last LayerNorm folds in
   const long long rows_expected =
       !valid_rows ? rows : (rows_hint > 0 ? rows_hint : (rows * 3LL + 4) / 5);
-  const int splits = splitk_splits(packed_cap, rows_expected, hidden, inter);
+  const int splits = splitk_splits(packed_cap, rows_expected, inter);
   if (splits > 1) {
     check_bt_error(bt_gemm_splitk(inter_matmul_buf, wt_out, splitk_buf, splits, valid_rows,
                                   packed_cap, hidden, inter, w_kn[3], stream));

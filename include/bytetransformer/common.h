@@ -52,31 +52,26 @@ typedef struct {
   int valid_word_num;
 } ET_Param;
 
-// FFN2 [k, n] with few rows and a long k runs as a split-k GEMM whose fp32 partial sums the last
-// LayerNorm folds in (bt_gemm_splitk / bt_splitk_layernorm), as long as that takes the tiles of the
-// launch no more than about one round of the chip's 256 CUs, and the partials of a launch of that
-// capacity fit the scratch area (4 splits of kSplitKMaxRows rows).  Two launches in us, whole k / two splits /
-// four, at k = 4 n (k = 2048 for n = 256):
-//   n = 256:  256 rows  9.2 / 8.0 / 7.5;   512 rows  9.4 / 8.3;   1024 rows 9.7 / 9.8
-//   n = 512:  192 rows  9.8 / 8.5 / 8.3;   576 rows 11.3 / 10.5;   896 rows 11.4 / 11.3
-//   n = 768:  192 rows 12.3 / 10.9 / 10.7; 640 rows 14.6 / 13.8;   704 rows 16.3 / 17.1
-//   n = 1024: 192 rows 15.9 / 12.5 / 12.3; 384 rows 16.8 / 16.2;   448 rows 17.1 / 17.4, 704 rows 20.6 / 23.3
-//   n = 1280: 128 rows 17.7 / 14.8 / 14.4; 160 rows 17.4 / 15.2 / 16.5; 384 rows 21.5 / 20.6; 448 rows 25.2 / 28.0
-//   n = 2048:  64 rows 28.1 / 21.3 / 20.7; 128 rows 25.0 / 20.9 / 21.7; 192 rows 29.0 / 26.0; 224 rows 29.3 / 30.3
+// FFN2 with few rows and a long k runs as a split-k GEMM whose fp32 partial sums the last
+// LayerNorm folds in (bt_gemm_splitk / bt_splitk_layernorm): 4 splits up to 192 expected
+// rows, 2 up to 640, none beyond, or when the partials of a launch of that
+// capacity exceed the scratch area (4 splits of kSplitKMaxRows rows).  A whole layer in us with k whole / in two
+// splits / in four, in stacks of 12 layers (hidden 768) and 24 whose weights no cache holds together; launched
+// alone over and over, weights and rows warm, the split of the wide ones looks worse than it is here:
+//   hidden 768:  192 rows  36.6 /  34.8 / 34.6; 576 rows  46.2 /  45.9; 640 rows  46.6 /  46.6; 704 rows  54.8 /  56.6
+//   hidden 1024: 192 rows  48.1 /  46.7 / 44.4; 576 rows  67.3 /  64.7; 640 rows  68.8 /  65.3; 704 rows  70.1 /  73.7
+//   hidden 1280: 192 rows  55.7 /  53.8 / 51.1; 512 rows  81.7 /  83.5; 640 rows  84.2 /  79.8; 704 rows  86.8 /  90.5
+//   hidden 2048: 192 rows 100.4 /  92.0 / 88.1; 512 rows 126.8 / 129.9; 640 rows 152.7 / 146.6; 704 rows 155.5 / 174.8
+// (weights as stored; pre-packed at 704 rows: hidden 768 49.8 / 51.9, hidden 1024 67.2 / 64.9)
 constexpr int kSplitKMaxRows = 512;
-inline int splitk_splits(long long rows_cap, long long rows_expected, int n, int k) {
+inline int splitk_splits(long long rows_cap, long long rows_expected, int k) {
   static const bool enabled = [] {
     const char *e = std::getenv("BT_SPLITK");     // BT_SPLITK=0 turns the split-k path off
     return !(e && e[0] == '0');
   }();
   if (!enabled || k < 2048) return 1;
-  const long long narrow = (n + 63) / 64;   // tile columns
-  if (rows_cap <= kSplitKMaxRows && rows_expected <= 192 && k % (4 * 64) == 0 &&
-      (rows_expected + 31) / 32 * narrow * 4 <= 384)
-    return 4;
-  if (rows_cap <= 2 * kSplitKMaxRows && rows_expected <= 704 && k % (2 * 64) == 0 &&
-      (rows_expected + 63) / 64 * narrow * 2 <= 240)
-    return 2;
+  if (rows_cap <= kSplitKMaxRows && rows_expected <= 192 && k % (4 * 64) == 0) return 4;
+  if (rows_cap <= 2 * kSplitKMaxRows && rows_expected <= 640 && k % (2 * 64) == 0) return 2;
   return 1;
 }
 inline unsigned long long splitk_scratch_bytes(unsigned long long max_rows,
