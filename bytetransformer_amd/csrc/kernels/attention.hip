@@ -134,8 +134,7 @@ __global__ __launch_bounds__(kAttThreads * KS, KS == 1 || KIND ? 2 : 4) void att
   constexpr int AHEAD = STAGES - 1;     // tiles in flight beyond the one being consumed
   constexpr int kSlotKeys = kKT * KS;   // keys per ring slot
   constexpr int kSlotHalfs = KS * 2 * kTileHalfs;
-  static_assert(STAGES >= 2 && STAGES <= 4, "ring depth");
-  static_assert(!ADD || STAGES % 2 == 0, "the additive terms alternate between two register sets");
+  static_assert(STAGES == 2 || (STAGES == 3 && !ADD), "ring depth; the additive terms alternate between two register sets");
   static_assert(KS == 1 || KS == 2, "key split");
   __shared__ __attribute__((aligned(1024))) half_t ring[STAGES * kSlotHalfs];
 
@@ -325,22 +324,12 @@ __global__ __launch_bounds__(kAttThreads * KS, KS == 1 || KIND ? 2 : 4) void att
     constexpr bool MASKED = decltype(masked_tag)::value;
     constexpr int ST = decltype(stage_tag)::value;
     // This wave's share of tile t has landed once only what was requested after it is outstanding: the
-    // four loads of each later tile and, from the second tile on, the terms of this one (four loads
-    // or more per query block).  A two-deep ring requests a tile last of all.
-    constexpr int TERMS = ADD && AHEAD > 1 ? 4 * QB : 0;
-    auto wait_tile = [&](auto terms_tag) {
-      constexpr int N = decltype(terms_tag)::value;
-      if (AHEAD > 2 && t + 2 < ntiles)
-        att_wait_vmcnt<8 + N>();
-      else if (AHEAD > 1 && t + 1 < ntiles)
-        att_wait_vmcnt<4 + N>();
-      else
-        att_wait_vmcnt<N>();
-    };
-    if (TERMS > 0 && t > 0)
-      wait_tile(std::integral_constant<int, TERMS>{});
+    // four loads of the next tile in a three-deep ring, nothing in a two-deep one, which requests a tile
+    // (and its terms before it) last of all.
+    if (AHEAD > 1 && t + 1 < ntiles)
+      att_wait_vmcnt<4>();
     else
-      wait_tile(std::integral_constant<int, 0>{});
+      att_wait_vmcnt<0>();
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
@@ -491,11 +480,8 @@ __global__ __launch_bounds__(kAttThreads * KS, KS == 1 || KIND ? 2 : 4) void att
   for (int t = 0; t < ntiles; t += STAGES) {
     step(t, std::integral_constant<int, 0>{});
     if (t + 1 < ntiles) step(t + 1, std::integral_constant<int, 1>{});
-    if constexpr (STAGES >= 3) {
+    if constexpr (STAGES == 3) {
       if (t + 2 < ntiles) step(t + 2, std::integral_constant<int, 2>{});
-    }
-    if constexpr (STAGES == 4) {
-      if (t + 3 < ntiles) step(t + 3, std::integral_constant<int, 3>{});
     }
   }
 

@@ -1015,6 +1015,7 @@ __device__ __forceinline__ void gemm_wave_k(const GemmArgs &p) {
   constexpr int NIA = BM / 8, NI = (BM + BN) / 8;   // 1 KB load instructions per k-step
   constexpr int STEP_HALFS = (BM + BN) * BK;
   static_assert(BN == 32 && KS == 4, "one MFMA block; the loop body names its four k parts");
+  static_assert(NW == 4, "a wave for each of the four quads of sums");
   static_assert((DEPTH - 1) * NI < 64, "pipeline depth");
   static_assert(BM * BN * sizeof(float) <= DEPTH * STEP_HALFS * sizeof(half_t), "sums fit the ring");
   extern __shared__ __attribute__((aligned(1024))) half_t gemm_smem[];
@@ -1125,7 +1126,7 @@ __device__ __forceinline__ void gemm_wave_k(const GemmArgs &p) {
   }
 
   // fold: quad q of a wave's sums (columns 8 q + 4 (lane >> 5) .. + 3 of row lane & 31) lies at 1 KB q
-  // of its ring, 16 bytes per lane; wave q < 4 adds quad q over the waves and stores it
+  // of its ring, 16 bytes per lane; wave q adds quad q over the waves and stores it
   {
     float4_t *own = (float4_t *)ring;
 #pragma unroll
@@ -1133,7 +1134,6 @@ __device__ __forceinline__ void gemm_wave_k(const GemmArgs &p) {
       own[q * 64 + lane] = float4_t{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
   }
   __syncthreads();
-  if (NW > 4 && wave >= 4) return;
   float4_t v = ((const float4_t *)gemm_smem)[wave * 64 + lane];
 #pragma unroll
   for (int w = 1; w < NW; ++w)
