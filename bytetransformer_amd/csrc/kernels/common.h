@@ -79,7 +79,7 @@ int option_f32_gemm_tile();  // -1 = heuristic, else index into the float GEMM's
 int option_attention_xcd_map();     // workgroup order of the attention kernels: 0 plain, 1 XCD-aware, 2 balanced (default), 3 balanced always
 int option_prefetch();       // 1 = honour the prefetch hints of the attention entries (default), 0 = ignore
 int option_attention_key_split();  // streaming attention, 64-query tiles: -1 heuristic, 0 four waves, 1 eight waves over two key halves
-int option_prefetch_min_grid();   // attention launches of fewer workgroups skip the cache warm-up (default 512)
+int option_prefetch_min_grid();   // attention launches of fewer workgroups bring workgroups of their own for the cache warm-up (default 512)
 
 inline hipStream_t as_stream(void *s) { return reinterpret_cast<hipStream_t>(s); }
 

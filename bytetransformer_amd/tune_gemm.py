@@ -12,6 +12,7 @@ import argparse
 import json
 import os
 import sys
+import textwrap
 
 M_STEP = 256                     # the tallest tile: run time steps with the count of row tiles
 M_GRID = (tuple(range(64, 1024, 64)) + tuple(range(1024, 2560, 128)) + tuple(range(2560, 8192, M_STEP))
@@ -144,15 +145,16 @@ def merge_runs(rows):
             for (m, n, k, epi, kn, full), by_tile in seen.items()]
 
 
-def write_inc(rows, path=INC):
+def write_inc(rows, path=INC, note=""):
     shapes = {}
     for r in merge_runs(rows):
         shapes.setdefault((r["N"], r["K"], EPI_CODE[r.get("epi", "plain")], r.get("kn", 0),
                            r.get("full", 0)), {})[r["M"]] = r["us"]
-    lines = ["// Generated by `python -m bytetransformer_amd.tune_gemm` from timings on one MI355X:",
+    lines = ["// Generated by `python -m bytetransformer_amd.tune_gemm` from timings on MI355X:",
              "// microseconds per launch of each tile shape (index = tile id; 0 = not measured)",
              "// at kTunedRows live rows, per weight shape, weight layout and launch shape (full = 1:",
              "// every row of the launch live; 0: a padded batch with 60 % live rows).  Do not edit by hand.",
+             *["// " + line for line in textwrap.wrap(note, 96)],
              "constexpr int kTunedPoints = %d;" % len(M_GRID),
              "constexpr int kTunedTiles = %d;" % len(TILES),
              "constexpr int kTunedStep = %d;" % M_STEP,
@@ -178,6 +180,7 @@ def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--json", help="also save the raw timings here")
     ap.add_argument("--from-json", nargs="+", help="build the table from saved timings instead")
+    ap.add_argument("--note", default="", help="which timings these are, for the head of the table")
     args = ap.parse_args()
     if args.from_json:
         rows = []
@@ -187,7 +190,7 @@ def main():
         rows = measure()
     if args.json:
         json.dump(rows, open(args.json, "w"))
-    print("wrote", write_inc(rows), file=sys.stderr)
+    print("wrote", write_inc(rows, note=args.note), file=sys.stderr)
 
 
 if __name__ == "__main__":

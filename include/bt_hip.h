@@ -247,7 +247,8 @@ int bt_gemm_bias_gelu(const void *a, const void *wt, const void *bias, void *c,
  * add_QKV_bias_padding (attention_nofused_utils.cu:143-184) / the in-kernel
  * bias add of attention_fused.cu:318-325.  The head split needs size_per_head == 64.
  * a_row_index (nullable, needs valid_rows): live row t of A is a[a_row_index[t], :] -
- * passing word_idx reads the valid tokens straight out of the padded input, which
+ * passing word_idx reads the valid tokens straight out of the padded input (every entry
+ * below rows_cap, the rows of both the input and qkv_heads), which
  * folds compressBertInput (remove_padding.h:104-121) into this GEMM's operand fetch.
  * size_per_head != 64: the projections stay token-major, qkv_heads = [rows_cap, 3 * hidden]
  * (Q | K | V per row), the layout bt_attention_generic_f16 reads.

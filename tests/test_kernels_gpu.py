@@ -1292,8 +1292,8 @@ def test_attention_prefetch_hint_changes_nothing(device, kind, lens, S):
         assert torch.equal(got[:M], base[:M])
     finally:
         ops.set_option("prefetch", 1)
-    # Small launches skip the warm-up by themselves; force it on so that the duty
-    # workgroups really run here.  The range sits inside a larger allocation (guard bytes on
+    # So far workgroups of their own did the warm-up (fewer than prefetch_min_grid of the attention's); now the
+    # last quarter of the attention's.  The range sits inside a larger allocation (guard bytes on
     # both sides, so a stray line would still land in owned memory), starts on a line
     # boundary or 16 bytes into one, and ends 0-5 bytes into a line: the last touched dword
     # must lie inside the range.
