@@ -352,7 +352,9 @@ __device__ __forceinline__ void touch_lines(const char *const (&base)[4], const 
       unsigned long long from = at[0];
 #pragma unroll
       for (int r = 1; r < 4; ++r) from = line >= end[r - 1] ? at[r] : from;
-      __builtin_memcpy(&got[u], (const char *)(from + line * 128ull), sizeof(unsigned));
+      // (in the global address space by name; ranges may start at any byte)
+      typedef unsigned any_byte __attribute__((aligned(1)));
+      got[u] = *(const __attribute__((address_space(1))) any_byte *)(from + line * 128ull);
     }
     asm volatile("" ::"v"(got[0]), "v"(got[1]));   // (both have returned)
   }
