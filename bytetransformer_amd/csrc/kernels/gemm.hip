@@ -15,10 +15,10 @@
 //     and makes the ds_read_b128 operand fetches conflict-free on the 64 banks;
 //   * a ring of STAGES tiles, one barrier per k-step, vmcnt-counted waits so
 //     later stages stay in flight across the barrier;
-//   * v_mfma_f32_32x32x16_f16 with the weight tile as the MFMA "A" operand and
-//     the activation tile as "B": a lane's accumulator quad holds 4 consecutive
-//     output columns of one row; operand fragments are double-buffered across
-//     the four k-slices of a tile;
+//   * v_mfma_f32_16x16x32_f16 with the weight tile as the MFMA "A" operand and
+//     the activation tile as "B": a lane's four sums of a block are 4 consecutive
+//     output columns of one row; operand fragments are double-buffered over
+//     sub-steps of eight products;
 //   * epilogue: bias / GELU on the accumulators, then each wave stages 32 rows
 //     at a time through a private LDS tile and writes 16-byte, row-contiguous
 //     global stores.
@@ -32,6 +32,7 @@
 #include "common.h"
 
 #include <type_traits>
+#include <utility>
 
 namespace bt {
 
@@ -205,19 +206,22 @@ __device__ __forceinline__ int swz(int row) { return (row >> 1) & 7; }
 
 // gemm_wave_k: columns of a tile, waves of a workgroup, k-steps in a wave's ring
 constexpr int kWaveKCols = 32, kWaveKWaves = 4, kWaveKDepth = 3;
+constexpr int kSchedMfma = 0x008, kSchedLdsRead = 0x100;   // instruction classes of sched_group_barrier
 constexpr int kBK = 64;   // k extent of one LDS tile (halfs) = 8 chunks of 16 bytes
 
 // A [K, N] weight tile sits in LDS as 64 k-rows of BN halfs and is read with the LDS
-// transpose read: the 32 lanes of one pass fetch 4 consecutive k-rows x 64 bytes.  Rows are
-// BN / 32 segments of 64 bytes long; with a multiple of four segments per row the four rows
-// start on the same bank and the segment is XORed with row & 3, with an odd multiple of
-// two (BN = 64, 192) rows r and r + 2 do and bit 0 of the segment is XORed with bit 1 of the
-// row.  Returned in 16-byte chunks (the unit a loading lane moves).
+// transpose read: the 32 lanes of one pass fetch 32 bytes of each of the k-rows r .. r + 3 and
+// r + 8 .. r + 11.  Rows are BN / 32 segments of 64 bytes long; with a multiple of four segments
+// per row the four rows start on the same bank and the segment is XORed with row & 3, with an odd
+// multiple of two (BN = 64, 192) rows r and r + 2 do and bit 0 of the segment is XORed with bit 1 of
+// the row; bit 3 of the row picks the half of the segment, which parts row r from row r + 8.
+// Returned in 16-byte chunks (the unit a loading lane moves).
 template <int BN>
 __device__ __forceinline__ int swz_kn(int k_row) {
   static_assert(BN == 32 || BN % 64 == 0, "whole 64-byte segment pairs");
-  if (BN == 32) return 0;   // four k-rows are 256 contiguous bytes
-  return (BN / 32) % 4 == 0 ? (k_row & 3) << 2 : ((k_row >> 1) & 1) << 2;
+  if (BN == 32) return 0;   // gemm_wave_k: four k-rows are 256 contiguous bytes
+  const int half = ((k_row >> 3) & 1) << 1;
+  return ((BN / 32) % 4 == 0 ? (k_row & 3) << 2 : ((k_row >> 1) & 1) << 2) | half;
 }
 
 template <int N>
@@ -276,15 +280,15 @@ __device__ __forceinline__ int kn_load_offset(int g, int lane, int N, int cols) 
   return c * 8 < cols ? (k_row * N + c * 8) * (int)sizeof(half_t) : 0x7ffffff0;
 }
 
-// Weight operand of one 32x32x16 MFMA (32 columns from n_base, 16 k-rows from k_base) out
-// of the LDS image of a [K, N] tile: lane l holds column n_base + (l & 31) at k-rows
-// k_base + 8 (l >> 5) .. + 7, gathered by two transpose reads of 4 k-rows x 16 columns per
-// 16 lanes.  `lane_part` = kn_frag_lane_part(lane).
+// Weight operand of one 16x16x32 MFMA (16 columns from n_base, 32 k-rows from k_base) out
+// of the LDS image of a [K, N] tile: lane l holds column n_base + (l & 15) at k-rows
+// k_base + 8 (l >> 4) .. + 7, gathered by two transpose reads of 4 k-rows x 16 columns per
+// 16 lanes.
 template <int BN>
 __device__ __forceinline__ half8_t load_kn_frag(const half_t *sW, int n_base, int k_base, int lane) {
-  const int lq = lane & 15, g2 = lane >> 4;
-  const int k_row = k_base + 8 * (g2 >> 1) + (lq >> 2);
-  const int col = n_base + 16 * (g2 & 1) + 4 * (lq & 3);
+  const int lq = lane & 15;
+  const int k_row = k_base + 8 * (lane >> 4) + (lq >> 2);
+  const int col = n_base + 4 * (lq & 3);
   const half_t *p0 = sW + k_row * BN + (((col >> 3) ^ swz_kn<BN>(k_row)) << 3) + (col & 7);
   const fp16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4f16(
       (__attribute__((address_space(3))) fp16x4_t *)p0);
@@ -296,25 +300,24 @@ __device__ __forceinline__ half8_t load_kn_frag(const half_t *sW, int n_base, in
 
 // ---- the epilogue's wave-private staging tile -------------------------------------------
 // 32 rows of WTN halfs, written 8 bytes per lane straight from the accumulator layout (lane l
-// owns row l & 31, the 8-byte half l >> 5 of a 16-byte chunk) and read back 16 bytes per lane,
-// row-contiguous, for the global stores.  With 128-byte rows (WTN = 64) the tile is
-// swizzled instead of padded: chunk ^= (row >> 1) & 7 and half ^= row >> 4 put the 32 lanes
-// of one write pass on 32 distinct bank pairs (a padded pitch leaves rows r and r + 16 on the
-// same banks: every write two passes); a reader undoes the half swap in registers.
+// owns row l & 15 of a 16-row block, the 8-byte half (l >> 4) & 1 of a 16-byte chunk) and read back
+// 16 bytes per lane, row-contiguous, for the global stores.  With 128-byte rows (WTN = 64) the tile is
+// swizzled instead of padded: chunk ^= (row >> 1) & 7 and half ^= row & 1 put the 16 lanes
+// of one write pass on 16 distinct bank pairs; a reader undoes the half swap in registers.
 template <int WTN>
 struct Staging {
   static constexpr bool kSwizzled = WTN == 64;
   static constexpr int kPitch = kSwizzled ? WTN : WTN + 8;   // halfs
   // where lane (row, half hf of the chunk) writes the 4 halfs of 16-byte chunk `chunk`
   __device__ static __forceinline__ int write_at(int row, int hf, int chunk) {
-    if (kSwizzled) return row * kPitch + ((chunk ^ ((row >> 1) & 7)) << 3) + (((hf ^ (row >> 4)) & 1) << 2);
+    if (kSwizzled) return row * kPitch + ((chunk ^ ((row >> 1) & 7)) << 3) + (((hf ^ row) & 1) << 2);
     return row * kPitch + (chunk << 3) + (hf << 2);
   }
   // the 8 halfs of chunk `chunk` of row `row`, in order
   __device__ static __forceinline__ uint4_t read(const half_t *st, int row, int chunk) {
     if (kSwizzled) {
       const uint4_t v = *(const uint4_t *)(st + row * kPitch + ((chunk ^ ((row >> 1) & 7)) << 3));
-      return (row >> 4) & 1 ? uint4_t{v[2], v[3], v[0], v[1]} : v;
+      return row & 1 ? uint4_t{v[2], v[3], v[0], v[1]} : v;
     }
     return *(const uint4_t *)(st + row * kPitch + (chunk << 3));
   }
@@ -371,6 +374,150 @@ __device__ __forceinline__ void regw_store(const RegW &w, half_t *sW) {
   }
 }
 
+// ---- a wave's share of a tile: products and stores ----------------------------------------
+// 16x16 blocks on v_mfma_f32_16x16x32_f16, the weight as its "A" operand: a lane's four sums of block
+// (i, j) are columns 16 i + 4 (lane >> 4) .. + 3 of row 16 j + (lane & 15).
+// The chip runs these loops against its power limit (1.45 - 1.8 GHz of 2.4 inside the products of a
+// forward), and this instruction does more with it than v_mfma_f32_32x32x16_f16: on operands in
+// registers 1870 against 1600 TFLOP/s, with the loop's LDS reads 1585 against 1420 (8 waves, 64x128).
+// Products of a forward, with the reads placed by hand (`schedule`): FFN1 at 4800 rows 30.9 -> 29.5 us, at
+// 9830 rows 56.6 -> 53.6, FFN2 27.4 -> 24.6 and 46.9 -> 43.9, projection 11.1 -> 9.9.
+template <int BM, int BN, int WTM, int WTN, bool TR>
+struct WaveTile {
+  static constexpr int TM = WTM / 16, TN = WTN / 16;
+  // A large wave tile takes its longer side in parts of eight products (the reads for the next eight then
+  // fit under them and the fragments requested ahead fit the registers); the other side's fragments serve
+  // all parts of 32 k.
+  static constexpr bool kByRows = TM > TN;
+  static constexpr int PARTS = TM * TN <= 8 ? 1 : TM * TN / 8;
+  static_assert((kByRows ? TM : TN) % PARTS == 0, "whole parts");
+  static constexpr int PM = kByRows ? TM / PARTS : TM, PN = kByRows ? TN : TN / PARTS;
+  static constexpr int SUBSTEPS = kBK / 32 * PARTS;
+  float4_t acc[TN][TM];
+  half8_t fw[2][PN], fa[2][PM];
+
+  // the sums start from the bias of their columns (n: column of this lane's first sum in block 0)
+  template <bool BIAS>
+  __device__ __forceinline__ void start(const half_t *bias, int n, int n_last) {
+#pragma unroll
+    for (int i = 0; i < TN; ++i) {
+      float4_t init = {0.f, 0.f, 0.f, 0.f};
+      if (BIAS) {
+        const half4_t b = *(const half4_t *)(bias + min(n + i * 16, n_last));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) init[e] = (float)b[e];
+      }
+#pragma unroll
+      for (int j = 0; j < TM; ++j) acc[i][j] = init;
+    }
+  }
+
+  // fragments of sub-step u (32 k, one part) of the k-step whose tiles lie at sA; the wave tile starts at
+  // row m_w and column n_w of the tile
+  __device__ __forceinline__ void load(const half_t *sA, int m_w, int n_w, int lane, int u) {
+    const half_t *sW = sA + BM * kBK;
+    const int ks = u / PARTS, part = u % PARTS;
+    const int fr = lane & 15, chunk = 4 * ks + (lane >> 4);
+    if (!kByRows || part == 0) {
+#pragma unroll
+      for (int i = 0; i < PN; ++i) {
+        const int n = n_w + ((kByRows ? 0 : part * PN) + i) * 16;
+        fw[(kByRows ? ks : u) & 1][i] = TR ? load_kn_frag<BN>(sW, n, 32 * ks, lane)
+                                           : *(const half8_t *)(sW + (n + fr) * kBK + ((chunk ^ swz(n + fr + BM)) * 8));
+      }
+    }
+    if (kByRows || part == 0) {
+#pragma unroll
+      for (int j = 0; j < PM; ++j) {
+        const int r = m_w + ((kByRows ? part * PM : 0) + j) * 16 + fr;
+        fa[(kByRows ? u : ks) & 1][j] = *(const half8_t *)(sA + r * kBK + ((chunk ^ swz(r)) * 8));
+      }
+    }
+  }
+
+  // Where the LDS reads of a k-step go: those of sub-step u + 1 are spread over the products of sub-step
+  // u, one read (two transpose reads where there are more reads than products) ahead of every few of them.
+  template <int U>
+  __device__ __forceinline__ static void schedule_substep() {
+    constexpr bool kNext = U + 1 < SUBSTEPS, kFirst = (U + 1) % PARTS == 0;
+    constexpr int R = (kNext && (!kByRows || kFirst) ? PN * (TR ? 2 : 1) : 0) + (kNext && (kByRows || kFirst) ? PM : 0);
+    constexpr int P = PN * PM, G = R < P ? (R > 0 ? R : 1) : P;   // groups of reads and products
+    if constexpr (R > 0) {
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        __builtin_amdgcn_sched_group_barrier(kSchedLdsRead, (R + G - 1) / G, 0);
+        __builtin_amdgcn_sched_group_barrier(kSchedMfma, P / G, 0);
+      }
+    }
+    if constexpr (R == 0 || P % G != 0) __builtin_amdgcn_sched_group_barrier(kSchedMfma, R == 0 ? P : P % G, 0);
+  }
+  template <int... U>
+  __device__ __forceinline__ static void schedule(std::integer_sequence<int, U...>) {
+    __builtin_amdgcn_sched_group_barrier(kSchedLdsRead, PN * (TR ? 2 : 1) + PM, 0);
+    (schedule_substep<U>(), ...);
+  }
+
+  // one k-step; `between(u)` runs ahead of the products of sub-step u
+  template <typename Between>
+  __device__ __forceinline__ void step(const half_t *sA, int m_w, int n_w, int lane, Between between) {
+    load(sA, m_w, n_w, lane, 0);
+#pragma unroll
+    for (int u = 0; u < SUBSTEPS; ++u) {
+      if (u + 1 < SUBSTEPS) load(sA, m_w, n_w, lane, u + 1);
+      between(u);
+      const int ks = u / PARTS, part = u % PARTS;
+      const int bw = (kByRows ? ks : u) & 1, ba = (kByRows ? u : ks) & 1;
+#pragma unroll
+      for (int i = 0; i < PN; ++i)
+#pragma unroll
+        for (int j = 0; j < PM; ++j) {
+          float4_t &sum = acc[(kByRows ? 0 : part * PN) + i][(kByRows ? part * PM : 0) + j];
+          sum = __builtin_amdgcn_mfma_f32_16x16x32_f16(fw[bw][i], fa[ba][j], sum, 0, 0, 0);
+        }
+    }
+    schedule(std::make_integer_sequence<int, SUBSTEPS>{});
+  }
+
+  // 32 rows at a time through the wave-private staging tile `st`; (m_first, n_first): the wave tile's
+  // corner in C
+  template <int EPI>
+  __device__ __forceinline__ void store(const GemmArgs &p, half_t *st, int m_first, int n_first, int M,
+                                        int lane) {
+    constexpr int CPRW = WTN / 8;   // 16-byte chunks per staged row
+    constexpr int RPS = 64 / CPRW;  // rows per store instruction
+    const int sr = lane / CPRW, sc = (lane % CPRW) * 8;
+#pragma unroll
+    for (int j = 0; j < TM; ++j) {
+#pragma unroll
+      for (int i = 0; i < TN; ++i) {
+        float4_t v = acc[i][j];
+        if (EPI == kEpiBiasGelu) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = gelu_tanh_f32(v[e]);
+        }
+        *(half4_t *)(st + Staging<WTN>::write_at((j & 1) * 16 + (lane & 15), (lane >> 4) & 1, i * 2 + (lane >> 5))) =
+            half4_t{(half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3]};
+      }
+      if ((j & 1) == 0) continue;
+#pragma unroll
+      for (int r0 = 0; r0 < 32; r0 += RPS) {
+        const int r = r0 + sr;
+        if (sr >= RPS || r >= 32) continue;   // lanes left over when 64 % CPRW != 0
+        const int m = m_first + (j - 1) * 16 + r, n = n_first + sc;
+        const uint4_t v = Staging<WTN>::read(st, r, sc >> 3);
+        if (m < M && n < p.N) {
+          if (EPI == kEpiQkvSplit) {
+            // column n = which*H + g*64 + dd  ->  [which*heads + g][m][dd]
+            *(uint4_t *)(p.c + ((size_t)(n >> 6) * p.rows_cap + m) * 64 + (n & 63)) = v;
+          } else {
+            *(uint4_t *)(p.c + (size_t)m * p.N + n) = v;
+          }
+        }
+      }
+    }
+  }
+};
+
 // XCD-aware tile order over the live tiles of M rows; false: the workgroup has none.  The k slices of a
 // split launch follow each other in it.  (As rows of the grid they left the workgroups of the dead rows
 // between them, and the live ones of the second slice came to lie on the CUs of the first: 230 of 384 rows,
@@ -403,13 +550,12 @@ __device__ __forceinline__ bool tile_at(const GemmArgs &p, int M, int bid, int &
   return true;
 }
 
-template <int BM, int BN, int STAGES, int WM, int WN, int NP, int SCHED, int EPI, bool WKN>
+template <int BM, int BN, int STAGES, int WM, int WN, int NP, int EPI, bool WKN>
 __device__ __forceinline__ void gemm_tile(const GemmArgs &p) {
   constexpr int BK = kBK;
   constexpr int NW = WM * WN;                   // waves that run the MFMAs
   constexpr int NL = NP > 0 ? NP : NW;          // waves that issue the global loads
   constexpr int WTM = BM / WM, WTN = BN / WN;   // wave tile
-  constexpr int TM = WTM / 32, TN = WTN / 32;   // 32x32 MFMA blocks per wave
   constexpr int ROWS = BM + BN;                 // A rows then W rows in one stage
   constexpr int NI = ROWS / 8 / NL;             // load instructions per loading wave per stage
   constexpr int NIA = BM / 8 / NL;              // ... of which the first NIA fetch A rows
@@ -541,47 +687,9 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &p) {
 
   // ---- computing side -------------------------------------------------------
   const int wm = wave / WN, wn = wave % WN;
-  // The accumulators start from the bias of their column (element 4q + e of block (i, j)
-  // is column n0 + wn*WTN + 32 i + 8 q + 4 (lane >> 5) + e), so the epilogue adds nothing.
   constexpr bool kHasBias = EPI == kEpiBiasGelu || EPI == kEpiQkvSplit || EPI == kEpiBias;
-  float16_t acc[TN][TM];
-#pragma unroll
-  for (int i = 0; i < TN; ++i) {
-    float16_t init;
-#pragma unroll
-    for (int v = 0; v < 16; ++v) init[v] = 0.f;
-    if (kHasBias) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int n = min(n0 + wn * WTN + i * 32 + q * 8 + (lane >> 5) * 4, p.N - 4);
-        const half4_t b = *(const half4_t *)(p.bias + n);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) init[4 * q + e] = (float)b[e];
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < TM; ++j) acc[i][j] = init;
-  }
-
-  const int fr_row = lane & 31, fr_kc = lane >> 5;
-  half8_t fw[2][TN], fa[2][TM];
-  auto load_frags = [&](int st, int ks, int b) {
-    const half_t *sA = smem + st * STAGE_HALFS;
-    const half_t *sB = sA + BM * BK;
-#pragma unroll
-    for (int i = 0; i < TN; ++i) {
-      const int r = wn * WTN + i * 32 + fr_row;
-      if (WKN && !kRegW)
-        fw[b][i] = load_kn_frag<BN>(sB, wn * WTN + i * 32, 16 * ks, lane);
-      else
-        fw[b][i] = *(const half8_t *)(sB + r * BK + (((2 * ks + fr_kc) ^ swz(r + BM)) * 8));
-    }
-#pragma unroll
-    for (int j = 0; j < TM; ++j) {
-      const int r = wm * WTM + j * 32 + fr_row;
-      fa[b][j] = *(const half8_t *)(sA + r * BK + (((2 * ks + fr_kc) ^ swz(r)) * 8));
-    }
-  };
+  WaveTile<BM, BN, WTM, WTN, WKN && !kRegW> tile;
+  tile.template start<kHasBias>(p.bias, n0 + wn * WTN + (lane >> 4) * 4, p.N - 4);
   int stage = 0;
   for (int kt = 0; kt < nk; ++kt) {
     // tile kt has landed for this wave once only the younger stages' loads are outstanding
@@ -602,25 +710,13 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &p) {
       if (ps >= STAGES) ps -= STAGES;
       BT_ISSUE_LOADS(kt + STAGES - 1, ps);
     }
-    load_frags(stage, 0, 0);
-    // compiler scheduling strategy that interleaves the LDS reads with the MFMAs
-    if (SCHED == 0) __builtin_amdgcn_iglp_opt(0);
-    if (SCHED == 1) __builtin_amdgcn_iglp_opt(1);
-#pragma unroll
-    for (int ks = 0; ks < BK / 16; ++ks) {
-      if (ks + 1 < BK / 16) load_frags(stage, ks + 1, (ks + 1) & 1);
-      if (kRegW && ks == 1 && kt + 1 < nk) {
+    tile.step(smem + stage * STAGE_HALFS, wm * WTM, wn * WTN, lane, [&](int u) {
+      if (kRegW && u == 2 && kt + 1 < nk) {
         wait_vmcnt<NIA>();            // the weight registers of step kt + 1 (older than its A loads)
         BT_STORE_W(stage ^ 1);
         if (kt + 2 < nk) BT_LOAD_W(kt + 2);
       }
-#pragma unroll
-      for (int i = 0; i < TN; ++i)
-#pragma unroll
-        for (int j = 0; j < TM; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fw[ks & 1][i], fa[ks & 1][j],
-                                                            acc[i][j], 0, 0, 0);
-    }
+    });
     if (++stage == STAGES) stage = 0;
   }
 
@@ -628,69 +724,24 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &p) {
 #undef BT_LOAD_W
 #undef BT_STORE_W
   // ---- epilogue -------------------------------------------------------------
-  // accumulator block (i, j), quad q: columns n..n+3 of row m with
-  //   n = n0 + wn*WTN + i*32 + q*8 + (lane>>5)*4,  m = m0 + wm*WTM + j*32 + (lane&31)
   constexpr int EP = Staging<WTN>::kPitch;   // pitch (halfs) of the wave-private staging tile
   static_assert((size_t)NW * 32 * EP <= (size_t)STAGES * STAGE_HALFS, "staging fits the ring");
   __builtin_amdgcn_s_barrier();   // all waves are done with the last stage
-  half_t *st = smem + wave * 32 * EP;
-  const int row_in = lane & 31, col_in = (lane >> 5) * 4;
   if (EPI == kEpiPartial) {
-    // fp32 partial sums straight from the accumulators: 16 bytes per lane and quad
+    // fp32 partial sums straight from the accumulators: 16 bytes per lane and block
     float *dst = p.c32 + (size_t)split * p.rows_cap * p.N;
 #pragma unroll
-    for (int j = 0; j < TM; ++j) {
-      const int m = m0 + wm * WTM + j * 32 + row_in;
+    for (int j = 0; j < WTM / 16; ++j) {
+      const int m = m0 + wm * WTM + j * 16 + (lane & 15);
 #pragma unroll
-      for (int i = 0; i < TN; ++i)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int n = n0 + wn * WTN + i * 32 + q * 8 + col_in;
-          if (m < M && n < p.N)
-            *(float4_t *)(dst + (size_t)m * p.N + n) =
-                float4_t{acc[i][j][4 * q + 0], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2],
-                         acc[i][j][4 * q + 3]};
-        }
+      for (int i = 0; i < WTN / 16; ++i) {
+        const int n = n0 + wn * WTN + i * 16 + (lane >> 4) * 4;
+        if (m < M && n < p.N) *(float4_t *)(dst + (size_t)m * p.N + n) = tile.acc[i][j];
+      }
     }
     return;
   }
-  constexpr int CPRW = WTN / 8;   // 16-byte chunks per staged row
-  constexpr int RPS = 64 / CPRW;  // rows per store instruction
-  const int sr = lane / CPRW, sc = (lane % CPRW) * 8;
-#pragma unroll
-  for (int j = 0; j < TM; ++j) {
-#pragma unroll
-    for (int i = 0; i < TN; ++i) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        float v0 = acc[i][j][4 * q + 0], v1 = acc[i][j][4 * q + 1];
-        float v2 = acc[i][j][4 * q + 2], v3 = acc[i][j][4 * q + 3];
-        if (EPI == kEpiBiasGelu) {
-          v0 = gelu_tanh_f32(v0);
-          v1 = gelu_tanh_f32(v1);
-          v2 = gelu_tanh_f32(v2);
-          v3 = gelu_tanh_f32(v3);
-        }
-        *(half4_t *)(st + Staging<WTN>::write_at(row_in, lane >> 5, i * 4 + q)) =
-            half4_t{(half_t)v0, (half_t)v1, (half_t)v2, (half_t)v3};
-      }
-    }
-#pragma unroll
-    for (int r0 = 0; r0 < 32; r0 += RPS) {
-      const int r = r0 + sr;
-      if (sr >= RPS || r >= 32) continue;   // lanes left over when 64 % CPRW != 0
-      const int m = m0 + wm * WTM + j * 32 + r, n = n0 + wn * WTN + sc;
-      const uint4_t v = Staging<WTN>::read(st, r, sc >> 3);
-      if (m < M && n < p.N) {
-        if (EPI == kEpiQkvSplit) {
-          // column n = which*H + g*64 + dd  ->  [which*heads + g][m][dd]
-          *(uint4_t *)(p.c + ((size_t)(n >> 6) * p.rows_cap + m) * 64 + (n & 63)) = v;
-        } else {
-          *(uint4_t *)(p.c + (size_t)m * p.N + n) = v;
-        }
-      }
-    }
-  }
+  tile.template store<EPI>(p, smem + wave * 32 * EP, m0 + wm * WTM, n0 + wn * WTN, M, lane);
 }
 
 // ---- persistent form ---------------------------------------------------------------
@@ -702,13 +753,12 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &p) {
 // the first store instruction on: with 228 tiles on 256 CUs the last 7 us of the 31 us of
 // the FFN1 product at batch 16 x 512 are 29.5 MB of stores.)  The grid no longer depends
 // on the row count: a workgroup counts its tiles from the device-side row count.
-template <int BM, int BN, int STAGES, int WM, int WN, int NP, int SCHED, int EPI, bool WKN>
+template <int BM, int BN, int STAGES, int WM, int WN, int NP, int EPI, bool WKN>
 __device__ __forceinline__ void gemm_tiles_flat(const GemmArgs &p) {
   constexpr int BK = kBK;
   constexpr int NW = WM * WN;
   constexpr int NL = NP > 0 ? NP : NW;
   constexpr int WTM = BM / WM, WTN = BN / WN;
-  constexpr int TM = WTM / 32, TN = WTN / 32;
   constexpr int ROWS = BM + BN;
   constexpr int NI = ROWS / 8 / NL;
   constexpr int NIA = BM / 8 / NL;
@@ -867,57 +917,11 @@ __device__ __forceinline__ void gemm_tiles_flat(const GemmArgs &p) {
 
   // ---- computing side ---------------------------------------------------------------
   const int wm = wave / WN, wn = wave % WN;
-  // The accumulators of a tile start from the bias of their columns (element 4q + e of
-  // block (i, j) is column n0 + wn*WTN + 32 i + 8 q + 4 (lane >> 5) + e).
-  float16_t acc[TN][TM];
-  auto init_acc = [&](const half_t *bias_of_tile, int n_limit) {
-#pragma unroll
-    for (int i = 0; i < TN; ++i) {
-      float16_t init;
-#pragma unroll
-      for (int v = 0; v < 16; ++v) init[v] = 0.f;
-      if (kHasBias) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int n = min(wn * WTN + i * 32 + q * 8 + (lane >> 5) * 4, n_limit);
-          const half4_t b = *(const half4_t *)(bias_of_tile + n);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) init[4 * q + e] = (float)b[e];
-        }
-      }
-#pragma unroll
-      for (int j = 0; j < TM; ++j) acc[i][j] = init;
-    }
-  };
+  WaveTile<BM, BN, WTM, WTN, WKN> tile;
+  const int n_lane = wn * WTN + (lane >> 4) * 4;
   int cL = L0, c_slot = 0;
-  {
-    const int n0 = (cL % p.tiles_n) * BN;
-    init_acc(kHasBias ? p.bias + n0 : nullptr, p.N - 4 - n0);   // the first tile: straight from memory
-  }
-
-  const int fr_row = lane & 31, fr_kc = lane >> 5;
-  half8_t fw[2][TN], fa[2][TM];
-  auto load_frags = [&](int st, int ks, int b) {
-    const half_t *sA = smem + st * STAGE_HALFS;
-    const half_t *sB = sA + BM * BK;
-#pragma unroll
-    for (int i = 0; i < TN; ++i) {
-      const int r = wn * WTN + i * 32 + fr_row;
-      if (WKN)
-        fw[b][i] = load_kn_frag<BN>(sB, wn * WTN + i * 32, 16 * ks, lane);
-      else
-        fw[b][i] = *(const half8_t *)(sB + r * BK + (((2 * ks + fr_kc) ^ swz(r + BM)) * 8));
-    }
-#pragma unroll
-    for (int j = 0; j < TM; ++j) {
-      const int r = wm * WTM + j * 32 + fr_row;
-      fa[b][j] = *(const half8_t *)(sA + r * BK + (((2 * ks + fr_kc) ^ swz(r)) * 8));
-    }
-  };
-  const int row_in = lane & 31, col_in = (lane >> 5) * 4;
-  constexpr int CPRW = WTN / 8;   // 16-byte chunks per staged row
-  constexpr int RPS = 64 / CPRW;  // rows per store instruction
-  const int sr = lane / CPRW, sc = (lane % CPRW) * 8;
+  // the first tile's bias straight from memory
+  tile.template start<kHasBias>(p.bias, (cL % p.tiles_n) * BN + n_lane, p.N - 4);
 
   int stage = 0, kt = 0;
   for (int g = 0; g < total; ++g) {
@@ -930,63 +934,18 @@ __device__ __forceinline__ void gemm_tiles_flat(const GemmArgs &p) {
       if (ps >= STAGES) ps -= STAGES;
       issue_next(ps);
     }
-    load_frags(stage, 0, 0);
-    if (SCHED == 0) __builtin_amdgcn_iglp_opt(0);
-    if (SCHED == 1) __builtin_amdgcn_iglp_opt(1);
-#pragma unroll
-    for (int ks = 0; ks < BK / 16; ++ks) {
-      if (ks + 1 < BK / 16) load_frags(stage, ks + 1, (ks + 1) & 1);
-#pragma unroll
-      for (int i = 0; i < TN; ++i)
-#pragma unroll
-        for (int j = 0; j < TM; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fw[ks & 1][i], fa[ks & 1][j],
-                                                            acc[i][j], 0, 0, 0);
-    }
+    tile.step(smem + stage * STAGE_HALFS, wm * WTM, wn * WTN, lane, [](int) {});
     if (++kt == nk) {
       // ---- this tile is complete: store it, start the next from its bias ----
       kt = 0;
       const int tm = cL / p.tiles_n, tn = cL - tm * p.tiles_n;
       const int m0 = tm * BM, n0 = tn * BN;
       __builtin_amdgcn_s_barrier();   // all waves are done reading this stage: it becomes the staging area
-      half_t *st = smem + stage * STAGE_HALFS + wave * 32 * EP;
-#pragma unroll
-      for (int j = 0; j < TM; ++j) {
-#pragma unroll
-        for (int i = 0; i < TN; ++i) {
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            float v0 = acc[i][j][4 * q + 0], v1 = acc[i][j][4 * q + 1];
-            float v2 = acc[i][j][4 * q + 2], v3 = acc[i][j][4 * q + 3];
-            if (EPI == kEpiBiasGelu) {
-              v0 = gelu_tanh_f32(v0);
-              v1 = gelu_tanh_f32(v1);
-              v2 = gelu_tanh_f32(v2);
-              v3 = gelu_tanh_f32(v3);
-            }
-            *(half4_t *)(st + Staging<WTN>::write_at(row_in, lane >> 5, i * 4 + q)) =
-                half4_t{(half_t)v0, (half_t)v1, (half_t)v2, (half_t)v3};
-          }
-        }
-#pragma unroll
-        for (int r0 = 0; r0 < 32; r0 += RPS) {
-          const int r = r0 + sr;
-          if (sr >= RPS || r >= 32) continue;   // lanes left over when 64 % CPRW != 0
-          const int m = m0 + wm * WTM + j * 32 + r, n = n0 + wn * WTN + sc;
-          const uint4_t v = Staging<WTN>::read(st, r, sc >> 3);
-          if (m < M && n < p.N) {
-            if (EPI == kEpiQkvSplit) {
-              // column n = which*H + g*64 + dd  ->  [which*heads + g][m][dd]
-              *(uint4_t *)(p.c + ((size_t)(n >> 6) * p.rows_cap + m) * 64 + (n & 63)) = v;
-            } else {
-              *(uint4_t *)(p.c + (size_t)m * p.N + n) = v;
-            }
-          }
-        }
-      }
+      tile.template store<EPI>(p, smem + stage * STAGE_HALFS + wave * 32 * EP, m0 + wm * WTM, n0 + wn * WTN, M, lane);
       cL += wgx;
       if (++c_slot == STAGES) c_slot = 0;
-      if (g + 1 < total) init_acc(s_bias + c_slot * BN, BN - 4);   // from LDS, where the loading side has put it
+      // (from LDS, where the loading side has put it)
+      if (g + 1 < total) tile.template start<kHasBias>(s_bias + c_slot * BN, n_lane, BN - 4);
     }
     if (++stage == STAGES) stage = 0;
   }
@@ -994,17 +953,17 @@ __device__ __forceinline__ void gemm_tiles_flat(const GemmArgs &p) {
 
 #endif  // __HIP_DEVICE_COMPILE__
 
-template <int BM, int BN, int STAGES, int WM, int WN, int NP, int SCHED, int EPI, bool WKN>
+template <int BM, int BN, int STAGES, int WM, int WN, int NP, int EPI, bool WKN>
 __global__ __launch_bounds__((WM * WN + NP) * 64) void gemm_flat_kernel(BT_GEMM_FIRST, GemmArgs rest) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  gemm_tiles_flat<BM, BN, STAGES, WM, WN, NP, SCHED, EPI, WKN>(gemm_args(BT_GEMM_FIRST_NAMES, rest));
+  gemm_tiles_flat<BM, BN, STAGES, WM, WN, NP, EPI, WKN>(gemm_args(BT_GEMM_FIRST_NAMES, rest));
 #endif
 }
 
-template <int BM, int BN, int STAGES, int WM, int WN, int NP, int SCHED, int EPI, bool WKN>
+template <int BM, int BN, int STAGES, int WM, int WN, int NP, int EPI, bool WKN>
 __global__ __launch_bounds__((WM * WN + NP) * 64) void gemm_kernel(BT_GEMM_FIRST, GemmArgs rest) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  gemm_tile<BM, BN, STAGES, WM, WN, NP, SCHED, EPI, WKN>(gemm_args(BT_GEMM_FIRST_NAMES, rest));
+  gemm_tile<BM, BN, STAGES, WM, WN, NP, EPI, WKN>(gemm_args(BT_GEMM_FIRST_NAMES, rest));
 #endif
 }
 
@@ -1216,12 +1175,12 @@ __global__ __launch_bounds__(256) void transpose_kernel(TransposeArgs a) {
                     threadIdx.x, true);
 }
 
-template <int BM, int BN, int STAGES, int WM, int WN, int NP, int SCHED, int EPI, bool WKN>
+template <int BM, int BN, int STAGES, int WM, int WN, int NP, int EPI, bool WKN>
 static int launch_gemm_tile_as(GemmArgs p, hipStream_t s, int splits) {
   constexpr size_t smem = (size_t)STAGES * (BM + BN) * kBK * sizeof(half_t);
   static_assert(smem <= 160 * 1024, "LDS budget");
   static std::atomic<bool> configured[kMaxDevices];
-  const int rc = allow_dynamic_lds(gemm_kernel<BM, BN, STAGES, WM, WN, NP, SCHED, EPI, WKN>, smem,
+  const int rc = allow_dynamic_lds(gemm_kernel<BM, BN, STAGES, WM, WN, NP, EPI, WKN>, smem,
                                    configured, "hipFuncSetAttribute(gemm_kernel)");
   if (rc != BT_OK) return rc;
   const int tiles_m = (p.rows_cap + BM - 1) / BM;
@@ -1229,16 +1188,16 @@ static int launch_gemm_tile_as(GemmArgs p, hipStream_t s, int splits) {
   p.splits = splits;
   p.tile_grid = (tiles_m * p.tiles_n * splits + 7) / 8 * 8;
   const dim3 grid(p.tile_grid);
-  gemm_kernel<BM, BN, STAGES, WM, WN, NP, SCHED, EPI, WKN>
+  gemm_kernel<BM, BN, STAGES, WM, WN, NP, EPI, WKN>
       <<<grid, (WM * WN + NP) * 64, smem, s>>>(BT_GEMM_FIRST_OF(p), p);
   BT_CHECK_LAUNCH("gemm_kernel");
   return BT_OK;
 }
 
-template <int BM, int BN, int STAGES, int WM, int WN, int NP, int SCHED, int EPI>
+template <int BM, int BN, int STAGES, int WM, int WN, int NP, int EPI>
 static int launch_gemm_tile(GemmArgs p, hipStream_t s, int splits = 1) {
-  return p.w_kn ? launch_gemm_tile_as<BM, BN, STAGES, WM, WN, NP, SCHED, EPI, true>(p, s, splits)
-                : launch_gemm_tile_as<BM, BN, STAGES, WM, WN, NP, SCHED, EPI, false>(p, s, splits);
+  return p.w_kn ? launch_gemm_tile_as<BM, BN, STAGES, WM, WN, NP, EPI, true>(p, s, splits)
+                : launch_gemm_tile_as<BM, BN, STAGES, WM, WN, NP, EPI, false>(p, s, splits);
 }
 
 template <int EPI, bool WKN>
@@ -1267,12 +1226,12 @@ static int cu_count();
 
 // Persistent launch: about one workgroup per CU (a multiple of 8, one share per XCD), each
 // looping over its tiles on the device.
-template <int BM, int BN, int STAGES, int WM, int WN, int NP, int SCHED, int EPI, bool WKN>
+template <int BM, int BN, int STAGES, int WM, int WN, int NP, int EPI, bool WKN>
 static int launch_gemm_flat_as(GemmArgs p, hipStream_t s) {
   constexpr size_t smem = (size_t)STAGES * (BM + BN) * kBK * sizeof(half_t) + STAGES * BN * sizeof(half_t);
   static_assert(smem <= 160 * 1024, "LDS budget");
   static std::atomic<bool> configured[kMaxDevices];
-  const int rc = allow_dynamic_lds(gemm_flat_kernel<BM, BN, STAGES, WM, WN, NP, SCHED, EPI, WKN>,
+  const int rc = allow_dynamic_lds(gemm_flat_kernel<BM, BN, STAGES, WM, WN, NP, EPI, WKN>,
                                    smem, configured, "hipFuncSetAttribute(gemm_flat_kernel)");
   if (rc != BT_OK) return rc;
   const int tiles_m = (p.rows_cap + BM - 1) / BM;
@@ -1283,16 +1242,16 @@ static int launch_gemm_flat_as(GemmArgs p, hipStream_t s) {
   if (wgs > tiles) wgs = tiles;
   p.tile_grid = (int)((wgs + 7) / 8 * 8);
   const dim3 grid((unsigned)p.tile_grid);
-  gemm_flat_kernel<BM, BN, STAGES, WM, WN, NP, SCHED, EPI, WKN>
+  gemm_flat_kernel<BM, BN, STAGES, WM, WN, NP, EPI, WKN>
       <<<grid, (WM * WN + NP) * 64, smem, s>>>(BT_GEMM_FIRST_OF(p), p);
   BT_CHECK_LAUNCH("gemm_flat_kernel");
   return BT_OK;
 }
 
-template <int BM, int BN, int STAGES, int WM, int WN, int NP, int SCHED, int EPI>
+template <int BM, int BN, int STAGES, int WM, int WN, int NP, int EPI>
 static int launch_gemm_flat(GemmArgs p, hipStream_t s) {
-  return p.w_kn ? launch_gemm_flat_as<BM, BN, STAGES, WM, WN, NP, SCHED, EPI, true>(p, s)
-                : launch_gemm_flat_as<BM, BN, STAGES, WM, WN, NP, SCHED, EPI, false>(p, s);
+  return p.w_kn ? launch_gemm_flat_as<BM, BN, STAGES, WM, WN, NP, EPI, true>(p, s)
+                : launch_gemm_flat_as<BM, BN, STAGES, WM, WN, NP, EPI, false>(p, s);
 }
 
 static int cu_count() {
@@ -1493,33 +1452,33 @@ static int launch_gemm(GemmArgs p, hipStream_t s) {
     case 14:
       return launch_gemm_wave_k<EPI>(p, s);
     case 0:
-      return launch_gemm_tile<256, 256, 2, 2, 4, 0, 1, EPI>(p, s);
+      return launch_gemm_tile<256, 256, 2, 2, 4, 0, EPI>(p, s);
     case 2:
-      return launch_gemm_tile<256, 128, 3, 4, 2, 4, 1, EPI>(p, s);
+      return launch_gemm_tile<256, 128, 3, 4, 2, 4, EPI>(p, s);
     case 3:
-      return launch_gemm_tile<256, 192, 2, 4, 2, 4, 1, EPI>(p, s);
+      return launch_gemm_tile<256, 192, 2, 4, 2, 4, EPI>(p, s);
     case 4:
-      return launch_gemm_tile<32, 64, 4, 1, 2, 2, 0, EPI>(p, s);
+      return launch_gemm_tile<32, 64, 4, 1, 2, 2, EPI>(p, s);
     case 5:
-      return launch_gemm_tile<128, 128, 2, 2, 2, 4, 0, EPI>(p, s);
+      return launch_gemm_tile<128, 128, 2, 2, 2, 4, EPI>(p, s);
     case 6:
-      return launch_gemm_flat<256, 128, 3, 4, 2, 4, 1, EPI>(p, s);
+      return launch_gemm_flat<256, 128, 3, 4, 2, 4, EPI>(p, s);
     case 7:
-      return launch_gemm_flat<128, 128, 3, 2, 2, 4, 0, EPI>(p, s);
+      return launch_gemm_flat<128, 128, 3, 2, 2, 4, EPI>(p, s);
     case 8:
-      return launch_gemm_flat<256, 256, 2, 2, 4, 0, 1, EPI>(p, s);
+      return launch_gemm_flat<256, 256, 2, 2, 4, 0, EPI>(p, s);
     case 9:
-      return launch_gemm_tile<64, 64, 4, 2, 2, 4, 0, EPI>(p, s);
+      return launch_gemm_tile<64, 64, 4, 2, 2, 4, EPI>(p, s);
     case 10:
-      return launch_gemm_tile<64, 128, 3, 2, 2, 4, 0, EPI>(p, s);
+      return launch_gemm_tile<64, 128, 3, 2, 2, 4, EPI>(p, s);
     case 11:
-      return launch_gemm_tile<96, 128, 3, 3, 2, 4, 0, EPI>(p, s);
+      return launch_gemm_tile<96, 128, 3, 3, 2, 4, EPI>(p, s);
     case 12:
-      return launch_gemm_tile<128, 192, 3, 2, 2, 4, 0, EPI>(p, s);
+      return launch_gemm_tile<128, 192, 3, 2, 2, 4, EPI>(p, s);
     case 13:
-      return launch_gemm_tile<192, 192, 2, 3, 2, 4, 0, EPI>(p, s);
+      return launch_gemm_tile<192, 192, 2, 3, 2, 4, EPI>(p, s);
     default:
-      return launch_gemm_tile<128, 128, 3, 2, 2, 4, 0, EPI>(p, s);
+      return launch_gemm_tile<128, 128, 3, 2, 2, 4, EPI>(p, s);
   }
 }
 
@@ -1629,8 +1588,8 @@ extern "C" int bt_gemm_splitk(const void *a, const void *wt, void *partials, int
   const long long rows = estimated_rows(p);
   if (wave_k_fits(p, splits)) return launch_gemm_wave_k<kEpiPartial>(p, as_stream(stream), splits);
   if ((rows + 31) / 32 * ((n + 63) / 64) * splits <= cu_count())
-    return launch_gemm_tile<32, 64, 4, 1, 2, 2, 0, kEpiPartial>(p, as_stream(stream), splits);
-  return launch_gemm_tile<64, 64, 4, 2, 2, 4, 0, kEpiPartial>(p, as_stream(stream), splits);
+    return launch_gemm_tile<32, 64, 4, 1, 2, 2, kEpiPartial>(p, as_stream(stream), splits);
+  return launch_gemm_tile<64, 64, 4, 2, 2, 4, kEpiPartial>(p, as_stream(stream), splits);
 }
 
 extern "C" int bt_gemm_bias_gelu(const void *a, const void *wt, const void *bias, void *c,
