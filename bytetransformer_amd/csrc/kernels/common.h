@@ -461,4 +461,20 @@ __device__ __forceinline__ AttWork att_work_balanced(const Args &p, unsigned int
   return w;
 }
 
+// Stores that write through the XCD's L2 instead of leaving the line dirty in it.  The L2s of the eight
+// XCDs are not coherent, so a kernel ends by writing its dirty lines back, and the next one waits for
+// that: 4 us behind a launch that stored 30 MB.  Written through, the lines leave while the other
+// workgroups still compute (and stay in the memory-side cache, which a non-temporal store would pass by).
+// FFN1 at 4800 rows 28.7 -> 26.3 us a launch, at 9830 rows 55.4 -> 52.1, projection at 4800 rows 9.8 ->
+// 9.0, QKV at 911 rows 8.8 -> 8.3.
+// (s_nop: what follows may overwrite the registers of a 16-byte store after two wait states, which the compiler
+// does not see of assembly.  The attention keeps ordinary stores: its rows leave in pieces of 32 bytes, which
+// the L2 joins; written through they cost 0.3 to 1.4 % of a forward.)
+__device__ __forceinline__ void store_through(void *to, uint4_t v) {
+  asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(to), "v"(v));
+}
+__device__ __forceinline__ void store_through(void *to, uint2_t v) {
+  asm volatile("global_store_dwordx2 %0, %1, off sc1" ::"v"(to), "v"(v));
+}
+
 }  // namespace bt

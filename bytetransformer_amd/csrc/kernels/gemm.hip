@@ -508,9 +508,9 @@ struct WaveTile {
         if (m < M && n < p.N) {
           if (EPI == kEpiQkvSplit) {
             // column n = which*H + g*64 + dd  ->  [which*heads + g][m][dd]
-            *(uint4_t *)(p.c + ((size_t)(n >> 6) * p.rows_cap + m) * 64 + (n & 63)) = v;
+            store_through(p.c + ((size_t)(n >> 6) * p.rows_cap + m) * 64 + (n & 63), v);
           } else {
-            *(uint4_t *)(p.c + (size_t)m * p.N + n) = v;
+            store_through(p.c + (size_t)m * p.N + n, v);
           }
         }
       }
@@ -736,7 +736,8 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &p) {
 #pragma unroll
       for (int i = 0; i < WTN / 16; ++i) {
         const int n = n0 + wn * WTN + i * 16 + (lane >> 4) * 4;
-        if (m < M && n < p.N) *(float4_t *)(dst + (size_t)m * p.N + n) = tile.acc[i][j];
+        if (m < M && n < p.N)
+          store_through(dst + (size_t)m * p.N + n, __builtin_bit_cast(uint4_t, tile.acc[i][j]));
       }
     }
     return;
@@ -1126,7 +1127,7 @@ __device__ __forceinline__ void gemm_wave_k(const GemmArgs &p) {
   const int m = m0 + fr_row, n = n0 + wave * 8 + fr_kc * 4;
   if (m >= M || n >= p.N) return;
   if (EPI == kEpiPartial) {
-    *(float4_t *)(p.c32 + ((size_t)split * p.rows_cap + m) * p.N + n) = v;
+    store_through(p.c32 + ((size_t)split * p.rows_cap + m) * p.N + n, __builtin_bit_cast(uint4_t, v));
     return;
   }
   if (EPI == kEpiBiasGelu || EPI == kEpiQkvSplit || EPI == kEpiBias) {
@@ -1140,7 +1141,7 @@ __device__ __forceinline__ void gemm_wave_k(const GemmArgs &p) {
   }
   half_t *dst = EPI == kEpiQkvSplit ? p.c + ((size_t)(n >> 6) * p.rows_cap + m) * 64 + (n & 63)
                                     : p.c + (size_t)m * p.N + n;
-  *(half4_t *)dst = half4_t{(half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3]};
+  store_through(dst, __builtin_bit_cast(uint2_t, half4_t{(half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3]}));
 }
 #endif  // __HIP_DEVICE_COMPILE__
 

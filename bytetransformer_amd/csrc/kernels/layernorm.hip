@@ -73,7 +73,7 @@ __device__ __forceinline__ void ln_finish(const half8_t (&av)[NC], const half8_t
     half8_t y;
 #pragma unroll
     for (int j = 0; j < 8; ++j) y[j] = (half_t)(v[i][j] * rstd * g[j] + bt_[j]);
-    if (live[i]) o[cc[i]] = y;
+    if (live[i]) store_through(o + cc[i], __builtin_bit_cast(uint4_t, y));
   }
 }
 
@@ -146,7 +146,7 @@ __device__ __forceinline__ void layernorm_block(
     const int M = idx[B];
     if (r >= M) {
       const half8_t z = {0, 0, 0, 0, 0, 0, 0, 0};
-      for (int c = lane; c < chunks; c += kWave) dst[dst_row * chunks + c] = z;
+      for (int c = lane; c < chunks; c += kWave) store_through(dst + dst_row * chunks + c, __builtin_bit_cast(uint4_t, z));
       return;
     }
     ln_finish<NC, GB32, kAffineEarly>(av, rv0, bias_v, gh, bh, g32, b32, gamma, beta, cc, live,
@@ -159,7 +159,7 @@ __device__ __forceinline__ void layernorm_block(
     const int start = idx[b], len = idx[b + 1] - start;
     if (s >= len) {
       const half8_t z = {0, 0, 0, 0, 0, 0, 0, 0};
-      for (int c = lane; c < chunks; c += kWave) dst[dst_row * chunks + c] = z;
+      for (int c = lane; c < chunks; c += kWave) store_through(dst + dst_row * chunks + c, __builtin_bit_cast(uint4_t, z));
       return;
     }
     src_row = (size_t)start + s;
