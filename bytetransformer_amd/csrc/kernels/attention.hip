@@ -46,6 +46,7 @@ struct AttArgs {
   float scale_log2e;   // scale * log2(e)
   int padded_rows;
   int nqb;             // query tiles per sequence (set by the launcher)
+  unsigned per_nqb, per_heads;   // floor(2^32 / nqb), floor(2^32 / heads) (set by the launcher)
   unsigned nqb_grid;   // host only: workgroups of the launch
   int xcd_map;         // 0: plain (tile, head, sequence) order, 1: XCD-aware, 2: XCD-aware and balanced over the CUs
   const int *mask_ok;  // optional int[256] from bt_mask_prefix_slots: all non-zero = the mask
@@ -67,22 +68,96 @@ struct AttItem {
   int rank, head, qb;
   bool exists;
 };
+// x / d for any 32-bit x, where inverse = floor(2^32 / d)  (2^32 - 1 for d = 1)
+__device__ __forceinline__ unsigned divide(unsigned x, unsigned d, unsigned inverse) {
+  const unsigned q = (unsigned)((unsigned long long)x * inverse >> 32);   // the quotient or one less
+  return q + (x - q * d >= d ? 1u : 0u);
+}
 __device__ __forceinline__ AttItem att_item(const AttArgs &p) {
   AttItem it;
-  const unsigned lin = blockIdx.x;
-  if (p.xcd_map) {
-    const unsigned slot = lin >> 3, pair = (slot / p.nqb) * 8 + (lin & 7);
-    it.qb = slot % p.nqb;
-    it.exists = pair < (unsigned)(p.B * p.heads);
-    it.rank = pair / p.heads;
-    it.head = pair % p.heads;
-  } else {
-    it.qb = lin % p.nqb;
-    it.head = (lin / p.nqb) % p.heads;
-    it.rank = lin / (p.nqb * p.heads);
-    it.exists = true;
-  }
+  const unsigned lin = workgroup_id();
+  const unsigned slot = p.xcd_map ? lin >> 3 : lin;
+  unsigned pair = divide(slot, p.nqb, p.per_nqb);
+  it.qb = slot - pair * p.nqb;
+  if (p.xcd_map) pair = pair * 8 + (lin & 7);
+  it.exists = pair < (unsigned)(p.B * p.heads);
+  it.rank = divide(pair, p.heads, p.per_heads);
+  it.head = pair - it.rank * p.heads;
   return it;
+}
+
+// What the streaming kernel needs to find its work, as leading kernel arguments of their own: those are in
+// scalar registers when a wave starts, where the struct's fields are memory reads.
+struct AttFirst {
+  const half_t *qkv;
+  const int *batch_idx, *order;   // order: seq_order, or the work list (kAttList)
+  unsigned batch_heads;           // B | heads << 16
+  int S, rows_cap;
+  unsigned grid_work, nqb, per_nqb, per_heads, flags;
+};
+constexpr unsigned kAttMap = 3, kAttList = 4, kAttPadded = 8, kAttEveryKey = 16;   // flags (kAttMap: xcd_map)
+#define BT_ATT_FIRST                                                                                   \
+  const half_t *qkv, const int *batch_idx, const int *order, unsigned batch_heads, int S, int rows_cap, \
+      unsigned grid_work, unsigned nqb, unsigned per_nqb, unsigned per_heads, unsigned flags
+#define BT_ATT_FIRST_NAMES \
+  qkv, batch_idx, order, batch_heads, S, rows_cap, grid_work, nqb, per_nqb, per_heads, flags
+#define BT_ATT_FIRST_OF(f) \
+  f.qkv, f.batch_idx, f.order, f.batch_heads, f.S, f.rows_cap, f.grid_work, f.nqb, f.per_nqb, f.per_heads, f.flags
+inline AttFirst att_first(const AttArgs &a) {
+  const bool list = a.xcd_map == 2 && a.work_list;
+  return AttFirst{a.qkv, a.batch_idx, list ? (const int *)a.work_list : a.seq_order,
+                  (unsigned)a.B | (unsigned)a.heads << 16, a.S, a.rows_cap, a.warm.grid_work, (unsigned)a.nqb, a.per_nqb,
+                  a.per_heads, (unsigned)a.xcd_map | (list ? kAttList : 0) | (a.padded_rows ? kAttPadded : 0) |
+                                   (a.every_key ? kAttEveryKey : 0)};
+}
+__device__ __forceinline__ AttArgs att_args(BT_ATT_FIRST, const AttArgs &rest) {
+  AttArgs p = rest;
+  p.qkv = qkv, p.batch_idx = batch_idx;
+  p.seq_order = flags & kAttList ? nullptr : order;
+  p.work_list = flags & kAttList ? (const int4 *)order : nullptr;
+  p.B = batch_heads & 0xffff, p.heads = batch_heads >> 16, p.S = S, p.rows_cap = rows_cap;
+  p.warm.grid_work = grid_work, p.nqb = nqb, p.per_nqb = per_nqb, p.per_heads = per_heads;
+  p.xcd_map = flags & kAttMap, p.padded_rows = (flags & kAttPadded) != 0, p.every_key = (flags & kAttEveryKey) != 0;
+  return p;
+}
+
+// What a workgroup of the streaming kernel works on, all of it in scalar registers.
+struct AttTile {
+  int b, head, qb, seq_start, seq_len;
+};
+// (scalar loads: nothing in these launches writes what they read.  With the work found in scalar registers
+// 12 layers take, before -> after: 4 x 96 443 -> 437 us, 7 x 217 627 -> 620, 100 x 120 1696 -> 1677.)
+template <typename T>
+__device__ __forceinline__ T scalar_load(const T *from) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return *(const __attribute__((address_space(4))) T *)from;
+#else
+  return *from;
+#endif
+}
+template <int BQ>
+__device__ __forceinline__ bool att_tile(const AttArgs &p, AttTile &t) {
+  if (workgroup_id() >= p.warm.grid_work) return false;
+  if (p.work_list) {
+    // the balanced order, looked up by an earlier launch: one scalar load
+    typedef int entry_t __attribute__((ext_vector_type(4)));
+    const entry_t w = scalar_load((const entry_t *)p.work_list + workgroup_id());
+    t = AttTile{w[0], w[1] & 0xffff, w[1] >> 16, w[2], w[3]};
+    return w[0] >= 0;
+  }
+  if (p.xcd_map == 2) {
+    const AttWork w = att_work_balanced<BQ>(p, workgroup_id());
+    t = AttTile{w.b, w.head, w.qb, w.seq_start, w.len};
+    return w.exists;
+  }
+  const AttItem item = att_item(p);
+  if (!item.exists) return false;
+  const int b = p.seq_order ? scalar_load(p.seq_order + item.rank) : item.rank;
+  // (no offsets: padded rows under a mask tensor, which says everything)
+  const int start = p.batch_idx ? scalar_load(p.batch_idx + b) : b * p.S;
+  const int len = p.batch_idx ? scalar_load(p.batch_idx + b + 1) - start : p.S;
+  t = AttTile{b, item.head, item.qb, start, len};
+  return true;
 }
 
 // 16-byte chunk swizzles of a [rows][64] fp16 tile (8 chunks per 128-byte row).
@@ -127,8 +202,8 @@ constexpr int kTileHalfs = kKT * kHeadDim;       // one K or V tile
 // and output, and the two halves are merged through LDS at the end.  The dependency chain
 // of a query tile - what bounds a launch of a few workgroups per CU, where the longest
 // sequence's workgroups finish last - is half as long, and twice the waves hide it.
-template <int QB, int KIND, int STAGES, int KS = 1>
-__global__ __launch_bounds__(kAttThreads * KS, KS == 1 || KIND ? 2 : 4) void attention_grouped_kernel(AttArgs p) {
+template <int QB, int KIND, int STAGES, int KS>
+__device__ __forceinline__ void attention_tile(const AttArgs &p, const AttTile &item, half_t *ring) {
   constexpr bool ADD = KIND != kAddNone;
   constexpr int BQ = 4 * QB * 16;
   constexpr int AHEAD = STAGES - 1;     // tiles in flight beyond the one being consumed
@@ -136,63 +211,26 @@ __global__ __launch_bounds__(kAttThreads * KS, KS == 1 || KIND ? 2 : 4) void att
   constexpr int kSlotHalfs = KS * 2 * kTileHalfs;
   static_assert(STAGES == 2 || (STAGES == 3 && !ADD), "ring depth; the additive terms alternate between two register sets");
   static_assert(KS == 1 || KS == 2, "key split");
-  __shared__ __attribute__((aligned(1024))) half_t ring[STAGES * kSlotHalfs];
-
-  if (blockIdx.x >= p.warm.grid_work) {
-    warm_slice<kAttThreads * KS>(p.warm);
-    return;
-  }
-  int b, head, seq_start, seq_len, qb_index;
-  if (p.xcd_map == 2 && p.work_list) {
-    // the balanced order, looked up by an earlier launch: one scalar load
-    const int4 w = p.work_list[blockIdx.x];
-    if (w.x < 0) {
-      warm_slice<kAttThreads * KS>(p.warm);
-      return;
-    }
-    b = w.x, head = w.y & 0xffff, qb_index = w.y >> 16, seq_start = w.z, seq_len = w.w;
-  } else if (p.xcd_map == 2) {
-    const AttWork w = att_work_balanced<BQ>(p, blockIdx.x);
-    if (!w.exists) {
-      warm_slice<kAttThreads * KS>(p.warm);
-      return;
-    }
-    b = w.b, head = w.head, seq_start = w.seq_start, seq_len = w.len, qb_index = w.qb;
-  } else {
-    const AttItem item = att_item(p);
-    if (!item.exists) {
-      warm_slice<kAttThreads * KS>(p.warm);
-      return;
-    }
-    b = p.seq_order ? p.seq_order[item.rank] : item.rank, head = item.head;
-    if (p.batch_idx) {
-      seq_start = p.batch_idx[b];
-      seq_len = p.batch_idx[b + 1] - seq_start;
-    } else {   // no offsets: padded rows under a mask tensor, which says everything
-      seq_start = b * p.S;
-      seq_len = p.S;
-    }
-    qb_index = item.qb;
-  }
+  const int b = item.b, head = item.head, seq_start = item.seq_start, seq_len = item.seq_len, qb_index = item.qb;
   // A mask tensor that the device-side check found to be the plain prefix mask adds 0 to
   // the logits of the sequence's keys and removes the others: the lengths say the same.
   const half_t *mask = KIND & kAddMask ? p.mask : nullptr;
   if ((KIND & kAddMask) && p.mask_ok) {
-    const int l = threadIdx.x & 63;
+    const int l = thread_id() & 63;
     const int ok = p.mask_ok[l] & p.mask_ok[l + 64] & p.mask_ok[l + 128] & p.mask_ok[l + 192];
     if (__builtin_amdgcn_ballot_w64(ok == 0) == 0) mask = nullptr;
   }
   // with a mask tensor every one of the S key rows takes part
-  const int klen = mask || p.every_key ? p.S : seq_len;
+  int klen = mask || p.every_key ? p.S : seq_len;
   const int row_start = p.padded_rows ? b * p.S : seq_start;
   const int nq = p.padded_rows ? p.S : klen;
   const int q0 = qb_index * BQ;
-  if (q0 >= nq) {
-    warm_slice<kAttThreads * KS>(p.warm);
-    return;
-  }
+  if (q0 >= nq) return;
+  // (as a vector value: with a scalar length the compiler reshapes the loop over the key tiles, copies the
+  // running output in every tile and needs 132 registers instead of 116, three waves per SIMD instead of four)
+  asm("" : "+v"(klen));
 
-  const int tid = threadIdx.x, lane = tid & 63;
+  const int tid = thread_id(), lane = tid & 63;
   const int wave_all = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wave = wave_all & 3;        // which 16-query blocks
   const int grp = KS > 1 ? wave_all >> 2 : 0;   // which 64-key half of a ring slot (KS = 2)
@@ -501,10 +539,7 @@ __global__ __launch_bounds__(kAttThreads * KS, KS == 1 || KIND ? 2 : 4) void att
       }
     }
     __syncthreads();
-    if (grp == 1) {
-      warm_slice<kAttThreads * KS>(p.warm);
-      return;
-    }
+    if (grp == 1) return;
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
       const float m_other = xch[(qb * 21 + 20) * 64];
@@ -533,6 +568,14 @@ __global__ __launch_bounds__(kAttThreads * KS, KS == 1 || KIND ? 2 : 4) void att
       *(half4_t *)(dst + 16 * db) = half4_t{(half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3]};
     }
   }
+}
+
+template <int QB, int KIND, int STAGES, int KS = 1>
+__global__ __launch_bounds__(kAttThreads * KS, KS == 1 || KIND ? 2 : 4) void attention_grouped_kernel(BT_ATT_FIRST, AttArgs rest) {
+  const AttArgs p = att_args(BT_ATT_FIRST_NAMES, rest);
+  __shared__ __attribute__((aligned(1024))) half_t ring[STAGES * KS * 2 * kTileHalfs];
+  AttTile item;
+  if (att_tile<64 * QB>(p, item)) attention_tile<QB, KIND, STAGES, KS>(p, item, ring);
   warm_slice<kAttThreads * KS>(p.warm);
 }
 
@@ -540,10 +583,10 @@ __global__ __launch_bounds__(kAttThreads * KS, KS == 1 || KIND ? 2 : 4) void att
 template <int BQ>
 __global__ __launch_bounds__(kAttThreads) void attention_worklist_kernel(AttArgs p, int4 *list,
                                                                         unsigned entries) {
-  const unsigned e = blockIdx.x * (kAttThreads / 64) + (threadIdx.x >> 6);
+  const unsigned e = workgroup_id() * (kAttThreads / 64) + (thread_id() >> 6);
   if (e >= entries) return;
   const AttWork w = att_work_balanced<BQ>(p, e);
-  if ((threadIdx.x & 63) == 0)
+  if ((thread_id() & 63) == 0)
     list[e] = w.exists ? int4{w.b, w.head | (w.qb << 16), w.seq_start, w.len} : int4{-1, 0, 0, 0};
 }
 
@@ -559,7 +602,7 @@ __global__ __launch_bounds__(kAttThreads) void attention_short_kernel(AttArgs p)
   half_t *sK = att_smem;                      // [KEYS][64] swizzled
   half_t *sV = att_smem + KEYS * kHeadDim;    // [KEYS][64] swizzled
 
-  if (blockIdx.x >= p.warm.grid_work) {
+  if (workgroup_id() >= p.warm.grid_work) {
     warm_slice<kAttThreads>(p.warm);
     return;
   }
@@ -579,7 +622,7 @@ __global__ __launch_bounds__(kAttThreads) void attention_short_kernel(AttArgs p)
     return;
   }
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = thread_id(), lane = tid & 63, wave = tid >> 6;
   const int lq = lane & 15, lg = lane >> 4;
   const int H = p.heads * kHeadDim;
   const int q = q0 + wave * 16 + lq;
@@ -699,7 +742,9 @@ __global__ __launch_bounds__(kAttThreads) void attention_short_kernel(AttArgs p)
 
 // Size of the 1-D grid for `nqb` query tiles per sequence; fills the mapping fields.
 static unsigned att_grid(AttArgs &a, int nqb, bool streaming = false) {
+  auto inverse = [](unsigned d) { return (unsigned)(d > 1 ? (1ull << 32) / d : 0xffffffffull); };
   a.nqb = nqb;
+  a.per_nqb = inverse(nqb), a.per_heads = inverse(a.heads);
   a.xcd_map = option_attention_xcd_map();
   const unsigned pairs = (unsigned)a.B * a.heads;
   // The balanced list is the streaming kernel's, and pays from the third round of 32
@@ -817,12 +862,13 @@ static void launch_grouped(const AttArgs &a, bool wide, int seq_len, unsigned gr
   // per CU the four-wave form is faster (batch 16 x 512: 16.3 against 19.6 us).  Decided by the
   // workgroups of the attention itself: those that a warm-up hint adds leave the sums as they are.
   const int ks = option_attention_key_split();
+  const AttFirst f = att_first(a);
   if (wide)
-    attention_grouped_kernel<2, KIND, kWideStages><<<grid, kAttThreads, 0, s>>>(a);
+    attention_grouped_kernel<2, KIND, kWideStages><<<grid, kAttThreads, 0, s>>>(BT_ATT_FIRST_OF(f), a);
   else if (ks == 1 || (ks < 0 && seq_len >= 512 && a.warm.grid_work <= 256))
-    attention_grouped_kernel<1, KIND, 2, 2><<<grid, 2 * kAttThreads, 0, s>>>(a);
+    attention_grouped_kernel<1, KIND, 2, 2><<<grid, 2 * kAttThreads, 0, s>>>(BT_ATT_FIRST_OF(f), a);
   else
-    attention_grouped_kernel<1, KIND, 2><<<grid, kAttThreads, 0, s>>>(a);
+    attention_grouped_kernel<1, KIND, 2><<<grid, kAttThreads, 0, s>>>(BT_ATT_FIRST_OF(f), a);
 }
 AttListPlan att_worklist_plan(int B, int S, int heads) {
   AttListPlan out{0, 64, 0};

@@ -157,9 +157,9 @@ struct WarmDuty {
 template <int THREADS>
 __device__ __forceinline__ void warm_slice(const WarmDuty &w) {
   const unsigned lines = w.end[kWarmRanges - 1];
-  if (!lines || blockIdx.x < w.first) return;
-  const unsigned first = (blockIdx.x - w.first) * w.per;
-  touch_lines(w.base, w.end, first + threadIdx.x, min(first + w.per, lines), THREADS);
+  if (!lines || workgroup_id() < w.first) return;
+  const unsigned first = (workgroup_id() - w.first) * w.per;
+  touch_lines(w.base, w.end, first + thread_id(), min(first + w.per, lines), THREADS);
 }
 // Who takes part, for a launch of `grid` workgroups (grown here by the ones that only warm).
 //   Two workgroups per CU and more (option prefetch_min_grid): the last quarter of the issue order -

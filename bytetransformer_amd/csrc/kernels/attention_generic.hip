@@ -69,20 +69,20 @@ __global__ __launch_bounds__(kGenThreads, 2) void attention_generic_kernel(Gener
   constexpr int NLD = CPR / 4;                // load instructions per wave for K, and as many for V
   __shared__ __attribute__((aligned(1024))) half_t ring[2 * 2 * kTile];
 
-  if (blockIdx.x >= p.warm.grid_work) {
+  if (workgroup_id() >= p.warm.grid_work) {
     warm_slice<kGenThreads>(p.warm);
     return;
   }
   int b, head, seq_start, seq_len, qb_index;
   if (p.balanced) {
-    const AttWork w = att_work_balanced<BQ>(p, blockIdx.x);
+    const AttWork w = att_work_balanced<BQ>(p, workgroup_id());
     if (!w.exists) {
       warm_slice<kGenThreads>(p.warm);
       return;
     }
     b = w.b, head = w.head, seq_start = w.seq_start, seq_len = w.len, qb_index = w.qb;
   } else {
-    const unsigned lin = blockIdx.x, slot = lin >> 3;
+    const unsigned lin = workgroup_id(), slot = lin >> 3;
     const unsigned pair = (slot / p.nqb) * 8 + (lin & 7);
     if (pair >= (unsigned)(p.B * p.heads)) {
       warm_slice<kGenThreads>(p.warm);
@@ -104,7 +104,7 @@ __global__ __launch_bounds__(kGenThreads, 2) void attention_generic_kernel(Gener
     return;
   }
 
-  const int tid = threadIdx.x, lane = tid & 63;
+  const int tid = thread_id(), lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lq = lane & 15, lg = lane >> 4;
   const int d = p.d, dc = d >> 3;             // head size, in 16-byte chunks

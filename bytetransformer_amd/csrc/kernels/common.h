@@ -385,6 +385,12 @@ __device__ __forceinline__ TilePanels tile_panels(int tiles_m, int tiles_n, int 
   return TilePanels{tiles_m, tiles_n, __builtin_amdgcn_readfirstlane(max(1, min(gn, tiles_n)))};
 }
 
+// blockIdx.x and threadIdx.x without the call that some floating-point flags keep from being inlined
+// (attention.hip): behind it the workgroup's number counts as a vector value, and every address and branch
+// at the head of a kernel with it.
+__device__ __forceinline__ unsigned workgroup_id() { return __builtin_amdgcn_workgroup_id_x(); }
+__device__ __forceinline__ unsigned thread_id() { return __builtin_amdgcn_workitem_id_x(); }
+
 // ---- balanced work list of the streaming attention kernels -------------------------
 // Within an XCD the hardware deals consecutive workgroups to its 32 CUs round-robin
 // (slot s of the XCD lands on CU s % 32), and a launch of a few workgroups per CU is
@@ -423,7 +429,7 @@ struct AttListArgs {
 template <int BQ, typename Args>
 __device__ __forceinline__ AttWork att_work_balanced(const Args &p, unsigned int workgroup) {
   AttWork w{0, 0, 0, 0, 0, false};
-  const int lane = threadIdx.x & 63;
+  const int lane = thread_id() & 63;
   const int x = workgroup & 7, s = workgroup >> 3;
   const int round = s >> 5, pos = s & 31;
   const int j = (round << 5) + ((round & 1) ? 31 - pos : pos);
