@@ -72,6 +72,8 @@ KERNEL_ABI = {
     "bt_add_bias_residual_layernorm_restore": (c_int, [_P, _P, _P, _P, _P, c_int, _P, _IP, _IP,
                                                        c_int, c_int, c_int, c_float, _P]),
     "bt_gemm_splitk": (c_int, [_P, _P, _P, c_int, _IP, c_int, c_int, c_int, c_int, _P]),
+    "bt_gemm_splitk_rows": (c_int, [_P, _P, _P, c_int, _IP, c_int, c_int, c_int, c_int, c_int, _P]),
+    "bt_gemm_splitk_slices": (c_int, [c_int, c_int, c_int, c_int, c_int]),
     "bt_splitk_layernorm": (c_int, [_P, c_int, _P, _IP, _P, _P, _P, c_int, _P, _IP, _IP, c_int,
                                     c_int, c_int, c_int, c_float, _P]),
     "bt_gemm_f32": (c_int, [_P, _IP, _P, _P, _P, c_int, _IP, c_int, c_int, c_int, c_int, _P]),

@@ -45,12 +45,7 @@ void BertEncoder<OpType>::infer(BertEncoderInferParam<DataType_> ip) {
   const unsigned long long max_tensor = max_rows * hidden;
 
   uint8_t *base = (uint8_t *)ip.buf;
-  DataType_ *qkv_buf = (DataType_ *)base;
-  DataType_ *attr_out_buf = qkv_buf + 3 * tensor;
-  DataType_ *attr_matmul_buf = qkv_buf + 4 * tensor;   // projection, then LN1 in place
-  DataType_ *hidden_buf = qkv_buf + 5 * tensor;        // FFN2 out, then LN2 in place = next input
-  DataType_ *inter_matmul_buf = qkv_buf + 6 * tensor;
-  unsigned long long off = align_up((6 + intermediate_size_) * max_tensor * sizeof(DataType_), 256);
+  unsigned long long off = 0;
   ET_Param et_param;
   et_param.word_idx = (int *)(base + off);
   et_param.batch_idx = et_param.word_idx + max_rows;
@@ -59,8 +54,17 @@ void BertEncoder<OpType>::infer(BertEncoderInferParam<DataType_> ip) {
   int *mask_slots = seq_order + max_batch_size_;       // int[256], padded path only
   off += align_up((max_rows * 2 + 2 * (unsigned long long)max_batch_size_ + 2 + 256) * sizeof(int),
                   256);
-  float *splitk_buf = (float *)(base + off);
-  off += align_up(splitk_scratch_bytes(max_rows, (unsigned long long)hidden), 256);
+  DataType_ *inter_matmul_buf = (DataType_ *)(base + off);
+  DataType_ *attr_matmul_buf = inter_matmul_buf + intermediate_size_ * max_tensor;   // projection, then LN1 in place
+  DataType_ *hidden_buf = attr_matmul_buf + max_tensor;   // FFN2 out, then LN2 in place = next input
+  // (what FFN2 leaves dead lies next to the split-k area: together they are what its partial sums may use)
+  DataType_ *qkv_buf = hidden_buf + max_tensor;
+  DataType_ *attr_out_buf = qkv_buf + 3 * tensor;
+  off += align_up((6 + intermediate_size_) * max_tensor * sizeof(DataType_), 256);
+  float *partials = (float *)qkv_buf;
+  const unsigned long long splitk_bytes = splitk_scratch_bytes(max_rows, (unsigned long long)hidden);
+  const unsigned long long partials_bytes = (base + off + splitk_bytes) - (uint8_t *)qkv_buf;
+  off += align_up(splitk_bytes, 256);
   // the streaming attention's balanced work list: built once per forward beside the offsets
   void *work_list = nullptr;
   if (OpType == OperationType::HALF && size_per_head_ == 64 &&
@@ -183,15 +187,13 @@ void BertEncoder<OpType>::infer(BertEncoderInferParam<DataType_> ip) {
                                      stream));
 
     // few rows, long k: FFN2 as split-k partial sums that the last LayerNorm folds in
-    const long long rows_expected =
-        !valid_rows ? rows : (rows_hint > 0 ? rows_hint : (rows * 3LL + 4) / 5);
-    const int splits = splitk_splits(rows, rows_expected, inter);
+    const int splits = ffn2_slices(rows, valid_rows != nullptr, hidden, inter, partials_bytes);
     if (splits > 1) {
       const bool restore = last && is_remove_padding_;
-      check_bt_error(bt_gemm_splitk(inter_matmul_buf, wt_out, splitk_buf, splits, valid_rows, rows,
-                                    hidden, inter, weight_kn, stream));
+      check_bt_error(bt_gemm_splitk_rows(inter_matmul_buf, wt_out, partials, splits, valid_rows, rows, rows_hint,
+                                         hidden, inter, weight_kn, stream));
       check_bt_error(bt_splitk_layernorm(
-          splitk_buf, splits, attr_matmul_buf, nullptr, w.output_bias, w.output_layernorm_gamma,
+          partials, splits, attr_matmul_buf, nullptr, w.output_bias, w.output_layernorm_gamma,
           w.output_layernorm_beta, use_fp32_ ? 1 : 0,
           restore ? (void *)ip.transformer_output : (void *)ffn2_out,
           restore ? et_param.batch_idx : nullptr, restore ? nullptr : valid_rows, batch_size,

@@ -89,19 +89,25 @@ void BertTransformer<OpType>::bert_infer(BertTransformerInferParam infer_param) 
   const unsigned long long max_rows = (unsigned long long)max_batch_size_ * max_seq_len_;
   const unsigned long long max_tensor = max_rows * hidden;
   uint8_t *base = (uint8_t *)infer_param.buf;
-  DataType_ *inner_buf = (DataType_ *)base;
-  DataType_ *qkv_buf = inner_buf;
-  DataType_ *attr_out_buf = inner_buf + 3 * tensor;
-  DataType_ *attr_matmul_buf = inner_buf + 4 * tensor;
-  DataType_ *inter_matmul_buf = inner_buf + 5 * tensor;
-  unsigned long long off =
-      align_up((5 + param_.intermediate_size) * max_tensor * sizeof(DataType_), 256);
+  // (what FFN2 leaves dead - Q, K, V and the attention's output - lies next to the split-k area: together
+  // they are what its partial sums may use)
+  unsigned long long off = 0;
   ET_Param et_param;
   et_param.word_idx = (int *)(base + off);
   et_param.batch_idx = et_param.word_idx + max_rows;
   et_param.valid_word_num = rows;
   int *seq_order = et_param.batch_idx + max_batch_size_ + 1;   // int[max_batch_size]
   off += align_up((max_rows * 2 + 2 * (unsigned long long)max_batch_size_ + 2) * sizeof(int), 256);
+  DataType_ *inter_matmul_buf = (DataType_ *)(base + off);
+  DataType_ *attr_matmul_buf = inter_matmul_buf + param_.intermediate_size * max_tensor;
+  off += align_up((1 + param_.intermediate_size) * max_tensor * sizeof(DataType_), 256);
+  const unsigned long long copies_off = off;
+  off += align_up((4 + 2 * (unsigned long long)param_.intermediate_size) * hidden * hidden * sizeof(DataType_), 256);
+  DataType_ *qkv_buf = (DataType_ *)(base + off);
+  DataType_ *attr_out_buf = qkv_buf + 3 * tensor;
+  off += align_up(4 * max_tensor * sizeof(DataType_), 256);
+  float *partials = (float *)qkv_buf;
+  const unsigned long long partials_bytes = base + off + splitk_scratch_bytes(max_rows, hidden) - (uint8_t *)qkv_buf;
   const bool have_offsets =
       infer_param.offsets && infer_param.offsets->batch_idx && infer_param.offsets->word_idx;
   const bool streaming_fp16 = OpType == OperationType::HALF && size_per_head_ == 64 &&
@@ -133,7 +139,7 @@ void BertTransformer<OpType>::bert_infer(BertTransformerInferParam infer_param) 
     }
   } else {
     // (copies made by the launch ahead of the layer, or by the first LayerNorm's launch)
-    DataType_ *slot = (DataType_ *)(base + off);
+    DataType_ *slot = (DataType_ *)(base + copies_off);
     for (int i = 0; i < 4; ++i) {
       if (lp.copy[i]) {
         pack_src[pack_count] = w_use[i];
@@ -155,10 +161,6 @@ void BertTransformer<OpType>::bert_infer(BertTransformerInferParam infer_param) 
       slot += (size_t)w_k[i] * w_n[i];
     }
   }
-  off += align_up((4 + 2 * (unsigned long long)param_.intermediate_size) * hidden * hidden *
-                      sizeof(DataType_),
-                  256);
-  float *splitk_buf = (float *)(base + off);
 
   // Padded rows, fp16 streaming attention: the mask tensor is applied unless one pass over
   // it finds the plain prefix mask of its lengths; the prologue leaves that verdict in the
@@ -214,7 +216,7 @@ void BertTransformer<OpType>::bert_infer(BertTransformerInferParam infer_param) 
     // (the compress step of bert_transformer.cu:68-78 folded into its consumers).
     gather = et_param.word_idx;
     restore_target = transformer_out;
-    transformer_out = inner_buf;  // FFN2 output reuses the dead qkv region
+    transformer_out = qkv_buf;  // FFN2 output reuses the dead qkv region
     valid_rows = et_param.batch_idx + batch_size;
     if (have_offsets && rows_hint > 0 && rows_hint < rows) packed_cap = rows_hint;
     rows_hint = rows_to_plan_for(rows_hint, true, batch_size, rows);
@@ -333,14 +335,13 @@ void BertTransformer<OpType>::bert_infer(BertTransformerInferParam infer_param) 
                                    stream));
 
   // few rows, long k: FFN2 as split-k partial sums that the last LayerNorm folds in
-  const long long rows_expected =
-      !valid_rows ? rows : (rows_hint > 0 ? rows_hint : (rows * 3LL + 4) / 5);
-  const int splits = splitk_splits(packed_cap, rows_expected, inter);
+  const int splits =
+      ffn2_slices(packed_cap, valid_rows != nullptr, hidden, inter, partials_bytes);
   if (splits > 1) {
-    check_bt_error(bt_gemm_splitk(inter_matmul_buf, wt_out, splitk_buf, splits, valid_rows,
-                                  packed_cap, hidden, inter, w_kn[3], stream));
+    check_bt_error(bt_gemm_splitk_rows(inter_matmul_buf, wt_out, partials, splits, valid_rows, packed_cap,
+                                       rows_hint, hidden, inter, w_kn[3], stream));
     check_bt_error(bt_splitk_layernorm(
-        splitk_buf, splits, attr_matmul_buf, nullptr, param_.output_bias,
+        partials, splits, attr_matmul_buf, nullptr, param_.output_bias,
         param_.output_layernorm_gamma, param_.output_layernorm_beta, use_fp32_ ? 1 : 0,
         is_remove_padding_ ? restore_target : transformer_out,
         is_remove_padding_ ? et_param.batch_idx : nullptr, nullptr, batch_size, seq_len,

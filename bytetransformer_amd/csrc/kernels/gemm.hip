@@ -1390,8 +1390,55 @@ static bool tuned_mean(const LikelyRows &likely, int n, int k, int epi, int kn, 
 
 // Whether the tiles of gemm_wave_k fit one round: a workgroup fills its CU's LDS, so a second round
 // doubles the launch.
-static bool wave_k_fits(const GemmArgs &p, int splits) {
-  return (estimated_rows(p) + 31) / 32 * ((p.N + kWaveKCols - 1) / kWaveKCols) * splits <= cu_count();
+static bool wave_k_fits(const GemmArgs &p) {
+  return (estimated_rows(p) + 31) / 32 * ((p.N + kWaveKCols - 1) / kWaveKCols) <= cu_count();
+}
+
+// ---- products in k slices ----------------------------------------------------------------
+// FFN2 of up to two thousand rows is a few dozen tiles with a k loop four times as long as the other
+// products': k slices give the idle CUs a share of it, and the LayerNorm that reads the result anyway adds
+// the slices up.  The pair's time is, within 3 % (84 pairs of tile and slices, hidden 768 and 1024, 32
+// to 2736 rows), that of the tile - fixed + k-steps of a slice x step - plus what the LayerNorm reads.
+// Pairs of FFN2 and LayerNorm, k whole -> in slices, us: hidden 768, 230 rows 14.7 -> 10.3 (four slices of
+// 64x64 tiles; two of 32x64 tiles 10.7), 768 rows 16.1 -> 12.8, 911 rows 16.2 -> 14.4, 1500 rows 20.2 -> 16.7,
+// 2000 rows 21.1 -> 19.5; hidden 1024, 640 rows 17.8 -> 14.8, 1300 rows 25.0 -> 21.3.
+struct SliceModel {
+  int id, bm, bn;
+  float fixed_us, step_us;   // launch and LayerNorm of few rows included
+  bool shares_cu;            // a second workgroup fits the CU
+};
+static const SliceModel kSliceModels[] = {
+    {14, 32, kWaveKCols, 9.49f, 0.010f, false}, {4, 32, 64, 8.37f, 0.115f, true},
+    {9, 64, 64, 9.04f, 0.111f, true},           {10, 64, 128, 9.37f, 0.195f, true},
+    {11, 96, 128, 10.39f, 0.242f, false},       {1, 128, 128, 10.53f, 0.231f, false},
+    {12, 128, 192, 12.05f, 0.321f, false}};
+constexpr int kMostSlices = 4;
+// Beyond this many results the slices cost the memory system more than the idle CUs give (2000 rows of
+// 1024: 27.3 against 27.8 us, 2400 rows of 768: 22.8 against 21.9).
+constexpr float kSlicedResults = 1.6e6f;
+// What a tile's launch takes beyond the LayerNorm and the launches themselves, so again in a second round.
+constexpr float kPairUs = 6.f;
+
+static float slice_pair_us(const SliceModel &c, long long m, int n, int k, int splits) {
+  const long long tiles = ((m + c.bm - 1) / c.bm) * ((n + c.bn - 1) / c.bn) * splits;
+  // (a tile that fills its CU finds some CU busy at the last few per cent: 252 workgroups 21.6 us, 216 16.7)
+  const long long at_once = c.shares_cu ? cu_count() : cu_count() - cu_count() / 16;
+  const float rounds = (float)((tiles + at_once - 1) / at_once);
+  const float mn = (float)m * (float)n * 1e-6f, extra = (float)(splits - 1);
+  return kPairUs + rounds * (c.fixed_us - kPairUs + c.step_us * (float)(k / kBK) / (float)splits) + 2.16f * mn +
+         0.49f * mn * extra - (splits > 1 ? 0.86f + 0.12f * (extra - 1.f) : 0.f);
+}
+
+// The fastest tile for a number of slices, and the pair's time with it.
+static const SliceModel &fastest_sliced(const LikelyRows &likely, int n, int k, int splits, float *us) {
+  const SliceModel *best = nullptr;
+  for (const SliceModel &c : kSliceModels) {
+    if (splits == 1 && c.id == 14) continue;   // (measured in slices only)
+    float t = 0.f;
+    for (int i = 0; i < likely.count; ++i) t += likely.weight[i] * slice_pair_us(c, likely.rows[i], n, k, splits);
+    if (!best || t < *us) best = &c, *us = t;
+  }
+  return *best;
 }
 
 template <int EPI>
@@ -1448,7 +1495,7 @@ static int launch_gemm(GemmArgs p, hipStream_t s) {
         choice = tuned;
     }
   }
-  if (forced < 0 && choice == 4 && wave_k_fits(p, 1)) choice = 14;
+  if (forced < 0 && choice == 4 && wave_k_fits(p)) choice = 14;
   switch (choice) {
     case 14:
       return launch_gemm_wave_k<EPI>(p, s);
@@ -1570,9 +1617,42 @@ extern "C" int bt_gemm(const void *a, const void *wt, void *c, const int *valid_
   return launch_gemm<kEpiPlain>(p, as_stream(stream));
 }
 
+// The number of slices changes the order of the sums, so it follows from the sizes of the call alone, not from
+// a row count that a caller may know in one call and not in the next: a padded batch is taken to be 60 %
+// full or, less likely, full.
+extern "C" int bt_gemm_splitk_slices(int rows_cap, int all_live, int n, int k, int most) {
+  if (rows_cap <= 0 || n <= 0 || k < kBK || k % kBK != 0) return 1;
+  if (cu_count() != 256) return 0;
+  GemmArgs p{};
+  p.rows_cap = rows_cap;
+  const LikelyRows full(p);
+  p.rows_cap = (int)((rows_cap * 3LL + 4) / 5);
+  const LikelyRows part(p);
+  const float fills = all_live ? 1.f : 1.f / 3.f;
+  if ((float)(all_live ? full : part).rows[0] * (float)n > kSlicedResults) return 1;
+  int best = 1;
+  float best_us = 0.f;
+  for (int s = 1; s <= kMostSlices && (s == 1 || s <= most); ++s) {
+    if (k / kBK % s != 0) continue;
+    float at_full = 0.f, at_part = 0.f;
+    fastest_sliced(full, n, k, s, &at_full);
+    fastest_sliced(part, n, k, s, &at_part);
+    const float us = fills * at_full + (1.f - fills) * at_part;
+    // (asked to be worth it)
+    if (s == 1 || us < (best == 1 ? 0.97f : 1.f) * best_us) best = s, best_us = us;
+  }
+  return best;
+}
+
 extern "C" int bt_gemm_splitk(const void *a, const void *wt, void *partials, int splits,
                               const int *valid_rows, int rows_cap, int n, int k, int weight_kn,
                               void *stream) {
+  return bt_gemm_splitk_rows(a, wt, partials, splits, valid_rows, rows_cap, 0, n, k, weight_kn, stream);
+}
+
+extern "C" int bt_gemm_splitk_rows(const void *a, const void *wt, void *partials, int splits,
+                                   const int *valid_rows, int rows_cap, int rows_hint, int n, int k,
+                                   int weight_kn, void *stream) {
   int rc = check_gemm_args("bt_gemm_splitk", a, wt, partials, rows_cap, n, k, weight_kn);
   if (rc) return rc;
   BT_REQUIRE(splits >= 1 && splits <= 16 && k % (splits * kBK) == 0, BT_ERR_INVALID_ARGUMENT,
@@ -1580,17 +1660,27 @@ extern "C" int bt_gemm_splitk(const void *a, const void *wt, void *partials, int
              k / kBK);
   if (rows_cap == 0) return BT_OK;
   GemmArgs p{(const half_t *)a, (const half_t *)wt, nullptr, nullptr, valid_rows, nullptr,
-             rows_cap,          n,                  k,       0,       0,          (float *)partials,
+             rows_cap,          n,                  k,       0,       rows_hint,  (float *)partials,
              weight_kn};
-  // Small tiles only: splitting k is for launches whose k loop is the whole run time.  Waves over k while
-  // their tiles fit one round (12 layers at 1 x 32 in all: -2.4 %), 32 rows while
-  // one round of workgroups covers them all, then 64 (hidden 768, k 3072 in two splits with the
-  // LayerNorm behind it: 320 rows 11.6 against 12.1 us, 400 rows 14.0 against 13.0).
-  const long long rows = estimated_rows(p);
-  if (wave_k_fits(p, splits)) return launch_gemm_wave_k<kEpiPartial>(p, as_stream(stream), splits);
-  if ((rows + 31) / 32 * ((n + 63) / 64) * splits <= cu_count())
-    return launch_gemm_tile<32, 64, 4, 1, 2, 2, kEpiPartial>(p, as_stream(stream), splits);
-  return launch_gemm_tile<64, 64, 4, 2, 2, 4, kEpiPartial>(p, as_stream(stream), splits);
+  float us = 0.f;
+  hipStream_t st = as_stream(stream);
+  int tile = fastest_sliced(LikelyRows(p), n, k, splits, &us).id;
+  if (rows_hint > 0) {
+    // (the waves of tile 14 add up in an order of their own: not for a row count's sake either)
+    GemmArgs unnamed = p;
+    unnamed.rows_hint = 0;
+    const int without = fastest_sliced(LikelyRows(unnamed), n, k, splits, &us).id;
+    if ((tile == 14) != (without == 14)) tile = without;
+  }
+  switch (tile) {
+    case 14: return launch_gemm_wave_k<kEpiPartial>(p, st, splits);
+    case 4: return launch_gemm_tile<32, 64, 4, 1, 2, 2, kEpiPartial>(p, st, splits);
+    case 9: return launch_gemm_tile<64, 64, 4, 2, 2, 4, kEpiPartial>(p, st, splits);
+    case 10: return launch_gemm_tile<64, 128, 3, 2, 2, 4, kEpiPartial>(p, st, splits);
+    case 11: return launch_gemm_tile<96, 128, 3, 3, 2, 4, kEpiPartial>(p, st, splits);
+    case 12: return launch_gemm_tile<128, 192, 3, 2, 2, 4, kEpiPartial>(p, st, splits);
+    default: return launch_gemm_tile<128, 128, 3, 2, 2, 4, kEpiPartial>(p, st, splits);
+  }
 }
 
 extern "C" int bt_gemm_bias_gelu(const void *a, const void *wt, const void *bias, void *c,

@@ -392,8 +392,8 @@ extern "C" int bt_splitk_layernorm(const void *partials, int splits, const void 
                                    float eps, void *stream) {
   BT_REQUIRE(partials && residual && bias && gamma && beta && dst, BT_ERR_INVALID_ARGUMENT,
              "bt_splitk_layernorm: null pointer argument");
-  BT_REQUIRE(splits == 2 || splits == 4, BT_ERR_UNSUPPORTED,
-             "bt_splitk_layernorm: splits=%d (supported: 2, 4)", splits);
+  BT_REQUIRE(splits >= 2 && splits <= 4, BT_ERR_UNSUPPORTED,
+             "bt_splitk_layernorm: splits=%d (supported: 2, 3, 4)", splits);
   BT_REQUIRE(rows_cap >= 0, BT_ERR_INVALID_ARGUMENT, "bt_splitk_layernorm: negative rows_cap");
   hipStream_t s = as_stream(stream);
   if (batch_idx) {
@@ -406,21 +406,13 @@ extern "C" int bt_splitk_layernorm(const void *partials, int splits, const void 
     BT_REQUIRE(!residual_row_index, BT_ERR_INVALID_ARGUMENT,
                "bt_splitk_layernorm: no residual gather in restore mode");
     const int padded = batch_size * seq_len;
-    return splits == 2
-               ? launch_ln<true, 2>(partials, residual, bias, gamma, beta, gamma_beta_fp32, dst,
-                                    batch_idx, nullptr, batch_size, seq_len, padded, hidden_dim,
-                                    eps, s, "bt_splitk_layernorm", rows_cap)
-               : launch_ln<true, 4>(partials, residual, bias, gamma, beta, gamma_beta_fp32, dst,
-                                    batch_idx, nullptr, batch_size, seq_len, padded, hidden_dim,
-                                    eps, s, "bt_splitk_layernorm", rows_cap);
+    const auto launch = splits == 2 ? launch_ln<true, 2> : splits == 3 ? launch_ln<true, 3> : launch_ln<true, 4>;
+    return launch(partials, residual, bias, gamma, beta, gamma_beta_fp32, dst, batch_idx, nullptr, batch_size,
+                  seq_len, padded, hidden_dim, eps, s, "bt_splitk_layernorm", rows_cap);
   }
   BT_REQUIRE(!residual_row_index || valid_rows, BT_ERR_INVALID_ARGUMENT,
              "bt_splitk_layernorm: residual_row_index needs valid_rows");
-  return splits == 2
-             ? launch_ln<false, 2>(partials, residual, bias, gamma, beta, gamma_beta_fp32, dst,
-                                   valid_rows, residual_row_index, 0, 1, rows_cap, hidden_dim, eps,
-                                   s, "bt_splitk_layernorm")
-             : launch_ln<false, 4>(partials, residual, bias, gamma, beta, gamma_beta_fp32, dst,
-                                   valid_rows, residual_row_index, 0, 1, rows_cap, hidden_dim, eps,
-                                   s, "bt_splitk_layernorm");
+  const auto launch = splits == 2 ? launch_ln<false, 2> : splits == 3 ? launch_ln<false, 3> : launch_ln<false, 4>;
+  return launch(partials, residual, bias, gamma, beta, gamma_beta_fp32, dst, valid_rows, residual_row_index, 0, 1,
+                rows_cap, hidden_dim, eps, s, "bt_splitk_layernorm", 0);
 }

@@ -424,7 +424,7 @@ int bt_add_bias_residual_layernorm_restore(const void *out, const void *residual
  * dividing k / 64.
  *
  * bt_splitk_layernorm: the add-bias + residual + LayerNorm entry points with the fp32
- * partials (summed, rounded to fp16 once) in the place of `out`; splits 2 or 4.
+ * partials (summed, rounded to fp16 once) in the place of `out`; splits 2, 3 or 4.
  * batch_idx == NULL: packed rows, dst [rows_cap, hidden] (valid_rows / residual_row_index as
  * in bt_add_bias_residual_layernorm); batch_idx != NULL: dst is the padded
  * [batch_size, seq_len, hidden] output with zero fill, and rows_cap (<= batch_size *
@@ -433,6 +433,15 @@ int bt_add_bias_residual_layernorm_restore(const void *out, const void *residual
  */
 int bt_gemm_splitk(const void *a, const void *wt, void *partials, int splits,
                    const int *valid_rows, int rows_cap, int n, int k, int weight_kn, void *stream);
+/* ... with the expected number of live rows (0 = unknown), for the choice of tile only. */
+int bt_gemm_splitk_rows(const void *a, const void *wt, void *partials, int splits,
+                        const int *valid_rows, int rows_cap, int rows_hint, int n, int k,
+                        int weight_kn, void *stream);
+/*
+ * How many slices (1 = leave k whole, at most `most`) make the pair fastest for a product of these
+ * sizes; all_live = every row of rows_cap is live.  0 on a part that the answer was not measured on.
+ */
+int bt_gemm_splitk_slices(int rows_cap, int all_live, int n, int k, int most);
 
 int bt_splitk_layernorm(const void *partials, int splits, const void *residual,
                         const int *residual_row_index, const void *bias, const void *gamma,

@@ -86,10 +86,9 @@ class BertEncoder {
   int num_layers() const { return (int)layers_.size(); }
   bool is_remove_padding() const { return is_remove_padding_; }
 
-  // Scratch (elements of DataType_, T = max_batch*max_seq*hidden): [0,3T) qkv heads |
-  // [3T,4T) attention out | [4T,5T) projection / LN1 | [5T,6T) packed hidden state |
-  // [6T,(6+mult)T) FFN1 | word_idx int[B*S] | batch_idx int[B+1] | seq order int[B] |
-  // split-k partial sums | the streaming attention's work list
+  // Scratch (elements of DataType_, T = max_batch*max_seq*hidden): word_idx int[B*S] | batch_idx
+  // int[B+1] | seq order int[B] | FFN1 mult*T | projection / LN1 T | packed hidden state T | qkv heads
+  // 3T | attention out T (FFN2's partial sums start where the qkv heads were) | split-k partial sums | the streaming attention's work list
   unsigned long long cal_bufsize() const {
     const unsigned long long rows = (unsigned long long)max_batch_size_ * max_seq_len_;
     const unsigned long long tensor = rows * head_num_ * size_per_head_;

@@ -155,15 +155,15 @@ class BertTransformer {
   bool is_remove_padding() const { return is_remove_padding_; }
 
   // Scratch layout (elements of DataType_, T = max_batch*max_seq*hidden):
-  //   [0,3T) qkv heads | [3T,4T) attention out | [4T,5T) projection / LN1 |
-  //   [5T,(5+mult)T) FFN1 | word_idx int[B*S] | batch_idx int[B+1] | seq order int[B] |
-  //   pre-packed weights (3+1+2*mult)*H*H | split-k partial sums | attention scratch (256 ints)
+  //   word_idx int[B*S] | batch_idx int[B+1] | seq order int[B] | FFN1 mult*T | projection / LN1 T |
+  //   pre-packed weights (3+1+2*mult)*H*H | qkv heads 3T | attention out T (FFN2's partial sums start
+  //   where the qkv heads were) | split-k partial sums | attention scratch (256 ints)
   unsigned long long cal_bufsize() {
     const unsigned long long rows = (unsigned long long)max_batch_size_ * max_seq_len_;
     const unsigned long long hidden = (unsigned long long)head_num_ * size_per_head_;
     const unsigned long long tensor = rows * hidden;
-    inner_buf_size_ = (5 + param_.intermediate_size) * tensor * sizeof(DataType_);
-    inner_buf_size_ = align_up(inner_buf_size_, 256);
+    inner_buf_size_ = align_up((1 + param_.intermediate_size) * tensor * sizeof(DataType_), 256);
+    inner_buf_size_ += align_up(4 * tensor * sizeof(DataType_), 256);
     inner_buf_size_ += align_up((rows * 2 + 2 * max_batch_size_ + 2) * sizeof(int), 256);
     inner_buf_size_ += align_up(
         (4 + 2 * (unsigned long long)param_.intermediate_size) * hidden * hidden *

@@ -53,7 +53,8 @@ typedef struct {
 } ET_Param;
 
 // FFN2 with few rows and a long k runs as a split-k GEMM whose fp32 partial sums the last
-// LayerNorm folds in (bt_gemm_splitk / bt_splitk_layernorm): 4 splits up to 192 expected
+// LayerNorm folds in (bt_gemm_splitk_rows / bt_splitk_layernorm).  This is the rule where the kernels
+// library has no measurements (bt_gemm_splitk_slices): 4 splits up to 192 expected
 // rows, 2 up to 640, none beyond, or when the partials of a launch of that
 // capacity exceed the scratch area (4 splits of kSplitKMaxRows rows).  A whole layer in us with k whole / in two
 // splits / in four, in stacks of 12 layers (hidden 768) and 24 whose weights no cache holds together; launched
@@ -80,6 +81,15 @@ inline unsigned long long splitk_scratch_bytes(unsigned long long max_rows,
                                       ? max_rows
                                       : (unsigned long long)kSplitKMaxRows;
   return 4ull * rows * hidden * sizeof(float);   // (= 2 splits of up to twice as many rows)
+}
+// The slices of a layer's FFN2.  `area_bytes` = what the caller can give the partial sums: the activations
+// that are dead by then and the scratch behind them.
+inline int ffn2_slices(int rows_cap, bool packed, int n, int k, unsigned long long area_bytes) {
+  const int rule = splitk_splits(rows_cap, packed ? (rows_cap * 3LL + 4) / 5 : rows_cap, k);
+  if (k < 2048 || splitk_splits(1, 1, 2048) == 1) return rule;   // (short k, or turned off)
+  const unsigned long long fit = area_bytes / ((unsigned long long)rows_cap * n * sizeof(float));
+  const int slices = bt_gemm_splitk_slices(rows_cap, packed ? 0 : 1, n, k, (int)(fit < 16 ? fit : 16));
+  return slices > 0 ? slices : rule;
 }
 
 // Row count that tiles are chosen for.  Without one from the caller the products take 60 % of the

@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 import torch
 
-from bytetransformer_amd import ops, workload
+from bytetransformer_amd import _lib, ops, workload
 from oracle import bert_oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -1415,3 +1415,53 @@ def test_attention_large_logits_do_not_overflow(device):
         assert np.isfinite(g[:M]).all()
         err = np.abs(g[:M].astype(np.float64) - exp)
         assert err.max() <= 2e-2, err.max()
+
+
+@pytest.mark.parametrize("w_kn", [False, True])
+@pytest.mark.parametrize("splits", [2, 3, 4])
+def test_splitk_slices_at_the_edges_of_their_tiles(device, splits, w_kn):
+    """Row counts around the tiles that the slices are made for (32 to 128 rows), with launches sized for more and
+    a last column tile that is not full: the sums of float products of halfs, in any order, differ from float64
+    by less than K * 2^-24 of the sum of magnitudes; rows past the live ones stay as they are."""
+    _say("splitk slices", splits, w_kn)
+    torch.manual_seed(splits)
+    N, K = 776, 768
+    w = (torch.randn(K, N, device=device) * 0.05).half()
+    wt = w if w_kn else w.t().contiguous()
+    for M in (1, 31, 33, 64, 95, 129, 250, 385, 511, 700, 1025, 1500, 2047):
+        rows = M + 37
+        a = torch.randn(rows, K, device=device).half()
+        a[M:] = float("nan")
+        live = torch.tensor([M], dtype=torch.int32, device=device)
+        got = torch.full((splits, rows, N), 7.0, device=device)
+        rc = _lib.kernel_lib().bt_gemm_splitk_rows(a.data_ptr(), wt.data_ptr(), got.data_ptr(), splits, live.data_ptr(), rows,
+                                                   M, N, K, int(w_kn), torch.cuda.current_stream().cuda_stream)
+        assert rc == 0
+        ref = a[:M].double() @ w.double()
+        bound = K * 2.0 ** -24 * (a[:M].double().abs() @ w.double().abs()) + 1e-30
+        assert ((got[:, :M].double().sum(0) - ref).abs() <= bound).all(), M
+        assert (got[:, M:] == 7.0).all(), M
+
+
+def test_splitk_three_slices_restored(device):
+    """Three partial sums folded into the padded output, as into the packed one, and as their sum through the plain
+    LayerNorm: the kernels may round a result to half by way of a float or straight, which is one last bit apart."""
+    torch.manual_seed(3)
+    B, S, H = 2, 40, 768
+    lens = np.array([40, 9])
+    bi = torch.tensor([0, 40, 49], dtype=torch.int32, device=device)
+    parts = torch.randn(3, 49, H, device=device)
+    res, bias, gamma, beta = (torch.randn(*s, device=device).half() for s in ((49, H), (H,), (H,), (H,)))
+    out = torch.full((B, S, H), 5.0, dtype=torch.float16, device=device)
+    ops.splitk_layernorm(parts, res, bias, gamma, beta, out, batch_idx=bi, batch_size=B, seq_len=S)
+    packed = torch.empty(49, H, dtype=torch.float16, device=device)
+    ops.splitk_layernorm(parts, res, bias, gamma, beta, packed)
+    want = torch.zeros_like(out)
+    want[0], want[1, :9] = packed[:40], packed[40:]
+    def last_bit_apart(x, y):
+        x, y = x.double(), y.double()
+        return ((x - y).abs() <= torch.maximum(x.abs(), y.abs()) * 2.0 ** -10 + 2.0 ** -24).all()
+    assert last_bit_apart(out, want) and not out[1, 9:].any()
+    plain = ((parts[0] + parts[1]) + parts[2]).half()
+    ref = ops.add_bias_residual_layernorm(plain, res, bias, gamma, beta)
+    assert last_bit_apart(packed, ref)
