@@ -439,7 +439,7 @@ __device__ __forceinline__ void f32_gemm_tile(const F32GemmArgs &p) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) v[i][e] = gelu_tanh(v[i][e]);
     }
-    *(float4_t *)(p.c + (size_t)m * p.N + n) = v[i];
+    store_through(p.c + (size_t)m * p.N + n, __builtin_bit_cast(uint4_t, v[i]));
   }
 }
 #endif
@@ -781,13 +781,24 @@ __global__ __launch_bounds__(kF32LnRows *kWave) void f32_layernorm_kernel(
   const int r = blockIdx.x * kF32LnRows + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (r >= rows_cap) return;
+  // what no loaded value points at is requested first: behind the statistics, gamma and beta were one more
+  // round trip (rows too wide for the registers keep it)
+  constexpr bool kEarly = NC <= 4;
+  float4_t bias_v[kEarly ? NC : 1], gamma_v[kEarly ? NC : 1], beta_v[kEarly ? NC : 1];
+  if (kEarly) {
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+      const int c = min(lane + i * kWave, chunks - 1);
+      bias_v[i] = bias[c], gamma_v[i] = gamma[c], beta_v[i] = beta[c];
+    }
+  }
   size_t src_row;
   if (RESTORE) {
     const int b = r / S, s = r - b * S;
     const int start = idx[b], len = idx[b + 1] - start;
     if (s >= len) {
       const float4_t z = {0.f, 0.f, 0.f, 0.f};
-      for (int c = lane; c < chunks; c += kWave) dst[(size_t)r * chunks + c] = z;
+      for (int c = lane; c < chunks; c += kWave) store_through(dst + (size_t)r * chunks + c, __builtin_bit_cast(uint4_t, z));
       return;
     }
     src_row = (size_t)start + s;
@@ -806,7 +817,7 @@ __global__ __launch_bounds__(kF32LnRows *kWave) void f32_layernorm_kernel(
     const int c = lane + i * kWave;
     v[i] = float4_t{0.f, 0.f, 0.f, 0.f};
     if (c < chunks) {
-      v[i] = a[c] + rs[c] + bias[c];
+      v[i] = a[c] + rs[c] + (kEarly ? bias_v[i] : bias[c]);
       sum += v[i][0] + v[i][1] + v[i][2] + v[i][3];
     }
   }
@@ -825,7 +836,9 @@ __global__ __launch_bounds__(kF32LnRows *kWave) void f32_layernorm_kernel(
 #pragma unroll
   for (int i = 0; i < NC; ++i) {
     const int c = lane + i * kWave;
-    if (c < chunks) o[c] = v[i] * rstd * gamma[c] + beta[c];
+    if (c < chunks)
+      store_through(o + c, __builtin_bit_cast(uint4_t, v[i] * rstd * (kEarly ? gamma_v[i] : gamma[c]) +
+                                                           (kEarly ? beta_v[i] : beta[c])));
   }
 }
 
