@@ -202,15 +202,18 @@ constexpr int kTileHalfs = kKT * kHeadDim;       // one K or V tile
 // and output, and the two halves are merged through LDS at the end.  The dependency chain
 // of a query tile - what bounds a launch of a few workgroups per CU, where the longest
 // sequence's workgroups finish last - is half as long, and twice the waves hide it.
-template <int QB, int KIND, int STAGES, int KS>
+// WQ = 1, KS = 4, one stage: 16 queries per workgroup, whose four waves take a 64-key tile each.  For a launch that
+// leaves most CUs idle: up to 256 keys are one step instead of four in a row (12 layers at 1 x 256 under a mask,
+// 192 workgroups instead of 48: 429 -> 409 us; at 1 x 128 392 -> 388, at 2 x 120 410 -> 408.  With a second
+// stage for longer sequences a workgroup fills the CU, and those of the warm-up wait for it: 436 -> 454).
+template <int QB, int KIND, int STAGES, int KS, int WQ>
 __device__ __forceinline__ void attention_tile(const AttArgs &p, const AttTile &item, half_t *ring) {
   constexpr bool ADD = KIND != kAddNone;
-  constexpr int BQ = 4 * QB * 16;
-  constexpr int AHEAD = STAGES - 1;     // tiles in flight beyond the one being consumed
+  constexpr int BQ = WQ * QB * 16, kWaves = WQ * KS;
+  constexpr int AHEAD = STAGES > 1 ? STAGES - 1 : 1;     // tiles in flight beyond the one being consumed
   constexpr int kSlotKeys = kKT * KS;   // keys per ring slot
   constexpr int kSlotHalfs = KS * 2 * kTileHalfs;
-  static_assert(STAGES == 2 || (STAGES == 3 && !ADD), "ring depth; the additive terms alternate between two register sets");
-  static_assert(KS == 1 || KS == 2, "key split");
+  static_assert(STAGES <= 2 || (STAGES == 3 && !ADD), "ring depth (one: all keys fit a slot); the additive terms alternate between two register sets");
   const int b = item.b, head = item.head, seq_start = item.seq_start, seq_len = item.seq_len, qb_index = item.qb;
   // A mask tensor that the device-side check found to be the plain prefix mask adds 0 to
   // the logits of the sequence's keys and removes the others: the lengths say the same.
@@ -232,8 +235,8 @@ __device__ __forceinline__ void attention_tile(const AttArgs &p, const AttTile &
 
   const int tid = thread_id(), lane = tid & 63;
   const int wave_all = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wave = wave_all & 3;        // which 16-query blocks
-  const int grp = KS > 1 ? wave_all >> 2 : 0;   // which 64-key half of a ring slot (KS = 2)
+  const int wave = wave_all % WQ;       // which 16-query blocks
+  const int grp = KS > 1 ? wave_all / WQ : 0;   // which 64 keys of a ring slot
   const int lq = lane & 15, lg = lane >> 4;
 
   const size_t head_stride = (size_t)p.rows_cap * kHeadDim;
@@ -273,15 +276,15 @@ __device__ __forceinline__ void attention_tile(const AttArgs &p, const AttTile &
   }
 
   // Slot copy: 16 load instructions per 64-key tile (8 rows each; 0-7 = K, 8-15 = V),
-  // four per wave.  Lane -> (row, slot) and fetches the chunk the swizzle puts
+  // 16 / WQ per wave.  Lane -> (row, slot) and fetches the chunk the swizzle puts
   // in that slot.
   const int ld_row = lane >> 3, ld_slot = lane & 7;
   auto issue_tile = [&](int t, int stage) {
     half_t *sbase = ring + stage * kSlotHalfs;
     const int k0 = t * kSlotKeys;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int id_all = i * 4 * KS + wave_all;   // 0 .. 16 KS - 1
+    for (int i = 0; i < 16 / WQ; ++i) {
+      const int id_all = i * kWaves + wave_all;   // 0 .. 16 KS - 1
       const int sub = id_all >> 4, id = id_all & 15;
       const int row = (id & 7) * 8 + ld_row;
       const int key = min(k0 + sub * kKT + row, klen - 1);
@@ -373,7 +376,7 @@ __device__ __forceinline__ void attention_tile(const AttArgs &p, const AttTile &
     asm volatile("" ::: "memory");
     if (kTermsAhead && t + 1 < ntiles) fetch_terms(t + 1, std::integral_constant<int, (ST + 1) & 1>{});
     if (ADD && !kTermsAhead) fetch_terms(t, std::integral_constant<int, ST & 1>{});
-    if (t + AHEAD < ntiles) issue_tile(t + AHEAD, (ST + AHEAD) % STAGES);
+    if (STAGES > 1 && t + AHEAD < ntiles) issue_tile(t + AHEAD, (ST + AHEAD) % STAGES);
     // a wave whose queries all lie past the sequence, or whose half of the slot lies past
     // the last key, only copies and keeps the barriers
     const int k0 = t * kSlotKeys + grp * kKT;
@@ -517,41 +520,49 @@ __device__ __forceinline__ void attention_tile(const AttArgs &p, const AttTile &
   // one turn of the ring per iteration: tile t sits in stage t % STAGES
   for (int t = 0; t < ntiles; t += STAGES) {
     step(t, std::integral_constant<int, 0>{});
-    if (t + 1 < ntiles) step(t + 1, std::integral_constant<int, 1>{});
+    if constexpr (STAGES >= 2) {
+      if (t + 1 < ntiles) step(t + 1, std::integral_constant<int, 1>{});
+    }
     if constexpr (STAGES == 3) {
       if (t + 2 < ntiles) step(t + 2, std::integral_constant<int, 2>{});
     }
   }
 
   if (KS > 1) {
-    // fold the second key half into the first: waves 4-7 hand over maximum, sum and output
+    // fold the other keys into the first group's: its waves get maximum, sum and output handed over
     // through the ring (lane-major, one word per lane and item: no bank conflicts)
     float *xch = (float *)ring + (size_t)wave * (21 * QB) * 64 + lane;
+    constexpr int kGroup = WQ * 21 * QB * 64;   // words of one group
+    static_assert((KS - 1) * kGroup * sizeof(float) <= STAGES * kSlotHalfs * sizeof(half_t), "the groups fit the ring");
     __syncthreads();           // every wave is done reading the ring
-    if (grp == 1) {
+    if (grp > 0) {
 #pragma unroll
       for (int qb = 0; qb < QB; ++qb) {
-        xch[(qb * 21 + 20) * 64] = m_run[qb];
+        float *to = xch + (grp - 1) * kGroup + qb * 21 * 64;
+        to[20 * 64] = m_run[qb];
 #pragma unroll
         for (int db = 0; db < 5; ++db)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) xch[(qb * 21 + db * 4 + r) * 64] = o[db][qb][r];
+          for (int r = 0; r < 4; ++r) to[(db * 4 + r) * 64] = o[db][qb][r];
       }
     }
     __syncthreads();
-    if (grp == 1) return;
+    if (grp > 0) return;
 #pragma unroll
-    for (int qb = 0; qb < QB; ++qb) {
-      const float m_other = xch[(qb * 21 + 20) * 64];
-      const float m_new = fmaxf(m_run[qb], m_other);
-      const float a_mine = fast_exp2((m_run[qb] - m_new) * cs);
-      const float a_other = fast_exp2((m_other - m_new) * cs);
+    for (int g = 0; g < KS - 1; ++g)
 #pragma unroll
-      for (int db = 0; db < 5; ++db)
+      for (int qb = 0; qb < QB; ++qb) {
+        const float *from = xch + g * kGroup + qb * 21 * 64;
+        const float m_other = from[20 * 64];
+        const float m_new = fmaxf(m_run[qb], m_other);
+        const float a_mine = fast_exp2((m_run[qb] - m_new) * cs);
+        const float a_other = fast_exp2((m_other - m_new) * cs);
+        m_run[qb] = m_new;
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          o[db][qb][r] = o[db][qb][r] * a_mine + xch[(qb * 21 + db * 4 + r) * 64] * a_other;
-    }
+        for (int db = 0; db < 5; ++db)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) o[db][qb][r] = o[db][qb][r] * a_mine + from[(db * 4 + r) * 64] * a_other;
+      }
   }
 
   // O / (l + 1e-6) -> fp16, token-major [row][head*64 + d]
@@ -570,13 +581,13 @@ __device__ __forceinline__ void attention_tile(const AttArgs &p, const AttTile &
   }
 }
 
-template <int QB, int KIND, int STAGES, int KS = 1>
-__global__ __launch_bounds__(kAttThreads * KS, KS == 1 || KIND ? 2 : 4) void attention_grouped_kernel(BT_ATT_FIRST, AttArgs rest) {
+template <int QB, int KIND, int STAGES, int KS = 1, int WQ = 4>
+__global__ __launch_bounds__(64 * WQ * KS, KS == 2 && !KIND ? 4 : 2) void attention_grouped_kernel(BT_ATT_FIRST, AttArgs rest) {
   const AttArgs p = att_args(BT_ATT_FIRST_NAMES, rest);
   __shared__ __attribute__((aligned(1024))) half_t ring[STAGES * KS * 2 * kTileHalfs];
   AttTile item;
-  if (att_tile<64 * QB>(p, item)) attention_tile<QB, KIND, STAGES, KS>(p, item, ring);
-  warm_slice<kAttThreads * KS>(p.warm);
+  if (att_tile<16 * WQ * QB>(p, item)) attention_tile<QB, KIND, STAGES, KS, WQ>(p, item, ring);
+  warm_slice<64 * WQ * KS>(p.warm);
 }
 
 // The balanced order of a launch of `entries` workgroups as a list: one wave per entry.
@@ -841,20 +852,28 @@ namespace bt {
 // third stage did (-0.1 to -2.8 % per forward from batch 1 x 256 to batch 16 x 384; with the
 // balanced work list also -0.8 to -1.9 % at batch 32 x 256 / 384 and 16 x 768, so the switch
 // sits at 1300 workgroups of 128 queries; batch 16 x 512 is within 0.3 % either way).
+// 16-query tiles whose waves share the keys for sequences of 65 to 256 tokens, while a launch of them leaves
+// CUs to the warm-up.
 struct GroupedPlan {
   bool wide;        // 128-query tiles
+  bool narrow;      // 16-query tiles
   unsigned grid;
 };
+constexpr long long kNarrowBlocks = 208;   // (252 workgroups and those of the warm-up: 3 x 100 388 -> 398 us)
 static GroupedPlan plan_grouped(AttArgs &a, int batch_size, int seq_len, int head_num) {
   const long long blocks128 = (long long)((seq_len + 127) / 128) * head_num * batch_size;
   const int qb = option_attention_qb();
   GroupedPlan plan;
   plan.wide = qb == 2 || (qb < 0 && blocks128 >= 1300);
-  plan.grid = att_grid(a, plan.wide ? (seq_len + 127) / 128 : (seq_len + 63) / 64, true);
+  const long long blocks16 = (long long)((seq_len + 15) / 16) * head_num * batch_size;
+  plan.narrow = qb < 0 && option_attention_key_split() < 0 && option_attention_xcd_map() != 3 && seq_len > kKT && seq_len <= 4 * kKT &&
+                blocks16 <= kNarrowBlocks;
+  plan.grid = att_grid(a, plan.wide ? (seq_len + 127) / 128 : plan.narrow ? (seq_len + 15) / 16 : (seq_len + 63) / 64,
+                       true);
   return plan;
 }
 template <int KIND>
-static void launch_grouped(const AttArgs &a, bool wide, int seq_len, unsigned grid, hipStream_t s) {
+static void launch_grouped(const AttArgs &a, const GroupedPlan &plan, int seq_len, unsigned grid, hipStream_t s) {
   // (the additive terms alternate between two register sets, so their kernels take an even ring)
   constexpr int kWideStages = KIND == kAddNone ? 3 : 2;
   // eight waves over two key halves: pays for a few long sequences that leave most CUs
@@ -863,7 +882,9 @@ static void launch_grouped(const AttArgs &a, bool wide, int seq_len, unsigned gr
   // workgroups of the attention itself: those that a warm-up hint adds leave the sums as they are.
   const int ks = option_attention_key_split();
   const AttFirst f = att_first(a);
-  if (wide)
+  if (plan.narrow)
+    attention_grouped_kernel<1, KIND, 1, 4, 1><<<grid, kAttThreads, 0, s>>>(BT_ATT_FIRST_OF(f), a);
+  else if (plan.wide)
     attention_grouped_kernel<2, KIND, kWideStages><<<grid, kAttThreads, 0, s>>>(BT_ATT_FIRST_OF(f), a);
   else if (ks == 1 || (ks < 0 && seq_len >= 512 && a.warm.grid_work <= 256))
     attention_grouped_kernel<1, KIND, 2, 2><<<grid, 2 * kAttThreads, 0, s>>>(BT_ATT_FIRST_OF(f), a);
@@ -952,11 +973,11 @@ extern "C" int bt_attention_grouped(const void *qkv_heads, void *attention_outpu
   rc = plan_warm_duty("bt_attention_grouped", a.warm, grid, prefetch, prefetch_bytes, prefetch_count);
   if (rc) return rc;
   switch (add_kind(a.mask, a.bias, a.scale_log2e)) {
-    case kAddNone: launch_grouped<kAddNone>(a, plan.wide, seq_len, grid, s); break;
-    case kAddMask: launch_grouped<kAddMask>(a, plan.wide, seq_len, grid, s); break;
-    case kAddBias: launch_grouped<kAddBias>(a, plan.wide, seq_len, grid, s); break;
-    case kAddZero: launch_grouped<kAddZero>(a, plan.wide, seq_len, grid, s); break;
-    default: launch_grouped<kAddBoth>(a, plan.wide, seq_len, grid, s); break;
+    case kAddNone: launch_grouped<kAddNone>(a, plan, seq_len, grid, s); break;
+    case kAddMask: launch_grouped<kAddMask>(a, plan, seq_len, grid, s); break;
+    case kAddBias: launch_grouped<kAddBias>(a, plan, seq_len, grid, s); break;
+    case kAddZero: launch_grouped<kAddZero>(a, plan, seq_len, grid, s); break;
+    default: launch_grouped<kAddBoth>(a, plan, seq_len, grid, s); break;
   }
   BT_CHECK_LAUNCH("attention_grouped_kernel");
   return BT_OK;

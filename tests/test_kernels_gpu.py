@@ -1,6 +1,7 @@
 """Per-kernel parity: every C-ABI entry point of libbt_hip.so against the CPU
 oracle on the same seeded inputs.  Integer outputs and copies are bit-exact;
 fp16 results carry the tolerance written in each test."""
+import ctypes
 import math
 
 import numpy as np
@@ -1465,3 +1466,40 @@ def test_splitk_three_slices_restored(device):
     plain = ((parts[0] + parts[1]) + parts[2]).half()
     ref = ops.add_bias_residual_layernorm(plain, res, bias, gamma, beta)
     assert last_bit_apart(packed, ref)
+
+
+@pytest.mark.parametrize("kind", ["none", "mask", "bias", "both", "zero"])
+def test_attention_of_sixteen_queries_a_workgroup(device, kind):
+    """Few sequences of more than one key tile: queries and keys around the tiles of 16, 64 and 256, ragged lengths
+    (an empty one too), with a warm-up hint.  As the four-wave form within the rounding of the probabilities: both
+    round them to half before the second product, in units that differ by at most 2^8, and the output to half."""
+    _say("narrow attention", kind)
+    rs = np.random.RandomState(11)
+    for B, S, heads, lens in ((1, 65, 2, (65,)), (1, 256, 12, (256,)), (1, 321, 12, (257,)), (2, 100, 3, (100, 17)),
+                              (3, 240, 2, (0, 240, 193)), (1, 1000, 4, (999,))):
+        padded = kind in ("mask", "both")
+        rows = B * S
+        qkv = torch.randn(3, heads, rows, 64, device=device).half()
+        off = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+        bi = torch.from_numpy(off).to(device)
+        mask = (torch.rand(B, S, S, device=device) < 0.7).half() if padded else None
+        bias = torch.randn(heads, S, S, device=device).half() if kind in ("bias", "both") else None
+        scale = -0.1 if kind == "zero" else 0.125
+        w = torch.randn(1 << 16, device=device).half()
+        got = {}
+        for split in (-1, 0):
+            ops.set_option("attention_key_split", split)
+            try:
+                out = torch.zeros(rows, heads * 64, dtype=torch.float16, device=device)
+                ptrs = (ctypes.c_void_p * 1)(w.data_ptr())
+                size = (ctypes.c_ulonglong * 1)(w.numel() * 2)
+                rc = _lib.kernel_lib().bt_attention_grouped(
+                    qkv.data_ptr(), out.data_ptr(), bi.data_ptr(), None, mask.data_ptr() if padded else None,
+                    bias.data_ptr() if bias is not None else None, B, S, rows, heads, 64, scale, int(padded), ptrs, size, 1,
+                    None, None, torch.cuda.current_stream().cuda_stream)
+                assert rc == 0
+                got[split] = out.double()
+            finally:
+                ops.set_option("attention_key_split", -1)
+        bound = 2.0 ** -9 * got[0].abs() + 2.0 ** -9 * 4
+        assert ((got[-1] - got[0]).abs() <= bound).all(), (B, S, heads)
