@@ -84,6 +84,11 @@ __device__ __forceinline__ GemmArgs gemm_args(BT_GEMM_FIRST, const GemmArgs &res
   return p;
 }
 
+// Where a product takes its rows from, as a template parameter: the code that counts the mask rows is 9 KB,
+// three quarters of a small kernel, and the kernels of a layer share an instruction cache of 64 KB (12 layers
+// without it where no mask is counted: 1 x 32 385 -> 374 us, 4 x 96 430 -> 422, 7 x 217 638 -> 626).
+constexpr int kMaskNone = 0, kMaskF16 = 1, kMaskF32 = 2;
+
 // ---- rows from the mask ---------------------------------------------------------
 constexpr int kMaskRowsMaxBatch = 64;   // one wave scans the lengths
 
@@ -97,14 +102,15 @@ struct MaskRows {
 
 // All `nwaves` waves of the workgroup take part (one barrier inside).  `s_len`: 64 ints of
 // LDS that nothing else writes until every wave has left this function.
+template <int MASK>
 __device__ __forceinline__ MaskRows mask_rows_setup(const GemmArgs &p, int wave, int nwaves,
                                                     int lane, int *s_len) {
+  using T = std::conditional_t<MASK == kMaskF32, float, half_t>;
   const int B = p.mask_B, S = p.mask_S;
   const size_t plane = (size_t)S * S;
   // R rows per wave in flight at a time: two for up to 2 * nwaves sequences (their 16-byte
   // loads cover rows of up to 1024 halfs in one round trip), four beyond
-  auto count_rows = [&](auto elem_tag, auto r_tag) {
-    using T = decltype(elem_tag);
+  auto count_rows = [&](auto r_tag) {
     constexpr int R = decltype(r_tag)::value;
     const T *m = (const T *)p.mask;
     for (int b0 = wave; b0 < B; b0 += R * nwaves) {
@@ -123,11 +129,7 @@ __device__ __forceinline__ MaskRows mask_rows_setup(const GemmArgs &p, int wave,
   };
   using two = std::integral_constant<int, 2>;
   using four = std::integral_constant<int, 4>;
-  if (p.mask_f32) {
-    if (B <= 2 * nwaves) count_rows(float{}, two{}); else count_rows(float{}, four{});
-  } else {
-    if (B <= 2 * nwaves) count_rows(half_t{}, two{}); else count_rows(half_t{}, four{});
-  }
+  if (B <= 2 * nwaves) count_rows(two{}); else count_rows(four{});
   __syncthreads();
   MaskRows mr;
   mr.len = lane < B ? s_len[lane] : 0;
@@ -550,7 +552,7 @@ __device__ __forceinline__ bool tile_at(const GemmArgs &p, int M, int bid, int &
   return true;
 }
 
-template <int BM, int BN, int STAGES, int WM, int WN, int NP, int EPI, bool WKN>
+template <int BM, int BN, int STAGES, int WM, int WN, int NP, int EPI, bool WKN, int MASK>
 __device__ __forceinline__ void gemm_tile(const GemmArgs &p) {
   constexpr int BK = kBK;
   constexpr int NW = WM * WN;                   // waves that run the MFMAs
@@ -574,10 +576,10 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &p) {
   const int bid = (int)blockIdx.x;
   int M;
   MaskRows mr{};
-  if (p.mask) {
+  if constexpr (MASK != kMaskNone) {
     // the last ring stage is first written after the first barrier of the k loop, which
     // every wave reaches only after it has read the lengths
-    mr = mask_rows_setup(p, wave, NW + NP, lane, (int *)(smem + (STAGES - 1) * STAGE_HALFS));
+    mr = mask_rows_setup<MASK>(p, wave, NW + NP, lane, (int *)(smem + (STAGES - 1) * STAGE_HALFS));
     M = min(mr.M, p.rows_cap);
     if (bid == 0 && wave < NW) mask_rows_write(p, mr, tid, NW * 64, lane);
   } else {
@@ -607,7 +609,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &p) {
   // (load clocks ~ MFMA clocks) that serialisation costs half of the throughput.
   const bool loader = NP == 0 || wave >= NW;
   const int lw = NP == 0 ? wave : wave - NW;    // index among the loading waves
-  const bool gather = p.a_row_index != nullptr || p.mask != nullptr;
+  const bool gather = MASK != kMaskNone || p.a_row_index != nullptr;
   const rsrc_t rs_a =
       gather ? make_rsrc(p.a + k_first, ((size_t)p.rows_cap * p.K - k_first) * sizeof(half_t))
              : make_rsrc(p.a + (size_t)m0 * p.K + k_first,
@@ -622,7 +624,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &p) {
   int voff[NI];
   if (loader) {
     MaskRowSpan span{};
-    if (p.mask) span = mask_rows_span(mr, p.mask_B, lane, m0, min(m0 + BM, M) - 1);
+    if constexpr (MASK != kMaskNone) span = mask_rows_span(mr, p.mask_B, lane, m0, min(m0 + BM, M) - 1);
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
       const int r = (i * NL + lw) * 8 + (lane >> 3);
@@ -630,7 +632,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &p) {
       int row = i < NIA ? r : r - BM;
       if (i < NIA && gather) {   // live rows only hold valid indices
         const int live_row = min(m0 + r, M - 1);
-        row = p.mask ? mask_rows_map(mr, span, live_row) : p.a_row_index[live_row];
+        row = MASK != kMaskNone ? mask_rows_map(mr, span, live_row) : p.a_row_index[live_row];
       }
       voff[i] = (row * p.K + kc * 8) * (int)sizeof(half_t);
       if (WKN && i >= NIA) voff[i] = kn_load_offset<BN>((i - NIA) * NL + lw, lane, p.N, p.N - n0);
@@ -754,7 +756,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &p) {
 // the first store instruction on: with 228 tiles on 256 CUs the last 7 us of the 31 us of
 // the FFN1 product at batch 16 x 512 are 29.5 MB of stores.)  The grid no longer depends
 // on the row count: a workgroup counts its tiles from the device-side row count.
-template <int BM, int BN, int STAGES, int WM, int WN, int NP, int EPI, bool WKN>
+template <int BM, int BN, int STAGES, int WM, int WN, int NP, int EPI, bool WKN, int MASK>
 __device__ __forceinline__ void gemm_tiles_flat(const GemmArgs &p) {
   constexpr int BK = kBK;
   constexpr int NW = WM * WN;
@@ -779,9 +781,9 @@ __device__ __forceinline__ void gemm_tiles_flat(const GemmArgs &p) {
   const int bid = (int)blockIdx.x;
   int M;
   MaskRows mr{};
-  if (p.mask) {
+  if constexpr (MASK != kMaskNone) {
     // (the last ring stage: first written after the first barrier of the k loop)
-    mr = mask_rows_setup(p, wave, NW + NP, lane, (int *)(smem + (STAGES - 1) * STAGE_HALFS));
+    mr = mask_rows_setup<MASK>(p, wave, NW + NP, lane, (int *)(smem + (STAGES - 1) * STAGE_HALFS));
     M = min(mr.M, p.rows_cap);
     if (bid == 0 && wave < NW) mask_rows_write(p, mr, tid, NW * 64, lane);
   } else {
@@ -804,7 +806,7 @@ __device__ __forceinline__ void gemm_tiles_flat(const GemmArgs &p) {
   // ---- loading side: a cursor (tile, k-step) STAGES - 1 steps ahead of the products ----
   const bool loader = NP == 0 || wave >= NW;
   const int lw = NP == 0 ? wave : wave - NW;
-  const bool gather = p.a_row_index != nullptr || p.mask != nullptr;
+  const bool gather = MASK != kMaskNone || p.a_row_index != nullptr;
   rsrc_t rs_a = make_rsrc(p.a, 0), rs_w = make_rsrc(p.wt, 0);
   constexpr bool kHasBias = EPI == kEpiBiasGelu || EPI == kEpiQkvSplit || EPI == kEpiBias;
   // The bias of a tile's columns reaches the computing waves through LDS, fetched by the
@@ -824,12 +826,12 @@ __device__ __forceinline__ void gemm_tiles_flat(const GemmArgs &p) {
   auto fetch_indices = [&](int Lt) {
     const int m0 = (Lt / p.tiles_n) * BM;
     MaskRowSpan span{};
-    if (p.mask) span = mask_rows_span(mr, p.mask_B, lane, m0, min(m0 + BM, M) - 1);
+    if constexpr (MASK != kMaskNone) span = mask_rows_span(mr, p.mask_B, lane, m0, min(m0 + BM, M) - 1);
 #pragma unroll
     for (int i = 0; i < NIA; ++i) {
       const int r = (i * NL + lw) * 8 + (lane >> 3);
       const int live_row = min(m0 + r, M - 1);   // live rows only hold valid indices
-      idx_next[i] = p.mask ? mask_rows_map(mr, span, live_row) : p.a_row_index[live_row];
+      idx_next[i] = MASK != kMaskNone ? mask_rows_map(mr, span, live_row) : p.a_row_index[live_row];
     }
   };
   auto load_setup = [&](int Lt, bool more, bool bias_to_lds) {
@@ -954,17 +956,17 @@ __device__ __forceinline__ void gemm_tiles_flat(const GemmArgs &p) {
 
 #endif  // __HIP_DEVICE_COMPILE__
 
-template <int BM, int BN, int STAGES, int WM, int WN, int NP, int EPI, bool WKN>
+template <int BM, int BN, int STAGES, int WM, int WN, int NP, int EPI, bool WKN, int MASK>
 __global__ __launch_bounds__((WM * WN + NP) * 64) void gemm_flat_kernel(BT_GEMM_FIRST, GemmArgs rest) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  gemm_tiles_flat<BM, BN, STAGES, WM, WN, NP, EPI, WKN>(gemm_args(BT_GEMM_FIRST_NAMES, rest));
+  gemm_tiles_flat<BM, BN, STAGES, WM, WN, NP, EPI, WKN, MASK>(gemm_args(BT_GEMM_FIRST_NAMES, rest));
 #endif
 }
 
-template <int BM, int BN, int STAGES, int WM, int WN, int NP, int EPI, bool WKN>
+template <int BM, int BN, int STAGES, int WM, int WN, int NP, int EPI, bool WKN, int MASK>
 __global__ __launch_bounds__((WM * WN + NP) * 64) void gemm_kernel(BT_GEMM_FIRST, GemmArgs rest) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  gemm_tile<BM, BN, STAGES, WM, WN, NP, EPI, WKN>(gemm_args(BT_GEMM_FIRST_NAMES, rest));
+  gemm_tile<BM, BN, STAGES, WM, WN, NP, EPI, WKN, MASK>(gemm_args(BT_GEMM_FIRST_NAMES, rest));
 #endif
 }
 
@@ -994,7 +996,7 @@ __device__ __forceinline__ half8_t lds_wait_operand(uint2_t (&w)[2]) {
   return __builtin_bit_cast(half8_t, uint4_t{w[0][0], w[0][1], w[1][0], w[1][1]});
 }
 
-template <int EPI, bool WKN>
+template <int EPI, bool WKN, int MASK>
 __device__ __forceinline__ void gemm_wave_k(const GemmArgs &p) {
   constexpr int BM = 32, BN = kWaveKCols, BK = kBK, NW = kWaveKWaves, DEPTH = kWaveKDepth;
   constexpr int KS = BK / 16;
@@ -1012,8 +1014,8 @@ __device__ __forceinline__ void gemm_wave_k(const GemmArgs &p) {
   half_t *ring = gemm_smem + wave * DEPTH * STEP_HALFS;
   int M;
   MaskRows mr{};
-  if (p.mask) {
-    mr = mask_rows_setup(p, wave, NW, lane, (int *)(gemm_smem + NW * DEPTH * STEP_HALFS));
+  if constexpr (MASK != kMaskNone) {
+    mr = mask_rows_setup<MASK>(p, wave, NW, lane, (int *)(gemm_smem + NW * DEPTH * STEP_HALFS));
     M = min(mr.M, p.rows_cap);
     if (bid == 0) mask_rows_write(p, mr, tid, NW * 64, lane);
   } else {
@@ -1026,7 +1028,7 @@ __device__ __forceinline__ void gemm_wave_k(const GemmArgs &p) {
   const int k_first = EPI == kEpiPartial ? split * nk * BK : 0;
   const int mine = (nk - wave + NW - 1) / NW;   // (0 where there are fewer steps than waves)
 
-  const bool gather = p.a_row_index != nullptr || p.mask != nullptr;
+  const bool gather = MASK != kMaskNone || p.a_row_index != nullptr;
   const rsrc_t rs_a =
       gather ? make_rsrc(p.a + k_first, ((size_t)p.rows_cap * p.K - k_first) * sizeof(half_t))
              : make_rsrc(p.a + (size_t)m0 * p.K + k_first,
@@ -1039,7 +1041,7 @@ __device__ __forceinline__ void gemm_wave_k(const GemmArgs &p) {
   int voff[NI];
   {
     MaskRowSpan span{};
-    if (p.mask) span = mask_rows_span(mr, p.mask_B, lane, m0, min(m0 + BM, M) - 1);
+    if constexpr (MASK != kMaskNone) span = mask_rows_span(mr, p.mask_B, lane, m0, min(m0 + BM, M) - 1);
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
       const int r = i * 8 + (lane >> 3);
@@ -1047,7 +1049,7 @@ __device__ __forceinline__ void gemm_wave_k(const GemmArgs &p) {
       int row = i < NIA ? r : r - BM;
       if (i < NIA && gather) {
         const int live_row = min(m0 + r, M - 1);
-        row = p.mask ? mask_rows_map(mr, span, live_row) : p.a_row_index[live_row];
+        row = MASK != kMaskNone ? mask_rows_map(mr, span, live_row) : p.a_row_index[live_row];
       }
       voff[i] = (row * p.K + kc * 8) * (int)sizeof(half_t);
       if (WKN && i >= NIA) voff[i] = kn_load_offset<BN>(i - NIA, lane, p.N, p.N - n0);
@@ -1145,10 +1147,10 @@ __device__ __forceinline__ void gemm_wave_k(const GemmArgs &p) {
 }
 #endif  // __HIP_DEVICE_COMPILE__
 
-template <int EPI, bool WKN>
+template <int EPI, bool WKN, int MASK>
 __global__ __launch_bounds__(kWaveKWaves * 64) void gemm_wave_k_kernel(BT_GEMM_FIRST, GemmArgs rest) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  gemm_wave_k<EPI, WKN>(gemm_args(BT_GEMM_FIRST_NAMES, rest));
+  gemm_wave_k<EPI, WKN, MASK>(gemm_args(BT_GEMM_FIRST_NAMES, rest));
 #endif
 }
 
@@ -1176,12 +1178,23 @@ __global__ __launch_bounds__(256) void transpose_kernel(TransposeArgs a) {
                     threadIdx.x, true);
 }
 
-template <int BM, int BN, int STAGES, int WM, int WN, int NP, int EPI, bool WKN>
+// Calls `launch` with the weight layout and the source of the rows as compile-time constants.
+template <int EPI, typename Launch>
+static int by_layout(const GemmArgs &p, Launch launch) {
+  auto with = [&](auto mask) { return p.w_kn ? launch(std::true_type{}, mask) : launch(std::false_type{}, mask); };
+  if constexpr (EPI == kEpiQkvSplit || EPI == kEpiBias) {
+    if (p.mask && p.mask_f32) return with(std::integral_constant<int, kMaskF32>{});
+    if (p.mask) return with(std::integral_constant<int, kMaskF16>{});
+  }
+  return with(std::integral_constant<int, kMaskNone>{});
+}
+
+template <int BM, int BN, int STAGES, int WM, int WN, int NP, int EPI, bool WKN, int MASK>
 static int launch_gemm_tile_as(GemmArgs p, hipStream_t s, int splits) {
   constexpr size_t smem = (size_t)STAGES * (BM + BN) * kBK * sizeof(half_t);
   static_assert(smem <= 160 * 1024, "LDS budget");
   static std::atomic<bool> configured[kMaxDevices];
-  const int rc = allow_dynamic_lds(gemm_kernel<BM, BN, STAGES, WM, WN, NP, EPI, WKN>, smem,
+  const int rc = allow_dynamic_lds(gemm_kernel<BM, BN, STAGES, WM, WN, NP, EPI, WKN, MASK>, smem,
                                    configured, "hipFuncSetAttribute(gemm_kernel)");
   if (rc != BT_OK) return rc;
   const int tiles_m = (p.rows_cap + BM - 1) / BM;
@@ -1189,7 +1202,7 @@ static int launch_gemm_tile_as(GemmArgs p, hipStream_t s, int splits) {
   p.splits = splits;
   p.tile_grid = (tiles_m * p.tiles_n * splits + 7) / 8 * 8;
   const dim3 grid(p.tile_grid);
-  gemm_kernel<BM, BN, STAGES, WM, WN, NP, EPI, WKN>
+  gemm_kernel<BM, BN, STAGES, WM, WN, NP, EPI, WKN, MASK>
       <<<grid, (WM * WN + NP) * 64, smem, s>>>(BT_GEMM_FIRST_OF(p), p);
   BT_CHECK_LAUNCH("gemm_kernel");
   return BT_OK;
@@ -1197,42 +1210,45 @@ static int launch_gemm_tile_as(GemmArgs p, hipStream_t s, int splits) {
 
 template <int BM, int BN, int STAGES, int WM, int WN, int NP, int EPI>
 static int launch_gemm_tile(GemmArgs p, hipStream_t s, int splits = 1) {
-  return p.w_kn ? launch_gemm_tile_as<BM, BN, STAGES, WM, WN, NP, EPI, true>(p, s, splits)
-                : launch_gemm_tile_as<BM, BN, STAGES, WM, WN, NP, EPI, false>(p, s, splits);
+  return by_layout<EPI>(p, [&](auto wkn, auto mask) {
+    return launch_gemm_tile_as<BM, BN, STAGES, WM, WN, NP, EPI, wkn(), mask()>(p, s, splits);
+  });
 }
 
-template <int EPI, bool WKN>
+template <int EPI, bool WKN, int MASK>
 static int launch_gemm_wave_k_as(GemmArgs p, hipStream_t s, int splits) {
   // (and 256 bytes for the lengths of a launch that counts the mask rows)
   constexpr size_t smem = (size_t)kWaveKWaves * kWaveKDepth * (32 + kWaveKCols) * kBK * sizeof(half_t) + 256;
   static_assert(smem <= 160 * 1024, "LDS budget");
   static std::atomic<bool> configured[kMaxDevices];
-  const int rc = allow_dynamic_lds(gemm_wave_k_kernel<EPI, WKN>, smem, configured,
+  const int rc = allow_dynamic_lds(gemm_wave_k_kernel<EPI, WKN, MASK>, smem, configured,
                                    "hipFuncSetAttribute(gemm_wave_k_kernel)");
   if (rc != BT_OK) return rc;
   p.tiles_n = (p.N + kWaveKCols - 1) / kWaveKCols;
   p.splits = splits;
   p.tile_grid = ((p.rows_cap + 31) / 32 * p.tiles_n * splits + 7) / 8 * 8;
-  gemm_wave_k_kernel<EPI, WKN><<<dim3(p.tile_grid), kWaveKWaves * 64, smem, s>>>(BT_GEMM_FIRST_OF(p), p);
+  gemm_wave_k_kernel<EPI, WKN, MASK><<<dim3(p.tile_grid), kWaveKWaves * 64, smem, s>>>(BT_GEMM_FIRST_OF(p), p);
   BT_CHECK_LAUNCH("gemm_wave_k_kernel");
   return BT_OK;
 }
 
 template <int EPI>
 static int launch_gemm_wave_k(GemmArgs p, hipStream_t s, int splits = 1) {
-  return p.w_kn ? launch_gemm_wave_k_as<EPI, true>(p, s, splits) : launch_gemm_wave_k_as<EPI, false>(p, s, splits);
+  return by_layout<EPI>(p, [&](auto wkn, auto mask) {
+    return launch_gemm_wave_k_as<EPI, wkn(), mask()>(p, s, splits);
+  });
 }
 
 static int cu_count();
 
 // Persistent launch: about one workgroup per CU (a multiple of 8, one share per XCD), each
 // looping over its tiles on the device.
-template <int BM, int BN, int STAGES, int WM, int WN, int NP, int EPI, bool WKN>
+template <int BM, int BN, int STAGES, int WM, int WN, int NP, int EPI, bool WKN, int MASK>
 static int launch_gemm_flat_as(GemmArgs p, hipStream_t s) {
   constexpr size_t smem = (size_t)STAGES * (BM + BN) * kBK * sizeof(half_t) + STAGES * BN * sizeof(half_t);
   static_assert(smem <= 160 * 1024, "LDS budget");
   static std::atomic<bool> configured[kMaxDevices];
-  const int rc = allow_dynamic_lds(gemm_flat_kernel<BM, BN, STAGES, WM, WN, NP, EPI, WKN>,
+  const int rc = allow_dynamic_lds(gemm_flat_kernel<BM, BN, STAGES, WM, WN, NP, EPI, WKN, MASK>,
                                    smem, configured, "hipFuncSetAttribute(gemm_flat_kernel)");
   if (rc != BT_OK) return rc;
   const int tiles_m = (p.rows_cap + BM - 1) / BM;
@@ -1243,7 +1259,7 @@ static int launch_gemm_flat_as(GemmArgs p, hipStream_t s) {
   if (wgs > tiles) wgs = tiles;
   p.tile_grid = (int)((wgs + 7) / 8 * 8);
   const dim3 grid((unsigned)p.tile_grid);
-  gemm_flat_kernel<BM, BN, STAGES, WM, WN, NP, EPI, WKN>
+  gemm_flat_kernel<BM, BN, STAGES, WM, WN, NP, EPI, WKN, MASK>
       <<<grid, (WM * WN + NP) * 64, smem, s>>>(BT_GEMM_FIRST_OF(p), p);
   BT_CHECK_LAUNCH("gemm_flat_kernel");
   return BT_OK;
@@ -1251,8 +1267,9 @@ static int launch_gemm_flat_as(GemmArgs p, hipStream_t s) {
 
 template <int BM, int BN, int STAGES, int WM, int WN, int NP, int EPI>
 static int launch_gemm_flat(GemmArgs p, hipStream_t s) {
-  return p.w_kn ? launch_gemm_flat_as<BM, BN, STAGES, WM, WN, NP, EPI, true>(p, s)
-                : launch_gemm_flat_as<BM, BN, STAGES, WM, WN, NP, EPI, false>(p, s);
+  return by_layout<EPI>(p, [&](auto wkn, auto mask) {
+    return launch_gemm_flat_as<BM, BN, STAGES, WM, WN, NP, EPI, wkn(), mask()>(p, s);
+  });
 }
 
 static int cu_count() {
