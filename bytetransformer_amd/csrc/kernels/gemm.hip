@@ -520,7 +520,7 @@ struct WaveTile {
   }
 };
 
-// XCD-aware tile order over the live tiles of M rows; false: the workgroup has none.  The k slices of a
+// XCD-aware tile order over the live tiles of M rows: position `bid` of `end`; false: it has no tile.  The k slices of a
 // split launch follow each other in it.  (As rows of the grid they left the workgroups of the dead rows
 // between them, and the live ones of the second slice came to lie on the CUs of the first: 230 of 384 rows,
 // hidden 768, FFN2 in two slices with the LayerNorm behind it 13.6 -> 11.1 us.)
@@ -552,8 +552,8 @@ __device__ __forceinline__ bool tile_at(const GemmArgs &p, int M, int bid, int &
   return true;
 }
 
-template <int BM, int BN, int STAGES, int WM, int WN, int NP, int EPI, bool WKN, int MASK>
-__device__ __forceinline__ void gemm_tile(const GemmArgs &p) {
+template <int BM, int BN, int STAGES, int WM, int WN, int NP, int EPI, bool WKN, int MASK, bool LOOP>
+__device__ __forceinline__ int gemm_tile(const GemmArgs &p, const int bid) {
   constexpr int BK = kBK;
   constexpr int NW = WM * WN;                   // waves that run the MFMAs
   constexpr int NL = NP > 0 ? NP : NW;          // waves that issue the global loads
@@ -571,9 +571,10 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &p) {
   extern __shared__ __attribute__((aligned(1024))) half_t gemm_smem[];
   half_t *smem = gemm_smem;
 
-  const int tid = threadIdx.x, lane = tid & 63;
+  int tid = threadIdx.x;
+  if constexpr (LOOP) asm volatile("" : "+v"(tid));   // (so that its uses are not computed ahead of the loop and kept)
+  const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int bid = (int)blockIdx.x;
   int M;
   MaskRows mr{};
   if constexpr (MASK != kMaskNone) {
@@ -587,7 +588,8 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &p) {
   }
 
   int split, tile_m, tile_n;
-  if (!tile_at<BM, BN>(p, M, bid, split, tile_m, tile_n)) return;
+  if (!tile_at<BM, BN>(p, M, bid, split, tile_m, tile_n)) return 0;
+  const int end = ((M + BM - 1) / BM * p.tiles_n * p.splits + 7) / 8 * 8;
   const int m0 = tile_m * BM, n0 = tile_n * BN;
   // slice y of a split-k launch: the k range [y, y + 1) * K / splits
   const int nk = EPI == kEpiPartial ? p.K / BK / p.splits : p.K / BK;
@@ -684,7 +686,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &p) {
       if (++stage == STAGES) stage = 0;
     }
     __builtin_amdgcn_s_barrier();                 // pairs with the barrier before the epilogue
-    return;
+    return end;
   }
 
   // ---- computing side -------------------------------------------------------
@@ -742,9 +744,10 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &p) {
           store_through(dst + (size_t)m * p.N + n, __builtin_bit_cast(uint4_t, tile.acc[i][j]));
       }
     }
-    return;
+    return end;
   }
   tile.template store<EPI>(p, smem + wave * 32 * EP, m0 + wm * WTM, n0 + wn * WTN, M, lane);
+  return end;
 }
 
 // ---- persistent form ---------------------------------------------------------------
@@ -956,6 +959,24 @@ __device__ __forceinline__ void gemm_tiles_flat(const GemmArgs &p) {
 
 #endif  // __HIP_DEVICE_COMPILE__
 
+// ---- launches of more capacity than rows -------------------------------------------------
+// A workgroup that finds no rows needs as much LDS as one that does, and waits for it: with workgroups for the
+// padded batch (16 x 512, 4800 of 8192 rows) QKV took 23.1 us instead of 20.9, FFN1 27.6 (26.0), the projection
+// 9.5 (8.5), FFN2 26.3 (24.7); 12 layers there 1362 -> 1331 us, at 16 x 1024 2495 -> 2479.  Where one workgroup
+// fills a CU and there would be a third of a round too many, a launch therefore has workgroups for the
+// expected rows, in whole rounds, and one whose position is followed by further ones (the rows were more) goes on to them.  `tile` returns the number of
+// positions (0: none here).  Everywhere else a kernel without the loop is 0.2 us faster.
+// Nothing of a tile stays in registers for the next.
+template <typename Tile>
+__device__ __forceinline__ void for_each_tile(const GemmArgs &p, Tile tile) {
+  for (int bid = (int)blockIdx.x;;) {
+    const int end = tile(bid);
+    bid += p.tile_grid;
+    if (bid >= end) return;
+    __syncthreads();   // every wave is done with the LDS of this tile
+  }
+}
+
 template <int BM, int BN, int STAGES, int WM, int WN, int NP, int EPI, bool WKN, int MASK>
 __global__ __launch_bounds__((WM * WN + NP) * 64) void gemm_flat_kernel(BT_GEMM_FIRST, GemmArgs rest) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -963,10 +984,14 @@ __global__ __launch_bounds__((WM * WN + NP) * 64) void gemm_flat_kernel(BT_GEMM_
 #endif
 }
 
-template <int BM, int BN, int STAGES, int WM, int WN, int NP, int EPI, bool WKN, int MASK>
+template <int BM, int BN, int STAGES, int WM, int WN, int NP, int EPI, bool WKN, int MASK, bool LOOP>
 __global__ __launch_bounds__((WM * WN + NP) * 64) void gemm_kernel(BT_GEMM_FIRST, GemmArgs rest) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  gemm_tile<BM, BN, STAGES, WM, WN, NP, EPI, WKN, MASK>(gemm_args(BT_GEMM_FIRST_NAMES, rest));
+  const GemmArgs p = gemm_args(BT_GEMM_FIRST_NAMES, rest);
+  if constexpr (LOOP)
+    for_each_tile(p, [&](int bid) { return gemm_tile<BM, BN, STAGES, WM, WN, NP, EPI, WKN, MASK, LOOP>(p, bid); });
+  else
+    gemm_tile<BM, BN, STAGES, WM, WN, NP, EPI, WKN, MASK, LOOP>(p, (int)blockIdx.x);
 #endif
 }
 
@@ -1178,6 +1203,18 @@ __global__ __launch_bounds__(256) void transpose_kernel(TransposeArgs a) {
                     threadIdx.x, true);
 }
 
+static int cu_count();
+static long long estimated_rows(const GemmArgs &p);
+// Workgroups of a launch whose kernel can go on to further tiles (see for_each_tile): for the expected rows, of
+// which a fifth more may come where the number is a guess, in whole rounds of the chip; `all` at most.
+static int launched_tiles(const GemmArgs &p, int bm, int all) {
+  const bool guess = (p.valid_rows || p.mask) && p.rows_hint <= 0;
+  const long long rows = guess ? (estimated_rows(p) * 6 + 4) / 5 : estimated_rows(p);
+  const long long expected = (rows + bm - 1) / bm * p.tiles_n * p.splits, round = cu_count();
+  const long long rounds = (expected + round - 1) / round * round;
+  return rounds < all ? (int)rounds : all;
+}
+
 // Calls `launch` with the weight layout and the source of the rows as compile-time constants.
 template <int EPI, typename Launch>
 static int by_layout(const GemmArgs &p, Launch launch) {
@@ -1189,23 +1226,34 @@ static int by_layout(const GemmArgs &p, Launch launch) {
   return with(std::integral_constant<int, kMaskNone>{});
 }
 
+template <int BM, int BN, int STAGES, int WM, int WN, int NP, int EPI, bool WKN, int MASK, bool LOOP>
+static int launch_gemm_kernel(const GemmArgs &p, hipStream_t s, size_t smem) {
+  static std::atomic<bool> configured[kMaxDevices];
+  const int rc = allow_dynamic_lds(gemm_kernel<BM, BN, STAGES, WM, WN, NP, EPI, WKN, MASK, LOOP>, smem,
+                                   configured, "hipFuncSetAttribute(gemm_kernel)");
+  if (rc != BT_OK) return rc;
+  gemm_kernel<BM, BN, STAGES, WM, WN, NP, EPI, WKN, MASK, LOOP>
+      <<<dim3(p.tile_grid), (WM * WN + NP) * 64, smem, s>>>(BT_GEMM_FIRST_OF(p), p);
+  BT_CHECK_LAUNCH("gemm_kernel");
+  return BT_OK;
+}
+
 template <int BM, int BN, int STAGES, int WM, int WN, int NP, int EPI, bool WKN, int MASK>
 static int launch_gemm_tile_as(GemmArgs p, hipStream_t s, int splits) {
   constexpr size_t smem = (size_t)STAGES * (BM + BN) * kBK * sizeof(half_t);
   static_assert(smem <= 160 * 1024, "LDS budget");
-  static std::atomic<bool> configured[kMaxDevices];
-  const int rc = allow_dynamic_lds(gemm_kernel<BM, BN, STAGES, WM, WN, NP, EPI, WKN, MASK>, smem,
-                                   configured, "hipFuncSetAttribute(gemm_kernel)");
-  if (rc != BT_OK) return rc;
   const int tiles_m = (p.rows_cap + BM - 1) / BM;
   p.tiles_n = (p.N + BN - 1) / BN;
   p.splits = splits;
   p.tile_grid = (tiles_m * p.tiles_n * splits + 7) / 8 * 8;
-  const dim3 grid(p.tile_grid);
-  gemm_kernel<BM, BN, STAGES, WM, WN, NP, EPI, WKN, MASK>
-      <<<grid, (WM * WN + NP) * 64, smem, s>>>(BT_GEMM_FIRST_OF(p), p);
-  BT_CHECK_LAUNCH("gemm_kernel");
-  return BT_OK;
+  if constexpr (smem > 80 * 1024 && EPI != kEpiPartial) {
+    const int launched = launched_tiles(p, BM, p.tile_grid) / 8 * 8;
+    if (p.tile_grid - launched > cu_count() / 3) {   // (32 or 48 fewer: 7 x 217 -0.5 %, heads of 128 -0.6 %)
+      p.tile_grid = launched;
+      return launch_gemm_kernel<BM, BN, STAGES, WM, WN, NP, EPI, WKN, MASK, true>(p, s, smem);
+    }
+  }
+  return launch_gemm_kernel<BM, BN, STAGES, WM, WN, NP, EPI, WKN, MASK, false>(p, s, smem);
 }
 
 template <int BM, int BN, int STAGES, int WM, int WN, int NP, int EPI>
@@ -1238,8 +1286,6 @@ static int launch_gemm_wave_k(GemmArgs p, hipStream_t s, int splits = 1) {
     return launch_gemm_wave_k_as<EPI, wkn(), mask()>(p, s, splits);
   });
 }
-
-static int cu_count();
 
 // Persistent launch: about one workgroup per CU (a multiple of 8, one share per XCD), each
 // looping over its tiles on the device.

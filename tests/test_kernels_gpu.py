@@ -1503,3 +1503,64 @@ def test_attention_of_sixteen_queries_a_workgroup(device, kind):
                 ops.set_option("attention_key_split", -1)
         bound = 2.0 ** -9 * got[0].abs() + 2.0 ** -9 * 4
         assert ((got[-1] - got[0]).abs() <= bound).all(), (B, S, heads)
+
+
+@pytest.mark.parametrize("tile", [0, 1, 2, 3, 4, 5, 9, 10, 11, 12, 13, 14])
+@pytest.mark.parametrize("w_kn", [False, True])
+def test_gemm_of_more_rows_than_it_was_told(device, tile, w_kn):
+    """A launch is sized for the rows that its caller expects, in whole rounds of the chip; with a single row expected
+    its workgroups go through two and more tiles each, and the results are those of a launch that knew, bit for
+    bit: plain, GELU, the head split with gathered rows and with rows counted from the mask, and k slices."""
+    _say("gemm more rows", tile, w_kn)
+    torch.manual_seed(tile)
+    heads, K = 12, 768
+    S, B = {0: 1700, 2: 1700, 3: 1700, 13: 1700, 4: 600, 14: 300}.get(tile, 1024), 8
+    lens = torch.randint(S // 2, S + 1, (B,))
+    lens[0] = S
+    rows, M = B * S, int(lens.sum())
+    x = torch.randn(rows, K, device=device).half()
+    ws = {n: (torch.randn(K, n, device=device) * 0.05).half() for n in (768, 2304, 3072)}
+    ws = {n: w if w_kn else w.t().contiguous() for n, w in ws.items()}
+    bias = {n: torch.randn(n, device=device).half() for n in ws}
+    live = torch.tensor([M], dtype=torch.int32, device=device)
+    mask = (torch.arange(S)[None] < lens[:, None]).half()[:, None, :].expand(B, S, S).contiguous().to(device)
+    order = torch.cat([torch.arange(b * S, b * S + n) for b, n in enumerate(lens.tolist())]).int().to(device)
+    s = torch.cuda.current_stream().cuda_stream
+    lib = _lib.kernel_lib()
+
+    def run(hint):
+        out = []
+        c = torch.zeros(rows, 3072, dtype=torch.float16, device=device)
+        assert lib.bt_gemm_bias_gelu(x.data_ptr(), ws[3072].data_ptr(), bias[3072].data_ptr(), c.data_ptr(), live.data_ptr(),
+                                     rows, hint, 3072, K, int(w_kn), s) == 0
+        out.append(c)
+        c = torch.zeros(rows, 768, dtype=torch.float16, device=device)
+        assert lib.bt_gemm(x.data_ptr(), ws[768].data_ptr(), c.data_ptr(), live.data_ptr(), rows, hint, 768, K, int(w_kn), s) == 0
+        out.append(c)
+        c = torch.zeros(3 * rows, 768, dtype=torch.float16, device=device)
+        assert lib.bt_gemm_qkv_bias_split(x.data_ptr(), order.data_ptr(), ws[2304].data_ptr(), bias[2304].data_ptr(),
+                                          c.data_ptr(), live.data_ptr(), rows, hint, heads, 64, int(w_kn), s) == 0
+        out.append(c)
+        if lib.bt_gemm_qkv_mask_rows_supported(B, S, 1):
+            c = torch.zeros(3 * rows, 768, dtype=torch.float16, device=device)
+            ints = torch.zeros(3, rows + 1, dtype=torch.int32, device=device)
+            assert lib.bt_gemm_qkv_bias_split_mask_rows(
+                x.data_ptr(), mask.data_ptr(), 1, B, S, ws[2304].data_ptr(), bias[2304].data_ptr(), c.data_ptr(),
+                ints[0].data_ptr(), ints[1].data_ptr(), ints[2].data_ptr(), hint, heads, 64, int(w_kn), s) == 0
+            out += [c, ints]
+        return out
+
+    ops.set_option("gemm_tile", tile)
+    try:
+        for few, known in zip(run(1), run(M)):
+            assert torch.equal(few, known)
+            assert known.any()
+    finally:
+        ops.set_option("gemm_tile", -1)
+    parts = []
+    for hint in (1, M):
+        c = torch.zeros(3, rows, 768, device=device)
+        assert lib.bt_gemm_splitk_rows(x.data_ptr(), ws[768].data_ptr(), c.data_ptr(), 3, live.data_ptr(), rows, hint, 768, K,
+                                       int(w_kn), s) == 0
+        parts.append(c)
+    assert torch.equal(*parts)
