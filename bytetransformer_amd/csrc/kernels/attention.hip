@@ -859,7 +859,12 @@ struct GroupedPlan {
   bool narrow;      // 16-query tiles
   unsigned grid;
 };
-constexpr long long kNarrowBlocks = 208;   // (252 workgroups and those of the warm-up: 3 x 100 388 -> 398 us)
+constexpr long long kNarrowBlocks = 208;
+// Two or three key tiles leave waves without keys and fewer turns to save, so it has to be fewer workgroups there.
+// 64-query against 16-query tiles, whole forwards: 12 heads at 1 x 96 (72 workgroups of 16 queries) 402 / 399 us,
+// 1 x 128 (96) 401 / 398, 2 x 96 (144) 412 / 408, 1 x 180 (144) 423 / 429, 2 x 120 (192) 422 / 438; 16 heads, 24
+// layers, at 1 x 140 (144) 972 / 944, 1 x 190 (192) 1058 / 1080, 2 x 90 (192) 1021 / 1061.
+constexpr long long kNarrowBlocksShort = 160;
 static GroupedPlan plan_grouped(AttArgs &a, int batch_size, int seq_len, int head_num) {
   const long long blocks128 = (long long)((seq_len + 127) / 128) * head_num * batch_size;
   const int qb = option_attention_qb();
@@ -867,7 +872,7 @@ static GroupedPlan plan_grouped(AttArgs &a, int batch_size, int seq_len, int hea
   plan.wide = qb == 2 || (qb < 0 && blocks128 >= 1300);
   const long long blocks16 = (long long)((seq_len + 15) / 16) * head_num * batch_size;
   plan.narrow = qb < 0 && option_attention_key_split() < 0 && option_attention_xcd_map() != 3 && seq_len > kKT && seq_len <= 4 * kKT &&
-                blocks16 <= kNarrowBlocks;
+                blocks16 <= (seq_len > 3 * kKT ? kNarrowBlocks : kNarrowBlocksShort);
   plan.grid = att_grid(a, plan.wide ? (seq_len + 127) / 128 : plan.narrow ? (seq_len + 15) / 16 : (seq_len + 63) / 64,
                        true);
   return plan;
