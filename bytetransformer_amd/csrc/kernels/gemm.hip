@@ -1462,30 +1462,35 @@ static bool wave_k_fits(const GemmArgs &p) {
 // products': k slices give the idle CUs a share of it, and the LayerNorm that reads the result anyway adds
 // the slices up.  The pair's time is, within 3 % (84 pairs of tile and slices, hidden 768 and 1024, 32
 // to 2736 rows), that of the tile - fixed + k-steps of a slice x step - plus what the LayerNorm reads.
+// Tile 14 is priced by what layers with it take (hidden 1024, 64 rows, two slices / four, us: 40.1 / 38.0, the
+// 32x64 tile 42.0 / 38.5): launched alone, its weight warm, the number of slices seems to make no difference.
 // Pairs of FFN2 and LayerNorm, k whole -> in slices, us: hidden 768, 230 rows 14.7 -> 10.3 (four slices of
 // 64x64 tiles; two of 32x64 tiles 10.7), 768 rows 16.1 -> 12.8, 911 rows 16.2 -> 14.4, 1500 rows 20.2 -> 16.7,
 // 2000 rows 21.1 -> 19.5; hidden 1024, 640 rows 17.8 -> 14.8, 1300 rows 25.0 -> 21.3.
 struct SliceModel {
   int id, bm, bn;
   float fixed_us, step_us;   // launch and LayerNorm of few rows included
-  bool shares_cu;            // a second workgroup fits the CU
-};
+  int busy_cus;              // (a tile that fills its CU finds some CU busy at the last few per cent: 252
+};                           // workgroups 21.6 us, 216 16.7; the short ones of tile 14 fill the chip, 256)
 static const SliceModel kSliceModels[] = {
-    {14, 32, kWaveKCols, 9.49f, 0.010f, false}, {4, 32, 64, 8.37f, 0.115f, true},
-    {9, 64, 64, 9.04f, 0.111f, true},           {10, 64, 128, 9.37f, 0.195f, true},
-    {11, 96, 128, 10.39f, 0.242f, false},       {1, 128, 128, 10.53f, 0.231f, false},
-    {12, 128, 192, 12.05f, 0.321f, false}};
+    {14, 32, kWaveKCols, 8.00f, 0.080f, 0}, {4, 32, 64, 8.37f, 0.115f, 0},
+    {9, 64, 64, 9.04f, 0.111f, 0},          {10, 64, 128, 9.37f, 0.195f, 0},
+    {11, 96, 128, 10.39f, 0.242f, 16},      {1, 128, 128, 10.53f, 0.231f, 16},
+    {12, 128, 192, 12.05f, 0.321f, 16}};
 constexpr int kMostSlices = 4;
-// Beyond this many results the slices cost the memory system more than the idle CUs give (2000 rows of
-// 1024: 27.3 against 27.8 us, 2400 rows of 768: 22.8 against 21.9).
-constexpr float kSlicedResults = 1.6e6f;
+// Beyond this many results the slices cost the memory system more than the idle CUs give.  Layers of rows
+// that are all live, 600 MB of weights walked through, k whole / in two slices, us: hidden 512 (k 2048)
+// 1024 rows 43.5 / 43.0, 1088 rows 46.6 / 47.2, 1984 rows 49.1 / 50.9; hidden 576 1024 rows 45.9 / 46.7, 1600
+// rows 56.9 / 58.4; hidden 640 (k 2560) 1984 rows 63.1 / 62.4; hidden 768 2112 rows 74.2 / 72.5, 2400 rows
+// 76.7 / 75.5, 2600 rows 94.1 / 94.2; hidden 1024 1600 rows 90.7 / 87.2, 1984 rows 90.2 / 91.2, 2600
+// rows 118.9 / 128.6.
+static float sliced_results(int k) { return k < 2560 ? 0.55e6f : 1.9e6f; }
 // What a tile's launch takes beyond the LayerNorm and the launches themselves, so again in a second round.
 constexpr float kPairUs = 6.f;
 
 static float slice_pair_us(const SliceModel &c, long long m, int n, int k, int splits) {
   const long long tiles = ((m + c.bm - 1) / c.bm) * ((n + c.bn - 1) / c.bn) * splits;
-  // (a tile that fills its CU finds some CU busy at the last few per cent: 252 workgroups 21.6 us, 216 16.7)
-  const long long at_once = c.shares_cu ? cu_count() : cu_count() - cu_count() / 16;
+  const long long at_once = cu_count() - c.busy_cus;
   const float rounds = (float)((tiles + at_once - 1) / at_once);
   const float mn = (float)m * (float)n * 1e-6f, extra = (float)(splits - 1);
   return kPairUs + rounds * (c.fixed_us - kPairUs + c.step_us * (float)(k / kBK) / (float)splits) + 2.16f * mn +
@@ -1692,7 +1697,7 @@ extern "C" int bt_gemm_splitk_slices(int rows_cap, int all_live, int n, int k, i
   p.rows_cap = (int)((rows_cap * 3LL + 4) / 5);
   const LikelyRows part(p);
   const float fills = all_live ? 1.f : 1.f / 3.f;
-  if ((float)(all_live ? full : part).rows[0] * (float)n > kSlicedResults) return 1;
+  if ((float)(all_live ? full : part).rows[0] * (float)n > sliced_results(k)) return 1;
   int best = 1;
   float best_us = 0.f;
   for (int s = 1; s <= kMostSlices && (s == 1 || s <= most); ++s) {

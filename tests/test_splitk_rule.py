@@ -1,10 +1,11 @@
-"""How many k slices the layer gives FFN2: the rule of include/bytetransformer/common.h, compiled as the host compiles it."""
+"""How many k slices the layer gives FFN2: the measured rule of the kernels library, and the rule of
+include/bytetransformer/common.h for parts that it was not measured on, compiled as the host compiles it."""
 import os
 import subprocess
 
 import pytest
 
-from bytetransformer_amd import build
+from bytetransformer_amd import _lib, build
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 SOURCE = """
@@ -40,3 +41,25 @@ def answers(tmp_path_factory):
 def test_slices(answers, i):
     args, want = CASES[i]
     assert answers[i] == want, args
+
+
+# rows that are all live, hidden, k -> slices, each the fastest of a layer's measured ones or within 1 % of it
+@pytest.mark.parametrize("rows,n,k,slices", [
+    (32, 768, 3072, 4), (900, 768, 3072, 4), (1500, 768, 3072, 3), (1984, 768, 3072, 2), (2240, 768, 3072, 2), (2400, 768, 3072, 2),
+    (2600, 768, 3072, 1), (64, 1024, 4096, 4), (96, 1024, 4096, 4), (1600, 1024, 4096, 2), (2240, 1024, 4096, 1),
+    (64, 1280, 5120, 4), (512, 512, 2048, 4), (1088, 512, 2048, 1), (1984, 512, 2048, 1), (1280, 576, 2304, 1)])
+def test_measured_slices(rows, n, k, slices):
+    assert _lib.kernel_lib().bt_gemm_splitk_slices(rows, 1, n, k, 16) == slices
+
+
+def test_slices_of_a_padded_batch():
+    """60 % of the rows, or less likely all of them; never more slices than there is room for; whole k for short k or no rows."""
+    ask = _lib.kernel_lib().bt_gemm_splitk_slices
+    assert ask(384, 0, 768, 3072, 16) in (3, 4)
+    assert ask(4000, 0, 768, 3072, 16) == 1 and ask(3000, 0, 768, 3072, 16) == 2
+    for most in (0, 1, 2, 3, 16):
+        assert 1 <= ask(1500, 0, 768, 3072, most) <= max(most, 1)
+    assert ask(0, 0, 768, 3072, 16) == ask(100, 0, 768, 32, 16) == ask(100, 0, 768, 3000, 16) == 1
+    for n, k in ((768, 3072), (1024, 4096), (512, 2048), (640, 2560)):
+        for rows in range(1, 3000, 61):
+            assert (k // 64) % ask(rows, 0, n, k, 16) == 0
