@@ -187,7 +187,7 @@ void BertEncoder<OpType>::infer(BertEncoderInferParam<DataType_> ip) {
                                      stream));
 
     // few rows, long k: FFN2 as split-k partial sums that the last LayerNorm folds in
-    const int splits = ffn2_slices(rows, valid_rows != nullptr, hidden, inter, partials_bytes);
+    const int splits = ffn2_slices(rows, valid_rows == nullptr, hidden, inter, partials_bytes);
     if (splits > 1) {
       const bool restore = last && is_remove_padding_;
       check_bt_error(bt_gemm_splitk_rows(inter_matmul_buf, wt_out, partials, splits, valid_rows, rows, rows_hint,

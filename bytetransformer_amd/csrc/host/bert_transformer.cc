@@ -210,6 +210,11 @@ void BertTransformer<OpType>::bert_infer(BertTransformerInferParam infer_param) 
   // FFN2.  The QKV product and the attention keep batch * seq_len: it is the row stride
   // of the per-head Q/K/V layout and the extent of the gathered input.
   int packed_cap = rows;
+  // ... and the products behind the attention take every row of it for live: choices made from
+  // sizes alone (FFN2's slices, tile 14) then follow the count itself instead of a padded batch's
+  // 60 %.  Their rows lie in the scratch, so a row too many costs time only; the LayerNorms,
+  // which read through the caller's word_idx, keep the device's count.
+  bool all_live = !is_remove_padding_;
   if (is_remove_padding_) {
     // The packed copy of the input is never materialised: the QKV GEMM and the
     // first LayerNorm read valid token t from the padded input at row word_idx[t]
@@ -218,7 +223,10 @@ void BertTransformer<OpType>::bert_infer(BertTransformerInferParam infer_param) 
     restore_target = transformer_out;
     transformer_out = qkv_buf;  // FFN2 output reuses the dead qkv region
     valid_rows = et_param.batch_idx + batch_size;
-    if (have_offsets && rows_hint > 0 && rows_hint < rows) packed_cap = rows_hint;
+    if (have_offsets && rows_hint > 0 && rows_hint <= rows) {
+      packed_cap = rows_hint;
+      all_live = true;
+    }
     rows_hint = rows_to_plan_for(rows_hint, true, batch_size, rows);
   }
 
@@ -315,8 +323,9 @@ void BertTransformer<OpType>::bert_infer(BertTransformerInferParam infer_param) 
   }
   attention_layer_->infer(attention_infer_param);
 
+  const int *product_rows = all_live ? nullptr : valid_rows;
   check_bt_error(
-      bt_gemm(attr_out_buf, wt_proj, attr_matmul_buf, valid_rows, packed_cap, rows_hint, hidden,
+      bt_gemm(attr_out_buf, wt_proj, attr_matmul_buf, product_rows, packed_cap, rows_hint, hidden,
               hidden, w_kn[1], stream));
 
   if (ln_count > 0)
@@ -331,14 +340,13 @@ void BertTransformer<OpType>::bert_infer(BertTransformerInferParam infer_param) 
         valid_rows, packed_cap, hidden, layernorm_eps, stream));
 
   check_bt_error(bt_gemm_bias_gelu(attr_matmul_buf, wt_inter, param_.inter_bias, inter_matmul_buf,
-                                   valid_rows, packed_cap, rows_hint, inter, hidden, w_kn[2],
+                                   product_rows, packed_cap, rows_hint, inter, hidden, w_kn[2],
                                    stream));
 
   // few rows, long k: FFN2 as split-k partial sums that the last LayerNorm folds in
-  const int splits =
-      ffn2_slices(packed_cap, valid_rows != nullptr, hidden, inter, partials_bytes);
+  const int splits = ffn2_slices(packed_cap, all_live, hidden, inter, partials_bytes);
   if (splits > 1) {
-    check_bt_error(bt_gemm_splitk_rows(inter_matmul_buf, wt_out, partials, splits, valid_rows, packed_cap,
+    check_bt_error(bt_gemm_splitk_rows(inter_matmul_buf, wt_out, partials, splits, product_rows, packed_cap,
                                        rows_hint, hidden, inter, w_kn[3], stream));
     check_bt_error(bt_splitk_layernorm(
         partials, splits, attr_matmul_buf, nullptr, param_.output_bias,
@@ -350,7 +358,7 @@ void BertTransformer<OpType>::bert_infer(BertTransformerInferParam infer_param) 
   }
 
   check_bt_error(
-      bt_gemm(inter_matmul_buf, wt_out, transformer_out, valid_rows, packed_cap, rows_hint, hidden,
+      bt_gemm(inter_matmul_buf, wt_out, transformer_out, product_rows, packed_cap, rows_hint, hidden,
               inter, w_kn[3], stream));
 
   if (is_remove_padding_)

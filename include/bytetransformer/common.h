@@ -84,11 +84,12 @@ inline unsigned long long splitk_scratch_bytes(unsigned long long max_rows,
 }
 // The slices of a layer's FFN2.  `area_bytes` = what the caller can give the partial sums: the activations
 // that are dead by then and the scratch behind them.
-inline int ffn2_slices(int rows_cap, bool packed, int n, int k, unsigned long long area_bytes) {
-  const int rule = splitk_splits(rows_cap, packed ? (rows_cap * 3LL + 4) / 5 : rows_cap, k);
+// `all_live` = the launch has rows_cap rows, not a padded batch's share of them.
+inline int ffn2_slices(int rows_cap, bool all_live, int n, int k, unsigned long long area_bytes) {
+  const int rule = splitk_splits(rows_cap, all_live ? rows_cap : (rows_cap * 3LL + 4) / 5, k);
   if (k < 2048 || splitk_splits(1, 1, 2048) == 1) return rule;   // (short k, or turned off)
   const unsigned long long fit = area_bytes / ((unsigned long long)rows_cap * n * sizeof(float));
-  const int slices = bt_gemm_splitk_slices(rows_cap, packed ? 0 : 1, n, k, (int)(fit < 16 ? fit : 16));
+  const int slices = bt_gemm_splitk_slices(rows_cap, all_live ? 1 : 0, n, k, (int)(fit < 16 ? fit : 16));
   return slices > 0 ? slices : rule;
 }
 

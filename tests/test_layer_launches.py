@@ -1,0 +1,130 @@
+"""What a layer and an encoder launch, seen on the host: their own sources linked against launch entries that only
+write down what they were asked for, beside the kernels library for every question that a host function answers."""
+import os
+import subprocess
+
+import pytest
+
+from bytetransformer_amd import _lib, build
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+HOST = os.path.join(build.CSRC, "host")
+SOURCE = r"""
+#include <dlfcn.h>
+
+#include <cstdio>
+#include <cstdlib>
+#include <vector>
+
+#include "bytetransformer/bert_encoder.h"
+#include "bytetransformer/bert_transformer.h"
+using namespace bytetransformer;
+
+static int slices = 0, asked = 0, live_by_size = 0;   // of FFN2; questions after them; products of known rows
+extern "C" {
+int bt_layer_prologue(const void *, int, int, int, int *, int *, int *, int *, void *, int, int, int, const void *const *,
+                      void *const *, const int *, const int *, int, const void *const *, const unsigned long long *, void *) { return 0; }
+int bt_gemm_qkv_bias_split(const void *, const int *, const void *, const void *, void *, const int *, int, int, int, int, int, void *) { return 0; }
+int bt_gemm_qkv_bias_split_mask_rows(const void *, const void *, int, int, int, const void *, const void *, void *, int *, int *,
+                                     int *, int, int, int, int, void *) { return 0; }
+int bt_attention_grouped(const void *, void *, const int *, const int *, const void *, const void *, int, int, int, int, int,
+                         float, int, const void *const *, const unsigned long long *, int, const int *, const void *, void *) { return 0; }
+int bt_mask_prefix_slots(const void *, int, int, int, const int *, int *, void *) { return 0; }
+int bt_add_bias_residual_layernorm(void *, const void *, const int *, const void *, const void *, const void *, int, const int *,
+                                   int, int, float, void *) { return 0; }
+int bt_add_bias_residual_layernorm_copy(void *, const void *, const int *, const void *, const void *, const void *, int,
+                                        const int *, int, int, float, int, const void *const *, void *const *, const int *,
+                                        const int *, void *) { return 0; }
+int bt_add_bias_residual_layernorm_restore(const void *, const void *, const void *, const void *, const void *, int, void *,
+                                           const int *, const int *, int, int, int, float, void *) { return 0; }
+int bt_splitk_layernorm(const void *, int, const void *, const int *, const void *, const void *, const void *, int, void *,
+                        const int *, const int *, int, int, int, int, float, void *) { return 0; }
+int bt_gemm(const void *, const void *, void *, const int *live, int, int, int n, int k, int, void *) {
+  if (k > n) slices = 1;
+  live_by_size += live == nullptr;
+  return 0;
+}
+int bt_gemm_bias_gelu(const void *, const void *, const void *, void *, const int *live, int, int, int, int, int, void *) {
+  live_by_size += live == nullptr;
+  return 0;
+}
+int bt_gemm_splitk_rows(const void *, const void *, void *, int splits, const int *live, int, int, int, int, int, void *) {
+  slices = splits;
+  live_by_size += live == nullptr;
+  return 0;
+}
+int bt_gemm_splitk_slices(int rows_cap, int all_live, int n, int k, int most) {
+  ++asked;
+  return ((int (*)(int, int, int, int, int))dlsym(RTLD_NEXT, "bt_gemm_splitk_slices"))(rows_cap, all_live, n, k, most);
+}
+}
+
+// argv: layer|encoder  heads  batch  seq_len  live rows that the caller vouches for (-1: no offsets)
+int main(int, char **argv) {
+  const int heads = std::atoi(argv[2]), batch = std::atoi(argv[3]), seq = std::atoi(argv[4]), live = std::atoi(argv[5]);
+  static char some[4096];
+  const __half *t = (const __half *)some;
+  BertTransformerParam<OperationType::HALF> w;
+  w.attention_param.attr_bias_QKV = t;
+  w.attr_kernel_QKV = w.attr_output_kernel = w.inter_kernel = w.output_kernel = t;
+  if (argv[1][0] == 'l') {
+    BertTransformer<OperationType::HALF> layer(batch, heads, 64, seq);
+    layer.initialize(w);
+    layer.cal_bufsize();
+    BertTransformerInferParam<__half> ip{t, t, (__half *)some, some, batch, seq, nullptr, nullptr};
+    ET_Param offsets{(int *)some, (int *)some, live};
+    if (live >= 0) ip.offsets = &offsets;
+    layer.infer(ip);
+  } else {
+    BertEncoder<OperationType::HALF> encoder(batch, heads, 64, seq);
+    encoder.initialize(std::vector<BertTransformerParam<OperationType::HALF>>(12, w));
+    encoder.cal_bufsize();
+    BertEncoderInferParam<__half> ip{};
+    ip.input_tensor = ip.atten_mask = t, ip.transformer_output = (__half *)some, ip.buf = some;
+    ip.batch_size = batch, ip.seq_len = seq;
+    encoder.infer(ip);
+  }
+  std::printf("%d %d %d\n", slices, live_by_size, asked);
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def launches(tmp_path_factory):
+    tmp = tmp_path_factory.mktemp("launches")
+    source, program = str(tmp / "launches.cc"), str(tmp / "launches")
+    with open(source, "w") as f:
+        f.write(SOURCE)
+    subprocess.run(["g++"] + build.HOST_FLAGS +
+                   ["-I", os.path.join(ROOT, "include"), "-I", HOST, "-I", os.path.join(build.ROCM, "include"), source] +
+                   [os.path.join(HOST, f) for f in ("bert_transformer.cc", "bert_encoder.cc", "attention.cc")] +
+                   ["-L", build.LIB, "-lbt_hip", "-L", os.path.join(build.ROCM, "lib"), "-lamdhip64", "-ldl",
+                    "-Wl,-rpath," + build.LIB, "-Wl,-rpath," + os.path.join(build.ROCM, "lib"), "-o", program], check=True)
+    env = {k: v for k, v in os.environ.items() if k != "BT_SPLITK"}
+
+    def run(*args):
+        out = subprocess.run([program] + [str(a) for a in args], check=True, stdout=subprocess.PIPE, text=True, env=env)
+        return tuple(int(v) for v in out.stdout.split())
+    return run
+
+
+# live rows of hidden 768 -> slices: what the sizes give where every row is live (a padded batch of 900 rows gets 2,
+# one of 1050 gets 2, of 2400 three)
+@pytest.mark.parametrize("live,slices", [(32, 4), (900, 4), (1050, 4), (1500, 3), (2100, 2), (2400, 2), (3400, 1), (8192, 1)])
+def test_offsets_with_their_count(launches, live, slices):
+    got, live_by_size, _ = launches("layer", 12, 16, 512, live)
+    assert got == slices == _lib.kernel_lib().bt_gemm_splitk_slices(live, 1, 768, 3072, 16)
+    assert live_by_size == 3
+
+
+@pytest.mark.parametrize("batch,seq_len", [(16, 512), (4, 96), (7, 217), (8, 300)])
+def test_offsets_without_their_count(launches, batch, seq_len):
+    """A caller that does not know the count gets the slices of one that passes no offsets."""
+    own = launches("layer", 12, batch, seq_len, -1)
+    assert launches("layer", 12, batch, seq_len, 0) == own
+    assert own[1] == 0
+
+
+def test_padded_rows_are_all_live(launches):
+    got = launches("layer", 12, 2, 200, -1)
+    assert got[0] == _lib.kernel_lib().bt_gemm_splitk_slices(400, 1, 768, 3072, 16)
