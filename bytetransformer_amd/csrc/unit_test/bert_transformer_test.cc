@@ -127,6 +127,7 @@ struct Options {
   bool is_remove_padding = true, use_fused_attention = true;
   std::string dir = ".";
   bool synthetic = false;
+  bool offsets = false;   // built once ahead of the layer, with their count
   std::vector<int> lens;
 };
 
@@ -214,6 +215,18 @@ static int run(const Options &o) {
     HIP_OK(hipMalloc(&out, N * H * sizeof(T)));
     BertTransformerInferParam<T> infer_param{(const T *)dev[12], (const T *)dev[13], (T *)out, buf,
                                              batch_size,         seq_len,            nullptr,  stream};
+    ET_Param offsets{};
+    if (o.offsets) {
+      int *ints;
+      HIP_OK(hipMalloc(&ints, (N + 2 * (size_t)batch_size + 1) * sizeof(int)));
+      offsets.word_idx = ints;
+      offsets.batch_idx = ints + N;
+      int *order = offsets.batch_idx + batch_size + 1;
+      check_bt_error(bt_build_offsets(dev[13], Traits<Op>::dtype, batch_size, seq_len, offsets.batch_idx,
+                                      offsets.word_idx, order, &offsets.valid_word_num, stream));
+      infer_param.offsets = &offsets;
+      infer_param.seq_order = order;
+    }
     layer.infer(infer_param);
     HIP_OK(hipStreamSynchronize(stream));
 
@@ -271,7 +284,7 @@ int main(int argc, char *argv[]) {
   if (argc < 5) {
     printf("./bert_transformer_test <batch_size> <seq_len> <head_num> <size_per_head> "
            "[--data DIR] [--iters N] [--tol MAX_ABS] [--no-rm] [--no-fused] [--fp32] "
-           "[--synthetic [--lens L0,L1,...]] [--option NAME=VALUE ...]\n");
+           "[--synthetic [--lens L0,L1,...]] [--offsets] [--option NAME=VALUE ...]\n");
     return 0;
   }
   Options o;
@@ -289,6 +302,7 @@ int main(int argc, char *argv[]) {
     else if (!strcmp(argv[i], "--no-fused")) o.use_fused_attention = false;
     else if (!strcmp(argv[i], "--fp32")) fp32 = true;
     else if (!strcmp(argv[i], "--synthetic")) o.synthetic = true;
+    else if (!strcmp(argv[i], "--offsets")) o.offsets = true;
     else if (!strcmp(argv[i], "--option") && i + 1 < argc) {
       // a tuning knob of the kernel library (bt_set_option), e.g. qkv_mask_rows=0
       const std::string kv = argv[++i];

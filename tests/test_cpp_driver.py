@@ -40,7 +40,9 @@ def test_text_fixture_format(tmp_path):
 @pytest.mark.gpu
 @pytest.mark.parametrize("batch,seq,heads,extra", [(4, 48, 2, []), (2, 40, 2, []),
                                                    (5, 100, 4, ["--no-fused"]),
-                                                   (4, 48, 2, ["--fp32"]), (2, 40, 2, ["--fp32"])])
+                                                   (4, 48, 2, ["--fp32"]), (2, 40, 2, ["--fp32"]),
+                                                   (4, 48, 2, ["--offsets"]), (5, 60, 8, ["--offsets"]),
+                                                   (2, 40, 2, ["--offsets"]), (4, 48, 2, ["--offsets", "--fp32"])])
 def test_cpp_driver_matches_exported_expectation(device, tmp_path, batch, seq, heads, extra):
     print("cpp driver", batch, seq, heads, extra, flush=True)
     X.export(str(tmp_path), batch=batch, seq=seq, heads=heads, seed=batch)
