@@ -1179,6 +1179,22 @@ __global__ __launch_bounds__(kWaveKWaves * 64) void gemm_wave_k_kernel(BT_GEMM_F
 #endif
 }
 
+// Plain products whose live rows only the device knows: tile 14 where they fit one round of it, else tile 4
+// (see takes_wave_k).  `splits` brings the most rows of tile 14: an argument that is there at wave launch.
+template <bool WKN>
+__global__ __launch_bounds__(kWaveKWaves * 64) void gemm_few_rows_kernel(BT_GEMM_FIRST, GemmArgs rest) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  GemmArgs p = gemm_args(BT_GEMM_FIRST_NAMES, rest);
+  p.splits = 1;
+  if (*valid_rows <= splits) {
+    gemm_wave_k<kEpiPlain, WKN, kMaskNone>(p);
+  } else {
+    p.tiles_n = (p.N + 63) / 64;
+    gemm_tile<32, 64, 4, 1, 2, 2, kEpiPlain, WKN, kMaskNone, false>(p, (int)blockIdx.x);
+  }
+#endif
+}
+
 // ---- weight pre-pack: wt[n][k] = w[k][n] for up to four matrices in one launch ---
 struct TransposeJob {
   const half_t *w;
@@ -1285,6 +1301,26 @@ static int launch_gemm_wave_k(GemmArgs p, hipStream_t s, int splits = 1) {
   return by_layout<EPI>(p, [&](auto wkn, auto mask) {
     return launch_gemm_wave_k_as<EPI, wkn(), mask()>(p, s, splits);
   });
+}
+
+template <bool WKN>
+static int launch_gemm_few_rows_as(GemmArgs p, hipStream_t s) {
+  constexpr size_t smem = (size_t)kWaveKWaves * kWaveKDepth * (32 + kWaveKCols) * kBK * sizeof(half_t);
+  static_assert(smem >= 4 * (32 + 64) * kBK * sizeof(half_t), "room for the ring of tile 4");
+  static std::atomic<bool> configured[kMaxDevices];
+  const int rc = allow_dynamic_lds(gemm_few_rows_kernel<WKN>, smem, configured, "hipFuncSetAttribute(gemm_few_rows_kernel)");
+  if (rc != BT_OK) return rc;
+  p.tiles_n = (p.N + kWaveKCols - 1) / kWaveKCols;
+  // (one round of either tile: what the few rows take, or the capacity in the wider tiles)
+  p.splits = cu_count() / p.tiles_n * 32;
+  const int few = p.splits / 32 * p.tiles_n, wide = (p.rows_cap + 31) / 32 * ((p.N + 63) / 64);
+  p.tile_grid = ((few > wide ? few : wide) + 7) / 8 * 8;
+  gemm_few_rows_kernel<WKN><<<dim3(p.tile_grid), kWaveKWaves * 64, smem, s>>>(BT_GEMM_FIRST_OF(p), p);
+  BT_CHECK_LAUNCH("gemm_few_rows_kernel");
+  return BT_OK;
+}
+static int launch_gemm_few_rows(const GemmArgs &p, hipStream_t s) {
+  return p.w_kn ? launch_gemm_few_rows_as<true>(p, s) : launch_gemm_few_rows_as<false>(p, s);
 }
 
 // Persistent launch: about one workgroup per CU (a multiple of 8, one share per XCD), each
@@ -1451,10 +1487,22 @@ static bool tuned_mean(const LikelyRows &likely, int n, int k, int epi, int kn, 
   return true;
 }
 
-// Whether the tiles of gemm_wave_k fit one round: a workgroup fills its CU's LDS, so a second round
-// doubles the launch.
-static bool wave_k_fits(const GemmArgs &p) {
-  return (estimated_rows(p) + 31) / 32 * ((p.N + kWaveKCols - 1) / kWaveKCols) <= cu_count();
+// How a product runs on tile 14, whose waves share k and add up in an order of their own: a row count that a
+// caller knows in one call and not in the next must not change a bit, so this follows from sizes, and from the
+// live rows themselves.  A workgroup fills its CU's LDS, so its tiles have to fit one round: us of tile 14 / tile
+// 4 in one round and in two, projection at hidden 768 4.4 / 4.8 (320 rows), 6.6 / 4.8 (352); hidden 1024 5.1 / 5.6
+// (256), 7.2 / 5.6 (288); hidden 512 3.8 / 4.1 (512); QKV at hidden 768 4.3 / 4.6 (32 rows), 4.8 / 4.8 (96), 6.7 / 4.7
+// (128); FFN1 4.9 / 5.1 (32), 5.1 / 5.2 (64), 8.2 / 5.3 (96).  A plain product of a padded batch whose capacity
+// does not fit, but fits in tile 4, finds its rows on the device, where the kernel takes the one or the other (four
+// sequences of 96, all full: 4.9 us a projection in place of 6.7 without a row count; with one, 12 layers 483
+// and 486 us).  In the products with more columns, whose gain is small, the second tile's code costs more than
+// that (with it in both, 4 x 32 406 -> 416 us).  With fewer than four k-steps a wave has nothing to do.
+enum WaveK { kWaveKNo, kWaveKYes, kWaveKDevice };
+static WaveK takes_wave_k(const GemmArgs &p, bool plain) {
+  const long long tiles_m = (p.rows_cap + 31) / 32, tiles_n = (p.N + kWaveKCols - 1) / kWaveKCols;
+  if (p.K < kWaveKWaves * kBK || tiles_n > cu_count()) return kWaveKNo;
+  if (tiles_m * tiles_n <= cu_count()) return kWaveKYes;
+  return plain && p.valid_rows && tiles_m * ((p.N + 63) / 64) <= cu_count() ? kWaveKDevice : kWaveKNo;
 }
 
 // ---- products in k slices ----------------------------------------------------------------
@@ -1532,14 +1580,16 @@ static int launch_gemm(GemmArgs p, hipStream_t s) {
   //  12: 128x192, 3, 2x2, 4   } memory-side cache, best of tiles 0-8 and now: FFN2 at 920 rows 17.0 ->
   //  13: 192x192, 2, 3x2, 4   } 13.0 us (9), at 2000 rows 20.6 -> 17.5 (10), at 5600 rows 35.6 -> 30.2
   //                           (12); QKV at 3600 rows 19.6 -> 18.6 (13), at 1300 rows 9.6 -> 9.1 (11)
-  //  14:  32x32, four waves over k (gemm_wave_k): in place of tile 4 while its workgroups fit one
-  //                           round (the rule measured both ways: 1 x 256 with the FFN2 in 384
-  //                           workgroups 509 us, with tile 4 there 456)
+  //  14:  32x32, four waves over k (gemm_wave_k), where takes_wave_k() says so
   // The choice minimises the time of the launch: for the weight shapes of BERT-base and BERT-large
   // by a table of measured times (gemm_tuned.inc) where it names a clearly faster tile, else by the
   // model of model_us().
-  const int forced = option_gemm_tile();
-  int choice = forced;
+  int choice = option_gemm_tile();
+  if (choice < 0) {
+    const WaveK few = takes_wave_k(p, EPI == kEpiPlain);
+    if (few == kWaveKDevice) return launch_gemm_few_rows(p, s);
+    if (few == kWaveKYes) choice = 14;
+  }
   if (choice < 0) {
     const LikelyRows likely(p);
     float us[kTunedTiles];
@@ -1563,7 +1613,6 @@ static int launch_gemm(GemmArgs p, hipStream_t s) {
         choice = tuned;
     }
   }
-  if (forced < 0 && choice == 4 && wave_k_fits(p)) choice = 14;
   switch (choice) {
     case 14:
       return launch_gemm_wave_k<EPI>(p, s);

@@ -1564,3 +1564,89 @@ def test_gemm_of_more_rows_than_it_was_told(device, tile, w_kn):
                                        int(w_kn), s) == 0
         parts.append(c)
     assert torch.equal(*parts)
+
+
+@pytest.mark.parametrize("w_kn", [False, True])
+@pytest.mark.parametrize("S,hidden", [(24, 768), (96, 768), (121, 768), (128, 768), (160, 768), (75, 1024), (200, 512), (1024, 768)])
+def test_row_hints_never_change_a_bit(device, S, hidden, w_kn):
+    """Four sequences, from nearly empty to full: a hint of any size, and none, give the same bits in every product that
+    takes one, also where it changes the tile (capacities around those that fit one round of the chip)."""
+    _say("row hints", S, hidden, w_kn)
+    torch.manual_seed(S)
+    B, K, heads = 4, hidden, hidden // 64
+    rows = B * S
+    x = torch.randn(rows, K, device=device).half()
+    ws = {n: (torch.randn(K, n, device=device) * 0.05).half() for n in (K, 3 * K, 4 * K)}
+    ws = {n: w if w_kn else w.t().contiguous() for n, w in ws.items()}
+    w32 = torch.randn(K, K, device=device) * 0.05
+    bias = {n: torch.randn(n, device=device).half() for n in ws}
+    s = torch.cuda.current_stream().cuda_stream
+    lib = _lib.kernel_lib()
+    kn = int(w_kn)
+    for fill in (0.3, 0.6, 1.0):
+        lens = torch.tensor([max(1, int(S * fill * f)) for f in (1.0, 0.9, 0.7, 0.2)]) if fill < 1 else torch.full((B,), S)
+        M = int(lens.sum())
+        live = torch.tensor([M], dtype=torch.int32, device=device)
+        mask = (torch.arange(S)[None] < lens[:, None]).half()[:, None, :].expand(B, S, S).contiguous().to(device)
+        order = torch.cat([torch.arange(b * S, b * S + n) for b, n in enumerate(lens.tolist())])
+        order = torch.cat([order, torch.zeros(rows - M, dtype=torch.int64)]).int().to(device)
+        first = None
+        for hint in (0, 1, M // 2, M, (rows + M) // 2, rows):
+            got = [torch.zeros(rows, K, dtype=torch.float16, device=device),
+                   torch.zeros(rows, 4 * K, dtype=torch.float16, device=device),
+                   torch.zeros(3 * rows, K, dtype=torch.float16, device=device),
+                   torch.zeros(3 * rows, K, dtype=torch.float16, device=device),
+                   torch.zeros(2, rows, K, device=device), torch.zeros(rows, K, device=device)]
+            ints = torch.zeros(3, rows + 1, dtype=torch.int32, device=device)
+            w = {n: t.data_ptr() for n, t in ws.items()}
+            p = [t.data_ptr() for t in got]
+            rc = [lib.bt_gemm(x.data_ptr(), w[K], p[0], live.data_ptr(), rows, hint, K, K, kn, s),
+                  lib.bt_gemm_bias_gelu(x.data_ptr(), w[4 * K], bias[4 * K].data_ptr(), p[1], live.data_ptr(), rows, hint, 4 * K,
+                                        K, kn, s),
+                  lib.bt_gemm_qkv_bias_split(x.data_ptr(), order.data_ptr(), w[3 * K], bias[3 * K].data_ptr(), p[2],
+                                             live.data_ptr(), rows, hint, heads, 64, kn, s),
+                  lib.bt_gemm_qkv_bias_split_mask_rows(x.data_ptr(), mask.data_ptr(), 1, B, S, w[3 * K], bias[3 * K].data_ptr(),
+                                                       p[3], ints[0].data_ptr(), ints[1].data_ptr(), ints[2].data_ptr(), hint,
+                                                       heads, 64, kn, s),
+                  lib.bt_gemm_splitk_rows(x.data_ptr(), w[K], p[4], 2, live.data_ptr(), rows, hint, K, K, kn, s),
+                  lib.bt_gemm_f32(x.float().data_ptr(), None, w32.data_ptr(), None, p[5], 0, live.data_ptr(), rows, hint, K, K, s)]
+            assert rc == [0] * 6
+            torch.cuda.synchronize()
+            assert torch.equal(got[2], got[3]), hint
+            if first is None:
+                first = got
+            for i, (a, b) in enumerate(zip(first, got)):
+                assert torch.equal(a, b), (i, fill, hint)
+        ref = x[:M].double() @ (ws[K] if w_kn else ws[K].t()).double()
+        bound = 2.0 ** -10 * ref.abs() + K * 2.0 ** -24 * (x[:M].double().abs() @ (ws[K] if w_kn else ws[K].t()).double().abs()) + 2.0 ** -24
+        assert ((first[0][:M].double() - ref).abs() <= bound).all() and not first[0][M:].any()
+
+
+@pytest.mark.parametrize("w_kn", [False, True])
+@pytest.mark.parametrize("N,K", [(768, 768), (776, 320), (40, 256)])
+def test_plain_product_of_rows_that_only_the_device_knows(device, N, K, w_kn):
+    """Bit for bit tile 14 up to the rows that fit one round of it, tile 4 beyond, and rows past the live ones untouched;
+    a count beyond the capacity means all of it."""
+    _say("few rows", N, K, w_kn)
+    torch.manual_seed(N)
+    few = 256 // ((N + 31) // 32) * 32
+    rows = min(few + few // 2, 256 // ((N + 63) // 64) * 32)
+    a = torch.randn(rows, K, device=device).half()
+    w = (torch.randn(K, N, device=device) * 0.05).half()
+    wt = w if w_kn else w.t().contiguous()
+    lib = _lib.kernel_lib()
+    for M in (0, 1, 31, 33, few - 1, few, few + 1, few + 33, rows - 1, rows, rows + 50):
+        live = torch.tensor([M], dtype=torch.int32, device=device)
+        got = {}
+        for tile in (-1, 14 if M <= few else 4):
+            ops.set_option("gemm_tile", tile)
+            try:
+                c = torch.full((rows, N), 7.0, dtype=torch.float16, device=device)
+                assert lib.bt_gemm(a.data_ptr(), wt.data_ptr(), c.data_ptr(), live.data_ptr(), rows, 0, N, K, int(w_kn),
+                                   torch.cuda.current_stream().cuda_stream) == 0
+                got[tile] = c
+            finally:
+                ops.set_option("gemm_tile", -1)
+        first, second = got.values()
+        assert torch.equal(first, second), M
+        assert (first[M:] == 7.0).all() and (M == 0 or not (first[:M] == 7.0).all())

@@ -798,6 +798,26 @@ def test_layer_prepack_choice_never_changes_the_result(device):
                tag="layer_prepack " + cfg.name)
 
 
+def test_first_and_later_calls_on_a_mask_give_the_same_bits(device):
+    """The operator learns the number of valid tokens behind its first call on a mask: batches that are nearly empty
+    and full, around the sizes where the tiles of a few rows end."""
+    _say("first and later calls")
+    bt.load_th_op()
+    op = torch.ops.ByteTransformer.BertTransformer
+    for batch, seq, heads, lens in ((4, 96, 12, (96,) * 4), (8, 64, 12, (64,) * 8), (5, 96, 12, (90, 96, 1, 2, 96)),
+                                    (8, 64, 12, (64, 3, 3, 3, 3, 3, 3, 3)), (4, 96, 16, (96,) * 4), (3, 400, 8, (400, 400, 2))):
+        cfg = workload.EncoderConfig("again", batch, seq, heads, layers=1, lens=lens, seed=batch)
+        wl = workload.make_workload(cfg, bias_std=0.05, random_affine=True)
+        w = [_dev(wl.layers[0][n], device) for n in workload.WEIGHT_NAMES]
+        x, m = _dev(wl.x, device), _dev(wl.mask, device)
+        torch.ops.ByteTransformer.clear_caches()
+        first = op(heads, 64, *w, x, m, True, True)
+        torch.cuda.synchronize()
+        for _ in range(2):
+            assert torch.equal(op(heads, 64, *w, x, m, True, True), first), cfg
+            torch.cuda.synchronize()
+
+
 def test_qkv_rows_from_the_mask_never_change_the_result(device):
     """A padding-free layer may start with the QKV product that counts the mask rows itself
     instead of the prologue launch: never, wherever the entry takes the shape (without the
