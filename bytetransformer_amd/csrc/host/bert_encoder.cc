@@ -85,6 +85,9 @@ void BertEncoder<OpType>::infer(BertEncoderInferParam<DataType_> ip) {
   const int *valid_rows = is_remove_padding_ ? et_param.batch_idx + batch_size : nullptr;
   const int rows_hint = rows_to_plan_for(ip.valid_rows_hint, is_remove_padding_, batch_size, rows);
   const int L = (int)layers_.size();
+  // few rows, long k: FFN2 as split-k partial sums that the last LayerNorm folds in (the same in every layer)
+  const int splits =
+      OpType == OperationType::HALF ? ffn2_slices(rows, valid_rows == nullptr, hidden, inter, partials_bytes) : 1;
 
   for (int l = 0; l < L; ++l) {
     const auto &w = layers_[l];
@@ -186,8 +189,6 @@ void BertEncoder<OpType>::infer(BertEncoderInferParam<DataType_> ip) {
                                      valid_rows, rows, rows_hint, inter, hidden, weight_kn,
                                      stream));
 
-    // few rows, long k: FFN2 as split-k partial sums that the last LayerNorm folds in
-    const int splits = ffn2_slices(rows, valid_rows == nullptr, hidden, inter, partials_bytes);
     if (splits > 1) {
       const bool restore = last && is_remove_padding_;
       check_bt_error(bt_gemm_splitk_rows(inter_matmul_buf, wt_out, partials, splits, valid_rows, rows, rows_hint,

@@ -31,6 +31,7 @@
 // `valid_rows`; workgroups beyond the live tiles retire at once.
 #include "common.h"
 
+#include <cstring>
 #include <type_traits>
 #include <utility>
 
@@ -1505,6 +1506,26 @@ static WaveK takes_wave_k(const GemmArgs &p, bool plain) {
   return plain && p.valid_rows && tiles_m * ((p.N + 63) / 64) <= cu_count() ? kWaveKDevice : kWaveKNo;
 }
 
+// What a question about sizes was answered before, on this thread: a forward asks the same few in every layer,
+// and pricing them anew costs the host 0.3 to 0.9 us each, while issuing a launch takes 3 to 4.
+template <int KEYS, typename Ask>
+static int remembered(const int (&sizes)[KEYS], Ask ask) {
+  struct Entry {
+    int sizes[KEYS], answer;
+    bool known;
+  };
+  thread_local Entry entries[32];   // (of this question alone: one table per `Ask`)
+  unsigned at = 0;
+  for (int v : sizes) at = (at ^ (unsigned)v) * 0x9e3779b1u;
+  Entry &e = entries[at >> 27];
+  if (!e.known || memcmp(e.sizes, sizes, sizeof(sizes)) != 0) {
+    e.answer = ask();
+    memcpy(e.sizes, sizes, sizeof(sizes));
+    e.known = true;
+  }
+  return e.answer;
+}
+
 // ---- products in k slices ----------------------------------------------------------------
 // FFN2 of up to two thousand rows is a few dozen tiles with a k loop four times as long as the other
 // products': k slices give the idle CUs a share of it, and the LayerNorm that reads the result anyway adds
@@ -1737,9 +1758,7 @@ extern "C" int bt_gemm(const void *a, const void *wt, void *c, const int *valid_
 // The number of slices changes the order of the sums, so it follows from the sizes of the call alone, not from
 // a row count that a caller may know in one call and not in the next: a padded batch is taken to be 60 %
 // full or, less likely, full.
-extern "C" int bt_gemm_splitk_slices(int rows_cap, int all_live, int n, int k, int most) {
-  if (rows_cap <= 0 || n <= 0 || k < kBK || k % kBK != 0) return 1;
-  if (cu_count() != 256) return 0;
+static int fastest_slices(int rows_cap, bool all_live, int n, int k, int most) {
   GemmArgs p{};
   p.rows_cap = rows_cap;
   const LikelyRows full(p);
@@ -1761,6 +1780,13 @@ extern "C" int bt_gemm_splitk_slices(int rows_cap, int all_live, int n, int k, i
   return best;
 }
 
+extern "C" int bt_gemm_splitk_slices(int rows_cap, int all_live, int n, int k, int most) {
+  if (rows_cap <= 0 || n <= 0 || k < kBK || k % kBK != 0) return 1;
+  if (cu_count() != 256) return 0;
+  return remembered({rows_cap, all_live ? 1 : 0, n, k, most},
+                    [&] { return fastest_slices(rows_cap, all_live != 0, n, k, most); });
+}
+
 extern "C" int bt_gemm_splitk(const void *a, const void *wt, void *partials, int splits,
                               const int *valid_rows, int rows_cap, int n, int k, int weight_kn,
                               void *stream) {
@@ -1779,16 +1805,17 @@ extern "C" int bt_gemm_splitk_rows(const void *a, const void *wt, void *partials
   GemmArgs p{(const half_t *)a, (const half_t *)wt, nullptr, nullptr, valid_rows, nullptr,
              rows_cap,          n,                  k,       0,       rows_hint,  (float *)partials,
              weight_kn};
-  float us = 0.f;
   hipStream_t st = as_stream(stream);
-  int tile = fastest_sliced(LikelyRows(p), n, k, splits, &us).id;
-  if (rows_hint > 0) {
+  const int tile = remembered({rows_cap, valid_rows != nullptr, rows_hint, n, k, splits}, [&] {
+    float us = 0.f;
+    const int named = fastest_sliced(LikelyRows(p), n, k, splits, &us).id;
+    if (rows_hint <= 0) return named;
     // (the waves of tile 14 add up in an order of their own: not for a row count's sake either)
     GemmArgs unnamed = p;
     unnamed.rows_hint = 0;
     const int without = fastest_sliced(LikelyRows(unnamed), n, k, splits, &us).id;
-    if ((tile == 14) != (without == 14)) tile = without;
-  }
+    return (named == 14) != (without == 14) ? without : named;
+  });
   switch (tile) {
     case 14: return launch_gemm_wave_k<kEpiPartial>(p, st, splits);
     case 4: return launch_gemm_tile<32, 64, 4, 1, 2, 2, kEpiPartial>(p, st, splits);

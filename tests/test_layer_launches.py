@@ -128,3 +128,9 @@ def test_offsets_without_their_count(launches, batch, seq_len):
 def test_padded_rows_are_all_live(launches):
     got = launches("layer", 12, 2, 200, -1)
     assert got[0] == _lib.kernel_lib().bt_gemm_splitk_slices(400, 1, 768, 3072, 16)
+
+
+@pytest.mark.parametrize("batch,seq_len", [(1, 32), (4, 96), (16, 512)])
+def test_an_encoder_asks_once_for_its_slices(launches, batch, seq_len):
+    slices, _, asked = launches("encoder", 12, batch, seq_len, -1)
+    assert asked == 1 and slices == launches("layer", 12, batch, seq_len, -1)[0]

@@ -2,6 +2,8 @@
 include/bytetransformer/common.h for parts that it was not measured on, compiled as the host compiles it."""
 import os
 import subprocess
+import threading
+import time
 
 import pytest
 
@@ -63,3 +65,36 @@ def test_slices_of_a_padded_batch():
     for n, k in ((768, 3072), (1024, 4096), (512, 2048), (640, 2560)):
         for rows in range(1, 3000, 61):
             assert (k // 64) % ask(rows, 0, n, k, 16) == 0
+
+
+def test_remembered_answers_are_those_of_their_sizes():
+    """Far more sizes than are remembered, in several orders and on several threads at once."""
+    ask = _lib.kernel_lib().bt_gemm_splitk_slices
+    sizes = [(rows, live, n, 4 * n, most) for n in (512, 768, 1024) for rows in range(1, 3000, 37) for live in (0, 1)
+             for most in (2, 16)]
+    first = [ask(*s) for s in sizes]
+    seen = {}
+
+    def again(step):
+        seen[step] = [ask(*sizes[i * step % len(sizes)]) for i in range(len(sizes))]
+    threads = [threading.Thread(target=again, args=(step,)) for step in (1, 7, 11, 13)]
+    [t.start() for t in threads]
+    [t.join() for t in threads]
+    for step, got in seen.items():
+        assert got == [first[i * step % len(sizes)] for i in range(len(sizes))], step
+
+
+def test_a_size_is_priced_once():
+    """A forward asks the same in every layer: the answer is looked up, for less than a third of what it costs to find."""
+    ask = _lib.kernel_lib().bt_gemm_splitk_slices
+
+    def ns(rows):
+        best = []
+        for _ in range(7):
+            t0 = time.perf_counter_ns()
+            for r in rows:
+                ask(r, 0, 768, 3072, 16)
+            best.append(time.perf_counter_ns() - t0)
+        return min(best) / len(rows)
+    other = ns([0] * 600)                        # (the call itself; no rows are answered at once)
+    assert ns([384] * 600) - other < (ns(list(range(300, 900))) - other) / 3
