@@ -78,17 +78,48 @@ struct GemmArgs {
 #define BT_GEMM_FIRST_NAMES a, wt, valid_rows, mask, rows_cap, N, K, tiles_n, splits, tile_grid
 #define BT_GEMM_FIRST_OF(p) \
   p.a, p.wt, p.valid_rows, p.mask, p.rows_cap, p.N, p.K, p.tiles_n, p.splits, p.tile_grid
-__device__ __forceinline__ GemmArgs gemm_args(BT_GEMM_FIRST, const GemmArgs &rest) {
-  GemmArgs p = rest;
-  p.a = a, p.wt = wt, p.valid_rows = valid_rows, p.mask = mask;
-  p.rows_cap = rows_cap, p.N = N, p.K = K, p.tiles_n = tiles_n, p.splits = splits, p.tile_grid = tile_grid;
-  return p;
-}
-
 // Where a product takes its rows from, as a template parameter: the code that counts the mask rows is 9 KB,
 // three quarters of a small kernel, and the kernels of a layer share an instruction cache of 64 KB (12 layers
 // without it where no mask is counted: 1 x 32 385 -> 374 us, 4 x 96 430 -> 422, 7 x 217 638 -> 626).
 constexpr int kMaskNone = 0, kMaskF16 = 1, kMaskF32 = 2;
+
+// ... and what it needs later.  Every argument byte costs the host: beside ten leading arguments a launch takes
+// 3.0 us to issue with 24 bytes more, 3.6 with 48, and 3.8 with the whole of GemmArgs (128), so the fields of a
+// launch that counts mask rows travel with those launches only.
+template <int MASK>
+struct GemmTail {
+  const half_t *bias;
+  void *out;   // c or c32
+  const int *a_row_index;
+  int mask_B, mask_S;
+  int *out_batch_idx, *out_word_idx, *out_seq_order;
+};
+template <>
+struct GemmTail<kMaskNone> {
+  const half_t *bias;
+  void *out;
+  const int *a_row_index;
+};
+template <int MASK>
+static GemmTail<MASK> gemm_tail(const GemmArgs &p) {
+  void *out = p.c32 ? (void *)p.c32 : (void *)p.c;
+  if constexpr (MASK == kMaskNone)
+    return {p.bias, out, p.a_row_index};
+  else
+    return {p.bias, out, p.a_row_index, p.mask_B, p.mask_S, p.out_batch_idx, p.out_word_idx, p.out_seq_order};
+}
+template <int MASK>
+__device__ __forceinline__ GemmArgs gemm_args(BT_GEMM_FIRST, const GemmTail<MASK> &tail) {
+  GemmArgs p{};
+  p.a = a, p.wt = wt, p.valid_rows = valid_rows, p.mask = mask;
+  p.rows_cap = rows_cap, p.N = N, p.K = K, p.tiles_n = tiles_n, p.splits = splits, p.tile_grid = tile_grid;
+  p.bias = tail.bias, p.c = (half_t *)tail.out, p.c32 = (float *)tail.out, p.a_row_index = tail.a_row_index;
+  if constexpr (MASK != kMaskNone) {
+    p.mask_B = tail.mask_B, p.mask_S = tail.mask_S;
+    p.out_batch_idx = tail.out_batch_idx, p.out_word_idx = tail.out_word_idx, p.out_seq_order = tail.out_seq_order;
+  }
+  return p;
+}
 
 // ---- rows from the mask ---------------------------------------------------------
 constexpr int kMaskRowsMaxBatch = 64;   // one wave scans the lengths
@@ -979,16 +1010,16 @@ __device__ __forceinline__ void for_each_tile(const GemmArgs &p, Tile tile) {
 }
 
 template <int BM, int BN, int STAGES, int WM, int WN, int NP, int EPI, bool WKN, int MASK>
-__global__ __launch_bounds__((WM * WN + NP) * 64) void gemm_flat_kernel(BT_GEMM_FIRST, GemmArgs rest) {
+__global__ __launch_bounds__((WM * WN + NP) * 64) void gemm_flat_kernel(BT_GEMM_FIRST, GemmTail<MASK> tail) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  gemm_tiles_flat<BM, BN, STAGES, WM, WN, NP, EPI, WKN, MASK>(gemm_args(BT_GEMM_FIRST_NAMES, rest));
+  gemm_tiles_flat<BM, BN, STAGES, WM, WN, NP, EPI, WKN, MASK>(gemm_args<MASK>(BT_GEMM_FIRST_NAMES, tail));
 #endif
 }
 
 template <int BM, int BN, int STAGES, int WM, int WN, int NP, int EPI, bool WKN, int MASK, bool LOOP>
-__global__ __launch_bounds__((WM * WN + NP) * 64) void gemm_kernel(BT_GEMM_FIRST, GemmArgs rest) {
+__global__ __launch_bounds__((WM * WN + NP) * 64) void gemm_kernel(BT_GEMM_FIRST, GemmTail<MASK> tail) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  const GemmArgs p = gemm_args(BT_GEMM_FIRST_NAMES, rest);
+  const GemmArgs p = gemm_args<MASK>(BT_GEMM_FIRST_NAMES, tail);
   if constexpr (LOOP)
     for_each_tile(p, [&](int bid) { return gemm_tile<BM, BN, STAGES, WM, WN, NP, EPI, WKN, MASK, LOOP>(p, bid); });
   else
@@ -1174,18 +1205,18 @@ __device__ __forceinline__ void gemm_wave_k(const GemmArgs &p) {
 #endif  // __HIP_DEVICE_COMPILE__
 
 template <int EPI, bool WKN, int MASK>
-__global__ __launch_bounds__(kWaveKWaves * 64) void gemm_wave_k_kernel(BT_GEMM_FIRST, GemmArgs rest) {
+__global__ __launch_bounds__(kWaveKWaves * 64) void gemm_wave_k_kernel(BT_GEMM_FIRST, GemmTail<MASK> tail) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  gemm_wave_k<EPI, WKN, MASK>(gemm_args(BT_GEMM_FIRST_NAMES, rest));
+  gemm_wave_k<EPI, WKN, MASK>(gemm_args<MASK>(BT_GEMM_FIRST_NAMES, tail));
 #endif
 }
 
 // Plain products whose live rows only the device knows: tile 14 where they fit one round of it, else tile 4
 // (see takes_wave_k).  `splits` brings the most rows of tile 14: an argument that is there at wave launch.
 template <bool WKN>
-__global__ __launch_bounds__(kWaveKWaves * 64) void gemm_few_rows_kernel(BT_GEMM_FIRST, GemmArgs rest) {
+__global__ __launch_bounds__(kWaveKWaves * 64) void gemm_few_rows_kernel(BT_GEMM_FIRST, GemmTail<kMaskNone> tail) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  GemmArgs p = gemm_args(BT_GEMM_FIRST_NAMES, rest);
+  GemmArgs p = gemm_args<kMaskNone>(BT_GEMM_FIRST_NAMES, tail);
   p.splits = 1;
   if (*valid_rows <= splits) {
     gemm_wave_k<kEpiPlain, WKN, kMaskNone>(p);
@@ -1250,7 +1281,7 @@ static int launch_gemm_kernel(const GemmArgs &p, hipStream_t s, size_t smem) {
                                    configured, "hipFuncSetAttribute(gemm_kernel)");
   if (rc != BT_OK) return rc;
   gemm_kernel<BM, BN, STAGES, WM, WN, NP, EPI, WKN, MASK, LOOP>
-      <<<dim3(p.tile_grid), (WM * WN + NP) * 64, smem, s>>>(BT_GEMM_FIRST_OF(p), p);
+      <<<dim3(p.tile_grid), (WM * WN + NP) * 64, smem, s>>>(BT_GEMM_FIRST_OF(p), gemm_tail<MASK>(p));
   BT_CHECK_LAUNCH("gemm_kernel");
   return BT_OK;
 }
@@ -1292,7 +1323,8 @@ static int launch_gemm_wave_k_as(GemmArgs p, hipStream_t s, int splits) {
   p.tiles_n = (p.N + kWaveKCols - 1) / kWaveKCols;
   p.splits = splits;
   p.tile_grid = ((p.rows_cap + 31) / 32 * p.tiles_n * splits + 7) / 8 * 8;
-  gemm_wave_k_kernel<EPI, WKN, MASK><<<dim3(p.tile_grid), kWaveKWaves * 64, smem, s>>>(BT_GEMM_FIRST_OF(p), p);
+  gemm_wave_k_kernel<EPI, WKN, MASK>
+      <<<dim3(p.tile_grid), kWaveKWaves * 64, smem, s>>>(BT_GEMM_FIRST_OF(p), gemm_tail<MASK>(p));
   BT_CHECK_LAUNCH("gemm_wave_k_kernel");
   return BT_OK;
 }
@@ -1316,7 +1348,8 @@ static int launch_gemm_few_rows_as(GemmArgs p, hipStream_t s) {
   p.splits = cu_count() / p.tiles_n * 32;
   const int few = p.splits / 32 * p.tiles_n, wide = (p.rows_cap + 31) / 32 * ((p.N + 63) / 64);
   p.tile_grid = ((few > wide ? few : wide) + 7) / 8 * 8;
-  gemm_few_rows_kernel<WKN><<<dim3(p.tile_grid), kWaveKWaves * 64, smem, s>>>(BT_GEMM_FIRST_OF(p), p);
+  gemm_few_rows_kernel<WKN>
+      <<<dim3(p.tile_grid), kWaveKWaves * 64, smem, s>>>(BT_GEMM_FIRST_OF(p), gemm_tail<kMaskNone>(p));
   BT_CHECK_LAUNCH("gemm_few_rows_kernel");
   return BT_OK;
 }
@@ -1343,7 +1376,7 @@ static int launch_gemm_flat_as(GemmArgs p, hipStream_t s) {
   p.tile_grid = (int)((wgs + 7) / 8 * 8);
   const dim3 grid((unsigned)p.tile_grid);
   gemm_flat_kernel<BM, BN, STAGES, WM, WN, NP, EPI, WKN, MASK>
-      <<<grid, (WM * WN + NP) * 64, smem, s>>>(BT_GEMM_FIRST_OF(p), p);
+      <<<grid, (WM * WN + NP) * 64, smem, s>>>(BT_GEMM_FIRST_OF(p), gemm_tail<MASK>(p));
   BT_CHECK_LAUNCH("gemm_flat_kernel");
   return BT_OK;
 }

@@ -50,6 +50,22 @@ def test_no_kernel_spills(code_objects):
     assert not bad, bad
 
 
+def test_products_bring_few_argument_bytes(code_objects):
+    """Every argument byte costs the host, most of it beyond 80 (0.5 us a launch): only launches that count mask rows
+    bring their fields."""
+    sizes = {}
+    for code in code_objects:
+        for block in re.split(r"\n  - \.agpr_count", _tool("llvm-readelf", "--notes", code))[1:]:
+            name = re.search(r"\.name: +(\S+)", block).group(1)
+            m = re.search(r"gemm_(?:flat_|wave_k_|few_rows_)?kernelI(.*)EEv", name)
+            if m and "f32" not in name:
+                ints = re.findall(r"L[ib](\d+)E", m.group(1) + "E")
+                mask = {"gemm_kernel": ints[8:9], "gemm_flat": ints[8:9], "gemm_wave": ints[2:3]}.get(
+                    re.search(r"gemm_[a-z]+", name).group(0), ["0"])[0]
+                sizes.setdefault(mask != "0", set()).add(int(re.search(r"\.kernarg_segment_size: +(\d+)", block).group(1)))
+    assert max(sizes[False]) <= 80 and max(sizes[True]) <= 112, sizes
+
+
 # Wait states between a matrix instruction and the first other use of its result, which the hardware does not enforce:
 # passes + 4 on the XDL units (16-bit operands), passes + 2 on the others.
 RESULT_WAIT = {"v_mfma_f32_32x32x2_f32": 16 + 2, "v_mfma_f32_32x32x16_f16": 8 + 4, "v_mfma_f32_32x32x16_bf16": 8 + 4,
