@@ -473,14 +473,20 @@ __device__ __forceinline__ AttWork att_work_balanced(const Args &p, unsigned int
 // workgroups still compute (and stay in the memory-side cache, which a non-temporal store would pass by).
 // FFN1 at 4800 rows 28.7 -> 26.3 us a launch, at 9830 rows 55.4 -> 52.1, projection at 4800 rows 9.8 ->
 // 9.0, QKV at 911 rows 8.8 -> 8.3.
-// (s_nop: what follows may overwrite the registers of a 16-byte store after two wait states, which the compiler
-// does not see of assembly.  The attention keeps ordinary stores: its rows leave in pieces of 32 bytes, which
-// the L2 joins; written through they cost 0.3 to 1.4 % of a forward.)
+// The attention keeps ordinary stores: its rows leave in pieces of 32 bytes, which the L2 joins; written through
+// they cost 0.3 to 1.4 % of a forward.
+// (Stores that the compiler knows, agent scope being what writes through: it keeps them in order with other
+// accesses to the same memory and waits for what a matrix instruction has yet to write into their registers.)
 __device__ __forceinline__ void store_through(void *to, uint4_t v) {
-  asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(to), "v"(v));
+#if defined(__HIP_DEVICE_COMPILE__)
+  __builtin_amdgcn_global_store_b128((__attribute__((address_space(1))) uint4_t *)to, v, "agent");
+#endif
 }
 __device__ __forceinline__ void store_through(void *to, uint2_t v) {
-  asm volatile("global_store_dwordx2 %0, %1, off sc1" ::"v"(to), "v"(v));
+#if defined(__HIP_DEVICE_COMPILE__)
+  __hip_atomic_store((__attribute__((address_space(1))) unsigned long long *)to, __builtin_bit_cast(unsigned long long, v),
+                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#endif
 }
 
 }  // namespace bt

@@ -145,6 +145,16 @@ def test_no_kernel_reads_a_matrix_result_early(code_objects):
     assert not early, early
 
 
+def test_the_compiler_knows_every_store():
+    """Assembly that stores is nothing to the compiler: it neither waits for the matrix instruction whose result goes
+    out nor keeps the store in order with other accesses to the same memory."""
+    folder = os.path.join(build.CSRC, "kernels")
+    hidden = [(f, text) for f in sorted(os.listdir(folder)) if f.endswith((".h", ".hip"))
+              for text in re.findall(r"\basm(?:\s+volatile)?\s*\(([^;]*);", open(os.path.join(folder, f)).read())
+              if re.search(r"(global|buffer|flat|scratch)_(store|atomic)|ds_(write|add|max)", text)]
+    assert not hidden, hidden
+
+
 LOAD = re.compile(r"(ds_read|ds_bpermute|ds_permute|ds_swizzle|global_load|buffer_load|flat_load|scratch_load)")
 COUNTED = {"lgkmcnt": re.compile(r"ds_"), "vmcnt": re.compile(r"(global|buffer|flat|scratch)_(load|store|atomic)")}
 
