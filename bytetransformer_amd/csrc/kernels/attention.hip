@@ -860,19 +860,24 @@ struct GroupedPlan {
   unsigned grid;
 };
 constexpr long long kNarrowBlocks = 208;
-// Two or three key tiles leave waves without keys and fewer turns to save, so it has to be fewer workgroups there.
-// 64-query against 16-query tiles, whole forwards: 12 heads at 1 x 96 (72 workgroups of 16 queries) 402 / 399 us,
-// 1 x 128 (96) 401 / 398, 2 x 96 (144) 412 / 408, 1 x 180 (144) 423 / 429, 2 x 120 (192) 422 / 438; 16 heads, 24
-// layers, at 1 x 140 (144) 972 / 944, 1 x 190 (192) 1058 / 1080, 2 x 90 (192) 1021 / 1061.
-constexpr long long kNarrowBlocksShort = 160;
+// Two or three key tiles leave waves without keys and fewer turns to save, so it has to be fewer workgroups there; so it
+// has where the three weights to warm up fill the 12 MB that a launch takes on (hidden 816 and more), since every
+// workgroup beyond 160 takes one from the warm-up.  Whole forwards, 64-query against 16-query tiles, us, operator /
+// graph (full, 60 % full): 12 heads, 12 layers, at 1 x 128 (96 workgroups of 16 queries) 378 374 / 368 368, 369 367;
+// 2 x 96 (144) 387 381; 1 x 180 (144) 398 387 / 394 386, 385 387; 2 x 120 (192) 393 392; 1 x 256 (192) 414 395 / 413 396,
+// 405 396; 16 heads, 24 layers, at 1 x 128 (128) 938 929; 1 x 160 (160) 995 968; 2 x 96 (192) 1030 1073 / 920 951, 904 949;
+// 1 x 190 (192) 1060 1083 / 934 955, 917 953; 1 x 200 (208) 1035 1041 / 951 955, 916 951; 1 x 256 (256) 1094 1103.
+constexpr long long kNarrowBlocksFew = 160;
+constexpr int kNarrowHidden = 816;
 static GroupedPlan plan_grouped(AttArgs &a, int batch_size, int seq_len, int head_num) {
   const long long blocks128 = (long long)((seq_len + 127) / 128) * head_num * batch_size;
   const int qb = option_attention_qb();
   GroupedPlan plan;
   plan.wide = qb == 2 || (qb < 0 && blocks128 >= 1300);
   const long long blocks16 = (long long)((seq_len + 15) / 16) * head_num * batch_size;
-  plan.narrow = qb < 0 && option_attention_key_split() < 0 && option_attention_xcd_map() != 3 && seq_len > kKT && seq_len <= 4 * kKT &&
-                blocks16 <= (seq_len > 3 * kKT ? kNarrowBlocks : kNarrowBlocksShort);
+  const long long most = seq_len > 3 * kKT && head_num * kHeadDim < kNarrowHidden ? kNarrowBlocks : kNarrowBlocksFew;
+  plan.narrow = qb < 0 && option_attention_key_split() < 0 && option_attention_xcd_map() != 3 && seq_len > kKT &&
+                seq_len <= 4 * kKT && blocks16 <= most && cu_count() == 256;
   plan.grid = att_grid(a, plan.wide ? (seq_len + 127) / 128 : plan.narrow ? (seq_len + 15) / 16 : (seq_len + 63) / 64,
                        true);
   return plan;

@@ -81,6 +81,8 @@ int option_prefetch();       // 1 = honour the prefetch hints of the attention e
 int option_attention_key_split();  // streaming attention, 64-query tiles: -1 heuristic, 0 four waves, 1 eight waves over two key halves
 int option_prefetch_min_grid();   // attention launches of fewer workgroups bring workgroups of their own for the cache warm-up (default 512)
 
+int cu_count();   // of the part that the process started on
+
 inline hipStream_t as_stream(void *s) { return reinterpret_cast<hipStream_t>(s); }
 
 // Every kernel moves tensors in 16-byte pieces: all tensor pointers of an entry point must

@@ -1251,7 +1251,6 @@ __global__ __launch_bounds__(256) void transpose_kernel(TransposeArgs a) {
                     threadIdx.x, true);
 }
 
-static int cu_count();
 static long long estimated_rows(const GemmArgs &p);
 // Workgroups of a launch whose kernel can go on to further tiles (see for_each_tile): for the expected rows, of
 // which a fifth more may come where the number is a guess, in whole rounds of the chip; `all` at most.
@@ -1388,7 +1387,7 @@ static int launch_gemm_flat(GemmArgs p, hipStream_t s) {
   });
 }
 
-static int cu_count() {
+int cu_count() {
   static const int cus = [] {
     int dev = 0, n = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
