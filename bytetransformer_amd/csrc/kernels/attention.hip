@@ -110,8 +110,36 @@ inline AttFirst att_first(const AttArgs &a) {
                   a.per_heads, (unsigned)a.xcd_map | (list ? kAttList : 0) | (a.padded_rows ? kAttPadded : 0) |
                                    (a.every_key ? kAttEveryKey : 0)};
 }
-__device__ __forceinline__ AttArgs att_args(BT_ATT_FIRST, const AttArgs &rest) {
-  AttArgs p = rest;
+// ... and what it needs later: every argument byte costs the host (4.6 us to issue a launch with the whole of AttArgs
+// here, 4.3 with this), so the additive terms travel with the kernels that apply them.
+struct AttTerms {
+  const half_t *mask, *bias;
+  const int *mask_ok;
+};
+struct AttNoTerms {};
+template <int KIND>
+struct AttTail : std::conditional_t<(KIND & kAddBoth) != 0, AttTerms, AttNoTerms> {
+  half_t *out;
+  float scale_log2e;
+  unsigned warm_first, warm_per;
+  unsigned warm_end[kWarmRanges];
+  const char *warm_base[kWarmRanges];
+};
+template <int KIND>
+static AttTail<KIND> att_tail(const AttArgs &a) {
+  AttTail<KIND> t{};
+  if constexpr ((KIND & kAddBoth) != 0) t.mask = a.mask, t.bias = a.bias, t.mask_ok = a.mask_ok;
+  t.out = a.out, t.scale_log2e = a.scale_log2e, t.warm_first = a.warm.first, t.warm_per = a.warm.per;
+  for (int r = 0; r < kWarmRanges; ++r) t.warm_end[r] = a.warm.end[r], t.warm_base[r] = a.warm.base[r];
+  return t;
+}
+template <int KIND>
+__device__ __forceinline__ AttArgs att_args(BT_ATT_FIRST, const AttTail<KIND> &tail) {
+  AttArgs p{};
+  if constexpr ((KIND & kAddBoth) != 0) p.mask = tail.mask, p.bias = tail.bias, p.mask_ok = tail.mask_ok;
+  p.out = tail.out, p.scale_log2e = tail.scale_log2e, p.warm.first = tail.warm_first, p.warm.per = tail.warm_per;
+#pragma unroll
+  for (int r = 0; r < kWarmRanges; ++r) p.warm.end[r] = tail.warm_end[r], p.warm.base[r] = tail.warm_base[r];
   p.qkv = qkv, p.batch_idx = batch_idx;
   p.seq_order = flags & kAttList ? nullptr : order;
   p.work_list = flags & kAttList ? (const int4 *)order : nullptr;
@@ -582,8 +610,8 @@ __device__ __forceinline__ void attention_tile(const AttArgs &p, const AttTile &
 }
 
 template <int QB, int KIND, int STAGES, int KS = 1, int WQ = 4>
-__global__ __launch_bounds__(64 * WQ * KS, KS == 2 && !KIND ? 4 : 2) void attention_grouped_kernel(BT_ATT_FIRST, AttArgs rest) {
-  const AttArgs p = att_args(BT_ATT_FIRST_NAMES, rest);
+__global__ __launch_bounds__(64 * WQ * KS, KS == 2 && !KIND ? 4 : 2) void attention_grouped_kernel(BT_ATT_FIRST, AttTail<KIND> tail) {
+  const AttArgs p = att_args<KIND>(BT_ATT_FIRST_NAMES, tail);
   __shared__ __attribute__((aligned(1024))) half_t ring[STAGES * KS * 2 * kTileHalfs];
   AttTile item;
   if (att_tile<16 * WQ * QB>(p, item)) attention_tile<QB, KIND, STAGES, KS, WQ>(p, item, ring);
@@ -892,14 +920,15 @@ static void launch_grouped(const AttArgs &a, const GroupedPlan &plan, int seq_le
   // workgroups of the attention itself: those that a warm-up hint adds leave the sums as they are.
   const int ks = option_attention_key_split();
   const AttFirst f = att_first(a);
+  const AttTail<KIND> t = att_tail<KIND>(a);
   if (plan.narrow)
-    attention_grouped_kernel<1, KIND, 1, 4, 1><<<grid, kAttThreads, 0, s>>>(BT_ATT_FIRST_OF(f), a);
+    attention_grouped_kernel<1, KIND, 1, 4, 1><<<grid, kAttThreads, 0, s>>>(BT_ATT_FIRST_OF(f), t);
   else if (plan.wide)
-    attention_grouped_kernel<2, KIND, kWideStages><<<grid, kAttThreads, 0, s>>>(BT_ATT_FIRST_OF(f), a);
+    attention_grouped_kernel<2, KIND, kWideStages><<<grid, kAttThreads, 0, s>>>(BT_ATT_FIRST_OF(f), t);
   else if (ks == 1 || (ks < 0 && seq_len >= 512 && a.warm.grid_work <= 256))
-    attention_grouped_kernel<1, KIND, 2, 2><<<grid, 2 * kAttThreads, 0, s>>>(BT_ATT_FIRST_OF(f), a);
+    attention_grouped_kernel<1, KIND, 2, 2><<<grid, 2 * kAttThreads, 0, s>>>(BT_ATT_FIRST_OF(f), t);
   else
-    attention_grouped_kernel<1, KIND, 2><<<grid, kAttThreads, 0, s>>>(BT_ATT_FIRST_OF(f), a);
+    attention_grouped_kernel<1, KIND, 2><<<grid, kAttThreads, 0, s>>>(BT_ATT_FIRST_OF(f), t);
 }
 AttListPlan att_worklist_plan(int B, int S, int heads) {
   AttListPlan out{0, 64, 0};

@@ -66,6 +66,18 @@ def test_products_bring_few_argument_bytes(code_objects):
     assert max(sizes[False]) <= 80 and max(sizes[True]) <= 112, sizes
 
 
+def test_the_streaming_attention_brings_few_argument_bytes(code_objects):
+    """The same for the 64-wide attention: 176 bytes as one struct before its first arguments came in registers."""
+    sizes = {}
+    for code in code_objects:
+        for block in re.split(r"\n  - \.agpr_count", _tool("llvm-readelf", "--notes", code))[1:]:
+            m = re.search(r"\.name: +\S*attention_grouped_kernelILi\dELi(\d)E", block)
+            if m:
+                terms = int(m.group(1)) in (1, 2, 3)
+                sizes.setdefault(terms, set()).add(int(re.search(r"\.kernarg_segment_size: +(\d+)", block).group(1)))
+    assert max(sizes[False]) <= 128 and max(sizes[True]) <= 152, sizes
+
+
 # Wait states between a matrix instruction and the first other use of its result, which the hardware does not enforce:
 # passes + 4 on the XDL units (16-bit operands), passes + 2 on the others.
 RESULT_WAIT = {"v_mfma_f32_32x32x2_f32": 16 + 2, "v_mfma_f32_32x32x16_f16": 8 + 4, "v_mfma_f32_32x32x16_bf16": 8 + 4,
