@@ -81,6 +81,9 @@ def pytest_generate_tests(metafunc):
     name = metafunc.function.__name__
     if ("gemm" in name or "splitk" in name) and "weight_layout" in metafunc.fixturenames:
         metafunc.parametrize("weight_layout", ["nk", "kn"], indirect=True)
+    values, ids = [0, 1, -1], ["four-waves", "key-split", "own-choice"]
+    most = 3 if "attention" in name else 2
+    metafunc.parametrize("attention_key_split", values[:most], ids=ids[:most], indirect=True)
 
 
 def _prep(w):
@@ -951,11 +954,12 @@ def test_mask_is_prefix(device, np_dtype):
 
 
 # ---- attention -----------------------------------------------------------------
-@pytest.fixture(autouse=True, params=[0, 1], ids=["four-waves", "key-split"])
+@pytest.fixture(autouse=True)
 def attention_key_split(request):
     """The streaming attention kernel's 64-query variant exists with four waves and with
     eight (two key halves merged at the end); every test of this file runs under both
-    (the option does not touch the other kernels)."""
+    (the option does not touch the other kernels).  Pinned to either, the form of 16 queries a
+    workgroup is never taken: the attention's tests run a third time on the library's own choice."""
     ops.set_option("attention_key_split", request.param)
     yield request.param
     ops.set_option("attention_key_split", -1)
@@ -983,6 +987,10 @@ ATT_CASES = [
     ("grouped", [1024, 205, 700], 1024, 2),
     ("grouped", [154], 256, 12),
     ("grouped", [33, 2, 47], 47, 5),
+    # 16 queries a workgroup, one to four key tiles
+    ("grouped", [65], 65, 2),
+    ("grouped", [100, 17], 100, 3),
+    ("grouped", [256, 0, 193], 256, 2),
 ]
 
 
@@ -1182,7 +1190,7 @@ def test_attention_work_list(device, lens, S, heads, padded, qb):
     assert ops.attention_worklist(bi, 1, 64, 2, False) is None
 
 
-@pytest.mark.parametrize("qb", [1, 2])
+@pytest.mark.parametrize("qb", [1, 2, -1])
 def test_attention_drops_a_prefix_mask_on_the_device(device, qb, att_order):
     """The streaming kernel with the verdict slots of the device-side mask check: a plain
     prefix mask is ignored (keys stop at the lengths: the values of the padded rows'
@@ -1444,6 +1452,53 @@ def test_splitk_slices_at_the_edges_of_their_tiles(device, splits, w_kn):
         assert (got[:, M:] == 7.0).all(), M
 
 
+@pytest.mark.parametrize("w_kn", [False, True])
+def test_splitk_on_waves_over_k(device, w_kn):
+    """FFN2 of up to 64 rows in four slices runs on tile 14, of 128 rows on another: every slice is, rounded to half,
+    the plain product of its share of k on that tile, bit for bit (some of 49152 sums and more differ between two
+    tiles).  A row hint on either side of the step never moves it."""
+    _say("splitk on tile 14", w_kn)
+    torch.manual_seed(14)
+    N, K, splits = 768, 3072, 4
+    lib, s = _lib.kernel_lib(), torch.cuda.current_stream().cuda_stream
+    w = (torch.randn(K, N, device=device) * 0.05).half()
+    wt = w if w_kn else w.t().contiguous()
+    a = torch.randn(160, K, device=device).half()
+
+    def sliced(rows, live, hint):
+        out = torch.full((splits, rows, N), 7.0, device=device)
+        assert lib.bt_gemm_splitk_rows(a.data_ptr(), wt.data_ptr(), out.data_ptr(), splits, live, rows, hint, N, K, int(w_kn),
+                                       s) == 0
+        return out
+
+    def plain(rows, tile, i):
+        part = w[i * 768:(i + 1) * 768]
+        x, part = a[:rows, i * 768:(i + 1) * 768].contiguous(), part.contiguous() if w_kn else part.t().contiguous()
+        out = torch.empty(rows, N, dtype=torch.float16, device=device)
+        ops.set_option("gemm_tile", tile)
+        try:
+            assert lib.bt_gemm(x.data_ptr(), part.data_ptr(), out.data_ptr(), None, rows, 0, N, 768, int(w_kn), s) == 0
+        finally:
+            ops.set_option("gemm_tile", -1)
+        return out
+
+    for rows in (1, 31, 33, 64, 128):
+        got = sliced(rows, None, 0).half()
+        on14, on4 = (torch.stack([plain(rows, tile, i) for i in range(splits)]) for tile in (14, 4))
+        if rows <= 64:
+            assert torch.equal(got, on14), rows
+        if rows == 64:
+            assert not torch.equal(on14, on4)
+        if rows == 128:
+            assert torch.equal(got, on4) and not torch.equal(got, on14)
+    for rows in (40, 64, 80, 100, 128, 160):
+        live = torch.tensor([rows // 2], dtype=torch.int32, device=device)
+        first = sliced(rows, live.data_ptr(), 0)
+        for hint in (1, 32, 64, 65, rows):
+            assert torch.equal(sliced(rows, live.data_ptr(), hint), first), (rows, hint)
+        assert (first[:, rows // 2:] == 7.0).all()
+
+
 def test_splitk_three_slices_restored(device):
     """Three partial sums folded into the padded output, as into the packed one, and as their sum through the plain
     LayerNorm: the kernels may round a result to half by way of a float or straight, which is one last bit apart."""
@@ -1470,13 +1525,13 @@ def test_splitk_three_slices_restored(device):
 
 @pytest.mark.parametrize("kind", ["none", "mask", "bias", "both", "zero"])
 def test_attention_of_sixteen_queries_a_workgroup(device, kind):
-    """Few sequences of more than one key tile: queries and keys around the tiles of 16, 64 and 256, ragged lengths
-    (an empty one too), with a warm-up hint.  As the four-wave form within the rounding of the probabilities: both
+    """Few sequences of more than one key tile: queries and keys around the tiles of 16, 64 and 256, up to the most
+    workgroups that take the form (160, 208 of four key tiles), ragged lengths (an empty one too), with a warm-up hint.  As the four-wave form within the rounding of the probabilities: both
     round them to half before the second product, in units that differ by at most 2^8, and the output to half."""
     _say("narrow attention", kind)
     rs = np.random.RandomState(11)
-    for B, S, heads, lens in ((1, 65, 2, (65,)), (1, 256, 12, (256,)), (1, 321, 12, (257,)), (2, 100, 3, (100, 17)),
-                              (3, 240, 2, (0, 240, 193)), (1, 1000, 4, (999,))):
+    for B, S, heads, lens in ((1, 65, 2, (65,)), (1, 256, 12, (256,)), (1, 193, 12, (193,)), (2, 100, 3, (100, 17)),
+                              (3, 240, 2, (0, 240, 193)), (4, 160, 4, (1, 64, 65, 160)), (2, 208, 8, (129, 208))):
         padded = kind in ("mask", "both")
         rows = B * S
         qkv = torch.randn(3, heads, rows, 64, device=device).half()
@@ -1503,6 +1558,7 @@ def test_attention_of_sixteen_queries_a_workgroup(device, kind):
                 ops.set_option("attention_key_split", -1)
         bound = 2.0 ** -9 * got[0].abs() + 2.0 ** -9 * 4
         assert ((got[-1] - got[0]).abs() <= bound).all(), (B, S, heads)
+        assert not torch.equal(got[-1], got[0]), (B, S, heads)   # (it is the other form)
 
 
 @pytest.mark.parametrize("B,S,heads,narrow", [(1, 144, 16, True), (1, 160, 16, True), (1, 161, 16, False), (1, 200, 16, False),
@@ -1525,9 +1581,11 @@ def test_which_attention_takes_sixteen_queries_a_workgroup(device, B, S, heads, 
 @pytest.mark.parametrize("tile", [0, 1, 2, 3, 4, 5, 9, 10, 11, 12, 13, 14])
 @pytest.mark.parametrize("w_kn", [False, True])
 def test_gemm_of_more_rows_than_it_was_told(device, tile, w_kn):
-    """A launch is sized for the rows that its caller expects, in whole rounds of the chip; with a single row expected
-    its workgroups go through two and more tiles each, and the results are those of a launch that knew, bit for
-    bit: plain, GELU, the head split with gathered rows and with rows counted from the mask, and k slices."""
+    """A launch of a tile that fills its CU (0 to 3, 11 to 13) is sized for the rows that its caller expects, in whole
+    rounds of the chip; with a single row expected its workgroups go through two and more tiles each, and the results
+    are those of a launch that knew, bit for bit: plain, GELU, the head split with gathered rows and with rows counted
+    from a mask of halfs or of floats.  The launches of the other tiles, and k slices, are sized for the capacity: there the
+    expected rows change nothing either."""
     _say("gemm more rows", tile, w_kn)
     torch.manual_seed(tile)
     heads, K = 12, 768
@@ -1558,13 +1616,14 @@ def test_gemm_of_more_rows_than_it_was_told(device, tile, w_kn):
         assert lib.bt_gemm_qkv_bias_split(x.data_ptr(), order.data_ptr(), ws[2304].data_ptr(), bias[2304].data_ptr(),
                                           c.data_ptr(), live.data_ptr(), rows, hint, heads, 64, int(w_kn), s) == 0
         out.append(c)
-        if lib.bt_gemm_qkv_mask_rows_supported(B, S, 1):
-            c = torch.zeros(3 * rows, 768, dtype=torch.float16, device=device)
-            ints = torch.zeros(3, rows + 1, dtype=torch.int32, device=device)
-            assert lib.bt_gemm_qkv_bias_split_mask_rows(
-                x.data_ptr(), mask.data_ptr(), 1, B, S, ws[2304].data_ptr(), bias[2304].data_ptr(), c.data_ptr(),
-                ints[0].data_ptr(), ints[1].data_ptr(), ints[2].data_ptr(), hint, heads, 64, int(w_kn), s) == 0
-            out += [c, ints]
+        for dtype, m in ((1, mask), (0, mask.float())):
+            if lib.bt_gemm_qkv_mask_rows_supported(B, S, dtype):
+                c = torch.zeros(3 * rows, 768, dtype=torch.float16, device=device)
+                ints = torch.zeros(3, rows + 1, dtype=torch.int32, device=device)
+                assert lib.bt_gemm_qkv_bias_split_mask_rows(
+                    x.data_ptr(), m.data_ptr(), dtype, B, S, ws[2304].data_ptr(), bias[2304].data_ptr(), c.data_ptr(),
+                    ints[0].data_ptr(), ints[1].data_ptr(), ints[2].data_ptr(), hint, heads, 64, int(w_kn), s) == 0
+                out += [c, ints]
         return out
 
     ops.set_option("gemm_tile", tile)

@@ -21,6 +21,12 @@ SOURCE = r"""
 using namespace bytetransformer;
 
 static int slices = 0, asked = 0, live_by_size = 0;   // of FFN2; questions after them; products of known rows
+struct Span {
+  const char *begin, *end;
+};
+static Span partials, scratch;
+static std::vector<Span> others;   // what the LayerNorm behind the slices reads and writes, and what outlives it
+static void take(const void *p, unsigned long long bytes) { others.push_back({(const char *)p, (const char *)p + bytes}); }
 extern "C" {
 int bt_layer_prologue(const void *, int, int, int, int *, int *, int *, int *, void *, int, int, int, const void *const *,
                       void *const *, const int *, const int *, int, const void *const *, const unsigned long long *, void *) { return 0; }
@@ -28,7 +34,11 @@ int bt_gemm_qkv_bias_split(const void *, const int *, const void *, const void *
 int bt_gemm_qkv_bias_split_mask_rows(const void *, const void *, int, int, int, const void *, const void *, void *, int *, int *,
                                      int *, int, int, int, int, void *) { return 0; }
 int bt_attention_grouped(const void *, void *, const int *, const int *, const void *, const void *, int, int, int, int, int,
-                         float, int, const void *const *, const unsigned long long *, int, const int *, const void *, void *) { return 0; }
+                         float, int, const void *const *, const unsigned long long *, int, const int *slots, const void *list, void *) {
+  if (slots) take(slots, 256 * sizeof(int));
+  if (list) take(list, 16);
+  return 0;
+}
 int bt_mask_prefix_slots(const void *, int, int, int, const int *, int *, void *) { return 0; }
 int bt_add_bias_residual_layernorm(void *, const void *, const int *, const void *, const void *, const void *, int, const int *,
                                    int, int, float, void *) { return 0; }
@@ -37,8 +47,15 @@ int bt_add_bias_residual_layernorm_copy(void *, const void *, const int *, const
                                         const int *, void *) { return 0; }
 int bt_add_bias_residual_layernorm_restore(const void *, const void *, const void *, const void *, const void *, int, void *,
                                            const int *, const int *, int, int, int, float, void *) { return 0; }
-int bt_splitk_layernorm(const void *, int, const void *, const int *, const void *, const void *, const void *, int, void *,
-                        const int *, const int *, int, int, int, int, float, void *) { return 0; }
+int bt_splitk_layernorm(const void *sums, int splits, const void *residual, const int *, const void *, const void *, const void *,
+                        int, void *dst, const int *offsets, const int *live, int, int, int rows, int n, float, void *) {
+  partials = {(const char *)sums, (const char *)sums + 4ull * splits * rows * n};
+  take(residual, 2ull * rows * n);
+  take(dst, 2ull * rows * n);
+  if (offsets) take(offsets, 4);
+  if (live) take(live, 4);
+  return 0;
+}
 int bt_gemm(const void *, const void *, void *, const int *live, int, int, int n, int k, int, void *) {
   if (k > n) slices = 1;
   live_by_size += live == nullptr;
@@ -48,8 +65,10 @@ int bt_gemm_bias_gelu(const void *, const void *, const void *, void *, const in
   live_by_size += live == nullptr;
   return 0;
 }
-int bt_gemm_splitk_rows(const void *, const void *, void *, int splits, const int *live, int, int, int, int, int, void *) {
+int bt_gemm_splitk_rows(const void *a, const void *, void *, int splits, const int *live, int rows, int, int, int k, int, void *) {
   slices = splits;
+  take(a, 2ull * rows * k);
+  if (live) take(live, 4);
   live_by_size += live == nullptr;
   return 0;
 }
@@ -59,32 +78,37 @@ int bt_gemm_splitk_slices(int rows_cap, int all_live, int n, int k, int most) {
 }
 }
 
-// argv: layer|encoder  heads  batch  seq_len  live rows that the caller vouches for (-1: no offsets)
-int main(int, char **argv) {
+// argv: layer|encoder  heads  batch  seq_len  live rows that the caller vouches for (-1: no offsets, -2: padded rows)
+// [batch and seq_len that the scratch is for]
+int main(int argc, char **argv) {
   const int heads = std::atoi(argv[2]), batch = std::atoi(argv[3]), seq = std::atoi(argv[4]), live = std::atoi(argv[5]);
+  const int most = argc > 7 ? std::atoi(argv[6]) : batch, longest = argc > 7 ? std::atoi(argv[7]) : seq;
+  const bool packed = live != -2;
   static char some[4096];
   const __half *t = (const __half *)some;
   BertTransformerParam<OperationType::HALF> w;
   w.attention_param.attr_bias_QKV = t;
   w.attr_kernel_QKV = w.attr_output_kernel = w.inter_kernel = w.output_kernel = t;
   if (argv[1][0] == 'l') {
-    BertTransformer<OperationType::HALF> layer(batch, heads, 64, seq);
+    BertTransformer<OperationType::HALF> layer(most, heads, 64, longest, true, packed);
     layer.initialize(w);
-    layer.cal_bufsize();
+    scratch = {some, some + layer.cal_bufsize()};
     BertTransformerInferParam<__half> ip{t, t, (__half *)some, some, batch, seq, nullptr, nullptr};
     ET_Param offsets{(int *)some, (int *)some, live};
     if (live >= 0) ip.offsets = &offsets;
     layer.infer(ip);
   } else {
-    BertEncoder<OperationType::HALF> encoder(batch, heads, 64, seq);
+    BertEncoder<OperationType::HALF> encoder(most, heads, 64, longest, true, packed);
     encoder.initialize(std::vector<BertTransformerParam<OperationType::HALF>>(12, w));
-    encoder.cal_bufsize();
+    scratch = {some, some + encoder.cal_bufsize()};
     BertEncoderInferParam<__half> ip{};
     ip.input_tensor = ip.atten_mask = t, ip.transformer_output = (__half *)some, ip.buf = some;
     ip.batch_size = batch, ip.seq_len = seq;
     encoder.infer(ip);
   }
-  std::printf("%d %d %d\n", slices, live_by_size, asked);
+  bool apart = partials.begin == partials.end || (partials.begin >= scratch.begin && partials.end <= scratch.end);
+  for (const Span &o : others) apart = apart && (o.begin >= partials.end || o.end <= partials.begin);
+  std::printf("%d %d %d %d\n", slices, live_by_size, asked, apart);
 }
 """
 
@@ -112,7 +136,7 @@ def launches(tmp_path_factory):
 # one of 1050 gets 2, of 2400 three)
 @pytest.mark.parametrize("live,slices", [(32, 4), (900, 4), (1050, 4), (1500, 3), (2100, 2), (2400, 2), (3400, 1), (8192, 1)])
 def test_offsets_with_their_count(launches, live, slices):
-    got, live_by_size, _ = launches("layer", 12, 16, 512, live)
+    got, live_by_size, _, _ = launches("layer", 12, 16, 512, live)
     assert got == slices == _lib.kernel_lib().bt_gemm_splitk_slices(live, 1, 768, 3072, 16)
     assert live_by_size == 3
 
@@ -120,8 +144,8 @@ def test_offsets_with_their_count(launches, live, slices):
 @pytest.mark.parametrize("batch,seq_len", [(16, 512), (4, 96), (7, 217), (8, 300)])
 def test_offsets_without_their_count(launches, batch, seq_len):
     """A caller that does not know the count gets the slices of one that passes no offsets."""
-    own = launches("layer", 12, batch, seq_len, -1)
-    assert launches("layer", 12, batch, seq_len, 0) == own
+    own = launches("layer", 12, batch, seq_len, -1)[:3]
+    assert launches("layer", 12, batch, seq_len, 0)[:3] == own
     assert own[1] == 0
 
 
@@ -132,5 +156,21 @@ def test_padded_rows_are_all_live(launches):
 
 @pytest.mark.parametrize("batch,seq_len", [(1, 32), (4, 96), (16, 512)])
 def test_an_encoder_asks_once_for_its_slices(launches, batch, seq_len):
-    slices, _, asked = launches("encoder", 12, batch, seq_len, -1)
+    slices, _, asked, _ = launches("encoder", 12, batch, seq_len, -1)
     assert asked == 1 and slices == launches("layer", 12, batch, seq_len, -1)[0]
+
+
+@pytest.mark.parametrize("kind", ["layer", "encoder"])
+@pytest.mark.parametrize("heads", [8, 12, 16])
+def test_partial_sums_lie_apart(launches, kind, heads):
+    """FFN2's partial sums lie in the scratch and touch nothing that their LayerNorm reads or writes, nor what a later
+    layer reads again: sizes around those where the slices change, packed and padded rows, exact counts, scratch for
+    just these sizes and for more."""
+    seen = set()
+    for batch, seq_len in ((1, 1), (1, 32), (3, 33), (4, 96), (1, 700), (7, 217), (8, 250), (8, 300), (8, 313), (5, 640), (16, 512)):
+        for live in (-1, -2) + ((batch * seq_len, batch * seq_len * 3 // 5) if kind == "layer" else ()):
+            for room in ((), (batch + 1, seq_len), (2 * batch, seq_len + 100)):
+                slices, _, _, apart = launches(kind, heads, batch, seq_len, live, *room)
+                assert apart, (batch, seq_len, live, room, slices)
+                seen.add(slices)
+    assert len(seen) >= 3, seen
