@@ -411,8 +411,8 @@ __device__ __forceinline__ void regw_store(const RegW &w, half_t *sW) {
 // ---- a wave's share of a tile: products and stores ----------------------------------------
 // 16x16 blocks on v_mfma_f32_16x16x32_f16, the weight as its "A" operand: a lane's four sums of block
 // (i, j) are columns 16 i + 4 (lane >> 4) .. + 3 of row 16 j + (lane & 15).
-// The chip runs these loops against its power limit (1.45 - 1.8 GHz of 2.4 inside the products of a
-// forward), and this instruction does more with it than v_mfma_f32_32x32x16_f16: on operands in
+// The chip runs these loops against its power limit (1.8 to 2.1 GHz of 2.4 in forwards of some thousand
+// rows), and this instruction does more with it than v_mfma_f32_32x32x16_f16: on operands in
 // registers 1870 against 1600 TFLOP/s, with the loop's LDS reads 1585 against 1420 (8 waves, 64x128).
 // Products of a forward, with the reads placed by hand (`schedule`): FFN1 at 4800 rows 30.9 -> 29.5 us, at
 // 9830 rows 56.6 -> 53.6, FFN2 27.4 -> 24.6 and 46.9 -> 43.9, projection 11.1 -> 9.9.
@@ -1456,8 +1456,9 @@ struct TileModel {
   float shared_us;           // > 0: one k-step's share of a CU that several tiles occupy
 };
 
-// Fitted to the table's measurements: on average the choice is 1.2 % slower than the fastest
-// tile, and 7 % or more in one case of twenty.
+// Fitted to the table's measurements.  Both were taken of these tiles on 32x32x16 instructions, with stores that
+// stayed in the L2 and a workgroup for every tile of the capacity; the kernels have become 4 to 13 % faster since, not all
+// tiles alike, and how far the choice is from the fastest tile of today has not been measured.
 static const TileModel kTileModels[] = {
     {0, 256, 256, 1.45f, 5.7f, 0.f},     {13, 192, 192, 0.95f, 4.7f, 0.f},  {3, 256, 192, 1.10f, 4.35f, 0.f},
     {12, 128, 192, 0.64f, 4.6f, 0.f},    {2, 256, 128, 0.79f, 4.4f, 0.f},   {1, 128, 128, 0.467f, 3.4f, 0.f},

@@ -1,7 +1,9 @@
 // The one thing the PyTorch operator keeps between calls: the number of valid tokens of a
-// mask tensor.  It is a HINT: it picks tile shapes and weight layouts, never a launch size;
-// the offsets themselves are rebuilt from the mask on the device in every call, and the
-// weights are read as they are at the call.  A stale count costs time and nothing else.
+// mask tensor.  It is a HINT: it picks tile shapes and weight layouts, and how many workgroups
+// some products start with (each goes on to further rows where there are more); the offsets
+// themselves are rebuilt from the mask on the device in every call, and the weights are read as
+// they are at the call.  A stale count costs time, whole extra rounds of the chip where it is far
+// too low, and never a bit.
 //
 // The host never waits for it (the reference blocks on this very count in every call,
 // remove_padding.h:99-100): the first layer call that meets a mask tensor hands the layer a

@@ -18,7 +18,8 @@
  *     their grids for `rows_cap` rows and retire rows >= M on the device, so
  *     the host never waits for M.  NULL means all rows_cap rows are live.
  *   - `rows_hint` arguments are the host's estimate of M (0 = none); they only
- *     steer the choice of tile shape and never affect results.
+ *     steer the choice of tile shape and the number of workgroups, each of which
+ *     goes on to further rows where there are more, and never affect results.
  *
  * Each declaration cites the reference interface it replaces (paths relative
  * to the ByteTransformer tree).

@@ -29,7 +29,9 @@ struct BertEncoderInferParam {
   // all layers' pre-packed weights as written by BertEncoder::prepack, or null: the
   // products then read the weights as they are stored
   const void *prepacked = nullptr;
-  int valid_rows_hint = 0;             // expected number of valid tokens (0 = unknown); tile choice only
+  // expected number of valid tokens (0 = unknown): tile shapes and how many workgroups some
+  // products start with, never a result
+  int valid_rows_hint = 0;
 };
 
 template <OperationType OpType>

@@ -65,7 +65,8 @@ struct BertTransformerInferParam {
   // int[batch_size*seq_len], valid_word_num = their total).  When set, infer()
   // skips its own mask prefix sum.  valid_word_num must be the exact total (as the
   // reference's ET_Param carries it) or 0 when the host does not know it: a positive
-  // value sizes the launches over packed rows and picks their tile shapes.
+  // value sizes the launches over packed rows and picks their tile shapes and FFN2's k slices
+  // (so that the last bits may differ from a call that leaves it 0).
   const ET_Param *offsets = NULL;
   // ... and the matching sequence order (int[batch_size], longest first), or NULL.
   const int *seq_order = NULL;
@@ -75,8 +76,9 @@ struct BertTransformerInferParam {
   // zero; 0 = it is not; -1 = not checked (the layer then checks on the device).
   int mask_prefix = -1;
   // Extension: the number of valid tokens the caller expects (0 = unknown) when it passes
-  // no offsets.  A hint: it picks tile shapes and the split-k FFN2, never a launch size, so
-  // a wrong value costs time and nothing else.
+  // no offsets.  A hint: it picks tile shapes and copies, and how many workgroups some products
+  // start with (each goes on to further rows where there are more), so a wrong value costs
+  // time and never changes a bit; the k slices of FFN2 do not follow it.
   int valid_rows_hint = 0;
   // Extension: where the layer leaves the number of valid tokens it counted (padding-free
   // layers that build their own offsets), or NULL.  Memory the device can write and the host
