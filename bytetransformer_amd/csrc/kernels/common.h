@@ -10,6 +10,7 @@
 #include <cstdint>
 #include <initializer_list>
 #include <cstdio>
+#include <type_traits>
 
 #include "bt_hip.h"
 
@@ -114,10 +115,25 @@ inline int check_generic_attention(const char *who, const void *qkv, const void 
 }
 
 // ---- wave64 reductions ----------------------------------------------------
+// Sum over the 64 lanes, as a wave-uniform value, with data-parallel-primitive adds only (the steps of
+// wave_inclusive_sum): a step is a few clocks, where one through the LDS pipe takes over a hundred.
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+#if defined(__HIP_DEVICE_COMPILE__)
+  const auto moved = [](float x, auto ctrl, auto rows) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), decltype(ctrl)::value,
+                                                                 decltype(rows)::value, 0xf, true));
+  };
+  using all = std::integral_constant<int, 0xf>;
+  v += moved(v, std::integral_constant<int, 0x111>{}, all{});   // row_shr:1
+  v += moved(v, std::integral_constant<int, 0x112>{}, all{});   // row_shr:2
+  v += moved(v, std::integral_constant<int, 0x114>{}, all{});   // row_shr:4
+  v += moved(v, std::integral_constant<int, 0x118>{}, all{});   // row_shr:8
+  v += moved(v, std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{});   // row_bcast:15 -> rows 1, 3
+  v += moved(v, std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{});   // row_bcast:31 -> rows 2, 3
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
+#else
   return v;
+#endif
 }
 
 __device__ __forceinline__ float wave_max(float v) {
