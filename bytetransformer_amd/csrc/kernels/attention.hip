@@ -68,11 +68,6 @@ struct AttItem {
   int rank, head, qb;
   bool exists;
 };
-// x / d for any 32-bit x, where inverse = floor(2^32 / d)  (2^32 - 1 for d = 1)
-__device__ __forceinline__ unsigned divide(unsigned x, unsigned d, unsigned inverse) {
-  const unsigned q = (unsigned)((unsigned long long)x * inverse >> 32);   // the quotient or one less
-  return q + (x - q * d >= d ? 1u : 0u);
-}
 __device__ __forceinline__ AttItem att_item(const AttArgs &p) {
   AttItem it;
   const unsigned lin = workgroup_id();
@@ -153,16 +148,8 @@ __device__ __forceinline__ AttArgs att_args(BT_ATT_FIRST, const AttTail<KIND> &t
 struct AttTile {
   int b, head, qb, seq_start, seq_len;
 };
-// (scalar loads: nothing in these launches writes what they read.  With the work found in scalar registers
+// (Found by scalar loads.  With the work in scalar registers
 // 12 layers take, before -> after: 4 x 96 443 -> 437 us, 7 x 217 627 -> 620, 100 x 120 1696 -> 1677.)
-template <typename T>
-__device__ __forceinline__ T scalar_load(const T *from) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  return *(const __attribute__((address_space(4))) T *)from;
-#else
-  return *from;
-#endif
-}
 template <int BQ>
 __device__ __forceinline__ bool att_tile(const AttArgs &p, AttTile &t) {
   if (workgroup_id() >= p.warm.grid_work) return false;
@@ -781,9 +768,8 @@ __global__ __launch_bounds__(kAttThreads) void attention_short_kernel(AttArgs p)
 
 // Size of the 1-D grid for `nqb` query tiles per sequence; fills the mapping fields.
 static unsigned att_grid(AttArgs &a, int nqb, bool streaming = false) {
-  auto inverse = [](unsigned d) { return (unsigned)(d > 1 ? (1ull << 32) / d : 0xffffffffull); };
   a.nqb = nqb;
-  a.per_nqb = inverse(nqb), a.per_heads = inverse(a.heads);
+  a.per_nqb = inverse_of(nqb), a.per_heads = inverse_of(a.heads);
   a.xcd_map = option_attention_xcd_map();
   const unsigned pairs = (unsigned)a.B * a.heads;
   // The balanced list is the streaming kernel's, and pays from the third round of 32

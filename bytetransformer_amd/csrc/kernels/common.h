@@ -142,6 +142,23 @@ __device__ __forceinline__ float wave_max(float v) {
   return v;
 }
 
+// ---- wave-uniform values ----------------------------------------------------
+// x / d for any 32-bit x, where inverse = floor(2^32 / d)  (2^32 - 1 for d = 1)
+__device__ __forceinline__ unsigned divide(unsigned x, unsigned d, unsigned inverse) {
+  const unsigned q = (unsigned)((unsigned long long)x * inverse >> 32);   // the quotient or one less
+  return q + (x - q * d >= d ? 1u : 0u);
+}
+inline unsigned inverse_of(unsigned d) { return d > 1 ? (unsigned)((1ull << 32) / d) : 0xffffffffu; }
+// A load into scalar registers, of what nothing in this launch writes, at a wave-uniform address.
+template <typename T>
+__device__ __forceinline__ T scalar_load(const T *from) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return *(const __attribute__((address_space(4))) T *)from;
+#else
+  return *from;
+#endif
+}
+
 // Inclusive prefix sum across the 64 lanes of a wave.
 __device__ __forceinline__ int wave_inclusive_scan(int v, int lane) {
 #pragma unroll

@@ -12,22 +12,34 @@ namespace bt {
 
 constexpr int kLnRowsPerBlock = 4;   // 2, 8 and 16 rows per workgroup measured 0-20 % slower
 
+// V consecutive halfs of a row: what a lane loads, adds and stores at a time.
+template <int V>
+struct LnVec;
+template <>
+struct LnVec<8> {
+  typedef half8_t halfs;
+  typedef uint4_t bits;
+};
+template <>
+struct LnVec<4> {
+  typedef half4_t halfs;
+  typedef uint2_t bits;
+};
+
 // Statistics and store of one row held in registers (x = (a + r) + bias, two fp16-rounded adds).
-template <int NC, bool GB32, bool kAffineEarly, int NG>
-__device__ __forceinline__ void ln_finish(const half8_t (&av)[NC], const half8_t (&rv)[NC],
-                                          const half8_t (&bias_v)[NC], const half8_t (&gh)[NC],
-                                          const half8_t (&bh)[NC], const float4_t (&g32)[NG][2],
-                                          const float4_t (&b32)[NG][2], const void *gamma,
-                                          const void *beta, const int (&cc)[NC],
-                                          const bool (&live)[NC], half8_t *o, float inv_n,
-                                          float eps) {
-  float v[NC][8];
+template <int NC, int V, bool GB32, bool kAffineEarly, int NG, typename H = typename LnVec<V>::halfs>
+__device__ __forceinline__ void ln_finish(const H (&av)[NC], const H (&rv)[NC], const H (&bias_v)[NC],
+                                          const H (&gh)[NC], const H (&bh)[NC],
+                                          const float4_t (&g32)[NG][V / 4], const float4_t (&b32)[NG][V / 4],
+                                          const void *gamma, const void *beta, const int (&cc)[NC],
+                                          const bool (&live)[NC], half_t *o, float inv_n, float eps) {
+  float v[NC][V];
   float sum = 0.f;
 #pragma unroll
   for (int i = 0; i < NC; ++i) {
-    const half8_t x = (av[i] + rv[i]) + bias_v[i];  // two fp16-rounded adds
+    const H x = (av[i] + rv[i]) + bias_v[i];  // two fp16-rounded adds
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
+    for (int j = 0; j < V; ++j) {
       v[i][j] = live[i] ? (float)x[j] : 0.f;
       sum += v[i][j];
     }
@@ -37,7 +49,7 @@ __device__ __forceinline__ void ln_finish(const half8_t (&av)[NC], const half8_t
 #pragma unroll
   for (int i = 0; i < NC; ++i) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
+    for (int j = 0; j < V; ++j) {
       v[i][j] = live[i] ? v[i][j] - mean : 0.f;
       sq += v[i][j] * v[i][j];
     }
@@ -46,34 +58,26 @@ __device__ __forceinline__ void ln_finish(const half8_t (&av)[NC], const half8_t
 
 #pragma unroll
   for (int i = 0; i < NC; ++i) {
-    float g[8], bt_[8];
+    float g[V], bt_[V];
     if (GB32) {
-      float4_t g0, g1, b0, b1;
-      if (kAffineEarly) {
-        g0 = g32[i][0], g1 = g32[i][1], b0 = b32[i][0], b1 = b32[i][1];
-      } else {
-        const float4_t *gp = (const float4_t *)gamma + 2 * cc[i];
-        const float4_t *bp = (const float4_t *)beta + 2 * cc[i];
-        g0 = gp[0], g1 = gp[1], b0 = bp[0], b1 = bp[1];
-      }
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        g[j] = g0[j];
-        g[4 + j] = g1[j];
-        bt_[j] = b0[j];
-        bt_[4 + j] = b1[j];
+      for (int h = 0; h < V / 4; ++h) {
+        const float4_t gv = kAffineEarly ? g32[kAffineEarly ? i : 0][h] : ((const float4_t *)gamma)[V / 4 * cc[i] + h];
+        const float4_t bv = kAffineEarly ? b32[kAffineEarly ? i : 0][h] : ((const float4_t *)beta)[V / 4 * cc[i] + h];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) g[4 * h + j] = gv[j], bt_[4 * h + j] = bv[j];
       }
     } else {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
+      for (int j = 0; j < V; ++j) {
         g[j] = (float)gh[i][j];
         bt_[j] = (float)bh[i][j];
       }
     }
-    half8_t y;
+    H y;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) y[j] = (half_t)(v[i][j] * rstd * g[j] + bt_[j]);
-    if (live[i]) store_through(o + cc[i], __builtin_bit_cast(uint4_t, y));
+    for (int j = 0; j < V; ++j) y[j] = (half_t)(v[i][j] * rstd * g[j] + bt_[j]);
+    if (live[i]) store_through(o + cc[i] * V, __builtin_bit_cast(typename LnVec<V>::bits, y));
   }
 }
 
@@ -86,140 +90,148 @@ __device__ __forceinline__ void ln_finish(const half8_t (&av)[NC], const half8_t
 // index or the sequence offsets, and on packed rows the row of `src` itself) is requested
 // at the top in one batch, a lane past the end of the row loads the last chunk again
 // instead of branching, and the only dependent step left is the row(s) behind an index.
-template <int NC, bool RESTORE, bool GB32, int SPLITS>
+// The row is a wave's, so what finds it (count, offsets, index, addresses) is scalar.
+//
+// FULL: the row is exactly NC chunks of V halfs for each of the 64 lanes (hidden 768 as three of 4, 512 and 1024 as
+// one and two of 8), so no lane holds a chunk that does not count: 12 elements a lane at hidden 768 instead of 16
+// behind selects.  A launch of a few rows is the length of one wave.
+template <int NC, int V, bool FULL, bool RESTORE, bool GB32, int SPLITS>
 __device__ __forceinline__ void layernorm_block(
-    int block, const half8_t *src, const half8_t *__restrict__ residual,
-    const half8_t *__restrict__ bias, const void *__restrict__ gamma,
-    const void *__restrict__ beta, half8_t *dst, const int *__restrict__ idx,
+    int block, const half_t *src, const half_t *__restrict__ residual,
+    const half_t *__restrict__ bias, const void *__restrict__ gamma,
+    const void *__restrict__ beta, half_t *dst, const int *__restrict__ idx,
     const int *__restrict__ residual_row_index, int B, int S, int rows_cap, int split_rows,
-    int chunks, float inv_n, float eps) {
-  const int r = block * kLnRowsPerBlock + (threadIdx.x >> 6);
+    int hidden, float inv_n, float eps, unsigned per_s) {
+  typedef typename LnVec<V>::halfs vec_t;
+  typedef typename LnVec<V>::bits bits_t;
+  const int r = block * kLnRowsPerBlock + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (r >= rows_cap) return;
+  const int H = FULL ? NC * V * kWave : hidden, chunks = H / V;
   // fp32 gamma / beta of wide rows would not fit the registers next to the row: those
   // instantiations fetch them after the statistics, as before
-  constexpr bool kAffineEarly = !GB32 || NC <= 2;
+  constexpr bool kAffineEarly = !GB32 || NC * V <= 16;
 
   int cc[NC];        // this lane's chunks, clamped into the row
   bool live[NC];
 #pragma unroll
   for (int i = 0; i < NC; ++i) {
     const int c = lane + i * kWave;
-    live[i] = c < chunks;
+    live[i] = FULL || c < chunks;
     cc[i] = live[i] ? c : chunks - 1;
   }
 
   // ---- first batch: nothing here depends on loaded data ----
-  half8_t bias_v[NC];
-  half8_t gh[NC], bh[NC];
-  float4_t g32[kAffineEarly && GB32 ? NC : 1][2], b32[kAffineEarly && GB32 ? NC : 1][2];
+  vec_t bias_v[NC];
+  vec_t gh[NC], bh[NC];
+  float4_t g32[kAffineEarly && GB32 ? NC : 1][V / 4], b32[kAffineEarly && GB32 ? NC : 1][V / 4];
 #pragma unroll
   for (int i = 0; i < NC; ++i) {
-    bias_v[i] = bias[cc[i]];
+    bias_v[i] = ((const vec_t *)bias)[cc[i]];
     if (kAffineEarly) {
       if (GB32) {
-        g32[i][0] = ((const float4_t *)gamma)[2 * cc[i]];
-        g32[i][1] = ((const float4_t *)gamma)[2 * cc[i] + 1];
-        b32[i][0] = ((const float4_t *)beta)[2 * cc[i]];
-        b32[i][1] = ((const float4_t *)beta)[2 * cc[i] + 1];
+#pragma unroll
+        for (int h = 0; h < V / 4; ++h) {
+          g32[i][h] = ((const float4_t *)gamma)[V / 4 * cc[i] + h];
+          b32[i][h] = ((const float4_t *)beta)[V / 4 * cc[i] + h];
+        }
       } else {
-        gh[i] = ((const half8_t *)gamma)[cc[i]];
-        bh[i] = ((const half8_t *)beta)[cc[i]];
+        gh[i] = ((const vec_t *)gamma)[cc[i]];
+        bh[i] = ((const vec_t *)beta)[cc[i]];
       }
     }
   }
+  auto row_of = [&](const half_t *tensor, size_t row, int i) { return ((const vec_t *)(tensor + row * H))[cc[i]]; };
+  auto zero_row = [&](size_t row) {
+    const vec_t z = {};
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+      if (live[i]) store_through(dst + row * H + cc[i] * V, __builtin_bit_cast(bits_t, z));
+  };
 
-  size_t src_row, dst_row = r;
-  half8_t av[NC];
+  size_t src_row = r, dst_row = r;
+  vec_t av[NC], rv[NC];
   if (RESTORE && residual_row_index && SPLITS == 0) {
     // restore through the row map (word_idx of the offsets: entry r < M is the padded
     // position of packed row r, the entries from M on are the padded positions that stay
     // empty): only the store address depends on a loaded value, so the rows are requested
     // together with it.  idx = batch_idx, M = idx[B].
-    src_row = r;
 #pragma unroll
-    for (int i = 0; i < NC; ++i) av[i] = src[src_row * chunks + cc[i]];
-    half8_t rv0[NC];
+    for (int i = 0; i < NC; ++i) av[i] = row_of(src, src_row, i);
 #pragma unroll
-    for (int i = 0; i < NC; ++i) rv0[i] = residual[src_row * chunks + cc[i]];
-    dst_row = (size_t)residual_row_index[r];
-    const int M = idx[B];
-    if (r >= M) {
-      const half8_t z = {0, 0, 0, 0, 0, 0, 0, 0};
-      for (int c = lane; c < chunks; c += kWave) store_through(dst + dst_row * chunks + c, __builtin_bit_cast(uint4_t, z));
-      return;
-    }
-    ln_finish<NC, GB32, kAffineEarly>(av, rv0, bias_v, gh, bh, g32, b32, gamma, beta, cc, live,
-                                      dst + dst_row * chunks, inv_n, eps);
+    for (int i = 0; i < NC; ++i) rv[i] = row_of(residual, src_row, i);
+    dst_row = (size_t)scalar_load(residual_row_index + r);
+    const int M = scalar_load(idx + B);
+    if (r >= M) return zero_row(dst_row);
+    ln_finish<NC, V, GB32, kAffineEarly>(av, rv, bias_v, gh, bh, g32, b32, gamma, beta, cc, live,
+                                         dst + dst_row * H, inv_n, eps);
     return;
   }
+  size_t res_row;
   if (RESTORE) {
     // r walks the padded [B, S] grid; idx = batch_idx
-    const int b = r / S, s = r - b * S;
-    const int start = idx[b], len = idx[b + 1] - start;
-    if (s >= len) {
-      const half8_t z = {0, 0, 0, 0, 0, 0, 0, 0};
-      for (int c = lane; c < chunks; c += kWave) store_through(dst + dst_row * chunks + c, __builtin_bit_cast(uint4_t, z));
-      return;
-    }
-    src_row = (size_t)start + s;
+    const int b = (int)divide((unsigned)r, (unsigned)S, per_s), s = r - b * S;
+    const int start = scalar_load(idx + b), len = scalar_load(idx + b + 1) - start;
+    if (s >= len) return zero_row(dst_row);
+    res_row = src_row = (size_t)start + s;
   } else {
     // idx = pointer to the live-row count (or null: all rows live): one scalar load, the same
     // address for every wave of the launch, and the one thing a wave waits for before it asks
     // for its rows - the waves of the rows past the count (40 % of a launch sized for the
     // padded batch) would otherwise read 1.5 KB each for nothing.
-    src_row = r;
-    const int M = idx ? *idx : rows_cap;
+    const int M = idx ? scalar_load(idx) : rows_cap;
     if (r >= M) return;
-    if (SPLITS == 0) {
-#pragma unroll
-      for (int i = 0; i < NC; ++i) av[i] = src[src_row * chunks + cc[i]];
-    }
-    const size_t res_row = residual_row_index ? (size_t)residual_row_index[src_row] : src_row;
-    residual += res_row * chunks;
+    res_row = residual_row_index ? (size_t)scalar_load(residual_row_index + src_row) : src_row;
   }
-  if (RESTORE) {
-    residual += src_row * chunks;
-    if (SPLITS == 0) {
+  if (SPLITS == 0) {
 #pragma unroll
-      for (int i = 0; i < NC; ++i) av[i] = src[src_row * chunks + cc[i]];
-    }
+    for (int i = 0; i < NC; ++i) av[i] = row_of(src, src_row, i);
   }
-  half8_t rv[NC];
 #pragma unroll
-  for (int i = 0; i < NC; ++i) rv[i] = residual[cc[i]];
+  for (int i = 0; i < NC; ++i) rv[i] = row_of(residual, res_row, i);
   if (SPLITS > 0) {
 #pragma unroll
-    for (int i = 0; i < NC; ++i) {
-      const float4_t *pp = (const float4_t *)src + (src_row * chunks + cc[i]) * 2;
-      float4_t lo = pp[0], hi = pp[1];
+    for (int i = 0; i < NC; ++i)
 #pragma unroll
-      for (int sp = 1; sp < SPLITS; ++sp) {
-        lo += pp[(size_t)sp * split_rows * chunks * 2];
-        hi += pp[(size_t)sp * split_rows * chunks * 2 + 1];
-      }
+      for (int h = 0; h < V / 4; ++h) {
+        const float4_t *pp = (const float4_t *)((const float *)src + src_row * H) + V / 4 * cc[i] + h;
+        float4_t part = pp[0];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        av[i][j] = (half_t)lo[j];
-        av[i][4 + j] = (half_t)hi[j];
+        for (int sp = 1; sp < SPLITS; ++sp) part += pp[(size_t)sp * split_rows * (H / 4)];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) av[i][4 * h + j] = (half_t)part[j];
       }
-    }
   }
 
-  ln_finish<NC, GB32, kAffineEarly>(av, rv, bias_v, gh, bh, g32, b32, gamma, beta, cc, live,
-                                    dst + dst_row * chunks, inv_n, eps);
+  ln_finish<NC, V, GB32, kAffineEarly>(av, rv, bias_v, gh, bh, g32, b32, gamma, beta, cc, live,
+                                       dst + dst_row * H, inv_n, eps);
 }
 
-template <int NC, bool RESTORE, bool GB32, int SPLITS>
+template <int NC, int V, bool FULL, bool RESTORE, bool GB32, int SPLITS>
 __global__ __launch_bounds__(kLnRowsPerBlock *kWave) void layernorm_kernel(
-    const half8_t *src, const half8_t *__restrict__ residual,
-    const half8_t *__restrict__ bias, const void *__restrict__ gamma,
-    const void *__restrict__ beta, half8_t *dst, const int *__restrict__ idx,
+    const half_t *src, const half_t *__restrict__ residual,
+    const half_t *__restrict__ bias, const void *__restrict__ gamma,
+    const void *__restrict__ beta, half_t *dst, const int *__restrict__ idx,
     const int *__restrict__ residual_row_index, int B, int S, int rows_cap, int split_rows,
-    int chunks, float inv_n, float eps) {
-  layernorm_block<NC, RESTORE, GB32, SPLITS>(blockIdx.x, src, residual, bias, gamma, beta, dst, idx,
-                                             residual_row_index, B, S, rows_cap, split_rows, chunks,
-                                             inv_n, eps);
+    int hidden, float inv_n, float eps, unsigned per_s) {
+  layernorm_block<NC, V, FULL, RESTORE, GB32, SPLITS>(blockIdx.x, src, residual, bias, gamma, beta, dst, idx,
+                                                      residual_row_index, B, S, rows_cap, split_rows, hidden,
+                                                      inv_n, eps, per_s);
+}
+
+// Calls `launch` with the way that rows of H halfs are dealt to a wave as compile-time constants.
+template <typename Launch>
+static void by_row_shape(int H, Launch launch) {
+  const auto with = [&](auto nc, auto v, auto full) { launch(nc, v, full); };
+  using std::integral_constant;
+  if (H == 768) return with(integral_constant<int, 3>{}, integral_constant<int, 4>{}, std::true_type{});
+  if (H == 512) return with(integral_constant<int, 1>{}, integral_constant<int, 8>{}, std::true_type{});
+  if (H == 1024) return with(integral_constant<int, 2>{}, integral_constant<int, 8>{}, std::true_type{});
+  const int nc = (H / 8 + kWave - 1) / kWave;
+  if (nc <= 1) return with(integral_constant<int, 1>{}, integral_constant<int, 8>{}, std::false_type{});
+  if (nc <= 2) return with(integral_constant<int, 2>{}, integral_constant<int, 8>{}, std::false_type{});
+  if (nc <= 4) return with(integral_constant<int, 4>{}, integral_constant<int, 8>{}, std::false_type{});
+  with(integral_constant<int, 8>{}, integral_constant<int, 8>{}, std::false_type{});
 }
 
 // The packed LayerNorm with k-contiguous weight copies riding along: the first `copy_blocks`
@@ -228,12 +240,12 @@ __global__ __launch_bounds__(kLnRowsPerBlock *kWave) void layernorm_kernel(
 // A launch of a few thousand rows moves its 20 MB at half of what the memory system
 // sustains, so the copy of a few MB costs this launch less than a launch of its own would,
 // and the product behind it (FFN1) reads its weight k-contiguous.
-template <int NC, bool GB32>
+template <int NC, int V, bool FULL, bool GB32>
 __global__ __launch_bounds__(kLnRowsPerBlock *kWave) void layernorm_copy_kernel(
-    const half8_t *src, const half8_t *__restrict__ residual,
-    const half8_t *__restrict__ bias, const void *__restrict__ gamma,
-    const void *__restrict__ beta, half8_t *dst, const int *__restrict__ idx,
-    const int *__restrict__ residual_row_index, int rows_cap, int chunks, float inv_n, float eps,
+    const half_t *src, const half_t *__restrict__ residual,
+    const half_t *__restrict__ bias, const void *__restrict__ gamma,
+    const void *__restrict__ beta, half_t *dst, const int *__restrict__ idx,
+    const int *__restrict__ residual_row_index, int rows_cap, int hidden, float inv_n, float eps,
     WeightJobs jobs, int copy_blocks) {
   static_assert(kLnRowsPerBlock * kWave == 256, "a tile is moved by 256 threads");
   if ((int)blockIdx.x < copy_blocks) {
@@ -243,9 +255,9 @@ __global__ __launch_bounds__(kLnRowsPerBlock *kWave) void layernorm_copy_kernel(
       transpose_tiles_64<1>(jobs, t0, tiles, threadIdx.x);
     return;
   }
-  layernorm_block<NC, false, GB32, 0>((int)blockIdx.x - copy_blocks, src, residual, bias, gamma,
-                                      beta, dst, idx, residual_row_index, 0, 1, rows_cap, rows_cap,
-                                      chunks, inv_n, eps);
+  layernorm_block<NC, V, FULL, false, GB32, 0>((int)blockIdx.x - copy_blocks, src, residual, bias, gamma,
+                                               beta, dst, idx, residual_row_index, 0, 1, rows_cap, rows_cap,
+                                               hidden, inv_n, eps, 0);
 }
 
 template <bool RESTORE, int SPLITS = 0>
@@ -257,34 +269,18 @@ static int launch_ln(const void *src, const void *residual, const void *bias, co
              who, H);
   BT_REQUIRE(aligned16({src, residual, bias, gamma, beta, dst}), BT_ERR_INVALID_ARGUMENT,
              "%s: tensor pointers must be 16-byte aligned", who);
-  const int chunks = H / 8;
-  const int nc = (chunks + kWave - 1) / kWave;
-  BT_REQUIRE(nc <= 8, BT_ERR_UNSUPPORTED, "%s: hidden_dim %d exceeds 4096", who, H);
+  BT_REQUIRE(H <= 8 * 8 * kWave, BT_ERR_UNSUPPORTED, "%s: hidden_dim %d exceeds 4096", who, H);
   if (rows_cap == 0) return BT_OK;
   const int grid = (rows_cap + kLnRowsPerBlock - 1) / kLnRowsPerBlock;
   const float inv_n = 1.0f / (float)H;
-#define BT_LN_LAUNCH(NC_, GB_)                                                                  \
-  layernorm_kernel<NC_, RESTORE, GB_, SPLITS><<<grid, kLnRowsPerBlock * kWave, 0, s>>>(         \
-      (const half8_t *)src, (const half8_t *)residual, (const half8_t *)bias, gamma, beta,      \
-      (half8_t *)dst, idx, residual_row_index, B, S, rows_cap, split_rows ? split_rows : rows_cap, \
-      chunks, inv_n, eps)
-#define BT_LN_NC(NC_)              \
-  do {                             \
-    if (gb32)                      \
-      BT_LN_LAUNCH(NC_, true);     \
-    else                           \
-      BT_LN_LAUNCH(NC_, false);    \
-  } while (0)
-  if (nc <= 1)
-    BT_LN_NC(1);
-  else if (nc <= 2)
-    BT_LN_NC(2);
-  else if (nc <= 4)
-    BT_LN_NC(4);
-  else
-    BT_LN_NC(8);
-#undef BT_LN_NC
-#undef BT_LN_LAUNCH
+  by_row_shape(H, [&](auto nc, auto v, auto full) {
+    const auto kernel = gb32 ? layernorm_kernel<nc(), v(), full(), RESTORE, true, SPLITS>
+                             : layernorm_kernel<nc(), v(), full(), RESTORE, false, SPLITS>;
+    kernel<<<grid, kLnRowsPerBlock * kWave, 0, s>>>((const half_t *)src, (const half_t *)residual, (const half_t *)bias,
+                                                    gamma, beta, (half_t *)dst, idx, residual_row_index, B, S,
+                                                    rows_cap, split_rows ? split_rows : rows_cap, H, inv_n, eps,
+                                                    inverse_of((unsigned)S));
+  });
   BT_CHECK_LAUNCH(who);
   return BT_OK;
 }
@@ -333,37 +329,20 @@ extern "C" int bt_add_bias_residual_layernorm_copy(
              who, H);
   BT_REQUIRE(aligned16({out, residual, bias, gamma, beta}), BT_ERR_INVALID_ARGUMENT,
              "%s: tensor pointers must be 16-byte aligned", who);
-  const int chunks = H / 8;
-  const int nc = (chunks + kWave - 1) / kWave;
-  BT_REQUIRE(nc <= 8, BT_ERR_UNSUPPORTED, "%s: hidden_dim %d exceeds 4096", who, H);
+  BT_REQUIRE(H <= 8 * 8 * kWave, BT_ERR_UNSUPPORTED, "%s: hidden_dim %d exceeds 4096", who, H);
   // one tile per copying workgroup up to 1024 of them (a BERT-large FFN weight has 1024 tiles)
   const int tiles = jobs.tile_end[jobs.count - 1];
   const int copy_blocks = tiles < 1024 ? tiles : 1024;
   const int grid = copy_blocks + (rows_cap + kLnRowsPerBlock - 1) / kLnRowsPerBlock;
   const float inv_n = 1.0f / (float)H;
   hipStream_t s = as_stream(stream);
-#define BT_LN_LAUNCH(NC_, GB_)                                                                  \
-  layernorm_copy_kernel<NC_, GB_><<<grid, kLnRowsPerBlock * kWave, 0, s>>>(                     \
-      (const half8_t *)out, (const half8_t *)residual, (const half8_t *)bias, gamma, beta,      \
-      (half8_t *)out, valid_rows, residual_row_index, rows_cap, chunks, inv_n, eps, jobs,       \
-      copy_blocks)
-#define BT_LN_NC(NC_)              \
-  do {                             \
-    if (gamma_beta_fp32)           \
-      BT_LN_LAUNCH(NC_, true);     \
-    else                           \
-      BT_LN_LAUNCH(NC_, false);    \
-  } while (0)
-  if (nc <= 1)
-    BT_LN_NC(1);
-  else if (nc <= 2)
-    BT_LN_NC(2);
-  else if (nc <= 4)
-    BT_LN_NC(4);
-  else
-    BT_LN_NC(8);
-#undef BT_LN_NC
-#undef BT_LN_LAUNCH
+  by_row_shape(H, [&](auto nc, auto v, auto full) {
+    const auto kernel = gamma_beta_fp32 ? layernorm_copy_kernel<nc(), v(), full(), true>
+                                        : layernorm_copy_kernel<nc(), v(), full(), false>;
+    kernel<<<grid, kLnRowsPerBlock * kWave, 0, s>>>((const half_t *)out, (const half_t *)residual, (const half_t *)bias,
+                                                    gamma, beta, (half_t *)out, valid_rows, residual_row_index,
+                                                    rows_cap, H, inv_n, eps, jobs, copy_blocks);
+  });
   BT_CHECK_LAUNCH(who);
   return BT_OK;
 }

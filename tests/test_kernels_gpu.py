@@ -248,6 +248,36 @@ def test_add_bias_residual_layernorm(device, H, gb32):
     assert np.all(err <= 2.0 ** -10 * np.abs(exp) + 1e-4)
 
 
+@pytest.mark.parametrize("gb32", [False, True])
+@pytest.mark.parametrize("H", [504, 512, 520, 760, 768, 776, 1016, 1024, 1032])
+def test_layernorm_rows_that_just_fill_the_lanes(device, H, gb32):
+    """Hidden sizes that deal every lane of a wave the same whole chunks, and the sizes around them: the packed form and
+    the restore of partial sums, whose rows find their sequence by a multiplication."""
+    _say("layernorm lanes", H, gb32)
+    rs = np.random.RandomState(H + gb32)
+    lens = [5, 0, 7, 1, 6]
+    B, S, M = len(lens), 7, sum(lens)
+    parts = rs.standard_normal((2, M, H)).astype(np.float32)
+    res = (rs.standard_normal((M, H)) * 2).astype(np.float16)
+    bias = (rs.standard_normal(H) * 0.5).astype(np.float16)
+    gdt = np.float32 if gb32 else np.float16
+    gamma, beta = (1 + 0.2 * rs.standard_normal(H)).astype(gdt), (0.3 * rs.standard_normal(H)).astype(gdt)
+    out = (parts[0] + parts[1]).astype(np.float16)
+    exp = O.add_bias_residual_layernorm(out, res, bias, gamma, beta, 1e-6)
+    args = [_dev(a, device) for a in (res, bias, gamma, beta)]
+    packed = ops.add_bias_residual_layernorm(_dev(out, device), *args, 1e-6).cpu().numpy()
+    bi = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    full = torch.full((B * S, H), float("nan"), dtype=torch.float16, device=device)
+    full = ops.splitk_layernorm(_dev(parts, device), *args, full, batch_idx=_dev(bi, device), batch_size=B, seq_len=S)
+    full = full.cpu().numpy().reshape(B, S, H)
+    # half an ulp of the fp16 result (2^-11) twice over, and the noise of the float statistics
+    for got in (packed, np.concatenate([full[b, :n] for b, n in enumerate(lens)])):
+        err = np.abs(got.astype(np.float64) - exp)
+        assert np.all(err <= 2.0 ** -10 * np.abs(exp) + 1e-4), err.max()
+    for b, n in enumerate(lens):
+        assert not full[b, n:].any()
+
+
 @pytest.mark.parametrize("H,gb32,rows,M", [(768, False, 300, 211), (1024, True, 37, 37),
                                            (64, False, 5, 0), (2048, False, 130, 129)])
 def test_layernorm_with_weight_copies_riding_along(device, H, gb32, rows, M):
