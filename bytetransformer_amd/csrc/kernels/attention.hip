@@ -804,14 +804,8 @@ static int check_att_args(const char *who, const void *qkv, const void *out, con
 template <int NKB, int KIND>
 static int launch_short_impl(const AttArgs &a, hipStream_t s) {
   constexpr size_t smem = (size_t)2 * NKB * 16 * kHeadDim * sizeof(half_t);
-  static_assert(smem <= 160 * 1024, "LDS budget");
-  static std::atomic<bool> configured[kMaxDevices];
-  const int rc = allow_dynamic_lds(attention_short_kernel<NKB, KIND>, smem, configured,
-                                   "hipFuncSetAttribute(attention_short_kernel)");
-  if (rc != BT_OK) return rc;
-  attention_short_kernel<NKB, KIND><<<a.nqb_grid, kAttThreads, smem, s>>>(a);
-  BT_CHECK_LAUNCH("attention_short_kernel");
-  return BT_OK;
+  static_assert(smem <= kMostLds, "LDS budget");
+  return Launch<attention_short_kernel<NKB, KIND>>::on(s, "attention_short_kernel", a.nqb_grid, kAttThreads, smem, a);
 }
 
 template <int NKB>
@@ -897,7 +891,7 @@ static GroupedPlan plan_grouped(AttArgs &a, int batch_size, int seq_len, int hea
   return plan;
 }
 template <int KIND>
-static void launch_grouped(const AttArgs &a, const GroupedPlan &plan, int seq_len, unsigned grid, hipStream_t s) {
+static int launch_grouped(const AttArgs &a, const GroupedPlan &plan, int seq_len, unsigned grid, hipStream_t s) {
   // (the additive terms alternate between two register sets, so their kernels take an even ring)
   constexpr int kWideStages = KIND == kAddNone ? 3 : 2;
   // eight waves over two key halves: pays for a few long sequences that leave most CUs
@@ -907,14 +901,14 @@ static void launch_grouped(const AttArgs &a, const GroupedPlan &plan, int seq_le
   const int ks = option_attention_key_split();
   const AttFirst f = att_first(a);
   const AttTail<KIND> t = att_tail<KIND>(a);
+  const char *who = "attention_grouped_kernel";
   if (plan.narrow)
-    attention_grouped_kernel<1, KIND, 1, 4, 1><<<grid, kAttThreads, 0, s>>>(BT_ATT_FIRST_OF(f), t);
-  else if (plan.wide)
-    attention_grouped_kernel<2, KIND, kWideStages><<<grid, kAttThreads, 0, s>>>(BT_ATT_FIRST_OF(f), t);
-  else if (ks == 1 || (ks < 0 && seq_len >= 512 && a.warm.grid_work <= 256))
-    attention_grouped_kernel<1, KIND, 2, 2><<<grid, 2 * kAttThreads, 0, s>>>(BT_ATT_FIRST_OF(f), t);
-  else
-    attention_grouped_kernel<1, KIND, 2><<<grid, kAttThreads, 0, s>>>(BT_ATT_FIRST_OF(f), t);
+    return Launch<attention_grouped_kernel<1, KIND, 1, 4, 1>>::on(s, who, grid, kAttThreads, 0, BT_ATT_FIRST_OF(f), t);
+  if (plan.wide)
+    return Launch<attention_grouped_kernel<2, KIND, kWideStages, 1, 4>>::on(s, who, grid, kAttThreads, 0, BT_ATT_FIRST_OF(f), t);
+  if (ks == 1 || (ks < 0 && seq_len >= 512 && a.warm.grid_work <= 256))
+    return Launch<attention_grouped_kernel<1, KIND, 2, 2, 4>>::on(s, who, grid, 2 * kAttThreads, 0, BT_ATT_FIRST_OF(f), t);
+  return Launch<attention_grouped_kernel<1, KIND, 2, 1, 4>>::on(s, who, grid, kAttThreads, 0, BT_ATT_FIRST_OF(f), t);
 }
 AttListPlan att_worklist_plan(int B, int S, int heads) {
   AttListPlan out{0, 64, 0};
@@ -998,12 +992,10 @@ extern "C" int bt_attention_grouped(const void *qkv_heads, void *attention_outpu
   rc = plan_warm_duty("bt_attention_grouped", a.warm, grid, prefetch, prefetch_bytes, prefetch_count);
   if (rc) return rc;
   switch (add_kind(a.mask, a.bias, a.scale_log2e)) {
-    case kAddNone: launch_grouped<kAddNone>(a, plan, seq_len, grid, s); break;
-    case kAddMask: launch_grouped<kAddMask>(a, plan, seq_len, grid, s); break;
-    case kAddBias: launch_grouped<kAddBias>(a, plan, seq_len, grid, s); break;
-    case kAddZero: launch_grouped<kAddZero>(a, plan, seq_len, grid, s); break;
-    default: launch_grouped<kAddBoth>(a, plan, seq_len, grid, s); break;
+    case kAddNone: return launch_grouped<kAddNone>(a, plan, seq_len, grid, s);
+    case kAddMask: return launch_grouped<kAddMask>(a, plan, seq_len, grid, s);
+    case kAddBias: return launch_grouped<kAddBias>(a, plan, seq_len, grid, s);
+    case kAddZero: return launch_grouped<kAddZero>(a, plan, seq_len, grid, s);
+    default: return launch_grouped<kAddBoth>(a, plan, seq_len, grid, s);
   }
-  BT_CHECK_LAUNCH("attention_grouped_kernel");
-  return BT_OK;
 }

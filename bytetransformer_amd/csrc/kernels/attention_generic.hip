@@ -338,23 +338,20 @@ __global__ __launch_bounds__(kGenThreads, 2) void attention_generic_kernel(Gener
 }
 
 template <int ND, int KIND>
-void launch_generic_kind(const GenericAttArgs &p, bool wide, unsigned grid, hipStream_t s) {
-  if constexpr (ND < 4 || KIND == kAddNone) {
-    if (wide) {
-      attention_generic_kernel<ND, KIND, 2><<<grid, kGenThreads, 0, s>>>(p);
-      return;
-    }
-  }
-  attention_generic_kernel<ND, KIND, 1><<<grid, kGenThreads, 0, s>>>(p);
+int launch_generic_kind(const GenericAttArgs &p, bool wide, unsigned grid, hipStream_t s) {
+  const char *who = "attention_generic_kernel";
+  if constexpr (ND < 4 || KIND == kAddNone)
+    if (wide) return Launch<attention_generic_kernel<ND, KIND, 2>>::on(s, who, grid, kGenThreads, 0, p);
+  return Launch<attention_generic_kernel<ND, KIND, 1>>::on(s, who, grid, kGenThreads, 0, p);
 }
 template <int ND>
-void launch_generic(const GenericAttArgs &p, int kind, bool wide, unsigned grid, hipStream_t s) {
+int launch_generic(const GenericAttArgs &p, int kind, bool wide, unsigned grid, hipStream_t s) {
   switch (kind) {
-    case kAddNone: launch_generic_kind<ND, kAddNone>(p, wide, grid, s); break;
-    case kAddMask: launch_generic_kind<ND, kAddMask>(p, wide, grid, s); break;
-    case kAddBias: launch_generic_kind<ND, kAddBias>(p, wide, grid, s); break;
-    case kAddZero: launch_generic_kind<ND, kAddZero>(p, wide, grid, s); break;
-    default: launch_generic_kind<ND, kAddBoth>(p, wide, grid, s); break;
+    case kAddNone: return launch_generic_kind<ND, kAddNone>(p, wide, grid, s);
+    case kAddMask: return launch_generic_kind<ND, kAddMask>(p, wide, grid, s);
+    case kAddBias: return launch_generic_kind<ND, kAddBias>(p, wide, grid, s);
+    case kAddZero: return launch_generic_kind<ND, kAddZero>(p, wide, grid, s);
+    default: return launch_generic_kind<ND, kAddBoth>(p, wide, grid, s);
   }
 }
 
@@ -397,13 +394,11 @@ extern "C" int bt_attention_generic_f16_warm(const void *qkv, void *out, const i
   if (rc != BT_OK) return rc;
   hipStream_t s = as_stream(stream);
   switch ((size_per_head + 31) / 32) {
-    case 1: launch_generic<1>(p, kind, wide, grid, s); break;
-    case 2: launch_generic<2>(p, kind, wide, grid, s); break;
-    case 3: launch_generic<3>(p, kind, wide, grid, s); break;
-    default: launch_generic<4>(p, kind, wide, grid, s); break;
+    case 1: return launch_generic<1>(p, kind, wide, grid, s);
+    case 2: return launch_generic<2>(p, kind, wide, grid, s);
+    case 3: return launch_generic<3>(p, kind, wide, grid, s);
+    default: return launch_generic<4>(p, kind, wide, grid, s);
   }
-  BT_CHECK_LAUNCH(who);
-  return BT_OK;
 }
 
 extern "C" int bt_attention_generic_f16(const void *qkv, void *out, const int *batch_idx,

@@ -47,31 +47,65 @@ int hip_fail(hipError_t e, const char *what);
       return ::bt::hip_fail(e__, what);           \
   } while (0)
 
-// ---- tuning options (bt_set_option) ----------------------------------------
-// Once-per-device set-up of a kernel's dynamic LDS limit (the attribute belongs to the
-// function on one device).  `done` is the kernel's own flag array; a lost race only
-// repeats an idempotent call.
+// ---- launches ---------------------------------------------------------------
+// A launch through the kernel's function handle, its arguments packed here.  Issuing a launch is what the host
+// does all day (12 layers at 1 x 32 are 84 of them, and take the GPU no longer than the host), and as <<<>>> with
+// a parameter each it looks the symbol up and copies argument by argument: us to issue an empty kernel of one / ten /
+// sixteen arguments 2.9 / 3.2 / 3.6 as <<<>>>, 2.7 / 2.95 / 3.2 so; 68 bytes of arguments 3.8 and 3.5, so no kernel
+// ends a few bytes behind a multiple of 16 beyond 64.
+// The handle, and the dynamic LDS limit beyond 64 KB, belong to the kernel on one device: they are looked up once
+// for each (a lost race only repeats an idempotent call).
 constexpr int kMaxDevices = 64;
-template <typename Kernel>
-inline int allow_dynamic_lds(Kernel kernel, size_t bytes, std::atomic<bool> (&done)[kMaxDevices],
-                             const char *what) {
-  int dev = 0;
-  hipError_t e = hipGetDevice(&dev);
-  if (e != hipSuccess) return hip_fail(e, "hipGetDevice");
-  if (dev < 0 || dev >= kMaxDevices) {
-    e = hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)bytes);
+constexpr size_t kMostLds = 160 * 1024;
+template <auto Kernel>
+struct Launch;
+template <typename... P, void (*Kernel)(P...)>
+struct Launch<Kernel> {
+  // 0 or a BT status
+  static int on(hipStream_t s, const char *what, unsigned grid, unsigned threads, size_t lds, P... args) {
+    hipFunction_t f = nullptr;
+    int rc = function(&f, what, lds > 64 * 1024);
+    if (rc != BT_OK) return rc;
+    alignas(16) unsigned char packed[kBytes];
+    size_t at = 0;
+    (pack(packed, at, args), ...);
+    size_t bytes = kBytes;
+    void *config[] = {HIP_LAUNCH_PARAM_BUFFER_POINTER, packed, HIP_LAUNCH_PARAM_BUFFER_SIZE, &bytes, HIP_LAUNCH_PARAM_END};
+    const hipError_t e = hipModuleLaunchKernel(f, grid, 1, 1, threads, 1, 1, (unsigned)lds, s, nullptr, config);
     return e == hipSuccess ? BT_OK : hip_fail(e, what);
   }
-  if (!done[dev].load(std::memory_order_acquire)) {
-    e = hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)bytes);
-    if (e != hipSuccess) return hip_fail(e, what);
-    done[dev].store(true, std::memory_order_release);
-  }
-  return BT_OK;
-}
 
+ private:
+  // (every argument at the next multiple of its alignment, as the kernel's argument segment lies)
+  static constexpr size_t total() {
+    size_t at = 0;
+    ((at = (at + alignof(P) - 1) / alignof(P) * alignof(P) + sizeof(P)), ...);
+    return at;
+  }
+  static constexpr size_t kBytes = total();
+  template <typename T>
+  static void pack(unsigned char *to, size_t &at, const T &v) {
+    at = (at + alignof(T) - 1) / alignof(T) * alignof(T);
+    __builtin_memcpy(to + at, &v, sizeof(T));
+    at += sizeof(T);
+  }
+  static int function(hipFunction_t *f, const char *what, bool large_lds) {
+    static std::atomic<hipFunction_t> known[kMaxDevices];
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return hip_fail(e, "hipGetDevice");
+    const bool kept = dev >= 0 && dev < kMaxDevices;
+    if (kept && (*f = known[dev].load(std::memory_order_acquire))) return BT_OK;
+    if (large_lds &&
+        (e = hipFuncSetAttribute((const void *)Kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMostLds)) != hipSuccess)
+      return hip_fail(e, what);
+    if ((e = hipGetFuncBySymbol(f, (const void *)Kernel)) != hipSuccess) return hip_fail(e, what);
+    if (kept) known[dev].store(*f, std::memory_order_release);
+    return BT_OK;
+  }
+};
+
+// ---- tuning options (bt_set_option) ----------------------------------------
 int option_gemm_tile();      // -1 = heuristic, else index into the tile table
 int option_gemm_table_margin();   // per cent by which a measured tile must beat the model's choice
 int option_layer_prepack();  // -1 = by the measured table, 0 = never, 1 = always
@@ -149,6 +183,12 @@ __device__ __forceinline__ unsigned divide(unsigned x, unsigned d, unsigned inve
   return q + (x - q * d >= d ? 1u : 0u);
 }
 inline unsigned inverse_of(unsigned d) { return d > 1 ? (unsigned)((1ull << 32) / d) : 0xffffffffu; }
+// x / d for wave-uniform 0 <= x < 2^21 and 0 < d, neither known to the host: a quarter of the instructions of a division.
+__device__ __forceinline__ int divide_small(int x, int d) {
+  int q = __builtin_amdgcn_readfirstlane((int)((float)x * __builtin_amdgcn_rcpf((float)d)));   // the quotient, one more or one less
+  q -= q * d > x ? 1 : 0;
+  return q + (x - q * d >= d ? 1 : 0);
+}
 // A load into scalar registers, of what nothing in this launch writes, at a wave-uniform address.
 template <typename T>
 __device__ __forceinline__ T scalar_load(const T *from) {
@@ -403,20 +443,21 @@ __device__ __forceinline__ void touch_lines(const char *const (&base)[4], const 
 // is close to a square of operand elements: gn BN = (per / gn) BM.  Plain row-major order
 // (gn = tiles_n) makes every XCD read the whole weight as soon as a range is a tile row
 // long: 28 MB instead of 7 MB for the QKV product of 256 rows at hidden 768.
+constexpr int kMostPanelTiles = 1 << 20;
 struct TilePanels {
   int tiles_m, tiles_n, gn;
-  __device__ __forceinline__ void locate(int L, int &tile_m, int &tile_n) const {
-    const int panel = L / (tiles_m * gn);
+  __device__ __forceinline__ void locate(int L, int &tile_m, int &tile_n) const {   // L < kMostPanelTiles
+    const int panel = divide_small(L, tiles_m * gn);
     const int r = L - panel * tiles_m * gn;
     const int w = min(gn, tiles_n - panel * gn);   // the last panel may be narrower
-    tile_m = r / w;
+    tile_m = divide_small(r, w);
     tile_n = panel * gn + r - tile_m * w;
   }
 };
 template <int BM, int BN>
 __device__ __forceinline__ TilePanels tile_panels(int tiles_m, int tiles_n, int per) {
   int gn = (int)(__builtin_amdgcn_sqrtf((float)per * ((float)BM / (float)BN)) + 0.5f);
-  gn = max(gn, (per + tiles_m - 1) / tiles_m);   // a range taller than the grid is wider instead
+  gn = max(gn, divide_small(per + tiles_m - 1, tiles_m));   // a range taller than the grid is wider instead
   return TilePanels{tiles_m, tiles_n, __builtin_amdgcn_readfirstlane(max(1, min(gn, tiles_n)))};
 }
 

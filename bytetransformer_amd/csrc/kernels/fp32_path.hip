@@ -221,7 +221,10 @@ __device__ __forceinline__ void f32_gemm_tile(const F32GemmArgs &p) {
     const int live = tiles_m * tiles_n, per = (live + 7) >> 3;
     const int bid = (int)blockIdx.x, L = (bid & 7) * per + (bid >> 3);
     if (bid >= per * 8 || L >= live) return;
-    tile_panels<TM, TN>(tiles_m, tiles_n, per).locate(L, tile_m, tile_n);
+    if (live < kMostPanelTiles)
+      tile_panels<TM, TN>(tiles_m, tiles_n, per).locate(L, tile_m, tile_n);
+    else
+      tile_m = L / tiles_n, tile_n = L - tile_m * tiles_n;
   }
   const int m0 = tile_m * TM, n0 = tile_n * TN;
   const int lane = threadIdx.x & 63;
@@ -856,22 +859,16 @@ int launch_f32_ln(const void *src, const void *residual, const void *bias, const
   if (rows_cap == 0) return BT_OK;
   const int grid = (rows_cap + kF32LnRows - 1) / kF32LnRows;
   const float inv_n = 1.0f / (float)H;
-#define BT_F32_LN(NC_)                                                                          \
-  f32_layernorm_kernel<NC_, RESTORE><<<grid, kF32LnRows * kWave, 0, s>>>(                       \
-      (const float4_t *)src, (const float4_t *)residual, (const float4_t *)bias,                \
-      (const float4_t *)gamma, (const float4_t *)beta, (float4_t *)dst, idx, residual_row_index, \
-      S, rows_cap, chunks, inv_n, eps)
-  if (nc <= 2)
-    BT_F32_LN(2);
-  else if (nc <= 4)
-    BT_F32_LN(4);
-  else if (nc <= 8)
-    BT_F32_LN(8);
-  else
-    BT_F32_LN(16);
-#undef BT_F32_LN
-  BT_CHECK_LAUNCH(who);
-  return BT_OK;
+  const auto with = [&](auto nc_tag) {
+    return Launch<f32_layernorm_kernel<nc_tag(), RESTORE>>::on(
+        s, who, grid, kF32LnRows * kWave, 0, (const float4_t *)src, (const float4_t *)residual, (const float4_t *)bias,
+        (const float4_t *)gamma, (const float4_t *)beta, (float4_t *)dst, idx, residual_row_index, S, rows_cap, chunks,
+        inv_n, eps);
+  };
+  if (nc <= 2) return with(std::integral_constant<int, 2>{});
+  if (nc <= 4) return with(std::integral_constant<int, 4>{});
+  if (nc <= 8) return with(std::integral_constant<int, 8>{});
+  return with(std::integral_constant<int, 16>{});
 }
 
 template <int MT, int NT, int NW, int DEPTH, bool RAGGED>
@@ -879,13 +876,9 @@ static int launch_f32_gemm_as(const F32GemmArgs &p, hipStream_t s) {
   constexpr int TM = 32 * MT, TN = 32 * NT, SLICE = (TM + TN) * 16;
   constexpr size_t smem = (size_t)NW * (DEPTH * SLICE > TM * TN ? DEPTH * SLICE : TM * TN) * sizeof(float);
   static_assert(smem <= 160 * 1024, "LDS budget");
-  static std::atomic<bool> configured[kMaxDevices];
-  const int rc = allow_dynamic_lds(f32_gemm_kernel<MT, NT, NW, DEPTH, RAGGED>, smem, configured,
-                                   "hipFuncSetAttribute(f32_gemm_kernel)");
-  if (rc != BT_OK) return rc;
   const long long tiles = (long long)((p.rows_cap + TM - 1) / TM) * ((p.N + TN - 1) / TN);
-  f32_gemm_kernel<MT, NT, NW, DEPTH, RAGGED><<<(unsigned)((tiles + 7) / 8 * 8), 64 * NW, smem, s>>>(p);
-  return BT_OK;
+  return Launch<f32_gemm_kernel<MT, NT, NW, DEPTH, RAGGED>>::on(s, "bt_gemm_f32", (unsigned)((tiles + 7) / 8 * 8),
+                                                                64 * NW, smem, p);
 }
 template <int MT, int NT, int NW, int DEPTH>
 static int launch_f32_gemm(const F32GemmArgs &p, hipStream_t s) {
@@ -943,19 +936,12 @@ extern "C" int bt_gemm_f32(const void *a, const int *a_row_index, const void *w,
   // the tiled kernels address the weight, and the rows of a tile, with 32-bit byte offsets
   if ((long long)n * k * 4 > kF32MaxBytes || (long long)k * 256 > kF32MaxBytes) tile = 3;
   hipStream_t s = as_stream(stream);
-  int rc = BT_OK;
-  if (tile == 0) {
-    rc = launch_f32_gemm<2, 2, 4, 2>(p, s);
-  } else if (tile == 1) {
-    rc = launch_f32_gemm<2, 1, 4, 3>(p, s);
-  } else if (tile == 2) {
-    rc = launch_f32_gemm<1, 1, 4, 4>(p, s);
-  } else {
-    const dim3 grid((n + 31) / 32, (rows_cap + 31) / 32);
-    BT_REQUIRE(grid.y <= 65535, BT_ERR_UNSUPPORTED, "bt_gemm_f32: too many rows");
-    f32_gemm_skinny_kernel<8><<<grid, 512, 0, s>>>(p);
-  }
-  if (rc != BT_OK) return rc;
+  if (tile == 0) return launch_f32_gemm<2, 2, 4, 2>(p, s);
+  if (tile == 1) return launch_f32_gemm<2, 1, 4, 3>(p, s);
+  if (tile == 2) return launch_f32_gemm<1, 1, 4, 4>(p, s);
+  const dim3 grid((n + 31) / 32, (rows_cap + 31) / 32);
+  BT_REQUIRE(grid.y <= 65535, BT_ERR_UNSUPPORTED, "bt_gemm_f32: too many rows");
+  f32_gemm_skinny_kernel<8><<<grid, 512, 0, s>>>(p);
   BT_CHECK_LAUNCH("bt_gemm_f32");
   return BT_OK;
 }
@@ -982,16 +968,13 @@ extern "C" int bt_attention_f32(const void *qkv, void *out, const int *batch_idx
   p.balanced = order == 3 || (order == 2 && per_xcd > 64 && batch_size <= 128);
   const unsigned grid = p.balanced ? (per_xcd + 31) / 32 * 32 * 8 : per_xcd * 8;
   hipStream_t s = as_stream(stream);
-#define BT_F32_ATT(ND_) f32_attention_kernel<ND_, kWaves><<<grid, 64 * kWaves, 0, s>>>(p)
+  const auto with = [&](auto nd) { return Launch<f32_attention_kernel<nd(), kWaves>>::on(s, who, grid, 64 * kWaves, 0, p); };
   switch ((size_per_head + 31) / 32) {
-    case 1: BT_F32_ATT(1); break;
-    case 2: BT_F32_ATT(2); break;
-    case 3: BT_F32_ATT(3); break;
-    default: BT_F32_ATT(4); break;
+    case 1: return with(std::integral_constant<int, 1>{});
+    case 2: return with(std::integral_constant<int, 2>{});
+    case 3: return with(std::integral_constant<int, 3>{});
+    default: return with(std::integral_constant<int, 4>{});
   }
-#undef BT_F32_ATT
-  BT_CHECK_LAUNCH(who);
-  return BT_OK;
 }
 
 extern "C" int bt_add_bias_residual_layernorm_f32(void *out, const void *residual,

@@ -67,56 +67,61 @@ struct GemmArgs {
   int *out_seq_order;   // [mask_B]
   int tile_grid;        // workgroups of the launch (set by the launcher)
   int splits;           // k slices (set by the launcher; 1 but for kEpiPartial)
+  unsigned per_n;       // device only: inverse of tiles_n, for divide()
 };
 
-// What a product needs before it can ask for its first operands, as leading kernel arguments of their
-// own: those are in scalar registers when a wave starts, where the fields of the struct are memory reads
-// (one more cache line of it before the first load cost a launch 0.15 us).
-#define BT_GEMM_FIRST                                                                              \
-  const half_t *a, const half_t *wt, const int *valid_rows, const void *mask, int rows_cap, int N, \
-      int K, int tiles_n, int splits, int tile_grid
-#define BT_GEMM_FIRST_NAMES a, wt, valid_rows, mask, rows_cap, N, K, tiles_n, splits, tile_grid
-#define BT_GEMM_FIRST_OF(p) \
-  p.a, p.wt, p.valid_rows, p.mask, p.rows_cap, p.N, p.K, p.tiles_n, p.splits, p.tile_grid
 // Where a product takes its rows from, as a template parameter: the code that counts the mask rows is 9 KB,
 // three quarters of a small kernel, and the kernels of a layer share an instruction cache of 64 KB (12 layers
 // without it where no mask is counted: 1 x 32 385 -> 374 us, 4 x 96 430 -> 422, 7 x 217 638 -> 626).
 constexpr int kMaskNone = 0, kMaskF16 = 1, kMaskF32 = 2;
 
-// ... and what it needs later.  Every argument byte costs the host: beside ten leading arguments a launch takes
+// What a product needs, as leading kernel arguments of their own: the first 64 bytes are in scalar registers when a
+// wave starts, where the fields of a struct are memory reads, one more round trip ahead of the first load or store.
+// `rows` is valid_rows, or the mask of a launch that counts its rows; `index` is a_row_index, or the counting launch's
+// out_batch_idx; k_splits is K | splits << 24; per_n the inverse of the tile columns.
+// (With the tile's column count, the row index and the pointers of bias and output behind them, and three
+// divisions to find the tile, a small product took 0.3 us longer to its first load.)
+#define BT_GEMM_FIRST                                                                              \
+  const half_t *a, const half_t *wt, const void *rows, const int *index, const half_t *bias, void *out, \
+      int rows_cap, int N, unsigned k_splits, unsigned per_n
+#define BT_GEMM_FIRST_NAMES a, wt, rows, index, bias, out, rows_cap, N, k_splits, per_n
+template <int MASK, typename Then>
+static int with_first_arguments(const GemmArgs &p, Then then) {
+  return then(p.a, p.wt, MASK != kMaskNone ? p.mask : (const void *)p.valid_rows,
+              MASK != kMaskNone ? (const int *)p.out_batch_idx : p.a_row_index, p.bias, p.c32 ? (void *)p.c32 : (void *)p.c,
+              p.rows_cap, p.N, (unsigned)p.K | (unsigned)p.splits << 24, inverse_of((unsigned)p.tiles_n));
+}
+// ... and what few need.  Every argument byte costs the host: beside ten leading arguments a launch takes
 // 3.0 us to issue with 24 bytes more, 3.6 with 48, and 3.8 with the whole of GemmArgs (128), so the fields of a
-// launch that counts mask rows travel with those launches only.
+// launch that counts mask rows, and the grid of one that loops, travel with those launches only.
 template <int MASK>
 struct GemmTail {
-  const half_t *bias;
-  void *out;   // c or c32
-  const int *a_row_index;
-  int mask_B, mask_S;
-  int *out_batch_idx, *out_word_idx, *out_seq_order;
+  int tile_grid, mask_B, mask_S;
+  int *out_word_idx, *out_seq_order;
 };
 template <>
 struct GemmTail<kMaskNone> {
-  const half_t *bias;
-  void *out;
-  const int *a_row_index;
+  int tile_grid, unused[3];   // (see Launch: 16 bytes are issued faster than 4)
 };
 template <int MASK>
 static GemmTail<MASK> gemm_tail(const GemmArgs &p) {
-  void *out = p.c32 ? (void *)p.c32 : (void *)p.c;
   if constexpr (MASK == kMaskNone)
-    return {p.bias, out, p.a_row_index};
+    return {p.tile_grid, {}};
   else
-    return {p.bias, out, p.a_row_index, p.mask_B, p.mask_S, p.out_batch_idx, p.out_word_idx, p.out_seq_order};
+    return {p.tile_grid, p.mask_B, p.mask_S, p.out_word_idx, p.out_seq_order};
 }
-template <int MASK>
+template <int MASK, int BN>
 __device__ __forceinline__ GemmArgs gemm_args(BT_GEMM_FIRST, const GemmTail<MASK> &tail) {
   GemmArgs p{};
-  p.a = a, p.wt = wt, p.valid_rows = valid_rows, p.mask = mask;
-  p.rows_cap = rows_cap, p.N = N, p.K = K, p.tiles_n = tiles_n, p.splits = splits, p.tile_grid = tile_grid;
-  p.bias = tail.bias, p.c = (half_t *)tail.out, p.c32 = (float *)tail.out, p.a_row_index = tail.a_row_index;
-  if constexpr (MASK != kMaskNone) {
+  p.a = a, p.wt = wt, p.bias = bias, p.c = (half_t *)out, p.c32 = (float *)out;
+  p.rows_cap = rows_cap, p.N = N, p.K = (int)(k_splits & 0xffffffu), p.splits = (int)(k_splits >> 24);
+  p.tiles_n = (N + BN - 1) / BN, p.per_n = per_n, p.tile_grid = tail.tile_grid;
+  if constexpr (MASK == kMaskNone) {
+    p.valid_rows = (const int *)rows, p.a_row_index = index;
+  } else {
+    p.mask = rows, p.out_batch_idx = const_cast<int *>(index);
     p.mask_B = tail.mask_B, p.mask_S = tail.mask_S;
-    p.out_batch_idx = tail.out_batch_idx, p.out_word_idx = tail.out_word_idx, p.out_seq_order = tail.out_seq_order;
+    p.out_word_idx = tail.out_word_idx, p.out_seq_order = tail.out_seq_order;
   }
   return p;
 }
@@ -565,11 +570,9 @@ __device__ __forceinline__ bool tile_at(const GemmArgs &p, int M, int bid, int &
   int L = (bid & 7) * per + (bid >> 3);
   if (bid >= per * 8 || L >= live) return false;
   split = 0;
-  if (p.splits > 1) {
-    split = L / tiles;
-    L -= split * tiles;
-  }
-  if (BM == 32 && tiles_m > 3) {
+  if (p.splits > 1)
+    for (; L >= tiles; L -= tiles) ++split;
+  if (BM == 32 && tiles_m > 3 && live < kMostPanelTiles) {
     // A few hundred rows: the launch is as long as it takes to fetch the weight, and in row-major
     // order every XCD fetches all of it (256 rows, QKV at hidden 768: 28 MB in all against
     // 7 MB in panels; 12 layers at batch 1 x 256: -8 %).  At two or three tile rows few workgroups
@@ -578,7 +581,7 @@ __device__ __forceinline__ bool tile_at(const GemmArgs &p, int M, int bid, int &
     // their index arithmetic costs up to 1 %.
     tile_panels<BM, BN>(tiles_m, p.tiles_n, per).locate(L, tile_m, tile_n);
   } else {
-    tile_m = L / p.tiles_n;
+    tile_m = (int)divide((unsigned)L, (unsigned)p.tiles_n, p.per_n);
     tile_n = L - tile_m * p.tiles_n;
   }
   return true;
@@ -624,7 +627,7 @@ __device__ __forceinline__ int gemm_tile(const GemmArgs &p, const int bid) {
   const int end = ((M + BM - 1) / BM * p.tiles_n * p.splits + 7) / 8 * 8;
   const int m0 = tile_m * BM, n0 = tile_n * BN;
   // slice y of a split-k launch: the k range [y, y + 1) * K / splits
-  const int nk = EPI == kEpiPartial ? p.K / BK / p.splits : p.K / BK;
+  const int nk = EPI == kEpiPartial ? divide_small(p.K / BK, p.splits) : p.K / BK;
   const int k_first = EPI == kEpiPartial ? split * nk * BK : 0;
 
   // ---- loading side ---------------------------------------------------------
@@ -827,6 +830,7 @@ __device__ __forceinline__ void gemm_tiles_flat(const GemmArgs &p) {
 
   // XCD x owns the contiguous range [x * per, (x + 1) * per) of the live tiles; its
   // workgroups take them round-robin
+  const auto tile_row = [&](int L) { return (int)divide((unsigned)L, (unsigned)p.tiles_n, p.per_n); };
   const int live = ((M + BM - 1) / BM) * p.tiles_n;
   const int per = (live + 7) >> 3;
   const int wgx = p.tile_grid >> 3;                      // workgroups per XCD
@@ -859,7 +863,7 @@ __device__ __forceinline__ void gemm_tiles_flat(const GemmArgs &p) {
   int ld_L = L0, ld_kt = 0, ld_left = loader ? total : 0;
   int ld_slot = 0;     // bias buffer of the tile being set up: its position in the sequence mod STAGES
   auto fetch_indices = [&](int Lt) {
-    const int m0 = (Lt / p.tiles_n) * BM;
+    const int m0 = tile_row(Lt) * BM;
     MaskRowSpan span{};
     if constexpr (MASK != kMaskNone) span = mask_rows_span(mr, p.mask_B, lane, m0, min(m0 + BM, M) - 1);
 #pragma unroll
@@ -870,7 +874,7 @@ __device__ __forceinline__ void gemm_tiles_flat(const GemmArgs &p) {
     }
   };
   auto load_setup = [&](int Lt, bool more, bool bias_to_lds) {
-    const int tm = Lt / p.tiles_n, tn = Lt - tm * p.tiles_n;
+    const int tm = tile_row(Lt), tn = Lt - tm * p.tiles_n;
     const int m0 = tm * BM, n0 = tn * BN;
     if (kHasBias && bias_to_lds && lw == 0) {
       // 4 bytes per lane and instruction: 128 columns each
@@ -959,7 +963,7 @@ __device__ __forceinline__ void gemm_tiles_flat(const GemmArgs &p) {
   const int n_lane = wn * WTN + (lane >> 4) * 4;
   int cL = L0, c_slot = 0;
   // the first tile's bias straight from memory
-  tile.template start<kHasBias>(p.bias, (cL % p.tiles_n) * BN + n_lane, p.N - 4);
+  tile.template start<kHasBias>(p.bias, (cL - tile_row(cL) * p.tiles_n) * BN + n_lane, p.N - 4);
 
   int stage = 0, kt = 0;
   for (int g = 0; g < total; ++g) {
@@ -976,7 +980,7 @@ __device__ __forceinline__ void gemm_tiles_flat(const GemmArgs &p) {
     if (++kt == nk) {
       // ---- this tile is complete: store it, start the next from its bias ----
       kt = 0;
-      const int tm = cL / p.tiles_n, tn = cL - tm * p.tiles_n;
+      const int tm = tile_row(cL), tn = cL - tm * p.tiles_n;
       const int m0 = tm * BM, n0 = tn * BN;
       __builtin_amdgcn_s_barrier();   // all waves are done reading this stage: it becomes the staging area
       tile.template store<EPI>(p, smem + stage * STAGE_HALFS + wave * 32 * EP, m0 + wm * WTM, n0 + wn * WTN, M, lane);
@@ -1012,18 +1016,26 @@ __device__ __forceinline__ void for_each_tile(const GemmArgs &p, Tile tile) {
 template <int BM, int BN, int STAGES, int WM, int WN, int NP, int EPI, bool WKN, int MASK>
 __global__ __launch_bounds__((WM * WN + NP) * 64) void gemm_flat_kernel(BT_GEMM_FIRST, GemmTail<MASK> tail) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  gemm_tiles_flat<BM, BN, STAGES, WM, WN, NP, EPI, WKN, MASK>(gemm_args<MASK>(BT_GEMM_FIRST_NAMES, tail));
+  gemm_tiles_flat<BM, BN, STAGES, WM, WN, NP, EPI, WKN, MASK>(gemm_args<MASK, BN>(BT_GEMM_FIRST_NAMES, tail));
 #endif
 }
 
 template <int BM, int BN, int STAGES, int WM, int WN, int NP, int EPI, bool WKN, int MASK, bool LOOP>
 __global__ __launch_bounds__((WM * WN + NP) * 64) void gemm_kernel(BT_GEMM_FIRST, GemmTail<MASK> tail) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  const GemmArgs p = gemm_args<MASK>(BT_GEMM_FIRST_NAMES, tail);
+  const GemmArgs p = gemm_args<MASK, BN>(BT_GEMM_FIRST_NAMES, tail);
   if constexpr (LOOP)
     for_each_tile(p, [&](int bid) { return gemm_tile<BM, BN, STAGES, WM, WN, NP, EPI, WKN, MASK, LOOP>(p, bid); });
   else
     gemm_tile<BM, BN, STAGES, WM, WN, NP, EPI, WKN, MASK, LOOP>(p, (int)blockIdx.x);
+#endif
+}
+// Without a mask to count and tiles to go on to there is no tail.
+template <int BM, int BN, int STAGES, int WM, int WN, int NP, int EPI, bool WKN>
+__global__ __launch_bounds__((WM * WN + NP) * 64) void gemm_short_kernel(BT_GEMM_FIRST) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  gemm_tile<BM, BN, STAGES, WM, WN, NP, EPI, WKN, kMaskNone, false>(gemm_args<kMaskNone, BN>(BT_GEMM_FIRST_NAMES, {}),
+                                                                    (int)blockIdx.x);
 #endif
 }
 
@@ -1081,7 +1093,7 @@ __device__ __forceinline__ void gemm_wave_k(const GemmArgs &p) {
   int split, tile_m, tile_n;
   if (!tile_at<BM, BN>(p, M, bid, split, tile_m, tile_n)) return;
   const int m0 = tile_m * BM, n0 = tile_n * BN;
-  const int nk = EPI == kEpiPartial ? p.K / BK / p.splits : p.K / BK;
+  const int nk = EPI == kEpiPartial ? divide_small(p.K / BK, p.splits) : p.K / BK;
   const int k_first = EPI == kEpiPartial ? split * nk * BK : 0;
   const int mine = (nk - wave + NW - 1) / NW;   // (0 where there are fewer steps than waves)
 
@@ -1113,6 +1125,10 @@ __device__ __forceinline__ void gemm_wave_k(const GemmArgs &p) {
     }
   }
   const int w_step_bytes = (WKN ? BK * p.N : BK) * (int)sizeof(half_t);
+  constexpr bool kHasBias = EPI == kEpiBiasGelu || EPI == kEpiQkvSplit || EPI == kEpiBias;
+  const int n = n0 + wave * 8 + (lane >> 5) * 4;   // of the sums that this lane stores
+  half4_t bias = {0, 0, 0, 0};
+  if (kHasBias) bias = *(const half4_t *)(p.bias + min(n, p.N - 4));   // (ahead of the operands: it has long arrived)
   auto issue = [&](int i, int slot) {
     const int kt = wave + i * NW;
     issue_stage_loads<NI, NIA>(rs_a, rs_w, voff, ring + slot * STEP_HALFS, 8 * BK,
@@ -1183,16 +1199,15 @@ __device__ __forceinline__ void gemm_wave_k(const GemmArgs &p) {
 #pragma unroll
   for (int w = 1; w < NW; ++w)
     v += ((const float4_t *)(gemm_smem + w * DEPTH * STEP_HALFS))[wave * 64 + lane];
-  const int m = m0 + fr_row, n = n0 + wave * 8 + fr_kc * 4;
+  const int m = m0 + fr_row;
   if (m >= M || n >= p.N) return;
   if (EPI == kEpiPartial) {
     store_through(p.c32 + ((size_t)split * p.rows_cap + m) * p.N + n, __builtin_bit_cast(uint4_t, v));
     return;
   }
-  if (EPI == kEpiBiasGelu || EPI == kEpiQkvSplit || EPI == kEpiBias) {
-    const half4_t b = *(const half4_t *)(p.bias + n);
+  if (kHasBias) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] += (float)b[e];
+    for (int e = 0; e < 4; ++e) v[e] += (float)bias[e];
   }
   if (EPI == kEpiBiasGelu) {
 #pragma unroll
@@ -1207,21 +1222,29 @@ __device__ __forceinline__ void gemm_wave_k(const GemmArgs &p) {
 template <int EPI, bool WKN, int MASK>
 __global__ __launch_bounds__(kWaveKWaves * 64) void gemm_wave_k_kernel(BT_GEMM_FIRST, GemmTail<MASK> tail) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  gemm_wave_k<EPI, WKN, MASK>(gemm_args<MASK>(BT_GEMM_FIRST_NAMES, tail));
+  gemm_wave_k<EPI, WKN, MASK>(gemm_args<MASK, kWaveKCols>(BT_GEMM_FIRST_NAMES, tail));
+#endif
+}
+template <int EPI, bool WKN>
+__global__ __launch_bounds__(kWaveKWaves * 64) void gemm_wave_k_short_kernel(BT_GEMM_FIRST) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  gemm_wave_k<EPI, WKN, kMaskNone>(gemm_args<kMaskNone, kWaveKCols>(BT_GEMM_FIRST_NAMES, {}));
 #endif
 }
 
 // Plain products whose live rows only the device knows: tile 14 where they fit one round of it, else tile 4
-// (see takes_wave_k).  `splits` brings the most rows of tile 14: an argument that is there at wave launch.
+// (see takes_wave_k).  The top bits of k_splits bring the most tile rows of tile 14.
 template <bool WKN>
-__global__ __launch_bounds__(kWaveKWaves * 64) void gemm_few_rows_kernel(BT_GEMM_FIRST, GemmTail<kMaskNone> tail) {
+__global__ __launch_bounds__(kWaveKWaves * 64) void gemm_few_rows_kernel(BT_GEMM_FIRST) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  GemmArgs p = gemm_args<kMaskNone>(BT_GEMM_FIRST_NAMES, tail);
+  GemmArgs p = gemm_args<kMaskNone, kWaveKCols>(BT_GEMM_FIRST_NAMES, {});
+  const int most_rows = p.splits * 32;
   p.splits = 1;
-  if (*valid_rows <= splits) {
+  if (*p.valid_rows <= most_rows) {
     gemm_wave_k<kEpiPlain, WKN, kMaskNone>(p);
   } else {
     p.tiles_n = (p.N + 63) / 64;
+    p.per_n = 0xffffffffu / (unsigned)p.tiles_n;
     gemm_tile<32, 64, 4, 1, 2, 2, kEpiPlain, WKN, kMaskNone, false>(p, (int)blockIdx.x);
   }
 #endif
@@ -1263,9 +1286,9 @@ static int launched_tiles(const GemmArgs &p, int bm, int all) {
 }
 
 // Calls `launch` with the weight layout and the source of the rows as compile-time constants.
-template <int EPI, typename Launch>
-static int by_layout(const GemmArgs &p, Launch launch) {
-  auto with = [&](auto mask) { return p.w_kn ? launch(std::true_type{}, mask) : launch(std::false_type{}, mask); };
+template <int EPI, typename Then>
+static int by_layout(const GemmArgs &p, Then then) {
+  auto with = [&](auto mask) { return p.w_kn ? then(std::true_type{}, mask) : then(std::false_type{}, mask); };
   if constexpr (EPI == kEpiQkvSplit || EPI == kEpiBias) {
     if (p.mask && p.mask_f32) return with(std::integral_constant<int, kMaskF32>{});
     if (p.mask) return with(std::integral_constant<int, kMaskF16>{});
@@ -1275,14 +1298,14 @@ static int by_layout(const GemmArgs &p, Launch launch) {
 
 template <int BM, int BN, int STAGES, int WM, int WN, int NP, int EPI, bool WKN, int MASK, bool LOOP>
 static int launch_gemm_kernel(const GemmArgs &p, hipStream_t s, size_t smem) {
-  static std::atomic<bool> configured[kMaxDevices];
-  const int rc = allow_dynamic_lds(gemm_kernel<BM, BN, STAGES, WM, WN, NP, EPI, WKN, MASK, LOOP>, smem,
-                                   configured, "hipFuncSetAttribute(gemm_kernel)");
-  if (rc != BT_OK) return rc;
-  gemm_kernel<BM, BN, STAGES, WM, WN, NP, EPI, WKN, MASK, LOOP>
-      <<<dim3(p.tile_grid), (WM * WN + NP) * 64, smem, s>>>(BT_GEMM_FIRST_OF(p), gemm_tail<MASK>(p));
-  BT_CHECK_LAUNCH("gemm_kernel");
-  return BT_OK;
+  return with_first_arguments<MASK>(p, [&](auto... first) {
+    if constexpr (MASK == kMaskNone && !LOOP)
+      return Launch<gemm_short_kernel<BM, BN, STAGES, WM, WN, NP, EPI, WKN>>::on(
+          s, "gemm_kernel", p.tile_grid, (WM * WN + NP) * 64, smem, first...);
+    else
+      return Launch<gemm_kernel<BM, BN, STAGES, WM, WN, NP, EPI, WKN, MASK, LOOP>>::on(
+          s, "gemm_kernel", p.tile_grid, (WM * WN + NP) * 64, smem, first..., gemm_tail<MASK>(p));
+  });
 }
 
 template <int BM, int BN, int STAGES, int WM, int WN, int NP, int EPI, bool WKN, int MASK>
@@ -1315,17 +1338,16 @@ static int launch_gemm_wave_k_as(GemmArgs p, hipStream_t s, int splits) {
   // (and 256 bytes for the lengths of a launch that counts the mask rows)
   constexpr size_t smem = (size_t)kWaveKWaves * kWaveKDepth * (32 + kWaveKCols) * kBK * sizeof(half_t) + 256;
   static_assert(smem <= 160 * 1024, "LDS budget");
-  static std::atomic<bool> configured[kMaxDevices];
-  const int rc = allow_dynamic_lds(gemm_wave_k_kernel<EPI, WKN, MASK>, smem, configured,
-                                   "hipFuncSetAttribute(gemm_wave_k_kernel)");
-  if (rc != BT_OK) return rc;
   p.tiles_n = (p.N + kWaveKCols - 1) / kWaveKCols;
   p.splits = splits;
   p.tile_grid = ((p.rows_cap + 31) / 32 * p.tiles_n * splits + 7) / 8 * 8;
-  gemm_wave_k_kernel<EPI, WKN, MASK>
-      <<<dim3(p.tile_grid), kWaveKWaves * 64, smem, s>>>(BT_GEMM_FIRST_OF(p), gemm_tail<MASK>(p));
-  BT_CHECK_LAUNCH("gemm_wave_k_kernel");
-  return BT_OK;
+  return with_first_arguments<MASK>(p, [&](auto... first) {
+    if constexpr (MASK == kMaskNone)
+      return Launch<gemm_wave_k_short_kernel<EPI, WKN>>::on(s, "gemm_wave_k_kernel", p.tile_grid, kWaveKWaves * 64, smem, first...);
+    else
+      return Launch<gemm_wave_k_kernel<EPI, WKN, MASK>>::on(s, "gemm_wave_k_kernel", p.tile_grid, kWaveKWaves * 64, smem,
+                                                            first..., gemm_tail<MASK>(p));
+  });
 }
 
 template <int EPI>
@@ -1339,18 +1361,15 @@ template <bool WKN>
 static int launch_gemm_few_rows_as(GemmArgs p, hipStream_t s) {
   constexpr size_t smem = (size_t)kWaveKWaves * kWaveKDepth * (32 + kWaveKCols) * kBK * sizeof(half_t);
   static_assert(smem >= 4 * (32 + 64) * kBK * sizeof(half_t), "room for the ring of tile 4");
-  static std::atomic<bool> configured[kMaxDevices];
-  const int rc = allow_dynamic_lds(gemm_few_rows_kernel<WKN>, smem, configured, "hipFuncSetAttribute(gemm_few_rows_kernel)");
-  if (rc != BT_OK) return rc;
   p.tiles_n = (p.N + kWaveKCols - 1) / kWaveKCols;
   // (one round of either tile: what the few rows take, or the capacity in the wider tiles)
-  p.splits = cu_count() / p.tiles_n * 32;
-  const int few = p.splits / 32 * p.tiles_n, wide = (p.rows_cap + 31) / 32 * ((p.N + 63) / 64);
-  p.tile_grid = ((few > wide ? few : wide) + 7) / 8 * 8;
-  gemm_few_rows_kernel<WKN>
-      <<<dim3(p.tile_grid), kWaveKWaves * 64, smem, s>>>(BT_GEMM_FIRST_OF(p), gemm_tail<kMaskNone>(p));
-  BT_CHECK_LAUNCH("gemm_few_rows_kernel");
-  return BT_OK;
+  p.splits = cu_count() / p.tiles_n;   // tile rows of one round, at most 255 of them
+  if (p.splits > 255) p.splits = 255;
+  const int few = p.splits * p.tiles_n, wide = (p.rows_cap + 31) / 32 * ((p.N + 63) / 64);
+  const int grid = ((few > wide ? few : wide) + 7) / 8 * 8;
+  return with_first_arguments<kMaskNone>(p, [&](auto... first) {
+    return Launch<gemm_few_rows_kernel<WKN>>::on(s, "gemm_few_rows_kernel", grid, kWaveKWaves * 64, smem, first...);
+  });
 }
 static int launch_gemm_few_rows(const GemmArgs &p, hipStream_t s) {
   return p.w_kn ? launch_gemm_few_rows_as<true>(p, s) : launch_gemm_few_rows_as<false>(p, s);
@@ -1362,10 +1381,6 @@ template <int BM, int BN, int STAGES, int WM, int WN, int NP, int EPI, bool WKN,
 static int launch_gemm_flat_as(GemmArgs p, hipStream_t s) {
   constexpr size_t smem = (size_t)STAGES * (BM + BN) * kBK * sizeof(half_t) + STAGES * BN * sizeof(half_t);
   static_assert(smem <= 160 * 1024, "LDS budget");
-  static std::atomic<bool> configured[kMaxDevices];
-  const int rc = allow_dynamic_lds(gemm_flat_kernel<BM, BN, STAGES, WM, WN, NP, EPI, WKN, MASK>,
-                                   smem, configured, "hipFuncSetAttribute(gemm_flat_kernel)");
-  if (rc != BT_OK) return rc;
   const int tiles_m = (p.rows_cap + BM - 1) / BM;
   p.tiles_n = (p.N + BN - 1) / BN;
   const long long tiles = (long long)tiles_m * p.tiles_n;
@@ -1373,11 +1388,11 @@ static int launch_gemm_flat_as(GemmArgs p, hipStream_t s) {
   long long wgs = (long long)cu_count() * per_cu;
   if (wgs > tiles) wgs = tiles;
   p.tile_grid = (int)((wgs + 7) / 8 * 8);
-  const dim3 grid((unsigned)p.tile_grid);
-  gemm_flat_kernel<BM, BN, STAGES, WM, WN, NP, EPI, WKN, MASK>
-      <<<grid, (WM * WN + NP) * 64, smem, s>>>(BT_GEMM_FIRST_OF(p), gemm_tail<MASK>(p));
-  BT_CHECK_LAUNCH("gemm_flat_kernel");
-  return BT_OK;
+  p.splits = 1;
+  return with_first_arguments<MASK>(p, [&](auto... first) {
+    return Launch<gemm_flat_kernel<BM, BN, STAGES, WM, WN, NP, EPI, WKN, MASK>>::on(
+        s, "gemm_flat_kernel", p.tile_grid, (WM * WN + NP) * 64, smem, first..., gemm_tail<MASK>(p));
+  });
 }
 
 template <int BM, int BN, int STAGES, int WM, int WN, int NP, int EPI>
@@ -1743,9 +1758,7 @@ extern "C" int bt_transpose_weights(int count, const void *const *w, void *const
     tiles += ((n[i] + 63) / 64) * ((k[i] + 63) / 64);
   }
   for (int i = count; i < 4; ++i) a.job[i] = a.job[0];
-  transpose_kernel<<<tiles, 256, 0, as_stream(stream)>>>(a);
-  BT_CHECK_LAUNCH("transpose_kernel");
-  return BT_OK;
+  return Launch<transpose_kernel>::on(as_stream(stream), "transpose_kernel", tiles, 256, 0, a);
 }
 
 extern "C" int bt_transpose_weight(const void *w, void *wt, int k, int n, void *stream) {

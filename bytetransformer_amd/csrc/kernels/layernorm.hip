@@ -33,28 +33,29 @@ __device__ __forceinline__ void ln_finish(const H (&av)[NC], const H (&rv)[NC], 
                                           const float4_t (&g32)[NG][V / 4], const float4_t (&b32)[NG][V / 4],
                                           const void *gamma, const void *beta, const int (&cc)[NC],
                                           const bool (&live)[NC], half_t *o, float inv_n, float eps) {
+  // (four sums side by side: a quarter of the chain)
   float v[NC][V];
-  float sum = 0.f;
+  float part[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int i = 0; i < NC; ++i) {
     const H x = (av[i] + rv[i]) + bias_v[i];  // two fp16-rounded adds
 #pragma unroll
     for (int j = 0; j < V; ++j) {
       v[i][j] = live[i] ? (float)x[j] : 0.f;
-      sum += v[i][j];
+      part[j & 3] += v[i][j];
     }
   }
-  const float mean = wave_sum(sum) * inv_n;
-  float sq = 0.f;
+  const float mean = wave_sum((part[0] + part[1]) + (part[2] + part[3])) * inv_n;
+  float sq[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int i = 0; i < NC; ++i) {
 #pragma unroll
     for (int j = 0; j < V; ++j) {
       v[i][j] = live[i] ? v[i][j] - mean : 0.f;
-      sq += v[i][j] * v[i][j];
+      sq[j & 3] += v[i][j] * v[i][j];
     }
   }
-  const float rstd = rsqrtf(wave_sum(sq) * inv_n + eps);
+  const float rstd = rsqrtf(wave_sum((sq[0] + sq[1]) + (sq[2] + sq[3])) * inv_n + eps);
 
 #pragma unroll
   for (int i = 0; i < NC; ++i) {
@@ -219,10 +220,9 @@ __global__ __launch_bounds__(kLnRowsPerBlock *kWave) void layernorm_kernel(
                                                       inv_n, eps, per_s);
 }
 
-// Calls `launch` with the way that rows of H halfs are dealt to a wave as compile-time constants.
-template <typename Launch>
-static void by_row_shape(int H, Launch launch) {
-  const auto with = [&](auto nc, auto v, auto full) { launch(nc, v, full); };
+// Calls `with` with the way that rows of H halfs are dealt to a wave as compile-time constants.
+template <typename Then>
+static int by_row_shape(int H, Then with) {
   using std::integral_constant;
   if (H == 768) return with(integral_constant<int, 3>{}, integral_constant<int, 4>{}, std::true_type{});
   if (H == 512) return with(integral_constant<int, 1>{}, integral_constant<int, 8>{}, std::true_type{});
@@ -231,7 +231,7 @@ static void by_row_shape(int H, Launch launch) {
   if (nc <= 1) return with(integral_constant<int, 1>{}, integral_constant<int, 8>{}, std::false_type{});
   if (nc <= 2) return with(integral_constant<int, 2>{}, integral_constant<int, 8>{}, std::false_type{});
   if (nc <= 4) return with(integral_constant<int, 4>{}, integral_constant<int, 8>{}, std::false_type{});
-  with(integral_constant<int, 8>{}, integral_constant<int, 8>{}, std::false_type{});
+  return with(integral_constant<int, 8>{}, integral_constant<int, 8>{}, std::false_type{});
 }
 
 // The packed LayerNorm with k-contiguous weight copies riding along: the first `copy_blocks`
@@ -273,16 +273,15 @@ static int launch_ln(const void *src, const void *residual, const void *bias, co
   if (rows_cap == 0) return BT_OK;
   const int grid = (rows_cap + kLnRowsPerBlock - 1) / kLnRowsPerBlock;
   const float inv_n = 1.0f / (float)H;
-  by_row_shape(H, [&](auto nc, auto v, auto full) {
-    const auto kernel = gb32 ? layernorm_kernel<nc(), v(), full(), RESTORE, true, SPLITS>
-                             : layernorm_kernel<nc(), v(), full(), RESTORE, false, SPLITS>;
-    kernel<<<grid, kLnRowsPerBlock * kWave, 0, s>>>((const half_t *)src, (const half_t *)residual, (const half_t *)bias,
-                                                    gamma, beta, (half_t *)dst, idx, residual_row_index, B, S,
-                                                    rows_cap, split_rows ? split_rows : rows_cap, H, inv_n, eps,
-                                                    inverse_of((unsigned)S));
+  return by_row_shape(H, [&](auto nc, auto v, auto full) {
+    const auto with = [&](auto affine32) {
+      return Launch<layernorm_kernel<nc(), v(), full(), RESTORE, affine32(), SPLITS>>::on(
+          s, who, grid, kLnRowsPerBlock * kWave, 0, (const half_t *)src, (const half_t *)residual, (const half_t *)bias,
+          gamma, beta, (half_t *)dst, idx, residual_row_index, B, S, rows_cap, split_rows ? split_rows : rows_cap, H,
+          inv_n, eps, inverse_of((unsigned)S));
+    };
+    return gb32 ? with(std::true_type{}) : with(std::false_type{});
   });
-  BT_CHECK_LAUNCH(who);
-  return BT_OK;
 }
 
 }  // namespace bt
@@ -336,15 +335,14 @@ extern "C" int bt_add_bias_residual_layernorm_copy(
   const int grid = copy_blocks + (rows_cap + kLnRowsPerBlock - 1) / kLnRowsPerBlock;
   const float inv_n = 1.0f / (float)H;
   hipStream_t s = as_stream(stream);
-  by_row_shape(H, [&](auto nc, auto v, auto full) {
-    const auto kernel = gamma_beta_fp32 ? layernorm_copy_kernel<nc(), v(), full(), true>
-                                        : layernorm_copy_kernel<nc(), v(), full(), false>;
-    kernel<<<grid, kLnRowsPerBlock * kWave, 0, s>>>((const half_t *)out, (const half_t *)residual, (const half_t *)bias,
-                                                    gamma, beta, (half_t *)out, valid_rows, residual_row_index,
-                                                    rows_cap, H, inv_n, eps, jobs, copy_blocks);
+  return by_row_shape(H, [&](auto nc, auto v, auto full) {
+    const auto with = [&](auto affine32) {
+      return Launch<layernorm_copy_kernel<nc(), v(), full(), affine32()>>::on(
+          s, who, grid, kLnRowsPerBlock * kWave, 0, (const half_t *)out, (const half_t *)residual, (const half_t *)bias,
+          gamma, beta, (half_t *)out, valid_rows, residual_row_index, rows_cap, H, inv_n, eps, jobs, copy_blocks);
+    };
+    return gamma_beta_fp32 ? with(std::true_type{}) : with(std::false_type{});
   });
-  BT_CHECK_LAUNCH(who);
-  return BT_OK;
 }
 
 extern "C" int bt_add_bias_residual_layernorm_restore(

@@ -22,6 +22,7 @@ void set_error(const char *fmt, ...) {
 }
 
 int hip_fail(hipError_t e, const char *what) {
+  (void)hipGetLastError();   // (reported here, not once more by whoever asks next)
   set_error("[BT][ERROR] HIP runtime error: %s (%s)", hipGetErrorString(e), what);
   return BT_ERR_HIP;
 }
@@ -521,9 +522,7 @@ extern "C" int bt_build_offsets(const void *atten_mask, int mask_dtype, int batc
 
 extern "C" int bt_publish_int(const int *src, int *dst, void *stream) {
   BT_REQUIRE(src && dst, BT_ERR_INVALID_ARGUMENT, "bt_publish_int: null pointer argument");
-  publish_int_kernel<<<1, kWave, 0, as_stream(stream)>>>(src, dst);
-  BT_CHECK_LAUNCH("publish_int_kernel");
-  return BT_OK;
+  return Launch<publish_int_kernel>::on(as_stream(stream), "publish_int_kernel", 1, kWave, 0, src, dst);
 }
 
 extern "C" int bt_layer_prologue(const void *atten_mask, int mask_dtype, int batch_size,
@@ -577,15 +576,12 @@ extern "C" int bt_layer_prologue(const void *atten_mask, int mask_dtype, int bat
   const int grid = ((mask_prefix_slots || weight_count > 0 || warming) ? kPrefixBlocks : offset_blocks) +
                    (pl.list ? kListBlocks : 0);
   if (mask_dtype == BT_F16)
-    layer_prologue_kernel<half_t><<<grid, kPrologueThreads, smem, s>>>(
-        (const half_t *)atten_mask, batch_idx, word_idx, seq_order, mask_prefix_slots, batch_size,
-        seq_len, offset_blocks, pw, pl);
-  else
-    layer_prologue_kernel<float><<<grid, kPrologueThreads, smem, s>>>(
-        (const float *)atten_mask, batch_idx, word_idx, seq_order, mask_prefix_slots, batch_size,
-        seq_len, offset_blocks, pw, pl);
-  BT_CHECK_LAUNCH("layer_prologue_kernel");
-  return BT_OK;
+    return Launch<layer_prologue_kernel<half_t>>::on(s, "layer_prologue_kernel", grid, kPrologueThreads, smem,
+                                                     (const half_t *)atten_mask, batch_idx, word_idx, seq_order,
+                                                     mask_prefix_slots, batch_size, seq_len, offset_blocks, pw, pl);
+  return Launch<layer_prologue_kernel<float>>::on(s, "layer_prologue_kernel", grid, kPrologueThreads, smem,
+                                                  (const float *)atten_mask, batch_idx, word_idx, seq_order,
+                                                  mask_prefix_slots, batch_size, seq_len, offset_blocks, pw, pl);
 }
 
 extern "C" int bt_mask_prefix_slots(const void *atten_mask, int mask_dtype, int batch_size,
