@@ -50,6 +50,11 @@ KERNEL_ABI = {
                                      POINTER(c_int), _P]),
     "bt_gemm": (c_int, [_P, _P, _P, _IP, c_int, c_int, c_int, c_int, c_int, _P]),
     "bt_gemm_bias_gelu": (c_int, [_P, _P, _P, _P, _IP, c_int, c_int, c_int, c_int, c_int, _P]),
+    "bt_split_f32": (c_int, [c_int, POINTER(c_void_p), POINTER(c_void_p), POINTER(c_void_p), POINTER(c_int), POINTER(c_int),
+                             c_int, _P, _P, _P, _P, _IP, _IP, _IP, c_int, c_int, _P]),
+    "bt_gemm_f32_split": (c_int, [_P, _IP, _P, _IP, _P, _P, _IP, _IP, c_int, c_int, c_int, _P]),
+    "bt_add_bias_residual_layernorm_f32_split": (c_int, [_P, _P, _IP, _P, _P, _P, _IP, c_int, c_int, c_float, _P, _IP, _IP,
+                                                         _P, c_int, _P]),
     "bt_gemm_qkv_bias_split": (c_int, [_P, _IP, _P, _P, _P, _IP, c_int, c_int, c_int, c_int,
                                        c_int, _P]),
     "bt_gemm_qkv_mask_rows_supported": (c_int, [c_int, c_int, c_int]),

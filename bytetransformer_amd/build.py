@@ -23,7 +23,7 @@ ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 HIPCC = os.path.join(ROCM, "bin", "hipcc")
 
 KERNEL_SOURCES = ["padding.hip", "layernorm.hip", "gemm.hip", "attention.hip",
-                  "attention_generic.hip", "fp32_path.hip"]
+                  "attention_generic.hip", "fp32_path.hip", "fp32_split.hip"]
 HOST_SOURCES = ["attention.cc", "bert_transformer.cc", "bert_encoder.cc", "c_api.cc"]
 HOST_DEVICE_SOURCE = "layer_static_scratch.hip"
 TH_OP_SOURCES = ["ths_op_f.cc", "ths_op.cc"]

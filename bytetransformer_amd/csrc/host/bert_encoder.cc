@@ -88,6 +88,12 @@ void BertEncoder<OpType>::infer(BertEncoderInferParam<DataType_> ip) {
   // few rows, long k: FFN2 as split-k partial sums that the last LayerNorm folds in (the same in every layer)
   const int splits =
       OpType == OperationType::HALF ? ffn2_slices(rows, valid_rows == nullptr, hidden, inter, partials_bytes) : 1;
+  // float: weights split afresh in every layer where the rows are worth it
+  const bool f32_split = OpType == OperationType::FP32 && f32_splits_operands(rows, !is_remove_padding_, hidden, inter);
+  uint8_t *split_at = base + off + align_up(attention_layer_->work_list_capacity(), 256);
+  void *w_pairs[4] = {split_at, split_at + 12ull * hidden * hidden, split_at + 16ull * hidden * hidden,
+                      split_at + 16ull * hidden * hidden + 4ull * hidden * inter};
+  const F32SplitScratch sp(split_at + align_up(layer_weight_elems() * sizeof(float), 256), max_rows, hidden, inter);
 
   for (int l = 0; l < L; ++l) {
     const auto &w = layers_[l];
@@ -102,8 +108,18 @@ void BertEncoder<OpType>::infer(BertEncoderInferParam<DataType_> ip) {
     attention_layer_->initialize(w.attention_param);
 
     if constexpr (OpType == OperationType::FP32) {
-      check_bt_error(bt_gemm_f32(x, gather, w.attr_kernel_QKV, w.attention_param.attr_bias_QKV,
-                                 qkv_buf, 0, valid_rows, rows, rows_hint, 3 * hidden, hidden, stream));
+      // (the input's pairs lie in FFN1's area until that is written)
+      if (f32_split) {
+        const void *ws[4] = {w.attr_kernel_QKV, w.attr_output_kernel, w.inter_kernel, w.output_kernel};
+        const int ks[4] = {hidden, hidden, hidden, inter}, ns[4] = {3 * hidden, hidden, inter, hidden};
+        check_bt_error(bt_split_f32(4, ws, w_pairs, sp.w_exps, ks, ns, 2, w.inter_bias, sp.bounds, x, inter_matmul_buf, sp.x_exps,
+                                    gather, valid_rows, rows, hidden, stream));
+        check_bt_error(bt_gemm_f32_split(inter_matmul_buf, sp.x_exps, w_pairs[0], sp.w_exps[0], w.attention_param.attr_bias_QKV,
+                                         qkv_buf, nullptr, valid_rows, rows, 3 * hidden, hidden, stream));
+      } else {
+        check_bt_error(bt_gemm_f32(x, gather, w.attr_kernel_QKV, w.attention_param.attr_bias_QKV,
+                                   qkv_buf, 0, valid_rows, rows, rows_hint, 3 * hidden, hidden, stream));
+      }
       struct AttentionInferParam<DataType_> att {
         qkv_buf, ip.atten_mask, attr_out_buf, nullptr, batch_size, seq_len, nullptr, stream,
             et_param
@@ -111,15 +127,31 @@ void BertEncoder<OpType>::infer(BertEncoderInferParam<DataType_> ip) {
       att.attention_bias = ip.attention_bias;
       att.seq_order = seq_order;
       attention_layer_->infer(att);
-      check_bt_error(bt_gemm_f32(attr_out_buf, nullptr, w.attr_output_kernel, nullptr,
-                                 attr_matmul_buf, 0, valid_rows, rows, rows_hint, hidden, hidden, stream));
-      check_bt_error(bt_add_bias_residual_layernorm_f32(
-          attr_matmul_buf, x, gather, w.attr_output_bias, w.attr_output_layernorm_gamma,
-          w.attr_output_layernorm_beta, valid_rows, rows, hidden, layernorm_eps, stream));
-      check_bt_error(bt_gemm_f32(attr_matmul_buf, nullptr, w.inter_kernel, w.inter_bias,
-                                 inter_matmul_buf, 1, valid_rows, rows, rows_hint, inter, hidden, stream));
-      check_bt_error(bt_gemm_f32(inter_matmul_buf, nullptr, w.output_kernel, nullptr, ffn2_out, 0,
-                                 valid_rows, rows, rows_hint, hidden, inter, stream));
+      if (f32_split) {
+        // (Q, K, V are dead: the attention's pairs take the first tensor's place, the LayerNorm's the second's)
+        DataType_ *att_pairs = qkv_buf, *ln_pairs = qkv_buf + tensor;
+        check_bt_error(bt_split_f32(0, nullptr, nullptr, nullptr, nullptr, nullptr, -1, nullptr, nullptr, attr_out_buf, att_pairs,
+                                    sp.att_exps, nullptr, valid_rows, rows, hidden, stream));
+        check_bt_error(bt_gemm_f32_split(att_pairs, sp.att_exps, w_pairs[1], sp.w_exps[1], nullptr, attr_matmul_buf, nullptr,
+                                         valid_rows, rows, hidden, hidden, stream));
+        check_bt_error(bt_add_bias_residual_layernorm_f32_split(
+            attr_matmul_buf, x, gather, w.attr_output_bias, w.attr_output_layernorm_gamma, w.attr_output_layernorm_beta,
+            valid_rows, rows, hidden, layernorm_eps, ln_pairs, sp.ln_exps, sp.gelu_exps, sp.bounds, sp.bound_count, stream));
+        check_bt_error(bt_gemm_f32_split(ln_pairs, sp.ln_exps, w_pairs[2], sp.w_exps[2], w.inter_bias, inter_matmul_buf,
+                                         sp.gelu_exps, valid_rows, rows, inter, hidden, stream));
+        check_bt_error(bt_gemm_f32_split(inter_matmul_buf, sp.gelu_exps, w_pairs[3], sp.w_exps[3], nullptr, ffn2_out, nullptr,
+                                         valid_rows, rows, hidden, inter, stream));
+      } else {
+        check_bt_error(bt_gemm_f32(attr_out_buf, nullptr, w.attr_output_kernel, nullptr,
+                                   attr_matmul_buf, 0, valid_rows, rows, rows_hint, hidden, hidden, stream));
+        check_bt_error(bt_add_bias_residual_layernorm_f32(
+            attr_matmul_buf, x, gather, w.attr_output_bias, w.attr_output_layernorm_gamma,
+            w.attr_output_layernorm_beta, valid_rows, rows, hidden, layernorm_eps, stream));
+        check_bt_error(bt_gemm_f32(attr_matmul_buf, nullptr, w.inter_kernel, w.inter_bias,
+                                   inter_matmul_buf, 1, valid_rows, rows, rows_hint, inter, hidden, stream));
+        check_bt_error(bt_gemm_f32(inter_matmul_buf, nullptr, w.output_kernel, nullptr, ffn2_out, 0,
+                                   valid_rows, rows, rows_hint, hidden, inter, stream));
+      }
       if (last && is_remove_padding_)
         check_bt_error(bt_add_bias_residual_layernorm_restore_f32(
             ffn2_out, attr_matmul_buf, w.output_bias, w.output_layernorm_gamma,

@@ -231,11 +231,28 @@ void BertTransformer<OpType>::bert_infer(BertTransformerInferParam infer_param) 
   }
 
   if constexpr (OpType == OperationType::FP32) {
-    // float: weights are consumed as stored, Q/K/V stay token-major [rows, 3H], gamma
-    // and beta are float by definition
-    check_bt_error(bt_gemm_f32(from_tensor, gather, param_.attr_kernel_QKV,
-                               param_.attention_param.attr_bias_QKV, qkv_buf, 0, valid_rows, rows, rows_hint,
-                               3 * hidden, hidden, stream));
+    // float: Q/K/V stay token-major [rows, 3H], gamma and beta are float by definition.  The weights are consumed as
+    // stored, or, where the rows are worth it, split afresh in every call (all four, and the input's rows, in one
+    // launch; the input's pairs lie in FFN1's area until that is written).
+    const bool split = f32_splits_operands(rows, !is_remove_padding_, hidden, inter);
+    const F32SplitScratch sp(base + off + align_up(splitk_scratch_bytes(max_rows, hidden), 256), max_rows, hidden, inter);
+    void *w_pairs[4];
+    {
+      uint8_t *slot = base + copies_off;
+      for (int i = 0; i < 4; ++i) w_pairs[i] = slot, slot += (size_t)w_k[i] * w_n[i] * sizeof(float);
+    }
+    if (split) {
+      const void *w[4] = {w_use[0], w_use[1], w_use[2], w_use[3]};
+      check_bt_error(bt_split_f32(4, w, w_pairs, sp.w_exps, w_k, w_n, 2, param_.inter_bias, sp.bounds, from_tensor,
+                                  inter_matmul_buf, sp.x_exps, gather, valid_rows, rows, hidden, stream));
+      check_bt_error(bt_gemm_f32_split(inter_matmul_buf, sp.x_exps, w_pairs[0], sp.w_exps[0],
+                                       param_.attention_param.attr_bias_QKV, qkv_buf, nullptr, valid_rows, rows,
+                                       3 * hidden, hidden, stream));
+    } else {
+      check_bt_error(bt_gemm_f32(from_tensor, gather, param_.attr_kernel_QKV,
+                                 param_.attention_param.attr_bias_QKV, qkv_buf, 0, valid_rows, rows, rows_hint,
+                                 3 * hidden, hidden, stream));
+    }
     if (infer_param.valid_word_num_out && is_remove_padding_ && !have_offsets)
       check_bt_error(bt_publish_int(et_param.batch_idx + batch_size,
                                     infer_param.valid_word_num_out, stream));
@@ -247,19 +264,36 @@ void BertTransformer<OpType>::bert_infer(BertTransformerInferParam infer_param) 
     attention_infer_param.seq_order = seq_order;
     attention_infer_param.mask_prefix = have_offsets ? infer_param.mask_prefix : -1;
     attention_layer_->infer(attention_infer_param);
-    check_bt_error(bt_gemm_f32(attr_out_buf, nullptr, param_.attr_output_kernel, nullptr,
-                               attr_matmul_buf, 0, valid_rows, packed_cap, rows_hint, hidden, hidden,
-                               stream));
-    check_bt_error(bt_add_bias_residual_layernorm_f32(
-        attr_matmul_buf, from_tensor, gather, param_.attr_output_bias,
-        param_.attr_output_layernorm_gamma, param_.attr_output_layernorm_beta, valid_rows,
-        packed_cap, hidden, layernorm_eps, stream));
-    check_bt_error(bt_gemm_f32(attr_matmul_buf, nullptr, param_.inter_kernel, param_.inter_bias,
-                               inter_matmul_buf, 1, valid_rows, packed_cap, rows_hint, inter, hidden,
-                               stream));
-    check_bt_error(bt_gemm_f32(inter_matmul_buf, nullptr, param_.output_kernel, nullptr,
-                               transformer_out, 0, valid_rows, packed_cap, rows_hint, hidden, inter,
-                               stream));
+    if (split) {
+      // (Q, K, V are dead: the attention's pairs take the first tensor's place, the LayerNorm's the second's)
+      DataType_ *att_pairs = qkv_buf, *ln_pairs = qkv_buf + tensor;
+      check_bt_error(bt_split_f32(0, nullptr, nullptr, nullptr, nullptr, nullptr, -1, nullptr, nullptr, attr_out_buf, att_pairs,
+                                  sp.att_exps, nullptr, valid_rows, packed_cap, hidden, stream));
+      check_bt_error(bt_gemm_f32_split(att_pairs, sp.att_exps, w_pairs[1], sp.w_exps[1], nullptr, attr_matmul_buf, nullptr,
+                                       valid_rows, packed_cap, hidden, hidden, stream));
+      check_bt_error(bt_add_bias_residual_layernorm_f32_split(
+          attr_matmul_buf, from_tensor, gather, param_.attr_output_bias, param_.attr_output_layernorm_gamma,
+          param_.attr_output_layernorm_beta, valid_rows, packed_cap, hidden, layernorm_eps, ln_pairs, sp.ln_exps, sp.gelu_exps,
+          sp.bounds, sp.bound_count, stream));
+      check_bt_error(bt_gemm_f32_split(ln_pairs, sp.ln_exps, w_pairs[2], sp.w_exps[2], param_.inter_bias, inter_matmul_buf,
+                                       sp.gelu_exps, valid_rows, packed_cap, inter, hidden, stream));
+      check_bt_error(bt_gemm_f32_split(inter_matmul_buf, sp.gelu_exps, w_pairs[3], sp.w_exps[3], nullptr, transformer_out,
+                                       nullptr, valid_rows, packed_cap, hidden, inter, stream));
+    } else {
+      check_bt_error(bt_gemm_f32(attr_out_buf, nullptr, param_.attr_output_kernel, nullptr,
+                                 attr_matmul_buf, 0, valid_rows, packed_cap, rows_hint, hidden, hidden,
+                                 stream));
+      check_bt_error(bt_add_bias_residual_layernorm_f32(
+          attr_matmul_buf, from_tensor, gather, param_.attr_output_bias,
+          param_.attr_output_layernorm_gamma, param_.attr_output_layernorm_beta, valid_rows,
+          packed_cap, hidden, layernorm_eps, stream));
+      check_bt_error(bt_gemm_f32(attr_matmul_buf, nullptr, param_.inter_kernel, param_.inter_bias,
+                                 inter_matmul_buf, 1, valid_rows, packed_cap, rows_hint, inter, hidden,
+                                 stream));
+      check_bt_error(bt_gemm_f32(inter_matmul_buf, nullptr, param_.output_kernel, nullptr,
+                                 transformer_out, 0, valid_rows, packed_cap, rows_hint, hidden, inter,
+                                 stream));
+    }
     if (is_remove_padding_)
       check_bt_error(bt_add_bias_residual_layernorm_restore_f32(
           transformer_out, attr_matmul_buf, param_.output_bias, param_.output_layernorm_gamma,

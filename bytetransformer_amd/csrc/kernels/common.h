@@ -90,17 +90,17 @@ struct Launch<Kernel> {
     at += sizeof(T);
   }
   static int function(hipFunction_t *f, const char *what, bool large_lds) {
-    static std::atomic<hipFunction_t> known[kMaxDevices];
+    static std::atomic<hipFunction_t> known[2][kMaxDevices];   // with the limit as it is, and raised
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return hip_fail(e, "hipGetDevice");
     const bool kept = dev >= 0 && dev < kMaxDevices;
-    if (kept && (*f = known[dev].load(std::memory_order_acquire))) return BT_OK;
+    if (kept && (*f = known[large_lds][dev].load(std::memory_order_acquire))) return BT_OK;
     if (large_lds &&
         (e = hipFuncSetAttribute((const void *)Kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMostLds)) != hipSuccess)
       return hip_fail(e, what);
     if ((e = hipGetFuncBySymbol(f, (const void *)Kernel)) != hipSuccess) return hip_fail(e, what);
-    if (kept) known[dev].store(*f, std::memory_order_release);
+    if (kept) known[large_lds][dev].store(*f, std::memory_order_release);
     return BT_OK;
   }
 };
@@ -170,10 +170,24 @@ __device__ __forceinline__ float wave_sum(float v) {
 #endif
 }
 
+// Largest over the 64 lanes of values that are not negative, wave-uniform, by the same steps.
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
+#if defined(__HIP_DEVICE_COMPILE__)
+  const auto moved = [](float x, auto ctrl, auto rows) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), decltype(ctrl)::value,
+                                                                 decltype(rows)::value, 0xf, true));
+  };
+  using all = std::integral_constant<int, 0xf>;
+  v = fmaxf(v, moved(v, std::integral_constant<int, 0x111>{}, all{}));
+  v = fmaxf(v, moved(v, std::integral_constant<int, 0x112>{}, all{}));
+  v = fmaxf(v, moved(v, std::integral_constant<int, 0x114>{}, all{}));
+  v = fmaxf(v, moved(v, std::integral_constant<int, 0x118>{}, all{}));
+  v = fmaxf(v, moved(v, std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{}));
+  v = fmaxf(v, moved(v, std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{}));
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
+#else
   return v;
+#endif
 }
 
 // ---- wave-uniform values ----------------------------------------------------

@@ -1,0 +1,47 @@
+// Floats as scaled pairs of fp16 numbers (fp32_split.hip says what they are): shared by the launches that make them.
+#pragma once
+#include "common.h"
+
+namespace bt {
+
+constexpr int kSplitChunk = 256;   // values of a weight's column that share a scale
+constexpr float kSplitLow = 1.0f / 2048.0f;   // what a pair's second number is worth
+
+struct SplitPair {
+  half_t h, l;
+};
+// of a scaled value: the second number is zero where the first is not finite
+__device__ __forceinline__ SplitPair split_pair(float x) {
+  const half_t h = (half_t)x;
+  const float rest = (x - (float)h) * 2048.0f;
+  return SplitPair{h, __builtin_fabsf((float)h) < __builtin_inff() ? (half_t)rest : (half_t)0.f};
+}
+// The exponent that brings a largest value m >= 0 to [2^14, 2^15) (0 for no value at all), held where 2^e is a float.
+__device__ __forceinline__ int split_exponent(float m) {
+  const int e = 14 + 127 - (int)(__builtin_bit_cast(unsigned, m) >> 23);
+  return m == 0.f ? 0 : min(e, 126);   // (at least -113: m is finite)
+}
+__device__ __forceinline__ float split_power(int e) { return __builtin_bit_cast(float, (unsigned)(e + 127) << 23); }
+
+// Four scaled values (float4 c of a row) into the row's pairs.
+__device__ __forceinline__ void split_store(half_t *row, int c, float4_t x) {
+  half4_t h, l;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const SplitPair p = split_pair(x[e]);
+    h[e] = p.h, l[e] = p.l;
+  }
+  half_t *to = row + (c >> 3) * 64 + (c & 7) * 4;
+  store_through(to, __builtin_bit_cast(uint2_t, h));
+  store_through(to + 32, __builtin_bit_cast(uint2_t, l));
+}
+
+// 0.5 x (1 + tanh(u)) == x / (1 + exp(-2u)),  u = 0.79788456 (x + 0.044715 x^3), the exponent folded into one polynomial
+__device__ __forceinline__ float f32_gelu(float x) {
+  constexpr float c1 = -2.0f * 0.7978845608028654f * 1.4426950408889634f;
+  constexpr float c3 = c1 * 0.044715f;
+  const float e = __builtin_amdgcn_exp2f(x * (c1 + c3 * x * x));
+  return x * __builtin_amdgcn_rcpf(1.0f + e);
+}
+
+}  // namespace bt

@@ -19,7 +19,7 @@
 // fp32 MFMA runs at 1/16 of the bf16 rate: the products of the linear layers multiply each float as
 // a sum of three bfloat16 instead (see below), the attention stays on v_mfma_f32_32x32x2_f32, compute
 // bound with a trivial memory system (one LDS buffer pair, register-staged global loads).
-#include "common.h"
+#include "f32_split.h"
 
 namespace bt {
 
@@ -29,15 +29,6 @@ namespace {
 
 constexpr float kLog2eF = 1.4426950408889634f;
 constexpr float kDeadLogit = -1.0e30f;
-
-__device__ __forceinline__ float gelu_tanh(float x) {
-  // 0.5 x (1 + tanh(u)) == x / (1 + exp(-2u)),  u = 0.79788456 (x + 0.044715 x^3)
-  // exponent folded into one polynomial: -2 u log2(e) = x (c1 + c3 x^2)
-  constexpr float c1 = -2.0f * 0.7978845608028654f * 1.4426950408889634f;
-  constexpr float c3 = c1 * 0.044715f;
-  const float e = __builtin_amdgcn_exp2f(x * (c1 + c3 * x * x));
-  return x * __builtin_amdgcn_rcpf(1.0f + e);
-}
 
 // ---------------------------------------------------------------------------
 // float operands as bfloat16 triples
@@ -180,7 +171,7 @@ __device__ __forceinline__ void f32_store_block(const F32GemmArgs &p, const floa
     range.add(sum[0]);
     if (!range.split_held()) f32_dot_again(f32_a_row(p, row), p.w + col, p.K, p.N, sum);
     float v = sum[0] + bv;
-    if (p.gelu) v = gelu_tanh(v);
+    if (p.gelu) v = f32_gelu(v);
     p.c[(size_t)row * p.N + col] = v;
   }
 }
@@ -440,7 +431,7 @@ __device__ __forceinline__ void f32_gemm_tile(const F32GemmArgs &p) {
     if (p.bias) v[i] += float4_t{p.bias[n], p.bias[n + 1], p.bias[n + 2], p.bias[n + 3]};
     if (p.gelu) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[i][e] = gelu_tanh(v[i][e]);
+      for (int e = 0; e < 4; ++e) v[i][e] = f32_gelu(v[i][e]);
     }
     store_through(p.c + (size_t)m * p.N + n, __builtin_bit_cast(uint4_t, v[i]));
   }
@@ -774,14 +765,24 @@ __global__ __launch_bounds__(64 * NW, 2) void f32_attention_kernel(F32AttArgs p)
 // ---------------------------------------------------------------------------
 constexpr int kF32LnRows = 4;
 
+// What a LayerNorm whose rows the next product reads as pairs writes beside them.
+struct F32LnPairs {
+  half_t *pairs;         // [rows][H / 32][64]
+  int *exps;             // [rows]
+  // exponents for the pairs of GELU(row . W + bias): |row . w| is at most |row|_2 sqrt(H) max |w|
+  int *gelu_exps;        // [rows]
+  const float *bounds;   // [bound_count][2]: largest |w| and |bias| of some columns each
+  int bound_count;
+};
+
 // One wave per row, float4 per lane, the row in registers between the two passes.
-template <int NC, bool RESTORE>
-__global__ __launch_bounds__(kF32LnRows *kWave) void f32_layernorm_kernel(
+template <int NC, bool RESTORE, bool PAIRS>
+__device__ __forceinline__ void f32_layernorm_block(
     const float4_t *src, const float4_t *__restrict__ residual, const float4_t *__restrict__ bias,
     const float4_t *__restrict__ gamma, const float4_t *__restrict__ beta, float4_t *dst,
     const int *__restrict__ idx, const int *__restrict__ residual_row_index, int S, int rows_cap,
-    int chunks, float inv_n, float eps) {
-  const int r = blockIdx.x * kF32LnRows + (threadIdx.x >> 6);
+    int chunks, float inv_n, float eps, const F32LnPairs &next) {
+  const int r = blockIdx.x * kF32LnRows + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (r >= rows_cap) return;
   // what no loaded value points at is requested first: behind the statistics, gamma and beta were one more
@@ -836,19 +837,65 @@ __global__ __launch_bounds__(kF32LnRows *kWave) void f32_layernorm_kernel(
   }
   const float rstd = rsqrtf(wave_sum(sq) * inv_n + eps);
   float4_t *o = dst + (size_t)r * chunks;
+  float most = 0.f, norm = 0.f;
 #pragma unroll
   for (int i = 0; i < NC; ++i) {
     const int c = lane + i * kWave;
-    if (c < chunks)
-      store_through(o + c, __builtin_bit_cast(uint4_t, v[i] * rstd * (kEarly ? gamma_v[i] : gamma[c]) +
-                                                           (kEarly ? beta_v[i] : beta[c])));
+    if (c >= chunks) continue;
+    v[i] = v[i] * rstd * (kEarly ? gamma_v[i] : gamma[c]) + (kEarly ? beta_v[i] : beta[c]);
+    store_through(o + c, __builtin_bit_cast(uint4_t, v[i]));
+    if (PAIRS)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float x = __builtin_fabsf(v[i][e]);
+        most = fmaxf(most, x < __builtin_inff() ? x : 0.f);
+        norm += v[i][e] * v[i][e];
+      }
   }
+  if (PAIRS) {
+    float w_most = 0.f, bias_most = 0.f;
+    for (int i = lane; i < next.bound_count; i += kWave) {
+      w_most = fmaxf(w_most, next.bounds[2 * i]);
+      bias_most = fmaxf(bias_most, next.bounds[2 * i + 1]);
+    }
+    const int e = split_exponent(wave_max(most));
+    const float scale = split_power(e);
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+      const int c = lane + i * kWave;
+      if (c < chunks) split_store(next.pairs + (size_t)r * chunks * 8, c, v[i] * scale);
+    }
+    // (where the bound is not finite neither are the results, or all of them are zero)
+    const float bound = sqrtf(wave_sum(norm) * (float)(chunks * 4)) * wave_max(w_most) + wave_max(bias_most);
+    if (lane == 0) {
+      next.exps[r] = e;
+      next.gelu_exps[r] = bound < __builtin_inff() ? split_exponent(bound) : 0;
+    }
+  }
+}
+
+template <int NC, bool RESTORE>
+__global__ __launch_bounds__(kF32LnRows *kWave) void f32_layernorm_kernel(
+    const float4_t *src, const float4_t *residual, const float4_t *bias, const float4_t *gamma, const float4_t *beta,
+    float4_t *dst, const int *idx, const int *residual_row_index, int S, int rows_cap, int chunks, float inv_n,
+    float eps) {
+  f32_layernorm_block<NC, RESTORE, false>(src, residual, bias, gamma, beta, dst, idx, residual_row_index, S, rows_cap, chunks,
+                                          inv_n, eps, F32LnPairs{});
+}
+template <int NC>
+__global__ __launch_bounds__(kF32LnRows *kWave) void f32_layernorm_pairs_kernel(
+    const float4_t *src, const float4_t *residual, const float4_t *bias, const float4_t *gamma, const float4_t *beta,
+    float4_t *dst, const int *idx, const int *residual_row_index, int rows_cap, int chunks, float inv_n, float eps,
+    F32LnPairs next) {
+  f32_layernorm_block<NC, false, true>(src, residual, bias, gamma, beta, dst, idx, residual_row_index, 1, rows_cap, chunks, inv_n,
+                                       eps, next);
 }
 
 template <bool RESTORE>
 int launch_f32_ln(const void *src, const void *residual, const void *bias, const void *gamma,
                   const void *beta, void *dst, const int *idx, const int *residual_row_index,
-                  int S, int rows_cap, int H, float eps, hipStream_t s, const char *who) {
+                  int S, int rows_cap, int H, float eps, hipStream_t s, const char *who,
+                  const F32LnPairs *next = nullptr) {
   BT_REQUIRE(H > 0 && H % 4 == 0, BT_ERR_UNSUPPORTED, "%s: hidden_dim %d must be a multiple of 4",
              who, H);
   BT_REQUIRE(aligned16({src, residual, bias, gamma, beta, dst}), BT_ERR_INVALID_ARGUMENT,
@@ -860,6 +907,12 @@ int launch_f32_ln(const void *src, const void *residual, const void *bias, const
   const int grid = (rows_cap + kF32LnRows - 1) / kF32LnRows;
   const float inv_n = 1.0f / (float)H;
   const auto with = [&](auto nc_tag) {
+    if constexpr (!RESTORE)
+      if (next)
+        return Launch<f32_layernorm_pairs_kernel<nc_tag()>>::on(
+            s, who, grid, kF32LnRows * kWave, 0, (const float4_t *)src, (const float4_t *)residual, (const float4_t *)bias,
+            (const float4_t *)gamma, (const float4_t *)beta, (float4_t *)dst, idx, residual_row_index, rows_cap, chunks,
+            inv_n, eps, *next);
     return Launch<f32_layernorm_kernel<nc_tag(), RESTORE>>::on(
         s, who, grid, kF32LnRows * kWave, 0, (const float4_t *)src, (const float4_t *)residual, (const float4_t *)bias,
         (const float4_t *)gamma, (const float4_t *)beta, (float4_t *)dst, idx, residual_row_index, S, rows_cap, chunks,
@@ -991,6 +1044,22 @@ extern "C" int bt_add_bias_residual_layernorm_f32(void *out, const void *residua
   return launch_f32_ln<false>(out, residual, bias, gamma, beta, out, valid_rows,
                               residual_row_index, 1, rows_cap, hidden_dim, eps, as_stream(stream),
                               "bt_add_bias_residual_layernorm_f32");
+}
+
+extern "C" int bt_add_bias_residual_layernorm_f32_split(
+    void *out, const void *residual, const int *residual_row_index, const void *bias, const void *gamma, const void *beta,
+    const int *valid_rows, int rows_cap, int hidden_dim, float eps, void *pairs, int *exps, int *gelu_exps, const float *bounds,
+    int bound_count, void *stream) {
+  const char *who = "bt_add_bias_residual_layernorm_f32_split";
+  BT_REQUIRE(out && residual && bias && gamma && beta && pairs && exps && gelu_exps && bounds, BT_ERR_INVALID_ARGUMENT,
+             "%s: null pointer argument", who);
+  BT_REQUIRE(rows_cap >= 0 && bound_count > 0, BT_ERR_INVALID_ARGUMENT, "%s: rows_cap=%d bound_count=%d", who, rows_cap, bound_count);
+  BT_REQUIRE(!residual_row_index || valid_rows, BT_ERR_INVALID_ARGUMENT, "%s: residual_row_index needs valid_rows", who);
+  BT_REQUIRE(hidden_dim % 32 == 0 && aligned16({pairs}), BT_ERR_UNSUPPORTED,
+             "%s: hidden_dim=%d must be a multiple of 32, the pairs 16-byte aligned", who, hidden_dim);
+  const F32LnPairs next{(half_t *)pairs, exps, gelu_exps, bounds, bound_count};
+  return launch_f32_ln<false>(out, residual, bias, gamma, beta, out, valid_rows, residual_row_index, 1, rows_cap, hidden_dim,
+                              eps, as_stream(stream), who, &next);
 }
 
 extern "C" int bt_add_bias_residual_layernorm_restore_f32(

@@ -1,0 +1,567 @@
+// The products of the float layer on fp16 matrix instructions, for batches whose operands are worth splitting
+// once: every operand is stored as pairs of fp16 numbers by the launch that makes it, and the products are the
+// tiled fp16 products' twins with three matrix instructions where those have one.
+//
+//   split_f32_kernel       weights [K, N] and gathered rows of the input -> their pairs, k-contiguous
+//   f32_split_gemm_kernel  c = a . w (+ bias), or the pairs of GELU(a . w + bias)
+//   f32_layernorm_split    (fp32_path.hip) writes the pairs of its rows beside the rows
+//
+// The pair.  A row (or 256 consecutive values of a weight's column) is scaled by a power of two that brings its largest value to [2^14, 2^15);
+// of x so scaled, h = fp16(x) and l = fp16((x - h) 2^11), round to nearest.  x - h is exact and at most 2^-11 |x|,
+// so h + l / 2^11 is x to 2^-23 of its own (three floats in four exactly), and since l has the exponent range of h
+// that holds down to 2^-27 of the largest value; what is smaller still is off by 2^-50 of that value at most
+// (h and l are subnormal there: off by 2^-25 in l, 2^-36 of a value scaled to 2^14 or more).
+// a . w is then the sum of ah wh and of (ah wl + al wh) / 2^11, each in float accumulators of its own; al wl, 2^-22
+// of a product, is left out.  Against the exact bfloat16 triples of bt_gemm_f32 (six matrix instructions, one
+// accumulator) the operands are rounded, but the sums are half to a sixth as many roundings: see
+// bt_gemm_f32_split in bt_hip.h for both errors.
+// Infinities and NaN keep their places in h (the scale comes from the finite values of a row); a sum that is not
+// finite is formed again from the pairs by float multiply-adds.
+//
+// In memory a row of K floats is K / 32 blocks of 128 bytes: 32 h, then 32 l.  A block is one k-step's row of an
+// LDS tile, so loads, swizzle and LDS reads are those of an fp16 product of 2 K halfs.
+#include "f32_split.h"
+#include "gemm_common.h"
+
+#include <cmath>
+
+namespace bt {
+namespace {
+
+typedef int int4_t __attribute__((ext_vector_type(4)));
+
+// ---------------------------------------------------------------------------
+// operands -> pairs
+// ---------------------------------------------------------------------------
+// A unit of a weight: 32 columns x 256 rows, which it reads once and scales by their own largest values.  (With one scale
+// for a whole column every unit had to see all of its rows first: 28.6 us for the weights of a layer of hidden 768 out of
+// HBM.)  What bounds it is the memory: 28 MB in and out.
+constexpr int kSplitThreads = 512, kSplitCols = 32;
+constexpr int kSplitPitch = 2 * kSplitChunk + 8;   // halfs of a column's rows in LDS
+
+struct SplitWeight {
+  const float *w;     // [K, N]
+  half_t *pairs;      // [N][K / 32][64]
+  int *exps;          // [ceil(K / 256)][N]
+  int K, N, strips, unit_end;
+};
+struct SplitArgs {
+  SplitWeight weight[4];
+  int count, units;
+  int bounded;              // the weight that `bounds` speaks of, -1: none
+  const float *bias;        // [N] its bias
+  float *bounds;            // [units of that weight][2]: largest |w| and largest |bias| of its columns
+  const float *rows;        // rows to split as well, or null
+  half_t *row_pairs;        // [rows_cap][K / 32][64]
+  int *row_exps;
+  const int *row_index, *valid_rows;
+  int rows_cap, hidden;
+};
+
+__device__ __forceinline__ float finite_or_zero(float x) {
+  return (__builtin_bit_cast(unsigned, x) & 0x7f800000u) == 0x7f800000u ? 0.f : __builtin_fabsf(x);
+}
+
+__device__ __forceinline__ void split_weight_unit(const SplitArgs &a, int unit) {
+  constexpr int kPasses = kSplitChunk / (kSplitThreads / 8);   // 64 rows each
+  __shared__ float4_t s_most[kSplitThreads / 64][8];
+  __shared__ float s_scale[kSplitCols];
+  __shared__ __attribute__((aligned(16))) half_t s_tile[kSplitCols * kSplitPitch];
+  int j = 0, first = 0;
+#pragma unroll
+  for (int i = 1; i < 4; ++i)
+    if (i < a.count && unit >= a.weight[i - 1].unit_end) j = i, first = a.weight[i - 1].unit_end;
+  const SplitWeight jb = a.weight[j];
+  const int u = unit - first, chunk = u / jb.strips, strip = u - chunk * jb.strips;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int cq = t & 7, r0 = t >> 3, n0 = strip * kSplitCols, k0 = chunk * kSplitChunk;
+  const float4_t *src = (const float4_t *)(jb.w + n0) + cq;
+
+  // thread: four columns of rows r0, r0 + 64, ... (K is a multiple of 64)
+  float4_t v[kPasses];
+#pragma unroll
+  for (int i = 0; i < kPasses; ++i) {
+    v[i] = float4_t{0.f, 0.f, 0.f, 0.f};
+    if (k0 + 64 * i < jb.K) v[i] = src[(size_t)(k0 + 64 * i + r0) * (jb.N / 4)];
+  }
+  float4_t most = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < kPasses; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) most[e] = fmaxf(most[e], finite_or_zero(v[i][e]));
+#pragma unroll
+  for (int o = 8; o < 64; o <<= 1)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) most[e] = fmaxf(most[e], __shfl_xor(most[e], o, 64));
+  if (lane < 8) s_most[wave][lane] = most;
+  __syncthreads();
+  if (t < kSplitCols) {
+    float m = 0.f;
+#pragma unroll
+    for (int w = 0; w < kSplitThreads / 64; ++w) m = fmaxf(m, s_most[w][t >> 2][t & 3]);
+    const int e = split_exponent(m);
+    s_scale[t] = split_power(e);
+    jb.exps[(size_t)chunk * jb.N + n0 + t] = e;
+    if (j == a.bounded) {
+      float b = __builtin_fabsf(a.bias[n0 + t]);
+#pragma unroll
+      for (int o = 1; o < 32; o <<= 1) m = fmaxf(m, __shfl_xor(m, o, 64)), b = fmaxf(b, __shfl_xor(b, o, 64));
+      if (t == 0) a.bounds[2 * u] = m, a.bounds[2 * u + 1] = b;
+    }
+  }
+  __syncthreads();
+  float scale[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) scale[e] = s_scale[4 * cq + e];
+#pragma unroll
+  for (int i = 0; i < kPasses; ++i) {
+    half_t *to = s_tile + (64 * i + (r0 & 32)) * 2 + (r0 & 31);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const SplitPair p = split_pair(v[i][e] * scale[e]);
+      to[(4 * cq + e) * kSplitPitch] = p.h;
+      to[(4 * cq + e) * kSplitPitch + 32] = p.l;
+    }
+  }
+  __syncthreads();
+  const int rows = min(kSplitChunk, jb.K - k0), chunks16 = rows / 4;   // 16-byte pieces of a column
+  for (int at = t; at < kSplitCols * (kSplitChunk / 4); at += kSplitThreads) {
+    const int n = at / (kSplitChunk / 4), c = at % (kSplitChunk / 4);
+    if (c < chunks16)
+      store_through(jb.pairs + (size_t)(n0 + n) * 2 * jb.K + 2 * k0 + c * 8, *(const uint4_t *)(s_tile + n * kSplitPitch + c * 8));
+  }
+}
+
+__global__ __launch_bounds__(kSplitThreads) void split_f32_kernel(SplitArgs a) {
+  if ((int)blockIdx.x < a.units) return split_weight_unit(a, blockIdx.x);
+  const int r = ((int)blockIdx.x - a.units) * (kSplitThreads / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int M = a.valid_rows ? min(scalar_load(a.valid_rows), a.rows_cap) : a.rows_cap;
+  if (r >= M) return;
+  const size_t from = a.row_index ? (size_t)scalar_load(a.row_index + r) : (size_t)r;
+  const float4_t *src = (const float4_t *)(a.rows + from * a.hidden);
+  float most = 0.f;
+  for (int c = lane; c < a.hidden / 4; c += 64) {
+    const float4_t v = src[c];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) most = fmaxf(most, finite_or_zero(v[e]));
+  }
+  const int e = split_exponent(wave_max(most));
+  if (lane == 0) a.row_exps[r] = e;
+  const float scale = split_power(e);
+  for (int c = lane; c < a.hidden / 4; c += 64) split_store(a.row_pairs + (size_t)r * 2 * a.hidden, c, src[c] * scale);
+}
+
+// ---------------------------------------------------------------------------
+// products
+// ---------------------------------------------------------------------------
+struct F32SplitTail {
+  const float *bias;   // [N] or null
+  const int *gelu_exps;   // GELU: exponent that a row of the result is scaled by
+};
+#define BT_F32_SPLIT_FIRST                                                                                  \
+  const half_t *a, const half_t *w, const int *valid_rows, const int *a_exps, const int *w_exps, void *out, \
+      int rows_cap, int N, int K, unsigned per_n
+
+#if defined(__HIP_DEVICE_COMPILE__)
+// A sum from the pairs themselves, k in order, by float multiply-adds (infinities and NaN among the operands).
+__device__ __forceinline__ float split_dot(const half_t *a, int a_exp, const half_t *w, const int *w_exp, int N, int K) {
+  float sum = 0.f;
+  for (int b = 0; b < K / 32; ++b) {
+    const int e = w_exp[(size_t)(b * 32 / kSplitChunk) * N];
+    for (int k = 0; k < 32; ++k) {
+      const float x = (float)a[b * 64 + k] + (float)a[b * 64 + 32 + k] * kSplitLow;
+      const float y = (float)w[b * 64 + k] + (float)w[b * 64 + 32 + k] * kSplitLow;
+      sum = __builtin_fmaf(__builtin_amdgcn_ldexpf(x, -a_exp), __builtin_amdgcn_ldexpf(y, -e), sum);
+    }
+  }
+  return sum;
+}
+
+// BM x BN tile, WM x WN waves that load and multiply, a ring of STAGES k-steps of 32 floats.  A wave's step is
+// 3 TM TN matrix instructions on 2 (TM + TN) LDS reads: the matrix pipe is what it waits for, from 64 x 64 a wave on.
+template <int BM, int BN, int WM, int WN, int KG, int STAGES, bool GELU>
+__device__ __forceinline__ void f32_split_tile(BT_F32_SPLIT_FIRST, const F32SplitTail &tail) {
+  constexpr int NG = WM * WN, NW = NG * KG, WTM = BM / WM, WTN = BN / WN, TM = WTM / 16, TN = WTN / 16;
+  constexpr int NI = (BM + BN) / 8 / NG, NIA = BM / 8 / NG;   // every group loads its own k-steps
+  constexpr int STEP_HALFS = (BM + BN) * kBK, STAGE_HALFS = KG * STEP_HALFS;
+  static_assert(BM % (8 * NG) == 0 && BN % (8 * NG) == 0, "tile rows must split evenly over the waves");
+  static_assert(WTN % 32 == 0, "whole blocks of pairs");
+  extern __shared__ __attribute__((aligned(1024))) half_t split_smem[];
+  const int lane = threadIdx.x & 63;
+  const int wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int group = KG > 1 ? wave_all / NG : 0, wave = wave_all % NG;
+  const int M = valid_rows ? min(scalar_load(valid_rows), rows_cap) : rows_cap;
+  int tile_m, tile_n;
+  {
+    // XCD x works on a contiguous range of the live tiles
+    const int tiles_n = (N + BN - 1) / BN, live = (M + BM - 1) / BM * tiles_n, per = (live + 7) >> 3;
+    const int bid = (int)blockIdx.x, L = (bid & 7) * per + (bid >> 3);
+    if (bid >= per * 8 || L >= live) return;
+    tile_m = (int)divide((unsigned)L, (unsigned)tiles_n, per_n);
+    tile_n = L - tile_m * tiles_n;
+  }
+  const int m0 = tile_m * BM, n0 = tile_n * BN, nk = K / 32 / KG;   // k-steps of a group: group, group + KG, ...
+  const size_t pitch = 2 * (size_t)K;   // halfs
+  const rsrc_t rs_a = make_rsrc(a + m0 * pitch, (rows_cap - m0) * pitch * sizeof(half_t));
+  const rsrc_t rs_w = make_rsrc(w + n0 * pitch, (N - n0) * pitch * sizeof(half_t));
+  int voff[NI];
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int r = (i * NG + wave) * 8 + (lane >> 3);
+    voff[i] = ((i < NIA ? r : r - BM) * 2 * K + (((lane & 7) ^ swz(r)) << 3)) * (int)sizeof(half_t);
+  }
+  auto issue = [&](int kt, int stage) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          i < NIA ? rs_a : rs_w,
+          (__attribute__((address_space(3))) void *)(split_smem + stage * STAGE_HALFS + group * STEP_HALFS + (i * NG + wave) * 8 * kBK),
+          16, voff[i], (kt * KG + group) * kBK * (int)sizeof(half_t), 0, 0);
+  };
+#pragma unroll
+  for (int s = 0; s < STAGES - 1; ++s)
+    if (s < nk) issue(s, s);
+
+  const int wm = wave / WN, wn = wave % WN, fr = lane & 15, lg = lane >> 4;
+  // hh, cross: the products of one chunk of the weight's column, then scaled and added to `sum`.  (In one chain over all of k
+  // the largest error of a result was up to 1.8 times that of the bfloat16 triples, whose waves share k.)
+  float4_t sum[TN][TM], hh[TN][TM], cross[TN][TM];
+  const float4_t zero4 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < TN; ++i)
+#pragma unroll
+    for (int j = 0; j < TM; ++j) sum[i][j] = hh[i][j] = cross[i][j] = zero4;
+  // The weight's scales: behind the ring, factor[c][n] = 2^(e - exponent of chunk c of column n), e[n] the smallest of the
+  // column's, so that no factor is above 1.  (They are on their way beside the first k-steps.)
+  const int chunks = (K + kSplitChunk - 1) / kSplitChunk;
+  float *factor = (float *)(split_smem + STAGES * STAGE_HALFS);
+  int *column_e = (int *)factor + chunks * BN;
+  for (int n = threadIdx.x; n < BN; n += NW * 64) {
+    const int *from = w_exps + min(n0 + n, N - 1);
+    int least = 1 << 20;
+    for (int c = 0; c < chunks; ++c) {
+      const int e = from[(size_t)c * N];
+      least = min(least, e);
+      ((int *)factor)[c * BN + n] = e;
+    }
+    for (int c = 0; c < chunks; ++c) factor[c * BN + n] = __builtin_amdgcn_ldexpf(1.f, least - ((int *)factor)[c * BN + n]);
+    column_e[n] = least;
+  }
+  __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): there, behind the first barrier of the loop
+  constexpr int kFold = kSplitChunk / 32 / KG;   // k-steps of a group in a chunk
+  const float *my_factor = factor + wn * WTN + 4 * lg;
+  auto fold = [&](int chunk) {
+#pragma unroll
+    for (int i = 0; i < TN; ++i) {
+      const float4_t f = *(const float4_t *)(my_factor + chunk * BN + 16 * i);
+#pragma unroll
+      for (int j = 0; j < TM; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          sum[i][j][e] = __builtin_fmaf(__builtin_fmaf(cross[i][j][e], kSplitLow, hh[i][j][e]), f[e], sum[i][j][e]);
+    }
+  };
+  // (swz does not depend on the 16-row block, so a fragment's address is this plus a constant)
+  const int at_h = fr * kBK + ((lg ^ swz(fr)) << 3), at_l = fr * kBK + (((4 + lg) ^ swz(fr)) << 3);
+
+  int stage = 0;
+  for (int kt = 0; kt < nk; ++kt) {
+    if (kt % kFold == 0 && kt > 0) {
+      fold(kt / kFold - 1);
+#pragma unroll
+      for (int i = 0; i < TN; ++i)
+#pragma unroll
+        for (int j = 0; j < TM; ++j) hh[i][j] = cross[i][j] = zero4;
+    }
+    wait_stages<NI, STAGES - 2>(nk - 1 - kt);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();   // k-step kt is in LDS; the stage of the step before is free
+    asm volatile("" ::: "memory");
+    if (kt + STAGES - 1 < nk) {
+      int ps = stage + STAGES - 1;
+      if (ps >= STAGES) ps -= STAGES;
+      issue(kt + STAGES - 1, ps);
+    }
+    const half_t *sA = split_smem + stage * STAGE_HALFS + group * STEP_HALFS + wm * WTM * kBK;
+    const half_t *sW = split_smem + stage * STAGE_HALFS + group * STEP_HALFS + (BM + wn * WTN) * kBK;
+    half8_t ah[TM], al[TM], wh[2], wl[2];
+    auto read_w = [&](int i) {
+      wh[i & 1] = *(const half8_t *)(sW + i * 16 * kBK + at_h);
+      wl[i & 1] = *(const half8_t *)(sW + i * 16 * kBK + at_l);
+    };
+    auto read_a = [&](int j) {
+      ah[j] = *(const half8_t *)(sA + j * 16 * kBK + at_h);
+      al[j] = *(const half8_t *)(sA + j * 16 * kBK + at_l);
+    };
+    auto times = [&](int i, int j, int part) {   // hh, wh al, wl ah
+      float4_t &to = part ? cross[i][j] : hh[i][j];
+      to = __builtin_amdgcn_mfma_f32_16x16x32_f16(part == 2 ? wl[i & 1] : wh[i & 1], part == 1 ? al[j] : ah[j], to, 0, 0, 0);
+    };
+    // The waves of a workgroup come from their barrier together, so reads that all products wait for would leave the
+    // matrix pipe idle for as long as the LDS takes to serve them: the first column block starts on the first row block's
+    // reads, those of the others come between its products.
+    read_w(0), read_a(0);
+    times(0, 0, 0), times(0, 0, 1);
+#pragma unroll
+    for (int j = 1; j < TM; ++j) {
+      read_a(j);
+      times(0, j - 1, 2), times(0, j, 0), times(0, j, 1);
+    }
+    if (TN > 1) read_w(1);
+    times(0, TM - 1, 2);
+#pragma unroll
+    for (int i = 1; i < TN; ++i) {
+      if (i + 1 < TN) read_w(i + 1);
+#pragma unroll
+      for (int part = 0; part < 3; ++part)
+#pragma unroll
+        for (int j = 0; j < TM; ++j) times(i, j, part);
+    }
+    __builtin_amdgcn_sched_group_barrier(kSchedLdsRead, 6, 0);   // (one row block ahead)
+    __builtin_amdgcn_sched_group_barrier(kSchedMfma, 2, 0);
+    __builtin_amdgcn_sched_group_barrier(kSchedLdsRead, 2, 0);   // (of row block 2, or of column block 1)
+#pragma unroll
+    for (int j = 2; j < TM; ++j) {
+      __builtin_amdgcn_sched_group_barrier(kSchedMfma, 3, 0);
+      __builtin_amdgcn_sched_group_barrier(kSchedLdsRead, 2, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(kSchedMfma, 4, 0);
+#pragma unroll
+    for (int i = 1; i < TN; ++i) {
+      if (i + 1 < TN) {
+        __builtin_amdgcn_sched_group_barrier(kSchedMfma, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(kSchedLdsRead, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(kSchedMfma, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(kSchedLdsRead, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(kSchedMfma, 3 * TM - 2, 0);
+      } else {
+        __builtin_amdgcn_sched_group_barrier(kSchedMfma, 3 * TM, 0);
+      }
+    }
+    if (++stage == STAGES) stage = 0;
+  }
+  fold((nk - 1) / kFold);
+
+  // Two groups share the rows of their sums: each hands over the blocks that are the other's and adds what it gets.
+  constexpr int kFirstRows = KG > 1 ? (TM + 1) / 2 : TM;   // row blocks of group 0
+  static_assert(KG <= 2, "two groups at most");
+  if (KG > 1) {
+    static_assert((size_t)NG * TN * TM * 256 * sizeof(float) <= (size_t)STAGES * STAGE_HALFS * sizeof(half_t), "sums fit the ring");
+    float4_t *shared = (float4_t *)split_smem + wave * (TN * TM * 64) + lane;
+    __builtin_amdgcn_s_barrier();   // everyone is done with the ring
+#pragma unroll
+    for (int j = 0; j < TM; ++j)
+      if ((j < kFirstRows) != (group == 0))
+#pragma unroll
+        for (int i = 0; i < TN; ++i) shared[(i * TM + j) * 64] = sum[i][j];
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < TM; ++j)
+      if ((j < kFirstRows) == (group == 0))
+#pragma unroll
+        for (int i = 0; i < TN; ++i) sum[i][j] += shared[(i * TM + j) * 64];
+  }
+
+  // lane: columns n .. n + 3 of block i, row m of block j
+  int4_t ew[TN];
+  float4_t bias[TN];
+#pragma unroll
+  for (int i = 0; i < TN; ++i) {
+    const int n = min(n0 + wn * WTN + 16 * i + 4 * lg, N - 4);
+    ew[i] = *(const int4_t *)(column_e + wn * WTN + 16 * i + 4 * lg);
+    bias[i] = float4_t{0.f, 0.f, 0.f, 0.f};
+    if (tail.bias)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) bias[i][e] = tail.bias[n + e];
+  }
+  constexpr int EP = 2 * WTN + 8;   // halfs of a staged row of pairs
+  static_assert(!GELU || (size_t)NW * 16 * EP <= (size_t)STAGES * STAGE_HALFS, "staging fits the ring");
+  half_t *staged = split_smem + wave_all * 16 * EP;
+  bool finite = true;
+  if (GELU) __builtin_amdgcn_s_barrier();   // everyone is done with the ring
+#pragma unroll
+  for (int j = 0; j < TM; ++j) {
+    if (KG > 1 && (j < kFirstRows) != (group == 0)) continue;
+    const int m_first = m0 + wm * WTM + 16 * j, m = m_first + fr, m_in = min(m, M - 1);
+    const int ea = a_exps[m_in];
+    float to_pair = 1.f;
+    if (GELU) to_pair = split_power(tail.gelu_exps[m_in]);
+#pragma unroll
+    for (int i = 0; i < TN; ++i) {
+      const int n = n0 + wn * WTN + 16 * i + 4 * lg;
+      float4_t v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float s = sum[i][j][e];
+        finite = finite && __builtin_fabsf(s) < __builtin_inff();
+        v[e] = __builtin_amdgcn_ldexpf(s, -(ea + ew[i][e]));
+      }
+      v += bias[i];
+      if (!GELU) {
+        if (m < M && n < N) store_through((float *)out + (size_t)m * N + n, __builtin_bit_cast(uint4_t, v));
+        continue;
+      }
+      half4_t h, l;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const SplitPair p = split_pair(f32_gelu(v[e]) * to_pair);
+        h[e] = p.h, l[e] = p.l;
+      }
+      half_t *to = staged + fr * EP + (i >> 1) * 64 + (i & 1) * 16 + 4 * lg;
+      *(half4_t *)to = h;
+      *(half4_t *)(to + 32) = l;
+    }
+    if (GELU) {
+      constexpr int CPR = WTN / 4, RPS = 64 / CPR;   // 16-byte chunks of a row; rows per store instruction
+      static_assert(64 % CPR == 0 && 16 % RPS == 0, "whole rows");
+#pragma unroll
+      for (int r = lane / CPR; r < 16; r += RPS) {
+        const int c = lane % CPR, n = n0 + wn * WTN + (c >> 3) * 32;
+        const uint4_t v = *(const uint4_t *)(staged + r * EP + c * 8);
+        if (m_first + r < M && n < N)
+          store_through((half_t *)out + (size_t)(m_first + r) * 2 * N + (n0 + wn * WTN) * 2 + c * 8, v);
+      }
+    }
+  }
+
+  // What is not finite in its place is formed again, one sum after the other: the operands hold infinities or NaN.
+  if (__builtin_amdgcn_ballot_w64(!finite) == 0) return;
+  __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): the stores above have returned
+  for (int at = lane + (group ? kFirstRows * 16 * WTN : 0); at < (group ? WTM : kFirstRows * 16) * WTN; at += 64) {
+    const int m = m0 + wm * WTM + at / WTN, n = n0 + wn * WTN + at % WTN;
+    if (m >= M || n >= N) continue;
+    float *to = (float *)out + (size_t)m * N + n;
+    half_t *pair = (half_t *)out + (size_t)m * 2 * N + (n >> 5) * 64 + (n & 31);
+    const float have = GELU ? (float)*(volatile half_t *)pair : *(volatile float *)to;
+    if (__builtin_fabsf(have) < __builtin_inff()) continue;
+    float v = split_dot(a + m * pitch, a_exps[m], w + n * pitch, w_exps + n, N, K);
+    if (tail.bias) v += tail.bias[n];
+    if (GELU) {
+      const SplitPair p = split_pair(f32_gelu(v) * split_power(tail.gelu_exps[m]));
+      *(volatile half_t *)pair = p.h;
+      *(volatile half_t *)(pair + 32) = p.l;
+    } else {
+      *(volatile float *)to = v;
+    }
+  }
+}
+#endif  // __HIP_DEVICE_COMPILE__
+
+template <int BM, int BN, int WM, int WN, int KG, int STAGES, bool GELU>
+__global__ __launch_bounds__(WM *WN *KG * 64, 2) void f32_split_gemm_kernel(BT_F32_SPLIT_FIRST, F32SplitTail tail) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  f32_split_tile<BM, BN, WM, WN, KG, STAGES, GELU>(a, w, valid_rows, a_exps, w_exps, out, rows_cap, N, K, per_n, tail);
+#endif
+}
+
+struct F32SplitArgs {
+  const half_t *a, *w;
+  const int *valid_rows, *a_exps, *w_exps;
+  void *out;
+  int rows_cap, N, K;
+  F32SplitTail tail;
+};
+template <int BM, int BN, int KG, int STAGES>
+size_t f32_split_lds(int k) {
+  return (size_t)KG * STAGES * (BM + BN) * kBK * sizeof(half_t) + (size_t)((k + kSplitChunk - 1) / kSplitChunk + 1) * BN * 4;
+}
+template <int BM, int BN, int WM, int WN, int KG, int STAGES>
+int launch_f32_split(const F32SplitArgs &p, hipStream_t s) {
+  const size_t smem = f32_split_lds<BM, BN, KG, STAGES>(p.K);
+  const int tiles_n = (p.N + BN - 1) / BN;
+  const unsigned grid = (unsigned)(((long long)((p.rows_cap + BM - 1) / BM) * tiles_n + 7) / 8 * 8);
+  const auto with = [&](auto gelu) {
+    return Launch<f32_split_gemm_kernel<BM, BN, WM, WN, KG, STAGES, gelu()>>::on(
+        s, "f32_split_gemm_kernel", grid, WM * WN * KG * 64, smem, p.a, p.w, p.valid_rows, p.a_exps, p.w_exps, p.out, p.rows_cap, p.N,
+        p.K, inverse_of((unsigned)tiles_n), p.tail);
+  };
+  return p.tail.gelu_exps ? with(std::true_type{}) : with(std::false_type{});
+}
+
+}  // namespace
+}  // namespace bt
+
+using namespace bt;
+
+extern "C" int bt_split_f32(int weight_count, const void *const *w, void *const *w_pairs, int *const *w_exps, const int *k,
+                            const int *n, int bounded, const void *bounded_bias, float *bounds, const void *rows,
+                            void *row_pairs, int *row_exps, const int *row_index, const int *valid_rows, int rows_cap,
+                            int hidden_dim, void *stream) {
+  const char *who = "bt_split_f32";
+  BT_REQUIRE(weight_count >= 0 && weight_count <= 4, BT_ERR_INVALID_ARGUMENT, "%s: weight_count=%d outside [0, 4]", who, weight_count);
+  BT_REQUIRE(weight_count == 0 || (w && w_pairs && w_exps && k && n), BT_ERR_INVALID_ARGUMENT, "%s: null pointer argument", who);
+  BT_REQUIRE(bounded < weight_count && (bounded < 0 || (bounded_bias && bounds)), BT_ERR_INVALID_ARGUMENT,
+             "%s: bounded=%d needs a weight, its bias and an array of bounds", who, bounded);
+  SplitArgs a{};
+  int units = 0;
+  for (int i = 0; i < weight_count; ++i) {
+    BT_REQUIRE(w[i] && w_pairs[i] && w_exps[i], BT_ERR_INVALID_ARGUMENT, "%s: null pointer of matrix %d", who, i);
+    BT_REQUIRE(aligned16({w[i], w_pairs[i], w_exps[i]}), BT_ERR_INVALID_ARGUMENT, "%s: pointers must be 16-byte aligned", who);
+    BT_REQUIRE(k[i] > 0 && n[i] > 0 && k[i] % 64 == 0 && n[i] % kSplitCols == 0, BT_ERR_UNSUPPORTED,
+               "%s: k=%d must be a multiple of 64 and n=%d of 32", who, k[i], n[i]);
+    const int strips = n[i] / kSplitCols;
+    units += strips * ((k[i] + kSplitChunk - 1) / kSplitChunk);
+    a.weight[i] = SplitWeight{(const float *)w[i], (half_t *)w_pairs[i], w_exps[i], k[i], n[i], strips, units};
+  }
+  a.count = weight_count, a.units = units;
+  a.bounded = bounded < 0 ? -1 : bounded, a.bias = (const float *)bounded_bias, a.bounds = bounds;
+  int row_blocks = 0;
+  if (rows) {
+    BT_REQUIRE(row_pairs && row_exps && row_pairs != rows, BT_ERR_INVALID_ARGUMENT, "%s: rows need an area of their own for the pairs", who);
+    BT_REQUIRE(aligned16({rows, row_pairs}), BT_ERR_INVALID_ARGUMENT, "%s: pointers must be 16-byte aligned", who);
+    BT_REQUIRE(rows_cap >= 0 && hidden_dim > 0 && hidden_dim % 32 == 0, BT_ERR_UNSUPPORTED,
+               "%s: hidden_dim=%d must be a multiple of 32", who, hidden_dim);
+    BT_REQUIRE(!row_index || valid_rows, BT_ERR_INVALID_ARGUMENT, "%s: row_index needs valid_rows", who);
+    a.rows = (const float *)rows, a.row_pairs = (half_t *)row_pairs, a.row_exps = row_exps;
+    a.row_index = row_index, a.valid_rows = valid_rows, a.rows_cap = rows_cap, a.hidden = hidden_dim;
+    row_blocks = (rows_cap + kSplitThreads / 64 - 1) / (kSplitThreads / 64);
+  }
+  if (units + row_blocks == 0) return BT_OK;
+  return Launch<split_f32_kernel>::on(as_stream(stream), who, units + row_blocks, kSplitThreads, 0, a);
+}
+
+extern "C" int bt_gemm_f32_split(const void *a_pairs, const int *a_exps, const void *w_pairs, const int *w_exps, const void *bias,
+                                 void *c, const int *gelu_exps, const int *valid_rows, int rows_cap, int n, int k,
+                                 void *stream) {
+  const char *who = "bt_gemm_f32_split";
+  BT_REQUIRE(a_pairs && a_exps && w_pairs && w_exps && c, BT_ERR_INVALID_ARGUMENT, "%s: null pointer argument", who);
+  BT_REQUIRE(aligned16({a_pairs, w_pairs, w_exps, c}), BT_ERR_INVALID_ARGUMENT, "%s: pointers must be 16-byte aligned", who);
+  BT_REQUIRE(rows_cap >= 0 && n > 0 && k > 0 && n % 32 == 0 && k % 64 == 0, BT_ERR_UNSUPPORTED,
+             "%s: n=%d must be a multiple of 32 and k=%d of 64", who, n, k);
+  BT_REQUIRE(k <= (1 << 14), BT_ERR_UNSUPPORTED, "%s: k=%d is beyond 2^14", who, k);   // (the scales of its chunks lie in LDS)
+  BT_REQUIRE(!gelu_exps || bias, BT_ERR_INVALID_ARGUMENT, "%s: gelu needs a bias", who);
+  if (rows_cap == 0) return BT_OK;
+  const F32SplitArgs p{(const half_t *)a_pairs, (const half_t *)w_pairs, valid_rows, a_exps, w_exps, c, rows_cap, n, k,
+                       {(const float *)bias, gelu_exps}};
+  hipStream_t s = as_stream(stream);
+  // Tiles: 0: 64x64, two groups of waves over k, two workgroups a CU | 1: 64x128 likewise, one | 2: 96x128, one group, two.
+  // What a step waits for is its operands: a CU takes in about 40 bytes a clock from the L2 and reads 128 from the LDS, and
+  // the larger the tile the fewer it needs, as long as no CU goes without.  us at 2458 rows of hidden 768, bt_gemm_f32 and
+  // tiles 0 / 1 / 2: QKV 62 and 43 / 51 / 32, projection 21 and 14.0 / 13.4 / 20.5, FFN1 79 and 59 / 67 / 51, FFN2 73 and 42 /
+  // 48 / 65.  (256x128, eight waves: 38 / 33 / 41 / 103, but 75 for FFN1 from 2561 rows on, a second round, and no
+  // registers to spare; 128x128, eight waves: 44 / 21 / 46 / 63.)  A launch is priced by its rounds of the chip, a last one
+  // that is partly full where two workgroups share a CU at half of one and half of its share: 5 us less than these
+  // and those of 600 and 4915 rows, give or take 15 %.  The groups add up in another order, so the choice follows from sizes
+  // alone, never from a row hint; a padded batch counts as 60 % full, give or take a fifth.
+  int tile = option_f32_gemm_tile();
+  if (tile < 0 || tile > 2) {
+    struct Candidate { int bm, bn, per_cu; float step, fixed; };   // of a round: us per 64 of k, and besides
+    static const Candidate candidates[3] = {{64, 64, 2, 0.66f, 7.f}, {64, 128, 1, 0.74f, 6.8f}, {96, 128, 2, 1.8f, 5.4f}};
+    const long long rows = valid_rows ? (rows_cap * 3LL + 4) / 5 : rows_cap;
+    float best = 0.f;
+    for (int t = 0; t < 3; ++t) {
+      const Candidate &c = candidates[t];
+      float us = 0.f;
+      for (int i = valid_rows ? 8 : 10; i <= (valid_rows ? 12 : 10); ++i) {
+        const float load = (float)(((rows * i / 10 + c.bm - 1) / c.bm) * ((n + c.bn - 1) / c.bn)) / (float)(cu_count() * c.per_cu);
+        const float full = floorf(load), part = load - full;
+        us += (full + (part == 0.f ? 0.f : c.per_cu == 1 ? 1.f : 0.5f + 0.5f * part)) * (c.step * (float)(k / 64) + c.fixed);
+      }
+      if (t == 0 || us < best) best = us, tile = t;
+    }
+  }
+  if (tile == 0) return launch_f32_split<64, 64, 2, 2, 2, 2>(p, s);
+  if (tile == 1) return launch_f32_split<64, 128, 2, 2, 2, 2>(p, s);
+  return launch_f32_split<96, 128, 2, 2, 1, 2>(p, s);
+}

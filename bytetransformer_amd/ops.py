@@ -416,6 +416,42 @@ def gemm_f32(a, w, bias=None, gelu=False, valid_rows=None, a_row_index=None, row
     return out
 
 
+def split_f32(ws, rows=None, bounded=-1, bounded_bias=None, row_index=None, valid_rows=None, rows_cap=None):
+    """Weights [K, N] and rows as scaled pairs of fp16 numbers: ([(pairs, exps)], (row pairs, row exps) or None, bounds)."""
+    _need_f32(*ws, rows, bounded_bias)
+    lib, n = kernel_lib(), len(ws)
+    dev = (ws[0] if n else rows).device
+    pairs = [torch.zeros(w.shape[1], w.shape[0] // 32, 64, dtype=torch.float16, device=dev) for w in ws]
+    exps = [torch.zeros((w.shape[0] + 255) // 256, w.shape[1], dtype=torch.int32, device=dev) for w in ws]
+    bounds = None
+    if bounded >= 0:
+        bounds = torch.zeros(exps[bounded].numel() // 32, 2, dtype=torch.float32, device=dev)
+    got, hidden = None, 0
+    if rows is not None:
+        hidden = rows.shape[1]
+        cap = rows.shape[0] if rows_cap is None else rows_cap
+        got = (torch.zeros(cap, hidden // 32, 64, dtype=torch.float16, device=dev),
+               torch.zeros(cap, dtype=torch.int32, device=dev))
+    ptrs = [(ctypes.c_void_p * max(n, 1))(*[t.data_ptr() for t in ts]) for ts in (ws, pairs, exps)]
+    sizes = [(ctypes.c_int * max(n, 1))(*[w.shape[d] for w in ws]) for d in (0, 1)]
+    _check(lib.bt_split_f32(n, *ptrs, *sizes, bounded, _ptr(bounded_bias), _ptr(bounds), _ptr(rows),
+                            _ptr(got[0] if got else None), _ptr(got[1] if got else None), _ptr(row_index),
+                            _ptr(valid_rows), got[0].shape[0] if got else 0, hidden, _stream()))
+    return list(zip(pairs, exps)), got, bounds
+
+
+def gemm_f32_split(a, w, bias=None, gelu_exps=None, valid_rows=None, out=None):
+    """c = a . w (+ bias) of split operands (pairs, exps), or the pairs of its GELU scaled by 2^gelu_exps."""
+    (ap, ae), (wp, we) = a, w
+    rows, n, k = ap.shape[0], wp.shape[0], wp.shape[1] * 32
+    if out is None:
+        out = torch.zeros(*((rows, n) if gelu_exps is None else (rows, n // 32, 64)), device=ap.device,
+                          dtype=torch.float32 if gelu_exps is None else torch.float16)
+    _check(kernel_lib().bt_gemm_f32_split(_ptr(ap), _ptr(ae), _ptr(wp), _ptr(we), _ptr(bias), _ptr(out), _ptr(gelu_exps),
+                                          _ptr(valid_rows), rows, n, k, _stream()))
+    return out
+
+
 def attention_f32(qkv, batch_idx, batch_size, seq_len, head_num, scale, padded_rows=False,
                   mask=None, bias=None, out=None, seq_order=None):
     """qkv [rows, 3 * hidden] (bias added) -> [rows, hidden]."""
@@ -456,6 +492,19 @@ def add_bias_residual_layernorm_f32(out, residual, bias, gamma, beta, eps=1e-6, 
         _ptr(out), _ptr(residual), _ptr(residual_row_index), _ptr(bias), _ptr(gamma), _ptr(beta),
         _ptr(valid_rows), rows, H, float(eps), _stream()))
     return out
+
+
+def add_bias_residual_layernorm_f32_split(out, residual, bias, gamma, beta, bounds, eps=1e-6, valid_rows=None,
+                                          residual_row_index=None):
+    """The float LayerNorm in place, and (pairs, exps, exponents for the pairs of the GELU behind it)."""
+    _need_f32(out, residual, bias, gamma, beta)
+    rows, hidden = out.shape
+    pairs = torch.zeros(rows, hidden // 32, 64, dtype=torch.float16, device=out.device)
+    exps, gelu_exps = (torch.zeros(rows, dtype=torch.int32, device=out.device) for _ in range(2))
+    _check(kernel_lib().bt_add_bias_residual_layernorm_f32_split(
+        _ptr(out), _ptr(residual), _ptr(residual_row_index), _ptr(bias), _ptr(gamma), _ptr(beta), _ptr(valid_rows), rows,
+        hidden, float(eps), _ptr(pairs), _ptr(exps), _ptr(gelu_exps), _ptr(bounds), bounds.shape[0], _stream()))
+    return pairs, exps, gelu_exps
 
 
 def add_bias_residual_layernorm_restore_f32(out, residual, bias, gamma, beta, batch_idx,

@@ -451,6 +451,35 @@ int bt_splitk_layernorm(const void *partials, int splits, const void *residual,
                         int hidden_dim, float eps, void *stream);
 
 /*
+ * Float operands as pairs of fp16 numbers, made once by the launch that has them in hand, for products on fp16 matrix
+ * instructions (no counterpart in the reference).  A row of K floats (of a weight's column, 256 at a time) is scaled by
+ * 2^e, which brings its largest finite value to [2^14, 2^15), and stored as K / 32 blocks of 128 bytes: 32 h, then 32 l,
+ * h = fp16(x 2^e), l = fp16((x 2^e - h) 2^11).  x is h + l / 2^11 to 2^-23 of itself where it is above 2^-27 of the
+ * row's largest value, and to 2^-50 of that value elsewhere; infinities and NaN are kept.
+ *   bt_split_f32       w[i] [k[i], n[i]] -> w_pairs[i] [n][k / 32][64], w_exps[i] int[ceil(k / 256)][n] (k a
+ *                      multiple of 64, n of 32), and, where rows != NULL, row row_index[r] (r without an index) of `rows` ->
+ *                      row_pairs[r], row_exps[r] for r < *valid_rows, in one launch.  bounded >= 0: pairs
+ *                      {largest |w|, largest |bounded_bias|} of that weight's columns, 32 of them and 256 rows at a time:
+ *                      bounds float[2 n / 32 ceil(k / 256)].
+ *   bt_gemm_f32_split  c = a . w + bias (bias nullable), float; gelu_exps != NULL: the pairs of GELU(a . w + bias),
+ *                      row r scaled by 2^gelu_exps[r]; n a multiple of 32, k of 64.  Distance from float64 (2-norm; largest
+ *                      difference over the largest result) for normal operands: k = 768 1.4e-7, 2.5e-7, k = 3072 1.5e-7,
+ *                      2.4e-7, where bt_gemm_f32 has 2.1e-7, 3.5e-7 and 4.3e-7, 7.0e-7.
+ *   bt_add_bias_residual_layernorm_f32_split  bt_add_bias_residual_layernorm_f32 that writes the pairs of its rows as
+ *                      well, and exponents that keep the pairs of GELU(row . W + b) in range for the W of `bounds`.
+ */
+int bt_split_f32(int weight_count, const void *const *w, void *const *w_pairs, int *const *w_exps, const int *k,
+                 const int *n, int bounded, const void *bounded_bias, float *bounds, const void *rows, void *row_pairs,
+                 int *row_exps, const int *row_index, const int *valid_rows, int rows_cap, int hidden_dim, void *stream);
+int bt_gemm_f32_split(const void *a_pairs, const int *a_exps, const void *w_pairs, const int *w_exps, const void *bias,
+                      void *c, const int *gelu_exps, const int *valid_rows, int rows_cap, int n, int k, void *stream);
+int bt_add_bias_residual_layernorm_f32_split(void *out, const void *residual, const int *residual_row_index,
+                                             const void *bias, const void *gamma, const void *beta,
+                                             const int *valid_rows, int rows_cap, int hidden_dim, float eps, void *pairs,
+                                             int *exps, int *gelu_exps, const float *bounds, int bound_count,
+                                             void *stream);
+
+/*
  * ---- OperationType::FP32 ------------------------------------------------------
  * The float flavour of the layer: every tensor (activations, weights, biases, gamma,
  * beta, mask, attention bias) is float, and so are the accumulators of the products.  Weights are

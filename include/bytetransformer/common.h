@@ -93,6 +93,39 @@ inline int ffn2_slices(int rows_cap, bool all_live, int n, int k, unsigned long 
   return slices > 0 ? slices : rule;
 }
 
+// Float layers on products of split operands (bt_gemm_f32_split): from how many rows the launches that split the
+// weights, afresh in every layer, cost less than the products gain.  12 layers of hidden 768, split / not, us: 8 x 100
+// (480 rows expected) 1559 / 1319, 8 x 160 (768) 1729 / 1592, 10 x 200 (1200) 2088 / 2050, 16 x 128 (1229) 2046 / 2096,
+// 16 x 256 (2458) 3010 / 3690.  Follows from sizes alone, never from a row hint: both ways are float arithmetic to a
+// few 1e-7, but not the same bits.  From hidden 512 on: there the roundings of a sum outweigh those of the pairs, and the
+// result is the nearer one to float64 (distance, pairs / whole floats: k = 64 9.8e-8 / 5.5e-8, 512 1.17e-07 / 1.71e-07).
+inline bool f32_splits_operands(long long rows_cap, bool all_live, long long hidden, long long inter) {
+  return hidden % 64 == 0 && inter % 64 == 0 && hidden >= 512 && hidden <= 4096 && inter <= (1 << 14) &&
+         (all_live ? rows_cap : rows_cap * 3 / 5) >= 1220;
+}
+// What such a layer needs besides its activations: exponents of four sets of rows and of four weights' columns, and the
+// bounds of FFN1's.
+struct F32SplitScratch {
+  int *x_exps, *att_exps, *ln_exps, *gelu_exps, *w_exps[4];
+  float *bounds;
+  int bound_count;
+  // (a weight's column has an exponent for every 256 of its rows; a pair of bounds for every 32 columns of those)
+  static unsigned long long chunks(unsigned long long k) { return (k + 255) / 256; }
+  static unsigned long long bytes(unsigned long long rows, unsigned long long hidden, unsigned long long inter) {
+    return (4 * ((rows + 3) / 4 * 4) + chunks(hidden) * (4 * hidden + inter) + chunks(inter) * hidden +
+            chunks(hidden) * inter / 16) * 4;
+  }
+  F32SplitScratch(void *at, unsigned long long rows, int hidden, int inter) {
+    rows = (rows + 3) / 4 * 4;
+    int *p = (int *)at;
+    const unsigned long long n[4] = {chunks(hidden) * 3 * hidden, chunks(hidden) * hidden, chunks(hidden) * inter, chunks(inter) * hidden};
+    for (int i = 0; i < 4; ++i) w_exps[i] = p, p += n[i];
+    x_exps = p, att_exps = p + rows, ln_exps = p + 2 * rows, gelu_exps = p + 3 * rows;
+    bounds = (float *)(p + 4 * rows);
+    bound_count = (int)(chunks(hidden) * inter / 32);
+  }
+};
+
 // Row count that tiles are chosen for.  Without one from the caller the products take 60 % of the
 // capacity for a guess and price a tile over 80-120 % of it, which is what a handful of sequence
 // lengths spreads over; the mean of 32 or more lies within 7 % and is named as it is (batch 128 of up to

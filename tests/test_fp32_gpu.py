@@ -201,6 +201,173 @@ def test_gemm_f32_bias_gelu_and_gather(device):
 
 
 # ---- LayerNorm -------------------------------------------------------------------
+# ---- split operands ----------------------------------------------------------------
+def _joined(pairs, exps):
+    """What pairs [rows, K / 32, 64] and an exponent per row (or per 256 of a row: [ceil(K / 256), rows]) stand for."""
+    p = pairs.cpu().numpy().astype(np.float64)
+    x = (p[:, :, :32] + p[:, :, 32:] / 2048).reshape(p.shape[0], -1)
+    e = exps.cpu().numpy()
+    e = e[:, None] if e.ndim == 1 else np.repeat(e.T, 256, axis=1)[:, :x.shape[1]]
+    with np.errstate(invalid="ignore"):
+        return x * 2.0 ** -e.astype(np.float64)
+
+
+def _pair_bound(x, groups=None):
+    """2^-23 of a value, 2^-50 of the largest that shares its scale (2^-25, half the spacing of
+    subnormal fp16, in l, worth 2^-11, of a value scaled to at least 2^14)."""
+    with np.errstate(invalid="ignore"):
+        fin = np.where(np.isfinite(x), np.abs(x), 0).astype(np.float64)
+    top = fin.max(1, keepdims=True)
+    if groups:
+        top = np.concatenate([np.repeat(fin[:, k:k + 256].max(1, keepdims=True), fin[:, k:k + 256].shape[1], 1)
+                              for k in range(0, x.shape[1], 256)], 1)
+    return fin * 2.0 ** -23 + top * 2.0 ** -50 + 2.0 ** -149
+
+
+@pytest.mark.parametrize("K,N", [(64, 32), (256, 96), (320, 64), (768, 160)])
+def test_split_f32_holds_what_it_was_given(device, K, N):
+    """Weights and gathered rows over the whole range of floats, zeros, infinities and NaN among them."""
+    _say("split_f32", K, N)
+    rs = np.random.RandomState(K)
+    w = (rs.standard_normal((K, N)) * 2.0 ** rs.randint(-20, 20, (K, N))).astype(np.float32)
+    w[:, 1] = 0
+    w[:, 2] *= np.float32(1e-30)
+    w[:, 3] = np.finfo(np.float32).max * rs.choice([-1, 1], K)
+    w[:, 4] = 2.0 ** -140
+    w[3, 5], w[K - 1, 6], w[K // 2, 7] = np.inf, -np.inf, np.nan
+    x = (rs.standard_normal((40, K)) * 2.0 ** rs.randint(-60, 60, (40, 1))).astype(np.float32)
+    x[11, 5], x[12, 6], x[13] = np.inf, np.nan, 0
+    idx = rs.permutation(40)[:33].astype(np.int32)
+    bias = rs.standard_normal(N).astype(np.float32)
+    vr = torch.tensor([31], dtype=torch.int32, device=device)
+    (wp,), rows, bounds = ops.split_f32([_dev(w, device)], _dev(x, device), 0, _dev(bias, device), _dev(idx, device), vr, 33)
+    for got, exp, groups in ((_joined(*wp), w.T, True), (_joined(*rows)[:31], x[idx[:31]], False)):
+        fin = np.isfinite(exp)
+        assert np.array_equal(np.isnan(got), np.isnan(exp)) and np.array_equal(got[np.isinf(exp)], exp[np.isinf(exp)])
+        off = np.abs(np.where(fin, got, 0) - np.where(fin, exp, 0).astype(np.float64))
+        assert np.all(off <= _pair_bound(exp, groups)), (off / _pair_bound(exp, groups)).max()
+    assert not rows[0][31:].any() and not rows[1][31:].any()       # rows past the live count untouched
+    top = np.where(np.isfinite(w), np.abs(w), 0)
+    assert bounds[:, 0].max().item() == top.max() and bounds[:, 1].max().item() == np.abs(bias).max()
+
+
+@pytest.mark.parametrize("tile", [-1, 0, 1, 2])
+@pytest.mark.parametrize("rows,M,N,K", [(300, 300, 768, 768), (200, 131, 160, 64), (97, 96, 32, 320), (64, 1, 2304, 768), (140, 140, 192, 512),
+                                        (130, 129, 96, 3072), (193, 193, 416, 832)])
+def test_gemm_f32_split_against_float64(device, tile, rows, M, N, K):
+    _say("gemm_f32_split", tile, rows, M, N, K)
+    rs = np.random.RandomState(rows + N + K)
+    x = (rs.standard_normal((rows, K)) * 2.0 ** rs.randint(-30, 30, (rows, 1))).astype(np.float32)
+    w = (rs.standard_normal((K, N)) * 2.0 ** rs.randint(-30, 30, (1, N)) * 2.0 ** rs.randint(-9, 9, (K // 64, 1)).repeat(64, 0))
+    w = w.astype(np.float32)
+    bias = np.zeros(N, np.float32)
+    vr = torch.tensor([M], dtype=torch.int32, device=device)
+    (wp,), a, _ = ops.split_f32([_dev(w, device)], _dev(x, device))
+    ops.set_option("f32_gemm_tile", tile)
+    try:
+        out = torch.full((rows, N), 7.0, dtype=torch.float32, device=device)
+        g = ops.gemm_f32_split(a, wp, None, None, vr, out).cpu().numpy()
+        gb = ops.gemm_f32_split(a, wp, _dev(bias, device), None, vr).cpu().numpy()
+    finally:
+        ops.set_option("f32_gemm_tile", -1)
+    exp = x[:M].astype(np.float64) @ w.astype(np.float64)
+    # each operand to 2^-23, the second numbers' product 2^-22 left out, K / 16 float roundings at most, which do not add up
+    # in one direction: (4 + sqrt(K) / 2) 2^-23 of sum |a||w|
+    bound = (4 + math.sqrt(K) / 2) * 2.0 ** -23 * (np.abs(x[:M]).astype(np.float64) @ np.abs(w).astype(np.float64))
+    assert np.all(np.abs(g[:M] - exp) <= bound), (np.abs(g[:M] - exp) / bound).max()
+    assert np.all(g[M:] == 7.0) and np.array_equal(gb[:M], g[:M])
+    if K >= 512 and M * N > 10000:
+        # from there on no further from float64 than the products of whole floats, on operands of one scale
+        y, v = rs.standard_normal((M, K)).astype(np.float32), (rs.standard_normal((K, N)) * 0.02).astype(np.float32)
+        (vp,), b, _ = ops.split_f32([_dev(v, device)], _dev(y, device))
+        ref = y.astype(np.float64) @ v.astype(np.float64)
+        mine = np.linalg.norm(ops.gemm_f32_split(b, vp).cpu().numpy() - ref)
+        whole = np.linalg.norm(ops.gemm_f32(_dev(y, device), _dev(v, device)).cpu().numpy() - ref)
+        _say("from float64: pairs %.2e whole %.2e" % (mine / np.linalg.norm(ref), whole / np.linalg.norm(ref)))
+        assert mine <= whole
+
+
+@pytest.mark.parametrize("tile", [0, 1, 2])
+def test_gemm_f32_split_passes_infinities_and_nan_on(device, tile):
+    _say("gemm_f32_split inf nan", tile)
+    rs = np.random.RandomState(3)
+    x, w = rs.standard_normal((70, 128)).astype(np.float32), rs.standard_normal((128, 64)).astype(np.float32)
+    x[3, 7], x[40, 100], x[41, 3], w[9, 5] = np.inf, -np.inf, np.nan, np.inf
+    x[50, 9] = 0                                      # 0 . inf
+    bias = rs.standard_normal(64).astype(np.float32)
+    with np.errstate(invalid="ignore", over="ignore"):
+        exp = x.astype(np.float64) @ w.astype(np.float64) + bias
+    (wp,), a, _ = ops.split_f32([_dev(w, device)], _dev(x, device))
+    ops.set_option("f32_gemm_tile", tile)
+    try:
+        g = ops.gemm_f32_split(a, wp, _dev(bias, device)).cpu().numpy()
+        ge = torch.full((70,), 6, dtype=torch.int32, device=device)
+        h = _joined(ops.gemm_f32_split(a, wp, _dev(bias, device), ge), ge)
+    finally:
+        ops.set_option("f32_gemm_tile", -1)
+    fin = np.isfinite(exp)
+    assert fin.mean() > 0.9
+    assert np.array_equal(np.isnan(g), np.isnan(exp)) and np.array_equal(g[np.isinf(exp)], exp[np.isinf(exp)])
+    assert np.abs(g[fin] - exp[fin]).max() <= 1e-4
+    gelu = exp[fin] / (1 + np.exp(-2 * 0.7978845608028654 * (exp[fin] + 0.044715 * exp[fin] ** 3)))
+    assert np.isfinite(h[fin]).all() and np.abs(h[fin] - gelu).max() <= 1e-4
+    assert np.all(np.isnan(h[~fin]) | np.isinf(h[~fin]) | (h[~fin] == 0))       # GELU(-inf) is -0 or NaN in float arithmetic
+
+
+@pytest.mark.parametrize("H", [64, 768, 1024])
+def test_layernorm_f32_split_keeps_the_gelu_in_range(device, H):
+    """The LayerNorm's rows are those of the plain one, its pairs stand for them, and the exponents it gives to FFN1 leave
+    every result of it finite and where it belongs, large weights and biases included."""
+    _say("layernorm_f32_split", H)
+    rs = np.random.RandomState(H)
+    rows, M, F = 45, 40, 96
+    out, res = rs.standard_normal((rows, H)).astype(np.float32), rs.standard_normal((50, H)).astype(np.float32)
+    ridx = rs.permutation(50)[:rows].astype(np.int32)
+    bias, beta = (rs.standard_normal(H).astype(np.float32) for _ in range(2))
+    gamma = (1 + rs.standard_normal(H)).astype(np.float32) * 30
+    w, b1 = (rs.standard_normal((H, F)) * 50).astype(np.float32), (rs.standard_normal(F) * 1e4).astype(np.float32)
+    vr = torch.tensor([M], dtype=torch.int32, device=device)
+    (wp,), _, bounds = ops.split_f32([_dev(w, device)], None, 0, _dev(b1, device))
+    args = [_dev(a, device) for a in (res, bias, gamma, beta)]
+    mine, plain = _dev(out, device), _dev(out, device)
+    pairs, exps, ge = ops.add_bias_residual_layernorm_f32_split(mine, *args, bounds, 1e-6, vr, _dev(ridx, device))
+    ops.add_bias_residual_layernorm_f32(plain, *args, 1e-6, valid_rows=vr, residual_row_index=_dev(ridx, device))
+    assert torch.equal(mine, plain)
+    ln = plain.cpu().numpy()[:M]
+    assert np.all(np.abs(_joined(pairs, exps)[:M] - ln) <= _pair_bound(ln))
+    got = _joined(ops.gemm_f32_split((pairs, exps), wp, _dev(b1, device), ge, vr), ge)[:M]
+    u = ln.astype(np.float64) @ w.astype(np.float64) + b1
+    with np.errstate(over="ignore"):
+        exp = u / (1 + np.exp(-2 * 0.7978845608028654 * (u + 0.044715 * u ** 3)))
+    assert np.isfinite(got).all()
+    # the product to 2^-20 of sum |a||w|, GELU in float, pairs to 2^-23
+    bound = 2.0 ** -20 * (np.abs(ln).astype(np.float64) @ np.abs(w).astype(np.float64) + np.abs(b1)) + 1e-6
+    assert np.all(np.abs(got - exp) <= bound), (np.abs(got - exp) / bound).max()
+
+
+@pytest.mark.parametrize("path", ["c_api", "th_op", "encoder"])
+@pytest.mark.parametrize("rm", [True, False])
+def test_fp32_layers_on_split_operands(device, path, rm):
+    """Sizes from which on a float layer splits its operands, against the oracle."""
+    _say("fp32 split layers", path, rm)
+    cfg = workload.EncoderConfig("f32s", 17, 120, 8, layers=2, dtype="fp32", lens=(120, 3, 41, 0, 64, 119) + (90,) * 11)
+    wl = workload.make_workload(cfg, bias_std=0.05, random_affine=True)
+    x, m = _dev(wl.x, device), _dev(wl.mask, device)
+    if path == "c_api":
+        got = bt.encoder_forward(_layers(wl, device, is_remove_padding=rm), x, m)
+    elif path == "th_op":
+        bt.load_th_op()
+        got = x
+        for w in wl.layers:
+            got = torch.ops.ByteTransformer.BertTransformer(
+                cfg.head_num, cfg.head_size, *[_dev(w[n], device) for n in workload.WEIGHT_NAMES], got, m, rm, True)
+    else:
+        got = bt.BertEncoder(cfg.head_num, cfg.head_size, [{k: _dev(v, device) for k, v in w.items()} for w in wl.layers],
+                             is_remove_padding=rm)(x, m)
+    got = got.cpu().numpy()
+    _f32_check(got if rm else O.masked_output(got, wl.lens), _oracle32(wl), wl.lens, "f32 split/%s" % path, rm)
+
+
 @pytest.mark.parametrize("H", [768, 1024, 64, 4096, 260])
 def test_layernorm_f32(device, H):
     _say("layernorm_f32", H)
