@@ -187,27 +187,14 @@ void BertEncoder<OpType>::infer(BertEncoderInferParam<DataType_> ip) {
     att.seq_order = seq_order;
     if (check_mask) att.mask_prefix_slots = mask_slots;
     att.work_list = work_list;
-    // warm the memory-side cache with what follows in memory order: the rest of this
-    // layer's weights and, when all layers are pre-packed back to back, the next
-    // layer's QKV matrix
-    if (ip.prepacked) {
-      att.prefetch[0] = wt_proj;
-      att.prefetch_bytes[0] = ((size_t)hidden * hidden + 2 * (size_t)hidden * inter) * sizeof(DataType_);
-      if (l + 1 < L) att.prefetch_bytes[0] += (size_t)3 * hidden * hidden * sizeof(DataType_);
-      att.prefetch_count = 1;
-    } else {
-      const void *next[3] = {wt_proj, wt_inter, wt_out};
-      const size_t elems[3] = {(size_t)hidden * hidden, (size_t)hidden * inter, (size_t)hidden * inter};
-      for (int i = 0; i < 3; ++i) {
-        att.prefetch[i] = next[i];
-        att.prefetch_bytes[i] = elems[i] * sizeof(DataType_);
-      }
-      att.prefetch_count = 3;
-      if (l + 1 < L) {
-        att.prefetch[3] = layers_[l + 1].attr_kernel_QKV;
-        att.prefetch_bytes[3] = (size_t)3 * hidden * hidden * sizeof(DataType_);
-        att.prefetch_count = 4;
-      }
+    // warm the caches with what follows: the rest of this layer's weights and the next layer's QKV matrix
+    const void *next[4] = {wt_proj, wt_inter, wt_out, nullptr};
+    if (l + 1 < L) next[3] = ip.prepacked ? (const void *)(wt_out + (size_t)hidden * inter) : layers_[l + 1].attr_kernel_QKV;
+    const int next_k[4] = {hidden, hidden, inter, hidden}, next_n[4] = {hidden, inter, hidden, 3 * hidden};
+    att.prefetch_count = l + 1 < L ? 4 : 3;
+    for (int i = 0; i < att.prefetch_count; ++i) {
+      att.prefetch[i] = next[i];
+      att.prefetch_bytes[i] = prefetch_weight(next_k[i], next_n[i], weight_kn, i == 2 ? splits : 1, valid_rows ? rows * 3LL / 5 : rows);
     }
     attention_layer_->infer(att);
 

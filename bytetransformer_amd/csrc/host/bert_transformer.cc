@@ -339,18 +339,20 @@ void BertTransformer<OpType>::bert_infer(BertTransformerInferParam infer_param) 
   // kernel finds its balanced order by a look-up of its own)
   attention_infer_param.work_list = nullptr;
   attention_infer_param.no_offsets = mask_direct;   // (nothing has written them)
+  // few rows, long k: FFN2 as split-k partial sums that the last LayerNorm folds in
+  const int splits = ffn2_slices(packed_cap, all_live, hidden, inter, partials_bytes);
   // the weight matrices the rest of the layer reads (as stored, or the copies that the first
-  // launch has made): the attention kernel pulls them into the memory-side cache while it
+  // launch has made): the attention kernel pulls them into the caches while it
   // runs.  A matrix that the first LayerNorm's launch copies is left alone: the copy reads
   // its source once either way, and the product reads the copy (same box, with / without
   // touching it: batch 16 x 512 1.519 / 1.514 ms, 16 x 1024 2.586 / 2.574, BERT-large 6.610 / 6.589).
   {
-    const size_t elems[3] = {(size_t)hidden * hidden, (size_t)hidden * inter, (size_t)hidden * inter};
+    const long long expected = all_live ? packed_cap : packed_cap * 3LL / 5;
     int pc = 0;
     for (int i = 0; i < 3; ++i) {
       if (lp.ln_copy[i + 1]) continue;
       attention_infer_param.prefetch[pc] = w_use[i + 1];
-      attention_infer_param.prefetch_bytes[pc] = elems[i] * sizeof(DataType_);
+      attention_infer_param.prefetch_bytes[pc] = prefetch_weight(w_k[i + 1], w_n[i + 1], w_kn[i + 1], i == 2 ? splits : 1, expected);
       ++pc;
     }
     attention_infer_param.prefetch_count = pc;
@@ -377,8 +379,6 @@ void BertTransformer<OpType>::bert_infer(BertTransformerInferParam infer_param) 
                                    product_rows, packed_cap, rows_hint, inter, hidden, w_kn[2],
                                    stream));
 
-  // few rows, long k: FFN2 as split-k partial sums that the last LayerNorm folds in
-  const int splits = ffn2_slices(packed_cap, all_live, hidden, inter, partials_bytes);
   if (splits > 1) {
     check_bt_error(bt_gemm_splitk_rows(inter_matmul_buf, wt_out, partials, splits, product_rows, packed_cap,
                                        rows_hint, hidden, inter, w_kn[3], stream));

@@ -116,25 +116,27 @@ template <int KIND>
 struct AttTail : std::conditional_t<(KIND & kAddBoth) != 0, AttTerms, AttNoTerms> {
   half_t *out;
   float scale_log2e;
-  unsigned warm_first, warm_per;
-  unsigned warm_end[kWarmRanges];
+  unsigned warm_first, warm_ends, warm_forms_turns;
+  unsigned warm_shape[kWarmRanges];
   const char *warm_base[kWarmRanges];
 };
 template <int KIND>
 static AttTail<KIND> att_tail(const AttArgs &a) {
   AttTail<KIND> t{};
   if constexpr ((KIND & kAddBoth) != 0) t.mask = a.mask, t.bias = a.bias, t.mask_ok = a.mask_ok;
-  t.out = a.out, t.scale_log2e = a.scale_log2e, t.warm_first = a.warm.first, t.warm_per = a.warm.per;
-  for (int r = 0; r < kWarmRanges; ++r) t.warm_end[r] = a.warm.end[r], t.warm_base[r] = a.warm.base[r];
+  t.out = a.out, t.scale_log2e = a.scale_log2e, t.warm_first = a.warm.first, t.warm_ends = a.warm.ends;
+  t.warm_forms_turns = a.warm.forms_turns;
+  for (int r = 0; r < kWarmRanges; ++r) t.warm_shape[r] = a.warm.shape[r], t.warm_base[r] = a.warm.base[r];
   return t;
 }
 template <int KIND>
 __device__ __forceinline__ AttArgs att_args(BT_ATT_FIRST, const AttTail<KIND> &tail) {
   AttArgs p{};
   if constexpr ((KIND & kAddBoth) != 0) p.mask = tail.mask, p.bias = tail.bias, p.mask_ok = tail.mask_ok;
-  p.out = tail.out, p.scale_log2e = tail.scale_log2e, p.warm.first = tail.warm_first, p.warm.per = tail.warm_per;
+  p.out = tail.out, p.scale_log2e = tail.scale_log2e, p.warm.first = tail.warm_first;
+  p.warm.ends = tail.warm_ends, p.warm.forms_turns = tail.warm_forms_turns;
 #pragma unroll
-  for (int r = 0; r < kWarmRanges; ++r) p.warm.end[r] = tail.warm_end[r], p.warm.base[r] = tail.warm_base[r];
+  for (int r = 0; r < kWarmRanges; ++r) p.warm.shape[r] = tail.warm_shape[r], p.warm.base[r] = tail.warm_base[r];
   p.qkv = qkv, p.batch_idx = batch_idx;
   p.seq_order = flags & kAttList ? nullptr : order;
   p.work_list = flags & kAttList ? (const int4 *)order : nullptr;

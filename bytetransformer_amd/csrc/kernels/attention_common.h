@@ -143,23 +143,63 @@ __device__ __forceinline__ float4_t add_terms(float4_t s, float scale, uint2_t m
 }
 
 // ---- cache warm-up on behalf of later kernels ------------------------------------------------
-// Ranges that the launches after this one will read (the layer's remaining weights): some workgroups
-// touch one dword per 128-byte line of their slice, so that the products find them in the memory-side
-// cache.  Range r holds the lines [end[r - 1], end[r]) of the concatenation (end[3] = 0: none).
+// Ranges that the launches after this one will read (the layer's remaining weights): some workgroups touch one
+// dword per 128-byte line of them.  A range is rows of `pitch` bytes, and the workgroups of XCD x touch one eighth of
+// it: 2^-cols of the bytes of 2^(cols - 3) of the rows.  For a weight that is the eighth whose tiles the XCD will
+// work on (tile_at: products of few rows go column by column), so they are found in its own L2 and not just in the
+// memory-side cache: 96 KB come to a CU in 1.2 us from the one and in 1.6 to 2.5 from the other.
+// 12 layers with the lines as they lie dealt out to all XCDs, and so, us: as stored 1 x 32 341 -> 331, 1 x 64 342 -> 339,
+// pre-packed (rows of 128 bytes) 1 x 32 318 -> 315.  With more rows than that order has (prefetch_weight) nothing is
+// gained, and the shorter runs cost: a wave's lines 1 KB apart 7 x 217 +4 %, eighths 16 x 512 +1 %.
 constexpr int kWarmRanges = 4;
 struct WarmDuty {
   const char *base[kWarmRanges];
-  unsigned end[kWarmRanges];
-  unsigned first;       // the workgroups from here on take part
-  unsigned per;         // lines of each
-  unsigned grid_work;   // workgroups of the attention itself: later ones do nothing else
+  unsigned shape[kWarmRanges];   // pitch / 64 | rows << 16, or how many lines
+  unsigned ends;                 // byte r: of an XCD's workgroups that take part, those below it take ranges 0 .. r
+  unsigned forms_turns;          // per range 4 bits, cols | rows first << 2; from bit 16: the most lines of a thread
+  unsigned first;                // the workgroups from here on take part, a multiple of 8
+  unsigned grid_work;            // workgroups of the attention itself: later ones do nothing else
 };
+constexpr unsigned kWarmRowsFirst = 4;   // form: the eighths are counted along the rows first
+constexpr unsigned kWarmLines = 8;       // form: no eighths, lines as they lie, dealt out to all XCDs
+__host__ __device__ constexpr unsigned warm_rows(unsigned shape, unsigned cols) {   // of an eighth
+  return ((shape >> 16) + (8u >> cols) - 1) >> (3 - cols);
+}
+__host__ __device__ constexpr unsigned warm_row_lines(unsigned shape, unsigned cols) {
+  return (((shape & 0xffffu) * 64u >> cols) + 127) / 128;
+}
 template <int THREADS>
 __device__ __forceinline__ void warm_slice(const WarmDuty &w) {
-  const unsigned lines = w.end[kWarmRanges - 1];
-  if (!lines || workgroup_id() < w.first) return;
-  const unsigned first = (workgroup_id() - w.first) * w.per;
-  touch_lines(w.base, w.end, first + thread_id(), min(first + w.per, lines), THREADS);
+  if (workgroup_id() < w.first) return;
+  const unsigned x = workgroup_id() & 7, mine = (workgroup_id() - w.first) >> 3;
+  // (a workgroup has one range: with the lines of all dealt out one after the other, every thread found its range by
+  // itself, and the attention of 1 x 256 took 8.1 us, of 8 x 64 4.75)
+  unsigned begin = 0, end = w.ends & 0xff, shape = w.shape[0], form = w.forms_turns & 15;
+  const char *from = w.base[0];
+#pragma unroll
+  for (int r = 1; r < kWarmRanges; ++r) {
+    const bool here = mine >= end;
+    begin = here ? end : begin, shape = here ? w.shape[r] : shape, form = here ? w.forms_turns >> 4 * r & 15 : form;
+    from = here ? w.base[r] : from, end = here ? w.ends >> 8 * r & 0xff : end;
+  }
+  if (mine >= end) return;
+  const unsigned turns = w.forms_turns >> 16;
+  if (form & kWarmLines) {
+    const unsigned parts = (end - begin) * 8;
+    touch_lines<THREADS>(min(shape, parts * THREADS * turns), (mine - begin) * 8 + x, parts,
+                         [&](unsigned l) { return (unsigned long long)from + l * 128ull; });
+    return;
+  }
+  const unsigned cols = form & 3, pitch = (shape & 0xffffu) * 64, rows = warm_rows(shape, cols), row_lines = warm_row_lines(shape, cols);
+  const unsigned at_row = (form & kWarmRowsFirst ? x & ((8u >> cols) - 1) : x >> cols) * rows;
+  const unsigned at_col = form & kWarmRowsFirst ? x >> (3 - cols) : x & ((1u << cols) - 1);
+  from += (unsigned long long)at_row * pitch + (at_col * (pitch >> cols) & ~63u);
+  const int last = (int)(shape >> 16) - 1 - (int)at_row;   // row of the share that is the range's last
+  const float inverse = __builtin_amdgcn_rcpf((float)row_lines);
+  touch_lines<THREADS>(min(rows * row_lines, (end - begin) * THREADS * turns), mine - begin, end - begin, [&](unsigned l) {
+    const int row = (int)(((float)l + 0.5f) * inverse);   // l / row_lines, exact below 2^21
+    return (unsigned long long)from + ((long long)min(row, last) * pitch + (l - row * row_lines) * 128);
+  });
 }
 // Who takes part, for a launch of `grid` workgroups (grown here by the ones that only warm).
 //   Two workgroups per CU and more (option prefetch_min_grid): the last quarter of the issue order -
@@ -169,44 +209,72 @@ __device__ __forceinline__ void warm_slice(const WarmDuty &w) {
 //   up, touch the weights meanwhile.  Left to the attention's own workgroups the touches lengthened
 //   it (+3 to +8 % per forward); with workgroups of their own 12 layers take 454 -> 412 us at batch
 //   1 x 32, 545 -> 490 at 1 x 256, 520 -> 477 at 4 x 96, 800 -> 762 at 7 x 217, 929 -> 875 at 6 x 250.
-//   More than 12 MB (BERT-large has 25 with the next layer's QKV weight) takes longer than the
-//   attention itself: 24 layers of hidden 1024 at 3 x 28, encoder entry 924 us with 12 MB, 935 with all.
+//   More than 15 MB (BERT-large has 25 with the next layer's QKV weight) takes longer than the
+//   attention itself and is cut to 12: 24 layers of hidden 1024, encoder entry, 3 x 28 924 us with 12 MB, 935 with all;
+//   10 x 100 1398 with 12, 1430 with 14.  Hidden 768 has 14.2 with the next QKV weight: 12 layers, all and with 12 (the
+//   QKV weight's end left out), us: 4 x 96 372 / 383, 8 x 64 417 / 424, 7 x 217 579 / 596.
 inline int plan_warm_duty(const char *who, WarmDuty &w, unsigned &grid, const void *const *ranges,
                           const unsigned long long *bytes, int count) {
   for (int r = 0; r < kWarmRanges; ++r) {
     w.base[r] = nullptr;
-    w.end[r] = 0;
+    w.shape[r] = 0;
   }
   w.first = w.grid_work = grid;
-  w.per = 0;
+  w.ends = w.forms_turns = 0;
   BT_REQUIRE(count >= 0 && count <= kWarmRanges, BT_ERR_INVALID_ARGUMENT,
              "%s: prefetch_count=%d outside [0, %d]", who, count, kWarmRanges);
   BT_REQUIRE(count == 0 || (ranges && bytes), BT_ERR_INVALID_ARGUMENT,
              "%s: prefetch ranges need their pointers and sizes", who);
   if (!count || !option_prefetch()) return BT_OK;
-  unsigned long long left;   // lines that the duty workgroups take on
+  unsigned per, most;   // workgroups of an XCD, and lines that they take on
   if (grid < (unsigned)option_prefetch_min_grid()) {
     const unsigned idle = grid < 256 ? 256 - grid : 0, extra = idle < 96 ? 96 : idle > 208 ? 208 : idle;
-    grid += extra;
-    left = 98304;   // 12 MB: what fits beside an attention of 4 to 6 us
+    w.first = (grid + 7) / 8 * 8;
+    per = extra / 8;
+    grid = w.first + per * 8;
+    unsigned long long all = 0;
+    for (int r = 0; r < count; ++r) all += ranges[r] ? bytes[r] & ((1ull << 40) - 1) : 0;
+    most = all <= (15ull << 20) ? 15360 : 12288;   // of 128 bytes and eight XCDs: 15 and 12 MB
   } else {
-    w.first = (unsigned)((unsigned long long)grid * 3 / 4);
-    left = (unsigned long long)(grid - w.first) * 4 * 256;
+    w.first = (unsigned)(((unsigned long long)grid * 3 / 4 + 7) / 8 * 8);
+    per = grid > w.first ? (grid - w.first) / 8 : 0;
+    if (per > 0xff) per = 0xff;
+    most = per * 4 * 256;
   }
-  unsigned end = 0;
-  for (int r = 0; r < kWarmRanges; ++r) {
-    if (r < count && ranges[r] && left) {
-      // one dword at the start of each 128-byte line; a last line of fewer than four bytes
-      // is left alone, so no byte outside the range is read
-      unsigned long long lines = (bytes[r] + 124) / 128;
-      if (lines > left) lines = left;
-      left -= lines;
-      w.base[r] = (const char *)ranges[r];
-      end += (unsigned)lines;
+  unsigned lines = 0, upto[kWarmRanges];
+  int at = 0;
+  for (int r = 0; r < count; ++r) {
+    const unsigned long long size = bytes[r] & ((1ull << 40) - 1);
+    unsigned pitch = (unsigned)(bytes[r] >> 40 & 0xffff) * 64, cols = (unsigned)(bytes[r] >> 56 & 3);
+    unsigned form = cols | (bytes[r] >> 58 & 1 ? kWarmRowsFirst : 0);
+    unsigned long long rows = pitch ? size / pitch : 0;
+    if (!rows || rows > 0xffff || rows * pitch != size || rows % (8u >> cols) || (pitch >> cols) % 64) {
+      // (of the last line at least four bytes lie inside the range, so no byte outside it is read)
+      rows = (size + 124) / 128;
+      if (rows > 0xffffff) rows = 0xffffff;
+      form = kWarmLines;
     }
-    w.end[r] = end;
+    if (!ranges[r] || !rows || lines >= most) continue;
+    w.base[at] = (const char *)ranges[r];
+    w.shape[at] = form == kWarmLines ? (unsigned)rows : pitch / 64 | (unsigned)rows << 16;
+    w.forms_turns |= form << 4 * at;
+    lines += form == kWarmLines ? (unsigned)(rows + 7) / 8 : warm_rows(w.shape[at], cols) * warm_row_lines(w.shape[at], cols);
+    upto[at++] = lines = lines < most ? lines : most;   // (what is beyond is the last range's end)
   }
-  if (end) w.per = (end + (grid - w.first) - 1) / (grid - w.first);
+  if (!at || !per) return BT_OK;
+  // workgroups by lines, one for a range at least, and turns enough for every line: a product that finds nine lines in ten
+  // takes nearly as long as one that finds none (7 x 217 with a tenth left out: FFN2 10.2 -> 12.9 us)
+  unsigned turns = 1;
+  for (int r = 0; r < at; ++r) {
+    unsigned end = (unsigned)(((unsigned long long)upto[r] * per + lines / 2) / lines);
+    const unsigned before = r ? w.ends >> 8 * (r - 1) & 0xff : 0, threads = 256;
+    if (end <= before) end = before + 1;
+    if (end > per) end = per;
+    for (int q = r; q < kWarmRanges; ++q) w.ends = (w.ends & ~(0xffu << 8 * q)) | end << 8 * q;
+    const unsigned mine = upto[r] - (r ? upto[r - 1] : 0), at_once = (end - before) * threads;
+    if (at_once && (mine + at_once - 1) / at_once > turns) turns = (mine + at_once - 1) / at_once;
+  }
+  w.forms_turns |= turns << 16;
   return BT_OK;
 }
 

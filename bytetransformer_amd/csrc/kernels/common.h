@@ -449,6 +449,22 @@ __device__ __forceinline__ void touch_lines(const char *const (&base)[4], const 
   }
 }
 
+// The same for lines 0 .. lines - 1, at(l) each, by workgroup `mine` of `per` (THREADS threads each).
+template <int THREADS, typename At>
+__device__ __forceinline__ void touch_lines(unsigned lines, unsigned mine, unsigned per, At at) {
+  constexpr int kFlight = 2;
+  for (unsigned l = mine * THREADS + __builtin_amdgcn_workitem_id_x(); l < lines; l += kFlight * per * THREADS) {
+    unsigned got[kFlight];
+#pragma unroll
+    for (int u = 0; u < kFlight; ++u) {
+      typedef unsigned any_byte __attribute__((aligned(1)));
+      const unsigned line = min(l + u * per * THREADS, lines - 1);
+      got[u] = *(const __attribute__((address_space(1))) any_byte *)at(line);
+    }
+    asm volatile("" ::"v"(got[0]), "v"(got[1]));   // (both have returned)
+  }
+}
+
 // ---- which tile a position of the XCD-aware order is ---------------------------------------
 // XCD x works on the positions [x * per, (x + 1) * per) and every XCD has an L2 of its own, so
 // what the launch fetches from the memory side is, per XCD, the distinct rows of A plus the

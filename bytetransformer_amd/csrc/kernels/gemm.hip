@@ -524,6 +524,7 @@ struct WaveTile {
 // split launch follow each other in it.  (As rows of the grid they left the workgroups of the dead rows
 // between them, and the live ones of the second slice came to lie on the CUs of the first: 230 of 384 rows,
 // hidden 768, FFN2 in two slices with the LayerNorm behind it 13.6 -> 11.1 us.)
+constexpr int kColumnRows = 256;   // rows of the launches whose 32-row tiles go column by column
 template <int BM, int BN>
 __device__ __forceinline__ bool tile_at(const GemmArgs &p, int M, int bid, int &split, int &tile_m, int &tile_n) {
   const int tiles_m = (M + BM - 1) / BM;
@@ -535,14 +536,21 @@ __device__ __forceinline__ bool tile_at(const GemmArgs &p, int M, int bid, int &
   split = 0;
   if (p.splits > 1)
     for (; L >= tiles; L -= tiles) ++split;
-  if (BM == 32 && tiles_m > 3 && live < kMostPanelTiles) {
+  if (BM == 32 && tiles_m > 1 && live < kMostPanelTiles) {
     // A few hundred rows: the launch is as long as it takes to fetch the weight, and in row-major
     // order every XCD fetches all of it (256 rows, QKV at hidden 768: 28 MB in all against
-    // 7 MB in panels; 12 layers at batch 1 x 256: -8 %).  At two or three tile rows few workgroups
-    // share a fetch and those of one XCD wait on the same lines (24 layers of hidden 1024 at 46
-    // rows: 941 us in panels, 917 row-major).  With the larger tiles the panels gain nothing and
-    // their index arithmetic costs up to 1 %.
-    tile_panels<BM, BN>(tiles_m, p.tiles_n, per).locate(L, tile_m, tile_n);
+    // 7 MB in panels; 12 layers at batch 1 x 256: -8 %).  Up to 256 rows the order is column by column: an XCD has an
+    // eighth of the weight to itself however many the rows, the eighth that the attention's launch has put into
+    // its L2 (warm_slice).  12 layers in panels (two or three tile rows row-major, as one always is) and so, us: as
+    // stored 1 x 64 346 -> 342, 1 x 128 376 -> 369, pre-packed 2 x 64 361 -> 354; 8 x 64, some 300 rows, 440 -> 444.  With
+    // the larger tiles neither gains anything (64 x 64: 1 x 256 416 -> 422) and the index arithmetic costs up to 1 %.
+    if (tiles_m <= kColumnRows / BM) {
+      const int column = divide_small(L, tiles_m);
+      tile_m = L - column * tiles_m;
+      tile_n = column;
+    } else {
+      tile_panels<BM, BN>(tiles_m, p.tiles_n, per).locate(L, tile_m, tile_n);
+    }
   } else {
     tile_m = (int)divide((unsigned)L, (unsigned)p.tiles_n, p.per_n);
     tile_n = L - tile_m * p.tiles_n;

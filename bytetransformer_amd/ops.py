@@ -268,11 +268,14 @@ def gemm_qkv_bias_split_mask_rows(x, mask, wt_qkv, bias_qkv, head_num, size_per_
 
 
 def _warm_ranges(prefetch):
-    """prefetch: None, one tensor or up to four, the ranges later kernels will read."""
+    """prefetch: None, one tensor or up to four, the ranges later kernels will read; (tensor, form) gives the bits from
+    40 up of its size, too."""
     ranges = [] if prefetch is None else ([prefetch] if torch.is_tensor(prefetch) else list(prefetch))
+    forms = [0 if torch.is_tensor(t) else t[1] for t in ranges]
+    ranges = [t if torch.is_tensor(t) else t[0] for t in ranges]
     n = len(ranges)
     ptrs = (ctypes.c_void_p * max(n, 1))(*[t.data_ptr() for t in ranges])
-    sizes = (ctypes.c_ulonglong * max(n, 1))(*[t.numel() * t.element_size() for t in ranges])
+    sizes = (ctypes.c_ulonglong * max(n, 1))(*[t.numel() * t.element_size() | f << 40 for t, f in zip(ranges, forms)])
     for t in ranges:
         _ptr(t)
     return ptrs, sizes, n

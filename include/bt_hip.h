@@ -308,6 +308,12 @@ int bt_gemm_qkv_bias_split_mask_rows(const void *from_tensor, const void *atten_
  *                     chip gets on top, touch them line by line so that they
  *                     sit in the memory-side cache by then; purely a hint, the results do
  *                     not depend on it.  No counterpart in the reference.
+ *                     A size is the low 40 bits; above them it may say how the range is shared
+ *                     among the XCDs, so that each finds its share in its own L2: bits 40-55 a row
+ *                     pitch / 64 (0: eighths as the bytes lie), 56-57 how often a row is halved,
+ *                     the rows as many times less than three, 58: consecutive XCDs take
+ *                     consecutive rows, not consecutive parts of one.  What does not divide is
+ *                     dealt out line by line.
  *   seq_order (nullable): a permutation of the sequence indices from
  *                     bt_build_offsets; workgroups are issued in that order so the
  *                     longest sequences start first.  Results do not depend on it.

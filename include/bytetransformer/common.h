@@ -52,6 +52,16 @@ typedef struct {
   int valid_word_num;
 } ET_Param;
 
+// What a product in `slices` of k will read of a weight, for the attention's warm-up (prefetch_bytes in bt_hip.h): the
+// XCDs' shares up to 256 expected rows, for which the products go column by column.
+inline unsigned long long prefetch_weight(unsigned long long k, unsigned long long n, bool weight_kn, int slices, long long rows) {
+  const unsigned long long bytes = k * n * 2, pitch = (weight_kn ? n : k) * 2;
+  const int halvings = slices == 1 ? 0 : slices == 2 ? 1 : slices == 4 ? 2 : slices == 8 ? 3 : -1;
+  if (rows > 256 || halvings < 0 || pitch % 64 || pitch / 64 > 0xffff || bytes >> 40) return bytes;
+  const unsigned long long cols = weight_kn ? 3 - halvings : halvings;
+  return bytes | pitch / 64 << 40 | cols << 56 | (weight_kn ? 0ull : 1ull) << 58;
+}
+
 // FFN2 with few rows and a long k runs as a split-k GEMM whose fp32 partial sums the last
 // LayerNorm folds in (bt_gemm_splitk_rows / bt_splitk_layernorm).  This is the rule where the kernels
 // library has no measurements (bt_gemm_splitk_slices): 4 splits up to 192 expected

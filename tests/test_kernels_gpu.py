@@ -1367,6 +1367,37 @@ def test_attention_prefetch_hint_changes_nothing(device, kind, lens, S):
         ops.set_option("prefetch_min_grid", 512)
 
 
+@pytest.mark.parametrize("kind", ["short", "grouped", "generic"])
+@pytest.mark.parametrize("min_grid", [512, 1])
+def test_attention_prefetch_of_shared_weights_changes_nothing(device, kind, min_grid):
+    """Weights whose eighths are named for the XCDs ([k, n] and [n, k], whole and in slices of k), ones that do not divide,
+    pitches of another size than the range: read only, and nothing of the result depends on them."""
+    rs = np.random.RandomState(5)
+    lens, S = [60, 7, 64], 64
+    bi, M, qkv = _attention_case(rs, lens, S, 2, scale_q=1.0)
+    if kind == "generic":
+        x = _dev(rs.standard_normal((M, 3 * 2 * 32)).astype(np.float16), device)
+        run = lambda **kw: ops.attention_generic_f16(x, _dev(bi, device), len(lens), S, 2, 0.125, False, **kw)
+    else:
+        fn = ops.attention_short if kind == "short" else ops.attention_grouped
+        run = lambda **kw: fn(_dev(qkv, device), _dev(bi, device), len(lens), S, 0.125, False, **kw)
+    base = run()
+    ops.set_option("prefetch_min_grid", min_grid)
+    try:
+        for k, n in ((768, 768), (3072, 768), (768, 3072), (64, 8), (576, 576), (192, 104)):
+            w = torch.full((k, n), 7, dtype=torch.float16, device=device)
+            for kn in (0, 1):
+                pitch = (n if kn else k) * 2
+                for halved in range(4):
+                    form = pitch // 64 | (3 - halved if kn else halved) << 16 | (0 if kn else 1) << 18
+                    _say("prefetch shares", kind, min_grid, k, n, kn, halved)
+                    got = run(prefetch=[(w, form), w, (w, form ^ 1), (w, 0xffff)])
+                    torch.cuda.synchronize()
+                    assert torch.equal(got[:M], base[:M]) and bool((w == 7).all())
+    finally:
+        ops.set_option("prefetch_min_grid", 512)
+
+
 @pytest.mark.parametrize("lens,S,heads", [([656], 656, 12), ([1024], 1024, 12), ([1024], 1024, 16), ([1088], 1088, 16),
                                           ([512, 300], 512, 12), ([640, 640], 640, 12)])
 def test_attention_prefetch_hint_leaves_the_choice_of_kernel(device, lens, S, heads):
