@@ -68,6 +68,7 @@ struct GemmArgs {
   int tile_grid;        // workgroups of the launch (set by the launcher)
   int splits;           // k slices (set by the launcher; 1 but for kEpiPartial)
   unsigned per_n;       // device only: inverse of tiles_n, for divide()
+  unsigned ratio, per_n_second;   // gemm_either_kernel (set by the launcher)
 };
 
 // Where a product takes its rows from, as a template parameter: the code that counts the mask rows is 9 KB,
@@ -101,12 +102,14 @@ struct GemmTail {
 };
 template <>
 struct GemmTail<kMaskNone> {
-  int tile_grid, unused[3];   // (see Launch: 16 bytes are issued faster than 4)
+  int tile_grid;
+  unsigned ratio, per_n_second;   // gemm_either_kernel
+  int unused;                     // (see Launch: 16 bytes are issued faster than 4)
 };
 template <int MASK>
 static GemmTail<MASK> gemm_tail(const GemmArgs &p) {
   if constexpr (MASK == kMaskNone)
-    return {p.tile_grid, {}};
+    return {p.tile_grid, p.ratio, p.per_n_second, 0};
   else
     return {p.tile_grid, p.mask_B, p.mask_S, p.out_word_idx, p.out_seq_order};
 }
@@ -1010,6 +1013,55 @@ __global__ __launch_bounds__((WM * WN + NP) * 64) void gemm_short_kernel(BT_GEMM
 #endif
 }
 
+// ---- one of two tiles ------------------------------------------------------------------
+// Products whose live rows only the device knows.  A tile is as good as the rounds of the chip that it takes, so the
+// one that suits up to 120 % of an expected row count takes 5 to 12 % longer than the best where fewer rows come, and
+// at the far side of a round's end the other way about.  Where two tiles of one workgroup size are each the better one
+// for some of the likely rows, the launch has both, and takes the one whose rounds cost less.
+// ratio: 256 x the second one's cost of a round over the first one's.
+// 12 layers without a row count, one tile and one of two, us: encoder 12 x 380 925 -> 896, 16 x 1024 2455 -> 2364, 20 x 200
+// 883 -> 846, 6 x 250 580 -> 567, per-layer entry 12 x 380 1064 -> 1020, 16 x 512 1583 -> 1527; where the rows are known nothing
+// changes, and a launch of two is asked to be 2.5 % better on the average of the likely rows (kPairMargin).  Of the
+// pairs whose workgroups go together these five have nearly all there is to gain.  Which is taken changes no bit.
+template <int BM_, int BN_, int STAGES_, int WM_, int WN_, int NP_>
+struct TileShape {
+  static constexpr int BM = BM_, BN = BN_, STAGES = STAGES_, WM = WM_, WN = WN_, NP = NP_;
+  static constexpr int kThreads = (WM * WN + NP) * 64;
+  static constexpr size_t kLds = (size_t)STAGES * (BM + BN) * kBK * sizeof(half_t);
+};
+constexpr int kEitherCus = 256;   // (of a chip with more or fewer the launcher makes no use of this)
+__host__ __device__ __forceinline__ int rounds_of(int rows, int bm, int tiles_n, int splits) {
+  return ((rows + bm - 1) / bm * tiles_n * splits + kEitherCus - 1) / kEitherCus;
+}
+__host__ __device__ __forceinline__ bool second_is_faster(int first_rounds, int second_rounds, unsigned ratio) {
+  return (unsigned)second_rounds * ratio < (unsigned)first_rounds * 256u;
+}
+template <typename A, typename B, int EPI, bool WKN>
+__global__ __launch_bounds__(A::kThreads > B::kThreads ? A::kThreads : B::kThreads) void gemm_either_kernel(BT_GEMM_FIRST, GemmTail<kMaskNone> tail) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  GemmArgs p = gemm_args<kMaskNone, A::BN>(BT_GEMM_FIRST_NAMES, tail);
+  const int M = min(*p.valid_rows, p.rows_cap), second_n = (p.N + B::BN - 1) / B::BN;
+  constexpr bool LOOP = EPI != kEpiPartial;
+  const auto run = [&](auto shape) {
+    using T = decltype(shape);
+    if (threadIdx.x >= T::kThreads) return;   // (whole waves; a barrier counts those that are left)
+    const auto tile = [&](int bid) {
+      return gemm_tile<T::BM, T::BN, T::STAGES, T::WM, T::WN, T::NP, EPI, WKN, kMaskNone, LOOP>(p, bid);
+    };
+    if constexpr (LOOP)
+      for_each_tile(p, tile);
+    else
+      tile((int)blockIdx.x);
+  };
+  if (second_is_faster(rounds_of(M, A::BM, p.tiles_n, p.splits), rounds_of(M, B::BM, second_n, p.splits), tail.ratio)) {
+    p.tiles_n = second_n, p.per_n = tail.per_n_second;
+    run(B{});
+  } else {
+    run(A{});
+  }
+#endif
+}
+
 // ---- a few rows: the waves share the k range, not the tile ----------------------------
 // One 32x32 tile per workgroup.  Its waves take the k-steps in turn (wave w: steps w, w + NW, ...),
 // each through a ring of its own that it fills and reads alone, so the loop has no barrier; their
@@ -1304,6 +1356,37 @@ static int launch_gemm_tile(GemmArgs p, hipStream_t s, int splits = 1) {
   });
 }
 
+template <typename A, typename B, int EPI>
+static int launch_gemm_either(GemmArgs p, hipStream_t s, unsigned ratio, int splits = 1) {
+  constexpr size_t smem = A::kLds > B::kLds ? A::kLds : B::kLds;
+  constexpr int kThreads = A::kThreads > B::kThreads ? A::kThreads : B::kThreads;
+  static_assert(smem <= 160 * 1024, "LDS budget");
+  p.splits = splits, p.ratio = ratio;
+  const auto grid = [&](int bm, int bn) {
+    p.tiles_n = (p.N + bn - 1) / bn;
+    const int all = ((p.rows_cap + bm - 1) / bm * p.tiles_n * splits + 7) / 8 * 8;
+    return EPI == kEpiPartial ? all : launched_tiles(p, bm, all) / 8 * 8;
+  };
+  const int second = grid(B::BM, B::BN);
+  p.per_n_second = inverse_of((unsigned)p.tiles_n);
+  const int first = grid(A::BM, A::BN);
+  p.tile_grid = first > second ? first : second;
+  const auto launch = [&](auto wkn) {
+    return with_first_arguments<kMaskNone>(p, [&](auto... arguments) {
+      return Launch<gemm_either_kernel<A, B, EPI, wkn()>>::on(s, "gemm_either_kernel", p.tile_grid, kThreads, smem, arguments...,
+                                                              gemm_tail<kMaskNone>(p));
+    });
+  };
+  return p.w_kn ? launch(std::true_type{}) : launch(std::false_type{});
+}
+using Tile1 = TileShape<128, 128, 3, 2, 2, 4>;
+using Tile2 = TileShape<256, 128, 3, 4, 2, 4>;
+using Tile3 = TileShape<256, 192, 2, 4, 2, 4>;
+using Tile9 = TileShape<64, 64, 4, 2, 2, 4>;
+using Tile10 = TileShape<64, 128, 3, 2, 2, 4>;
+using Tile11 = TileShape<96, 128, 3, 3, 2, 4>;
+using Tile12 = TileShape<128, 192, 3, 2, 2, 4>;
+
 template <int EPI, bool WKN, int MASK>
 static int launch_gemm_wave_k_as(GemmArgs p, hipStream_t s, int splits) {
   // (and 256 bytes for the lengths of a launch that counts the mask rows)
@@ -1507,6 +1590,86 @@ static bool tuned_mean(const LikelyRows &likely, int n, int k, int epi, int kn, 
   return true;
 }
 
+// The fastest tile for the likely rows: the model's, unless the table knows a clear win.
+static int fastest_tile(const GemmArgs &p, int epi) {
+  const LikelyRows likely(p);
+  float us[kTunedTiles];
+  int choice = fastest_by_model(likely, p.N, p.K, p.mask != nullptr);
+  // the table overrides the model only for a clear win: the timings come from a loop
+  // of identical launches, and differences of a few per cent do not carry over to the
+  // layer sequence
+  // (a launch whose estimated live rows fill its capacity to within one tile row is looked
+  // up among the all-live measurements)
+  if (tuned_mean(likely, p.N, p.K, epi, p.w_kn, estimated_rows(p) + kTunedStep > p.rows_cap, us)) {
+    if (p.mask)
+      for (int t = 0; t < kTunedTiles; ++t)
+        for (int i = 0; us[t] > 0.f && i < likely.count; ++i)
+          us[t] += likely.weight[i] * mask_rounds_us(t, likely.rows[i], p.N);
+    int tuned = -1;
+    for (int t = 0; t < kTunedTiles; ++t)
+      if (us[t] > 0.f && (tuned < 0 || us[t] < us[tuned])) tuned = t;
+    const float t_model = us[choice];
+    const float margin = 1.f - 0.01f * (float)option_gemm_table_margin();
+    if (tuned >= 0 && tuned != choice && (t_model <= 0.f || us[tuned] < margin * t_model))
+      choice = tuned;
+  }
+  return choice;
+}
+
+// The pairs that a launch may have (gemm_either_kernel), and what is asked of one beyond the fastest tile's time.
+struct TilePair {
+  int first, first_bm, first_bn, second, second_bm, second_bn;
+};
+static const TilePair kTilePairs[] = {
+    {9, 64, 64, 10, 64, 128}, {10, 64, 128, 1, 128, 128}, {10, 64, 128, 11, 96, 128},
+    {1, 128, 128, 12, 128, 192}, {2, 256, 128, 3, 256, 192}};
+constexpr float kPairMargin = 0.975f, kPairChoiceUs = 0.1f;
+
+// The fastest pair for `count` likely rows, given the times of both tiles at each: its number from 1 on (0: none below
+// `most_us`), and the ratio by which the device picks.
+template <typename Us>
+static int fastest_pair(const LikelyRows &likely, int n, int splits, int pairs, float most_us, unsigned &ratio, Us us) {
+  int best = 0;
+  for (int q = 0; q < pairs; ++q) {
+    const TilePair &c = kTilePairs[q];
+    float first[5], second[5], first_round = 0.f, second_round = 0.f;
+    int first_rounds[5], second_rounds[5];
+    for (int i = 0; i < likely.count; ++i) {
+      first[i] = us(c.first, i), second[i] = us(c.second, i);
+      first_rounds[i] = rounds_of((int)likely.rows[i], c.first_bm, (n + c.first_bn - 1) / c.first_bn, splits);
+      second_rounds[i] = rounds_of((int)likely.rows[i], c.second_bm, (n + c.second_bn - 1) / c.second_bn, splits);
+      first_round += likely.weight[i] * first[i] / (float)first_rounds[i];
+      second_round += likely.weight[i] * second[i] / (float)second_rounds[i];
+    }
+    const unsigned r = (unsigned)(256.f * second_round / first_round + 0.5f);
+    float t = kPairChoiceUs;
+    for (int i = 0; i < likely.count; ++i)
+      t += likely.weight[i] * (second_is_faster(first_rounds[i], second_rounds[i], r) ? second[i] : first[i]);
+    if (t < most_us && r < (1u << 20)) best = q + 1, most_us = t, ratio = r;
+  }
+  return best;
+}
+
+// For a launch that knows no row count: its tile | its pair << 4 | the pair's ratio << 8.
+static int tile_or_pair(const GemmArgs &p, int epi) {
+  const LikelyRows likely(p);
+  const int tile = fastest_tile(p, epi);
+  const float *table[5];
+  for (int i = 0; i < likely.count; ++i)
+    table[i] = tuned_times(likely.rows[i], p.N, p.K, epi, p.w_kn, estimated_rows(p) + kTunedStep > p.rows_cap);
+  const auto us = [&](int id, int i) {
+    if (table[i] && table[i][id] > 0.f) return table[i][id];
+    for (const TileModel &c : kTileModels)
+      if (c.id == id) return model_us(c, likely.rows[i], p.N, p.K);
+    return 0.f;
+  };
+  float one = 0.f;
+  for (int i = 0; i < likely.count; ++i) one += likely.weight[i] * us(tile, i);
+  unsigned ratio = 0;
+  const int pair = fastest_pair(likely, p.N, 1, 5, kPairMargin * one, ratio, us);
+  return tile | pair << 4 | (int)(ratio << 8);
+}
+
 // How a product runs on tile 14, whose waves share k and add up in an order of their own: a row count that a
 // caller knows in one call and not in the next must not change a bit, so this follows from sizes, and from the
 // live rows themselves.  A workgroup fills its CU's LDS, so its tiles have to fit one round: us of tile 14 / tile
@@ -1630,29 +1793,20 @@ static int launch_gemm(GemmArgs p, hipStream_t s) {
     if (few == kWaveKDevice) return launch_gemm_few_rows(p, s);
     if (few == kWaveKYes) choice = 14;
   }
-  if (choice < 0) {
-    const LikelyRows likely(p);
-    float us[kTunedTiles];
-    choice = fastest_by_model(likely, p.N, p.K, p.mask != nullptr);
-    // the table overrides the model only for a clear win: the timings come from a loop
-    // of identical launches, and differences of a few per cent do not carry over to the
-    // layer sequence
-    // (a launch whose estimated live rows fill its capacity to within one tile row is looked
-    // up among the all-live measurements)
-    if (tuned_mean(likely, p.N, p.K, EPI, p.w_kn, estimated_rows(p) + kTunedStep > p.rows_cap, us)) {
-      if (p.mask)
-        for (int t = 0; t < kTunedTiles; ++t)
-          for (int i = 0; us[t] > 0.f && i < likely.count; ++i)
-            us[t] += likely.weight[i] * mask_rounds_us(t, likely.rows[i], p.N);
-      int tuned = -1;
-      for (int t = 0; t < kTunedTiles; ++t)
-        if (us[t] > 0.f && (tuned < 0 || us[t] < us[tuned])) tuned = t;
-      const float t_model = us[choice];
-      const float margin = 1.f - 0.01f * (float)option_gemm_table_margin();
-      if (tuned >= 0 && tuned != choice && (t_model <= 0.f || us[tuned] < margin * t_model))
-        choice = tuned;
+  if (choice < 0 && p.valid_rows && !p.mask && p.rows_hint <= 0 && cu_count() == kEitherCus) {
+    const int answer = remembered({p.rows_cap, p.N, p.K, p.w_kn, option_gemm_table_margin()}, [&] { return tile_or_pair(p, EPI); });
+    const unsigned ratio = (unsigned)answer >> 8;
+    choice = answer & 15;
+    switch (answer >> 4 & 15) {
+      case 1: return launch_gemm_either<Tile9, Tile10, EPI>(p, s, ratio);
+      case 2: return launch_gemm_either<Tile10, Tile1, EPI>(p, s, ratio);
+      case 3: return launch_gemm_either<Tile10, Tile11, EPI>(p, s, ratio);
+      case 4: return launch_gemm_either<Tile1, Tile12, EPI>(p, s, ratio);
+      case 5: return launch_gemm_either<Tile2, Tile3, EPI>(p, s, ratio);
+      default: break;
     }
   }
+  if (choice < 0) choice = fastest_tile(p, EPI);
   switch (choice) {
     case 14:
       return launch_gemm_wave_k<EPI>(p, s);
@@ -1823,16 +1977,32 @@ extern "C" int bt_gemm_splitk_rows(const void *a, const void *wt, void *partials
              rows_cap,          n,                  k,       0,       rows_hint,  (float *)partials,
              weight_kn};
   hipStream_t st = as_stream(stream);
-  const int tile = remembered({rows_cap, valid_rows != nullptr, rows_hint, n, k, splits}, [&] {
+  const int answer = remembered({rows_cap, valid_rows != nullptr, rows_hint, n, k, splits}, [&] {
     float us = 0.f;
-    const int named = fastest_sliced(LikelyRows(p), n, k, splits, &us).id;
-    if (rows_hint <= 0) return named;
+    const LikelyRows likely(p);
+    const int named = fastest_sliced(likely, n, k, splits, &us).id;
+    if (rows_hint <= 0) {
+      unsigned ratio = 0;
+      const auto at = [&](int id, int i) {
+        for (const SliceModel &c : kSliceModels)
+          if (c.id == id) return slice_pair_us(c, likely.rows[i], n, k, splits);
+        return 0.f;
+      };
+      const bool either = valid_rows && named != 14 && splits > 1 && cu_count() == kEitherCus;
+      const int pair = either ? fastest_pair(likely, n, splits, 3, kPairMargin * us, ratio, at) : 0;
+      return named | pair << 4 | (int)(ratio << 8);
+    }
     // (the waves of tile 14 add up in an order of their own: not for a row count's sake either)
     GemmArgs unnamed = p;
     unnamed.rows_hint = 0;
     const int without = fastest_sliced(LikelyRows(unnamed), n, k, splits, &us).id;
     return (named == 14) != (without == 14) ? without : named;
   });
+  const unsigned ratio = (unsigned)answer >> 8;
+  if ((answer >> 4 & 15) == 1) return launch_gemm_either<Tile9, Tile10, kEpiPartial>(p, st, ratio, splits);
+  if ((answer >> 4 & 15) == 2) return launch_gemm_either<Tile10, Tile1, kEpiPartial>(p, st, ratio, splits);
+  if ((answer >> 4 & 15) == 3) return launch_gemm_either<Tile10, Tile11, kEpiPartial>(p, st, ratio, splits);
+  const int tile = answer & 15;
   switch (tile) {
     case 14: return launch_gemm_wave_k<kEpiPartial>(p, st, splits);
     case 4: return launch_gemm_tile<32, 64, 4, 1, 2, 2, kEpiPartial>(p, st, splits);

@@ -1367,6 +1367,48 @@ def test_attention_prefetch_hint_changes_nothing(device, kind, lens, S):
         ops.set_option("prefetch_min_grid", 512)
 
 
+@pytest.mark.parametrize("kind,n,k", [("plain", 768, 768), ("plain", 768, 3072), ("gelu", 3072, 768), ("qkv", 2304, 768),
+                                      ("plain", 640, 1280), ("partial", 768, 3072)])
+@pytest.mark.parametrize("w_kn", [False, True])
+def test_gemm_without_a_row_count_gives_the_bits_of_one_tile(device, kind, n, k, w_kn):
+    """Capacities at which a launch without a row count has one of two tiles, and the other's; few rows, both sides of a
+    round's end, all rows: the bits of the 128x128 tile, and nothing written past the live rows."""
+    rs = np.random.RandomState(n + k)
+    most = 1900 if kind == "partial" else 9000
+    a = _dev(rs.standard_normal((most, k)).astype(np.float16), device)
+    w = _dev((rs.standard_normal((k, n) if w_kn else (n, k)) * 0.05).astype(np.float16), device)
+    bias = _dev(rs.standard_normal(n).astype(np.float16), device)
+
+    def run(cap, vr):
+        if kind == "plain":
+            return ops.gemm(a[:cap], w, valid_rows=vr, out=torch.full((cap, n), 7.0, dtype=torch.float16, device=device), w_kn=w_kn)
+        if kind == "gelu":
+            return ops.gemm_bias_gelu(a[:cap], w, bias, valid_rows=vr, w_kn=w_kn,
+                                      out=torch.full((cap, n), 7.0, dtype=torch.float16, device=device))
+        if kind == "qkv":
+            out = torch.full((3, n // 192, cap, 64), 7.0, dtype=torch.float16, device=device)
+            return ops.gemm_qkv_bias_split(a[:cap], w, bias, n // 192, valid_rows=vr, w_kn=w_kn, out=out)
+        return ops.gemm_splitk(a[:cap], w, 3, valid_rows=vr, w_kn=w_kn)
+
+    for cap in ((900, 1500, 1900) if kind == "partial" else (1400, 2300, 2600, 3700, 4100, 4560, 5100, 6400, 8100, 9000)):
+        for M in (1, cap // 3, cap * 55 // 100, cap * 66 // 100, cap):
+            _say("two tiles", kind, n, k, w_kn, cap, M)
+            vr = torch.tensor([M], dtype=torch.int32, device=device)
+            got = run(cap, vr)
+            if kind == "partial":      # (no tile to pin: against float64, and the slices' own places)
+                wk = (w if w_kn else w.t()).double()
+                ref, size = a[:M].double() @ wk, a[:M].double().abs() @ wk.abs()
+                # (exact products; a float sum rounds once per 32 of k)
+                assert ((got[:, :M].double().sum(0) - ref).abs() <= k / 32 * 2.0 ** -24 * size).all()
+                continue
+            ops.set_option("gemm_tile", 1)
+            try:
+                one = run(cap, vr)
+            finally:
+                ops.set_option("gemm_tile", -1)
+            assert torch.equal(got, one)
+
+
 @pytest.mark.parametrize("kind", ["short", "grouped", "generic"])
 @pytest.mark.parametrize("min_grid", [512, 1])
 def test_attention_prefetch_of_shared_weights_changes_nothing(device, kind, min_grid):
