@@ -202,6 +202,28 @@ def test_build_offsets_threshold(device):
     assert np.array_equal(g_wi.cpu().numpy()[:M], wi)
 
 
+@pytest.mark.parametrize("dtype", [np.float16, np.float32])
+def test_mask_rows_of_any_length_are_counted_once(device, dtype):
+    """Rows of scattered ones whose length is a whole number of pieces or not, shorter than one, one wave's and one loop
+    turn's, through the offsets launch and the product that counts for itself."""
+    rs = np.random.RandomState(3)
+    w, bias = _dev(rs.standard_normal((192, 64)).astype(np.float16), device), _dev(np.zeros(192, np.float16), device)
+    for S in (1, 3, 4, 5, 7, 8, 9, 63, 64, 65, 66, 71, 72, 100, 127, 129, 217, 255, 257, 511, 513, 1027, 2047, 2050):
+        B = 7 if S < 600 else 3
+        mask = np.zeros((B, S, S), dtype)
+        mask[:, 0] = rs.randint(0, 2, (B, S))
+        mask[1, 0], mask[2, 0] = 1, 0
+        _say("mask rows", S, dtype)
+        bi, wi, M = O.build_offsets(mask)
+        m = _dev(mask, device)
+        g_bi, g_wi, g_M = ops.build_offsets(m, want_count=True)
+        assert g_M == M and np.array_equal(g_bi.cpu().numpy(), bi) and np.array_equal(g_wi.cpu().numpy()[:M], wi), S
+        if B * S * mask.itemsize <= 64 * 1024:
+            x = torch.zeros(B, S, 64, dtype=torch.float16, device=device)
+            _, q_bi, q_wi, _ = ops.gemm_qkv_bias_split_mask_rows(x, m, w, bias, 1)
+            assert np.array_equal(q_bi.cpu().numpy(), bi) and np.array_equal(q_wi.cpu().numpy()[:M], wi), S
+
+
 # ---- compress / restore (bit-exact copies) -------------------------------------
 @pytest.mark.parametrize("B,S,H", [(4, 50, 768), (16, 512, 768), (3, 9, 1024), (2, 5, 8)])
 def test_compress_bit_exact(device, B, S, H):
