@@ -64,7 +64,7 @@ struct Launch<Kernel> {
   // 0 or a BT status
   static int on(hipStream_t s, const char *what, unsigned grid, unsigned threads, size_t lds, P... args) {
     hipFunction_t f = nullptr;
-    int rc = function(&f, what, lds > 64 * 1024);
+    int rc = function(&f, s, what, lds > 64 * 1024);
     if (rc != BT_OK) return rc;
     alignas(16) unsigned char packed[kBytes];
     size_t at = 0;
@@ -89,17 +89,22 @@ struct Launch<Kernel> {
     __builtin_memcpy(to + at, &v, sizeof(T));
     at += sizeof(T);
   }
-  static int function(hipFunction_t *f, const char *what, bool large_lds) {
+  // The kernel on the stream's device (a launch by <<<>>> goes there too, whatever the current device is).
+  static int function(hipFunction_t *f, hipStream_t s, const char *what, bool large_lds) {
     static std::atomic<hipFunction_t> known[2][kMaxDevices];   // with the limit as it is, and raised
     int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return hip_fail(e, "hipGetDevice");
+    const bool named = reinterpret_cast<uintptr_t>(s) <= 2;   // null, hipStreamLegacy, hipStreamPerThread: the current device's
+    hipError_t e = named ? hipGetDevice(&dev) : hipStreamGetDevice(s, &dev);
+    if (e != hipSuccess) return hip_fail(e, what);
     const bool kept = dev >= 0 && dev < kMaxDevices;
     if (kept && (*f = known[large_lds][dev].load(std::memory_order_acquire))) return BT_OK;
-    if (large_lds &&
-        (e = hipFuncSetAttribute((const void *)Kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMostLds)) != hipSuccess)
-      return hip_fail(e, what);
-    if ((e = hipGetFuncBySymbol(f, (const void *)Kernel)) != hipSuccess) return hip_fail(e, what);
+    int current = dev;
+    if ((e = hipGetDevice(&current)) == hipSuccess && current != dev) e = hipSetDevice(dev);
+    if (e == hipSuccess && large_lds)
+      e = hipFuncSetAttribute((const void *)Kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMostLds);
+    if (e == hipSuccess) e = hipGetFuncBySymbol(f, (const void *)Kernel);
+    if (current != dev) (void)hipSetDevice(current);
+    if (e != hipSuccess) return hip_fail(e, what);
     if (kept) known[large_lds][dev].store(*f, std::memory_order_release);
     return BT_OK;
   }

@@ -106,6 +106,21 @@ def _gemm_splitk(*a, **k):
     return ops.gemm_splitk(*a, w_kn=_KN[0], **k)
 
 
+@pytest.mark.parametrize("which", ["null", "per_thread", "own"])
+def test_launches_go_to_the_stream_they_are_given(device, which):
+    """Null, the per-thread handle (hipStreamPerThread, 2) and a stream of one's own: the launch finds its kernel on each."""
+    own = torch.cuda.Stream(device)
+    handle = {"null": 0, "per_thread": 2, "own": own.cuda_stream}[which]
+    src, dst = torch.arange(7, 9, dtype=torch.int32, device=device), torch.zeros(2, dtype=torch.int32, device=device)
+    torch.cuda.synchronize()
+    for i in range(2):
+        rc = _lib.kernel_lib().bt_publish_int(ctypes.cast(src[i:].data_ptr(), ctypes.POINTER(ctypes.c_int)),
+                                              dst[i:].data_ptr(), handle)
+        assert rc == 0
+    torch.cuda.synchronize()
+    assert dst.tolist() == [7, 8]
+
+
 @pytest.mark.parametrize("B,S,dtype", [(1, 256, np.float16), (16, 512, np.float16),
                                        (3, 7, np.float32), (70, 33, np.float16),
                                        (130, 100, np.float16), (2, 1024, np.float16)])
