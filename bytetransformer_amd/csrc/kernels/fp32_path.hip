@@ -530,7 +530,8 @@ struct F32AttArgs {
 
 constexpr int kF32KT = 32;   // keys per tile
 
-// One workgroup = NW waves x 32 queries of one (sequence, head).  The logits are computed
+// One workgroup = NQ waves x 32 queries of one (sequence, head); KS groups of such waves share the keys, group g taking
+// the tiles g, g + KS, ..., and fold through LDS.  The logits are computed
 // transposed, S^T = K.Q^T (lane = query, 16 keys per lane), so their accumulator is
 // directly the "B" operand of O^T = V^T.P^T and the softmax statistics of a query are
 // lane-local up to one exchange between the two halves of the wave.  The MFMA's k index
@@ -543,13 +544,15 @@ constexpr int kF32KT = 32;   // keys per tile
 // loop, and behind it read the last one 7 wait states after the last matrix instruction, which takes 18 -
 // wrong last columns at head sizes 96 and 128, another way in every run.  (tests/test_kernel_resources.py
 // looks for such reads in every kernel.)
-template <int ND, int NW>
-__global__ __launch_bounds__(64 * NW, 2) void f32_attention_kernel(F32AttArgs p) {
+template <int ND, int NQ, int KS>
+__global__ __launch_bounds__(64 * NQ * KS, 2) void f32_attention_kernel(F32AttArgs p) {
   constexpr int D = 32 * ND;
-  constexpr int THREADS = 64 * NW, BQ = 32 * NW;   // 32 queries per wave
+  constexpr int THREADS = 64 * NQ * KS, BQ = 32 * NQ;   // 32 queries per wave
+  constexpr int STEP = kF32KT * KS;                     // keys of a turn
   constexpr int SK = D + 4, SV = D + 8;
-  __shared__ __attribute__((aligned(16))) float sK[kF32KT * SK];
-  __shared__ __attribute__((aligned(16))) float sV[kF32KT * SV];
+  __shared__ __attribute__((aligned(16))) float smem[STEP * (SK + SV)];
+  float *const sK = smem, *const sV = smem + STEP * SK;
+  static_assert(KS == 1 || NQ * 64 * (16 * ND + 2) <= STEP * (SK + SV), "a group's sums fit the tiles' place");
 
   // 1-D grid, XCD-aware: the hardware deals consecutive workgroup ids round-robin to the
   // 8 XCDs; XCD x works on the (sequence, head) pairs p = x (mod 8), the query tiles of
@@ -588,7 +591,8 @@ __global__ __launch_bounds__(64 * NW, 2) void f32_attention_kernel(F32AttArgs p)
     return;
   }
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave_all = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = wave_all % NQ, group = wave_all / NQ;
   const int l32 = lane & 31, half = lane >> 5;
   const int d = p.d;
   const int H = p.heads * d;
@@ -598,7 +602,7 @@ __global__ __launch_bounds__(64 * NW, 2) void f32_attention_kernel(F32AttArgs p)
   const float *V = K + H;
 
   const int q = q0 + wave * 32 + l32;       // this lane's query
-  const bool wave_live = q0 + wave * 32 < nq;
+  const bool query_live = q0 + wave * 32 < nq;
   const int qc = min(q, nq - 1);
 
   // Q^T operand: lane (query, half) holds Q[q][half*D/2 + i]
@@ -612,9 +616,9 @@ __global__ __launch_bounds__(64 * NW, 2) void f32_attention_kernel(F32AttArgs p)
     for (int j = 0; j < 4; ++j) qf[4 * i + j] = v[j];
   }
 
-  // tile staging: 32 keys x D floats of K and of V, NV float4 each per thread
+  // tile staging: 32 KS keys x D floats of K and of V, NV float4 each per thread
   constexpr int CPR = D / 4;   // float4 per row
-  constexpr int NV = kF32KT * CPR / THREADS;
+  constexpr int NV = STEP * CPR / THREADS;
   float4_t rk[NV], rv[NV];
   auto fetch = [&](int k0) {
 #pragma unroll
@@ -650,14 +654,15 @@ __global__ __launch_bounds__(64 * NW, 2) void f32_attention_kernel(F32AttArgs p)
   const float *mrow = p.mask ? p.mask + ((size_t)b * p.S + min(q, p.S - 1)) * p.S : nullptr;
   const float *brow = p.bias ? p.bias + ((size_t)head * p.S + min(q, p.S - 1)) * p.S : nullptr;
 
-  const int ntiles = (klen + kF32KT - 1) / kF32KT;
+  const int turns = (klen + STEP - 1) / STEP;
   fetch(0);
   stash();
   __syncthreads();
   const bool has_add = mrow || brow;
   const bool add_vec = (p.S & 3) == 0;
-  for (int t = 0; t < ntiles; ++t) {
-    const int k0 = t * kF32KT;
+  for (int t = 0; t < turns; ++t) {
+    const int k0 = t * STEP + group * kF32KT;
+    const bool wave_live = query_live && k0 < klen;
     // additive terms of this tile's 16 keys per lane (4 groups of 4 consecutive keys),
     // in the exp2 domain; issued ahead of the next tile's K / V so that the wait for
     // them does not include those
@@ -681,13 +686,13 @@ __global__ __launch_bounds__(64 * NW, 2) void f32_attention_kernel(F32AttArgs p)
         add[g] = (mv - 1.0f) * (10000.0f * kLog2eF) + bv * kLog2eF;
       }
     }
-    if (t + 1 < ntiles) fetch((t + 1) * kF32KT);
+    if (t + 1 < turns) fetch((t + 1) * STEP);
     if (wave_live) {
       // S^T = K . Q^T : A operand K[key = l32][k = half*D/2 + i]
       float16_t s;
 #pragma unroll
       for (int i = 0; i < 16; ++i) s[i] = 0.f;
-      const float *kp = &sK[l32 * SK + half * (D / 2)];
+      const float *kp = &sK[(group * kF32KT + l32) * SK + half * (D / 2)];
 #pragma unroll
       for (int i4 = 0; i4 < D / 8; ++i4) {
         const float4_t kv = *(const float4_t *)(kp + 4 * i4);
@@ -731,20 +736,45 @@ __global__ __launch_bounds__(64 * NW, 2) void f32_attention_kernel(F32AttArgs p)
       // O^T += V^T . P^T : A operand V[key(j, half)][d = 32*dt + l32], B operand P^T = x[j]
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
-        const float *vp = &sV[(8 * (j >> 2) + 4 * half + (j & 3)) * SV + l32];
+        const float *vp = &sV[(group * kF32KT + 8 * (j >> 2) + 4 * half + (j & 3)) * SV + l32];
 #pragma unroll
         for (int dt = 0; dt < ND; ++dt)
           o[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(vp[32 * dt], x[j], o[dt], 0, 0, 0);
       }
     }
     __syncthreads();
-    if (t + 1 < ntiles) {
+    if (t + 1 < turns) {
       stash();
       __syncthreads();
     }
   }
 
-  if (!wave_live || q >= nq) return;
+  // The other groups' sums come to the first one's waves by way of the tiles' place, which nobody reads any more.
+#pragma unroll
+  for (int g = 1; g < KS; ++g) {
+    float *const to = smem + wave * 64 * (16 * ND + 2) + lane;
+    if (group == g) {
+      to[0] = m_run, to[64] = l_run;
+#pragma unroll
+      for (int dt = 0; dt < ND; ++dt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) to[64 * (2 + 16 * dt + i)] = o[dt][i];
+    }
+    __syncthreads();
+    if (group == 0) {
+      const float m_new = fmaxf(m_run, to[0]);
+      const float mine = __builtin_amdgcn_exp2f(m_run - m_new), theirs = __builtin_amdgcn_exp2f(to[0] - m_new);
+      m_run = m_new;
+      l_run = l_run * mine + to[64] * theirs;
+#pragma unroll
+      for (int dt = 0; dt < ND; ++dt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[dt][i] = o[dt][i] * mine + to[64 * (2 + 16 * dt + i)] * theirs;
+    }
+    if (g + 1 < KS) __syncthreads();
+  }
+
+  if (group > 0 || !query_live || q >= nq) return;
   const float l_all = l_run + __shfl_xor(l_run, 32, 64);
   const float inv = 1.0f / (l_all + 1e-6f);
   // accumulator element i of d-tile dt: d = 32*dt + 8*(i/4) + 4*half + i%4, query = l32
@@ -1012,8 +1042,19 @@ extern "C" int bt_attention_f32(const void *qkv, void *out, const int *batch_idx
                (const float *)attention_bias, batch_size, seq_len, rows_cap, head_num, scale,
                padded_rows ? 1 : 0};
   p.d = size_per_head;
-  constexpr int kWaves = 4;    // 128 queries per workgroup (two-wave workgroups measured slower)
-  p.nqb = (seq_len + 32 * kWaves - 1) / (32 * kWaves);
+  // 64 queries whose keys two groups of waves share, or 128 (heads beyond 64 have no room in 64 KB of LDS for two groups'
+  // tiles).  A turn is 5000 clocks of dependent matrix instructions, so a launch of few workgroups is as long as its
+  // longest sequence has turns: us, 128 queries / shared, 12 heads of 64, lengths 0.2 to 1 of the maximum, 1 x 256
+  // 8.5 / 6.8, 2 x 100 8.4 / 6.7, 10 x 200 21.2 / 18.4, 16 x 256 34.3 / 23.4, 4 x 640 62.5 / 58.0, full 1 x 1024 91.0 / 52.0; 24 heads
+  // of 32, 7 x 333 27.1 / 17.4.  Up to 64 tokens the second group has next to nothing (1 x 64 5.6 / 6.3, 128 x 20 21.8 / 24.1);
+  // beyond two rounds of workgroups they are even (16 x 512 56.8 / 59.2, 32 x 512 121 / 117).  Against float64 the shared sums
+  // are the nearer ones (16 x 256 3.7e-7 / 3.4e-7, 1 x 1024 6.5e-7 / 5.0e-7).
+  // In a layer of 16 x 256, with the mask's rows, 41.8 / 32.6 us; 12 layers 2936 / 2824.
+  const int qb = option_attention_qb();
+  const long long blocks128 = (long long)((seq_len + 127) / 128) * head_num * batch_size;
+  const bool shared_keys = size_per_head <= 64 && (qb < 0 ? seq_len > 64 && blocks128 <= 2LL * cu_count() : qb == 1);
+  const int queries = shared_keys ? 64 : 128;   // of a workgroup
+  p.nqb = (seq_len + queries - 1) / queries;
   // the conditions of the fp16 streaming kernel: from the third round of 32 workgroups
   // per XCD on and up to 128 sequences, or always / never by the option
   const unsigned per_xcd = ((unsigned)batch_size * head_num + 7) / 8 * p.nqb;
@@ -1021,12 +1062,17 @@ extern "C" int bt_attention_f32(const void *qkv, void *out, const int *batch_idx
   p.balanced = order == 3 || (order == 2 && per_xcd > 64 && batch_size <= 128);
   const unsigned grid = p.balanced ? (per_xcd + 31) / 32 * 32 * 8 : per_xcd * 8;
   hipStream_t s = as_stream(stream);
-  const auto with = [&](auto nd) { return Launch<f32_attention_kernel<nd(), kWaves>>::on(s, who, grid, 64 * kWaves, 0, p); };
+  const auto with = [&](auto nd, auto nq, auto ks) {
+    return Launch<f32_attention_kernel<nd(), nq(), ks()>>::on(s, who, grid, 256, 0, p);
+  };
+  using one = std::integral_constant<int, 1>;
+  using two = std::integral_constant<int, 2>;
+  using four = std::integral_constant<int, 4>;
   switch ((size_per_head + 31) / 32) {
-    case 1: return with(std::integral_constant<int, 1>{});
-    case 2: return with(std::integral_constant<int, 2>{});
-    case 3: return with(std::integral_constant<int, 3>{});
-    default: return with(std::integral_constant<int, 4>{});
+    case 1: return shared_keys ? with(one{}, two{}, two{}) : with(one{}, four{}, one{});
+    case 2: return shared_keys ? with(two{}, two{}, two{}) : with(two{}, four{}, one{});
+    case 3: return with(std::integral_constant<int, 3>{}, four{}, one{});
+    default: return with(four{}, four{}, one{});
   }
 }
 

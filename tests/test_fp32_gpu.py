@@ -512,6 +512,46 @@ def test_attention_f32_mask_and_bias(device, padded, att_order):
         assert err.max() <= 2e-5, (b, err.max())
 
 
+@pytest.mark.parametrize("add", [False, True])
+@pytest.mark.parametrize("padded", [False, True])
+@pytest.mark.parametrize("lens,S,heads,d", [([65, 1, 0, 33], 65, 3, 64), ([128, 96, 64, 32], 128, 2, 64), ([97, 31], 97, 5, 40),
+                                            ([129, 63, 95], 131, 3, 32), ([16, 5], 16, 2, 8), ([400], 400, 1, 56)])
+def test_attention_f32_on_shared_keys(device, lens, S, heads, d, padded, add, att_order):
+    """64 queries whose keys two groups of waves share, and 128: lengths about a group's tile (32) and a turn (64), a group
+    without a key, a sequence without any. Sums of n keys in two orders, each of them off by at most a few n 2^-24 of values
+    of O(1): 2e-5, as in the tests above."""
+    rs = np.random.RandomState(S + heads + d)
+    B, H = len(lens), heads * d
+    bi = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    qkv = rs.standard_normal((B * S, 3 * H)).astype(np.float32)
+    if not padded:
+        qkv[bi[-1]:] = np.nan
+    mask = bias = None
+    if add:
+        bias = rs.standard_normal((heads, S, S)).astype(np.float32)
+        mask = (rs.rand(B, S, S) < 0.6).astype(np.float32)
+        mask[:, :, 0] = 1
+        if not padded:
+            for b, n in enumerate(lens):
+                mask[b, :, n:] = 0
+    scale = 1 / math.sqrt(d)
+    exp = _naive_attention(qkv, lens, S, heads, d, scale, padded, mask, bias)
+    on = [None if t is None else _dev(t, device) for t in (mask, bias)]
+    for qb in (1, 2):
+        ops.set_option("attention_qb", qb)
+        try:
+            g = ops.attention_f32(_dev(qkv, device), _dev(bi, device), B, S, heads, scale, padded_rows=padded, mask=on[0],
+                                  bias=on[1]).cpu().numpy()
+        finally:
+            ops.set_option("attention_qb", -1)
+        for b, n in enumerate(lens):
+            r0, nq = (b * S, S) if padded else (bi[b], n)
+            if n == 0:
+                continue
+            err = np.abs(g[r0:r0 + nq] - exp[r0:r0 + nq])
+            assert err.max() <= 2e-5, (qb, b, err.max())
+
+
 @pytest.mark.parametrize("padded", [False, True])
 @pytest.mark.parametrize("lens,S,heads,d", [([70, 9, 33], 72, 2, 128), ([40, 33], 40, 4, 32),
                                             ([150, 64, 1], 160, 2, 96), ([64, 38], 64, 3, 64),
