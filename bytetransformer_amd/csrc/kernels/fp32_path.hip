@@ -867,7 +867,7 @@ __device__ __forceinline__ void f32_layernorm_block(
   }
   const float rstd = rsqrtf(wave_sum(sq) * inv_n + eps);
   float4_t *o = dst + (size_t)r * chunks;
-  float most = 0.f, norm = 0.f;
+  float most = 0.f;
 #pragma unroll
   for (int i = 0; i < NC; ++i) {
     const int c = lane + i * kWave;
@@ -879,7 +879,6 @@ __device__ __forceinline__ void f32_layernorm_block(
       for (int e = 0; e < 4; ++e) {
         const float x = __builtin_fabsf(v[i][e]);
         most = fmaxf(most, x < __builtin_inff() ? x : 0.f);
-        norm += v[i][e] * v[i][e];
       }
   }
   if (PAIRS) {
@@ -890,16 +889,21 @@ __device__ __forceinline__ void f32_layernorm_block(
     }
     const int e = split_exponent(wave_max(most));
     const float scale = split_power(e);
+    float norm = 0.f;   // of the scaled row: at most 2^30 H
 #pragma unroll
     for (int i = 0; i < NC; ++i) {
       const int c = lane + i * kWave;
-      if (c < chunks) split_store(next.pairs + (size_t)r * chunks * 8, c, v[i] * scale);
+      if (c >= chunks) continue;
+      const float4_t x = v[i] * scale;
+      split_store(next.pairs + (size_t)r * chunks * 8, c, x);
+      norm += x[0] * x[0] + x[1] * x[1] + x[2] * x[2] + x[3] * x[3];
     }
-    // (where the bound is not finite neither are the results, or all of them are zero)
-    const float bound = sqrtf(wave_sum(norm) * (float)(chunks * 4)) * wave_max(w_most) + wave_max(bias_most);
+    // (a bound that is no float is the largest float: finite results fit it, and a row with an infinity or NaN has none)
+    const float row_norm = sqrtf(wave_sum(norm) * (float)(chunks * 4)) * split_power(-e);
+    const float bound = fminf(row_norm * wave_max(w_most) + wave_max(bias_most), 3.402823466e38f);
     if (lane == 0) {
       next.exps[r] = e;
-      next.gelu_exps[r] = bound < __builtin_inff() ? split_exponent(bound) : 0;
+      next.gelu_exps[r] = split_exponent(bound);
     }
   }
 }

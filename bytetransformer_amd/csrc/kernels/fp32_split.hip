@@ -50,7 +50,7 @@ struct SplitArgs {
   int count, units;
   int bounded;              // the weight that `bounds` speaks of, -1: none
   const float *bias;        // [N] its bias
-  float *bounds;            // [units of that weight][2]: largest |w| and largest |bias| of its columns
+  float *bounds;            // [units of that weight][2]: largest finite |w| and |bias| of its columns
   const float *rows;        // rows to split as well, or null
   half_t *row_pairs;        // [rows_cap][K / 32][64]
   int *row_exps;
@@ -103,7 +103,7 @@ __device__ __forceinline__ void split_weight_unit(const SplitArgs &a, int unit) 
     s_scale[t] = split_power(e);
     jb.exps[(size_t)chunk * jb.N + n0 + t] = e;
     if (j == a.bounded) {
-      float b = __builtin_fabsf(a.bias[n0 + t]);
+      float b = finite_or_zero(a.bias[n0 + t]);
 #pragma unroll
       for (int o = 1; o < 32; o <<= 1) m = fmaxf(m, __shfl_xor(m, o, 64)), b = fmaxf(b, __shfl_xor(b, o, 64));
       if (t == 0) a.bounds[2 * u] = m, a.bounds[2 * u + 1] = b;

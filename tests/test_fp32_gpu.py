@@ -345,6 +345,35 @@ def test_layernorm_f32_split_keeps_the_gelu_in_range(device, H):
     assert np.all(np.abs(got - exp) <= bound), (np.abs(got - exp) / bound).max()
 
 
+@pytest.mark.parametrize("size", [1e14, 1e19, 1e30])
+def test_layernorm_f32_split_bounds_rows_whose_squares_are_no_floats(device, size):
+    """Rows whose sum of squares leaves the float range, a product beyond fp16 that does not, and a bias with an infinity:
+    every finite result of FFN1 stays finite and where it belongs."""
+    _say("layernorm_f32_split large", size)
+    rs = np.random.RandomState(5)
+    rows, H, F = 33, 768, 64
+    zero = np.zeros(H, np.float32)
+    out, res = (rs.standard_normal((rows, H)).astype(np.float32) for _ in range(2))
+    gamma = (rs.standard_normal(H) * size).astype(np.float32)
+    w, b1 = (rs.standard_normal((H, F)) * (1e8 / size)).astype(np.float32), np.zeros(F, np.float32)
+    b1[5] = np.inf
+    (wp,), _, bounds = ops.split_f32([_dev(w, device)], None, 0, _dev(b1, device))
+    mine = _dev(out, device)
+    pairs, exps, ge = ops.add_bias_residual_layernorm_f32_split(mine, *[_dev(a, device) for a in (res, zero, gamma, zero)],
+                                                                bounds, 1e-6)
+    got = _joined(ops.gemm_f32_split((pairs, exps), wp, _dev(b1, device), ge), ge)
+    ln = mine.cpu().numpy()
+    assert np.isfinite(ln).all()
+    u = ln.astype(np.float64) @ w.astype(np.float64) + b1
+    fin = np.isfinite(u)
+    assert np.array_equal(fin, np.repeat([np.arange(F) != 5], rows, 0)) and np.abs(u[fin]).max() > 65504
+    exp = np.maximum(u, 0)                                          # GELU at 1e9: one side or the other
+    # the product to 2^-20 of sum |a||w|; GELU of what lies about zero differs from this by less than 1
+    bound = 2.0 ** -20 * (np.abs(ln).astype(np.float64) @ np.abs(w).astype(np.float64)) + 1
+    assert np.isfinite(got[fin]).all() and np.all(np.abs(got - exp)[fin] <= bound[fin])
+    assert np.all(np.isinf(got[:, 5]))
+
+
 @pytest.mark.parametrize("path", ["c_api", "th_op", "encoder"])
 @pytest.mark.parametrize("rm", [True, False])
 def test_fp32_layers_on_split_operands(device, path, rm):
