@@ -592,7 +592,7 @@ __global__ __launch_bounds__(64 * NQ * KS, 2) void f32_attention_kernel(F32AttAr
   }
 
   const int tid = threadIdx.x, lane = tid & 63, wave_all = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wave = wave_all % NQ, group = wave_all / NQ;
+  const int wave = KS > 1 ? wave_all % NQ : wave_all, group = KS > 1 ? wave_all / NQ : 0;
   const int l32 = lane & 31, half = lane >> 5;
   const int d = p.d;
   const int H = p.heads * d;
@@ -662,7 +662,7 @@ __global__ __launch_bounds__(64 * NQ * KS, 2) void f32_attention_kernel(F32AttAr
   const bool add_vec = (p.S & 3) == 0;
   for (int t = 0; t < turns; ++t) {
     const int k0 = t * STEP + group * kF32KT;
-    const bool wave_live = query_live && k0 < klen;
+    const bool wave_live = query_live && (KS == 1 || k0 < klen);
     // additive terms of this tile's 16 keys per lane (4 groups of 4 consecutive keys),
     // in the exp2 domain; issued ahead of the next tile's K / V so that the wait for
     // them does not include those
