@@ -394,7 +394,7 @@ __device__ __forceinline__ void f32_split_tile(BT_F32_SPLIT_FIRST, const F32Spli
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const float s = sum[i][j][e];
-        finite = finite && __builtin_fabsf(s) < __builtin_inff();
+        finite = finite && (__builtin_fabsf(s) < __builtin_inff() || m >= M);   // (dead rows hold what the scratch held before)
         v[e] = __builtin_amdgcn_ldexpf(s, -(ea + ew[i][e]));
       }
       v += bias[i];

@@ -314,6 +314,31 @@ def test_gemm_f32_split_passes_infinities_and_nan_on(device, tile):
     assert np.all(np.isnan(h[~fin]) | np.isinf(h[~fin]) | (h[~fin] == 0))       # GELU(-inf) is -0 or NaN in float arithmetic
 
 
+@pytest.mark.parametrize("tile", [0, 1, 2])
+def test_gemm_f32_split_leaves_dead_rows_alone(device, tile):
+    """What lies in the pairs of rows past the live count, infinities and NaN here, changes no bit of the others."""
+    _say("gemm_f32_split dead rows", tile)
+    rs = np.random.RandomState(tile)
+    rows, M, N, K = 150, 101, 160, 192
+    x, w = rs.standard_normal((rows, K)).astype(np.float32), rs.standard_normal((K, N)).astype(np.float32)
+    bias, vr = _dev(rs.standard_normal(N).astype(np.float32), device), torch.tensor([M], dtype=torch.int32, device=device)
+    ge = torch.full((rows,), 6, dtype=torch.int32, device=device)
+    (wp,), (pairs, exps), _ = ops.split_f32([_dev(w, device)], _dev(x, device))
+    dead = pairs.clone()
+    dead[M:] = float("nan")
+    dead[M:, ::2, ::3] = float("inf")
+    ops.set_option("f32_gemm_tile", tile)
+    try:
+        for g in (None, ge):
+            out = [torch.full((rows, N) if g is None else (rows, N // 32, 64), 7.0, device=device,
+                              dtype=torch.float32 if g is None else torch.float16) for _ in range(2)]
+            for p, o in zip((pairs, dead), out):
+                ops.gemm_f32_split((p, exps), wp, bias, g, vr, o)
+            assert torch.equal(*out) and bool((out[0][M:] == 7).all())
+    finally:
+        ops.set_option("f32_gemm_tile", -1)
+
+
 @pytest.mark.parametrize("H", [64, 768, 1024])
 def test_layernorm_f32_split_keeps_the_gelu_in_range(device, H):
     """The LayerNorm's rows are those of the plain one, its pairs stand for them, and the exponents it gives to FFN1 leave
