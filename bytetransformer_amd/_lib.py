@@ -29,6 +29,11 @@ _P = c_void_p
 _IP = c_void_p  # int* device pointers travel as raw addresses
 
 # name -> (restype, argtypes); mirrors include/bt_hip.h declaration by declaration
+class F32SplitMore(ctypes.Structure):
+    """bt_f32_split_more"""
+    _fields_ = [("tile_rows", c_int)]
+
+
 KERNEL_ABI = {
     "bt_version": (c_int, []),
     "bt_last_error_string": (c_char_p, []),
@@ -53,6 +58,7 @@ KERNEL_ABI = {
     "bt_split_f32": (c_int, [c_int, POINTER(c_void_p), POINTER(c_void_p), POINTER(c_void_p), POINTER(c_int), POINTER(c_int),
                              c_int, _P, _P, _P, _P, _IP, _IP, _IP, c_int, c_int, _P]),
     "bt_gemm_f32_split": (c_int, [_P, _IP, _P, _IP, _P, _P, _IP, _IP, c_int, c_int, c_int, _P]),
+    "bt_gemm_f32_split_with": (c_int, [_P, _IP, _P, _IP, _P, _P, _IP, _IP, c_int, c_int, c_int, POINTER(F32SplitMore), _P]),
     "bt_add_bias_residual_layernorm_f32_split": (c_int, [_P, _P, _IP, _P, _P, _P, _IP, c_int, c_int, c_float, _P, _IP, _IP,
                                                          _P, c_int, _P]),
     "bt_gemm_qkv_bias_split": (c_int, [_P, _IP, _P, _P, _P, _IP, c_int, c_int, c_int, c_int,

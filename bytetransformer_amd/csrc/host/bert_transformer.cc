@@ -267,18 +267,20 @@ void BertTransformer<OpType>::bert_infer(BertTransformerInferParam infer_param) 
     if (split) {
       // (Q, K, V are dead: the attention's pairs take the first tensor's place, the LayerNorm's the second's)
       DataType_ *att_pairs = qkv_buf, *ln_pairs = qkv_buf + tensor;
+      // (the tiles of the padded batch, also where the caller's offsets bring the count: the same bits with and without them)
+      const bt_f32_split_more more{rows};
       check_bt_error(bt_split_f32(0, nullptr, nullptr, nullptr, nullptr, nullptr, -1, nullptr, nullptr, attr_out_buf, att_pairs,
                                   sp.att_exps, nullptr, valid_rows, packed_cap, hidden, stream));
-      check_bt_error(bt_gemm_f32_split(att_pairs, sp.att_exps, w_pairs[1], sp.w_exps[1], nullptr, attr_matmul_buf, nullptr,
-                                       valid_rows, packed_cap, hidden, hidden, stream));
+      check_bt_error(bt_gemm_f32_split_with(att_pairs, sp.att_exps, w_pairs[1], sp.w_exps[1], nullptr, attr_matmul_buf, nullptr,
+                                            valid_rows, packed_cap, hidden, hidden, &more, stream));
       check_bt_error(bt_add_bias_residual_layernorm_f32_split(
           attr_matmul_buf, from_tensor, gather, param_.attr_output_bias, param_.attr_output_layernorm_gamma,
           param_.attr_output_layernorm_beta, valid_rows, packed_cap, hidden, layernorm_eps, ln_pairs, sp.ln_exps, sp.gelu_exps,
           sp.bounds, sp.bound_count, stream));
-      check_bt_error(bt_gemm_f32_split(ln_pairs, sp.ln_exps, w_pairs[2], sp.w_exps[2], param_.inter_bias, inter_matmul_buf,
-                                       sp.gelu_exps, valid_rows, packed_cap, inter, hidden, stream));
-      check_bt_error(bt_gemm_f32_split(inter_matmul_buf, sp.gelu_exps, w_pairs[3], sp.w_exps[3], nullptr, transformer_out,
-                                       nullptr, valid_rows, packed_cap, hidden, inter, stream));
+      check_bt_error(bt_gemm_f32_split_with(ln_pairs, sp.ln_exps, w_pairs[2], sp.w_exps[2], param_.inter_bias, inter_matmul_buf,
+                                            sp.gelu_exps, valid_rows, packed_cap, inter, hidden, &more, stream));
+      check_bt_error(bt_gemm_f32_split_with(inter_matmul_buf, sp.gelu_exps, w_pairs[3], sp.w_exps[3], nullptr, transformer_out,
+                                            nullptr, valid_rows, packed_cap, hidden, inter, &more, stream));
     } else {
       check_bt_error(bt_gemm_f32(attr_out_buf, nullptr, param_.attr_output_kernel, nullptr,
                                  attr_matmul_buf, 0, valid_rows, packed_cap, rows_hint, hidden, hidden,

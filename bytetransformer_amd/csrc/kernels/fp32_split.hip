@@ -524,6 +524,12 @@ extern "C" int bt_split_f32(int weight_count, const void *const *w, void *const 
 extern "C" int bt_gemm_f32_split(const void *a_pairs, const int *a_exps, const void *w_pairs, const int *w_exps, const void *bias,
                                  void *c, const int *gelu_exps, const int *valid_rows, int rows_cap, int n, int k,
                                  void *stream) {
+  return bt_gemm_f32_split_with(a_pairs, a_exps, w_pairs, w_exps, bias, c, gelu_exps, valid_rows, rows_cap, n, k, nullptr, stream);
+}
+
+extern "C" int bt_gemm_f32_split_with(const void *a_pairs, const int *a_exps, const void *w_pairs, const int *w_exps,
+                                      const void *bias, void *c, const int *gelu_exps, const int *valid_rows, int rows_cap,
+                                      int n, int k, const bt_f32_split_more *more, void *stream) {
   const char *who = "bt_gemm_f32_split";
   BT_REQUIRE(a_pairs && a_exps && w_pairs && w_exps && c, BT_ERR_INVALID_ARGUMENT, "%s: null pointer argument", who);
   BT_REQUIRE(aligned16({a_pairs, w_pairs, w_exps, c}), BT_ERR_INVALID_ARGUMENT, "%s: pointers must be 16-byte aligned", who);
@@ -543,12 +549,13 @@ extern "C" int bt_gemm_f32_split(const void *a_pairs, const int *a_exps, const v
   // registers to spare; 128x128, eight waves: 44 / 21 / 46 / 63.)  A launch is priced by its rounds of the chip, a last one
   // that is partly full where two workgroups share a CU at half of one and half of its share: 5 us less than these
   // and those of 600 and 4915 rows, give or take 15 %.  The groups add up in another order, so the choice follows from sizes
-  // alone, never from a row hint; a padded batch counts as 60 % full, give or take a fifth.
+  // alone, never from a row hint, and where the count is known in some calls only, from the capacity of all (tile_rows); a padded batch counts as 60 % full, give or take a fifth.
   int tile = option_f32_gemm_tile();
   if (tile < 0 || tile > 2) {
     struct Candidate { int bm, bn, per_cu; float step, fixed; };   // of a round: us per 64 of k, and besides
     static const Candidate candidates[3] = {{64, 64, 2, 0.66f, 7.f}, {64, 128, 1, 0.74f, 6.8f}, {96, 128, 2, 1.8f, 5.4f}};
-    const long long rows = valid_rows ? (rows_cap * 3LL + 4) / 5 : rows_cap;
+    const long long capacity = more && more->tile_rows > 0 ? more->tile_rows : rows_cap;
+    const long long rows = valid_rows ? (capacity * 3LL + 4) / 5 : capacity;
     float best = 0.f;
     for (int t = 0; t < 3; ++t) {
       const Candidate &c = candidates[t];

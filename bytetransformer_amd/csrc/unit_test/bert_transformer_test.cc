@@ -125,7 +125,7 @@ struct Options {
   int batch_size, seq_len, head_num, size_per_head, iters = 50;
   double tol = -1.0;
   bool is_remove_padding = true, use_fused_attention = true;
-  std::string dir = ".";
+  std::string dir = ".", dump;   // dump: file that receives the first call's output as it is
   bool synthetic = false;
   bool offsets = false;   // built once ahead of the layer, with their count
   std::vector<int> lens;
@@ -230,6 +230,16 @@ static int run(const Options &o) {
     layer.infer(infer_param);
     HIP_OK(hipStreamSynchronize(stream));
 
+    if (!o.dump.empty()) {
+      std::vector<T> got(N * H);
+      HIP_OK(hipMemcpy(got.data(), out, got.size() * sizeof(T), hipMemcpyDeviceToHost));
+      FILE *fd = fopen(o.dump.c_str(), "wb");
+      if (!fd || fwrite(got.data(), sizeof(T), got.size(), fd) != got.size() || fclose(fd)) {
+        fprintf(stderr, "cannot write %s\n", o.dump.c_str());
+        return 2;
+      }
+    }
+
     // compare valid rows and zero-filled rows alike: the exported expectation is
     // already multiplied by the row mask
     double max_diff = -1.0;
@@ -284,7 +294,7 @@ int main(int argc, char *argv[]) {
   if (argc < 5) {
     printf("./bert_transformer_test <batch_size> <seq_len> <head_num> <size_per_head> "
            "[--data DIR] [--iters N] [--tol MAX_ABS] [--no-rm] [--no-fused] [--fp32] "
-           "[--synthetic [--lens L0,L1,...]] [--offsets] [--option NAME=VALUE ...]\n");
+           "[--synthetic [--lens L0,L1,...]] [--offsets] [--dump FILE] [--option NAME=VALUE ...]\n");
     return 0;
   }
   Options o;
@@ -303,6 +313,7 @@ int main(int argc, char *argv[]) {
     else if (!strcmp(argv[i], "--fp32")) fp32 = true;
     else if (!strcmp(argv[i], "--synthetic")) o.synthetic = true;
     else if (!strcmp(argv[i], "--offsets")) o.offsets = true;
+    else if (!strcmp(argv[i], "--dump") && i + 1 < argc) o.dump = argv[++i];
     else if (!strcmp(argv[i], "--option") && i + 1 < argc) {
       // a tuning knob of the kernel library (bt_set_option), e.g. qkv_mask_rows=0
       const std::string kv = argv[++i];

@@ -471,6 +471,7 @@ int bt_splitk_layernorm(const void *partials, int splits, const void *residual,
  *                      row r scaled by 2^gelu_exps[r]; n a multiple of 32, k of 64.  Distance from float64 (2-norm; largest
  *                      difference over the largest result) for normal operands: k = 768 1.4e-7, 2.5e-7, k = 3072 1.5e-7,
  *                      2.4e-7, where bt_gemm_f32 has 2.1e-7, 3.5e-7 and 4.3e-7, 7.0e-7.
+ *   bt_gemm_f32_split_with  the same, told more (`more` nullable)
  *   bt_add_bias_residual_layernorm_f32_split  bt_add_bias_residual_layernorm_f32 that writes the pairs of its rows as
  *                      well, and exponents that keep the pairs of GELU(row . W + b) in range for the W of `bounds`.
  */
@@ -479,6 +480,14 @@ int bt_split_f32(int weight_count, const void *const *w, void *const *w_pairs, i
                  int *row_exps, const int *row_index, const int *valid_rows, int rows_cap, int hidden_dim, void *stream);
 int bt_gemm_f32_split(const void *a_pairs, const int *a_exps, const void *w_pairs, const int *w_exps, const void *bias,
                       void *c, const int *gelu_exps, const int *valid_rows, int rows_cap, int n, int k, void *stream);
+typedef struct bt_f32_split_more {
+  /* > 0: the tile is the one of a launch of this capacity.  Tiles add up in different orders, so a caller that knows its
+   * row count in one call and not in the next names the capacity here in both, and the bits stay. */
+  int tile_rows;
+} bt_f32_split_more;
+int bt_gemm_f32_split_with(const void *a_pairs, const int *a_exps, const void *w_pairs, const int *w_exps, const void *bias,
+                           void *c, const int *gelu_exps, const int *valid_rows, int rows_cap, int n, int k,
+                           const bt_f32_split_more *more, void *stream);
 int bt_add_bias_residual_layernorm_f32_split(void *out, const void *residual, const int *residual_row_index,
                                              const void *bias, const void *gamma, const void *beta,
                                              const int *valid_rows, int rows_cap, int hidden_dim, float eps, void *pairs,

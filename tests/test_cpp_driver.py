@@ -57,3 +57,21 @@ def test_cpp_driver_matches_exported_expectation(device, tmp_path, batch, seq, h
     m = re.search(r"max_diff ([0-9.]+)", out.stdout)
     assert m and float(m.group(1)) <= float(tol)
     assert "layer time costs" in out.stdout
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,seq,length", [(10, 500, 300), (16, 512, 250), (9, 300, 300)])
+def test_cpp_driver_float_layers_with_offsets_have_the_same_bits(device, tmp_path, batch, seq, length):
+    """A float layer on split operands, with offsets (and so the count) from the caller and without: a capacity and a count
+    that would have other tiles, which add up in another order."""
+    print("cpp driver float offsets", batch, seq, length, flush=True)
+    got = []
+    for extra in ([], ["--offsets"]):
+        to = str(tmp_path / ("out%d" % len(got)))
+        out = subprocess.run([DRIVER, str(batch), str(seq), "12", "64", "--fp32", "--synthetic", "--iters", "1", "--lens",
+                              ",".join([str(length)] * batch), "--dump", to] + extra,
+                             stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=120)
+        assert out.returncode == 0, out.stdout[-2000:]
+        got.append(np.fromfile(to, dtype=np.float32).reshape(batch, seq, 768))
+    assert np.isfinite(got[0]).all() and np.abs(got[0][:, :length]).mean() > 0.5 and not got[0][:, length:].any()
+    assert np.array_equal(*got)
