@@ -31,7 +31,7 @@ _IP = c_void_p  # int* device pointers travel as raw addresses
 # name -> (restype, argtypes); mirrors include/bt_hip.h declaration by declaration
 class F32SplitMore(ctypes.Structure):
     """bt_f32_split_more"""
-    _fields_ = [("tile_rows", c_int)]
+    _fields_ = [("tile_rows", c_int), ("raw", _P), ("a_raw", _P), ("w", _P)]
 
 
 KERNEL_ABI = {
@@ -57,10 +57,14 @@ KERNEL_ABI = {
     "bt_gemm_bias_gelu": (c_int, [_P, _P, _P, _P, _IP, c_int, c_int, c_int, c_int, c_int, _P]),
     "bt_split_f32": (c_int, [c_int, POINTER(c_void_p), POINTER(c_void_p), POINTER(c_void_p), POINTER(c_int), POINTER(c_int),
                              c_int, _P, _P, _P, _P, _IP, _IP, _IP, c_int, c_int, _P]),
+    "bt_split_f32_layer": (c_int, [c_int, POINTER(c_void_p), POINTER(c_void_p), POINTER(c_void_p), POINTER(c_int),
+                                   POINTER(c_int), c_int, _P, _P, _P, _P, _IP, _IP, _IP, c_int, c_int, c_int, _P]),
     "bt_gemm_f32_split": (c_int, [_P, _IP, _P, _IP, _P, _P, _IP, _IP, c_int, c_int, c_int, _P]),
     "bt_gemm_f32_split_with": (c_int, [_P, _IP, _P, _IP, _P, _P, _IP, _IP, c_int, c_int, c_int, POINTER(F32SplitMore), _P]),
     "bt_add_bias_residual_layernorm_f32_split": (c_int, [_P, _P, _IP, _P, _P, _P, _IP, c_int, c_int, c_float, _P, _IP, _IP,
                                                          _P, c_int, _P]),
+    "bt_add_bias_residual_layernorm_f32_split_layer": (c_int, [_P, _P, _IP, _P, _P, _P, _IP, c_int, c_int, c_float, _P, _IP,
+                                                               _IP, _P, c_int, _P, c_int, _P]),
     "bt_gemm_qkv_bias_split": (c_int, [_P, _IP, _P, _P, _P, _IP, c_int, c_int, c_int, c_int,
                                        c_int, _P]),
     "bt_gemm_qkv_mask_rows_supported": (c_int, [c_int, c_int, c_int]),

@@ -112,8 +112,8 @@ void BertEncoder<OpType>::infer(BertEncoderInferParam<DataType_> ip) {
       if (f32_split) {
         const void *ws[4] = {w.attr_kernel_QKV, w.attr_output_kernel, w.inter_kernel, w.output_kernel};
         const int ks[4] = {hidden, hidden, hidden, inter}, ns[4] = {3 * hidden, hidden, inter, hidden};
-        check_bt_error(bt_split_f32(4, ws, w_pairs, sp.w_exps, ks, ns, 2, w.inter_bias, sp.bounds, x, inter_matmul_buf, sp.x_exps,
-                                    gather, valid_rows, rows, hidden, stream));
+        check_bt_error(bt_split_f32_layer(4, ws, w_pairs, sp.w_exps, ks, ns, 2, w.inter_bias, sp.bounds, x, inter_matmul_buf,
+                                          sp.x_exps, gather, valid_rows, rows, hidden, 1, stream));
         check_bt_error(bt_gemm_f32_split(inter_matmul_buf, sp.x_exps, w_pairs[0], sp.w_exps[0], w.attention_param.attr_bias_QKV,
                                          qkv_buf, nullptr, valid_rows, rows, 3 * hidden, hidden, stream));
       } else {
@@ -130,17 +130,19 @@ void BertEncoder<OpType>::infer(BertEncoderInferParam<DataType_> ip) {
       if (f32_split) {
         // (Q, K, V are dead: the attention's pairs take the first tensor's place, the LayerNorm's the second's)
         DataType_ *att_pairs = qkv_buf, *ln_pairs = qkv_buf + tensor;
+        const bt_f32_split_more ffn1{0, sp.raw, nullptr, w.inter_kernel}, ffn2{0, nullptr, sp.raw, w.output_kernel};
         check_bt_error(bt_split_f32(0, nullptr, nullptr, nullptr, nullptr, nullptr, -1, nullptr, nullptr, attr_out_buf, att_pairs,
                                     sp.att_exps, nullptr, valid_rows, rows, hidden, stream));
         check_bt_error(bt_gemm_f32_split(att_pairs, sp.att_exps, w_pairs[1], sp.w_exps[1], nullptr, attr_matmul_buf, nullptr,
                                          valid_rows, rows, hidden, hidden, stream));
-        check_bt_error(bt_add_bias_residual_layernorm_f32_split(
+        check_bt_error(bt_add_bias_residual_layernorm_f32_split_layer(
             attr_matmul_buf, x, gather, w.attr_output_bias, w.attr_output_layernorm_gamma, w.attr_output_layernorm_beta,
-            valid_rows, rows, hidden, layernorm_eps, ln_pairs, sp.ln_exps, sp.gelu_exps, sp.bounds, sp.bound_count, stream));
-        check_bt_error(bt_gemm_f32_split(ln_pairs, sp.ln_exps, w_pairs[2], sp.w_exps[2], w.inter_bias, inter_matmul_buf,
-                                         sp.gelu_exps, valid_rows, rows, inter, hidden, stream));
-        check_bt_error(bt_gemm_f32_split(inter_matmul_buf, sp.gelu_exps, w_pairs[3], sp.w_exps[3], nullptr, ffn2_out, nullptr,
-                                         valid_rows, rows, hidden, inter, stream));
+            valid_rows, rows, hidden, layernorm_eps, ln_pairs, sp.ln_exps, sp.gelu_exps, sp.bounds, sp.bound_count, sp.raw, inter,
+            stream));
+        check_bt_error(bt_gemm_f32_split_with(ln_pairs, sp.ln_exps, w_pairs[2], sp.w_exps[2], w.inter_bias, inter_matmul_buf,
+                                              sp.gelu_exps, valid_rows, rows, inter, hidden, &ffn1, stream));
+        check_bt_error(bt_gemm_f32_split_with(inter_matmul_buf, sp.gelu_exps, w_pairs[3], sp.w_exps[3], nullptr, ffn2_out, nullptr,
+                                              valid_rows, rows, hidden, inter, &ffn2, stream));
       } else {
         check_bt_error(bt_gemm_f32(attr_out_buf, nullptr, w.attr_output_kernel, nullptr,
                                    attr_matmul_buf, 0, valid_rows, rows, rows_hint, hidden, hidden, stream));

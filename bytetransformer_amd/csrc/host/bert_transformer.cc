@@ -243,8 +243,8 @@ void BertTransformer<OpType>::bert_infer(BertTransformerInferParam infer_param) 
     }
     if (split) {
       const void *w[4] = {w_use[0], w_use[1], w_use[2], w_use[3]};
-      check_bt_error(bt_split_f32(4, w, w_pairs, sp.w_exps, w_k, w_n, 2, param_.inter_bias, sp.bounds, from_tensor,
-                                  inter_matmul_buf, sp.x_exps, gather, valid_rows, rows, hidden, stream));
+      check_bt_error(bt_split_f32_layer(4, w, w_pairs, sp.w_exps, w_k, w_n, 2, param_.inter_bias, sp.bounds, from_tensor,
+                                        inter_matmul_buf, sp.x_exps, gather, valid_rows, rows, hidden, 1, stream));
       check_bt_error(bt_gemm_f32_split(inter_matmul_buf, sp.x_exps, w_pairs[0], sp.w_exps[0],
                                        param_.attention_param.attr_bias_QKV, qkv_buf, nullptr, valid_rows, rows,
                                        3 * hidden, hidden, stream));
@@ -268,19 +268,22 @@ void BertTransformer<OpType>::bert_infer(BertTransformerInferParam infer_param) 
       // (Q, K, V are dead: the attention's pairs take the first tensor's place, the LayerNorm's the second's)
       DataType_ *att_pairs = qkv_buf, *ln_pairs = qkv_buf + tensor;
       // (the tiles of the padded batch, also where the caller's offsets bring the count: the same bits with and without them)
-      const bt_f32_split_more more{rows};
+      const auto more = [&](const DataType_ *weight, unsigned *raw = nullptr, const unsigned *a_raw = nullptr) {
+        return bt_f32_split_more{rows, raw, a_raw, weight};
+      };
+      const bt_f32_split_more proj = more(w_use[1]), ffn1 = more(w_use[2], sp.raw), ffn2 = more(w_use[3], nullptr, sp.raw);
       check_bt_error(bt_split_f32(0, nullptr, nullptr, nullptr, nullptr, nullptr, -1, nullptr, nullptr, attr_out_buf, att_pairs,
                                   sp.att_exps, nullptr, valid_rows, packed_cap, hidden, stream));
       check_bt_error(bt_gemm_f32_split_with(att_pairs, sp.att_exps, w_pairs[1], sp.w_exps[1], nullptr, attr_matmul_buf, nullptr,
-                                            valid_rows, packed_cap, hidden, hidden, &more, stream));
-      check_bt_error(bt_add_bias_residual_layernorm_f32_split(
+                                            valid_rows, packed_cap, hidden, hidden, &proj, stream));
+      check_bt_error(bt_add_bias_residual_layernorm_f32_split_layer(
           attr_matmul_buf, from_tensor, gather, param_.attr_output_bias, param_.attr_output_layernorm_gamma,
           param_.attr_output_layernorm_beta, valid_rows, packed_cap, hidden, layernorm_eps, ln_pairs, sp.ln_exps, sp.gelu_exps,
-          sp.bounds, sp.bound_count, stream));
+          sp.bounds, sp.bound_count, sp.raw, inter, stream));
       check_bt_error(bt_gemm_f32_split_with(ln_pairs, sp.ln_exps, w_pairs[2], sp.w_exps[2], param_.inter_bias, inter_matmul_buf,
-                                            sp.gelu_exps, valid_rows, packed_cap, inter, hidden, &more, stream));
+                                            sp.gelu_exps, valid_rows, packed_cap, inter, hidden, &ffn1, stream));
       check_bt_error(bt_gemm_f32_split_with(inter_matmul_buf, sp.gelu_exps, w_pairs[3], sp.w_exps[3], nullptr, transformer_out,
-                                            nullptr, valid_rows, packed_cap, hidden, inter, &more, stream));
+                                            nullptr, valid_rows, packed_cap, hidden, inter, &ffn2, stream));
     } else {
       check_bt_error(bt_gemm_f32(attr_out_buf, nullptr, param_.attr_output_kernel, nullptr,
                                  attr_matmul_buf, 0, valid_rows, packed_cap, rows_hint, hidden, hidden,

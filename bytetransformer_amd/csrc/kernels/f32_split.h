@@ -9,12 +9,14 @@ constexpr float kSplitLow = 1.0f / 2048.0f;   // what a pair's second number is 
 
 struct SplitPair {
   half_t h, l;
+  bool held;   // the value to 2^-22 of itself (what is not finite counts as held)
 };
 // of a scaled value: the second number is zero where the first is not finite
 __device__ __forceinline__ SplitPair split_pair(float x) {
   const half_t h = (half_t)x;
   const float rest = (x - (float)h) * 2048.0f;
-  return SplitPair{h, __builtin_fabsf((float)h) < __builtin_inff() ? (half_t)rest : (half_t)0.f};
+  const half_t l = __builtin_fabsf((float)h) < __builtin_inff() ? (half_t)rest : (half_t)0.f;
+  return SplitPair{h, l, !(__builtin_fabsf(rest - (float)l) > __builtin_fabsf(x) * kSplitLow)};
 }
 // The exponent that brings a largest value m >= 0 to [2^14, 2^15) (0 for no value at all), held where 2^e is a float.
 __device__ __forceinline__ int split_exponent(float m) {

@@ -803,6 +803,8 @@ struct F32LnPairs {
   int *gelu_exps;        // [rows]
   const float *bounds;   // [bound_count][2]: largest |w| and |bias| of some columns each
   int bound_count;
+  unsigned *raw;         // [rows][raw_words] cleared for the product that reads the pairs (its rows that stay floats), or null
+  int raw_words;
 };
 
 // One wave per row, float4 per lane, the row in registers between the two passes.
@@ -905,6 +907,7 @@ __device__ __forceinline__ void f32_layernorm_block(
       next.exps[r] = e;
       next.gelu_exps[r] = split_exponent(bound);
     }
+    if (lane < next.raw_words) next.raw[(size_t)r * next.raw_words + lane] = 0;
   }
 }
 
@@ -1100,14 +1103,24 @@ extern "C" int bt_add_bias_residual_layernorm_f32_split(
     void *out, const void *residual, const int *residual_row_index, const void *bias, const void *gamma, const void *beta,
     const int *valid_rows, int rows_cap, int hidden_dim, float eps, void *pairs, int *exps, int *gelu_exps, const float *bounds,
     int bound_count, void *stream) {
+  return bt_add_bias_residual_layernorm_f32_split_layer(out, residual, residual_row_index, bias, gamma, beta, valid_rows, rows_cap,
+                                                        hidden_dim, eps, pairs, exps, gelu_exps, bounds, bound_count, nullptr, 0,
+                                                        stream);
+}
+
+extern "C" int bt_add_bias_residual_layernorm_f32_split_layer(
+    void *out, const void *residual, const int *residual_row_index, const void *bias, const void *gamma, const void *beta,
+    const int *valid_rows, int rows_cap, int hidden_dim, float eps, void *pairs, int *exps, int *gelu_exps, const float *bounds,
+    int bound_count, unsigned *raw, int n, void *stream) {
   const char *who = "bt_add_bias_residual_layernorm_f32_split";
   BT_REQUIRE(out && residual && bias && gamma && beta && pairs && exps && gelu_exps && bounds, BT_ERR_INVALID_ARGUMENT,
              "%s: null pointer argument", who);
   BT_REQUIRE(rows_cap >= 0 && bound_count > 0, BT_ERR_INVALID_ARGUMENT, "%s: rows_cap=%d bound_count=%d", who, rows_cap, bound_count);
+  BT_REQUIRE(!raw || (n > 0 && n <= 1024 * kWave), BT_ERR_INVALID_ARGUMENT, "%s: n=%d outside [1, 2^16]", who, n);   // (a word a lane)
   BT_REQUIRE(!residual_row_index || valid_rows, BT_ERR_INVALID_ARGUMENT, "%s: residual_row_index needs valid_rows", who);
   BT_REQUIRE(hidden_dim % 32 == 0 && aligned16({pairs}), BT_ERR_UNSUPPORTED,
              "%s: hidden_dim=%d must be a multiple of 32, the pairs 16-byte aligned", who, hidden_dim);
-  const F32LnPairs next{(half_t *)pairs, exps, gelu_exps, bounds, bound_count};
+  const F32LnPairs next{(half_t *)pairs, exps, gelu_exps, bounds, bound_count, raw, raw ? (n + 1023) / 1024 : 0};
   return launch_f32_ln<false>(out, residual, bias, gamma, beta, out, valid_rows, residual_row_index, 1, rows_cap, hidden_dim,
                               eps, as_stream(stream), who, &next);
 }

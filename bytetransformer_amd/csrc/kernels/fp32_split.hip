@@ -15,8 +15,13 @@
 // of a product, is left out.  Against the exact bfloat16 triples of bt_gemm_f32 (six matrix instructions, one
 // accumulator) the operands are rounded, but the sums are half to a sixth as many roundings: see
 // bt_gemm_f32_split in bt_hip.h for both errors.
-// Infinities and NaN keep their places in h (the scale comes from the finite values of a row); a sum that is not
-// finite is formed again from the pairs by float multiply-adds.
+// Infinities and NaN keep their places in h (the scale comes from the finite values of a row); a row with a sum that is
+// not finite is formed again by float multiply-adds.
+//
+// The scale of FFN1's results has to be known before them, so it comes from a bound.  One large column makes that bound
+// and with it what 2^-50 is worth to the results of all others, be it 10^12 times as large as any of them.  So where
+// the pairs of a result's row do not hold what they should in some 32 columns, these columns stay floats in the
+// place of their pairs (as many bytes), with a bit that says so, and the product that reads that row forms its sums again.
 //
 // In memory a row of K floats is K / 32 blocks of 128 bytes: 32 h, then 32 l.  A block is one k-step's row of an
 // LDS tile, so loads, swizzle and LDS reads are those of an fp16 product of 2 K halfs.
@@ -49,6 +54,7 @@ struct SplitArgs {
   SplitWeight weight[4];
   int count, units;
   int bounded;              // the weight that `bounds` speaks of, -1: none
+  int gelu;                 // ... of GELU(. W + bias): what a bias adds to the largest |result| (else |bias|)
   const float *bias;        // [N] its bias
   float *bounds;            // [units of that weight][2]: largest finite |w| and |bias| of its columns
   const float *rows;        // rows to split as well, or null
@@ -103,7 +109,10 @@ __device__ __forceinline__ void split_weight_unit(const SplitArgs &a, int unit) 
     s_scale[t] = split_power(e);
     jb.exps[(size_t)chunk * jb.N + n0 + t] = e;
     if (j == a.bounded) {
-      float b = finite_or_zero(a.bias[n0 + t]);
+      // (|GELU(x)| <= x above zero, 0.17 and |x| below)
+      const float of = a.bias[n0 + t];
+      float b = finite_or_zero(of);
+      if (a.gelu && of < 0.f) b = fminf(b, 0.1701f);
 #pragma unroll
       for (int o = 1; o < 32; o <<= 1) m = fmaxf(m, __shfl_xor(m, o, 64)), b = fmaxf(b, __shfl_xor(b, o, 64));
       if (t == 0) a.bounds[2 * u] = m, a.bounds[2 * u + 1] = b;
@@ -158,24 +167,84 @@ __global__ __launch_bounds__(kSplitThreads) void split_f32_kernel(SplitArgs a) {
 struct F32SplitTail {
   const float *bias;   // [N] or null
   const int *gelu_exps;   // GELU: exponent that a row of the result is scaled by
+  unsigned *raw;          // GELU: a bit for every 32 columns of a row that are floats, [rows][ceil(N / 1024)], or null
+  const unsigned *a_raw;  // the same of the rows of a, or null
+  const float *w;         // [K, N] the weight itself, or null
 };
 #define BT_F32_SPLIT_FIRST                                                                                  \
   const half_t *a, const half_t *w, const int *valid_rows, const int *a_exps, const int *w_exps, void *out, \
       int rows_cap, int N, int K, unsigned per_n
 
 #if defined(__HIP_DEVICE_COMPILE__)
-// A sum from the pairs themselves, k in order, by float multiply-adds (infinities and NaN among the operands).
-__device__ __forceinline__ float split_dot(const half_t *a, int a_exp, const half_t *w, const int *w_exp, int N, int K) {
-  float sum = 0.f;
-  for (int b = 0; b < K / 32; ++b) {
-    const int e = w_exp[(size_t)(b * 32 / kSplitChunk) * N];
-    for (int k = 0; k < 32; ++k) {
-      const float x = (float)a[b * 64 + k] + (float)a[b * 64 + 32 + k] * kSplitLow;
-      const float y = (float)w[b * 64 + k] + (float)w[b * 64 + 32 + k] * kSplitLow;
-      sum = __builtin_fmaf(__builtin_amdgcn_ldexpf(x, -a_exp), __builtin_amdgcn_ldexpf(y, -e), sum);
+constexpr float kGeluFloor = 1.0f / (1 << 20);   // results below it may go: what they add is a rounding of what made the scale
+
+// Rows of a wave's 16 x WTN block again, by float multiply-adds over k, 256 values at a time: those that the matrix
+// instructions cannot form.  A lane has a column and four rows at a time; the loads of a row are the same for all of them.
+// (Some ten times as slow as the product of pairs, on rows that ordinary operands do not have.)
+template <int WTN, bool GELU>
+__device__ __forceinline__ void split_rows_again(BT_F32_SPLIT_FIRST, const F32SplitTail &tail, int m_first, unsigned rows,
+                                                 int n_first, int M, int lane) {
+  constexpr int kRows = 4, kSides = 64 / WTN;
+  const int side = lane / WTN, n = n_first + lane % WTN, n_in = min(n, N - 1);
+  const int a_words = (K + 1023) / 1024, out_words = (N + 1023) / 1024;
+  const size_t pitch = 2 * (size_t)K;
+  for (int first = 0; first < 16; first += kRows * kSides) {
+    if ((rows >> first & ((1u << kRows * kSides) - 1)) == 0) continue;
+    const int row = first + side * kRows;
+    float sum[kRows], part[kRows];
+    int ea[kRows];
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) sum[r] = part[r] = 0.f, ea[r] = a_exps[min(m_first + row + r, M - 1)];
+#pragma unroll 1
+    for (int b = 0; b < K / 32; ++b) {
+      const int ew = w_exps[(size_t)(b * 32 / kSplitChunk) * N + n_in];
+#pragma unroll 1
+      for (int k = 0; k < 32; k += 4) {
+        float y[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const half_t *pair = w + n_in * pitch + b * 64 + k + e;
+          y[e] = tail.w ? tail.w[(size_t)(b * 32 + k + e) * N + n_in]
+                        : __builtin_amdgcn_ldexpf((float)pair[0] + (float)pair[32] * kSplitLow, -ew);
+        }
+#pragma unroll
+        for (int r = 0; r < kRows; ++r) {
+          const size_t m = min(m_first + row + r, M - 1);
+          const half_t *pairs = a + m * pitch + b * 64;
+          float4_t x;
+          if (tail.a_raw && (tail.a_raw[m * a_words + (b >> 5)] >> (b & 31) & 1)) {
+            x = *(const float4_t *)((const float *)pairs + k);
+          } else {
+            const half4_t h = *(const half4_t *)(pairs + k), l = *(const half4_t *)(pairs + 32 + k);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[e] = __builtin_amdgcn_ldexpf((float)h[e] + (float)l[e] * kSplitLow, -ea[r]);
+          }
+#pragma unroll
+          for (int e = 0; e < 4; ++e) part[r] = __builtin_fmaf(x[e], y[e], part[r]);
+        }
+      }
+      if ((b + 1) % (kSplitChunk / 32) == 0 || b + 1 == K / 32)
+#pragma unroll
+        for (int r = 0; r < kRows; ++r) sum[r] += part[r], part[r] = 0.f;
+    }
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) {
+      const int m = m_first + row + r;
+      if (!(rows >> (row + r) & 1) || m >= M || n >= N) continue;
+      float v = sum[r];
+      if (tail.bias) v += tail.bias[n];
+      if (!GELU) {
+        ((float *)out)[(size_t)m * N + n] = v;
+      } else if (v = f32_gelu(v); tail.raw) {
+        ((float *)out)[(size_t)m * N + n] = v;
+        if (n % 32 == 0) atomicOr(tail.raw + (size_t)m * out_words + (n >> 10), 1u << (n >> 5 & 31));
+      } else {
+        const SplitPair p = split_pair(v * split_power(tail.gelu_exps[m]));
+        half_t *pair = (half_t *)out + (size_t)m * 2 * N + (n >> 5) * 64 + (n & 31);
+        pair[0] = p.h, pair[32] = p.l;
+      }
     }
   }
-  return sum;
 }
 
 // BM x BN tile, WM x WN waves that load and multiply, a ring of STAGES k-steps of 32 floats.  A wave's step is
@@ -232,6 +301,18 @@ __device__ __forceinline__ void f32_split_tile(BT_F32_SPLIT_FIRST, const F32Spli
   for (int i = 0; i < TN; ++i)
 #pragma unroll
     for (int j = 0; j < TM; ++j) sum[i][j] = hh[i][j] = cross[i][j] = zero4;
+  // (bit j: rows of block j that hold floats)
+  unsigned marked = 0;
+  if (tail.a_raw) {
+    const int words = (K + 1023) / 1024;
+#pragma unroll
+    for (int j = 0; j < TM; ++j) {
+      const unsigned *of = tail.a_raw + (size_t)min(m0 + wm * WTM + 16 * j + fr, M - 1) * words;
+      unsigned any = 0;
+      for (int i = 0; i < words; ++i) any |= of[i];
+      marked |= (any != 0 ? 1u : 0u) << j;
+    }
+  }
   // The weight's scales: behind the ring, factor[c][n] = 2^(e - exponent of chunk c of column n), e[n] the smallest of the
   // column's, so that no factor is above 1.  (They are on their way beside the first k-steps.)
   const int chunks = (K + kSplitChunk - 1) / kSplitChunk;
@@ -378,15 +459,17 @@ __device__ __forceinline__ void f32_split_tile(BT_F32_SPLIT_FIRST, const F32Spli
   constexpr int EP = 2 * WTN + 8;   // halfs of a staged row of pairs
   static_assert(!GELU || (size_t)NW * 16 * EP <= (size_t)STAGES * STAGE_HALFS, "staging fits the ring");
   half_t *staged = split_smem + wave_all * 16 * EP;
-  bool finite = true;
+  unsigned again[TM];   // rows of block j
   if (GELU) __builtin_amdgcn_s_barrier();   // everyone is done with the ring
 #pragma unroll
   for (int j = 0; j < TM; ++j) {
+    again[j] = 0;
     if (KG > 1 && (j < kFirstRows) != (group == 0)) continue;
     const int m_first = m0 + wm * WTM + 16 * j, m = m_first + fr, m_in = min(m, M - 1);
     const int ea = a_exps[m_in];
     float to_pair = 1.f;
     if (GELU) to_pair = split_power(tail.gelu_exps[m_in]);
+    bool wrong = marked >> j & 1;
 #pragma unroll
     for (int i = 0; i < TN; ++i) {
       const int n = n0 + wn * WTN + 16 * i + 4 * lg;
@@ -394,7 +477,7 @@ __device__ __forceinline__ void f32_split_tile(BT_F32_SPLIT_FIRST, const F32Spli
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const float s = sum[i][j][e];
-        finite = finite && (__builtin_fabsf(s) < __builtin_inff() || m >= M);   // (dead rows hold what the scratch held before)
+        wrong = wrong || !(__builtin_fabsf(s) < __builtin_inff());
         v[e] = __builtin_amdgcn_ldexpf(s, -(ea + ew[i][e]));
       }
       v += bias[i];
@@ -402,17 +485,54 @@ __device__ __forceinline__ void f32_split_tile(BT_F32_SPLIT_FIRST, const F32Spli
         if (m < M && n < N) store_through((float *)out + (size_t)m * N + n, __builtin_bit_cast(uint4_t, v));
         continue;
       }
-      half4_t h, l;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const SplitPair p = split_pair(f32_gelu(v[e]) * to_pair);
-        h[e] = p.h, l[e] = p.l;
-      }
-      half_t *to = staged + fr * EP + (i >> 1) * 64 + (i & 1) * 16 + 4 * lg;
-      *(half4_t *)to = h;
-      *(half4_t *)(to + 32) = l;
+      for (int e = 0; e < 4; ++e) v[e] = f32_gelu(v[e]);
+      sum[i][j] = v;
     }
+    // (dead rows hold what the scratch held before)
+    const unsigned long long rows = __builtin_amdgcn_ballot_w64(wrong && m < M);
+    again[j] = (unsigned)(rows | rows >> 16 | rows >> 32 | rows >> 48) & 0xffffu;
     if (GELU) {
+      // Floats stay where the pairs hold three results from kGeluFloor on no longer, or one where all are small.  Values from
+      // 2^-14 on are always held, so rows whose bound is below 2^8, as ordinary ones are, are through with a comparison.
+      bool raw = false;
+      if (tail.raw && __builtin_amdgcn_ballot_w64(to_pair * kGeluFloor < 1.0f / (1 << 13) && m < M) != 0) {
+        int lost = 0;
+        float most = 0.f;
+#pragma unroll
+        for (int i = 0; i < TN; ++i)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float v = n0 + wn * WTN + 16 * i + 4 * lg < N ? sum[i][j][e] : 0.f, scaled = v * to_pair;
+            lost += !split_pair(scaled).held && __builtin_fabsf(v) >= kGeluFloor ? 1 : 0;
+            most = fmaxf(most, __builtin_fabsf(scaled));
+          }
+#pragma unroll
+        for (int o = 16; o < 64; o <<= 1) lost += __shfl_xor(lost, o, 64), most = fmaxf(most, __shfl_xor(most, o, 64));
+        raw = m < M && (lost >= 3 || (lost > 0 && most < 1.0f / 256));
+        const int n_first = n0 + wn * WTN;
+        if (raw && lg == 0)
+#pragma unroll
+          for (int n = n_first; n < n_first + WTN; n += 32)
+            if (n < N) atomicOr(tail.raw + (size_t)m * ((N + 1023) / 1024) + (n >> 10), 1u << (n >> 5 & 31));
+      }
+#pragma unroll
+      for (int i = 0; i < TN; ++i) {
+        half_t *to = staged + fr * EP + (i >> 1) * 64;
+        const int at = (i & 1) * 16 + 4 * lg;
+        half4_t h, l;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const SplitPair p = split_pair(sum[i][j][e] * to_pair);
+          h[e] = p.h, l[e] = p.l;
+        }
+        if (raw) {
+          *(float4_t *)((float *)to + at) = sum[i][j];
+        } else {
+          *(half4_t *)(to + at) = h;
+          *(half4_t *)(to + 32 + at) = l;
+        }
+      }
       constexpr int CPR = WTN / 4, RPS = 64 / CPR;   // 16-byte chunks of a row; rows per store instruction
       static_assert(64 % CPR == 0 && 16 % RPS == 0, "whole rows");
 #pragma unroll
@@ -425,31 +545,26 @@ __device__ __forceinline__ void f32_split_tile(BT_F32_SPLIT_FIRST, const F32Spli
     }
   }
 
-  // What is not finite in its place is formed again, one sum after the other: the operands hold infinities or NaN.
-  if (__builtin_amdgcn_ballot_w64(!finite) == 0) return;
+  unsigned any = 0;
+#pragma unroll
+  for (int j = 0; j < TM; ++j) any |= again[j];
+  if (any == 0) return;
   __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): the stores above have returned
-  for (int at = lane + (group ? kFirstRows * 16 * WTN : 0); at < (group ? WTM : kFirstRows * 16) * WTN; at += 64) {
-    const int m = m0 + wm * WTM + at / WTN, n = n0 + wn * WTN + at % WTN;
-    if (m >= M || n >= N) continue;
-    float *to = (float *)out + (size_t)m * N + n;
-    half_t *pair = (half_t *)out + (size_t)m * 2 * N + (n >> 5) * 64 + (n & 31);
-    const float have = GELU ? (float)*(volatile half_t *)pair : *(volatile float *)to;
-    if (__builtin_fabsf(have) < __builtin_inff()) continue;
-    float v = split_dot(a + m * pitch, a_exps[m], w + n * pitch, w_exps + n, N, K);
-    if (tail.bias) v += tail.bias[n];
-    if (GELU) {
-      const SplitPair p = split_pair(f32_gelu(v) * split_power(tail.gelu_exps[m]));
-      *(volatile half_t *)pair = p.h;
-      *(volatile half_t *)(pair + 32) = p.l;
-    } else {
-      *(volatile float *)to = v;
-    }
+  // (one copy of the code: the block's rows picked by a loop that stays one)
+#pragma unroll 1
+  for (int j = 0; j < TM; ++j) {
+    unsigned rows = again[0];
+#pragma unroll
+    for (int i = 1; i < TM; ++i) rows = i == j ? again[i] : rows;
+    if (rows)
+      split_rows_again<WTN, GELU>(a, w, valid_rows, a_exps, w_exps, out, rows_cap, N, K, per_n, tail, m0 + wm * WTM + 16 * j, rows,
+                                  n0 + wn * WTN, M, lane);
   }
 }
 #endif  // __HIP_DEVICE_COMPILE__
 
 template <int BM, int BN, int WM, int WN, int KG, int STAGES, bool GELU>
-__global__ __launch_bounds__(WM *WN *KG * 64, 2) void f32_split_gemm_kernel(BT_F32_SPLIT_FIRST, F32SplitTail tail) {
+__global__ __launch_bounds__(WM *WN *KG * 64, WM *WN *KG == 8 && BN == 64 ? 4 : 2) void f32_split_gemm_kernel(BT_F32_SPLIT_FIRST, F32SplitTail tail) {
 #if defined(__HIP_DEVICE_COMPILE__)
   f32_split_tile<BM, BN, WM, WN, KG, STAGES, GELU>(a, w, valid_rows, a_exps, w_exps, out, rows_cap, N, K, per_n, tail);
 #endif
@@ -488,6 +603,14 @@ extern "C" int bt_split_f32(int weight_count, const void *const *w, void *const 
                             const int *n, int bounded, const void *bounded_bias, float *bounds, const void *rows,
                             void *row_pairs, int *row_exps, const int *row_index, const int *valid_rows, int rows_cap,
                             int hidden_dim, void *stream) {
+  return bt_split_f32_layer(weight_count, w, w_pairs, w_exps, k, n, bounded, bounded_bias, bounds, rows, row_pairs, row_exps,
+                            row_index, valid_rows, rows_cap, hidden_dim, 0, stream);
+}
+
+extern "C" int bt_split_f32_layer(int weight_count, const void *const *w, void *const *w_pairs, int *const *w_exps,
+                                  const int *k, const int *n, int bounded, const void *bounded_bias, float *bounds,
+                                  const void *rows, void *row_pairs, int *row_exps, const int *row_index,
+                                  const int *valid_rows, int rows_cap, int hidden_dim, int layer, void *stream) {
   const char *who = "bt_split_f32";
   BT_REQUIRE(weight_count >= 0 && weight_count <= 4, BT_ERR_INVALID_ARGUMENT, "%s: weight_count=%d outside [0, 4]", who, weight_count);
   BT_REQUIRE(weight_count == 0 || (w && w_pairs && w_exps && k && n), BT_ERR_INVALID_ARGUMENT, "%s: null pointer argument", who);
@@ -506,6 +629,7 @@ extern "C" int bt_split_f32(int weight_count, const void *const *w, void *const 
   }
   a.count = weight_count, a.units = units;
   a.bounded = bounded < 0 ? -1 : bounded, a.bias = (const float *)bounded_bias, a.bounds = bounds;
+  a.gelu = layer;
   int row_blocks = 0;
   if (rows) {
     BT_REQUIRE(row_pairs && row_exps && row_pairs != rows, BT_ERR_INVALID_ARGUMENT, "%s: rows need an area of their own for the pairs", who);
@@ -538,8 +662,10 @@ extern "C" int bt_gemm_f32_split_with(const void *a_pairs, const int *a_exps, co
   BT_REQUIRE(k <= (1 << 14), BT_ERR_UNSUPPORTED, "%s: k=%d is beyond 2^14", who, k);   // (the scales of its chunks lie in LDS)
   BT_REQUIRE(!gelu_exps || bias, BT_ERR_INVALID_ARGUMENT, "%s: gelu needs a bias", who);
   if (rows_cap == 0) return BT_OK;
+  const bt_f32_split_more none{}, &m = more ? *more : none;
+  BT_REQUIRE(!m.raw || gelu_exps, BT_ERR_INVALID_ARGUMENT, "%s: floats among the pairs of a result that is not pairs", who);
   const F32SplitArgs p{(const half_t *)a_pairs, (const half_t *)w_pairs, valid_rows, a_exps, w_exps, c, rows_cap, n, k,
-                       {(const float *)bias, gelu_exps}};
+                       {(const float *)bias, gelu_exps, m.raw, m.a_raw, (const float *)m.w}};
   hipStream_t s = as_stream(stream);
   // Tiles: 0: 64x64, two groups of waves over k, two workgroups a CU | 1: 64x128 likewise, one | 2: 96x128, one group, two.
   // What a step waits for is its operands: a CU takes in about 40 bytes a clock from the L2 and reads 128 from the LDS, and
@@ -554,7 +680,7 @@ extern "C" int bt_gemm_f32_split_with(const void *a_pairs, const int *a_exps, co
   if (tile < 0 || tile > 2) {
     struct Candidate { int bm, bn, per_cu; float step, fixed; };   // of a round: us per 64 of k, and besides
     static const Candidate candidates[3] = {{64, 64, 2, 0.66f, 7.f}, {64, 128, 1, 0.74f, 6.8f}, {96, 128, 2, 1.8f, 5.4f}};
-    const long long capacity = more && more->tile_rows > 0 ? more->tile_rows : rows_cap;
+    const long long capacity = m.tile_rows > 0 ? m.tile_rows : rows_cap;
     const long long rows = valid_rows ? (capacity * 3LL + 4) / 5 : capacity;
     float best = 0.f;
     for (int t = 0; t < 3; ++t) {

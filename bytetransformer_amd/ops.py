@@ -6,7 +6,7 @@ import ctypes
 
 import torch
 
-from ._lib import kernel_lib
+from ._lib import F32SplitMore, kernel_lib
 
 BT_F32, BT_F16 = 0, 1
 
@@ -419,7 +419,7 @@ def gemm_f32(a, w, bias=None, gelu=False, valid_rows=None, a_row_index=None, row
     return out
 
 
-def split_f32(ws, rows=None, bounded=-1, bounded_bias=None, row_index=None, valid_rows=None, rows_cap=None):
+def split_f32(ws, rows=None, bounded=-1, bounded_bias=None, row_index=None, valid_rows=None, rows_cap=None, layer=False):
     """Weights [K, N] and rows as scaled pairs of fp16 numbers: ([(pairs, exps)], (row pairs, row exps) or None, bounds)."""
     _need_f32(*ws, rows, bounded_bias)
     lib, n = kernel_lib(), len(ws)
@@ -437,21 +437,23 @@ def split_f32(ws, rows=None, bounded=-1, bounded_bias=None, row_index=None, vali
                torch.zeros(cap, dtype=torch.int32, device=dev))
     ptrs = [(ctypes.c_void_p * max(n, 1))(*[t.data_ptr() for t in ts]) for ts in (ws, pairs, exps)]
     sizes = [(ctypes.c_int * max(n, 1))(*[w.shape[d] for w in ws]) for d in (0, 1)]
-    _check(lib.bt_split_f32(n, *ptrs, *sizes, bounded, _ptr(bounded_bias), _ptr(bounds), _ptr(rows),
-                            _ptr(got[0] if got else None), _ptr(got[1] if got else None), _ptr(row_index),
-                            _ptr(valid_rows), got[0].shape[0] if got else 0, hidden, _stream()))
+    _check(lib.bt_split_f32_layer(n, *ptrs, *sizes, bounded, _ptr(bounded_bias), _ptr(bounds), _ptr(rows),
+                                  _ptr(got[0] if got else None), _ptr(got[1] if got else None), _ptr(row_index),
+                                  _ptr(valid_rows), got[0].shape[0] if got else 0, hidden, int(layer), _stream()))
     return list(zip(pairs, exps)), got, bounds
 
 
-def gemm_f32_split(a, w, bias=None, gelu_exps=None, valid_rows=None, out=None):
-    """c = a . w (+ bias) of split operands (pairs, exps), or the pairs of its GELU scaled by 2^gelu_exps."""
+def gemm_f32_split(a, w, bias=None, gelu_exps=None, valid_rows=None, out=None, raw=None, a_raw=None, weight=None, tile_rows=0):
+    """c = a . w (+ bias) of split operands (pairs, exps), or the pairs of its GELU scaled by 2^gelu_exps; raw, a_raw
+    (int32 [rows, ceil(columns / 1024)]) and the weight itself as in bt_f32_split_more."""
     (ap, ae), (wp, we) = a, w
     rows, n, k = ap.shape[0], wp.shape[0], wp.shape[1] * 32
     if out is None:
         out = torch.zeros(*((rows, n) if gelu_exps is None else (rows, n // 32, 64)), device=ap.device,
                           dtype=torch.float32 if gelu_exps is None else torch.float16)
-    _check(kernel_lib().bt_gemm_f32_split(_ptr(ap), _ptr(ae), _ptr(wp), _ptr(we), _ptr(bias), _ptr(out), _ptr(gelu_exps),
-                                          _ptr(valid_rows), rows, n, k, _stream()))
+    more = F32SplitMore(tile_rows, _ptr(raw), _ptr(a_raw), _ptr(weight))
+    _check(kernel_lib().bt_gemm_f32_split_with(_ptr(ap), _ptr(ae), _ptr(wp), _ptr(we), _ptr(bias), _ptr(out), _ptr(gelu_exps),
+                                               _ptr(valid_rows), rows, n, k, ctypes.byref(more), _stream()))
     return out
 
 
@@ -498,15 +500,16 @@ def add_bias_residual_layernorm_f32(out, residual, bias, gamma, beta, eps=1e-6, 
 
 
 def add_bias_residual_layernorm_f32_split(out, residual, bias, gamma, beta, bounds, eps=1e-6, valid_rows=None,
-                                          residual_row_index=None):
+                                          residual_row_index=None, raw=None):
     """The float LayerNorm in place, and (pairs, exps, exponents for the pairs of the GELU behind it)."""
     _need_f32(out, residual, bias, gamma, beta)
     rows, hidden = out.shape
     pairs = torch.zeros(rows, hidden // 32, 64, dtype=torch.float16, device=out.device)
     exps, gelu_exps = (torch.zeros(rows, dtype=torch.int32, device=out.device) for _ in range(2))
-    _check(kernel_lib().bt_add_bias_residual_layernorm_f32_split(
+    _check(kernel_lib().bt_add_bias_residual_layernorm_f32_split_layer(
         _ptr(out), _ptr(residual), _ptr(residual_row_index), _ptr(bias), _ptr(gamma), _ptr(beta), _ptr(valid_rows), rows,
-        hidden, float(eps), _ptr(pairs), _ptr(exps), _ptr(gelu_exps), _ptr(bounds), bounds.shape[0], _stream()))
+        hidden, float(eps), _ptr(pairs), _ptr(exps), _ptr(gelu_exps), _ptr(bounds), bounds.shape[0], _ptr(raw),
+        0 if raw is None else raw.shape[1] * 1024, _stream()))
     return pairs, exps, gelu_exps
 
 

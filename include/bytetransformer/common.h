@@ -113,17 +113,18 @@ inline bool f32_splits_operands(long long rows_cap, bool all_live, long long hid
   return hidden % 64 == 0 && inter % 64 == 0 && hidden >= 512 && hidden <= 4096 && inter <= (1 << 14) &&
          (all_live ? rows_cap : rows_cap * 3 / 5) >= 1220;
 }
-// What such a layer needs besides its activations: exponents of four sets of rows and of four weights' columns, and the
-// bounds of FFN1's.
+// What such a layer needs besides its activations: exponents of four sets of rows and of four weights' columns, the
+// bounds of FFN1's, and the bits of FFN1's results that stay floats.
 struct F32SplitScratch {
   int *x_exps, *att_exps, *ln_exps, *gelu_exps, *w_exps[4];
   float *bounds;
+  unsigned *raw;
   int bound_count;
   // (a weight's column has an exponent for every 256 of its rows; a pair of bounds for every 32 columns of those)
   static unsigned long long chunks(unsigned long long k) { return (k + 255) / 256; }
   static unsigned long long bytes(unsigned long long rows, unsigned long long hidden, unsigned long long inter) {
     return (4 * ((rows + 3) / 4 * 4) + chunks(hidden) * (4 * hidden + inter) + chunks(inter) * hidden +
-            chunks(hidden) * inter / 16) * 4;
+            chunks(hidden) * inter / 16 + rows * ((inter + 1023) / 1024)) * 4;
   }
   F32SplitScratch(void *at, unsigned long long rows, int hidden, int inter) {
     rows = (rows + 3) / 4 * 4;
@@ -133,6 +134,7 @@ struct F32SplitScratch {
     x_exps = p, att_exps = p + rows, ln_exps = p + 2 * rows, gelu_exps = p + 3 * rows;
     bounds = (float *)(p + 4 * rows);
     bound_count = (int)(chunks(hidden) * inter / 32);
+    raw = (unsigned *)(bounds + 2 * bound_count);
   }
 };
 

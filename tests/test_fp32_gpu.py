@@ -399,6 +399,96 @@ def test_layernorm_f32_split_bounds_rows_whose_squares_are_no_floats(device, siz
     assert np.all(np.isinf(got[:, 5]))
 
 
+def _with_raw(pairs, exps, raw):
+    """What pairs stand for where some blocks of 32 are floats."""
+    bits = raw.cpu().numpy().view(np.uint32)
+    bits = (bits[:, :, None] >> np.arange(32, dtype=np.uint32) & 1).reshape(len(bits), -1)[:, :pairs.shape[1]]
+    got = _joined(pairs, exps)
+    floats = pairs.cpu().numpy().view(np.float32).reshape(got.shape)
+    return np.where(np.repeat(bits, 32, axis=1) == 1, floats.astype(np.float64), got), bits
+
+
+def _gelu64(u):
+    with np.errstate(over="ignore", invalid="ignore"):
+        return np.where(np.isneginf(u), -0.0, u / (1 + np.exp(-2 * 0.7978845608028654 * (u + 0.044715 * u ** 3))))
+
+
+@pytest.mark.parametrize("tile", [-1, 0, 1, 2])
+@pytest.mark.parametrize("what", ["ordinary", "bias -1e12", "bias -1e30", "bias 1e12", "bias 1e30", "weight 1e9", "weight 1e20"])
+def test_one_large_column_of_ffn1_leaves_the_others_alone(device, tile, what):
+    """FFN1 and FFN2 as a layer runs them, with one column of FFN1 that is out of all proportion and that FFN2 gives no
+    weight: every other result of FFN1, and every result of FFN2, is what it would be without that column."""
+    _say("one large column", tile, what)
+    rs = np.random.RandomState(11)
+    M, rows, H, F = 69, 75, 768, 1088
+    col, zero = 77, np.zeros(H, np.float32)
+    out, res = (rs.standard_normal((rows, H)).astype(np.float32) for _ in range(2))
+    gamma = (1 + 0.05 * rs.standard_normal(H)).astype(np.float32)
+    w1, b1 = (rs.standard_normal((H, F)) * 0.05).astype(np.float32), (rs.standard_normal(F) * 0.1).astype(np.float32)
+    w2 = (rs.standard_normal((F, H)) * 0.05).astype(np.float32)
+    if what.startswith("bias"):
+        b1[col] = float(what[5:])
+    elif what.startswith("weight"):
+        w1[33, col] = float(what[7:])
+    w2[col] = 0
+    vr = torch.tensor([M], dtype=torch.int32, device=device)
+    w1d, w2d, b1d = _dev(w1, device), _dev(w2, device), _dev(b1, device)
+    wp, _, bounds = ops.split_f32([w1d, w2d], None, 0, b1d, layer=True)
+    mine = _dev(out, device)
+    raw = torch.full((rows, (F + 1023) // 1024), -1, dtype=torch.int32, device=device)
+    ops.set_option("f32_gemm_tile", tile)
+    try:
+        pairs, exps, ge = ops.add_bias_residual_layernorm_f32_split(mine, *[_dev(a, device) for a in (res, zero, gamma, zero)],
+                                                                    bounds, 1e-6, vr, raw=raw)
+        mid = ops.gemm_f32_split((pairs, exps), wp[0], b1d, ge, vr, raw=raw, weight=w1d)
+        got2 = ops.gemm_f32_split((mid, ge), wp[1], None, None, vr, torch.full((rows, H), 7.0, device=device), a_raw=raw,
+                                  weight=w2d).cpu().numpy()
+    finally:
+        ops.set_option("f32_gemm_tile", -1)
+    got, bits = _with_raw(mid, ge, raw)
+    assert np.all(raw.cpu().numpy()[M:] == -1) and bool(bits[:M].any()) == (what not in ("ordinary", "bias -1e12", "bias -1e30"))
+    ln = mine.cpu().numpy()[:M].astype(np.float64)
+    u = ln @ w1.astype(np.float64) + b1
+    exp = _gelu64(u)
+    others = np.arange(F) != col
+    # the product to 2^-20 of sum |a||w|, GELU in float, pairs to 2^-22
+    bound = 2.0 ** -20 * (np.abs(ln) @ np.abs(w1).astype(np.float64) + np.abs(b1)) + 1e-6
+    off = np.abs(got[:M] - exp)
+    assert np.all(off[:, others] <= bound[:, others]), (off / bound)[:, others].max()
+    assert np.all(off[:, col] <= bound[:, col])
+    exp2 = got[:M][:, others] @ w2[others].astype(np.float64)
+    bound2 = (4 + math.sqrt(F) / 2) * 2.0 ** -23 * (np.abs(got[:M][:, others]) @ np.abs(w2[others]).astype(np.float64))
+    assert np.all(np.abs(got2[:M] - exp2) <= bound2), (np.abs(got2[:M] - exp2) / bound2).max()
+    assert np.all(got2[M:] == 7.0)
+
+
+@pytest.mark.parametrize("path", ["th_op", "encoder"])
+@pytest.mark.parametrize("rm", [True, False])
+@pytest.mark.parametrize("value", [-1e12, -1e30, 1e12])
+def test_fp32_layers_with_one_large_ffn1_bias(device, path, rm, value):
+    """Layers that split their operands, against the oracle without the column, whose GELU is zero or has no weight behind it."""
+    _say("fp32 layers, large bias", path, rm, value)
+    cfg = workload.EncoderConfig("f32big", 17, 120, 8, layers=2, dtype="fp32", lens=(120, 3, 41, 0, 64, 119) + (90,) * 11)
+    wl = workload.make_workload(cfg, bias_std=0.05, random_affine=True)
+    for w in wl.layers:
+        w["inter_kernel"][:, 5], w["inter_bias"][5], w["output_kernel"][5] = 0, 0, 0
+    exp = _oracle32(wl)
+    for w in wl.layers:
+        w["inter_bias"][5] = value
+    x, m = _dev(wl.x, device), _dev(wl.mask, device)
+    if path == "th_op":
+        bt.load_th_op()
+        got = x
+        for w in wl.layers:
+            got = torch.ops.ByteTransformer.BertTransformer(
+                cfg.head_num, cfg.head_size, *[_dev(w[n], device) for n in workload.WEIGHT_NAMES], got, m, rm, True)
+    else:
+        got = bt.BertEncoder(cfg.head_num, cfg.head_size, [{k: _dev(v, device) for k, v in w.items()} for w in wl.layers],
+                             is_remove_padding=rm)(x, m)
+    got = got.cpu().numpy()
+    _f32_check(got if rm else O.masked_output(got, wl.lens), exp, wl.lens, "f32 large bias/%s" % path, rm)
+
+
 @pytest.mark.parametrize("path", ["c_api", "th_op", "encoder"])
 @pytest.mark.parametrize("rm", [True, False])
 def test_fp32_layers_on_split_operands(device, path, rm):
