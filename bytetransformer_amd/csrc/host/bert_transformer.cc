@@ -242,12 +242,13 @@ void BertTransformer<OpType>::bert_infer(BertTransformerInferParam infer_param) 
       for (int i = 0; i < 4; ++i) w_pairs[i] = slot, slot += (size_t)w_k[i] * w_n[i] * sizeof(float);
     }
     if (split) {
+      const bt_f32_split_more more{0, nullptr, nullptr, w_use[0], from_tensor, gather};
       const void *w[4] = {w_use[0], w_use[1], w_use[2], w_use[3]};
       check_bt_error(bt_split_f32_layer(4, w, w_pairs, sp.w_exps, w_k, w_n, 2, param_.inter_bias, sp.bounds, from_tensor,
                                         inter_matmul_buf, sp.x_exps, gather, valid_rows, rows, hidden, 1, stream));
-      check_bt_error(bt_gemm_f32_split(inter_matmul_buf, sp.x_exps, w_pairs[0], sp.w_exps[0],
-                                       param_.attention_param.attr_bias_QKV, qkv_buf, nullptr, valid_rows, rows,
-                                       3 * hidden, hidden, stream));
+      check_bt_error(bt_gemm_f32_split_with(inter_matmul_buf, sp.x_exps, w_pairs[0], sp.w_exps[0],
+                                            param_.attention_param.attr_bias_QKV, qkv_buf, nullptr, valid_rows, rows,
+                                            3 * hidden, hidden, &more, stream));
     } else {
       check_bt_error(bt_gemm_f32(from_tensor, gather, param_.attr_kernel_QKV,
                                  param_.attention_param.attr_bias_QKV, qkv_buf, 0, valid_rows, rows, rows_hint,
@@ -268,12 +269,10 @@ void BertTransformer<OpType>::bert_infer(BertTransformerInferParam infer_param) 
       // (Q, K, V are dead: the attention's pairs take the first tensor's place, the LayerNorm's the second's)
       DataType_ *att_pairs = qkv_buf, *ln_pairs = qkv_buf + tensor;
       // (the tiles of the padded batch, also where the caller's offsets bring the count: the same bits with and without them)
-      const auto more = [&](const DataType_ *weight, unsigned *raw = nullptr, const unsigned *a_raw = nullptr) {
-        return bt_f32_split_more{rows, raw, a_raw, weight};
-      };
-      const bt_f32_split_more proj = more(w_use[1]), ffn1 = more(w_use[2], sp.raw), ffn2 = more(w_use[3], nullptr, sp.raw);
-      check_bt_error(bt_split_f32(0, nullptr, nullptr, nullptr, nullptr, nullptr, -1, nullptr, nullptr, attr_out_buf, att_pairs,
-                                  sp.att_exps, nullptr, valid_rows, packed_cap, hidden, stream));
+      const bt_f32_split_more proj{rows, nullptr, nullptr, w_use[1], attr_out_buf, nullptr},
+          ffn1{rows, sp.raw, nullptr, w_use[2], attr_matmul_buf, nullptr}, ffn2{rows, nullptr, sp.raw, w_use[3], nullptr, nullptr};
+      check_bt_error(bt_split_f32_layer(0, nullptr, nullptr, nullptr, nullptr, nullptr, -1, nullptr, nullptr, attr_out_buf,
+                                        att_pairs, sp.att_exps, nullptr, valid_rows, packed_cap, hidden, 1, stream));
       check_bt_error(bt_gemm_f32_split_with(att_pairs, sp.att_exps, w_pairs[1], sp.w_exps[1], nullptr, attr_matmul_buf, nullptr,
                                             valid_rows, packed_cap, hidden, hidden, &proj, stream));
       check_bt_error(bt_add_bias_residual_layernorm_f32_split_layer(

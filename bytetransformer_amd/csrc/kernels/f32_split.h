@@ -25,18 +25,40 @@ __device__ __forceinline__ int split_exponent(float m) {
 }
 __device__ __forceinline__ float split_power(int e) { return __builtin_bit_cast(float, (unsigned)(e + 127) << 23); }
 
-// Four scaled values (float4 c of a row) into the row's pairs.
-__device__ __forceinline__ void split_store(half_t *row, int c, float4_t x) {
+// What a value v says of its row (or chunk of a column): the pairs hold a row unless a fifth of its values that are not zero
+// lie so far below the largest that they are lost, and the sum of these is positive.  (A few small ones among others
+// lose nothing that shows beside those.)
+__device__ __forceinline__ int split_score(float v, float scale) {
+  const float x = v * scale;
+  return v == 0.f ? 0 : split_pair(x).held && x != 0.f ? -1 : 4;
+}
+__device__ __forceinline__ int split_score(float4_t v, float scale) {
+  return split_score(v[0], scale) + split_score(v[1], scale) + split_score(v[2], scale) + split_score(v[3], scale);
+}
+// No scaled value from here on is lost (half the spacing of l is 2^-36 of it, and held is 2^-22 of the value).
+constexpr float kSplitHeldFrom = 1.0f / (1 << 14);
+// An exponent that carries this mark is that of a row whose sums are formed from its floats.
+constexpr int kSplitMark = 1 << 12;
+__device__ __forceinline__ bool split_marked(int e) { return e >= kSplitMark / 2; }
+__device__ __forceinline__ int split_unmarked(int e) { return split_marked(e) ? e - kSplitMark : e; }
+
+// Four scaled values (float4 c of a row) into the row's pairs; true if one may be lost.
+__device__ __forceinline__ bool split_store(half_t *row, int c, float4_t x) {
   half4_t h, l;
+  bool small = false;
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     const SplitPair p = split_pair(x[e]);
-    h[e] = p.h, l[e] = p.l;
+    h[e] = p.h, l[e] = p.l, small = small || __builtin_fabsf(x[e]) < kSplitHeldFrom;
   }
   half_t *to = row + (c >> 3) * 64 + (c & 7) * 4;
   store_through(to, __builtin_bit_cast(uint2_t, h));
   store_through(to + 32, __builtin_bit_cast(uint2_t, l));
+  return small;
 }
+
+// Where a row of pairs holds floats instead: a word that is not zero if it does at all, and a bit for every 32 columns.
+__host__ __device__ constexpr int split_raw_words(int columns) { return 1 + (columns + 1023) / 1024; }
 
 // 0.5 x (1 + tanh(u)) == x / (1 + exp(-2u)),  u = 0.79788456 (x + 0.044715 x^3), the exponent folded into one polynomial
 __device__ __forceinline__ float f32_gelu(float x) {

@@ -803,7 +803,7 @@ struct F32LnPairs {
   int *gelu_exps;        // [rows]
   const float *bounds;   // [bound_count][2]: largest |w| and |bias| of some columns each
   int bound_count;
-  unsigned *raw;         // [rows][raw_words] cleared for the product that reads the pairs (its rows that stay floats), or null
+  unsigned *raw;         // [rows][raw_words] cleared for the product that reads the pairs (its rows that stay floats), or null: no marks either
   int raw_words;
 };
 
@@ -892,19 +892,28 @@ __device__ __forceinline__ void f32_layernorm_block(
     const int e = split_exponent(wave_max(most));
     const float scale = split_power(e);
     float norm = 0.f;   // of the scaled row: at most 2^30 H
+    bool small = false;
 #pragma unroll
     for (int i = 0; i < NC; ++i) {
       const int c = lane + i * kWave;
       if (c >= chunks) continue;
       const float4_t x = v[i] * scale;
-      split_store(next.pairs + (size_t)r * chunks * 8, c, x);
+      small = split_store(next.pairs + (size_t)r * chunks * 8, c, x) || small;
       norm += x[0] * x[0] + x[1] * x[1] + x[2] * x[2] + x[3] * x[3];
     }
     // (a bound that is no float is the largest float: finite results fit it, and a row with an infinity or NaN has none)
     const float row_norm = sqrtf(wave_sum(norm) * (float)(chunks * 4)) * split_power(-e);
     const float bound = fminf(row_norm * wave_max(w_most) + wave_max(bias_most), 3.402823466e38f);
+    bool marked = false;
+    if (next.raw && __builtin_amdgcn_ballot_w64(small) != 0) {
+      int score = 0;
+#pragma unroll
+      for (int i = 0; i < NC; ++i)
+        if (lane + i * kWave < chunks) score += split_score(v[i], scale);
+      marked = wave_total(score) > 0;
+    }
     if (lane == 0) {
-      next.exps[r] = e;
+      next.exps[r] = e + (marked ? kSplitMark : 0);
       next.gelu_exps[r] = split_exponent(bound);
     }
     if (lane < next.raw_words) next.raw[(size_t)r * next.raw_words + lane] = 0;
@@ -1116,11 +1125,11 @@ extern "C" int bt_add_bias_residual_layernorm_f32_split_layer(
   BT_REQUIRE(out && residual && bias && gamma && beta && pairs && exps && gelu_exps && bounds, BT_ERR_INVALID_ARGUMENT,
              "%s: null pointer argument", who);
   BT_REQUIRE(rows_cap >= 0 && bound_count > 0, BT_ERR_INVALID_ARGUMENT, "%s: rows_cap=%d bound_count=%d", who, rows_cap, bound_count);
-  BT_REQUIRE(!raw || (n > 0 && n <= 1024 * kWave), BT_ERR_INVALID_ARGUMENT, "%s: n=%d outside [1, 2^16]", who, n);   // (a word a lane)
+  BT_REQUIRE(!raw || (n > 0 && split_raw_words(n) <= kWave), BT_ERR_INVALID_ARGUMENT, "%s: n=%d", who, n);   // (a word a lane)
   BT_REQUIRE(!residual_row_index || valid_rows, BT_ERR_INVALID_ARGUMENT, "%s: residual_row_index needs valid_rows", who);
   BT_REQUIRE(hidden_dim % 32 == 0 && aligned16({pairs}), BT_ERR_UNSUPPORTED,
              "%s: hidden_dim=%d must be a multiple of 32, the pairs 16-byte aligned", who, hidden_dim);
-  const F32LnPairs next{(half_t *)pairs, exps, gelu_exps, bounds, bound_count, raw, raw ? (n + 1023) / 1024 : 0};
+  const F32LnPairs next{(half_t *)pairs, exps, gelu_exps, bounds, bound_count, raw, raw ? split_raw_words(n) : 0};
   return launch_f32_ln<false>(out, residual, bias, gamma, beta, out, valid_rows, residual_row_index, 1, rows_cap, hidden_dim,
                               eps, as_stream(stream), who, &next);
 }

@@ -16,7 +16,10 @@
 // accumulator) the operands are rounded, but the sums are half to a sixth as many roundings: see
 // bt_gemm_f32_split in bt_hip.h for both errors.
 // Infinities and NaN keep their places in h (the scale comes from the finite values of a row); a row with a sum that is
-// not finite is formed again by float multiply-adds.
+// not finite is formed again, from the floats.
+//
+// Rows and chunks of columns of which the pairs hold less, because a few values are out of all proportion to the rest, are
+// marked (split_score), and what they enter is summed from the floats: a zero meets the large value as like as not.
 //
 // The scale of FFN1's results has to be known before them, so it comes from a bound.  One large column makes that bound
 // and with it what 2^-50 is worth to the results of all others, be it 10^12 times as large as any of them.  So where
@@ -54,7 +57,7 @@ struct SplitArgs {
   SplitWeight weight[4];
   int count, units;
   int bounded;              // the weight that `bounds` speaks of, -1: none
-  int gelu;                 // ... of GELU(. W + bias): what a bias adds to the largest |result| (else |bias|)
+  int layer;                // bounds of GELU(. W + bias): what a bias adds to the largest |result| (else |bias|); marks
   const float *bias;        // [N] its bias
   float *bounds;            // [units of that weight][2]: largest finite |w| and |bias| of its columns
   const float *rows;        // rows to split as well, or null
@@ -72,6 +75,7 @@ __device__ __forceinline__ void split_weight_unit(const SplitArgs &a, int unit) 
   constexpr int kPasses = kSplitChunk / (kSplitThreads / 8);   // 64 rows each
   __shared__ float4_t s_most[kSplitThreads / 64][8];
   __shared__ float s_scale[kSplitCols];
+  __shared__ int s_score[kSplitThreads / 64][8][2];   // two columns each
   __shared__ __attribute__((aligned(16))) half_t s_tile[kSplitCols * kSplitPitch];
   int j = 0, first = 0;
 #pragma unroll
@@ -101,18 +105,19 @@ __device__ __forceinline__ void split_weight_unit(const SplitArgs &a, int unit) 
     for (int e = 0; e < 4; ++e) most[e] = fmaxf(most[e], __shfl_xor(most[e], o, 64));
   if (lane < 8) s_most[wave][lane] = most;
   __syncthreads();
+  int column_e = 0;
   if (t < kSplitCols) {
     float m = 0.f;
 #pragma unroll
     for (int w = 0; w < kSplitThreads / 64; ++w) m = fmaxf(m, s_most[w][t >> 2][t & 3]);
     const int e = split_exponent(m);
     s_scale[t] = split_power(e);
-    jb.exps[(size_t)chunk * jb.N + n0 + t] = e;
+    column_e = e;
     if (j == a.bounded) {
       // (|GELU(x)| <= x above zero, 0.17 and |x| below)
       const float of = a.bias[n0 + t];
       float b = finite_or_zero(of);
-      if (a.gelu && of < 0.f) b = fminf(b, 0.1701f);
+      if (a.layer && of < 0.f) b = fminf(b, 0.1701f);
 #pragma unroll
       for (int o = 1; o < 32; o <<= 1) m = fmaxf(m, __shfl_xor(m, o, 64)), b = fmaxf(b, __shfl_xor(b, o, 64));
       if (t == 0) a.bounds[2 * u] = m, a.bounds[2 * u + 1] = b;
@@ -122,17 +127,32 @@ __device__ __forceinline__ void split_weight_unit(const SplitArgs &a, int unit) 
   float scale[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) scale[e] = s_scale[4 * cq + e];
+  int score[2] = {0, 0};   // columns 0 and 1, 2 and 3: 16 bits each, at most 1024
 #pragma unroll
   for (int i = 0; i < kPasses; ++i) {
     half_t *to = s_tile + (64 * i + (r0 & 32)) * 2 + (r0 & 31);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const SplitPair p = split_pair(v[i][e] * scale[e]);
+      const float x = v[i][e] * scale[e];
+      const SplitPair p = split_pair(x);
       to[(4 * cq + e) * kSplitPitch] = p.h;
       to[(4 * cq + e) * kSplitPitch + 32] = p.l;
+      score[e >> 1] += split_score(v[i][e], scale[e]) * (e & 1 ? 1 << 16 : 1);
     }
   }
+#pragma unroll
+  for (int o = 8; o < 64; o <<= 1)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) score[h] += __shfl_xor(score[h], o, 64);
+  if (lane < 8) s_score[wave][lane][0] = score[0], s_score[wave][lane][1] = score[1];
   __syncthreads();
+  if (t < kSplitCols) {
+    int both = 0;
+#pragma unroll
+    for (int w = 0; w < kSplitThreads / 64; ++w) both += s_score[w][t >> 2][t >> 1 & 1];
+    const int low = (int)(short)(both & 0xffff), mine = t & 1 ? (both - low) >> 16 : low;
+    jb.exps[(size_t)chunk * jb.N + n0 + t] = column_e + (a.layer && mine > 0 ? kSplitMark : 0);
+  }
   const int rows = min(kSplitChunk, jb.K - k0), chunks16 = rows / 4;   // 16-byte pieces of a column
   for (int at = t; at < kSplitCols * (kSplitChunk / 4); at += kSplitThreads) {
     const int n = at / (kSplitChunk / 4), c = at % (kSplitChunk / 4);
@@ -156,9 +176,17 @@ __global__ __launch_bounds__(kSplitThreads) void split_f32_kernel(SplitArgs a) {
     for (int e = 0; e < 4; ++e) most = fmaxf(most, finite_or_zero(v[e]));
   }
   const int e = split_exponent(wave_max(most));
-  if (lane == 0) a.row_exps[r] = e;
   const float scale = split_power(e);
-  for (int c = lane; c < a.hidden / 4; c += 64) split_store(a.row_pairs + (size_t)r * 2 * a.hidden, c, src[c] * scale);
+  bool small = false;
+  for (int c = lane; c < a.hidden / 4; c += 64)
+    small = split_store(a.row_pairs + (size_t)r * 2 * a.hidden, c, src[c] * scale) || small;
+  bool marked = false;
+  if (a.layer && __builtin_amdgcn_ballot_w64(small) != 0) {
+    int score = 0;
+    for (int c = lane; c < a.hidden / 4; c += 64) score += split_score(src[c], scale);
+    marked = wave_total(score) > 0;
+  }
+  if (lane == 0) a.row_exps[r] = e + (marked ? kSplitMark : 0);
 }
 
 // ---------------------------------------------------------------------------
@@ -167,83 +195,71 @@ __global__ __launch_bounds__(kSplitThreads) void split_f32_kernel(SplitArgs a) {
 struct F32SplitTail {
   const float *bias;   // [N] or null
   const int *gelu_exps;   // GELU: exponent that a row of the result is scaled by
-  unsigned *raw;          // GELU: a bit for every 32 columns of a row that are floats, [rows][ceil(N / 1024)], or null
+  unsigned *raw;          // GELU: where a row of the result holds floats, [rows][split_raw_words(N)], or null
   const unsigned *a_raw;  // the same of the rows of a, or null
   const float *w;         // [K, N] the weight itself, or null
+  const float *a_rows;    // row a_row_index[r] (r without an index) is what row r of a was made of, or null
+  const int *a_row_index;
 };
 #define BT_F32_SPLIT_FIRST                                                                                  \
   const half_t *a, const half_t *w, const int *valid_rows, const int *a_exps, const int *w_exps, void *out, \
       int rows_cap, int N, int K, unsigned per_n
+constexpr int kF32SplitFirstBytes = 64;   // the tail's place among the arguments
 
 #if defined(__HIP_DEVICE_COMPILE__)
 constexpr float kGeluFloor = 1.0f / (1 << 20);   // results below it may go: what they add is a rounding of what made the scale
 
-// Rows of a wave's 16 x WTN block again, by float multiply-adds over k, 256 values at a time: those that the matrix
-// instructions cannot form.  A lane has a column and four rows at a time; the loads of a row are the same for all of them.
-// (Some ten times as slow as the product of pairs, on rows that ordinary operands do not have.)
-template <int WTN, bool GELU>
-__device__ __forceinline__ void split_rows_again(BT_F32_SPLIT_FIRST, const F32SplitTail &tail, int m_first, unsigned rows,
-                                                 int n_first, int M, int lane) {
-  constexpr int kRows = 4, kSides = 64 / WTN;
-  const int side = lane / WTN, n = n_first + lane % WTN, n_in = min(n, N - 1);
-  const int a_words = (K + 1023) / 1024, out_words = (N + 1023) / 1024;
-  const size_t pitch = 2 * (size_t)K;
-  for (int first = 0; first < 16; first += kRows * kSides) {
-    if ((rows >> first & ((1u << kRows * kSides) - 1)) == 0) continue;
-    const int row = first + side * kRows;
-    float sum[kRows], part[kRows];
-    int ea[kRows];
+// Sums of 16 rows and 16 TN columns on float matrix instructions, from the floats where there are any: those that the pairs
+// do not give.  Lane (fr, lg): columns 16 i + 4 lg .. + 3 of row fr, as the products of pairs leave them; it brings row fr
+// and columns 16 i + fr, values 4 lg .. 4 lg + 3 of every 16 of k, four loads of a column being one step's operands.
+// Summed 256 values at a time.  It waits for its own loads at every step: a layer of 16 x 256, hidden 768, whose FFN2
+// comes from here takes 584 us in place of 213 (by float multiply-adds, four rows a lane, 1860).
+template <int TN>
+__device__ __forceinline__ void split_sums_of_floats(const half_t *a, const half_t *w, const int *a_exps, const int *w_exps,
+                                                     const F32SplitTail &tail, int N, int K, int m, int n_first, int fr, int lg,
+                                                     float4_t (&sum)[TN]) {
+  const float4_t zero4 = {0.f, 0.f, 0.f, 0.f};
+  float4_t part[TN];
 #pragma unroll
-    for (int r = 0; r < kRows; ++r) sum[r] = part[r] = 0.f, ea[r] = a_exps[min(m_first + row + r, M - 1)];
+  for (int i = 0; i < TN; ++i) sum[i] = part[i] = zero4;
+  const int ea = split_unmarked(a_exps[m]);
+  const unsigned *raw = tail.a_raw ? tail.a_raw + (size_t)m * split_raw_words(K) : nullptr;
+  const float *row = tail.a_rows ? tail.a_rows + (size_t)(tail.a_row_index ? tail.a_row_index[m] : m) * K : nullptr;
 #pragma unroll 1
-    for (int b = 0; b < K / 32; ++b) {
-      const int ew = w_exps[(size_t)(b * 32 / kSplitChunk) * N + n_in];
-#pragma unroll 1
-      for (int k = 0; k < 32; k += 4) {
-        float y[4];
+  for (int k0 = 0; k0 < K; k0 += 16) {
+    const int b = k0 >> 5, k = (k0 & 16) + 4 * lg;   // in its block
+    float4_t x, y[TN];
+    if (row) {
+      x = *(const float4_t *)(row + k0 + 4 * lg);
+    } else {
+      const half_t *block = a + (size_t)m * 2 * K + b * 64;
+      const half4_t h = *(const half4_t *)(block + k), l = *(const half4_t *)(block + 32 + k);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const half_t *pair = w + n_in * pitch + b * 64 + k + e;
-          y[e] = tail.w ? tail.w[(size_t)(b * 32 + k + e) * N + n_in]
-                        : __builtin_amdgcn_ldexpf((float)pair[0] + (float)pair[32] * kSplitLow, -ew);
-        }
-#pragma unroll
-        for (int r = 0; r < kRows; ++r) {
-          const size_t m = min(m_first + row + r, M - 1);
-          const half_t *pairs = a + m * pitch + b * 64;
-          float4_t x;
-          if (tail.a_raw && (tail.a_raw[m * a_words + (b >> 5)] >> (b & 31) & 1)) {
-            x = *(const float4_t *)((const float *)pairs + k);
-          } else {
-            const half4_t h = *(const half4_t *)(pairs + k), l = *(const half4_t *)(pairs + 32 + k);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) x[e] = __builtin_amdgcn_ldexpf((float)h[e] + (float)l[e] * kSplitLow, -ea[r]);
-          }
-#pragma unroll
-          for (int e = 0; e < 4; ++e) part[r] = __builtin_fmaf(x[e], y[e], part[r]);
-        }
-      }
-      if ((b + 1) % (kSplitChunk / 32) == 0 || b + 1 == K / 32)
-#pragma unroll
-        for (int r = 0; r < kRows; ++r) sum[r] += part[r], part[r] = 0.f;
+      for (int e = 0; e < 4; ++e) x[e] = __builtin_amdgcn_ldexpf((float)h[e] + (float)l[e] * kSplitLow, -ea);
+      if (raw && (raw[1 + (b >> 5)] >> (b & 31) & 1)) x = *(const float4_t *)((const float *)block + k);
     }
 #pragma unroll
-    for (int r = 0; r < kRows; ++r) {
-      const int m = m_first + row + r;
-      if (!(rows >> (row + r) & 1) || m >= M || n >= N) continue;
-      float v = sum[r];
-      if (tail.bias) v += tail.bias[n];
-      if (!GELU) {
-        ((float *)out)[(size_t)m * N + n] = v;
-      } else if (v = f32_gelu(v); tail.raw) {
-        ((float *)out)[(size_t)m * N + n] = v;
-        if (n % 32 == 0) atomicOr(tail.raw + (size_t)m * out_words + (n >> 10), 1u << (n >> 5 & 31));
+    for (int i = 0; i < TN; ++i) {
+      const int n = min(n_first + 16 * i + fr, N - 1);
+      if (tail.w) {
+        const float *from = tail.w + (size_t)k0 * N;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[i][e] = from[(unsigned)((4 * lg + e) * N + n)];
       } else {
-        const SplitPair p = split_pair(v * split_power(tail.gelu_exps[m]));
-        half_t *pair = (half_t *)out + (size_t)m * 2 * N + (n >> 5) * 64 + (n & 31);
-        pair[0] = p.h, pair[32] = p.l;
+        const half_t *block = w + (size_t)n * 2 * K + b * 64;
+        const half4_t h = *(const half4_t *)(block + k), l = *(const half4_t *)(block + 32 + k);
+        const int ew = split_unmarked(w_exps[(size_t)(k0 / kSplitChunk) * N + n]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[i][e] = __builtin_amdgcn_ldexpf((float)h[e] + (float)l[e] * kSplitLow, -ew);
       }
     }
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int i = 0; i < TN; ++i) part[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(y[i][e], x[e], part[i], 0, 0, 0);
+    if ((k0 + 16) % kSplitChunk == 0 || k0 + 16 >= K)
+#pragma unroll
+      for (int i = 0; i < TN; ++i) sum[i] += part[i], part[i] = zero4;
   }
 }
 
@@ -301,17 +317,13 @@ __device__ __forceinline__ void f32_split_tile(BT_F32_SPLIT_FIRST, const F32Spli
   for (int i = 0; i < TN; ++i)
 #pragma unroll
     for (int j = 0; j < TM; ++j) sum[i][j] = hh[i][j] = cross[i][j] = zero4;
-  // (bit j: rows of block j that hold floats)
-  unsigned marked = 0;
-  if (tail.a_raw) {
-    const int words = (K + 1023) / 1024;
+  // (of row fr of block j: on their way beside the first k-steps, looked at behind the last)
+  int ea[TM];
+  unsigned holds_floats[TM];
 #pragma unroll
-    for (int j = 0; j < TM; ++j) {
-      const unsigned *of = tail.a_raw + (size_t)min(m0 + wm * WTM + 16 * j + fr, M - 1) * words;
-      unsigned any = 0;
-      for (int i = 0; i < words; ++i) any |= of[i];
-      marked |= (any != 0 ? 1u : 0u) << j;
-    }
+  for (int j = 0; j < TM; ++j) {
+    const size_t m = min(m0 + wm * WTM + 16 * j + fr, M - 1);
+    ea[j] = a_exps[m], holds_floats[j] = tail.a_raw ? tail.a_raw[m * split_raw_words(K)] : 0;
   }
   // The weight's scales: behind the ring, factor[c][n] = 2^(e - exponent of chunk c of column n), e[n] the smallest of the
   // column's, so that no factor is above 1.  (They are on their way beside the first k-steps.)
@@ -320,14 +332,15 @@ __device__ __forceinline__ void f32_split_tile(BT_F32_SPLIT_FIRST, const F32Spli
   int *column_e = (int *)factor + chunks * BN;
   for (int n = threadIdx.x; n < BN; n += NW * 64) {
     const int *from = w_exps + min(n0 + n, N - 1);
-    int least = 1 << 20;
+    int least = 1 << 20, mark = 0;
     for (int c = 0; c < chunks; ++c) {
-      const int e = from[(size_t)c * N];
+      const int e = split_unmarked(from[(size_t)c * N]);
+      mark |= split_marked(from[(size_t)c * N]) ? kSplitMark : 0;
       least = min(least, e);
       ((int *)factor)[c * BN + n] = e;
     }
     for (int c = 0; c < chunks; ++c) factor[c * BN + n] = __builtin_amdgcn_ldexpf(1.f, least - ((int *)factor)[c * BN + n]);
-    column_e[n] = least;
+    column_e[n] = least + mark;
   }
   __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): there, behind the first barrier of the loop
   constexpr int kFold = kSplitChunk / 32 / KG;   // k-steps of a group in a chunk
@@ -447,10 +460,16 @@ __device__ __forceinline__ void f32_split_tile(BT_F32_SPLIT_FIRST, const F32Spli
   // lane: columns n .. n + 3 of block i, row m of block j
   int4_t ew[TN];
   float4_t bias[TN];
+  bool column = false;   // one of the wave's columns is marked
 #pragma unroll
   for (int i = 0; i < TN; ++i) {
     const int n = min(n0 + wn * WTN + 16 * i + 4 * lg, N - 4);
     ew[i] = *(const int4_t *)(column_e + wn * WTN + 16 * i + 4 * lg);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      column = column || (split_marked(ew[i][e]) && n0 + wn * WTN + 16 * i + 4 * lg < N);
+      ew[i][e] = split_unmarked(ew[i][e]);
+    }
     bias[i] = float4_t{0.f, 0.f, 0.f, 0.f};
     if (tail.bias)
 #pragma unroll
@@ -459,27 +478,64 @@ __device__ __forceinline__ void f32_split_tile(BT_F32_SPLIT_FIRST, const F32Spli
   constexpr int EP = 2 * WTN + 8;   // halfs of a staged row of pairs
   static_assert(!GELU || (size_t)NW * 16 * EP <= (size_t)STAGES * STAGE_HALFS, "staging fits the ring");
   half_t *staged = split_smem + wave_all * 16 * EP;
-  unsigned again[TM];   // rows of block j
-  if (GELU) __builtin_amdgcn_s_barrier();   // everyone is done with the ring
+  column = __builtin_amdgcn_ballot_w64(column) != 0;
+  // Rows that the pairs do not give: marked ones, those under a marked column, and those with a sum that is not finite.
+  // (Dead rows hold what the scratch held before, and do not count.)
+  unsigned again[TM], any = 0;
 #pragma unroll
   for (int j = 0; j < TM; ++j) {
     again[j] = 0;
     if (KG > 1 && (j < kFirstRows) != (group == 0)) continue;
+    const int m = m0 + wm * WTM + 16 * j + fr;
+    bool wrong = column || split_marked(ea[j]) || holds_floats[j] != 0;
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) wrong = wrong || !(__builtin_fabsf(sum[i][j][e]) < __builtin_inff());
+    const unsigned long long rows = __builtin_amdgcn_ballot_w64(wrong && m < M);
+    again[j] = (unsigned)(rows | rows >> 16 | rows >> 32 | rows >> 48) & 0xffffu;
+    any |= again[j];
+  }
+  if (any != 0) {
+    // (What only this needs is read from the arguments here: held in registers from the start, it pushed others of the loop out.)
+    typedef const __attribute__((address_space(4))) char *arguments_t;
+    arguments_t late = (arguments_t)__builtin_amdgcn_kernarg_segment_ptr() + kF32SplitFirstBytes;
+    asm volatile("" : "+s"(late));
+    const F32SplitTail rare = *(const __attribute__((address_space(4))) F32SplitTail *)late;
+    // (one copy of the code, two column blocks at a time, in the registers that a loop leaves: whose sums they are is picked
+    // behind it)
+#pragma unroll 1
+    for (int at = 0; at < TM * (TN / 2); ++at) {
+      const int j = at / (TN / 2), half = at % (TN / 2);
+      unsigned rows = again[0];
+#pragma unroll
+      for (int q = 1; q < TM; ++q) rows = q == j ? again[q] : rows;
+      if (rows == 0) continue;
+      float4_t formed[2];
+      split_sums_of_floats<2>(a, w, a_exps, w_exps, rare, N, K, min(m0 + wm * WTM + 16 * j + fr, M - 1),
+                              n0 + wn * WTN + 32 * half, fr, lg, formed);
+#pragma unroll
+      for (int q = 0; q < TM; ++q)
+#pragma unroll
+        for (int i = 0; i < TN; ++i)
+          if (q == j && i / 2 == half && (rows >> fr & 1)) sum[i][q] = formed[i & 1];
+    }
+  }
+  if (GELU) __builtin_amdgcn_s_barrier();   // everyone is done with the ring
+#pragma unroll
+  for (int j = 0; j < TM; ++j) {
+    if (KG > 1 && (j < kFirstRows) != (group == 0)) continue;
     const int m_first = m0 + wm * WTM + 16 * j, m = m_first + fr, m_in = min(m, M - 1);
-    const int ea = a_exps[m_in];
+    const bool formed = again[j] >> fr & 1;   // (not scaled)
+    const int e_row = split_unmarked(ea[j]);
     float to_pair = 1.f;
     if (GELU) to_pair = split_power(tail.gelu_exps[m_in]);
-    bool wrong = marked >> j & 1;
 #pragma unroll
     for (int i = 0; i < TN; ++i) {
       const int n = n0 + wn * WTN + 16 * i + 4 * lg;
       float4_t v;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float s = sum[i][j][e];
-        wrong = wrong || !(__builtin_fabsf(s) < __builtin_inff());
-        v[e] = __builtin_amdgcn_ldexpf(s, -(ea + ew[i][e]));
-      }
+      for (int e = 0; e < 4; ++e) v[e] = __builtin_amdgcn_ldexpf(sum[i][j][e], formed ? 0 : -(e_row + ew[i][e]));
       v += bias[i];
       if (!GELU) {
         if (m < M && n < N) store_through((float *)out + (size_t)m * N + n, __builtin_bit_cast(uint4_t, v));
@@ -489,14 +545,11 @@ __device__ __forceinline__ void f32_split_tile(BT_F32_SPLIT_FIRST, const F32Spli
       for (int e = 0; e < 4; ++e) v[e] = f32_gelu(v[e]);
       sum[i][j] = v;
     }
-    // (dead rows hold what the scratch held before)
-    const unsigned long long rows = __builtin_amdgcn_ballot_w64(wrong && m < M);
-    again[j] = (unsigned)(rows | rows >> 16 | rows >> 32 | rows >> 48) & 0xffffu;
     if (GELU) {
-      // Floats stay where the pairs hold three results from kGeluFloor on no longer, or one where all are small.  Values from
-      // 2^-14 on are always held, so rows whose bound is below 2^8, as ordinary ones are, are through with a comparison.
+      // Floats stay where the pairs hold three results from kGeluFloor on no longer, or one where all are small.  Rows
+      // whose bound is below 2^9, as ordinary ones are, lose none of those and are through with a comparison.
       bool raw = false;
-      if (tail.raw && __builtin_amdgcn_ballot_w64(to_pair * kGeluFloor < 1.0f / (1 << 13) && m < M) != 0) {
+      if (tail.raw && __builtin_amdgcn_ballot_w64(to_pair * kGeluFloor < kSplitHeldFrom && m < M) != 0) {
         int lost = 0;
         float most = 0.f;
 #pragma unroll
@@ -511,10 +564,13 @@ __device__ __forceinline__ void f32_split_tile(BT_F32_SPLIT_FIRST, const F32Spli
         for (int o = 16; o < 64; o <<= 1) lost += __shfl_xor(lost, o, 64), most = fmaxf(most, __shfl_xor(most, o, 64));
         raw = m < M && (lost >= 3 || (lost > 0 && most < 1.0f / 256));
         const int n_first = n0 + wn * WTN;
-        if (raw && lg == 0)
+        if (raw && lg == 0) {
+          unsigned *words = tail.raw + (size_t)m * split_raw_words(N);
+          words[0] = 1;
 #pragma unroll
           for (int n = n_first; n < n_first + WTN; n += 32)
-            if (n < N) atomicOr(tail.raw + (size_t)m * ((N + 1023) / 1024) + (n >> 10), 1u << (n >> 5 & 31));
+            if (n < N) atomicOr(words + 1 + (n >> 10), 1u << (n >> 5 & 31));
+        }
       }
 #pragma unroll
       for (int i = 0; i < TN; ++i) {
@@ -543,22 +599,6 @@ __device__ __forceinline__ void f32_split_tile(BT_F32_SPLIT_FIRST, const F32Spli
           store_through((half_t *)out + (size_t)(m_first + r) * 2 * N + (n0 + wn * WTN) * 2 + c * 8, v);
       }
     }
-  }
-
-  unsigned any = 0;
-#pragma unroll
-  for (int j = 0; j < TM; ++j) any |= again[j];
-  if (any == 0) return;
-  __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): the stores above have returned
-  // (one copy of the code: the block's rows picked by a loop that stays one)
-#pragma unroll 1
-  for (int j = 0; j < TM; ++j) {
-    unsigned rows = again[0];
-#pragma unroll
-    for (int i = 1; i < TM; ++i) rows = i == j ? again[i] : rows;
-    if (rows)
-      split_rows_again<WTN, GELU>(a, w, valid_rows, a_exps, w_exps, out, rows_cap, N, K, per_n, tail, m0 + wm * WTM + 16 * j, rows,
-                                  n0 + wn * WTN, M, lane);
   }
 }
 #endif  // __HIP_DEVICE_COMPILE__
@@ -629,7 +669,7 @@ extern "C" int bt_split_f32_layer(int weight_count, const void *const *w, void *
   }
   a.count = weight_count, a.units = units;
   a.bounded = bounded < 0 ? -1 : bounded, a.bias = (const float *)bounded_bias, a.bounds = bounds;
-  a.gelu = layer;
+  a.layer = layer;
   int row_blocks = 0;
   if (rows) {
     BT_REQUIRE(row_pairs && row_exps && row_pairs != rows, BT_ERR_INVALID_ARGUMENT, "%s: rows need an area of their own for the pairs", who);
@@ -664,8 +704,9 @@ extern "C" int bt_gemm_f32_split_with(const void *a_pairs, const int *a_exps, co
   if (rows_cap == 0) return BT_OK;
   const bt_f32_split_more none{}, &m = more ? *more : none;
   BT_REQUIRE(!m.raw || gelu_exps, BT_ERR_INVALID_ARGUMENT, "%s: floats among the pairs of a result that is not pairs", who);
+  BT_REQUIRE(aligned16({m.a, m.w}), BT_ERR_INVALID_ARGUMENT, "%s: pointers must be 16-byte aligned", who);
   const F32SplitArgs p{(const half_t *)a_pairs, (const half_t *)w_pairs, valid_rows, a_exps, w_exps, c, rows_cap, n, k,
-                       {(const float *)bias, gelu_exps, m.raw, m.a_raw, (const float *)m.w}};
+                       {(const float *)bias, gelu_exps, m.raw, m.a_raw, (const float *)m.w, (const float *)m.a, m.a_row_index}};
   hipStream_t s = as_stream(stream);
   // Tiles: 0: 64x64, two groups of waves over k, two workgroups a CU | 1: 64x128 likewise, one | 2: 96x128, one group, two.
   // What a step waits for is its operands: a CU takes in about 40 bytes a clock from the L2 and reads 128 from the LDS, and

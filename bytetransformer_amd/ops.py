@@ -443,17 +443,18 @@ def split_f32(ws, rows=None, bounded=-1, bounded_bias=None, row_index=None, vali
     return list(zip(pairs, exps)), got, bounds
 
 
-def gemm_f32_split(a, w, bias=None, gelu_exps=None, valid_rows=None, out=None, raw=None, a_raw=None, weight=None, tile_rows=0):
+def gemm_f32_split(a, w, bias=None, gelu_exps=None, valid_rows=None, out=None, raw=None, a_raw=None, weight=None, rows=None,
+                   row_index=None, tile_rows=0):
     """c = a . w (+ bias) of split operands (pairs, exps), or the pairs of its GELU scaled by 2^gelu_exps; raw, a_raw
-    (int32 [rows, ceil(columns / 1024)]) and the weight itself as in bt_f32_split_more."""
+    (int32 [rows, 1 + ceil(columns / 1024)]), the weight and the rows themselves as in bt_f32_split_more."""
     (ap, ae), (wp, we) = a, w
-    rows, n, k = ap.shape[0], wp.shape[0], wp.shape[1] * 32
+    cap, n, k = ap.shape[0], wp.shape[0], wp.shape[1] * 32
     if out is None:
-        out = torch.zeros(*((rows, n) if gelu_exps is None else (rows, n // 32, 64)), device=ap.device,
+        out = torch.zeros(*((cap, n) if gelu_exps is None else (cap, n // 32, 64)), device=ap.device,
                           dtype=torch.float32 if gelu_exps is None else torch.float16)
-    more = F32SplitMore(tile_rows, _ptr(raw), _ptr(a_raw), _ptr(weight))
+    more = F32SplitMore(tile_rows, _ptr(raw), _ptr(a_raw), _ptr(weight), _ptr(rows), _ptr(row_index))
     _check(kernel_lib().bt_gemm_f32_split_with(_ptr(ap), _ptr(ae), _ptr(wp), _ptr(we), _ptr(bias), _ptr(out), _ptr(gelu_exps),
-                                               _ptr(valid_rows), rows, n, k, ctypes.byref(more), _stream()))
+                                               _ptr(valid_rows), cap, n, k, ctypes.byref(more), _stream()))
     return out
 
 
@@ -509,7 +510,7 @@ def add_bias_residual_layernorm_f32_split(out, residual, bias, gamma, beta, boun
     _check(kernel_lib().bt_add_bias_residual_layernorm_f32_split_layer(
         _ptr(out), _ptr(residual), _ptr(residual_row_index), _ptr(bias), _ptr(gamma), _ptr(beta), _ptr(valid_rows), rows,
         hidden, float(eps), _ptr(pairs), _ptr(exps), _ptr(gelu_exps), _ptr(bounds), bounds.shape[0], _ptr(raw),
-        0 if raw is None else raw.shape[1] * 1024, _stream()))
+        0 if raw is None else (raw.shape[1] - 1) * 1024, _stream()))
     return pairs, exps, gelu_exps
 
 

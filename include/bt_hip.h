@@ -471,13 +471,16 @@ int bt_splitk_layernorm(const void *partials, int splits, const void *residual,
  *                      row r scaled by 2^gelu_exps[r]; n a multiple of 32, k of 64.  Distance from float64 (2-norm; largest
  *                      difference over the largest result) for normal operands: k = 768 1.4e-7, 2.5e-7, k = 3072 1.5e-7,
  *                      2.4e-7, where bt_gemm_f32 has 2.1e-7, 3.5e-7 and 4.3e-7, 7.0e-7.
- *   bt_gemm_f32_split_with  the same, told more (`more` nullable).  It forms the rows of which a_raw has a bit, and those
- *                      with a sum that is not finite, by float multiply-adds over k, some ten times as slowly.
+ *   bt_gemm_f32_split_with  the same, told more (`more` nullable).  The rows of which a_raw speaks or whose exponent has that
+ *                      mark, those with a sum that is not finite, and all where a weight's column has the mark, it forms from
+ *                      the floats (float matrix instructions, three to five times as slowly).
  *   bt_split_f32_layer  layer = 1: the second of a pair of bounds is what a bias adds to the largest |GELU(. W + bias)|, so
- *                      a large negative one counts for nothing.
+ *                      a large negative one counts for nothing; and 2^12 is added to the exponent of a row, or of 256 values of
+ *                      a column, whose pairs hold less than four fifths of its values (that are not zero) to 2^-22 of themselves.
  *   bt_add_bias_residual_layernorm_f32_split  bt_add_bias_residual_layernorm_f32 that writes the pairs of its rows as
  *                      well, and exponents that keep the pairs of GELU(row . W + b) in range for the W of `bounds`;
- *                      ..._layer clears the rows of `raw` (of bt_f32_split_more; nullable) for a W of n columns, at most 2^16.
+ *                      ..._layer clears the rows of `raw` (of bt_f32_split_more; nullable) for a W of n columns, at most 63 * 1024,
+ *                      and marks exponents.
  */
 int bt_split_f32(int weight_count, const void *const *w, void *const *w_pairs, int *const *w_exps, const int *k,
                  const int *n, int bounded, const void *bounded_bias, float *bounds, const void *rows, void *row_pairs,
@@ -492,12 +495,16 @@ typedef struct bt_f32_split_more {
   /* > 0: the tile is the one of a launch of this capacity.  Tiles add up in different orders, so a caller that knows its
    * row count in one call and not in the next names the capacity here in both, and the bits stay. */
   int tile_rows;
-  /* gelu_exps != NULL: [rows_cap][ceil(n / 1024)], all zero.  Bit b of a row is set where its columns 32 b .. 32 b + 31
-   * are floats in the place of their pairs, because the pairs would not hold them (one large column of the weight, say,
-   * that makes the exponent); without it they are pairs all the same, to 2^-50 of that column. */
+  /* gelu_exps != NULL: [rows_cap][1 + ceil(n / 1024)], all zero.  Where columns 32 b .. 32 b + 31 of a row are floats in the
+   * place of their pairs, because the pairs would not hold them (one large column of the weight, say, that makes the
+   * exponent), the first word of the row and bit b of the others are set; without it they are pairs all the same, to 2^-50
+   * of that column. */
   unsigned *raw;
   const unsigned *a_raw;   /* what the product that made a_pairs left in its `raw` */
-  const void *w;           /* float [k, n], the weight itself, for rows that are summed by float multiply-adds */
+  /* The operands themselves, for rows that are formed from floats (NULL: those that the pairs stand for): float [k, n], and rows
+   * a_row_index[r] (r without an index) of `a` */
+  const void *w, *a;
+  const int *a_row_index;
 } bt_f32_split_more;
 int bt_gemm_f32_split_with(const void *a_pairs, const int *a_exps, const void *w_pairs, const int *w_exps, const void *bias,
                            void *c, const int *gelu_exps, const int *valid_rows, int rows_cap, int n, int k,

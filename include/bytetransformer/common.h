@@ -124,7 +124,7 @@ struct F32SplitScratch {
   static unsigned long long chunks(unsigned long long k) { return (k + 255) / 256; }
   static unsigned long long bytes(unsigned long long rows, unsigned long long hidden, unsigned long long inter) {
     return (4 * ((rows + 3) / 4 * 4) + chunks(hidden) * (4 * hidden + inter) + chunks(inter) * hidden +
-            chunks(hidden) * inter / 16 + rows * ((inter + 1023) / 1024)) * 4;
+            chunks(hidden) * inter / 16 + rows * (1 + (inter + 1023) / 1024)) * 4;
   }
   F32SplitScratch(void *at, unsigned long long rows, int hidden, int inter) {
     rows = (rows + 3) / 4 * 4;

@@ -401,7 +401,9 @@ def test_layernorm_f32_split_bounds_rows_whose_squares_are_no_floats(device, siz
 
 def _with_raw(pairs, exps, raw):
     """What pairs stand for where some blocks of 32 are floats."""
-    bits = raw.cpu().numpy().view(np.uint32)
+    words = raw.cpu().numpy().view(np.uint32)
+    bits = words[:, 1:]
+    assert np.array_equal(words[:, 0] != 0, bits.any(1))
     bits = (bits[:, :, None] >> np.arange(32, dtype=np.uint32) & 1).reshape(len(bits), -1)[:, :pairs.shape[1]]
     got = _joined(pairs, exps)
     floats = pairs.cpu().numpy().view(np.float32).reshape(got.shape)
@@ -435,7 +437,7 @@ def test_one_large_column_of_ffn1_leaves_the_others_alone(device, tile, what):
     w1d, w2d, b1d = _dev(w1, device), _dev(w2, device), _dev(b1, device)
     wp, _, bounds = ops.split_f32([w1d, w2d], None, 0, b1d, layer=True)
     mine = _dev(out, device)
-    raw = torch.full((rows, (F + 1023) // 1024), -1, dtype=torch.int32, device=device)
+    raw = torch.full((rows, 1 + (F + 1023) // 1024), -1, dtype=torch.int32, device=device)
     ops.set_option("f32_gemm_tile", tile)
     try:
         pairs, exps, ge = ops.add_bias_residual_layernorm_f32_split(mine, *[_dev(a, device) for a in (res, zero, gamma, zero)],
@@ -460,6 +462,98 @@ def test_one_large_column_of_ffn1_leaves_the_others_alone(device, tile, what):
     bound2 = (4 + math.sqrt(F) / 2) * 2.0 ** -23 * (np.abs(got[:M][:, others]) @ np.abs(w2[others]).astype(np.float64))
     assert np.all(np.abs(got2[:M] - exp2) <= bound2), (np.abs(got2[:M] - exp2) / bound2).max()
     assert np.all(got2[M:] == 7.0)
+
+
+@pytest.mark.parametrize("tile", [0, 1, 2])
+@pytest.mark.parametrize("kind", ["ordinary", "small ones", "feature 1e16", "feature 1e30", "two values", "weight row 1e20",
+                                  "weight 1e25", "both"])
+def test_operands_out_of_proportion_are_summed_from_the_floats(device, tile, kind):
+    """Values that leave their row, or their chunk of a column, no bits, and that meet a zero: the other products are summed
+    as floats.  A few small values among ordinary ones are none of that."""
+    _say("out of proportion", tile, kind)
+    rs = np.random.RandomState(6)
+    rows, M, N, K = 77, 70, 160, 320
+    x, w = rs.standard_normal((90, K)).astype(np.float32), (rs.standard_normal((K, N)) * 0.05).astype(np.float32)
+    bias = rs.standard_normal(N).astype(np.float32)
+    idx = rs.permutation(90)[:rows].astype(np.int32)
+    marked_rows, marked_columns = np.zeros(90, bool), np.zeros((2, N), bool)
+    if kind == "small ones":
+        x[:, ::10] *= np.float32(1e-15)
+        w[::10] *= np.float32(1e-15)
+    if kind.startswith("feature") or kind == "both":
+        at = rs.permutation(90)[:40]
+        x[at, 7] = 1e30 if kind == "both" else float(kind[8:])
+        w[7] = 0
+        marked_rows[at] = True
+    if kind == "two values":
+        x[:20] = 0
+        x[:20, 3], x[:20, 9], w[3] = 1e30, rs.standard_normal(20), 0
+        marked_rows[:20] = True
+    if kind in ("weight row 1e20", "both"):
+        w[5], x[:, 5] = 1e20, 0
+        marked_columns[0] = True
+    if kind == "weight 1e25":
+        w[300, 33], x[:, 300] = -1e25, 0
+        marked_columns[1, 33] = True
+    xd, wd, vr = _dev(x, device), _dev(w, device), torch.tensor([M], dtype=torch.int32, device=device)
+    (wp,), a, _ = ops.split_f32([wd], xd, row_index=_dev(idx, device), valid_rows=vr, rows_cap=rows, layer=True)
+    assert np.array_equal(a[1].cpu().numpy()[:M] >= 2048, marked_rows[idx[:M]])
+    assert np.array_equal(wp[1].cpu().numpy() >= 2048, marked_columns)
+    live = x[idx[:M]].astype(np.float64)
+    exp, size = live @ w.astype(np.float64) + bias, np.abs(live) @ np.abs(w).astype(np.float64) + np.abs(bias)
+    bound = (4 + math.sqrt(K) / 2) * 2.0 ** -23 * size
+    ge = torch.full((rows,), 7, dtype=torch.int32, device=device)
+    more = dict(weight=wd, rows=xd, row_index=_dev(idx, device))
+    ops.set_option("f32_gemm_tile", tile)
+    try:
+        got = ops.gemm_f32_split(a, wp, _dev(bias, device), None, vr, torch.full((rows, N), 7.0, device=device), **more).cpu().numpy()
+        raw = torch.zeros(rows, 2, dtype=torch.int32, device=device)
+        gelu, _ = _with_raw(ops.gemm_f32_split(a, wp, _dev(bias, device), ge, vr, raw=raw, **more), ge, raw)
+    finally:
+        ops.set_option("f32_gemm_tile", -1)
+    assert np.all(np.abs(got[:M] - exp) <= bound), (np.abs(got[:M] - exp) / bound).max()
+    assert np.all(got[M:] == 7.0)
+    # GELU's slope is below 1.13, its float arithmetic good to 2^-20 of the argument
+    assert np.all(np.abs(gelu[:M] - _gelu64(exp)) <= 2 * bound + 2.0 ** -20 * np.abs(exp)), "gelu"
+
+
+@pytest.mark.parametrize("path", ["th_op", "encoder"])
+@pytest.mark.parametrize("rm", [True, False])
+def test_fp32_layers_with_weights_that_nothing_meets(device, path, rm):
+    """A model whose last features are padding: zero wherever they are computed, so that what lies in the rows of the weights
+    that read them, 1e20 here, counts for nothing."""
+    _say("fp32 layers, weights that nothing meets", path, rm)
+    cfg = workload.EncoderConfig("f32pad", 17, 120, 8, layers=2, dtype="fp32", lens=(120, 3, 41, 0, 64, 119) + (90,) * 11)
+    wl = workload.make_workload(cfg, bias_std=0.05, random_affine=True)
+    H, at = cfg.hidden, cfg.hidden - 3
+    wl.x[..., at:] = 0
+    readers = ("qkv_kernel", "attr_output_kernel", "inter_kernel", "output_kernel")
+    for w in wl.layers:
+        w["qkv_kernel"][:, 2 * H + at:], w["qkv_bias"][2 * H + at:] = 0, 0          # V
+        w["inter_kernel"][:, at:H], w["inter_bias"][at:H] = 0, 0
+        for n in ("attr_output", "output"):
+            w[n + "_kernel"][:, at:], w[n + "_bias"][at:] = 0, 0
+            w[n + "_layernorm_gamma"][at:], w[n + "_layernorm_beta"][at:] = 0, 0
+        for n in readers:
+            w[n][at:H] = 0
+    exp = _oracle32(wl)
+    for w in wl.layers:
+        w["qkv_kernel"][at:, :2 * H + at] = 1e20
+        w["attr_output_kernel"][at:, :at] = -1e20
+        w["inter_kernel"][at:, :at], w["inter_kernel"][at:, H:] = 1e20, -1e20
+        w["output_kernel"][at:H, :at] = 1e20
+    x, m = _dev(wl.x, device), _dev(wl.mask, device)
+    if path == "th_op":
+        bt.load_th_op()
+        got = x
+        for w in wl.layers:
+            got = torch.ops.ByteTransformer.BertTransformer(
+                cfg.head_num, cfg.head_size, *[_dev(w[n], device) for n in workload.WEIGHT_NAMES], got, m, rm, True)
+    else:
+        got = bt.BertEncoder(cfg.head_num, cfg.head_size, [{k: _dev(v, device) for k, v in w.items()} for w in wl.layers],
+                             is_remove_padding=rm)(x, m)
+    got = got.cpu().numpy()
+    _f32_check(got if rm else O.masked_output(got, wl.lens), exp, wl.lens, "f32 padding/%s" % path, rm)
 
 
 @pytest.mark.parametrize("path", ["th_op", "encoder"])

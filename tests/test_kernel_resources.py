@@ -80,8 +80,8 @@ def test_the_streaming_attention_brings_few_argument_bytes(code_objects):
 
 # Wait states between a matrix instruction and the first other use of its result, which the hardware does not enforce:
 # passes + 4 on the XDL units (16-bit operands), passes + 2 on the others.
-RESULT_WAIT = {"v_mfma_f32_32x32x2_f32": 16 + 2, "v_mfma_f32_32x32x16_f16": 8 + 4, "v_mfma_f32_32x32x16_bf16": 8 + 4,
-               "v_mfma_f32_16x16x32_f16": 4 + 4}
+RESULT_WAIT = {"v_mfma_f32_32x32x2_f32": 16 + 2, "v_mfma_f32_16x16x4_f32": 8 + 2, "v_mfma_f32_32x32x16_f16": 8 + 4,
+               "v_mfma_f32_32x32x16_bf16": 8 + 4, "v_mfma_f32_16x16x32_f16": 4 + 4}
 
 
 def _registers(operand):
