@@ -99,8 +99,9 @@ class BertEncoder {
     n += align_up((rows * 2 + 2 * (unsigned long long)max_batch_size_ + 2 + 256) * sizeof(int), 256);
     n += align_up(splitk_scratch_bytes(rows, (unsigned long long)head_num_ * size_per_head_), 256);
     n += align_up(attention_layer_->work_list_capacity(), 256);   // the attention's work list
-    if (OpType == OperationType::FP32) {   // split operands: a layer's weights, exponents and bounds
-      const unsigned long long hidden = (unsigned long long)head_num_ * size_per_head_;
+    const unsigned long long hidden = (unsigned long long)head_num_ * size_per_head_;
+    // split operands, where a batch can be large enough for them: a layer's weights, exponents and bounds
+    if (OpType == OperationType::FP32 && f32_splits_operands(rows, !is_remove_padding_, hidden, hidden * intermediate_size_)) {
       n += align_up(layer_weight_elems() * sizeof(float), 256);
       n += align_up(F32SplitScratch::bytes(rows, hidden, hidden * intermediate_size_), 256);
     }

@@ -172,7 +172,10 @@ class BertTransformer {
             sizeof(DataType_),
         256);
     inner_buf_size_ += align_up(splitk_scratch_bytes(rows, hidden), 256);
-    if (OpType == OperationType::FP32)   // split operands: exponents and bounds (the pairs of the weights lie in the copies' place)
+    // split operands, where a batch can be large enough for them: exponents and bounds (the pairs of the weights lie in the
+    // copies' place)
+    if (OpType == OperationType::FP32 &&
+        f32_splits_operands(rows, !is_remove_padding_, hidden, hidden * param_.intermediate_size))
       inner_buf_size_ += align_up(F32SplitScratch::bytes(rows, hidden, hidden * param_.intermediate_size), 256);
     return inner_buf_size_ + attention_layer_->cal_bufsize();
   }

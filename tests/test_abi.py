@@ -217,3 +217,24 @@ def test_layer_plan_is_a_host_side_decision():
     finally:
         assert kl.bt_set_option(b"qkv_mask_rows", -1) == 0
     assert lib.bt_encoder_layer_plan(None, 1, 1, 0, (ctypes.c_int * 6)()) != 0
+
+
+@pytest.mark.parametrize("heads,remove_padding,most", [(12, 1, 2033), (12, 0, 1219), (7, 1, None), (65, 1, None)])
+def test_float_scratch_holds_split_operands_where_a_batch_can_need_them(heads, remove_padding, most):
+    """The scratch of a float encoder: a layer's weights more from the first row count on that splits its operands (`most` is
+    the last that does not; None: hidden sizes that never do), and none before."""
+    lib = bt.host_lib()
+    H = heads * 64
+    weights = 12 * H * H * 4
+
+    def size(rows, entry):
+        cfg = _lib.EncoderConfig(0, rows, 1, heads, 64, 4, 1, remove_padding, 1, 1.0, 1e-6)
+        return getattr(lib, entry)(ctypes.byref(cfg))
+
+    assert size(8, "bt_encoder_forward_bufsize") < weights / 2
+    sizes = [size(rows, "bt_encoder_forward_bufsize") for rows in range(8, 4001)]
+    steps = [8 + i for i, (a, b) in enumerate(zip(sizes, sizes[1:])) if b - a > weights / 2]
+    assert steps == ([most] if most else []), steps
+    if most:
+        grown = size(most + 1, "bt_encoder_bufsize") - size(most, "bt_encoder_bufsize")
+        assert 100000 < grown < 1 << 20, grown                    # exponents and bounds; the pairs have the copies' place
