@@ -1958,6 +1958,57 @@ extern "C" int bt_gemm_splitk_slices(int rows_cap, int all_live, int n, int k, i
                     [&] { return fastest_slices(rows_cap, all_live != 0, n, k, most); });
 }
 
+// For a launch in slices: its tile | its pair << 4 | the pair's ratio << 8.
+static int sliced_tile_or_pair(const GemmArgs &p, int splits) {
+  float us = 0.f;
+  const LikelyRows likely(p);
+  const int named = fastest_sliced(likely, p.N, p.K, splits, &us).id;
+  if (p.rows_hint <= 0) {
+    unsigned ratio = 0;
+    const auto at = [&](int id, int i) {
+      for (const SliceModel &c : kSliceModels)
+        if (c.id == id) return slice_pair_us(c, likely.rows[i], p.N, p.K, splits);
+      return 0.f;
+    };
+    const bool either = p.valid_rows && named != 14 && splits > 1 && cu_count() == kEitherCus;
+    const int pair = either ? fastest_pair(likely, p.N, splits, 3, kPairMargin * us, ratio, at) : 0;
+    return named | pair << 4 | (int)(ratio << 8);
+  }
+  // (the waves of tile 14 add up in an order of their own: not for a row count's sake either)
+  GemmArgs unnamed = p;
+  unnamed.rows_hint = 0;
+  const int without = fastest_sliced(LikelyRows(unnamed), p.N, p.K, splits, &us).id;
+  return (named == 14) != (without == 14) ? without : named;
+}
+
+extern "C" int bt_gemm_tiles(int epilogue, int rows_cap, int n, int k, int weight_kn, int splits, int *tiles) {
+  const char *who = "bt_gemm_tiles";
+  BT_REQUIRE(tiles, BT_ERR_INVALID_ARGUMENT, "%s: null pointer argument", who);
+  BT_REQUIRE(epilogue >= kEpiPlain && epilogue <= kEpiPartial && rows_cap > 0 && n > 0 && k >= kBK && k % kBK == 0,
+             BT_ERR_INVALID_ARGUMENT, "%s: epilogue=%d rows_cap=%d n=%d k=%d", who, epilogue, rows_cap, n, k);
+  const int some = 0;
+  GemmArgs p{};
+  p.valid_rows = &some;   // (not read: it says that the launch finds its rows on the device)
+  p.rows_cap = rows_cap, p.N = n, p.K = k, p.w_kn = weight_kn;
+  int answer;
+  if (epilogue == kEpiPartial) {
+    BT_REQUIRE(splits >= 1 && splits <= 16 && k % (splits * kBK) == 0, BT_ERR_INVALID_ARGUMENT, "%s: splits=%d", who, splits);
+    answer = sliced_tile_or_pair(p, splits);
+  } else {
+    const WaveK few = takes_wave_k(p, epilogue == kEpiPlain);
+    if (few != kWaveKNo) {
+      tiles[0] = 14, tiles[1] = few == kWaveKDevice ? 4 : -1, tiles[2] = 0;
+      return BT_OK;
+    }
+    answer = cu_count() == kEitherCus ? tile_or_pair(p, epilogue) : fastest_tile(p, epilogue);
+  }
+  const int pair = answer >> 4 & 15;
+  tiles[0] = pair ? kTilePairs[pair - 1].first : answer & 15;
+  tiles[1] = pair ? kTilePairs[pair - 1].second : -1;
+  tiles[2] = (int)((unsigned)answer >> 8);
+  return BT_OK;
+}
+
 extern "C" int bt_gemm_splitk(const void *a, const void *wt, void *partials, int splits,
                               const int *valid_rows, int rows_cap, int n, int k, int weight_kn,
                               void *stream) {
@@ -1977,27 +2028,7 @@ extern "C" int bt_gemm_splitk_rows(const void *a, const void *wt, void *partials
              rows_cap,          n,                  k,       0,       rows_hint,  (float *)partials,
              weight_kn};
   hipStream_t st = as_stream(stream);
-  const int answer = remembered({rows_cap, valid_rows != nullptr, rows_hint, n, k, splits}, [&] {
-    float us = 0.f;
-    const LikelyRows likely(p);
-    const int named = fastest_sliced(likely, n, k, splits, &us).id;
-    if (rows_hint <= 0) {
-      unsigned ratio = 0;
-      const auto at = [&](int id, int i) {
-        for (const SliceModel &c : kSliceModels)
-          if (c.id == id) return slice_pair_us(c, likely.rows[i], n, k, splits);
-        return 0.f;
-      };
-      const bool either = valid_rows && named != 14 && splits > 1 && cu_count() == kEitherCus;
-      const int pair = either ? fastest_pair(likely, n, splits, 3, kPairMargin * us, ratio, at) : 0;
-      return named | pair << 4 | (int)(ratio << 8);
-    }
-    // (the waves of tile 14 add up in an order of their own: not for a row count's sake either)
-    GemmArgs unnamed = p;
-    unnamed.rows_hint = 0;
-    const int without = fastest_sliced(LikelyRows(unnamed), n, k, splits, &us).id;
-    return (named == 14) != (without == 14) ? without : named;
-  });
+  const int answer = remembered({rows_cap, valid_rows != nullptr, rows_hint, n, k, splits}, [&] { return sliced_tile_or_pair(p, splits); });
   const unsigned ratio = (unsigned)answer >> 8;
   if ((answer >> 4 & 15) == 1) return launch_gemm_either<Tile9, Tile10, kEpiPartial>(p, st, ratio, splits);
   if ((answer >> 4 & 15) == 2) return launch_gemm_either<Tile10, Tile1, kEpiPartial>(p, st, ratio, splits);

@@ -375,7 +375,14 @@ def add_bias_residual_layernorm_restore(out, residual, bias, gamma, beta, batch_
     return out_padded
 
 
-def gemm_splitk(a, wt, splits, valid_rows=None, out=None, w_kn=False):
+def gemm_tiles(epilogue, rows_cap, n, k, w_kn=False, splits=1):
+    """bt_gemm_tiles: (tile, -1, 0), or two tiles and the ratio by which the device picks."""
+    tiles = (ctypes.c_int * 3)()
+    _check(kernel_lib().bt_gemm_tiles(epilogue, rows_cap, n, k, int(w_kn), splits, tiles))
+    return tuple(tiles)
+
+
+def gemm_splitk(a, wt, splits, valid_rows=None, out=None, w_kn=False, rows_hint=0):
     """fp32 partial sums [splits, rows, N] of a . w over `splits` k ranges."""
     rows, N, K = _gemm_shapes("gemm_splitk", a, wt, w_kn, None)
     if out is not None and out.numel() < splits * rows * N:
@@ -383,8 +390,8 @@ def gemm_splitk(a, wt, splits, valid_rows=None, out=None, w_kn=False):
                          % (out.numel(), splits * rows * N))
     if out is None:
         out = torch.zeros(splits, rows, N, dtype=torch.float32, device=a.device)
-    _check(kernel_lib().bt_gemm_splitk(_ptr(a), _ptr(wt), _ptr(out), int(splits), _ptr(valid_rows),
-                                       rows, N, K, int(w_kn), _stream()))
+    _check(kernel_lib().bt_gemm_splitk_rows(_ptr(a), _ptr(wt), _ptr(out), int(splits), _ptr(valid_rows),
+                                            rows, int(rows_hint), N, K, int(w_kn), _stream()))
     return out
 
 

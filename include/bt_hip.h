@@ -58,7 +58,8 @@ const char *bt_last_error_string(void);
  *   "gemm_table_margin"  4 (default), 0..100: per cent by which a tile's measured time must beat
  *                   that of the cost model's choice before the measured table overrides the
  *                   model (100 = the model alone decides)
- *   "attention_qb"  -1 heuristic | 1 | 2: 16-query blocks per wave in the grouped kernel
+ *   "attention_qb"  -1 heuristic | 1 | 2: 16-query blocks per wave in the grouped kernel; in bt_attention_f32, heads of up to
+ *                   64, 1: 64 queries a workgroup, whose keys two groups of waves share | 2: 128 queries
  *   "attention_key_split"  -1 heuristic | 0 | 1: the 64-query streaming attention with four waves,
  *                   or with eight: two groups of four take alternate 64-key halves of every ring
  *                   slot and are merged at the end
@@ -83,7 +84,8 @@ const char *bt_last_error_string(void);
  *   "prefetch_min_grid"  512 (default): attention launches of fewer workgroups leave the hint to
  *                   workgroups of their own, larger ones to their last quarter; 1 = always the latter
  *   "f32_gemm_tile" -1 heuristic | 0: 64x64 tile | 1: 64x32 | 2: 32x32 (four waves over k each) | 3: 32x32,
- *                   eight waves over k, 64-bit addresses (bt_gemm_f32 only)
+ *                   eight waves over k, 64-bit addresses (bt_gemm_f32); in bt_gemm_f32_split 0: 64x64, two groups of
+ *                   waves over k | 1: 64x128, likewise | 2: 96x128, one group | 3: as -1
  *   "attention_short_limit"  0 (default) .. 512: the host library sends sequences up to this
  *                   length to bt_attention_short when use_fused_attention is set; 0 = always
  *                   the streaming kernel, which measures faster at every length
@@ -444,6 +446,13 @@ int bt_gemm_splitk(const void *a, const void *wt, void *partials, int splits,
 int bt_gemm_splitk_rows(const void *a, const void *wt, void *partials, int splits,
                         const int *valid_rows, int rows_cap, int rows_hint, int n, int k,
                         int weight_kn, void *stream);
+/*
+ * What a launch with valid_rows, and no estimate of them, has for these sizes (a question for tests and benchmarks; epilogue
+ * 0: bt_gemm, 1: bt_gemm_bias_gelu, 2: bt_gemm_qkv_bias_split, 3: bt_gemm_splitk in `splits` slices): tiles[0] its tile
+ * ("gemm_tile" above), or, with tiles[1] >= 0, the first of two.  It runs the second one where, in rounds of 256 workgroups,
+ * second * tiles[2] < first * 256 (tiles 14 and 4: where the live rows do not fit one round).
+ */
+int bt_gemm_tiles(int epilogue, int rows_cap, int n, int k, int weight_kn, int splits, int *tiles);
 /*
  * How many slices (1 = leave k whole, at most `most`) make the pair fastest for a product of these
  * sizes; all_live = every row of rows_cap is live.  0 on a part that the answer was not measured on.

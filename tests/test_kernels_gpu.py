@@ -1446,6 +1446,71 @@ def test_gemm_without_a_row_count_gives_the_bits_of_one_tile(device, kind, n, k,
             assert torch.equal(got, one)
 
 
+TILE_SIZES = {1: (128, 128), 2: (256, 128), 3: (256, 192), 9: (64, 64), 10: (64, 128), 11: (96, 128), 12: (128, 192)}
+TWO_TILES = {(9, 10), (10, 1), (10, 11), (1, 12), (2, 3)}
+
+
+def _takes_the_second(tiles, rows, n, splits):
+    rounds = [-(-(-(-rows // TILE_SIZES[t][0]) * -(-n // TILE_SIZES[t][1]) * splits) // 256) for t in tiles[:2]]
+    return rounds[1] * tiles[2] < rounds[0] * 256
+
+
+def _two_tile_launches(kind, n, k, splits, most):
+    """{pair: (capacity, rows that run the first tile, rows that run the second)} over the capacities up to `most`."""
+    found = {}
+    for cap in range(300, most + 1, 20):
+        tiles = ops.gemm_tiles(("plain", "gelu", "qkv", "partial").index(kind), cap, n, k, splits=splits)
+        if tiles[:2] not in TWO_TILES or tiles[:2] in found:
+            continue
+        rows = {_takes_the_second(tiles, m, n, splits): m for m in range(1, cap + 1, 7)}   # (the largest of either kind)
+        if len(rows) == 2:
+            found[tiles[:2]] = (cap, rows[False], rows[True])
+    return found
+
+
+def test_every_pair_of_tiles_is_taken_and_both_ways(device):
+    """The bits of a launch that has two tiles, on rows for either, against those of the first alone (in slices: of a launch
+    that names its rows), and nothing written past the live rows: over these products every pair comes up."""
+    seen = set()
+    for kind, n, k, splits, most in (("plain", 768, 768, 1, 16384), ("plain", 768, 3072, 1, 16384), ("gelu", 3072, 768, 1, 16384),
+                                     ("qkv", 2304, 768, 1, 16384), ("plain", 640, 1280, 1, 9000), ("partial", 768, 3072, 2, 2400),
+                                     ("partial", 768, 3072, 3, 2400), ("partial", 512, 2048, 4, 1500)):
+        launches = _two_tile_launches(kind, n, k, splits, most)
+        rs = np.random.RandomState(n + k)
+        w = _dev((rs.standard_normal((n, k)) * 0.05).astype(np.float16), device)
+        bias = _dev(rs.standard_normal(n).astype(np.float16), device)
+        for pair, (cap, *some) in launches.items():
+            a = _dev(rs.standard_normal((cap, k)).astype(np.float16), device)
+
+            def run(vr, **kw):
+                if kind == "qkv":
+                    out = torch.full((3, n // 192, cap, 64), 7.0, dtype=torch.float16, device=device)
+                    ops.gemm_qkv_bias_split(a, w, bias, n // 192, valid_rows=vr, out=out)
+                    return out.reshape(-1, cap, 64)
+                if kind == "partial":
+                    return ops.gemm_splitk(a, w, splits, valid_rows=vr, out=torch.full((splits, cap, n), 7.0, device=device), **kw)
+                out = torch.full((cap, n), 7.0, dtype=torch.float16, device=device)
+                ops.gemm(a, w, valid_rows=vr, out=out) if kind == "plain" else ops.gemm_bias_gelu(a, w, bias, valid_rows=vr, out=out)
+                return out[None]
+
+            for M in some:
+                _say("two tiles, both ways", kind, n, k, splits, pair, cap, M)
+                vr = torch.tensor([M], dtype=torch.int32, device=device)
+                got = run(vr)
+                if kind == "partial":
+                    one = run(vr, rows_hint=M)
+                else:
+                    ops.set_option("gemm_tile", pair[0])
+                    try:
+                        one = run(vr)
+                    finally:
+                        ops.set_option("gemm_tile", -1)
+                assert torch.equal(got[:, :M], one[:, :M]) and bool((got[:, M:] == 7).all())
+            seen.add((kind == "partial", pair))
+    _say("pairs", sorted(seen))
+    assert {p for _, p in seen} == TWO_TILES and any(sliced for sliced, _ in seen)
+
+
 @pytest.mark.parametrize("kind", ["short", "grouped", "generic"])
 @pytest.mark.parametrize("min_grid", [512, 1])
 def test_attention_prefetch_of_shared_weights_changes_nothing(device, kind, min_grid):
