@@ -213,7 +213,8 @@ constexpr float kGeluFloor = 1.0f / (1 << 20);   // results below it may go: wha
 // do not give.  Lane (fr, lg): columns 16 i + 4 lg .. + 3 of row fr, as the products of pairs leave them; it brings row fr
 // and columns 16 i + fr, values 4 lg .. 4 lg + 3 of every 16 of k, four loads of a column being one step's operands.
 // Summed 256 values at a time.  It waits for its own loads at every step: a layer of 16 x 256, hidden 768, whose FFN2
-// comes from here takes 584 us in place of 213 (by float multiply-adds, four rows a lane, 1860).
+// comes from here takes 830 us in place of 211, one whose QKV product does 646 in place of 296 (alone, launches included; by
+// float multiply-adds, four rows a lane, 1860 and 2550).
 template <int TN>
 __device__ __forceinline__ void split_sums_of_floats(const half_t *a, const half_t *w, const int *a_exps, const int *w_exps,
                                                      const F32SplitTail &tail, int N, int K, int m, int n_first, int fr, int lg,
@@ -487,38 +488,40 @@ __device__ __forceinline__ void f32_split_tile(BT_F32_SPLIT_FIRST, const F32Spli
     again[j] = 0;
     if (KG > 1 && (j < kFirstRows) != (group == 0)) continue;
     const int m = m0 + wm * WTM + 16 * j + fr;
-    bool wrong = column || split_marked(ea[j]) || holds_floats[j] != 0;
+    float none[2] = {0.f, 0.f};   // (0 . x is NaN where x is not finite)
 #pragma unroll
     for (int i = 0; i < TN; ++i)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) wrong = wrong || !(__builtin_fabsf(sum[i][j][e]) < __builtin_inff());
+      for (int e = 0; e < 4; ++e) none[e & 1] = __builtin_fmaf(sum[i][j][e], 0.f, none[e & 1]);
+    const bool wrong = column || split_marked(ea[j]) || holds_floats[j] != 0 || none[0] + none[1] != 0.f;
     const unsigned long long rows = __builtin_amdgcn_ballot_w64(wrong && m < M);
     again[j] = (unsigned)(rows | rows >> 16 | rows >> 32 | rows >> 48) & 0xffffu;
     any |= again[j];
   }
-  if (any != 0) {
+  if (__builtin_expect(any != 0, 0)) {
     // (What only this needs is read from the arguments here: held in registers from the start, it pushed others of the loop out.)
     typedef const __attribute__((address_space(4))) char *arguments_t;
     arguments_t late = (arguments_t)__builtin_amdgcn_kernarg_segment_ptr() + kF32SplitFirstBytes;
     asm volatile("" : "+s"(late));
     const F32SplitTail rare = *(const __attribute__((address_space(4))) F32SplitTail *)late;
-    // (one copy of the code, two column blocks at a time, in the registers that a loop leaves: whose sums they are is picked
-    // behind it)
+    // (one copy of the code, a column block or two at a time, in the registers that the ring's loop leaves: whose sums they
+    // are is picked behind it)
+    constexpr int CN = TN > 2 ? 2 : 1;
 #pragma unroll 1
-    for (int at = 0; at < TM * (TN / 2); ++at) {
-      const int j = at / (TN / 2), half = at % (TN / 2);
+    for (int at = 0; at < TM * (TN / CN); ++at) {
+      const int j = at / (TN / CN), c = at % (TN / CN);
       unsigned rows = again[0];
 #pragma unroll
       for (int q = 1; q < TM; ++q) rows = q == j ? again[q] : rows;
       if (rows == 0) continue;
-      float4_t formed[2];
-      split_sums_of_floats<2>(a, w, a_exps, w_exps, rare, N, K, min(m0 + wm * WTM + 16 * j + fr, M - 1),
-                              n0 + wn * WTN + 32 * half, fr, lg, formed);
+      float4_t formed[CN];
+      split_sums_of_floats<CN>(a, w, a_exps, w_exps, rare, N, K, min(m0 + wm * WTM + 16 * j + fr, M - 1),
+                               n0 + wn * WTN + 16 * CN * c, fr, lg, formed);
 #pragma unroll
       for (int q = 0; q < TM; ++q)
 #pragma unroll
         for (int i = 0; i < TN; ++i)
-          if (q == j && i / 2 == half && (rows >> fr & 1)) sum[i][q] = formed[i & 1];
+          if (q == j && i / CN == c && (rows >> fr & 1)) sum[i][q] = formed[i % CN];
     }
   }
   if (GELU) __builtin_amdgcn_s_barrier();   // everyone is done with the ring
@@ -548,7 +551,7 @@ __device__ __forceinline__ void f32_split_tile(BT_F32_SPLIT_FIRST, const F32Spli
     if (GELU) {
       // Floats stay where the pairs hold three results from kGeluFloor on no longer, or one where all are small.  Rows
       // whose bound is below 2^9, as ordinary ones are, lose none of those and are through with a comparison.
-      bool raw = false;
+      bool raw = false, some_raw = false;
       if (tail.raw && __builtin_amdgcn_ballot_w64(to_pair * kGeluFloor < kSplitHeldFrom && m < M) != 0) {
         int lost = 0;
         float most = 0.f;
@@ -563,6 +566,7 @@ __device__ __forceinline__ void f32_split_tile(BT_F32_SPLIT_FIRST, const F32Spli
 #pragma unroll
         for (int o = 16; o < 64; o <<= 1) lost += __shfl_xor(lost, o, 64), most = fmaxf(most, __shfl_xor(most, o, 64));
         raw = m < M && (lost >= 3 || (lost > 0 && most < 1.0f / 256));
+        some_raw = __builtin_amdgcn_ballot_w64(raw) != 0;
         const int n_first = n0 + wn * WTN;
         if (raw && lg == 0) {
           unsigned *words = tail.raw + (size_t)m * split_raw_words(N);
@@ -582,12 +586,15 @@ __device__ __forceinline__ void f32_split_tile(BT_F32_SPLIT_FIRST, const F32Spli
           const SplitPair p = split_pair(sum[i][j][e] * to_pair);
           h[e] = p.h, l[e] = p.l;
         }
-        if (raw) {
-          *(float4_t *)((float *)to + at) = sum[i][j];
-        } else {
-          *(half4_t *)(to + at) = h;
-          *(half4_t *)(to + 32 + at) = l;
-        }
+        *(half4_t *)(to + at) = h;
+        *(half4_t *)(to + 32 + at) = l;
+      }
+      if (some_raw) {
+        asm volatile("" ::: "memory");   // (over the pairs, of which all are there before)
+        if (raw)
+#pragma unroll
+          for (int i = 0; i < TN; ++i)
+            *(float4_t *)((float *)(staged + fr * EP + (i >> 1) * 64) + (i & 1) * 16 + 4 * lg) = sum[i][j];
       }
       constexpr int CPR = WTN / 4, RPS = 64 / CPR;   // 16-byte chunks of a row; rows per store instruction
       static_assert(64 % CPR == 0 && 16 % RPS == 0, "whole rows");
@@ -711,8 +718,8 @@ extern "C" int bt_gemm_f32_split_with(const void *a_pairs, const int *a_exps, co
   // Tiles: 0: 64x64, two groups of waves over k, two workgroups a CU | 1: 64x128 likewise, one | 2: 96x128, one group, two.
   // What a step waits for is its operands: a CU takes in about 40 bytes a clock from the L2 and reads 128 from the LDS, and
   // the larger the tile the fewer it needs, as long as no CU goes without.  us at 2458 rows of hidden 768, bt_gemm_f32 and
-  // tiles 0 / 1 / 2: QKV 62 and 43 / 51 / 32, projection 21 and 14.0 / 13.4 / 20.5, FFN1 79 and 59 / 67 / 51, FFN2 73 and 42 /
-  // 48 / 65.  (256x128, eight waves: 38 / 33 / 41 / 103, but 75 for FFN1 from 2561 rows on, a second round, and no
+  // tiles 0 / 1 / 2: QKV 57 and 41 / 46 / 28, projection 21 and 13.1 / 12.6 / 17.4, FFN1 77 and 61 / 69 / 49, FFN2 68 and 40 /
+  // 45 / 62.  (256x128, eight waves: 38 / 33 / 41 / 103, but 75 for FFN1 from 2561 rows on, a second round, and no
   // registers to spare; 128x128, eight waves: 44 / 21 / 46 / 63.)  A launch is priced by its rounds of the chip, a last one
   // that is partly full where two workgroups share a CU at half of one and half of its share: 5 us less than these
   // and those of 600 and 4915 rows, give or take 15 %.  The groups add up in another order, so the choice follows from sizes
