@@ -51,8 +51,9 @@ int hip_fail(hipError_t e, const char *what);
 // A launch through the kernel's function handle, its arguments packed here.  Issuing a launch is what the host
 // does all day (12 layers at 1 x 32 are 84 of them, and take the GPU no longer than the host), and as <<<>>> with
 // a parameter each it looks the symbol up and copies argument by argument: us to issue an empty kernel of one / ten /
-// sixteen arguments 2.9 / 3.2 / 3.6 as <<<>>>, 2.7 / 2.95 / 3.2 so; 68 bytes of arguments 3.8 and 3.5, so no kernel
-// ends a few bytes behind a multiple of 16 beyond 64.
+// sixteen arguments 2.9 / 3.2 / 3.6 as <<<>>>, 2.7 / 2.95 / 3.2 so; 68 bytes of arguments 3.8 and 3.5, so the
+// products and the LayerNorm of half-precision layers end at 64 or a multiple of 16 beyond.  (Others do not, the float
+// LayerNorm's 84 bytes among them: those layers are not bound by the host.)
 // The handle, and the dynamic LDS limit beyond 64 KB, belong to the kernel on one device: they are looked up once
 // for each (a lost race only repeats an idempotent call).
 constexpr int kMaxDevices = 64;
@@ -254,7 +255,7 @@ __device__ __forceinline__ int wave_total(int v) {
 // 2048 / R halfs are one round trip; element by element a 512-token row was eight
 // dependent ones).  Rows may start at any element; the last piece of a row that does not divide lies
 // over the one before it and counts what that one has not (element by element, as those rows were read before, each
-// was up to 16 dependent round trips: 12 layers, operator, 12 x 380 986 -> 945 us, 16 x 250 971 -> 950, 24 x 100 722 -> 708).
+// was up to 16 dependent round trips: 12 layers, operator, 12 x 380 857 -> 820 us, 16 x 250 931 -> 908, 24 x 100 707 -> 694).
 template <typename T, int R>
 __device__ __forceinline__ void wave_row_lengths(const T *const *row, int S, int lane,
                                                  int (&count)[R]) {

@@ -25,9 +25,9 @@ __device__ __forceinline__ int split_exponent(float m) {
 }
 __device__ __forceinline__ float split_power(int e) { return __builtin_bit_cast(float, (unsigned)(e + 127) << 23); }
 
-// What a value v says of its row (or chunk of a column): the pairs hold a row unless a fifth of its values that are not zero
-// lie so far below the largest that they are lost, and the sum of these is positive.  (A few small ones among others
-// lose nothing that shows beside those.)
+// What a value v says of its row (or chunk of a column).  The pairs hold a row, and the sum over it is not positive, unless
+// more than a fifth of its values that are not zero lie so far below the largest that they are lost.  (A few small ones
+// among others lose nothing that shows beside those.)
 __device__ __forceinline__ int split_score(float v, float scale) {
   const float x = v * scale;
   return v == 0.f ? 0 : split_pair(x).held && x != 0.f ? -1 : 4;

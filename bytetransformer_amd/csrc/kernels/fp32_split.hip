@@ -23,7 +23,7 @@
 //
 // The scale of FFN1's results has to be known before them, so it comes from a bound.  One large column makes that bound
 // and with it what 2^-50 is worth to the results of all others, be it 10^12 times as large as any of them.  So where
-// the pairs of a result's row do not hold what they should in some 32 columns, these columns stay floats in the
+// the pairs of a result's row do not hold what they should in the columns of a wave, these stay floats in the
 // place of their pairs (as many bytes), with a bit that says so, and the product that reads that row forms its sums again.
 //
 // In memory a row of K floats is K / 32 blocks of 128 bytes: 32 h, then 32 l.  A block is one k-step's row of an

@@ -478,8 +478,9 @@ int bt_splitk_layernorm(const void *partials, int splits, const void *residual,
  *                      bounds float[2 n / 32 ceil(k / 256)].
  *   bt_gemm_f32_split  c = a . w + bias (bias nullable), float; gelu_exps != NULL: the pairs of GELU(a . w + bias),
  *                      row r scaled by 2^gelu_exps[r]; n a multiple of 32, k of 64.  Distance from float64 (2-norm; largest
- *                      difference over the largest result) for normal operands: k = 768 1.4e-7, 2.5e-7, k = 3072 1.5e-7,
- *                      2.4e-7, where bt_gemm_f32 has 2.1e-7, 3.5e-7 and 4.3e-7, 7.0e-7.
+ *                      difference over the largest result) for normal operands: k = 768 1.19e-7, 1.7e-7 (96x128 tile
+ *                      1.36e-7, 2.1e-7), k = 3072 1.32e-7, 1.6e-7 (1.48e-7, 1.8e-7), where bt_gemm_f32 has 2.1e-7, 3.5e-7 and
+ *                      4.3e-7, 7.4e-7.
  *   bt_gemm_f32_split_with  the same, told more (`more` nullable).  The rows of which a_raw speaks or whose exponent has that
  *                      mark, those with a sum that is not finite, and all where a weight's column has the mark, it forms from
  *                      the floats (float matrix instructions, three to five times as slowly).

@@ -105,10 +105,11 @@ inline int ffn2_slices(int rows_cap, bool all_live, int n, int k, unsigned long 
 
 // Float layers on products of split operands (bt_gemm_f32_split): from how many rows the launches that split the
 // weights, afresh in every layer, cost less than the products gain.  12 layers of hidden 768, split / not, us: 8 x 100
-// (480 rows expected) 1559 / 1319, 8 x 160 (768) 1729 / 1592, 10 x 200 (1200) 2088 / 2050, 16 x 128 (1229) 2046 / 2096,
-// 16 x 256 (2458) 3010 / 3690.  Follows from sizes alone, never from a row hint: both ways are float arithmetic to a
-// few 1e-7, but not the same bits.  From hidden 512 on: there the roundings of a sum outweigh those of the pairs, and the
-// result is the nearer one to float64 (distance, pairs / whole floats: k = 64 9.8e-8 / 5.5e-8, 512 1.17e-07 / 1.71e-07).
+// (480 rows expected) 1512 / 1241, 8 x 160 (768) 1675 / 1336, 10 x 160 (960) 1756 / 1499, 10 x 200 (1200) 1873 / 1904,
+// 16 x 128 (1229) 1881 / 2368, 16 x 256 (2458) 2336 / 3062; measured at this width alone.  Follows from sizes alone, never
+// from a row hint: both ways are float arithmetic to a few 1e-7, but not the same bits.  From hidden 512 on: there the
+// roundings of a sum outweigh those of the pairs, and the result is the nearer one to float64 (distance, pairs / whole
+// floats: k = 64 9.8e-8 / 5.5e-8, 512 1.17e-07 / 1.71e-07).
 inline bool f32_splits_operands(long long rows_cap, bool all_live, long long hidden, long long inter) {
   return hidden % 64 == 0 && inter % 64 == 0 && hidden >= 512 && hidden <= 4096 && inter <= (1 << 14) &&
          (all_live ? rows_cap : rows_cap * 3 / 5) >= 1220;

@@ -416,10 +416,10 @@ def _gelu64(u):
 
 
 @pytest.mark.parametrize("tile", [-1, 0, 1, 2])
-@pytest.mark.parametrize("what", ["ordinary", "bias -1e12", "bias -1e30", "bias 1e12", "bias 1e30", "weight 1e9", "weight 1e20"])
+@pytest.mark.parametrize("what", ["ordinary", "bias -1e12", "bias -1e30", "bias 1e12", "bias 1e30", "weight 1e9", "weight 1e20", "gamma 1e20"])
 def test_one_large_column_of_ffn1_leaves_the_others_alone(device, tile, what):
     """FFN1 and FFN2 as a layer runs them, with one column of FFN1 that is out of all proportion and that FFN2 gives no
-    weight: every other result of FFN1, and every result of FFN2, is what it would be without that column."""
+    weight (or one of the LayerNorm, that FFN1 gives none): every other result of FFN1, and every result of FFN2, is what it would be without that column."""
     _say("one large column", tile, what)
     rs = np.random.RandomState(11)
     M, rows, H, F = 69, 75, 768, 1088
@@ -432,6 +432,8 @@ def test_one_large_column_of_ffn1_leaves_the_others_alone(device, tile, what):
         b1[col] = float(what[5:])
     elif what.startswith("weight"):
         w1[33, col] = float(what[7:])
+    elif what.startswith("gamma"):
+        gamma[9], w1[9] = float(what[6:]), 0
     w2[col] = 0
     vr = torch.tensor([M], dtype=torch.int32, device=device)
     w1d, w2d, b1d = _dev(w1, device), _dev(w2, device), _dev(b1, device)
@@ -442,7 +444,7 @@ def test_one_large_column_of_ffn1_leaves_the_others_alone(device, tile, what):
     try:
         pairs, exps, ge = ops.add_bias_residual_layernorm_f32_split(mine, *[_dev(a, device) for a in (res, zero, gamma, zero)],
                                                                     bounds, 1e-6, vr, raw=raw)
-        mid = ops.gemm_f32_split((pairs, exps), wp[0], b1d, ge, vr, raw=raw, weight=w1d)
+        mid = ops.gemm_f32_split((pairs, exps), wp[0], b1d, ge, vr, raw=raw, weight=w1d, rows=mine)
         got2 = ops.gemm_f32_split((mid, ge), wp[1], None, None, vr, torch.full((rows, H), 7.0, device=device), a_raw=raw,
                                   weight=w2d).cpu().numpy()
     finally:
