@@ -1019,8 +1019,10 @@ __global__ __launch_bounds__((WM * WN + NP) * 64) void gemm_short_kernel(BT_GEMM
 // at the far side of a round's end the other way about.  Where two tiles of one workgroup size are each the better one
 // for some of the likely rows, the launch has both, and takes the one whose rounds cost less.
 // ratio: 256 x the second one's cost of a round over the first one's.
-// 12 layers without a row count, one tile and one of two, us: encoder 12 x 380 925 -> 896, 16 x 1024 2455 -> 2364, 20 x 200
-// 883 -> 846, 6 x 250 580 -> 567, per-layer entry 12 x 380 1064 -> 1020, 16 x 512 1583 -> 1527; where the rows are known nothing
+// 12 layers without a row count, one tile and one of two, us (the rows of one draw of lengths): encoder 12 x 380 874 -> 835,
+// with a bias 895 -> 855, 16 x 1024 2687 -> 2597, 20 x 200 845 -> 822, 6 x 250 515 -> 493, per-layer entry 12 x 380 981 -> 938,
+// 16 x 512 1644 -> 1592; other lengths gain less, none at those of 100 x 120, and FFN2's slices at six heads of 128, 8 x 300,
+// 821 -> 825; where the rows are known nothing
 // changes, and a launch of two is asked to be 2.5 % better on the average of the likely rows (kPairMargin).  Of the
 // pairs whose workgroups go together these five have nearly all there is to gain.  Which is taken changes no bit.
 template <int BM_, int BN_, int STAGES_, int WM_, int WN_, int NP_>
