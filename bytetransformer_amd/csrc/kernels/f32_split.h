@@ -9,14 +9,17 @@ constexpr float kSplitLow = 1.0f / 2048.0f;   // what a pair's second number is 
 
 struct SplitPair {
   half_t h, l;
-  bool held;   // the value to 2^-22 of itself (what is not finite counts as held)
+  float off;   // what the pair leaves out
+  __device__ __forceinline__ bool held(float x) const {   // the value to 2^-22 of itself (what is not finite counts as held)
+    return !(__builtin_fabsf(off) > __builtin_fabsf(x) * 0x1p-22f);
+  }
 };
 // of a scaled value: the second number is zero where the first is not finite
 __device__ __forceinline__ SplitPair split_pair(float x) {
   const half_t h = (half_t)x;
   const float rest = (x - (float)h) * 2048.0f;
   const half_t l = __builtin_fabsf((float)h) < __builtin_inff() ? (half_t)rest : (half_t)0.f;
-  return SplitPair{h, l, !(__builtin_fabsf(rest - (float)l) > __builtin_fabsf(x) * kSplitLow)};
+  return SplitPair{h, l, (rest - (float)l) * kSplitLow};
 }
 // The exponent that brings a largest value m >= 0 to [2^14, 2^15) (0 for no value at all), held where 2^e is a float.
 __device__ __forceinline__ int split_exponent(float m) {
@@ -25,17 +28,22 @@ __device__ __forceinline__ int split_exponent(float m) {
 }
 __device__ __forceinline__ float split_power(int e) { return __builtin_bit_cast(float, (unsigned)(e + 127) << 23); }
 
-// What a value v says of its row (or chunk of a column).  The pairs hold a row, and the sum over it is not positive, unless
-// more than a fifth of its values that are not zero lie so far below the largest that they are lost.  (A few small ones
-// among others lose nothing that shows beside those.)
-__device__ __forceinline__ int split_score(float v, float scale) {
+// What a value v says of its row (or chunk of a column): how far off its pair is, relative to the value and squared, less what
+// it may be.  Where the sum is positive the pairs are off by more than 2^-22.5 of their values in the root mean square - the
+// error of products that all weigh the same, whatever the scales of their operands - and the row is marked.  (Ordinary rows
+// are at 2^-24.6; a value that does this alone lies below 2^-31 of the largest, in one chunk of ten million and one row of
+// five.)
+__device__ __forceinline__ float split_score(float v, float scale) {
   const float x = v * scale;
-  return v == 0.f ? 0 : split_pair(x).held && x != 0.f ? -1 : 4;
+  const SplitPair p = split_pair(x);
+  const float off = p.off * __builtin_amdgcn_rcpf(x);
+  const float mine = x == 0.f ? 1.f : fminf(off * off, 1.f);   // (NaN: 1; only finite values count)
+  return v == 0.f || !(__builtin_fabsf(v) < __builtin_inff()) ? 0.f : mine - 0x1p-45f;
 }
-__device__ __forceinline__ int split_score(float4_t v, float scale) {
-  return split_score(v[0], scale) + split_score(v[1], scale) + split_score(v[2], scale) + split_score(v[3], scale);
+__device__ __forceinline__ float split_score(float4_t v, float scale) {
+  return (split_score(v[0], scale) + split_score(v[1], scale)) + (split_score(v[2], scale) + split_score(v[3], scale));
 }
-// No scaled value from here on is lost (half the spacing of l is 2^-36 of it, and held is 2^-22 of the value).
+// No scaled value from here on is lost (what its pair leaves out is 2^-36 at most, 2^-22 of the value).
 constexpr float kSplitHeldFrom = 1.0f / (1 << 14);
 // An exponent that carries this mark is that of a row whose sums are formed from its floats.
 constexpr int kSplitMark = 1 << 12;

@@ -906,11 +906,11 @@ __device__ __forceinline__ void f32_layernorm_block(
     const float bound = fminf(row_norm * wave_max(w_most) + wave_max(bias_most), 3.402823466e38f);
     bool marked = false;
     if (next.raw && __builtin_amdgcn_ballot_w64(small) != 0) {
-      int score = 0;
+      float score = 0.f;
 #pragma unroll
       for (int i = 0; i < NC; ++i)
         if (lane + i * kWave < chunks) score += split_score(v[i], scale);
-      marked = wave_total(score) > 0;
+      marked = wave_sum(score) > 0.f;
     }
     if (lane == 0) {
       next.exps[r] = e + (marked ? kSplitMark : 0);

@@ -18,8 +18,8 @@
 // Infinities and NaN keep their places in h (the scale comes from the finite values of a row); a row with a sum that is
 // not finite is formed again, from the floats.
 //
-// Rows and chunks of columns of which the pairs hold less, because a few values are out of all proportion to the rest, are
-// marked (split_score), and what they enter is summed from the floats: a zero meets the large value as like as not.
+// Rows and chunks of columns of which the pairs hold less, because some values are out of all proportion to the rest, are
+// marked (split_score), and what they enter is summed from the floats: the large value may meet a zero, the small one a large.
 //
 // The scale of FFN1's results has to be known before them, so it comes from a bound.  One large column makes that bound
 // and with it what 2^-50 is worth to the results of all others, be it 10^12 times as large as any of them.  So where
@@ -75,7 +75,8 @@ __device__ __forceinline__ void split_weight_unit(const SplitArgs &a, int unit) 
   constexpr int kPasses = kSplitChunk / (kSplitThreads / 8);   // 64 rows each
   __shared__ float4_t s_most[kSplitThreads / 64][8];
   __shared__ float s_scale[kSplitCols];
-  __shared__ int s_score[kSplitThreads / 64][8][2];   // two columns each
+  __shared__ float4_t s_score[kSplitThreads / 64][8];
+  __shared__ int s_small[kSplitThreads / 64];
   __shared__ __attribute__((aligned(16))) half_t s_tile[kSplitCols * kSplitPitch];
   int j = 0, first = 0;
 #pragma unroll
@@ -127,7 +128,7 @@ __device__ __forceinline__ void split_weight_unit(const SplitArgs &a, int unit) 
   float scale[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) scale[e] = s_scale[4 * cq + e];
-  int score[2] = {0, 0};   // columns 0 and 1, 2 and 3: 16 bits each, at most 1024
+  bool small = false;
 #pragma unroll
   for (int i = 0; i < kPasses; ++i) {
     half_t *to = s_tile + (64 * i + (r0 & 32)) * 2 + (r0 & 31);
@@ -137,22 +138,38 @@ __device__ __forceinline__ void split_weight_unit(const SplitArgs &a, int unit) 
       const SplitPair p = split_pair(x);
       to[(4 * cq + e) * kSplitPitch] = p.h;
       to[(4 * cq + e) * kSplitPitch + 32] = p.l;
-      score[e >> 1] += split_score(v[i][e], scale[e]) * (e & 1 ? 1 << 16 : 1);
+      small = small || (__builtin_fabsf(x) < kSplitHeldFrom && v[i][e] != 0.f);
     }
   }
-#pragma unroll
-  for (int o = 8; o < 64; o <<= 1)
-#pragma unroll
-    for (int h = 0; h < 2; ++h) score[h] += __shfl_xor(score[h], o, 64);
-  if (lane < 8) s_score[wave][lane][0] = score[0], s_score[wave][lane][1] = score[1];
+  const bool wave_small = a.layer && __builtin_amdgcn_ballot_w64(small) != 0;
+  if (lane == 0) s_small[wave] = wave_small;
   __syncthreads();
-  if (t < kSplitCols) {
-    int both = 0;
+  int any_small = 0;
 #pragma unroll
-    for (int w = 0; w < kSplitThreads / 64; ++w) both += s_score[w][t >> 2][t >> 1 & 1];
-    const int low = (int)(short)(both & 0xffff), mine = t & 1 ? (both - low) >> 16 : low;
-    jb.exps[(size_t)chunk * jb.N + n0 + t] = column_e + (a.layer && mine > 0 ? kSplitMark : 0);
+  for (int w = 0; w < kSplitThreads / 64; ++w) any_small |= s_small[w];
+  bool marked = false;
+  if (__builtin_amdgcn_readfirstlane(any_small)) {   // (of the units of ordinary weights perhaps one)
+    float4_t score = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int k = k0 + r0; k < min(k0 + kSplitChunk, jb.K); k += 64) {   // (read once more: in registers from before, half as many waves fit)
+      const float4_t again = src[(size_t)k * (jb.N / 4)];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) score[e] += split_score(again[e], scale[e]);
+    }
+#pragma unroll
+    for (int o = 8; o < 64; o <<= 1)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) score[e] += __shfl_xor(score[e], o, 64);
+    if (lane < 8) s_score[wave][lane] = score;
+    __syncthreads();
+    if (t < kSplitCols) {
+      float all = 0.f;
+#pragma unroll
+      for (int w = 0; w < kSplitThreads / 64; ++w) all += s_score[w][t >> 2][t & 3];
+      marked = all > 0.f;
+    }
   }
+  if (t < kSplitCols) jb.exps[(size_t)chunk * jb.N + n0 + t] = column_e + (marked ? kSplitMark : 0);
   const int rows = min(kSplitChunk, jb.K - k0), chunks16 = rows / 4;   // 16-byte pieces of a column
   for (int at = t; at < kSplitCols * (kSplitChunk / 4); at += kSplitThreads) {
     const int n = at / (kSplitChunk / 4), c = at % (kSplitChunk / 4);
@@ -182,9 +199,9 @@ __global__ __launch_bounds__(kSplitThreads) void split_f32_kernel(SplitArgs a) {
     small = split_store(a.row_pairs + (size_t)r * 2 * a.hidden, c, src[c] * scale) || small;
   bool marked = false;
   if (a.layer && __builtin_amdgcn_ballot_w64(small) != 0) {
-    int score = 0;
+    float score = 0.f;
     for (int c = lane; c < a.hidden / 4; c += 64) score += split_score(src[c], scale);
-    marked = wave_total(score) > 0;
+    marked = wave_sum(score) > 0.f;
   }
   if (lane == 0) a.row_exps[r] = e + (marked ? kSplitMark : 0);
 }
@@ -212,8 +229,8 @@ constexpr float kGeluFloor = 1.0f / (1 << 20);   // results below it may go: wha
 // Sums of 16 rows and 16 TN columns on float matrix instructions, from the floats where there are any: those that the pairs
 // do not give.  Lane (fr, lg): columns 16 i + 4 lg .. + 3 of row fr, as the products of pairs leave them; it brings row fr
 // and columns 16 i + fr, values 4 lg .. 4 lg + 3 of every 16 of k, four loads of a column being one step's operands.
-// Summed 256 values at a time.  It waits for its own loads at every step: a layer of 16 x 256, hidden 768, whose FFN2
-// comes from here takes 830 us in place of 211, one whose QKV product does 646 in place of 296 (alone, launches included; by
+// Summed 64 values at a time (256: 2.9e-7 from float64 at k = 768, bt_gemm_f32 has 2.1e-7; 64: 1.6e-7).  It waits for its own loads at every step: a layer of 16 x 256, hidden 768, whose FFN2
+// comes from here takes 853 us in place of 211, one whose QKV product does 652 in place of 296 (alone, launches included; by
 // float multiply-adds, four rows a lane, 1860 and 2550).
 template <int TN>
 __device__ __forceinline__ void split_sums_of_floats(const half_t *a, const half_t *w, const int *a_exps, const int *w_exps,
@@ -258,7 +275,7 @@ __device__ __forceinline__ void split_sums_of_floats(const half_t *a, const half
     for (int e = 0; e < 4; ++e)
 #pragma unroll
       for (int i = 0; i < TN; ++i) part[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(y[i][e], x[e], part[i], 0, 0, 0);
-    if ((k0 + 16) % kSplitChunk == 0 || k0 + 16 >= K)
+    if ((k0 + 16) % 64 == 0)
 #pragma unroll
       for (int i = 0; i < TN; ++i) sum[i] += part[i], part[i] = zero4;
   }
@@ -560,7 +577,7 @@ __device__ __forceinline__ void f32_split_tile(BT_F32_SPLIT_FIRST, const F32Spli
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             const float v = n0 + wn * WTN + 16 * i + 4 * lg < N ? sum[i][j][e] : 0.f, scaled = v * to_pair;
-            lost += !split_pair(scaled).held && __builtin_fabsf(v) >= kGeluFloor ? 1 : 0;
+            lost += !split_pair(scaled).held(scaled) && __builtin_fabsf(v) >= kGeluFloor ? 1 : 0;
             most = fmaxf(most, __builtin_fabsf(scaled));
           }
 #pragma unroll

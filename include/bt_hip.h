@@ -486,7 +486,7 @@ int bt_splitk_layernorm(const void *partials, int splits, const void *residual,
  *                      the floats (float matrix instructions, three to five times as slowly).
  *   bt_split_f32_layer  layer = 1: the second of a pair of bounds is what a bias adds to the largest |GELU(. W + bias)|, so
  *                      a large negative one counts for nothing; and 2^12 is added to the exponent of a row, or of 256 values of
- *                      a column, whose pairs hold less than four fifths of its values (that are not zero) to 2^-22 of themselves.
+ *                      a column, whose pairs are off by more than 2^-22.5 of its values in the root mean square.
  *   bt_add_bias_residual_layernorm_f32_split  bt_add_bias_residual_layernorm_f32 that writes the pairs of its rows as
  *                      well, and exponents that keep the pairs of GELU(row . W + b) in range for the W of `bounds`;
  *                      ..._layer clears the rows of `raw` (of bt_f32_split_more; nullable) for a W of n columns, at most 63 * 1024,

@@ -467,11 +467,11 @@ def test_one_large_column_of_ffn1_leaves_the_others_alone(device, tile, what):
 
 
 @pytest.mark.parametrize("tile", [0, 1, 2])
-@pytest.mark.parametrize("kind", ["ordinary", "small ones", "feature 1e16", "feature 1e30", "two values", "weight row 1e20",
+@pytest.mark.parametrize("kind", ["ordinary", "scales", "small ones", "feature 1e16", "feature 1e30", "two values", "weight row 1e20",
                                   "weight 1e25", "both"])
 def test_operands_out_of_proportion_are_summed_from_the_floats(device, tile, kind):
     """Values that leave their row, or their chunk of a column, no bits, and that meet a zero: the other products are summed
-    as floats.  A few small values among ordinary ones are none of that."""
+    as floats.  Scales that differ by a factor of a thousand are none of that."""
     _say("out of proportion", tile, kind)
     rs = np.random.RandomState(6)
     rows, M, N, K = 77, 70, 160, 320
@@ -479,9 +479,13 @@ def test_operands_out_of_proportion_are_summed_from_the_floats(device, tile, kin
     bias = rs.standard_normal(N).astype(np.float32)
     idx = rs.permutation(90)[:rows].astype(np.int32)
     marked_rows, marked_columns = np.zeros(90, bool), np.zeros((2, N), bool)
+    if kind == "scales":
+        by = (2.0 ** rs.uniform(-5, 5, K)).astype(np.float32)
+        x, w = x * by, (w.T / by).T.copy()
     if kind == "small ones":
         x[:, ::10] *= np.float32(1e-15)
-        w[::10] *= np.float32(1e-15)
+        w[::10] *= np.float32(1e15)
+        marked_rows[:], marked_columns[:] = True, True
     if kind.startswith("feature") or kind == "both":
         at = rs.permutation(90)[:40]
         x[at, 7] = 1e30 if kind == "both" else float(kind[8:])
@@ -517,6 +521,32 @@ def test_operands_out_of_proportion_are_summed_from_the_floats(device, tile, kin
     assert np.all(got[M:] == 7.0)
     # GELU's slope is below 1.13, its float arithmetic good to 2^-20 of the argument
     assert np.all(np.abs(gelu[:M] - _gelu64(exp)) <= 2 * bound + 2.0 ** -20 * np.abs(exp)), "gelu"
+
+
+@pytest.mark.parametrize("K", [768, 3072])
+@pytest.mark.parametrize("where", ["rows", "weight", "both"])
+def test_split_operands_of_any_scales_are_as_near_as_whole_floats(device, K, where):
+    """Features whose scales differ by up to 2^76 (16 standard deviations of 2^12), with weights of one scale, the other way
+    about, and inversely, so that every product counts: no further from float64 than the products of whole floats, or than
+    operands off by 2^-22.5 each, from where on they are marked."""
+    rs = np.random.RandomState(K)
+    rows, N = 200, 256
+    for bits in (0, 1, 2, 3, 4, 6, 8, 12):
+        by, by2 = 2.0 ** (bits * rs.standard_normal(K)), 2.0 ** (bits * rs.standard_normal(K))
+        x, w = rs.standard_normal((rows, K)), rs.standard_normal((K, N)) * 0.02
+        if where != "weight":
+            x *= by
+        if where != "rows":
+            w *= (1 / by if where == "both" else by2)[:, None]
+        xd, wd = _dev(x.astype(np.float32), device), _dev(w.astype(np.float32), device)
+        (wp,), a, _ = ops.split_f32([wd], xd, layer=True)
+        ref = xd.double() @ wd.double()
+        far = lambda got: ((got.double() - ref).norm() / ref.norm()).item()   # noqa: E731
+        mine, whole = far(ops.gemm_f32_split(a, wp, weight=wd, rows=xd)), far(ops.gemm_f32(xd, wd))
+        marked = [int((e >= 2048).sum()) for e in (a[1], wp[1])]
+        _say("scales", where, K, bits, "pairs %.2e whole %.2e" % (mine, whole), "marked", marked)
+        assert mine <= max(whole, 2.0 ** -22)
+        assert bits > 2 or not any(marked)
 
 
 @pytest.mark.parametrize("path", ["th_op", "encoder"])
