@@ -151,7 +151,8 @@ __device__ __forceinline__ void split_weight_unit(const SplitArgs &a, int unit) 
   if (__builtin_amdgcn_readfirstlane(any_small)) {   // (of the units of ordinary weights perhaps one)
     float4_t score = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
-    for (int k = k0 + r0; k < min(k0 + kSplitChunk, jb.K); k += 64) {   // (read once more: in registers from before, half as many waves fit)
+    // (read once more: with the values in registers from before, half as many waves fit)
+    for (int k = k0 + r0; k < min(k0 + kSplitChunk, jb.K); k += 64) {
       const float4_t again = src[(size_t)k * (jb.N / 4)];
 #pragma unroll
       for (int e = 0; e < 4; ++e) score[e] += split_score(again[e], scale[e]);
@@ -229,9 +230,10 @@ constexpr float kGeluFloor = 1.0f / (1 << 20);   // results below it may go: wha
 // Sums of 16 rows and 16 TN columns on float matrix instructions, from the floats where there are any: those that the pairs
 // do not give.  Lane (fr, lg): columns 16 i + 4 lg .. + 3 of row fr, as the products of pairs leave them; it brings row fr
 // and columns 16 i + fr, values 4 lg .. 4 lg + 3 of every 16 of k, four loads of a column being one step's operands.
-// Summed 64 values at a time (256: 2.9e-7 from float64 at k = 768, bt_gemm_f32 has 2.1e-7; 64: 1.6e-7).  It waits for its own loads at every step: a layer of 16 x 256, hidden 768, whose FFN2
-// comes from here takes 853 us in place of 211, one whose QKV product does 652 in place of 296 (alone, launches included; by
-// float multiply-adds, four rows a lane, 1860 and 2550).
+// Summed 64 values at a time (256: 2.9e-7 from float64 at k = 768, where bt_gemm_f32 has 2.1e-7; 64: 1.6e-7).  It waits for
+// its own loads at every step: a layer of 16 x 256, hidden 768, whose FFN2 comes from here takes 853 us in place of 211, one
+// whose QKV product does 652 in place of 296 (alone, launches included; by float multiply-adds, four rows a lane, 1860 and
+// 2550).
 template <int TN>
 __device__ __forceinline__ void split_sums_of_floats(const half_t *a, const half_t *w, const int *a_exps, const int *w_exps,
                                                      const F32SplitTail &tail, int N, int K, int m, int n_first, int fr, int lg,
@@ -628,7 +630,8 @@ __device__ __forceinline__ void f32_split_tile(BT_F32_SPLIT_FIRST, const F32Spli
 #endif  // __HIP_DEVICE_COMPILE__
 
 template <int BM, int BN, int WM, int WN, int KG, int STAGES, bool GELU>
-__global__ __launch_bounds__(WM *WN *KG * 64, WM *WN *KG == 8 && BN == 64 ? 4 : 2) void f32_split_gemm_kernel(BT_F32_SPLIT_FIRST, F32SplitTail tail) {
+__global__ __launch_bounds__(WM *WN *KG * 64, WM *WN *KG == 8 && BN == 64 ? 4 : 2)
+void f32_split_gemm_kernel(BT_F32_SPLIT_FIRST, F32SplitTail tail) {
 #if defined(__HIP_DEVICE_COMPILE__)
   f32_split_tile<BM, BN, WM, WN, KG, STAGES, GELU>(a, w, valid_rows, a_exps, w_exps, out, rows_cap, N, K, per_n, tail);
 #endif
@@ -740,7 +743,8 @@ extern "C" int bt_gemm_f32_split_with(const void *a_pairs, const int *a_exps, co
   // registers to spare; 128x128, eight waves: 44 / 21 / 46 / 63.)  A launch is priced by its rounds of the chip, a last one
   // that is partly full where two workgroups share a CU at half of one and half of its share: 5 us less than these
   // and those of 600 and 4915 rows, give or take 15 %.  The groups add up in another order, so the choice follows from sizes
-  // alone, never from a row hint, and where the count is known in some calls only, from the capacity of all (tile_rows); a padded batch counts as 60 % full, give or take a fifth.
+  // alone, never from a row hint, and where the count is known in some calls only, from the capacity of all (tile_rows);
+  // a padded batch counts as 60 % full, give or take a fifth.
   int tile = option_f32_gemm_tile();
   if (tile < 0 || tile > 2) {
     struct Candidate { int bm, bn, per_cu; float step, fixed; };   // of a round: us per 64 of k, and besides
