@@ -308,7 +308,8 @@ __device__ __forceinline__ void f32_split_tile(BT_F32_SPLIT_FIRST, const F32Spli
   }
   const int m0 = tile_m * BM, n0 = tile_n * BN, nk = K / 32 / KG;   // k-steps of a group: group, group + KG, ...
   const size_t pitch = 2 * (size_t)K;   // halfs
-  const rsrc_t rs_a = make_rsrc(a + m0 * pitch, (rows_cap - m0) * pitch * sizeof(half_t));
+  // (dead rows read as zero: the ones of the last tile would come from HBM, where nothing of this call is)
+  const rsrc_t rs_a = make_rsrc(a + m0 * pitch, (M - m0) * pitch * sizeof(half_t));
   const rsrc_t rs_w = make_rsrc(w + n0 * pitch, (N - n0) * pitch * sizeof(half_t));
   int voff[NI];
 #pragma unroll
