@@ -90,6 +90,9 @@ KERNEL_ABI = {
     "bt_gemm_splitk_rows": (c_int, [_P, _P, _P, c_int, _IP, c_int, c_int, c_int, c_int, c_int, _P]),
     "bt_gemm_tiles": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int, POINTER(c_int)]),
     "bt_gemm_splitk_slices": (c_int, [c_int, c_int, c_int, c_int, c_int]),
+    "bt_layernorm_gemm_bias_gelu_pays": (c_int, [c_int, c_int, c_int, c_int, c_int]),
+    "bt_layernorm_gemm_bias_gelu": (c_int, [_P, _P, _IP, _P, _P, _P, _P, _P, _P, _P, _IP, c_int, c_int, c_int, c_int, c_int,
+                                            c_float, _P]),
     "bt_splitk_layernorm": (c_int, [_P, c_int, _P, _IP, _P, _P, _P, c_int, _P, _IP, _IP, c_int,
                                     c_int, c_int, c_int, c_float, _P]),
     "bt_gemm_f32": (c_int, [_P, _IP, _P, _P, _P, c_int, _IP, c_int, c_int, c_int, c_int, _P]),

@@ -22,7 +22,7 @@ INC = os.path.join(ROOT, "include")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 HIPCC = os.path.join(ROCM, "bin", "hipcc")
 
-KERNEL_SOURCES = ["padding.hip", "layernorm.hip", "gemm.hip", "attention.hip",
+KERNEL_SOURCES = ["padding.hip", "layernorm.hip", "layernorm_gelu.hip", "gemm.hip", "attention.hip",
                   "attention_generic.hip", "fp32_path.hip", "fp32_split.hip"]
 HOST_SOURCES = ["attention.cc", "bert_transformer.cc", "bert_encoder.cc", "c_api.cc"]
 HOST_DEVICE_SOURCE = "layer_static_scratch.hip"

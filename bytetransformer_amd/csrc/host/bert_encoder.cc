@@ -88,6 +88,9 @@ void BertEncoder<OpType>::infer(BertEncoderInferParam<DataType_> ip) {
   // few rows, long k: FFN2 as split-k partial sums that the last LayerNorm folds in (the same in every layer)
   const int splits =
       OpType == OperationType::HALF ? ffn2_slices(rows, valid_rows == nullptr, hidden, inter, partials_bytes) : 1;
+  // few rows: the first LayerNorm in FFN1's launch, which reads the projection from where Q was
+  const bool norm_in_ffn1 = OpType == OperationType::HALF && !use_fp32_ &&
+                            bt_layernorm_gemm_bias_gelu_pays(rows, valid_rows == nullptr, inter, hidden, ip.prepacked ? 0 : 1);
   // float: weights split afresh in every layer where the rows are worth it
   const bool f32_split = OpType == OperationType::FP32 && f32_splits_operands(rows, !is_remove_padding_, hidden, inter);
   uint8_t *split_at = base + off + align_up(attention_layer_->work_list_capacity(), 256);
@@ -204,15 +207,22 @@ void BertEncoder<OpType>::infer(BertEncoderInferParam<DataType_> ip) {
     }
     attention_layer_->infer(att);
 
-    check_bt_error(bt_gemm(attr_out_buf, wt_proj, attr_matmul_buf, valid_rows, rows, rows_hint,
+    check_bt_error(bt_gemm(attr_out_buf, wt_proj, norm_in_ffn1 ? qkv_buf : attr_matmul_buf, valid_rows, rows, rows_hint,
                            hidden, hidden, weight_kn, stream));
-    check_bt_error(bt_add_bias_residual_layernorm(
-        attr_matmul_buf, x, gather, w.attr_output_bias, w.attr_output_layernorm_gamma,
-        w.attr_output_layernorm_beta, use_fp32_ ? 1 : 0, valid_rows, rows, hidden, layernorm_eps,
-        stream));
-    check_bt_error(bt_gemm_bias_gelu(attr_matmul_buf, wt_inter, w.inter_bias, inter_matmul_buf,
-                                     valid_rows, rows, rows_hint, inter, hidden, weight_kn,
-                                     stream));
+    if (norm_in_ffn1) {
+      check_bt_error(bt_layernorm_gemm_bias_gelu(
+          qkv_buf, x, gather, w.attr_output_bias, w.attr_output_layernorm_gamma, w.attr_output_layernorm_beta,
+          attr_matmul_buf, wt_inter, w.inter_bias, inter_matmul_buf, valid_rows, rows, valid_rows == nullptr, inter, hidden,
+          weight_kn, layernorm_eps, stream));
+    } else {
+      check_bt_error(bt_add_bias_residual_layernorm(
+          attr_matmul_buf, x, gather, w.attr_output_bias, w.attr_output_layernorm_gamma,
+          w.attr_output_layernorm_beta, use_fp32_ ? 1 : 0, valid_rows, rows, hidden, layernorm_eps,
+          stream));
+      check_bt_error(bt_gemm_bias_gelu(attr_matmul_buf, wt_inter, w.inter_bias, inter_matmul_buf,
+                                       valid_rows, rows, rows_hint, inter, hidden, weight_kn,
+                                       stream));
+    }
 
     if (splits > 1) {
       const bool restore = last && is_remove_padding_;

@@ -364,11 +364,19 @@ void BertTransformer<OpType>::bert_infer(BertTransformerInferParam infer_param) 
   attention_layer_->infer(attention_infer_param);
 
   const int *product_rows = all_live ? nullptr : valid_rows;
+  // few rows: the first LayerNorm in FFN1's launch, which reads the projection from where Q was
+  const bool norm_in_ffn1 = ln_count == 0 && !use_fp32_ && bt_layernorm_gemm_bias_gelu_pays(packed_cap, all_live, inter, hidden, w_kn[2]);
+  DataType_ *proj_out = norm_in_ffn1 ? qkv_buf : attr_matmul_buf;
   check_bt_error(
-      bt_gemm(attr_out_buf, wt_proj, attr_matmul_buf, product_rows, packed_cap, rows_hint, hidden,
+      bt_gemm(attr_out_buf, wt_proj, proj_out, product_rows, packed_cap, rows_hint, hidden,
               hidden, w_kn[1], stream));
 
-  if (ln_count > 0)
+  if (norm_in_ffn1)
+    check_bt_error(bt_layernorm_gemm_bias_gelu(
+        proj_out, from_tensor, gather, param_.attr_output_bias, param_.attr_output_layernorm_gamma,
+        param_.attr_output_layernorm_beta, attr_matmul_buf, wt_inter, param_.inter_bias, inter_matmul_buf, valid_rows,
+        packed_cap, all_live, inter, hidden, w_kn[2], layernorm_eps, stream));
+  else if (ln_count > 0)
     check_bt_error(bt_add_bias_residual_layernorm_copy(
         attr_matmul_buf, from_tensor, gather, param_.attr_output_bias,
         param_.attr_output_layernorm_gamma, param_.attr_output_layernorm_beta, use_fp32_ ? 1 : 0,
@@ -379,9 +387,10 @@ void BertTransformer<OpType>::bert_infer(BertTransformerInferParam infer_param) 
         param_.attr_output_layernorm_gamma, param_.attr_output_layernorm_beta, use_fp32_ ? 1 : 0,
         valid_rows, packed_cap, hidden, layernorm_eps, stream));
 
-  check_bt_error(bt_gemm_bias_gelu(attr_matmul_buf, wt_inter, param_.inter_bias, inter_matmul_buf,
-                                   product_rows, packed_cap, rows_hint, inter, hidden, w_kn[2],
-                                   stream));
+  if (!norm_in_ffn1)
+    check_bt_error(bt_gemm_bias_gelu(attr_matmul_buf, wt_inter, param_.inter_bias, inter_matmul_buf,
+                                     product_rows, packed_cap, rows_hint, inter, hidden, w_kn[2],
+                                     stream));
 
   if (splits > 1) {
     check_bt_error(bt_gemm_splitk_rows(inter_matmul_buf, wt_out, partials, splits, product_rows, packed_cap,

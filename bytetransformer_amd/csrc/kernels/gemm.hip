@@ -232,15 +232,6 @@ __device__ __forceinline__ void mask_rows_write(const GemmArgs &p, const MaskRow
   }
 }
 
-__device__ __forceinline__ float gelu_tanh_f32(float x) {
-  // 0.5 x (1 + tanh(u)) == x / (1 + exp(-2u)),  u = 0.79788456 (x + 0.044715 x^3)
-  // exponent folded into one polynomial: -2 u log2(e) = x (c1 + c3 x^2)
-  constexpr float c1 = -2.0f * 0.7978845608028654f * 1.4426950408889634f;
-  constexpr float c3 = c1 * 0.044715f;
-  const float e = __builtin_amdgcn_exp2f(x * (c1 + c3 * x * x));
-  return x * __builtin_amdgcn_rcpf(1.0f + e);
-}
-
 // gemm_wave_k: columns of a tile, waves of a workgroup, k-steps in a wave's ring
 constexpr int kWaveKCols = 32, kWaveKWaves = 4, kWaveKDepth = 3;
 

@@ -12,6 +12,15 @@ constexpr int kSchedMfma = 0x008, kSchedLdsRead = 0x100;   // instruction classe
 // slots.  The 16 lanes that one ds_read_b128 pass serves then touch every bank once.
 __device__ __forceinline__ int swz(int row) { return (row >> 1) & 7; }
 
+__device__ __forceinline__ float gelu_tanh_f32(float x) {
+  // 0.5 x (1 + tanh(u)) == x / (1 + exp(-2u)),  u = 0.79788456 (x + 0.044715 x^3)
+  // exponent folded into one polynomial: -2 u log2(e) = x (c1 + c3 x^2)
+  constexpr float c1 = -2.0f * 0.7978845608028654f * 1.4426950408889634f;
+  constexpr float c3 = c1 * 0.044715f;
+  const float e = __builtin_amdgcn_exp2f(x * (c1 + c3 * x * x));
+  return x * __builtin_amdgcn_rcpf(1.0f + e);
+}
+
 template <int N>
 __device__ __forceinline__ void wait_vmcnt() {
   // s_waitcnt immediate on gfx9: vmcnt[3:0], expcnt[6:4], lgkmcnt[11:8], vmcnt[5:4] in [15:14]

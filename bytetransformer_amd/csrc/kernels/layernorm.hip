@@ -6,25 +6,11 @@
 // Numerics follow bytetransformer/include/layernorm.h:114-159,273-296,334-373:
 // x = (out + residual) + bias with both adds rounded to fp16, mean and biased
 // variance in fp32 (two-pass), y = (x - mean) * rsqrt(var + eps) * gamma + beta.
-#include "common.h"
+#include "layernorm_row.h"
 
 namespace bt {
 
 constexpr int kLnRowsPerBlock = 4;   // 2, 8 and 16 rows per workgroup measured 0-20 % slower
-
-// V consecutive halfs of a row: what a lane loads, adds and stores at a time.
-template <int V>
-struct LnVec;
-template <>
-struct LnVec<8> {
-  typedef half8_t halfs;
-  typedef uint4_t bits;
-};
-template <>
-struct LnVec<4> {
-  typedef half4_t halfs;
-  typedef uint2_t bits;
-};
 
 // Statistics and store of one row held in registers (x = (a + r) + bias, two fp16-rounded adds).
 template <int NC, int V, bool GB32, bool kAffineEarly, int NG, typename H = typename LnVec<V>::halfs>
@@ -33,29 +19,8 @@ __device__ __forceinline__ void ln_finish(const H (&av)[NC], const H (&rv)[NC], 
                                           const float4_t (&g32)[NG][V / 4], const float4_t (&b32)[NG][V / 4],
                                           const void *gamma, const void *beta, const int (&cc)[NC],
                                           const bool (&live)[NC], half_t *o, float inv_n, float eps) {
-  // (four sums side by side: a quarter of the chain)
   float v[NC][V];
-  float part[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int i = 0; i < NC; ++i) {
-    const H x = (av[i] + rv[i]) + bias_v[i];  // two fp16-rounded adds
-#pragma unroll
-    for (int j = 0; j < V; ++j) {
-      v[i][j] = live[i] ? (float)x[j] : 0.f;
-      part[j & 3] += v[i][j];
-    }
-  }
-  const float mean = wave_sum((part[0] + part[1]) + (part[2] + part[3])) * inv_n;
-  float sq[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int i = 0; i < NC; ++i) {
-#pragma unroll
-    for (int j = 0; j < V; ++j) {
-      v[i][j] = live[i] ? v[i][j] - mean : 0.f;
-      sq[j & 3] += v[i][j] * v[i][j];
-    }
-  }
-  const float rstd = rsqrtf(wave_sum((sq[0] + sq[1]) + (sq[2] + sq[3])) * inv_n + eps);
+  const float rstd = ln_statistics<NC, V>(av, rv, bias_v, live, inv_n, eps, v);
 
 #pragma unroll
   for (int i = 0; i < NC; ++i) {

@@ -395,6 +395,25 @@ def gemm_splitk(a, wt, splits, valid_rows=None, out=None, w_kn=False, rows_hint=
     return out
 
 
+def layernorm_gemm_bias_gelu_pays(rows_cap, all_live, n, k, w_kn=False):
+    """Whether a layer of these sizes has its first LayerNorm in FFN1's launch."""
+    return bool(kernel_lib().bt_layernorm_gemm_bias_gelu_pays(rows_cap, int(all_live), n, k, int(w_kn)))
+
+
+def layernorm_gemm_bias_gelu(src, residual, bias, gamma, beta, w, ffn_bias, eps=1e-6, valid_rows=None,
+                             residual_row_index=None, all_live=True, w_kn=False, dst=None, out=None):
+    """(LayerNorm(src + residual + bias), gelu(that . w + ffn_bias)) of a few dozen rows in one launch."""
+    rows, N, K = _gemm_shapes("layernorm_gemm_bias_gelu", src, w, w_kn, None)
+    dst = torch.empty_like(src) if dst is None else dst
+    out = torch.empty(rows, N, dtype=src.dtype, device=src.device) if out is None else out
+    if dst.numel() < rows * K or out.numel() < rows * N or ffn_bias.numel() != N or min(residual.shape[-1], bias.numel(), gamma.numel(), beta.numel()) < K:
+        raise ValueError("layernorm_gemm_bias_gelu: a tensor is smaller than what the launch reads or writes")
+    _check(kernel_lib().bt_layernorm_gemm_bias_gelu(
+        _ptr(src), _ptr(residual), _ptr(residual_row_index), _ptr(bias), _ptr(gamma), _ptr(beta), _ptr(dst), _ptr(w),
+        _ptr(ffn_bias), _ptr(out), _ptr(valid_rows), rows, int(all_live), N, K, int(w_kn), float(eps), _stream()))
+    return dst, out
+
+
 def splitk_layernorm(partials, residual, bias, gamma, beta, dst, eps=1e-6, valid_rows=None,
                      residual_row_index=None, batch_idx=None, batch_size=0, seq_len=1):
     splits, rows, H = partials.shape

@@ -466,6 +466,19 @@ int bt_splitk_layernorm(const void *partials, int splits, const void *residual,
                         int hidden_dim, float eps, void *stream);
 
 /*
+ * bt_add_bias_residual_layernorm and bt_gemm_bias_gelu in one launch, for a few dozen fp16 rows (no counterpart in the
+ * reference): dst = LayerNorm(src + residual + bias), out[rows_cap, n] = gelu(dst . w + ffn_bias).  gamma and beta are
+ * halfs; dst may be neither src nor residual.  all_live: every row of rows_cap is expected to be live, else 60 % of them;
+ * like rows_cap it decides the tile, never what is computed.
+ * bt_layernorm_gemm_bias_gelu_pays: whether there is such a launch for these sizes and it is the faster way (0 without a GPU).
+ */
+int bt_layernorm_gemm_bias_gelu_pays(int rows_cap, int all_live, int n, int k, int weight_kn);
+int bt_layernorm_gemm_bias_gelu(const void *src, const void *residual, const int *residual_row_index,
+                                const void *bias, const void *gamma, const void *beta, void *dst, const void *w,
+                                const void *ffn_bias, void *out, const int *valid_rows, int rows_cap, int all_live,
+                                int n, int hidden_dim, int weight_kn, float eps, void *stream);
+
+/*
  * Float operands as pairs of fp16 numbers, made once by the launch that has them in hand, for products on fp16 matrix
  * instructions (no counterpart in the reference).  A row of K floats (of a weight's column, 256 at a time) is scaled by
  * 2^e, which brings its largest finite value to [2^14, 2^15), and stored as K / 32 blocks of 128 bytes: 32 h, then 32 l,

@@ -65,6 +65,11 @@ int bt_gemm_bias_gelu(const void *, const void *, const void *, void *, const in
   live_by_size += live == nullptr;
   return 0;
 }
+int bt_layernorm_gemm_bias_gelu(const void *, const void *, const int *, const void *, const void *, const void *, void *,
+                                const void *, const void *, void *, const int *, int, int all_live, int, int, int, float, void *) {
+  live_by_size += all_live;
+  return 0;
+}
 int bt_gemm_splitk_rows(const void *a, const void *, void *, int splits, const int *live, int rows, int, int, int k, int, void *) {
   slices = splits;
   take(a, 2ull * rows * k);
