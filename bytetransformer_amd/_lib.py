@@ -31,7 +31,8 @@ _IP = c_void_p  # int* device pointers travel as raw addresses
 # name -> (restype, argtypes); mirrors include/bt_hip.h declaration by declaration
 class F32SplitMore(ctypes.Structure):
     """bt_f32_split_more"""
-    _fields_ = [("tile_rows", c_int), ("raw", _P), ("a_raw", _P), ("w", _P), ("a", _P), ("a_row_index", _P)]
+    _fields_ = [("tile_rows", c_int), ("raw", _P), ("a_raw", _P), ("w", _P), ("a", _P), ("a_row_index", _P),
+                ("rows_hint", c_int)]
 
 
 KERNEL_ABI = {

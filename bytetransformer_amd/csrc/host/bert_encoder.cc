@@ -117,7 +117,7 @@ void BertEncoder<OpType>::infer(BertEncoderInferParam<DataType_> ip) {
         const int ks[4] = {hidden, hidden, hidden, inter}, ns[4] = {3 * hidden, hidden, inter, hidden};
         check_bt_error(bt_split_f32_layer(4, ws, w_pairs, sp.w_exps, ks, ns, 2, w.inter_bias, sp.bounds, x, inter_matmul_buf,
                                           sp.x_exps, gather, valid_rows, rows, hidden, 1, stream));
-        const bt_f32_split_more qkv{0, nullptr, nullptr, w.attr_kernel_QKV, x, gather};
+        const bt_f32_split_more qkv{0, nullptr, nullptr, w.attr_kernel_QKV, x, gather, ip.valid_rows_hint};
         check_bt_error(bt_gemm_f32_split_with(inter_matmul_buf, sp.x_exps, w_pairs[0], sp.w_exps[0],
                                               w.attention_param.attr_bias_QKV, qkv_buf, nullptr, valid_rows, rows, 3 * hidden,
                                               hidden, &qkv, stream));
@@ -135,9 +135,9 @@ void BertEncoder<OpType>::infer(BertEncoderInferParam<DataType_> ip) {
       if (f32_split) {
         // (Q, K, V are dead: the attention's pairs take the first tensor's place, the LayerNorm's the second's)
         DataType_ *att_pairs = qkv_buf, *ln_pairs = qkv_buf + tensor;
-        const bt_f32_split_more proj{0, nullptr, nullptr, w.attr_output_kernel, attr_out_buf, nullptr},
-            ffn1{0, sp.raw, nullptr, w.inter_kernel, attr_matmul_buf, nullptr},
-            ffn2{0, nullptr, sp.raw, w.output_kernel, nullptr, nullptr};
+        const bt_f32_split_more proj{0, nullptr, nullptr, w.attr_output_kernel, attr_out_buf, nullptr, ip.valid_rows_hint},
+            ffn1{0, sp.raw, nullptr, w.inter_kernel, attr_matmul_buf, nullptr, ip.valid_rows_hint},
+            ffn2{0, nullptr, sp.raw, w.output_kernel, nullptr, nullptr, ip.valid_rows_hint};
         check_bt_error(bt_split_f32_layer(0, nullptr, nullptr, nullptr, nullptr, nullptr, -1, nullptr, nullptr, attr_out_buf,
                                           att_pairs, sp.att_exps, nullptr, valid_rows, rows, hidden, 1, stream));
         check_bt_error(bt_gemm_f32_split_with(att_pairs, sp.att_exps, w_pairs[1], sp.w_exps[1], nullptr, attr_matmul_buf, nullptr,

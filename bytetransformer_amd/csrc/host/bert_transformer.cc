@@ -202,6 +202,7 @@ void BertTransformer<OpType>::bert_infer(BertTransformerInferParam infer_param) 
   const int *valid_rows = nullptr;
   const int *gather = nullptr;
   DataType_ *restore_target = nullptr;
+  int known_rows = 0;   // of packed rows, 0: the host does not know
   // Row capacity of the launches over packed rows that follow the attention.  A caller
   // that passes offsets of its own vouches for their exact live count, so these launches
   // are then sized for it instead of batch * seq_len: no workgroups
@@ -227,6 +228,7 @@ void BertTransformer<OpType>::bert_infer(BertTransformerInferParam infer_param) 
       packed_cap = rows_hint;
       all_live = true;
     }
+    known_rows = rows_hint;
     rows_hint = rows_to_plan_for(rows_hint, true, batch_size, rows);
   }
 
@@ -242,7 +244,7 @@ void BertTransformer<OpType>::bert_infer(BertTransformerInferParam infer_param) 
       for (int i = 0; i < 4; ++i) w_pairs[i] = slot, slot += (size_t)w_k[i] * w_n[i] * sizeof(float);
     }
     if (split) {
-      const bt_f32_split_more more{0, nullptr, nullptr, w_use[0], from_tensor, gather};
+      const bt_f32_split_more more{0, nullptr, nullptr, w_use[0], from_tensor, gather, known_rows};
       const void *w[4] = {w_use[0], w_use[1], w_use[2], w_use[3]};
       check_bt_error(bt_split_f32_layer(4, w, w_pairs, sp.w_exps, w_k, w_n, 2, param_.inter_bias, sp.bounds, from_tensor,
                                         inter_matmul_buf, sp.x_exps, gather, valid_rows, rows, hidden, 1, stream));
@@ -269,8 +271,9 @@ void BertTransformer<OpType>::bert_infer(BertTransformerInferParam infer_param) 
       // (Q, K, V are dead: the attention's pairs take the first tensor's place, the LayerNorm's the second's)
       DataType_ *att_pairs = qkv_buf, *ln_pairs = qkv_buf + tensor;
       // (the tiles of the padded batch, also where the caller's offsets bring the count: the same bits with and without them)
-      const bt_f32_split_more proj{rows, nullptr, nullptr, w_use[1], attr_out_buf, nullptr},
-          ffn1{rows, sp.raw, nullptr, w_use[2], attr_matmul_buf, nullptr}, ffn2{rows, nullptr, sp.raw, w_use[3], nullptr, nullptr};
+      const bt_f32_split_more proj{rows, nullptr, nullptr, w_use[1], attr_out_buf, nullptr, known_rows},
+          ffn1{rows, sp.raw, nullptr, w_use[2], attr_matmul_buf, nullptr, known_rows},
+          ffn2{rows, nullptr, sp.raw, w_use[3], nullptr, nullptr, known_rows};
       check_bt_error(bt_split_f32_layer(0, nullptr, nullptr, nullptr, nullptr, nullptr, -1, nullptr, nullptr, attr_out_buf,
                                         att_pairs, sp.att_exps, nullptr, valid_rows, packed_cap, hidden, 1, stream));
       check_bt_error(bt_gemm_f32_split_with(att_pairs, sp.att_exps, w_pairs[1], sp.w_exps[1], nullptr, attr_matmul_buf, nullptr,

@@ -314,8 +314,9 @@ __device__ __forceinline__ void f32_split_tile(BT_F32_SPLIT_FIRST, const F32Spli
   int voff[NI];
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
-    const int r = (i * NG + wave) * 8 + (lane >> 3);
-    voff[i] = ((i < NIA ? r : r - BM) * 2 * K + (((lane & 7) ^ swz(r)) << 3)) * (int)sizeof(half_t);
+    // (BM rows further on the swizzle is the same, and so the offsets of the two operands)
+    const int r = ((i < NIA ? i : i - NIA) * NG + wave) * 8 + (lane >> 3);
+    voff[i] = (r * 2 * K + (((lane & 7) ^ swz(r)) << 3)) * (int)sizeof(half_t);
   }
   auto issue = [&](int kt, int stage) {
 #pragma unroll
@@ -338,20 +339,22 @@ __device__ __forceinline__ void f32_split_tile(BT_F32_SPLIT_FIRST, const F32Spli
   for (int i = 0; i < TN; ++i)
 #pragma unroll
     for (int j = 0; j < TM; ++j) sum[i][j] = hh[i][j] = cross[i][j] = zero4;
-  // (of row fr of block j: on their way beside the first k-steps, looked at behind the last)
-  int ea[TM];
-  unsigned holds_floats[TM];
-#pragma unroll
-  for (int j = 0; j < TM; ++j) {
-    const size_t m = min(m0 + wm * WTM + 16 * j + fr, M - 1);
-    ea[j] = a_exps[m], holds_floats[j] = tail.a_raw ? tail.a_raw[m * split_raw_words(K)] : 0;
-  }
   // The weight's scales: behind the ring, factor[c][n] = 2^(e - exponent of chunk c of column n), e[n] the smallest of the
   // column's, so that no factor is above 1.  (They are on their way beside the first k-steps.)
   const int chunks = (K + kSplitChunk - 1) / kSplitChunk;
   float *factor = (float *)(split_smem + STAGES * STAGE_HALFS);
   int *column_e = (int *)factor + chunks * BN;
-  for (int n = threadIdx.x; n < BN; n += NW * 64) {
+  // ... the columns' bias, the rows' exponents and whether they hold floats: looked at behind the last k-step (in registers
+  // from before it on, the 256 x 128 tile spilled)
+  int *row_e = column_e + BN;
+  float *column_bias = (float *)(row_e + 2 * BM);
+  static_assert(BM <= NW * 64 && BN <= NW * 64, "a thread each");
+  int e_of_row = 0, raw_of_row = 0;
+  if ((int)threadIdx.x < BM) {
+    const size_t m = min(m0 + (int)threadIdx.x, M - 1);
+    e_of_row = a_exps[m], raw_of_row = tail.a_raw ? (int)tail.a_raw[m * split_raw_words(K)] : 0;
+  }
+  if (const int n = threadIdx.x; n < BN) {
     const int *from = w_exps + min(n0 + n, N - 1);
     int least = 1 << 20, mark = 0;
     for (int c = 0; c < chunks; ++c) {
@@ -362,7 +365,9 @@ __device__ __forceinline__ void f32_split_tile(BT_F32_SPLIT_FIRST, const F32Spli
     }
     for (int c = 0; c < chunks; ++c) factor[c * BN + n] = __builtin_amdgcn_ldexpf(1.f, least - ((int *)factor)[c * BN + n]);
     column_e[n] = least + mark;
+    column_bias[n] = tail.bias ? tail.bias[min(n0 + n, N - 1)] : 0.f;
   }
+  if ((int)threadIdx.x < BM) row_e[threadIdx.x] = e_of_row, row_e[BM + threadIdx.x] = raw_of_row;
   __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): there, behind the first barrier of the loop
   constexpr int kFold = kSplitChunk / 32 / KG;   // k-steps of a group in a chunk
   const float *my_factor = factor + wn * WTN + 4 * lg;
@@ -462,7 +467,7 @@ __device__ __forceinline__ void f32_split_tile(BT_F32_SPLIT_FIRST, const F32Spli
   constexpr int kFirstRows = KG > 1 ? (TM + 1) / 2 : TM;   // row blocks of group 0
   static_assert(KG <= 2, "two groups at most");
   if (KG > 1) {
-    static_assert((size_t)NG * TN * TM * 256 * sizeof(float) <= (size_t)STAGES * STAGE_HALFS * sizeof(half_t), "sums fit the ring");
+    static_assert(KG == 1 || (size_t)NG * TN * TM * 256 * sizeof(float) <= (size_t)STAGES * STAGE_HALFS * sizeof(half_t), "sums fit the ring");
     float4_t *shared = (float4_t *)split_smem + wave * (TN * TM * 64) + lane;
     __builtin_amdgcn_s_barrier();   // everyone is done with the ring
 #pragma unroll
@@ -479,22 +484,19 @@ __device__ __forceinline__ void f32_split_tile(BT_F32_SPLIT_FIRST, const F32Spli
   }
 
   // lane: columns n .. n + 3 of block i, row m of block j
-  int4_t ew[TN];
-  float4_t bias[TN];
+  int ea[TM];
+  unsigned holds_floats[TM];
+#pragma unroll
+  for (int j = 0; j < TM; ++j) {
+    const int r = wm * WTM + 16 * j + fr;
+    ea[j] = row_e[r], holds_floats[j] = (unsigned)row_e[BM + r];
+  }
   bool column = false;   // one of the wave's columns is marked
 #pragma unroll
   for (int i = 0; i < TN; ++i) {
-    const int n = min(n0 + wn * WTN + 16 * i + 4 * lg, N - 4);
-    ew[i] = *(const int4_t *)(column_e + wn * WTN + 16 * i + 4 * lg);
+    const int4_t marks = *(const int4_t *)(column_e + wn * WTN + 16 * i + 4 * lg);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      column = column || (split_marked(ew[i][e]) && n0 + wn * WTN + 16 * i + 4 * lg < N);
-      ew[i][e] = split_unmarked(ew[i][e]);
-    }
-    bias[i] = float4_t{0.f, 0.f, 0.f, 0.f};
-    if (tail.bias)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) bias[i][e] = tail.bias[n + e];
+    for (int e = 0; e < 4; ++e) column = column || (split_marked(marks[e]) && n0 + wn * WTN + 16 * i + 4 * lg < N);
   }
   constexpr int EP = 2 * WTN + 8;   // halfs of a staged row of pairs
   static_assert(!GELU || (size_t)NW * 16 * EP <= (size_t)STAGES * STAGE_HALFS, "staging fits the ring");
@@ -543,6 +545,16 @@ __device__ __forceinline__ void f32_split_tile(BT_F32_SPLIT_FIRST, const F32Spli
         for (int i = 0; i < TN; ++i)
           if (q == j && i / CN == c && (rows >> fr & 1)) sum[i][q] = formed[i % CN];
     }
+  }
+  asm volatile("" ::: "memory");   // (read once more: kept from before, sixteen registers that the sums of floats want)
+  int4_t ew[TN];
+  float4_t bias[TN];
+#pragma unroll
+  for (int i = 0; i < TN; ++i) {
+    bias[i] = *(const float4_t *)(column_bias + wn * WTN + 16 * i + 4 * lg);
+    ew[i] = *(const int4_t *)(column_e + wn * WTN + 16 * i + 4 * lg);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) ew[i][e] = split_unmarked(ew[i][e]);
   }
   if (GELU) __builtin_amdgcn_s_barrier();   // everyone is done with the ring
 #pragma unroll
@@ -647,7 +659,7 @@ struct F32SplitArgs {
 };
 template <int BM, int BN, int KG, int STAGES>
 size_t f32_split_lds(int k) {
-  return (size_t)KG * STAGES * (BM + BN) * kBK * sizeof(half_t) + (size_t)((k + kSplitChunk - 1) / kSplitChunk + 1) * BN * 4;
+  return (size_t)KG * STAGES * (BM + BN) * kBK * sizeof(half_t) + (size_t)((k + kSplitChunk - 1) / kSplitChunk + 2) * BN * 4 + 2 * BM * 4;
 }
 template <int BM, int BN, int WM, int WN, int KG, int STAGES>
 int launch_f32_split(const F32SplitArgs &p, hipStream_t s) {
@@ -766,5 +778,11 @@ extern "C" int bt_gemm_f32_split_with(const void *a_pairs, const int *a_exps, co
   }
   if (tile == 0) return launch_f32_split<64, 64, 2, 2, 2, 2>(p, s);
   if (tile == 1) return launch_f32_split<64, 128, 2, 2, 2, 2>(p, s);
+  // 256x128 with eight waves, a workgroup a CU, gives the bits of 96x128 (the same order of a sum, the same columns a wave),
+  // so what the caller knows of the live rows may decide: where one round of it takes the place of more than one of those.
+  const long long known = valid_rows ? m.rows_hint : rows_cap, tiles_n = (n + 127) / 128;
+  if (known > 0 && (known + 255) / 256 * tiles_n <= cu_count() && (known + 95) / 96 * tiles_n > 2 * cu_count() &&
+      option_f32_gemm_tile() < 0)
+    return launch_f32_split<256, 128, 4, 2, 1, 2>(p, s);
   return launch_f32_split<96, 128, 2, 2, 1, 2>(p, s);
 }

@@ -470,7 +470,7 @@ def split_f32(ws, rows=None, bounded=-1, bounded_bias=None, row_index=None, vali
 
 
 def gemm_f32_split(a, w, bias=None, gelu_exps=None, valid_rows=None, out=None, raw=None, a_raw=None, weight=None, rows=None,
-                   row_index=None, tile_rows=0):
+                   row_index=None, tile_rows=0, rows_hint=0):
     """c = a . w (+ bias) of split operands (pairs, exps), or the pairs of its GELU scaled by 2^gelu_exps; raw, a_raw
     (int32 [rows, 1 + ceil(columns / 1024)]), the weight and the rows themselves as in bt_f32_split_more."""
     (ap, ae), (wp, we) = a, w
@@ -478,7 +478,7 @@ def gemm_f32_split(a, w, bias=None, gelu_exps=None, valid_rows=None, out=None, r
     if out is None:
         out = torch.zeros(*((cap, n) if gelu_exps is None else (cap, n // 32, 64)), device=ap.device,
                           dtype=torch.float32 if gelu_exps is None else torch.float16)
-    more = F32SplitMore(tile_rows, _ptr(raw), _ptr(a_raw), _ptr(weight), _ptr(rows), _ptr(row_index))
+    more = F32SplitMore(tile_rows, _ptr(raw), _ptr(a_raw), _ptr(weight), _ptr(rows), _ptr(row_index), rows_hint)
     _check(kernel_lib().bt_gemm_f32_split_with(_ptr(ap), _ptr(ae), _ptr(wp), _ptr(we), _ptr(bias), _ptr(out), _ptr(gelu_exps),
                                                _ptr(valid_rows), cap, n, k, ctypes.byref(more), _stream()))
     return out

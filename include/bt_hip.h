@@ -528,6 +528,7 @@ typedef struct bt_f32_split_more {
    * a_row_index[r] (r without an index) of `a` */
   const void *w, *a;
   const int *a_row_index;
+  int rows_hint;   /* how many rows are live, as far as the caller knows (0: it does not): chooses among tiles that give the same bits */
 } bt_f32_split_more;
 int bt_gemm_f32_split_with(const void *a_pairs, const int *a_exps, const void *w_pairs, const int *w_exps, const void *bias,
                            void *c, const int *gelu_exps, const int *valid_rows, int rows_cap, int n, int k,

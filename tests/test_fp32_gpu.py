@@ -287,6 +287,33 @@ def test_gemm_f32_split_against_float64(device, tile, rows, M, N, K):
         assert mine <= whole
 
 
+@pytest.mark.parametrize("rows,M,N,K", [(2561, 2560, 3072, 64), (3000, 2049, 3072, 768), (2560, 2305, 3070 // 32 * 32, 320), (2100, 2100, 4096, 128)])
+def test_gemm_f32_split_known_rows_change_no_bit(device, rows, M, N, K):
+    """The tile that a known row count may choose gives the bits of the other, among rows and columns out of proportion too."""
+    _say("gemm_f32_split rows_hint", rows, M, N, K)
+    rs = np.random.RandomState(rows + K)
+    x, w = rs.standard_normal((rows, K)).astype(np.float32), (rs.standard_normal((K, N)) * 0.02).astype(np.float32)
+    x[5, 1], x[M - 1, 2], x[300, 3] = 1e20, 1e20, np.inf
+    w[7, 40], w[9, N - 1] = 1e12, 1e-30
+    bias = _dev((rs.standard_normal(N) * 0.1).astype(np.float32), device)
+    vr = torch.tensor([M], dtype=torch.int32, device=device)
+    wd, xd = _dev(w, device), _dev(x, device)
+    (wp,), a, _ = ops.split_f32([wd], xd, layer=True)
+    ge = torch.full((rows,), 9, dtype=torch.int32, device=device)
+    got = []
+    for tile, hint in ((2, 0), (-1, M)):
+        ops.set_option("f32_gemm_tile", tile)
+        try:
+            raw = torch.zeros(rows, 1 + (N + 1023) // 1024, dtype=torch.int32, device=device)
+            got.append((ops.gemm_f32_split(a, wp, bias, None, vr, weight=wd, rows=xd, rows_hint=hint),
+                        ops.gemm_f32_split(a, wp, bias, ge, vr, raw=raw, weight=wd, rows=xd, rows_hint=hint), raw))
+        finally:
+            ops.set_option("f32_gemm_tile", -1)
+    for one, other in zip(*got):
+        assert torch.equal(one.view(torch.int32), other.view(torch.int32))
+    assert not got[1][0][M:].any() and got[1][0][:M].isfinite().float().mean() > 0.9
+
+
 @pytest.mark.parametrize("tile", [0, 1, 2])
 def test_gemm_f32_split_passes_infinities_and_nan_on(device, tile):
     _say("gemm_f32_split inf nan", tile)
