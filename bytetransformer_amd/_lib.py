@@ -60,6 +60,8 @@ KERNEL_ABI = {
                              c_int, _P, _P, _P, _P, _IP, _IP, _IP, c_int, c_int, _P]),
     "bt_split_f32_layer": (c_int, [c_int, POINTER(c_void_p), POINTER(c_void_p), POINTER(c_void_p), POINTER(c_int),
                                    POINTER(c_int), c_int, _P, _P, _P, _P, _IP, _IP, _IP, c_int, c_int, c_int, _P]),
+    "bt_split_f32_layer_mask_rows": (c_int, [c_int, POINTER(c_void_p), POINTER(c_void_p), POINTER(c_void_p), POINTER(c_int),
+                                             POINTER(c_int), c_int, _P, _P, _P, _P, _IP, _P, c_int, c_int, _IP, _IP, _IP, c_int, _P]),
     "bt_gemm_f32_split": (c_int, [_P, _IP, _P, _IP, _P, _P, _IP, _IP, c_int, c_int, c_int, _P]),
     "bt_gemm_f32_split_with": (c_int, [_P, _IP, _P, _IP, _P, _P, _IP, _IP, c_int, c_int, c_int, POINTER(F32SplitMore), _P]),
     "bt_add_bias_residual_layernorm_f32_split": (c_int, [_P, _P, _IP, _P, _P, _P, _IP, c_int, c_int, c_float, _P, _IP, _IP,

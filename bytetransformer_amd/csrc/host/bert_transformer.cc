@@ -188,7 +188,13 @@ void BertTransformer<OpType>::bert_infer(BertTransformerInferParam infer_param) 
         warm[warm_count] = w_use[i];
         warm_bytes[warm_count++] = (unsigned long long)w_k[i] * w_n[i] * sizeof(DataType_);
       }
-  if (!mask_direct && !qkv_mask_rows && (!have_offsets || mask_slots || pack_count > 0))
+  // float, operands split in every call: the launch that splits them counts the mask rows itself
+  const bool f32_split = OpType == OperationType::FP32 && f32_splits_operands(rows, !is_remove_padding_, hidden, inter);
+  int mask_rows_opt = -1;
+  if (f32_split) bt_get_option("qkv_mask_rows", &mask_rows_opt);
+  const bool split_mask_rows = f32_split && is_remove_padding_ && !have_offsets && mask_rows_opt != 0 &&
+                               bt_gemm_qkv_mask_rows_supported(batch_size, seq_len, Traits_::dtype);
+  if (!mask_direct && !qkv_mask_rows && !split_mask_rows && (!have_offsets || mask_slots || pack_count > 0))
     check_bt_error(bt_layer_prologue(atten_mask, Traits_::dtype, batch_size, seq_len,
                                      et_param.batch_idx, et_param.word_idx, seq_order,
                                      mask_slots, nullptr, head_num_, is_remove_padding_ ? 0 : 1,
@@ -236,7 +242,7 @@ void BertTransformer<OpType>::bert_infer(BertTransformerInferParam infer_param) 
     // float: Q/K/V stay token-major [rows, 3H], gamma and beta are float by definition.  The weights are consumed as
     // stored, or, where the rows are worth it, split afresh in every call (all four, and the input's rows, in one
     // launch; the input's pairs lie in FFN1's area until that is written).
-    const bool split = f32_splits_operands(rows, !is_remove_padding_, hidden, inter);
+    const bool split = f32_split;
     const F32SplitScratch sp(base + off + align_up(splitk_scratch_bytes(max_rows, hidden), 256), max_rows, hidden, inter);
     void *w_pairs[4];
     {
@@ -246,8 +252,13 @@ void BertTransformer<OpType>::bert_infer(BertTransformerInferParam infer_param) 
     if (split) {
       const bt_f32_split_more more{0, nullptr, nullptr, w_use[0], from_tensor, gather, known_rows};
       const void *w[4] = {w_use[0], w_use[1], w_use[2], w_use[3]};
-      check_bt_error(bt_split_f32_layer(4, w, w_pairs, sp.w_exps, w_k, w_n, 2, param_.inter_bias, sp.bounds, from_tensor,
-                                        inter_matmul_buf, sp.x_exps, gather, valid_rows, rows, hidden, 1, stream));
+      if (split_mask_rows)
+        check_bt_error(bt_split_f32_layer_mask_rows(4, w, w_pairs, sp.w_exps, w_k, w_n, 2, param_.inter_bias, sp.bounds,
+                                                    from_tensor, inter_matmul_buf, sp.x_exps, atten_mask, batch_size, seq_len,
+                                                    et_param.batch_idx, et_param.word_idx, seq_order, hidden, stream));
+      else
+        check_bt_error(bt_split_f32_layer(4, w, w_pairs, sp.w_exps, w_k, w_n, 2, param_.inter_bias, sp.bounds, from_tensor,
+                                          inter_matmul_buf, sp.x_exps, gather, valid_rows, rows, hidden, 1, stream));
       check_bt_error(bt_gemm_f32_split_with(inter_matmul_buf, sp.x_exps, w_pairs[0], sp.w_exps[0],
                                             param_.attention_param.attr_bias_QKV, qkv_buf, nullptr, valid_rows, rows,
                                             3 * hidden, hidden, &more, stream));

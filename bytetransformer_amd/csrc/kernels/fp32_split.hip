@@ -30,6 +30,7 @@
 // LDS tile, so loads, swizzle and LDS reads are those of an fp16 product of 2 K halfs.
 #include "f32_split.h"
 #include "gemm_common.h"
+#include "mask_rows.h"
 
 #include <cmath>
 
@@ -65,6 +66,11 @@ struct SplitArgs {
   int *row_exps;
   const int *row_index, *valid_rows;
   int rows_cap, hidden;
+  int row_blocks;           // workgroups for the rows
+  // a launch that counts the rows from the mask, and leaves the offsets for the launches behind it
+  const void *mask;
+  int mask_B, mask_S;
+  int *out_batch_idx, *out_word_idx, *out_seq_order;
 };
 
 __device__ __forceinline__ float finite_or_zero(float x) {
@@ -179,13 +185,25 @@ __device__ __forceinline__ void split_weight_unit(const SplitArgs &a, int unit) 
   }
 }
 
+// The rows' workgroups come first: theirs is the longer chain, above all where they count the mask rows, and the weights'
+// move in behind them.
+template <int MASK>
 __global__ __launch_bounds__(kSplitThreads) void split_f32_kernel(SplitArgs a) {
-  if ((int)blockIdx.x < a.units) return split_weight_unit(a, blockIdx.x);
-  const int r = ((int)blockIdx.x - a.units) * (kSplitThreads / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if ((int)blockIdx.x >= a.row_blocks) return split_weight_unit(a, (int)blockIdx.x - a.row_blocks);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = (int)blockIdx.x * (kSplitThreads / 64) + wave;
   const int lane = threadIdx.x & 63;
-  const int M = a.valid_rows ? min(scalar_load(a.valid_rows), a.rows_cap) : a.rows_cap;
-  if (r >= M) return;
-  const size_t from = a.row_index ? (size_t)scalar_load(a.row_index + r) : (size_t)r;
+  size_t from;
+  if constexpr (MASK != kMaskNone) {
+    __shared__ int s_len[kMaskRowsMaxBatch];
+    const MaskRows mr = mask_rows_setup<MASK>(a, wave, kSplitThreads / 64, lane, s_len);
+    if (blockIdx.x == 0) mask_rows_write(a, mr, (int)threadIdx.x, kSplitThreads, lane);
+    if (r >= min(mr.M, a.rows_cap)) return;
+    from = (size_t)__builtin_amdgcn_readfirstlane(mask_rows_map(mr, mask_rows_span(mr, a.mask_B, lane, r, r), r));
+  } else {
+    const int M = a.valid_rows ? min(scalar_load(a.valid_rows), a.rows_cap) : a.rows_cap;
+    if (r >= M) return;
+    from = a.row_index ? (size_t)scalar_load(a.row_index + r) : (size_t)r;
+  }
   const float4_t *src = (const float4_t *)(a.rows + from * a.hidden);
   float most = 0.f;
   for (int c = lane; c < a.hidden / 4; c += 64) {
@@ -687,16 +705,15 @@ extern "C" int bt_split_f32(int weight_count, const void *const *w, void *const 
                             row_index, valid_rows, rows_cap, hidden_dim, 0, stream);
 }
 
-extern "C" int bt_split_f32_layer(int weight_count, const void *const *w, void *const *w_pairs, int *const *w_exps,
-                                  const int *k, const int *n, int bounded, const void *bounded_bias, float *bounds,
-                                  const void *rows, void *row_pairs, int *row_exps, const int *row_index,
-                                  const int *valid_rows, int rows_cap, int hidden_dim, int layer, void *stream) {
+static int split_f32(SplitArgs a, int weight_count, const void *const *w, void *const *w_pairs, int *const *w_exps, const int *k,
+                     const int *n, int bounded, const void *bounded_bias, float *bounds, const void *rows, void *row_pairs,
+                     int *row_exps, const int *row_index, const int *valid_rows, int rows_cap, int hidden_dim, int layer,
+                     void *stream) {
   const char *who = "bt_split_f32";
   BT_REQUIRE(weight_count >= 0 && weight_count <= 4, BT_ERR_INVALID_ARGUMENT, "%s: weight_count=%d outside [0, 4]", who, weight_count);
   BT_REQUIRE(weight_count == 0 || (w && w_pairs && w_exps && k && n), BT_ERR_INVALID_ARGUMENT, "%s: null pointer argument", who);
   BT_REQUIRE(bounded < weight_count && (bounded < 0 || (bounded_bias && bounds)), BT_ERR_INVALID_ARGUMENT,
              "%s: bounded=%d needs a weight, its bias and an array of bounds", who, bounded);
-  SplitArgs a{};
   int units = 0;
   for (int i = 0; i < weight_count; ++i) {
     BT_REQUIRE(w[i] && w_pairs[i] && w_exps[i], BT_ERR_INVALID_ARGUMENT, "%s: null pointer of matrix %d", who, i);
@@ -721,8 +738,35 @@ extern "C" int bt_split_f32_layer(int weight_count, const void *const *w, void *
     a.row_index = row_index, a.valid_rows = valid_rows, a.rows_cap = rows_cap, a.hidden = hidden_dim;
     row_blocks = (rows_cap + kSplitThreads / 64 - 1) / (kSplitThreads / 64);
   }
+  a.row_blocks = row_blocks;
   if (units + row_blocks == 0) return BT_OK;
-  return Launch<split_f32_kernel>::on(as_stream(stream), who, units + row_blocks, kSplitThreads, 0, a);
+  if (a.mask) return Launch<split_f32_kernel<kMaskF32>>::on(as_stream(stream), who, units + row_blocks, kSplitThreads, 0, a);
+  return Launch<split_f32_kernel<kMaskNone>>::on(as_stream(stream), who, units + row_blocks, kSplitThreads, 0, a);
+}
+
+extern "C" int bt_split_f32_layer(int weight_count, const void *const *w, void *const *w_pairs, int *const *w_exps,
+                                  const int *k, const int *n, int bounded, const void *bounded_bias, float *bounds,
+                                  const void *rows, void *row_pairs, int *row_exps, const int *row_index,
+                                  const int *valid_rows, int rows_cap, int hidden_dim, int layer, void *stream) {
+  return split_f32(SplitArgs{}, weight_count, w, w_pairs, w_exps, k, n, bounded, bounded_bias, bounds, rows, row_pairs, row_exps,
+                   row_index, valid_rows, rows_cap, hidden_dim, layer, stream);
+}
+
+extern "C" int bt_split_f32_layer_mask_rows(int weight_count, const void *const *w, void *const *w_pairs, int *const *w_exps,
+                                            const int *k, const int *n, int bounded, const void *bounded_bias, float *bounds,
+                                            const void *rows, void *row_pairs, int *row_exps, const void *atten_mask,
+                                            int batch_size, int seq_len, int *batch_idx, int *word_idx, int *seq_order,
+                                            int hidden_dim, void *stream) {
+  const char *who = "bt_split_f32_layer_mask_rows";
+  BT_REQUIRE(rows && atten_mask && batch_idx, BT_ERR_INVALID_ARGUMENT, "%s: null pointer argument", who);
+  BT_REQUIRE(bt_gemm_qkv_mask_rows_supported(batch_size, seq_len, BT_F32), BT_ERR_UNSUPPORTED,
+             "%s: batch_size=%d seq_len=%d is outside what bt_gemm_qkv_mask_rows_supported allows", who, batch_size, seq_len);
+  BT_REQUIRE(aligned16({atten_mask}), BT_ERR_INVALID_ARGUMENT, "%s: tensor pointers must be 16-byte aligned", who);
+  SplitArgs a{};
+  a.mask = atten_mask, a.mask_B = batch_size, a.mask_S = seq_len;
+  a.out_batch_idx = batch_idx, a.out_word_idx = word_idx, a.out_seq_order = seq_order;
+  return split_f32(a, weight_count, w, w_pairs, w_exps, k, n, bounded, bounded_bias, bounds, rows, row_pairs, row_exps, nullptr,
+                   nullptr, batch_size * seq_len, hidden_dim, 1, stream);
 }
 
 extern "C" int bt_gemm_f32_split(const void *a_pairs, const int *a_exps, const void *w_pairs, const int *w_exps, const void *bias,

@@ -445,8 +445,11 @@ def gemm_f32(a, w, bias=None, gelu=False, valid_rows=None, a_row_index=None, row
     return out
 
 
-def split_f32(ws, rows=None, bounded=-1, bounded_bias=None, row_index=None, valid_rows=None, rows_cap=None, layer=False):
-    """Weights [K, N] and rows as scaled pairs of fp16 numbers: ([(pairs, exps)], (row pairs, row exps) or None, bounds)."""
+def split_f32(ws, rows=None, bounded=-1, bounded_bias=None, row_index=None, valid_rows=None, rows_cap=None, layer=False,
+              mask=None):
+    """Weights [K, N] and rows as scaled pairs of fp16 numbers: ([(pairs, exps)], (row pairs, row exps) or None, bounds).
+    With a float prefix mask [B, S, S] the rows are those of a padded [B * S, hidden] input that it names, and a fourth value
+    is (batch_idx, word_idx, seq_order)."""
     _need_f32(*ws, rows, bounded_bias)
     lib, n = kernel_lib(), len(ws)
     dev = (ws[0] if n else rows).device
@@ -463,6 +466,16 @@ def split_f32(ws, rows=None, bounded=-1, bounded_bias=None, row_index=None, vali
                torch.zeros(cap, dtype=torch.int32, device=dev))
     ptrs = [(ctypes.c_void_p * max(n, 1))(*[t.data_ptr() for t in ts]) for ts in (ws, pairs, exps)]
     sizes = [(ctypes.c_int * max(n, 1))(*[w.shape[d] for w in ws]) for d in (0, 1)]
+    if mask is not None:
+        _need_f32(mask)
+        B, S = mask.shape[:2]
+        if rows.shape[0] != B * S or mask.shape[2] != S:
+            raise ValueError("split_f32: a mask [B, S, S] names rows of [B * S, hidden]")
+        offsets = [torch.zeros(m, dtype=torch.int32, device=dev) for m in (B + 1, B * S, B)]
+        _check(lib.bt_split_f32_layer_mask_rows(n, *ptrs, *sizes, bounded, _ptr(bounded_bias), _ptr(bounds), _ptr(rows),
+                                                _ptr(got[0]), _ptr(got[1]), _ptr(mask), B, S, *[_ptr(o) for o in offsets], hidden,
+                                                _stream()))
+        return list(zip(pairs, exps)), got, bounds, tuple(offsets)
     _check(lib.bt_split_f32_layer(n, *ptrs, *sizes, bounded, _ptr(bounded_bias), _ptr(bounds), _ptr(rows),
                                   _ptr(got[0] if got else None), _ptr(got[1] if got else None), _ptr(row_index),
                                   _ptr(valid_rows), got[0].shape[0] if got else 0, hidden, int(layer), _stream()))

@@ -512,6 +512,12 @@ int bt_split_f32_layer(int weight_count, const void *const *w, void *const *w_pa
                        const int *n, int bounded, const void *bounded_bias, float *bounds, const void *rows, void *row_pairs,
                        int *row_exps, const int *row_index, const int *valid_rows, int rows_cap, int hidden_dim, int layer,
                        void *stream);
+/* ... layer = 1 for the rows of a padded [batch_size, seq_len, hidden_dim] input that a prefix mask names: the launch counts
+ * them itself and leaves batch_idx, word_idx and seq_order (as bt_gemm_qkv_bias_split_mask_rows, same sizes). */
+int bt_split_f32_layer_mask_rows(int weight_count, const void *const *w, void *const *w_pairs, int *const *w_exps,
+                                 const int *k, const int *n, int bounded, const void *bounded_bias, float *bounds,
+                                 const void *rows, void *row_pairs, int *row_exps, const void *atten_mask, int batch_size,
+                                 int seq_len, int *batch_idx, int *word_idx, int *seq_order, int hidden_dim, void *stream);
 int bt_gemm_f32_split(const void *a_pairs, const int *a_exps, const void *w_pairs, const int *w_exps, const void *bias,
                       void *c, const int *gelu_exps, const int *valid_rows, int rows_cap, int n, int k, void *stream);
 typedef struct bt_f32_split_more {

@@ -251,6 +251,28 @@ def test_split_f32_holds_what_it_was_given(device, K, N):
     assert bounds[:, 0].max().item() == top.max() and bounds[:, 1].max().item() == np.abs(bias).max()
 
 
+@pytest.mark.parametrize("lens,S", [([5], 5), ([0, 17, 0], 17), ([64, 1, 33], 64), ([200, 0, 131, 65, 200, 7, 1, 90, 199], 200), ([3] * 64, 8), ([100] * 33, 129)])
+def test_split_f32_counts_the_mask_rows(device, lens, S):
+    """The launch that counts its rows leaves the offsets of bt_build_offsets, and the same pairs of the same rows and weights."""
+    _say("split_f32 mask rows", len(lens), S)
+    rs = np.random.RandomState(S)
+    B, K = len(lens), 128
+    mask = np.zeros((B, S, S), np.float32)
+    for b, n in enumerate(lens):
+        mask[b, :, :n] = 1
+    x, w = _dev(rs.standard_normal((B * S, K)).astype(np.float32), device), _dev(rs.standard_normal((K, 64)).astype(np.float32), device)
+    m = _dev(mask, device)
+    (wp,), got, _, (batch_idx, word_idx, seq_order) = ops.split_f32([w], x, mask=m, layer=True)
+    exp_word = np.concatenate([b * S + np.arange(n) for b, n in enumerate(lens)] + [b * S + np.arange(n, S) for b, n in enumerate(lens)])
+    M = sum(lens)
+    assert np.array_equal(batch_idx.cpu().numpy(), np.concatenate([[0], np.cumsum(lens)]))
+    assert np.array_equal(word_idx.cpu().numpy(), exp_word)
+    assert np.array_equal(seq_order.cpu().numpy(), sorted(range(B), key=lambda b: (-lens[b], b)))
+    vr = torch.tensor([M], dtype=torch.int32, device=device)
+    (vp,), ref, _ = ops.split_f32([w], x, row_index=word_idx, valid_rows=vr, layer=True)
+    assert all(torch.equal(one, other) for one, other in zip(wp + got, vp + ref))
+
+
 @pytest.mark.parametrize("tile", [-1, 0, 1, 2])
 @pytest.mark.parametrize("rows,M,N,K", [(300, 300, 768, 768), (200, 131, 160, 64), (97, 96, 32, 320), (64, 1, 2304, 768), (140, 140, 192, 512),
                                         (130, 129, 96, 3072), (193, 193, 416, 832)])
