@@ -205,17 +205,30 @@ __global__ __launch_bounds__(kSplitThreads) void split_f32_kernel(SplitArgs a) {
     from = a.row_index ? (size_t)scalar_load(a.row_index + r) : (size_t)r;
   }
   const float4_t *src = (const float4_t *)(a.rows + from * a.hidden);
+  // up to 1024 values stay in registers, all asked for at once; of longer rows the rest is read again
+  constexpr int kKept = 4;
+  float4_t kept[kKept];
+#pragma unroll
+  for (int i = 0; i < kKept; ++i) {
+    kept[i] = float4_t{0.f, 0.f, 0.f, 0.f};
+    if (lane + 64 * i < a.hidden / 4) kept[i] = src[lane + 64 * i];
+  }
   float most = 0.f;
-  for (int c = lane; c < a.hidden / 4; c += 64) {
-    const float4_t v = src[c];
+  const auto look = [&](float4_t v) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) most = fmaxf(most, finite_or_zero(v[e]));
-  }
+  };
+#pragma unroll
+  for (int i = 0; i < kKept; ++i) look(kept[i]);
+  for (int c = lane + 64 * kKept; c < a.hidden / 4; c += 64) look(src[c]);
   const int e = split_exponent(wave_max(most));
   const float scale = split_power(e);
   bool small = false;
-  for (int c = lane; c < a.hidden / 4; c += 64)
-    small = split_store(a.row_pairs + (size_t)r * 2 * a.hidden, c, src[c] * scale) || small;
+  half_t *to = a.row_pairs + (size_t)r * 2 * a.hidden;
+#pragma unroll
+  for (int i = 0; i < kKept; ++i)
+    if (lane + 64 * i < a.hidden / 4) small = split_store(to, lane + 64 * i, kept[i] * scale) || small;
+  for (int c = lane + 64 * kKept; c < a.hidden / 4; c += 64) small = split_store(to, c, src[c] * scale) || small;
   bool marked = false;
   if (a.layer && __builtin_amdgcn_ballot_w64(small) != 0) {
     float score = 0.f;
