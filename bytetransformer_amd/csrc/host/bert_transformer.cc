@@ -112,7 +112,7 @@ void BertTransformer<OpType>::bert_infer(BertTransformerInferParam infer_param) 
       infer_param.offsets && infer_param.offsets->batch_idx && infer_param.offsets->word_idx;
   const bool streaming_fp16 = OpType == OperationType::HALF && size_per_head_ == 64 &&
                               !attention_layer_->uses_short_kernel(seq_len);
-  const LayerPlan lp = plan(batch_size, seq_len, have_offsets, infer_param.valid_rows_hint);
+  LayerPlan lp = plan(batch_size, seq_len, have_offsets, infer_param.valid_rows_hint);
   const bool mask_direct = lp.mask_direct;
   const bool qkv_mask_rows = lp.starts_with_qkv;
   // The four products read the [k, n] weights as the caller stores them, exactly as the
@@ -124,6 +124,26 @@ void BertTransformer<OpType>::bert_infer(BertTransformerInferParam infer_param) 
   const bool have_prepack = OpType == OperationType::HALF && param_.prepacked_kernels[0] &&
                             param_.prepacked_kernels[1] && param_.prepacked_kernels[2] &&
                             param_.prepacked_kernels[3];
+  // Row capacity of the launches over packed rows that follow the attention.  A caller
+  // that passes offsets of its own vouches for their exact live count, so these launches
+  // are then sized for it instead of batch * seq_len: no workgroups
+  // that only find out on the device that their rows do not exist (1.7-2.2 us per layer
+  // at batch 16 x 512), and a short sequence in a long padded row still takes the split-k
+  // FFN2.  The QKV product and the attention keep batch * seq_len: it is the row stride
+  // of the per-head Q/K/V layout and the extent of the gathered input.
+  const int vouched = have_offsets && is_remove_padding_ ? infer_param.offsets->valid_word_num : 0;
+  const bool exact = vouched > 0 && vouched <= rows;
+  const int packed_cap = exact ? vouched : rows;
+  // ... and the products behind the attention take every row of it for live: choices made from
+  // sizes alone (FFN2's slices, tile 14) then follow the count itself instead of a padded batch's
+  // 60 %.  Their rows lie in the scratch, so a row too many costs time only; the LayerNorms,
+  // which read through the caller's word_idx, keep the device's count.
+  const bool all_live = !is_remove_padding_ || exact;
+  // Few rows: the first LayerNorm in FFN1's launch.  It follows from sizes and from whose weights these are, not from a copy,
+  // and such a layer makes none for FFN1 nor beside the LayerNorm: copies change no bit.
+  const bool norm_in_ffn1 = OpType == OperationType::HALF && !use_fp32_ &&
+                            bt_layernorm_gemm_bias_gelu_pays(packed_cap, all_live, inter, hidden, have_prepack ? 0 : 1);
+  if (norm_in_ffn1) lp.copy[2] = lp.ln_copy[2] = lp.ln_copy[3] = false;
   const DataType_ *w_use[4] = {param_.attr_kernel_QKV, param_.attr_output_kernel,
                                param_.inter_kernel, param_.output_kernel};
   int w_kn[4] = {1, 1, 1, 1};
@@ -209,19 +229,6 @@ void BertTransformer<OpType>::bert_infer(BertTransformerInferParam infer_param) 
   const int *gather = nullptr;
   DataType_ *restore_target = nullptr;
   int known_rows = 0;   // of packed rows, 0: the host does not know
-  // Row capacity of the launches over packed rows that follow the attention.  A caller
-  // that passes offsets of its own vouches for their exact live count, so these launches
-  // are then sized for it instead of batch * seq_len: no workgroups
-  // that only find out on the device that their rows do not exist (1.7-2.2 us per layer
-  // at batch 16 x 512), and a short sequence in a long padded row still takes the split-k
-  // FFN2.  The QKV product and the attention keep batch * seq_len: it is the row stride
-  // of the per-head Q/K/V layout and the extent of the gathered input.
-  int packed_cap = rows;
-  // ... and the products behind the attention take every row of it for live: choices made from
-  // sizes alone (FFN2's slices, tile 14) then follow the count itself instead of a padded batch's
-  // 60 %.  Their rows lie in the scratch, so a row too many costs time only; the LayerNorms,
-  // which read through the caller's word_idx, keep the device's count.
-  bool all_live = !is_remove_padding_;
   if (is_remove_padding_) {
     // The packed copy of the input is never materialised: the QKV GEMM and the
     // first LayerNorm read valid token t from the padded input at row word_idx[t]
@@ -230,10 +237,6 @@ void BertTransformer<OpType>::bert_infer(BertTransformerInferParam infer_param) 
     restore_target = transformer_out;
     transformer_out = qkv_buf;  // FFN2 output reuses the dead qkv region
     valid_rows = et_param.batch_idx + batch_size;
-    if (have_offsets && rows_hint > 0 && rows_hint <= rows) {
-      packed_cap = rows_hint;
-      all_live = true;
-    }
     known_rows = rows_hint;
     rows_hint = rows_to_plan_for(rows_hint, true, batch_size, rows);
   }
@@ -378,8 +381,7 @@ void BertTransformer<OpType>::bert_infer(BertTransformerInferParam infer_param) 
   attention_layer_->infer(attention_infer_param);
 
   const int *product_rows = all_live ? nullptr : valid_rows;
-  // few rows: the first LayerNorm in FFN1's launch, which reads the projection from where Q was
-  const bool norm_in_ffn1 = ln_count == 0 && !use_fp32_ && bt_layernorm_gemm_bias_gelu_pays(packed_cap, all_live, inter, hidden, w_kn[2]);
+  // (FFN1's launch, where it has the LayerNorm, reads the projection from where Q was)
   DataType_ *proj_out = norm_in_ffn1 ? qkv_buf : attr_matmul_buf;
   check_bt_error(
       bt_gemm(attr_out_buf, wt_proj, proj_out, product_rows, packed_cap, rows_hint, hidden,

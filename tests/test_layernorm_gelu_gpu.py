@@ -2,6 +2,7 @@
 import pytest
 import torch
 
+import bytetransformer_amd as bt
 from bytetransformer_amd import ops
 
 pytestmark = pytest.mark.gpu
@@ -80,3 +81,28 @@ def test_sizes_that_keep_two_launches():
     with pytest.raises(ops.BtError):
         ops.layernorm_gemm_bias_gelu(x, x, v, v, v, torch.zeros(640, 2560, dtype=torch.float16, device="cuda"),
                                      torch.zeros(2560, dtype=torch.float16, device="cuda"), w_kn=True)
+
+
+@pytest.mark.parametrize("batch,seq_len", [(1, 32), (1, 72), (3, 14), (4, 25)])
+def test_weight_copies_change_no_bit(batch, seq_len):
+    """Never, always and the table's choice of copies, on padded and on packed rows."""
+    bt.load_th_op()
+    gen = torch.Generator(device="cuda").manual_seed(seq_len)
+
+    def normal(*shape, std=0.02, mean=0.0):
+        return torch.empty(shape, dtype=torch.float16, device="cuda").normal_(mean, std, generator=gen)
+
+    H = 768
+    w = [normal(H, 3 * H), normal(3 * H), normal(H, H), normal(H), normal(H, std=0.05, mean=1.0), normal(H), normal(H, 4 * H), normal(4 * H),
+         normal(4 * H, H), normal(H), normal(H, std=0.05, mean=1.0), normal(H)]
+    x = normal(batch, seq_len, H, std=1.0)
+    lens = torch.arange(seq_len, 0, -(seq_len // batch), device="cuda")[:batch]
+    mask = (torch.arange(seq_len, device="cuda")[None, None, :] < lens[:, None, None]).half().expand(batch, seq_len, seq_len).contiguous()
+    got = []
+    try:
+        for choice in (0, 1, -1):
+            ops.set_option("layer_prepack", choice)
+            got.append(torch.ops.ByteTransformer.BertTransformer(12, 64, *w, x, mask, True, True))
+    finally:
+        ops.set_option("layer_prepack", -1)
+    assert got[0].isfinite().all() and torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
