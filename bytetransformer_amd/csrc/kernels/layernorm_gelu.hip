@@ -9,50 +9,45 @@ constexpr int kLgRows = 16, kLgWaves = 8;
 // A workgroup normalises 16 rows (two a wave, in registers as the LayerNorm launch has them), keeps them in LDS as one
 // operand and multiplies them by COLS columns of the weight.  Every column tile of a row tile repeats the rows' work:
 // what it costs is less than a launch and its gap, and the weight, whose fetch is most of FFN1's time here, is on its way
-// meanwhile: it goes straight to registers, all of it requested at the head of the kernel behind the rows.
-// (12 layers, operator, 1 x 32, one box: 329 -> 311 us; the two launches and this one at other sizes: lg_cols.)
+// meanwhile: all of it is requested, straight into LDS, at the head of the kernel behind the rows.
+// (12 layers, operator, 1 x 32, one box: 330 -> 310 us.  With the weight in registers, each wave an eighth of k, the launch took
+// 0.2 to 0.4 us longer, hidden 768, 32 rows 5.28 / 5.04 for a [K, N] weight and 5.01 / 4.68 for [N, K], and added up in an
+// order of its own.)
 //
-// The waves share k; lane l of a wave has the W columns from W (l & 15) on at eight k, from 8 (l >> 4) on, of every 32: of
-// a [K, N] weight W neighbouring halfs of eight k-rows, which make W operands of a 16x16x32 instruction in lane, of an
-// [N, K] weight 16 bytes of each column.  Either way instruction j of the W has columns j, W + j, 2 W + j, ..., a lane's
-// sums are 4 W neighbouring columns of a row, and the bits are the same.
+// The results are, bit for bit, those of the two launches: a sum is formed in the order of the product that these sizes
+// would get (product_takes_wave_k).  SLICED: tile 14's, four slices of k, every fourth step of 64 each, added up in the end
+// and the bias behind them; a wave has a slice of half the columns.  Else that of all other tiles, one chain over k from the
+// bias on; four waves have 16 columns each.  (A 16x16x32 instruction gives the bits of two 32x32x16 ones.)
 template <int HIDDEN, int COLS>
 struct LgShape {
-  static constexpr int W = COLS / 16, KS = kLgWaves;   // columns a lane; slices of k
-  static constexpr int KB = HIDDEN / KS / 32;          // 32 k at a time, of a wave's share
-  static constexpr int PITCH = HIDDEN + 8;             // rows 16 bytes further on: 16 of them lie in different banks
-  static constexpr size_t kRowBytes = (size_t)kLgRows * PITCH * sizeof(half_t);
-  static constexpr size_t kLds = kRowBytes + (size_t)kLgRows * COLS * KS * sizeof(float);
-  static_assert(HIDDEN % (32 * KS) == 0 && kRowBytes % 16 == 0 && kLds <= 160 * 1024, "whole shares of k");
+  static constexpr int ROW_HALFS = kLgRows * HIDDEN, WEIGHT_HALFS = HIDDEN * COLS;
+  static constexpr size_t kOperands = (size_t)(ROW_HALFS + WEIGHT_HALFS) * sizeof(half_t);
+  static constexpr size_t kSums = (size_t)4 * kLgRows * COLS * sizeof(float);   // of the slices
+  static constexpr bool kSumsApart = kOperands + kSums <= 160 * 1024;           // else in the weight's place
+  static constexpr size_t kLds = kOperands + (kSumsApart ? kSums : 0);
+  static constexpr int LOADS = WEIGHT_HALFS / 512 / kLgWaves;   // 1 KB a wave's instruction
+  static_assert(HIDDEN % 256 == 0 && (COLS == 32 || COLS == 64) && kLds <= 160 * 1024, "whole rounds of the waves, LDS budget");
+  static_assert(kSums <= (size_t)WEIGHT_HALFS * sizeof(half_t), "sums fit the weight's place");
 };
 
-#if defined(__HIP_DEVICE_COMPILE__)
-// sizeof(T) bytes at `lane_bytes + scalar_bytes` of the descriptor.
-template <typename T>
-__device__ __forceinline__ T lg_load(rsrc_t rs, int lane_bytes, int scalar_bytes) {
-  if constexpr (sizeof(T) == 16)
-    return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b128(rs, lane_bytes, scalar_bytes, 0));
-  else if constexpr (sizeof(T) == 8)
-    return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(rs, lane_bytes, scalar_bytes, 0));
-  else
-    return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(rs, lane_bytes, scalar_bytes, 0));
-}
-#endif
+// Where chunk c (16 bytes) of row r of the normalised rows lies: 16 rows of one chunk, what a pass of the operand's reads
+// takes, are in 16 places of the 256 bytes that the banks hold.
+__device__ __forceinline__ int lg_chunk(int r, int c) { return c ^ r; }
 
-template <int HIDDEN, int COLS, bool WKN>
+template <int HIDDEN, int COLS, bool WKN, bool SLICED>
 __global__ __launch_bounds__(kLgWaves *kWave) void layernorm_gelu_kernel(
     const half_t *src, const half_t *residual, const int *residual_row_index, const int *valid_rows, const half_t *w,
     const half_t *bias, const half_t *gamma, const half_t *beta, half_t *dst, const half_t *ffn_bias, half_t *out,
     int rows_cap, int N, float eps, int unused) {
 #if defined(__HIP_DEVICE_COMPILE__)
   typedef LgShape<HIDDEN, COLS> Sh;
-  constexpr int W = Sh::W, KB = Sh::KB, KS = Sh::KS, PITCH = Sh::PITCH;
   constexpr int V = HIDDEN % 512 == 0 ? 8 : 4, NC = HIDDEN / kWave / V;
   constexpr int kWaveRows = kLgRows / kLgWaves;
   typedef typename LnVec<V>::halfs vec_t;
-  typedef _Float16 cols_t __attribute__((ext_vector_type(W)));
   static_assert(NC * V * kWave == HIDDEN, "a row fills the lanes");
+  static_assert(WKN || COLS == 32, "an [N, K] image is laid out for 32 columns");
   extern __shared__ __attribute__((aligned(1024))) half_t lg_smem[];
+  half_t *rows = lg_smem, *weight = lg_smem + Sh::ROW_HALFS;
 
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int M = valid_rows ? min(scalar_load(valid_rows), rows_cap) : rows_cap;
@@ -75,8 +70,12 @@ __global__ __launch_bounds__(kLgWaves *kWave) void layernorm_gelu_kernel(
   const auto load_row = [&](const half_t *tensor, int r, vec_t (&to)[NC]) {
     const rsrc_t rs = make_rsrc(tensor + (size_t)r * HIDDEN, HIDDEN * sizeof(half_t));
 #pragma unroll
-    for (int c = 0; c < NC; ++c)
-      to[c] = lg_load<vec_t>(rs, lane * (int)sizeof(vec_t), c * kWave * (int)sizeof(vec_t));
+    for (int c = 0; c < NC; ++c) {
+      if constexpr (V == 8)
+        to[c] = __builtin_bit_cast(vec_t, __builtin_amdgcn_raw_buffer_load_b128(rs, lane * 16, c * kWave * 16, 0));
+      else
+        to[c] = __builtin_bit_cast(vec_t, __builtin_amdgcn_raw_buffer_load_b64(rs, lane * 8, c * kWave * 8, 0));
+    }
   };
 #pragma unroll
   for (int i = 0; i < kWaveRows; ++i) load_row(src, row[i], av[i]);
@@ -85,27 +84,28 @@ __global__ __launch_bounds__(kLgWaves *kWave) void layernorm_gelu_kernel(
   load_row(bias, 0, bias_v);
   load_row(gamma, 0, gamma_v);
   load_row(beta, 0, beta_v);
-  // the sums that wave q < W folds and stores
-  const int fold_n = n0 + 4 * W * (lane >> 4) + 4 * min(wave, W - 1), fold_r = lane & 15;
-  const half4_t ffn_bias_v = *(const half4_t *)(ffn_bias + fold_n);
+  // wave t < COLS / 16 stores columns 16 t + 4 (lane >> 4) .. + 3 of row lane & 15
+  const int out_r = lane & 15, out_n = n0 + 16 * min(wave, COLS / 16 - 1) + 4 * (lane >> 4);
+  const half4_t ffn_bias_v = *(const half4_t *)(ffn_bias + out_n);
 
-  // the weight
-  const int slice_k = wave * KB * 32, lane_n = W * (lane & 15), lane_k = 8 * (lane >> 4);
-  // (one lane offset, the rest in scalars: with an address for every load this took 1.3 us of instructions)
-  const size_t first = WKN ? (size_t)slice_k * N + n0 : (size_t)n0 * HIDDEN + slice_k;
-  const rsrc_t rs_w = make_rsrc(w + first, ((size_t)HIDDEN * N - first) * sizeof(half_t));
-  const int lane_at = (WKN ? lane_k * N + lane_n : lane_n * HIDDEN + lane_k) * (int)sizeof(half_t);
-  cols_t rows_w[WKN ? KB : 1][8];
-  half8_t cols_w[WKN ? 1 : KB][W];
-#pragma unroll
-  for (int b = 0; b < KB; ++b) {
+  // the weight: instruction i of wave v lands KB 8 i + v of the image, a lane offset and the rest in scalars.  [K, N]: its k-rows
+  // of COLS columns (swz_kn); [N, K]: for every 64 k a tile of 32 columns (swz)
+  {
+    const rsrc_t rs = WKN ? make_rsrc(w + n0, ((size_t)HIDDEN * N - n0) * sizeof(half_t))
+                          : make_rsrc(w + (size_t)n0 * HIDDEN, (size_t)(N - n0) * HIDDEN * sizeof(half_t));
+    int lane_at, step;   // bytes; from one instruction to the next
     if constexpr (WKN) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) rows_w[b][e] = lg_load<cols_t>(rs_w, lane_at, (b * 32 + e) * N * (int)sizeof(half_t));
+      lane_at = kn_load_offset<COLS>(wave, lane, N, COLS);
+      step = 4096 / COLS * N * (int)sizeof(half_t);
     } else {
-#pragma unroll
-      for (int j = 0; j < W; ++j) cols_w[b][j] = lg_load<half8_t>(rs_w, lane_at, (j * HIDDEN + b * 32) * (int)sizeof(half_t));
+      const int col = (wave & 3) * 8 + (lane >> 3);
+      lane_at = (col * HIDDEN + (wave >> 2) * 64 + (((lane & 7) ^ swz(col)) << 3)) * (int)sizeof(half_t);
+      step = 128 * (int)sizeof(half_t);
     }
+#pragma unroll
+    for (int i = 0; i < Sh::LOADS; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void *)(weight + (8 * i + wave) * 512), 16,
+                                               lane_at, i * step, 0, 0);
   }
   __builtin_amdgcn_sched_barrier(0);   // (all requested before the first row is waited for)
 
@@ -115,75 +115,97 @@ __global__ __launch_bounds__(kLgWaves *kWave) void layernorm_gelu_kernel(
   for (int c = 0; c < NC; ++c) live[c] = true;
 #pragma unroll
   for (int i = 0; i < kWaveRows; ++i) {
+    const int r = wave * kWaveRows + i;
     float v[NC][V];
     const float rstd = ln_statistics<NC, V>(av[i], rv[i], bias_v, live, kInverse, eps, v);
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
       vec_t y;
 #pragma unroll
-      for (int j = 0; j < V; ++j) y[j] = (half_t)(v[c][j] * rstd * (float)gamma_v[c][j] + (float)beta_v[c][j]);
-      *(vec_t *)(lg_smem + (wave * kWaveRows + i) * PITCH + (lane + c * kWave) * V) = y;
-    }
-  }
-  __syncthreads();
-
-  float4_t acc[W] = {};
-#pragma unroll
-  for (int b = 0; b < KB; ++b) {
-    const half8_t fa = *(const half8_t *)(lg_smem + (lane & 15) * PITCH + slice_k + lane_k + b * 32);
-#pragma unroll
-    for (int j = 0; j < W; ++j) {
-      half8_t fw;
-      if constexpr (WKN) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) fw[e] = rows_w[b][e][j];
-      } else {
-        fw = cols_w[b][j];
+      for (int j = 0; j < V; ++j) {
+        float f = v[c][j] * rstd * (float)gamma_v[c][j] + (float)beta_v[c][j];
+        asm("" : "+v"(f));   // a float, then a half, as in the LayerNorm launch: not v_fma_mixlo_f16, which rounds once
+        y[j] = (half_t)f;
       }
-      acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fw, fa, acc[j], 0, 0, 0);
+      const int k = (lane + c * kWave) * V;
+      *(vec_t *)(rows + r * HIDDEN + lg_chunk(r, k >> 3) * 8 + (k & 7)) = y;
     }
   }
-
-  // fold: acc[j][v] is column 4 W (lane >> 4) + W v + j of row lane & 15; four neighbouring columns of a lane are quad h,
-  // which wave h adds up over the slices
-  float4_t *sums = (float4_t *)((char *)lg_smem + Sh::kRowBytes);
-#pragma unroll
-  for (int h = 0; h < W; ++h) {
-    float4_t four;
-#pragma unroll
-    for (int t = 0; t < 4; ++t) four[t] = acc[(4 * h + t) % W][(4 * h + t) / W];
-    sums[(wave * W + h) * kWave + lane] = four;
-  }
+  wait_vmcnt<0>();   // (the weight of this wave)
   __syncthreads();
-  if (wave < W && m0 + fold_r < M) {
-    float4_t v = sums[wave * kWave + lane];
+
+  // 32 k from k0 on: 16 columns from column n of the tile, and the rows
+  const auto columns = [&](int n, int k0) {
+    if constexpr (WKN) return load_kn_frag<COLS>(weight, n, k0, lane);
+    const int col = n + (lane & 15), chunk = (k0 & 63) / 8 + (lane >> 4);
+    return *(const half8_t *)(weight + (k0 >> 6) * (32 * 64) + col * 64 + ((chunk ^ swz(col)) << 3));
+  };
+  const auto operand = [&](int k0) {
+    return *(const half8_t *)(rows + (lane & 15) * HIDDEN + lg_chunk(lane & 15, k0 / 8 + (lane >> 4)) * 8);
+  };
+  float4_t v;
+  if constexpr (SLICED) {
+    constexpr int G = COLS / 32;   // 16 columns each, of a wave
+    const int slice = wave & 3, half = wave >> 2;
+    float4_t acc[G] = {};
 #pragma unroll
-    for (int s = 1; s < KS; ++s) v += sums[(s * W + wave) * kWave + lane];
+    for (int u = 0; u < HIDDEN / 128; ++u) {
+      const int k0 = (u >> 1) * 256 + slice * 64 + (u & 1) * 32;
+      const half8_t fa = operand(k0);
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+        acc[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(columns((half * G + g) * 16, k0), fa, acc[g], 0, 0, 0);
+    }
+    if (!Sh::kSumsApart) __syncthreads();   // everyone is done with the weight
+    float4_t *sums = (float4_t *)(Sh::kSumsApart ? weight + Sh::WEIGHT_HALFS : weight);
+#pragma unroll
+    for (int g = 0; g < G; ++g) sums[(slice * 2 * G + half * G + g) * kWave + lane] = acc[g];
+    __syncthreads();
+    if (wave < 2 * G) {
+      v = sums[wave * kWave + lane];
+#pragma unroll
+      for (int s = 1; s < 4; ++s) v += sums[(s * 2 * G + wave) * kWave + lane];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] += (float)ffn_bias_v[e];
+    }
+  } else if (wave < COLS / 16) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = (float)ffn_bias_v[e];
+#pragma unroll
+    for (int k0 = 0; k0 < HIDDEN; k0 += 32)
+      v = __builtin_amdgcn_mfma_f32_16x16x32_f16(columns(wave * 16, k0), operand(k0), v, 0, 0, 0);
+  }
+  if (wave < COLS / 16 && m0 + out_r < M) {
     half4_t y;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) y[e] = (half_t)gelu_tanh_f32(v[e] + (float)ffn_bias_v[e]);
-    store_through(out + (size_t)(m0 + fold_r) * N + fold_n, __builtin_bit_cast(uint2_t, y));
+    for (int e = 0; e < 4; ++e) y[e] = (half_t)gelu_tanh_f32(v[e]);
+    store_through(out + (size_t)(m0 + out_r) * N + out_n, __builtin_bit_cast(uint2_t, y));
   }
   // the normalised rows, for the last LayerNorm: row r by column tile r, r + tiles_n, ...
   for (int r = tile_n; r < kLgRows && m0 + r < M; r += tiles_n)
     if ((int)threadIdx.x < HIDDEN / 8)
-      store_through(dst + (size_t)(m0 + r) * HIDDEN + threadIdx.x * 8, *(const uint4_t *)(lg_smem + r * PITCH + threadIdx.x * 8));
+      store_through(dst + (size_t)(m0 + r) * HIDDEN + threadIdx.x * 8,
+                    *(const uint4_t *)(rows + r * HIDDEN + lg_chunk(r, threadIdx.x) * 8));
 #endif
 }
 
 // Columns of a tile, 0 where the two launches are the faster way: a workgroup repeats its rows' work, which pays while it
 // has little of the weight to fetch (some 30 bytes a clock come to a CU) and its tiles fit one round of the chip with the
 // rows that may be live (all of them, or 120 % of the expected share of a padded batch).  LayerNorm and FFN1, us as two
-// launches / one with 32 columns / with 64: hidden 768, [K, N] weight, 32 rows 7.01 / 5.18 / 5.95, 48 rows 6.99 / 6.89 (two
-// rounds) / 5.96, 80 rows 7.19 / - / 6.03, 96 rows 7.22 / - / 8.47 (two rounds); hidden 1024 32 rows 7.58 / 5.60 / 6.24, 64
-// rows 7.60 / - / 6.34.  [N, K] weight, whose 64-byte pieces arrive more slowly: hidden 768 32 rows 6.12 / 5.03 / 6.44, 64
-// rows 6.36 / 7.71 / 6.61; hidden 1024 32 rows 6.49 / 5.13 / 7.29.  Wider tiles for more rows: 128 columns 160 rows 8.19 / 7.67,
-// 7.65 / 10.55 for [N, K]; 32 rows by 128 columns 256 rows 8.51 / 9.42, 8.26 / 11.34.
+// launches / one with 32 columns / with 64, from the rows on where 32 and 64 columns take a second round: hidden 768, [K, N]
+// weight, 32 rows 7.06 / 5.08 / 5.64, 33 rows 6.74 / 6.79 / 5.67, 80 rows 7.20 / - / 5.77, 96 rows 7.21 / - / 9.27; hidden 1024
+// 32 rows 7.55 / 5.48 / 6.17, 33 rows 7.23 / 8.41 / 6.19, 64 rows 7.57 / 9.00 / 6.22, 65 rows 7.80 / - / 10.36.  [N, K] weight: hidden
+// 768 32 rows 6.21 / 4.69, 33 rows 6.26 / 6.25; hidden 1024 32 rows 6.42 / 4.79, 33 rows 6.76 / 7.95; 64 columns, whose 64-byte
+// pieces came more slowly while the weight went to registers, were slower there than the two launches (32 rows 6.44 and 7.29)
+// and have no image here.  Nor have other hidden sizes: these two are what has been measured.
 static int lg_cols(int rows_cap, int all_live, int n, int k, int weight_kn) {
   if ((k != 768 && k != 1024) || option_gemm_tile() >= 0) return 0;
   const long long rows = all_live ? rows_cap : (rows_cap * 18LL + 24) / 25;
-  for (int cols = 32; cols <= (weight_kn ? 64 : 32); cols *= 2)
+  for (int cols = 32; cols <= (weight_kn ? 64 : 32); cols *= 2) {
+    // (32 columns of rows that fit one round here always fit one of tile 14, so one chain over k is built for 64 only)
+    if (cols == 32 && !product_takes_wave_k(rows_cap, n, k)) continue;
     if (n % (8 * cols) == 0 && n >= kLgRows * cols && (rows + kLgRows - 1) / kLgRows * (n / cols) <= cu_count()) return cols;
+  }
   return 0;
 }
 
@@ -218,17 +240,20 @@ extern "C" int bt_layernorm_gemm_bias_gelu(const void *src, const void *residual
   BT_REQUIRE(cols, BT_ERR_UNSUPPORTED, "%s: %d rows of hidden_dim %d times %d columns are outside what "
              "bt_layernorm_gemm_bias_gelu_pays allows", who, rows_cap, hidden_dim, n);
   const unsigned grid = (unsigned)((rows_cap + kLgRows - 1) / kLgRows * (n / cols));
-  const auto launch = [&](auto hidden, auto width, auto kn) {
-    return Launch<layernorm_gelu_kernel<hidden(), width(), kn()>>::on(
+  const bool sliced = product_takes_wave_k(rows_cap, n, hidden_dim);
+  const auto launch = [&](auto hidden, auto width, auto kn, auto slices) {
+    return Launch<layernorm_gelu_kernel<hidden(), width(), kn(), slices()>>::on(
         as_stream(stream), who, grid, kLgWaves * kWave, LgShape<hidden(), width()>::kLds, (const half_t *)src,
         (const half_t *)residual, residual_row_index, valid_rows, (const half_t *)w, (const half_t *)bias, (const half_t *)gamma,
         (const half_t *)beta, (half_t *)dst, (const half_t *)ffn_bias, (half_t *)out, rows_cap, n, eps, 0);
   };
   using std::integral_constant;
   const auto by_tile = [&](auto hidden) {
-    if (cols == 64) return launch(hidden, integral_constant<int, 64>{}, std::true_type{});
-    return weight_kn ? launch(hidden, integral_constant<int, 32>{}, std::true_type{})
-                     : launch(hidden, integral_constant<int, 32>{}, std::false_type{});
+    if (cols == 64)
+      return sliced ? launch(hidden, integral_constant<int, 64>{}, std::true_type{}, std::true_type{})
+                    : launch(hidden, integral_constant<int, 64>{}, std::true_type{}, std::false_type{});
+    return weight_kn ? launch(hidden, integral_constant<int, 32>{}, std::true_type{}, std::true_type{})
+                     : launch(hidden, integral_constant<int, 32>{}, std::false_type{}, std::true_type{});
   };
   return hidden_dim == 768 ? by_tile(integral_constant<int, 768>{}) : by_tile(integral_constant<int, 1024>{});
 }

@@ -467,9 +467,9 @@ int bt_splitk_layernorm(const void *partials, int splits, const void *residual,
 
 /*
  * bt_add_bias_residual_layernorm and bt_gemm_bias_gelu in one launch, for a few dozen fp16 rows (no counterpart in the
- * reference): dst = LayerNorm(src + residual + bias), out[rows_cap, n] = gelu(dst . w + ffn_bias).  gamma and beta are
- * halfs; dst may be neither src nor residual.  all_live: every row of rows_cap is expected to be live, else 60 % of them;
- * like rows_cap it decides the tile, never what is computed.
+ * reference): dst = LayerNorm(src + residual + bias), out[rows_cap, n] = gelu(dst . w + ffn_bias), the bits of those two.  gamma
+ * and beta are halfs; dst may be neither src nor residual.  all_live: every row of rows_cap is expected to be live, else 60 %
+ * of them; it decides the tile, never what is computed.
  * bt_layernorm_gemm_bias_gelu_pays: whether there is such a launch for these sizes and it is the faster way (0 without a GPU).
  */
 int bt_layernorm_gemm_bias_gelu_pays(int rows_cap, int all_live, int n, int k, int weight_kn);

@@ -72,6 +72,36 @@ def test_both_layouts_give_the_same_bits():
     assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
 
 
+def _two_launches(rows, hidden, n, kn, live=None, gather=False):
+    """The inputs of _run through the LayerNorm's launch and FFN1's."""
+    gen = torch.Generator(device="cuda").manual_seed(rows * 7 + hidden + n)
+
+    def normal(*shape, std=1.0, mean=0.0):
+        return torch.empty(shape, dtype=torch.float16, device="cuda").normal_(mean, std, generator=gen)
+
+    src, residual, bias = normal(rows, hidden), normal(rows, hidden), normal(hidden, std=0.1)
+    gamma, beta, w, ffn_bias = normal(hidden, std=0.1, mean=1.0), normal(hidden, std=0.1), normal(hidden, n, std=0.02), normal(n, std=0.1)
+    count = None if live is None else torch.tensor([live], dtype=torch.int32, device="cuda")
+    index = torch.randperm(rows, generator=gen, device="cuda").int() if gather else None
+    ops.add_bias_residual_layernorm(src, residual, bias, gamma, beta, eps=EPS, valid_rows=count, residual_row_index=index)
+    return src, ops.gemm_bias_gelu(src, w if kn else w.t().contiguous(), ffn_bias, valid_rows=count, w_kn=kn)
+
+
+@pytest.mark.parametrize("rows,live", [(1, None), (16, None), (31, None), (32, None), (33, None), (64, None), (65, None), (80, None),
+                                       (44, 17), (64, 40), (88, 50), (111, 67), (111, 111)])
+@pytest.mark.parametrize("hidden,n", [(768, 3072), (768, 1024), (1024, 4096), (1024, 1024)])
+@pytest.mark.parametrize("kn", [True, False])
+def test_bits_of_the_two_launches(hidden, n, kn, rows, live):
+    """Sums in the order of the product that these sizes would get: four slices of k where that is tile 14 (at 3072 columns up
+    to 64 rows of capacity), one chain beyond."""
+    if not ops.layernorm_gemm_bias_gelu_pays(rows, live is None, n, hidden, w_kn=kn):
+        pytest.skip("two launches at these sizes")
+    gather = live is not None
+    got, want = _run(rows, hidden, n, kn, live, gather), _two_launches(rows, hidden, n, kn, live, gather)
+    m = rows if live is None else live
+    assert torch.equal(got[0][:m], want[0][:m]) and torch.equal(got[1][:m], want[1][:m])
+
+
 def test_sizes_that_keep_two_launches():
     for rows, n, k, kn in ((81, 3072, 768, True), (33, 3072, 768, False), (65, 4096, 1024, True), (33, 4096, 1024, False),
                            (32, 2048, 512, True), (32, 800, 768, True), (32, 3072, 640, True)):
