@@ -136,3 +136,31 @@ def test_weight_copies_change_no_bit(batch, seq_len):
     finally:
         ops.set_option("layer_prepack", -1)
     assert got[0].isfinite().all() and torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
+
+
+def _layer_inputs(batch, seq_len, H=768):
+    gen = torch.Generator(device="cuda").manual_seed(seq_len)
+
+    def normal(*shape, std=0.02, mean=0.0):
+        return torch.empty(shape, dtype=torch.float16, device="cuda").normal_(mean, std, generator=gen)
+
+    w = [normal(H, 3 * H), normal(3 * H), normal(H, H), normal(H), normal(H, std=0.05, mean=1.0), normal(H), normal(H, 4 * H), normal(4 * H),
+         normal(4 * H, H), normal(H), normal(H, std=0.05, mean=1.0), normal(H)]
+    x = normal(batch, seq_len, H, std=1.0)
+    lens = torch.arange(seq_len, 0, -(seq_len // batch), device="cuda")[:batch]
+    mask = (torch.arange(seq_len, device="cuda")[None, None, :] < lens[:, None, None]).half().expand(batch, seq_len, seq_len).contiguous()
+    return w, x, mask
+
+
+@pytest.mark.parametrize("packed", [True, False])
+@pytest.mark.parametrize("batch,seq_len", [(1, 32), (1, 72), (1, 200)])
+def test_ffn1_bias_inside_a_buffer(batch, seq_len, packed):
+    """A bias that starts 8 bytes into a flat parameter buffer, on both sides of the rows that this launch takes."""
+    bt.load_th_op()
+    w, x, mask = _layer_inputs(batch, seq_len)
+    want = torch.ops.ByteTransformer.BertTransformer(12, 64, *w, x, mask, packed, True)
+    flat = torch.zeros(w[7].numel() + 4, dtype=torch.float16, device="cuda")
+    flat[4:] = w[7]
+    w[7] = flat[4:]
+    assert w[7].data_ptr() % 16 == 8
+    assert torch.equal(torch.ops.ByteTransformer.BertTransformer(12, 64, *w, x, mask, packed, True), want)
