@@ -10,7 +10,7 @@ namespace bytetransformer {
 
 template <OperationType OpType>
 LayerPlan BertTransformer<OpType>::plan(int batch_size, int seq_len, bool have_offsets,
-                                        int valid_rows_hint) const {
+                                        int valid_rows_hint, int vouched_rows) const {
   LayerPlan lp;
   const int hidden = head_num_ * size_per_head_;
   const int inter = hidden * param_.intermediate_size;
@@ -43,6 +43,11 @@ LayerPlan BertTransformer<OpType>::plan(int batch_size, int seq_len, bool have_o
   const bool have_prepack = OpType == OperationType::HALF && param_.prepacked_kernels[0] &&
                             param_.prepacked_kernels[1] && param_.prepacked_kernels[2] &&
                             param_.prepacked_kernels[3];
+  // Few rows: the first LayerNorm in FFN1's launch.  It follows from sizes and from whose weights these are, not from a copy.
+  const bool exact = have_offsets && is_remove_padding_ && vouched_rows > 0 && vouched_rows <= rows;
+  lp.norm_in_ffn1 = OpType == OperationType::HALF && !use_fp32_ &&
+                    bt_layernorm_gemm_bias_gelu_pays(exact ? vouched_rows : (int)rows, !is_remove_padding_ || exact, inter, hidden,
+                                                     have_prepack ? 0 : 1);
   if (!have_prepack && OpType == OperationType::HALF && !lp.mask_direct) {
     const long long live = valid_rows_hint > 0  ? valid_rows_hint
                            : is_remove_padding_ ? (rows * 3LL + 4) / 5
@@ -52,7 +57,7 @@ LayerPlan BertTransformer<OpType>::plan(int batch_size, int seq_len, bool have_o
     lp.copies = plan_weight_copies(live, rows, hidden, inter, size_per_head_ == 64,
                                    !fits ? 0 : (qkv_mask_rows_opt == 1 ? 2 : 1),
                                    fits && ln_weight_copy != 0 && batch_size <= 32, lp.copy,
-                                   lp.ln_copy);
+                                   lp.ln_copy, lp.norm_in_ffn1);
   }
   lp.starts_with_qkv = fits && lp.copies == 0;
   return lp;
@@ -112,7 +117,8 @@ void BertTransformer<OpType>::bert_infer(BertTransformerInferParam infer_param) 
       infer_param.offsets && infer_param.offsets->batch_idx && infer_param.offsets->word_idx;
   const bool streaming_fp16 = OpType == OperationType::HALF && size_per_head_ == 64 &&
                               !attention_layer_->uses_short_kernel(seq_len);
-  LayerPlan lp = plan(batch_size, seq_len, have_offsets, infer_param.valid_rows_hint);
+  const int vouched = have_offsets && is_remove_padding_ ? infer_param.offsets->valid_word_num : 0;
+  const LayerPlan lp = plan(batch_size, seq_len, have_offsets, infer_param.valid_rows_hint, vouched);
   const bool mask_direct = lp.mask_direct;
   const bool qkv_mask_rows = lp.starts_with_qkv;
   // The four products read the [k, n] weights as the caller stores them, exactly as the
@@ -131,7 +137,6 @@ void BertTransformer<OpType>::bert_infer(BertTransformerInferParam infer_param) 
   // at batch 16 x 512), and a short sequence in a long padded row still takes the split-k
   // FFN2.  The QKV product and the attention keep batch * seq_len: it is the row stride
   // of the per-head Q/K/V layout and the extent of the gathered input.
-  const int vouched = have_offsets && is_remove_padding_ ? infer_param.offsets->valid_word_num : 0;
   const bool exact = vouched > 0 && vouched <= rows;
   const int packed_cap = exact ? vouched : rows;
   // ... and the products behind the attention take every row of it for live: choices made from
@@ -139,11 +144,7 @@ void BertTransformer<OpType>::bert_infer(BertTransformerInferParam infer_param) 
   // 60 %.  Their rows lie in the scratch, so a row too many costs time only; the LayerNorms,
   // which read through the caller's word_idx, keep the device's count.
   const bool all_live = !is_remove_padding_ || exact;
-  // Few rows: the first LayerNorm in FFN1's launch.  It follows from sizes and from whose weights these are, not from a copy,
-  // and such a layer makes none for FFN1 nor beside the LayerNorm: copies change no bit.
-  const bool norm_in_ffn1 = OpType == OperationType::HALF && !use_fp32_ &&
-                            bt_layernorm_gemm_bias_gelu_pays(packed_cap, all_live, inter, hidden, have_prepack ? 0 : 1);
-  if (norm_in_ffn1) lp.copy[2] = lp.ln_copy[2] = lp.ln_copy[3] = false;
+  const bool norm_in_ffn1 = lp.norm_in_ffn1;
   const DataType_ *w_use[4] = {param_.attr_kernel_QKV, param_.attr_output_kernel,
                                param_.inter_kernel, param_.output_kernel};
   int w_kn[4] = {1, 1, 1, 1};

@@ -67,7 +67,9 @@ int bt_encoder_layer_forward(const bt_encoder_config *cfg, const bt_layer_weight
  * weight made during the call, 1 = by the call's first launch (bt_layer_prologue), 2 = by the
  * launch of the first LayerNorm (FFN1, FFN2), 0 = read as stored; plan[4]: 1 when the layer starts with the QKV
  * product that counts the mask rows itself (bt_gemm_qkv_bias_split_mask_rows) instead of
- * bt_layer_prologue; plan[5]: 1 when a layer on padded rows goes without offsets altogether.
+ * bt_layer_prologue; plan[5]: 1 when a layer on padded rows goes without offsets altogether.  Whether the first LayerNorm
+ * runs in FFN1's launch, which then has no copy of its weight, bt_layernorm_gemm_bias_gelu_pays says; it asks for the GPU,
+ * and without one the plan is that of the two launches.
  */
 int bt_encoder_layer_plan(const bt_encoder_config *cfg, int batch_size, int seq_len,
                           int rows_hint, int *plan);

@@ -96,6 +96,7 @@ struct LayerPlan {
   bool copy[4] = {false, false, false, false};   // QKV, projection, FFN1, FFN2 run on a per-call copy
   int copies = 0;                                // ... made by the launch ahead of the layer
   bool ln_copy[4] = {false, false, false, false};   // FFN1, FFN2: ... made by the first LayerNorm's launch
+  bool norm_in_ffn1 = false;     // few rows: the first LayerNorm runs in FFN1's launch, which reads its weight as stored
 };
 
 template <OperationType OpType>
@@ -182,8 +183,9 @@ class BertTransformer {
 
   void infer(BertTransformerInferParam infer_param) { bert_infer(infer_param); }
 
-  // The plan of a call with these sizes (have_offsets: the caller passes offsets of its own).
-  LayerPlan plan(int batch_size, int seq_len, bool have_offsets, int valid_rows_hint) const;
+  // The plan of a call with these sizes (have_offsets: the caller passes offsets of its own; vouched_rows: with their
+  // exact count, 0 = without).
+  LayerPlan plan(int batch_size, int seq_len, bool have_offsets, int valid_rows_hint, int vouched_rows = 0) const;
 
   void bert_infer(BertTransformerInferParam infer_param);
 

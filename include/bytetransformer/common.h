@@ -161,17 +161,19 @@ inline int rows_to_plan_for(int given, bool packed, int batch_size, long long ro
 // it then makes the others as well; without it the FFN copies ride in the LayerNorm's launch
 // (or, if they may not, are dropped unless they pay for a prologue: up to 10 k padded rows
 // never copying then wins 1.5-1.8 % per forward and loses as much beyond).
-// Returns the number of prologue copies.
+// `norm_in_ffn1`: FFN1's launch has the first LayerNorm in it and reads its weight as stored, so it gets no copy, and no
+// LayerNorm's launch is there to make one.  Returns the number of prologue copies.
 inline int plan_weight_copies(long long live, long long padded_rows, int hidden, int inter,
                               bool split_heads, int first_launch, bool ln_can_copy, bool copy[4],
-                              bool ln_copy[4]) {
+                              bool ln_copy[4], bool norm_in_ffn1 = false) {
+  ln_can_copy = ln_can_copy && !norm_in_ffn1;
   const int n[4] = {3 * hidden, hidden, inter, hidden}, k[4] = {hidden, hidden, hidden, inter};
   const int epilogue[4] = {split_heads ? BT_EPILOGUE_QKV_SPLIT : -1, BT_EPILOGUE_PLAIN,
                            BT_EPILOGUE_BIAS_GELU, BT_EPILOGUE_PLAIN};
   float gain[4] = {0.f, 0.f, 0.f, 0.f}, early = 0.f, total = 0.f;
   bool want[4], want_ln[4];
   for (int i = 0; i < 4; ++i) {
-    if (epilogue[i] >= 0) gain[i] = bt_gemm_prepack_gain_us(live, n[i], k[i], epilogue[i]);
+    if (epilogue[i] >= 0 && !(norm_in_ffn1 && i == 2)) gain[i] = bt_gemm_prepack_gain_us(live, n[i], k[i], epilogue[i]);
     want[i] = gain[i] > 1.0f;
     // (the table's gain is less the 0.5 us per megabyte that a copy costs the prologue; the LayerNorm's
     // launch makes one for half of that: 6.7 us without and 7.8 us with FFN1's 4.7 MB at batch 16 x 512)

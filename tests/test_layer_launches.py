@@ -25,14 +25,22 @@ struct Span {
   const char *begin, *end;
 };
 static Span partials, scratch;
+static int prologues = 0, prologue_copies = 0, ln_copies = 0, norms_in_ffn1 = 0, qkv_starts = 0;
+static bool norm_pays = false, only_ffn1_gains = false;   // what the kernels library would say on a GPU; whose copies pay
 static std::vector<Span> others;   // what the LayerNorm behind the slices reads and writes, and what outlives it
 static void take(const void *p, unsigned long long bytes) { others.push_back({(const char *)p, (const char *)p + bytes}); }
 extern "C" {
-int bt_layer_prologue(const void *, int, int, int, int *, int *, int *, int *, void *, int, int, int, const void *const *,
-                      void *const *, const int *, const int *, int, const void *const *, const unsigned long long *, void *) { return 0; }
+int bt_layer_prologue(const void *, int, int, int, int *, int *, int *, int *, void *, int, int, int copies, const void *const *,
+                      void *const *, const int *, const int *, int, const void *const *, const unsigned long long *, void *) {
+  ++prologues, prologue_copies += copies;
+  return 0;
+}
 int bt_gemm_qkv_bias_split(const void *, const int *, const void *, const void *, void *, const int *, int, int, int, int, int, void *) { return 0; }
 int bt_gemm_qkv_bias_split_mask_rows(const void *, const void *, int, int, int, const void *, const void *, void *, int *, int *,
-                                     int *, int, int, int, int, void *) { return 0; }
+                                     int *, int, int, int, int, void *) {
+  ++qkv_starts;
+  return 0;
+}
 int bt_attention_grouped(const void *, void *, const int *, const int *, const void *, const void *, int, int, int, int, int,
                          float, int, const void *const *, const unsigned long long *, int, const int *slots, const void *list, void *) {
   if (slots) take(slots, 256 * sizeof(int));
@@ -43,8 +51,11 @@ int bt_mask_prefix_slots(const void *, int, int, int, const int *, int *, void *
 int bt_add_bias_residual_layernorm(void *, const void *, const int *, const void *, const void *, const void *, int, const int *,
                                    int, int, float, void *) { return 0; }
 int bt_add_bias_residual_layernorm_copy(void *, const void *, const int *, const void *, const void *, const void *, int,
-                                        const int *, int, int, float, int, const void *const *, void *const *, const int *,
-                                        const int *, void *) { return 0; }
+                                        const int *, int, int, float, int copies, const void *const *, void *const *, const int *,
+                                        const int *, void *) {
+  ln_copies += copies;
+  return 0;
+}
 int bt_add_bias_residual_layernorm_restore(const void *, const void *, const void *, const void *, const void *, int, void *,
                                            const int *, const int *, int, int, int, float, void *) { return 0; }
 int bt_splitk_layernorm(const void *sums, int splits, const void *residual, const int *, const void *, const void *, const void *,
@@ -68,7 +79,16 @@ int bt_gemm_bias_gelu(const void *, const void *, const void *, void *, const in
 int bt_layernorm_gemm_bias_gelu(const void *, const void *, const int *, const void *, const void *, const void *, void *,
                                 const void *, const void *, void *, const int *, int, int all_live, int, int, int, float, void *) {
   live_by_size += all_live;
+  ++norms_in_ffn1;
   return 0;
+}
+int bt_layernorm_gemm_bias_gelu_pays(int rows_cap, int all_live, int n, int k, int weight_kn) {
+  if (norm_pays) return rows_cap <= 111;
+  return ((int (*)(int, int, int, int, int))dlsym(RTLD_NEXT, "bt_layernorm_gemm_bias_gelu_pays"))(rows_cap, all_live, n, k, weight_kn);
+}
+float bt_gemm_prepack_gain_us(long long rows, int n, int k, int epilogue) {
+  if (only_ffn1_gains) return epilogue == BT_EPILOGUE_BIAS_GELU ? 5.f : 0.f;
+  return ((float (*)(long long, int, int, int))dlsym(RTLD_NEXT, "bt_gemm_prepack_gain_us"))(rows, n, k, epilogue);
 }
 int bt_gemm_splitk_rows(const void *a, const void *, void *, int splits, const int *live, int rows, int, int, int k, int, void *) {
   slices = splits;
@@ -85,7 +105,34 @@ int bt_gemm_splitk_slices(int rows_cap, int all_live, int n, int k, int most) {
 
 // argv: layer|encoder  heads  batch  seq_len  live rows that the caller vouches for (-1: no offsets, -2: padded rows)
 // [batch and seq_len that the scratch is for]
+// or: plan  heads  batch  seq_len  live  (1: the first LayerNorm's launch may be FFN1's)  (1: only FFN1's copy pays)
+// (1: the LayerNorm's launch may carry copies): launches of a layer, and what its plan says of them
+static int plan_and_launches(char **argv) {
+  const int heads = std::atoi(argv[2]), batch = std::atoi(argv[3]), seq = std::atoi(argv[4]), live = std::atoi(argv[5]);
+  norm_pays = std::atoi(argv[6]) != 0, only_ffn1_gains = std::atoi(argv[7]) != 0;
+  bt_set_option("ln_weight_copy", std::atoi(argv[8]));
+  bt_set_option("layer_prepack", only_ffn1_gains ? -1 : 1);
+  static char some[4096];
+  const __half *t = (const __half *)some;
+  BertTransformerParam<OperationType::HALF> w;
+  w.attention_param.attr_bias_QKV = t;
+  w.attr_kernel_QKV = w.attr_output_kernel = w.inter_kernel = w.output_kernel = t;
+  BertTransformer<OperationType::HALF> layer(batch, heads, 64, seq, true, live != -2);
+  layer.initialize(w);
+  BertTransformerInferParam<__half> ip{t, t, (__half *)some, some, batch, seq, nullptr, nullptr};
+  ET_Param offsets{(int *)some, (int *)some, live};
+  if (live >= 0) ip.offsets = &offsets;
+  const LayerPlan lp = layer.plan(batch, seq, live >= 0, 0, live > 0 ? live : 0);
+  layer.infer(ip);
+  int copies = 0, by_ln = 0;
+  for (int i = 0; i < 4; ++i) copies += lp.copy[i], by_ln += lp.ln_copy[i];
+  std::printf("%d %d %d %d %d %d %d %d %d\n", prologues, prologue_copies, copies, lp.copies, ln_copies, by_ln, norms_in_ffn1,
+              lp.norm_in_ffn1, qkv_starts == lp.starts_with_qkv);
+  return 0;
+}
+
 int main(int argc, char **argv) {
+  if (argv[1][0] == 'p') return plan_and_launches(argv);
   const int heads = std::atoi(argv[2]), batch = std::atoi(argv[3]), seq = std::atoi(argv[4]), live = std::atoi(argv[5]);
   const int most = argc > 7 ? std::atoi(argv[6]) : batch, longest = argc > 7 ? std::atoi(argv[7]) : seq;
   const bool packed = live != -2;
@@ -179,3 +226,22 @@ def test_partial_sums_lie_apart(launches, kind, heads):
                 assert apart, (batch, seq_len, live, room, slices)
                 seen.add(slices)
     assert len(seen) >= 3, seen
+
+
+@pytest.mark.parametrize("live", [-1, -2, 30])   # its own offsets, padded rows, offsets with their count
+@pytest.mark.parametrize("only_ffn1_gains", [0, 1])
+@pytest.mark.parametrize("ln_weight_copy", [0, 1])
+@pytest.mark.parametrize("norm_pays", [0, 1])
+@pytest.mark.parametrize("batch,seq_len", [(1, 32), (3, 14), (3, 60)])   # (up to two sequences: padded rows)
+def test_the_plan_is_what_is_launched(launches, batch, seq_len, norm_pays, ln_weight_copy, only_ffn1_gains, live):
+    """Copies and where they are made, whether the first LayerNorm is in FFN1's launch, and whether the layer starts with the
+    QKV product: with the LayerNorm in FFN1's launch there is no copy for FFN1, and no prologue that only it would need."""
+    prologues, made, planned, count, ln_made, ln_planned, norms, norm_planned, starts = launches(
+        "plan", 12, batch, seq_len, live, norm_pays, only_ffn1_gains, ln_weight_copy)
+    assert (made, ln_made, norms) == (planned, ln_planned, norm_planned) and count == planned and starts
+    rows = live if live > 0 and batch > 2 else batch * seq_len
+    assert norms == (norm_pays and rows <= 111)
+    if norms:
+        assert ln_made == 0 and made <= 3 and not (only_ffn1_gains and made)
+        if only_ffn1_gains and live == -1:
+            assert prologues == 0
