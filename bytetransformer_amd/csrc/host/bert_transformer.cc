@@ -209,7 +209,13 @@ void BertTransformer<OpType>::bert_infer(BertTransformerInferParam infer_param) 
         warm[warm_count] = w_use[i];
         warm_bytes[warm_count++] = (unsigned long long)w_k[i] * w_n[i] * sizeof(DataType_);
       }
-  // float, operands split in every call: the launch that splits them counts the mask rows itself
+  // float, operands split in every call: the launch that splits them counts the mask rows itself, in every workgroup of the
+  // rows, the dead ones too.  Beside the weights' workgroups that costs less than the launch it takes the place of, up to the 64
+  // sequences and 64 KB of mask rows that bt_gemm_qkv_mask_rows_supported allows: prologue and split / one launch, us, hidden
+  // 768: 16 x 128 15.4 / 11.6, 16 x 256 16.8 / 13.4, 64 x 40 18.5 / 18.2, 16 x 512 19.8 / 18.1, 64 x 128 23.1 / 18.0, 32 x 384
+  // 25.1 / 23.8, 16 x 1024 26.3 / 25.5, 32 x 512 25.5 / 24.9, 64 x 256 29.1 / 26.0; of twelve layers each 16 x 256 219.2 / 216.1,
+  // 16 x 1024 659.5 / 659.6, 64 x 256 622.1 / 619.3.  (The fp16 layer counts in every tile of the QKV product, of which a
+  // workgroup has several there: hence its 32 sequences.)
   const bool f32_split = OpType == OperationType::FP32 && f32_splits_operands(rows, !is_remove_padding_, hidden, inter);
   int mask_rows_opt = -1;
   if (f32_split) bt_get_option("qkv_mask_rows", &mask_rows_opt);
