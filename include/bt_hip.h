@@ -74,8 +74,10 @@ const char *bt_last_error_string(void);
  *                   offsets starts with bt_gemm_qkv_bias_split_mask_rows (one launch less,
  *                   every weight read as stored) where that entry takes the shape and no
  *                   per-call weight copy pays | always with bt_layer_prologue | with the
- *                   fused entry wherever it takes the shape, without copies.  Same results
- *                   either way.
+ *                   fused entry wherever it takes the shape, without copies.  A padding-free
+ *                   float layer that splits its operands counts the mask rows in that launch
+ *                   (bt_split_f32_layer_mask_rows) where it takes the shape | starts with
+ *                   bt_layer_prologue | as -1.  Same results either way.
  *   "ln_weight_copy"  1 (default) | 0: a padding-free fp16 layer that goes without
  *                   bt_layer_prologue lets the launch of its first LayerNorm make the k-contiguous
  *                   copies that pay for FFN1 and FFN2 (bt_add_bias_residual_layernorm_copy) | such

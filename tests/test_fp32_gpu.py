@@ -687,6 +687,30 @@ def test_fp32_layers_on_split_operands(device, path, rm):
     _f32_check(got if rm else O.masked_output(got, wl.lens), _oracle32(wl), wl.lens, "f32 split/%s" % path, rm)
 
 
+@pytest.mark.parametrize("lens,S", [((512, 0, 300, 37), 512), (None, 40), (None, 205), (None, 1024), (None, 20)])
+def test_fp32_layers_rows_from_the_mask_never_change_the_result(device, lens, S):
+    """Float layers that split their operands: rows counted by the launch that splits them, or by a prologue.  An empty
+    sequence, 64 sequences of a few dozen tokens, odd lengths, the most mask rows the launch takes, more sequences than it takes."""
+    _say("fp32 qkv_mask_rows", lens, S)
+    bt.load_th_op()
+    batch = len(lens) if lens else {40: 64, 205: 20, 1024: 16, 20: 128}[S]
+    assert batch * S * 3 // 5 >= 1220 and ops.get_option("qkv_mask_rows") == -1
+    cfg = workload.EncoderConfig("f32 mr", batch, S, 8, layers=1, dtype="fp32", lens=lens or (), seed=S)
+    wl = workload.make_workload(cfg, bias_std=0.05, random_affine=True)
+    w = [_dev(wl.layers[0][n], device) for n in workload.WEIGHT_NAMES]
+    x, m = _dev(wl.x, device), _dev(wl.mask, device)
+    got = {}
+    try:
+        for choice in (0, 1, -1):
+            ops.set_option("qkv_mask_rows", choice)
+            got[choice] = torch.ops.ByteTransformer.BertTransformer(8, 64, *w, x, m, True, True)
+    finally:
+        ops.set_option("qkv_mask_rows", -1)
+    assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[-1])
+    live = torch.arange(S, device=device)[None, :] < torch.as_tensor(np.asarray(wl.lens), device=device)[:, None]
+    assert got[-1][live].isfinite().all() and got[-1][live].any(-1).all() and not got[-1][~live].any()
+
+
 @pytest.mark.parametrize("H", [768, 1024, 64, 4096, 260])
 def test_layernorm_f32(device, H):
     _say("layernorm_f32", H)
