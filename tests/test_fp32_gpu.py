@@ -309,26 +309,31 @@ def test_gemm_f32_split_against_float64(device, tile, rows, M, N, K):
         assert mine <= whole
 
 
-@pytest.mark.parametrize("rows,M,N,K", [(2561, 2560, 3072, 64), (3000, 2049, 3072, 768), (2560, 2305, 3070 // 32 * 32, 320), (2100, 2100, 4096, 128)])
-def test_gemm_f32_split_known_rows_change_no_bit(device, rows, M, N, K):
+# hint None: the count itself; 0: padded rows, all of them live; else one that is out of date, and more rows than one round has
+@pytest.mark.parametrize("rows,M,N,K,hint", [(2561, 2560, 3072, 64, None), (3000, 2049, 3072, 768, None),
+                                             (2560, 2305, 3070 // 32 * 32, 320, None), (2100, 2048, 4096, 128, None),
+                                             (2300, 2300, 3072, 128, 0), (6000, 5801, 3072, 192, 2200), (5000, 30, 3072, 64, 2560)])
+def test_gemm_f32_split_known_rows_change_no_bit(device, rows, M, N, K, hint):
     """The tile that a known row count may choose gives the bits of the other, among rows and columns out of proportion too."""
-    _say("gemm_f32_split rows_hint", rows, M, N, K)
+    _say("gemm_f32_split rows_hint", rows, M, N, K, hint)
+    known, cus = hint or M, torch.cuda.get_device_properties(device).multi_processor_count
+    assert -(-known // 256) * -(-N // 128) <= cus and -(-known // 96) * -(-N // 128) > 2 * cus, "one round of the large tile for more"
     rs = np.random.RandomState(rows + K)
     x, w = rs.standard_normal((rows, K)).astype(np.float32), (rs.standard_normal((K, N)) * 0.02).astype(np.float32)
-    x[5, 1], x[M - 1, 2], x[300, 3] = 1e20, 1e20, np.inf
+    x[5, 1], x[M - 1, 2], x[min(300, M - 2), 3] = 1e20, 1e20, np.inf
     w[7, 40], w[9, N - 1] = 1e12, 1e-30
     bias = _dev((rs.standard_normal(N) * 0.1).astype(np.float32), device)
-    vr = torch.tensor([M], dtype=torch.int32, device=device)
+    vr = None if hint == 0 else torch.tensor([M], dtype=torch.int32, device=device)
     wd, xd = _dev(w, device), _dev(x, device)
     (wp,), a, _ = ops.split_f32([wd], xd, layer=True)
     ge = torch.full((rows,), 9, dtype=torch.int32, device=device)
     got = []
-    for tile, hint in ((2, 0), (-1, M)):
+    for tile, given in ((2, 0), (-1, known)):
         ops.set_option("f32_gemm_tile", tile)
         try:
             raw = torch.zeros(rows, 1 + (N + 1023) // 1024, dtype=torch.int32, device=device)
-            got.append((ops.gemm_f32_split(a, wp, bias, None, vr, weight=wd, rows=xd, rows_hint=hint),
-                        ops.gemm_f32_split(a, wp, bias, ge, vr, raw=raw, weight=wd, rows=xd, rows_hint=hint), raw))
+            got.append((ops.gemm_f32_split(a, wp, bias, None, vr, weight=wd, rows=xd, rows_hint=given),
+                        ops.gemm_f32_split(a, wp, bias, ge, vr, raw=raw, weight=wd, rows=xd, rows_hint=given), raw))
         finally:
             ops.set_option("f32_gemm_tile", -1)
     for one, other in zip(*got):

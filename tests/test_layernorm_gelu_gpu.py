@@ -61,6 +61,14 @@ def test_live_rows_on_the_device(rows, kn, share):
     _run(rows, 768, 3072, kn, live=int(-(-rows * share // 1)), gather=True)
 
 
+@pytest.mark.parametrize("kn,rows", [(True, 80), (True, 64), (False, 32)])
+@pytest.mark.parametrize("live", [0, 1, 31])
+def test_fewer_live_rows_than_vouched_for(rows, kn, live):
+    """A caller's count decides the tile, the device's what is computed."""
+    assert ops.layernorm_gemm_bias_gelu_pays(rows, True, 3072, 768, w_kn=kn)
+    _run(rows, 768, 3072, kn, live=live, gather=True, all_live=True)
+
+
 @pytest.mark.parametrize("n", [768, 1536])
 def test_narrow_products(n):
     for kn in (True, False):
