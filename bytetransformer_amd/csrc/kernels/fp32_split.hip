@@ -809,7 +809,7 @@ extern "C" int bt_gemm_f32_split_with(const void *a_pairs, const int *a_exps, co
   // What a step waits for is its operands: a CU takes in about 40 bytes a clock from the L2 and reads 128 from the LDS, and
   // the larger the tile the fewer it needs, as long as no CU goes without.  us at 2458 rows of hidden 768, bt_gemm_f32 and
   // tiles 0 / 1 / 2: QKV 57 and 41 / 46 / 28, projection 21 and 13.1 / 12.6 / 17.4, FFN1 77 and 61 / 69 / 49, FFN2 68 and 40 /
-  // 45 / 62.  (256x128, eight waves: 38 / 33 / 36 / 103, but 75 for FFN1 from 2561 rows on, a second round: below;
+  // 45 / 62.  (256x128, eight waves: 38 / 33 / 40 / 103, but 71 for FFN1 from 2561 rows on, a second round: below;
   // 128x128, eight waves: 44 / 21 / 46 / 63.)  A launch is priced by its rounds of the chip, a last one
   // that is partly full where two workgroups share a CU at half of one and half of its share: 5 us less than these
   // and those of 600 and 4915 rows, give or take 15 %.  The groups add up in another order, so the choice follows from sizes
@@ -837,7 +837,7 @@ extern "C" int bt_gemm_f32_split_with(const void *a_pairs, const int *a_exps, co
   if (tile == 1) return launch_f32_split<64, 128, 2, 2, 2, 2>(p, s);
   // 256x128 with eight waves, a workgroup a CU, gives the bits of 96x128 (the same order of a sum, the same columns a wave),
   // so what the caller knows of the live rows may decide: where one round of it takes the place of more than one of those
-  // (FFN1 of 2458 rows in a layer 54 -> 36 us; QKV there, one round either way, stays at 27).
+  // (FFN1 of 2458 rows, alone 51 -> 40 us, in a layer 51 -> 39; QKV there, one round either way, keeps the 96x128).
   const long long known = valid_rows ? m.rows_hint : rows_cap, tiles_n = (n + 127) / 128;
   if (known > 0 && (known + 255) / 256 * tiles_n <= cu_count() && (known + 95) / 96 * tiles_n > 2 * cu_count() &&
       option_f32_gemm_tile() < 0)
